@@ -50,7 +50,7 @@ typedef enum sa2_dtype { SA2_F32 = 0, SA2_BF16 = 1, SA2_F16 = 2 } sa2_dtype;
 /* flags */
 #define SA2_FLAG_AUTO 0u            /* matrix-pipe (MFMA) kernels when the shape allows, fp32-FMA kernels otherwise */
 #define SA2_FLAG_FORCE_GENERIC 1u   /* fp32-FMA kernels (any dtype, any D <= 256) */
-#define SA2_FLAG_FORCE_MFMA 2u      /* MFMA kernels (bf16 or fp16 with D 32, 64, 128 or 256; fp32 with D 32, 64 or 128;
+#define SA2_FLAG_FORCE_MFMA 2u      /* MFMA kernels (bf16 or fp16 with D 32, 64, 128 or 256; fp32 with D 32, 64, 96 or 128;
                                        16-byte aligned rows) or SA2_ERR_UNSUPPORTED; also takes the pre-pass kernels
                                        of the 16-bit D 32/64/128 path whenever the window sizes allow, whatever the
                                        problem size (SA2_FLAG_AUTO leaves them out for small grids) */
@@ -66,10 +66,11 @@ int sa2_version(void);
 /* Static, NUL-terminated description of a status code. */
 const char* sa2_strerror(int status);
 
-/* 1 if sa2_forward would take MFMA kernels for this problem under SA2_FLAG_AUTO
- * (given 16-byte aligned rows), 0 if it would take the fp32-FMA kernels.  sa2_backward makes the
- * same choice: its MFMA kernels take any K' window (one wider than their on-chip accumulators hold
- * is walked in segments of deltas). */
+/* 1 if head_dim is one that MFMA kernels of the element type have a width of their own for (the ones
+ * SA2_FLAG_FORCE_MFMA accepts, given 16-byte aligned rows), 0 otherwise.  Under SA2_FLAG_AUTO head_dim 16
+ * and other head dims up to 128 (multiples of 4 in fp32, of 8 in 16 bits) also run on the matrix pipes, in a wider
+ * kernel or, in 16 bits, in the fp32 MFMA kernels.  sa2_backward makes the same choice: its MFMA
+ * kernels take any K' window (one wider than their on-chip accumulators hold is walked in segments). */
 int sa2_uses_mfma(int B, int N, int H, int D, int w1, int w2, int dtype);
 
 /*

@@ -100,20 +100,24 @@ size_t dsum_bytes(int B, int N, int H) { return align_up((size_t)B * H * N * siz
 // 16-bit MFMA kernels for head_dim 256, or the fp32 MFMA kernels.
 enum KernelPath { PATH_GENERIC, PATH_MFMA16, PATH_WIDE16, PATH_MFMA32 };
 
+// Head dims the matrix-pipe kernels of the element type have a width of their own for.  The others run in the next
+// wider kernel (head_dim 16) or in the fp32 MFMA kernels, which SA2_FLAG_AUTO chooses; a forced call asks for these.
+bool own_width(int D, int dtype) { return D == 32 || D == 64 || D == 128 || D == (dtype == SA2_F32 ? 96 : 256); }
+
 KernelPath pick_path(const Problem& p, int dtype, unsigned flags, bool backward, int* status) {
     *status = SA2_OK;
     if (flags & SA2_FLAG_FORCE_GENERIC) return PATH_GENERIC;
     KernelPath path = PATH_GENERIC;
-    if (dtype == SA2_F32) {
-        const bool ok = (backward ? f32_mfma_bwd_supported(p.D, p.w2, dtype) : f32_mfma_supported(p.D, dtype)) &&
-                        f32_mfma_layout_ok(p, backward);
-        if (ok) path = PATH_MFMA32;
-    } else {
-        const bool ok = (backward ? mfma_bwd_supported(p.B, p.N, p.H, p.D, p.w1, p.w2, dtype)
-                                  : mfma_supported(p.B, p.N, p.H, p.D, p.w1, p.w2, dtype)) &&
-                        mfma_layout_ok(p, backward);
-        if (ok) path = PATH_MFMA16;
-        else if ((backward ? wide_bwd_supported(p.D, p.w2, dtype) : wide_supported(p.D, dtype)) && mfma_layout_ok(p, backward))
+    if ((flags & SA2_FLAG_FORCE_MFMA) && !own_width(p.D, dtype)) {
+        *status = SA2_ERR_UNSUPPORTED;
+        return path;
+    }
+    if ((backward ? f32_mfma_bwd_supported(p.D, p.w2, dtype) : f32_mfma_supported(p.D, dtype))) {
+        if (f32_mfma_layout_ok(p, dtype, backward)) path = PATH_MFMA32;
+    } else if (dtype != SA2_F32 && mfma_layout_ok(p, backward)) {
+        if (backward ? mfma_bwd_supported(p.B, p.N, p.H, p.D, p.w1, p.w2, dtype) : mfma_supported(p.B, p.N, p.H, p.D, p.w1, p.w2, dtype))
+            path = PATH_MFMA16;
+        else if (backward ? wide_bwd_supported(p.D, p.w2, dtype) : wide_supported(p.D, dtype))
             path = PATH_WIDE16;
     }
     if (path == PATH_GENERIC && (flags & SA2_FLAG_FORCE_MFMA)) *status = SA2_ERR_UNSUPPORTED;
@@ -146,6 +150,7 @@ const char* sa2_strerror(int status) {
 
 int sa2_uses_mfma(int B, int N, int H, int D, int w1, int w2, int dtype) {
     if (check_dims(B, N, H, D, w1, w2, dtype, 1) != SA2_OK) return 0;
+    if (!own_width(D, dtype)) return 0;
     return (mfma_supported(B, N, H, D, reach(w1, 1, N), reach(w2, 1, N), dtype) || wide_supported(D, dtype) ||
             f32_mfma_supported(D, dtype)) ? 1 : 0;
 }
@@ -180,7 +185,7 @@ int sa2_forward(const void* q, const void* k1, const void* k2, const void* v1, c
     if (rc != SA2_OK) return rc;
     return path == PATH_MFMA16 ? launch_mfma_fwd(p, dtype, st)
            : path == PATH_WIDE16 ? launch_wide_fwd(p, dtype, st)
-           : path == PATH_MFMA32 ? launch_f32_mfma_fwd(p, st) : launch_generic_fwd(p, dtype, st);
+           : path == PATH_MFMA32 ? launch_f32_mfma_fwd(p, dtype, st) : launch_generic_fwd(p, dtype, st);
 }
 
 size_t sa2_bwd_workspace_bytes(int B, int N, int H, int D, int w1, int w2, int dtype, unsigned flags) {
@@ -248,7 +253,7 @@ int sa2_backward(const void* q, const void* k1, const void* k2, const void* v1, 
     if (rc != SA2_OK) return rc;
     return path == PATH_MFMA16 ? launch_mfma_bwd(p, dtype, st)
            : path == PATH_WIDE16 ? launch_wide_bwd(p, dtype, st)
-           : path == PATH_MFMA32 ? launch_f32_mfma_bwd(p, st) : launch_generic_bwd(p, dtype, st);
+           : path == PATH_MFMA32 ? launch_f32_mfma_bwd(p, dtype, st) : launch_generic_bwd(p, dtype, st);
 }
 
 int sa2_backward_static_workspace(const void* q, const void* k1, const void* k2, const void* v1, const void* v2,

@@ -85,13 +85,14 @@ bool mfma_layout_ok(const Problem& p, bool backward);
 int launch_mfma_fwd(const Problem& p, int dtype, hipStream_t st);
 int launch_mfma_bwd(const Problem& p, int dtype, hipStream_t st);
 size_t mfma_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2);
-// fp32 tensors on the fp32 MFMA (head_dim 32, 64, 128; rows 16-byte aligned)
+// fp32 arithmetic on the fp32 MFMA: fp32 tensors of any head_dim up to 128 that is a multiple of 4, and 16-bit tensors
+// of the head dims the 16-bit kernels do not have (multiples of 8 up to 120); rows 16-byte aligned
 bool f32_mfma_supported(int D, int dtype);
 bool f32_mfma_bwd_supported(int D, int w2, int dtype);
-bool f32_mfma_layout_ok(const Problem& p, bool backward);
+bool f32_mfma_layout_ok(const Problem& p, int dtype, bool backward);
 size_t f32_mfma_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2);
-int launch_f32_mfma_fwd(const Problem& p, hipStream_t st);
-int launch_f32_mfma_bwd(const Problem& p, hipStream_t st);
+int launch_f32_mfma_fwd(const Problem& p, int dtype, hipStream_t st);
+int launch_f32_mfma_bwd(const Problem& p, int dtype, hipStream_t st);
 // 16-bit tensors with head_dim 256 on the 16-bit MFMA (rows 16-byte aligned)
 bool wide_supported(int D, int dtype);
 bool wide_bwd_supported(int D, int w2, int dtype);

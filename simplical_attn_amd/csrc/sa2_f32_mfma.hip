@@ -1,5 +1,5 @@
 // fp32 tensors on the matrix pipes of gfx950: forward and backward with v_mfma_f32_32x32x2_f32
-// (fp32 products, fp32 accumulation), head_dim 32, 64 or 128.
+// (fp32 products, fp32 accumulation), head dims up to 128 in kernels 32, 64, 96 and 128 columns wide.
 //
 // Same expanded-row view as the 16-bit kernels: rows r = (i, delta), Q~[r] = q[i] * (k2[i-delta] +
 // k2_bias) * scale*log2(e), dO~[r] = dO[i] * (v2[i-delta] + v2_bias), everything in fp32.  A 32x32x2
@@ -74,40 +74,78 @@ __device__ __forceinline__ int xcd_order(int pid, int total) {
     return (total & 7) == 0 ? (pid & 7) * (total >> 3) + (pid >> 3) : pid;
 }
 
-typedef float fx4 __attribute__((ext_vector_type(4)));      // 16 bytes in flight (a plain vector: stays in registers)
+typedef float fx4 __attribute__((ext_vector_type(4)));      // 16 bytes in flight (plain vectors: stay in registers)
+typedef unsigned ux2 __attribute__((ext_vector_type(2)));
+
+// The element type of the tensors: four columns as they lie in memory (Raw), their fp32 values, and fp32 values rounded
+// to the type.  Everything between the loads and the stores is fp32.
+struct MemF32 {
+    typedef float T;
+    typedef fx4 Raw;
+    static constexpr int DTYPE = SA2_F32;
+    static __device__ __forceinline__ fx4 widen(Raw x) { return x; }
+    static __device__ __forceinline__ void store(T* p, float a, float b, float c, float d) { *(float4*)p = make_float4(a, b, c, d); }
+};
+template <class E>
+struct Mem16 {
+    typedef uint16_t T;
+    typedef ux2 Raw;
+    static constexpr int DTYPE = E::DTYPE;
+    static __device__ __forceinline__ fx4 widen(Raw x) { return fx4{E::lo(x[0]), E::hi(x[0]), E::lo(x[1]), E::hi(x[1])}; }
+    static __device__ __forceinline__ void store(T* p, float a, float b, float c, float d) {
+        *(uint2*)p = make_uint2(E::pack(a, b), E::pack(c, d));
+    }
+};
+
+// Four columns of a row.  PAD: the tensors have width <= D columns; the kernel's columns from there on read as zeros
+// and are not written (rows are multiples of four elements, so four columns are inside or outside together).
+template <class T, bool PAD>
+__device__ __forceinline__ typename T::Raw raw4(const typename T::T* row, int col, int width) {
+    if constexpr (PAD) {
+        if (col >= width) return (typename T::Raw)(0);
+    }
+    return *(const typename T::Raw*)(row + col);
+}
+template <class T, bool PAD>
+__device__ __forceinline__ float4 cols4(const typename T::T* row, int col, int width) {
+    const fx4 x = T::widen(raw4<T, PAD>(row, col, width));
+    return make_float4(x[0], x[1], x[2], x[3]);
+}
 
 // Rows [j0, j0+32) of two tensors (clamped to the sequence) from global memory to registers, and
 // from there to the two tiles of a stage.
-template <int D>
-__device__ __forceinline__ void tile_load(fx4 (&a)[F32Cfg<D>::KR], fx4 (&b)[F32Cfg<D>::KR], const float* ap, int64_t as,
-                                          const float* bp, int64_t bs, int j0, int N, int tid) {
+template <class T, int D, bool PAD>
+__device__ __forceinline__ void tile_load(typename T::Raw (&a)[F32Cfg<D>::KR], typename T::Raw (&b)[F32Cfg<D>::KR], const typename T::T* ap,
+                                          int64_t as, const typename T::T* bp, int64_t bs, int j0, int N, int tid, int width) {
 #pragma unroll
     for (int u = 0; u < F32Cfg<D>::KR; ++u) {
         const int c = tid + XT * u;
         const int row = c / (D / 4), col = c - row * (D / 4);
         int j = j0 + row;
         j = j < N ? j : N - 1;
-        a[u] = *(const fx4*)(ap + (int64_t)j * as + col * 4);
-        b[u] = *(const fx4*)(bp + (int64_t)j * bs + col * 4);
+        a[u] = raw4<T, PAD>(ap + (int64_t)j * as, col * 4, width);
+        b[u] = raw4<T, PAD>(bp + (int64_t)j * bs, col * 4, width);
     }
 }
-template <int D>
-__device__ __forceinline__ void tile_store(const fx4 (&a)[F32Cfg<D>::KR], const fx4 (&b)[F32Cfg<D>::KR], float* stage, int tid) {
+template <class T, int D>
+__device__ __forceinline__ void tile_store(const typename T::Raw (&a)[F32Cfg<D>::KR], const typename T::Raw (&b)[F32Cfg<D>::KR], float* stage,
+                                           int tid) {
     using C = F32Cfg<D>;
 #pragma unroll
     for (int u = 0; u < C::KR; ++u) {
         const int c = tid + XT * u;
         const int row = c / (D / 4), col = c - row * (D / 4);
-        *(fx4*)(stage + row * C::RS + col * 4) = a[u];
-        *(fx4*)(stage + C::TILE + row * C::RS + col * 4) = b[u];
+        *(fx4*)(stage + row * C::RS + col * 4) = T::widen(a[u]);
+        *(fx4*)(stage + C::TILE + row * C::RS + col * 4) = T::widen(b[u]);
     }
 }
 
 // ================================================================== forward =====
-template <int D>
+template <class T, int D, bool PAD>
 __global__ __launch_bounds__(XT) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 2 : 1, D <= 64 ? 2 : 1)))
 void f32_fwd_kernel(Problem p, int nqb, int total) {
     using C = F32Cfg<D>;
+    typedef typename T::T EL;
     extern __shared__ __attribute__((aligned(16))) float smem_f[];
     float* mrg_m = smem_f + 2 * C::STAGE;        // [XW][32]
     float* mrg_l = mrg_m + XW * 32;              // [XW][32]
@@ -122,11 +160,11 @@ void f32_fwd_kernel(Problem p, int nqb, int total) {
     const int i0 = qb * BQ, i = i0 + ln, ic = i < N ? i : N - 1;
     const int i_last = i0 + BQ - 1 < N ? i0 + BQ - 1 : N - 1;
 
-    const float* qp = (const float*)p.q.p + p.q.off(b, 0, h);
-    const float* k1p = (const float*)p.k1.p + p.k1.off(b, 0, h);
-    const float* k2p = (const float*)p.k2.p + p.k2.off(b, 0, h);
-    const float* v1p = (const float*)p.v1.p + p.v1.off(b, 0, h);
-    const float* v2p = (const float*)p.v2.p + p.v2.off(b, 0, h);
+    const EL* qp = (const EL*)p.q.p + p.q.off(b, 0, h);
+    const EL* k1p = (const EL*)p.k1.p + p.k1.off(b, 0, h);
+    const EL* k2p = (const EL*)p.k2.p + p.k2.off(b, 0, h);
+    const EL* v1p = (const EL*)p.v1.p + p.v1.off(b, 0, h);
+    const EL* v2p = (const EL*)p.v2.p + p.v2.off(b, 0, h);
 
     const int jt_lo = (i0 - w1 > 0 ? i0 - w1 : 0) / TJ, jt_hi = i_last / TJ;
     const int nt = jt_hi - jt_lo + 1;
@@ -135,10 +173,10 @@ void f32_fwd_kernel(Problem p, int nqb, int total) {
     const int total_steps = nrounds * nt;
     const float qscale = p.scale * LOG2E;
 
-    fx4 tk[C::KR], tv[C::KR];                    // the tile on its way from global memory to LDS
-    tile_load<D>(tk, tv, k1p, p.k1.sn, v1p, p.v1.sn, jt_lo * TJ, N, tid);
-    tile_store<D>(tk, tv, smem_f, tid);
-    tile_load<D>(tk, tv, k1p, p.k1.sn, v1p, p.v1.sn, (jt_lo + 1 % nt) * TJ, N, tid);
+    typename T::Raw tk[C::KR], tv[C::KR];                    // the tile on its way from global memory to LDS
+    tile_load<T, D, PAD>(tk, tv, k1p, p.k1.sn, v1p, p.v1.sn, jt_lo * TJ, N, tid, p.D);
+    tile_store<T, D>(tk, tv, smem_f, tid);
+    tile_load<T, D, PAD>(tk, tv, k1p, p.k1.sn, v1p, p.v1.sn, (jt_lo + 1 % nt) * TJ, N, tid, p.D);
     __syncthreads();
 
     // the wavefront's running softmax over its units: reference exponent, sum, weighted output
@@ -159,8 +197,8 @@ void f32_fwd_kernel(Problem p, int nqb, int total) {
         if (ok) {
 #pragma unroll
             for (int gg = 0; gg < C::DG; ++gg) {
-                const float4 qa = *(const float4*)(qp + (int64_t)ic * p.q.sn + 8 * gg + 4 * hf);
-                const float4 kb = *(const float4*)(k2p + (int64_t)kr * p.k2.sn + 8 * gg + 4 * hf);
+                const float4 qa = cols4<T, PAD>(qp + (int64_t)ic * p.q.sn, 8 * gg + 4 * hf, p.D);
+                const float4 kb = cols4<T, PAD>(k2p + (int64_t)kr * p.k2.sn, 8 * gg + 4 * hf, p.D);
                 qf[4 * gg + 0] = qa.x * qscale * (kb.x + p.k2_bias);
                 qf[4 * gg + 1] = qa.y * qscale * (kb.y + p.k2_bias);
                 qf[4 * gg + 2] = qa.z * qscale * (kb.z + p.k2_bias);
@@ -228,8 +266,8 @@ void f32_fwd_kernel(Problem p, int nqb, int total) {
             }
             // (unconditional: past the last step this moves a tile nobody reads, which is cheaper than a branch
             // around register arrays)
-            tile_store<D>(tk, tv, smem_f + ((g + 1) & 1) * C::STAGE, tid);
-            tile_load<D>(tk, tv, k1p, p.k1.sn, v1p, p.v1.sn, (jt_lo + (g + 2) % nt) * TJ, N, tid);
+            tile_store<T, D>(tk, tv, smem_f + ((g + 1) & 1) * C::STAGE, tid);
+            tile_load<T, D, PAD>(tk, tv, k1p, p.k1.sn, v1p, p.v1.sn, (jt_lo + (g + 2) % nt) * TJ, N, tid, p.D);
             __syncthreads();
         }
 
@@ -241,12 +279,12 @@ void f32_fwd_kernel(Problem p, int nqb, int total) {
             const float a = fast_exp2(M - Mu), c = fast_exp2(m - Mu);
             L = L * a + lt * c;
             M = M_new;
-            const float* vrow = v2p + (int64_t)kr * p.v2.sn + 4 * hf;
+            const EL* vrow = v2p + (int64_t)kr * p.v2.sn;
 #pragma unroll
             for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
                 for (int g4 = 0; g4 < 4; ++g4) {
-                    const float4 x = *(const float4*)(vrow + dt * 32 + 8 * g4);
+                    const float4 x = cols4<T, PAD>(vrow, dt * 32 + 8 * g4 + 4 * hf, p.D);
                     oacc[dt][4 * g4 + 0] = oacc[dt][4 * g4 + 0] * a + c * racc[dt][4 * g4 + 0] * (x.x + p.v2_bias);
                     oacc[dt][4 * g4 + 1] = oacc[dt][4 * g4 + 1] * a + c * racc[dt][4 * g4 + 1] * (x.y + p.v2_bias);
                     oacc[dt][4 * g4 + 2] = oacc[dt][4 * g4 + 2] * a + c * racc[dt][4 * g4 + 2] * (x.z + p.v2_bias);
@@ -287,17 +325,18 @@ void f32_fwd_kernel(Problem p, int nqb, int total) {
         const bool big = Mu > LOG2_EPS;
         const float denom = big ? Ls + 1e-8f * fast_exp2(-Mu) : Ls * fast_exp2(Mu - LOG2_EPS) + 1.f;
         const float inv = big ? 1.f / denom : fast_exp2(Mu - LOG2_EPS) / denom;
-        float* orow = (float*)p.out.p + p.out.off(b, io, h);
+        EL* orow = (EL*)p.out.p + p.out.off(b, io, h);
 #pragma unroll
         for (int x = 0; x < C::DT; ++x) {
             const int col = 32 * x + 4 * (tid & 7);
+            if (PAD && col >= p.D) continue;
             float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
             for (int w = 0; w < XW; ++w) {
                 const float4 y = *(const float4*)(mrg + (w * 32 + row) * C::RS + col);
                 acc.x += wgt[w] * y.x; acc.y += wgt[w] * y.y; acc.z += wgt[w] * y.z; acc.w += wgt[w] * y.w;
             }
-            *(float4*)(orow + col) = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+            T::store(orow + col, acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
         }
         if ((tid & 7) == 0)
             p.lse[(int64_t)bh * N + io] = big ? LN2 * Mu + logf(denom) : LN_EPS + logf(denom);
@@ -306,10 +345,11 @@ void f32_fwd_kernel(Problem p, int nqb, int total) {
 
 // ============================================== backward, K' side: dQ, dK', dV' =====
 // SEG: the K' window is walked in segments of segw deltas (a kernel of its own; segw = w2 + 1 otherwise)
-template <int D, bool SEG>
+template <class T, int D, bool SEG, bool PAD>
 __global__ __launch_bounds__(XT) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 2 : 1, D <= 64 ? 2 : 1)))
 void f32_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_part, int segw) {
     using C = F32Cfg<D>;
+    typedef typename T::T EL;
     extern __shared__ __attribute__((aligned(16))) float smem_f[];
     float* dk_s = smem_f + 2 * C::STAGE;         // [32][RS]: dK' rows k0 .. k0+31 (before the scale)
     float* dv_s = dk_s + 32 * C::RS;             // [32][RS]: dV' rows
@@ -327,12 +367,12 @@ void f32_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_par
     const int NRS = 32 + segw - 1;               // rows of the accumulator
     int dbase = 0;                               // first delta of the current segment
 
-    const float* qp = (const float*)p.q.p + p.q.off(b, 0, h);
-    const float* k1p = (const float*)p.k1.p + p.k1.off(b, 0, h);
-    const float* k2p = (const float*)p.k2.p + p.k2.off(b, 0, h);
-    const float* v1p = (const float*)p.v1.p + p.v1.off(b, 0, h);
-    const float* v2p = (const float*)p.v2.p + p.v2.off(b, 0, h);
-    const float* dop = (const float*)p.dout.p + p.dout.off(b, 0, h);
+    const EL* qp = (const EL*)p.q.p + p.q.off(b, 0, h);
+    const EL* k1p = (const EL*)p.k1.p + p.k1.off(b, 0, h);
+    const EL* k2p = (const EL*)p.k2.p + p.k2.off(b, 0, h);
+    const EL* v1p = (const EL*)p.v1.p + p.v1.off(b, 0, h);
+    const EL* v2p = (const EL*)p.v2.p + p.v2.off(b, 0, h);
+    const EL* dop = (const EL*)p.dout.p + p.dout.off(b, 0, h);
     const bool want_dq = p.dq.p != nullptr;
 
     const int n_units = (w2 < N - 1 - k0 ? w2 : N - 1 - k0) + 1;       // delta with k0 + delta < N
@@ -341,7 +381,7 @@ void f32_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_par
 
     for (int c = tid; c < (NRS + 64) * C::RS; c += XT) dk_s[c] = 0.f;      // all three accumulators
 
-    fx4 tk[C::KR], tv[C::KR];                    // the tile on its way from global memory to LDS
+    typename T::Raw tk[C::KR], tv[C::KR];                    // the tile on its way from global memory to LDS
     for (int round = 0; round < nrounds; ++round) {
         // queries of the round's units: k0 + 4*round .. k0 + 31 + 4*round + 3 (within the sequence)
         const int d_first = round * XW, d_last = d_first + XW - 1 < n_units - 1 ? d_first + XW - 1 : n_units - 1;
@@ -361,10 +401,10 @@ void f32_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_par
         if (ok) {
 #pragma unroll
             for (int gg = 0; gg < C::DG; ++gg) {
-                const float4 qa = *(const float4*)(qp + (int64_t)ic * p.q.sn + 8 * gg + 4 * hf);
-                const float4 ka = *(const float4*)(k2p + (int64_t)kc * p.k2.sn + 8 * gg + 4 * hf);
-                const float4 da = *(const float4*)(dop + (int64_t)ic * p.dout.sn + 8 * gg + 4 * hf);
-                const float4 va = *(const float4*)(v2p + (int64_t)kc * p.v2.sn + 8 * gg + 4 * hf);
+                const float4 qa = cols4<T, PAD>(qp + (int64_t)ic * p.q.sn, 8 * gg + 4 * hf, p.D);
+                const float4 ka = cols4<T, PAD>(k2p + (int64_t)kc * p.k2.sn, 8 * gg + 4 * hf, p.D);
+                const float4 da = cols4<T, PAD>(dop + (int64_t)ic * p.dout.sn, 8 * gg + 4 * hf, p.D);
+                const float4 va = cols4<T, PAD>(v2p + (int64_t)kc * p.v2.sn, 8 * gg + 4 * hf, p.D);
                 qf[4 * gg + 0] = qa.x * qscale * (ka.x + p.k2_bias);
                 qf[4 * gg + 1] = qa.y * qscale * (ka.y + p.k2_bias);
                 qf[4 * gg + 2] = qa.z * qscale * (ka.z + p.k2_bias);
@@ -382,9 +422,9 @@ void f32_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_par
         for (int dt = 0; dt < C::DT; ++dt) racc[dt] = gacc[dt] = zero16();
 
         // (the previous round's last barrier has passed: both stages are free)
-        tile_load<D>(tk, tv, k1p, p.k1.sn, v1p, p.v1.sn, jt_lo * TJ, N, tid);
-        tile_store<D>(tk, tv, smem_f, tid);
-        if (nt > 1) tile_load<D>(tk, tv, k1p, p.k1.sn, v1p, p.v1.sn, (jt_lo + 1) * TJ, N, tid);
+        tile_load<T, D, PAD>(tk, tv, k1p, p.k1.sn, v1p, p.v1.sn, jt_lo * TJ, N, tid, p.D);
+        tile_store<T, D>(tk, tv, smem_f, tid);
+        if (nt > 1) tile_load<T, D, PAD>(tk, tv, k1p, p.k1.sn, v1p, p.v1.sn, (jt_lo + 1) * TJ, N, tid, p.D);
         __syncthreads();
         for (int s = 0; s < nt; ++s) {
             const int j0 = (jt_lo + s) * TJ;
@@ -426,8 +466,8 @@ void f32_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_par
                     }
                 }
             }
-            if (s + 1 < nt) tile_store<D>(tk, tv, smem_f + ((s + 1) & 1) * C::STAGE, tid);
-            if (s + 2 < nt) tile_load<D>(tk, tv, k1p, p.k1.sn, v1p, p.v1.sn, (jt_lo + s + 2) * TJ, N, tid);
+            if (s + 1 < nt) tile_store<T, D>(tk, tv, smem_f + ((s + 1) & 1) * C::STAGE, tid);
+            if (s + 2 < nt) tile_load<T, D, PAD>(tk, tv, k1p, p.k1.sn, v1p, p.v1.sn, (jt_lo + s + 2) * TJ, N, tid, p.D);
             __syncthreads();
         }
 
@@ -440,9 +480,9 @@ void f32_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_par
             if (row_ok) {
                 const int g4 = (wave + ph) & 3;
                 const int col = 8 * g4 + 4 * hf;
-                const float* qrow = qp + (int64_t)ic * p.q.sn + col;
-                const float* drow = dop + (int64_t)ic * p.dout.sn + col;
-                const float* krow = k2p + (int64_t)kc * p.k2.sn + col;
+                const EL* qrow = qp + (int64_t)ic * p.q.sn;
+                const EL* drow = dop + (int64_t)ic * p.dout.sn;
+                const EL* krow = k2p + (int64_t)kc * p.k2.sn;
                 float* dkrow = dk_s + ln * C::RS + col;
                 float* dvrow = dv_s + ln * C::RS + col;
                 float* dqrow = dq_s + (ln + delta - dbase) * C::RS + col;
@@ -455,8 +495,8 @@ void f32_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_par
                         gv[t] = g4 == 0 ? gacc[dt][t] : g4 == 1 ? gacc[dt][4 + t] : g4 == 2 ? gacc[dt][8 + t] : gacc[dt][12 + t];
                         rv[t] = g4 == 0 ? racc[dt][t] : g4 == 1 ? racc[dt][4 + t] : g4 == 2 ? racc[dt][8 + t] : racc[dt][12 + t];
                     }
-                    const float4 qx = *(const float4*)(qrow + dt * 32);
-                    const float4 dx = *(const float4*)(drow + dt * 32);
+                    const float4 qx = cols4<T, PAD>(qrow, dt * 32 + col, p.D);
+                    const float4 dx = cols4<T, PAD>(drow, dt * 32 + col, p.D);
                     float4 a = *(float4*)(dkrow + dt * 32);
                     a.x += gv[0] * qx.x; a.y += gv[1] * qx.y; a.z += gv[2] * qx.z; a.w += gv[3] * qx.w;
                     *(float4*)(dkrow + dt * 32) = a;
@@ -464,7 +504,7 @@ void f32_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_par
                     c.x += rv[0] * dx.x; c.y += rv[1] * dx.y; c.z += rv[2] * dx.z; c.w += rv[3] * dx.w;
                     *(float4*)(dvrow + dt * 32) = c;
                     if (want_dq) {
-                        const float4 kx = *(const float4*)(krow + dt * 32);
+                        const float4 kx = cols4<T, PAD>(krow, dt * 32 + col, p.D);
                         float4 o = *(float4*)(dqrow + dt * 32);
                         o.x += gv[0] * (kx.x + p.k2_bias); o.y += gv[1] * (kx.y + p.k2_bias);
                         o.z += gv[2] * (kx.z + p.k2_bias); o.w += gv[3] * (kx.w + p.k2_bias);
@@ -506,12 +546,15 @@ void f32_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_par
 #pragma unroll
             for (int x = 0; x < C::DT; ++x) {
                 const int col = 32 * x + 4 * (tid & 7);
+                if (PAD && col >= p.D) continue;
                 if (p.dk2.p) {
                     const float4 a = *(const float4*)(dk_s + row * C::RS + col);
-                    *(float4*)((float*)p.dk2.p + p.dk2.off(b, ko, h) + col) =
-                        make_float4(a.x * p.scale, a.y * p.scale, a.z * p.scale, a.w * p.scale);
+                    T::store((EL*)p.dk2.p + p.dk2.off(b, ko, h) + col, a.x * p.scale, a.y * p.scale, a.z * p.scale, a.w * p.scale);
                 }
-                if (p.dv2.p) *(float4*)((float*)p.dv2.p + p.dv2.off(b, ko, h) + col) = *(const float4*)(dv_s + row * C::RS + col);
+                if (p.dv2.p) {
+                    const float4 a = *(const float4*)(dv_s + row * C::RS + col);
+                    T::store((EL*)p.dv2.p + p.dv2.off(b, ko, h) + col, a.x, a.y, a.z, a.w);
+                }
             }
         }
     }
@@ -528,11 +571,12 @@ void f32_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_par
 }
 
 // dQ[i] = scale * sum over the K' blocks kb with 32*kb <= i <= 32*kb + 31 + w2, in block order
-template <int D>
+template <class T, int D>
 __global__ __launch_bounds__(256) void f32_dq_sum_kernel(Problem p, int nkb, const float* __restrict__ dq_part, int64_t chunks) {
     const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (c >= chunks) return;
     const int col = (int)(c % (D / 4));
+    if (col * 4 >= p.D) return;              // (the partials' rows have the kernel's width)
     const int64_t rowid = c / (D / 4);
     const int i = (int)(rowid % p.N);
     const int bh = (int)(rowid / p.N);
@@ -546,18 +590,18 @@ __global__ __launch_bounds__(256) void f32_dq_sum_kernel(Problem p, int nkb, con
         const float4 y = *(const float4*)(dq_part + (((int64_t)bh * nkb + kb) * NR + (i - 32 * kb)) * D + col * 4);
         acc.x += y.x; acc.y += y.y; acc.z += y.z; acc.w += y.w;
     }
-    float* orow = (float*)p.dq.p + p.dq.off(b, i, h);
-    *(float4*)(orow + col * 4) = make_float4(acc.x * p.scale, acc.y * p.scale, acc.z * p.scale, acc.w * p.scale);
+    T::store((typename T::T*)p.dq.p + p.dq.off(b, i, h) + col * 4, acc.x * p.scale, acc.y * p.scale, acc.z * p.scale, acc.w * p.scale);
 }
 
 // =================================================== backward, K side: dK, dV =====
 // nsplit > 1 (grids smaller than the chip): the workgroup takes the sp-th share of the key block's stream
 // of units and writes fp32 partial sums to `part` ([dK | dV][nsplit][B*H][N][D]) for f32_kv_sum_kernel.
-template <int D, bool SPLIT>
+template <class T, int D, bool SPLIT, bool PAD>
 __global__ __launch_bounds__(XT) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 2 : 1, D <= 64 ? 2 : 1)))
 void f32_bwd_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __restrict__ part) {
     const int nsplit = SPLIT ? nsplit_arg : 1;
     using C = F32Cfg<D>;
+    typedef typename T::T EL;
     extern __shared__ __attribute__((aligned(16))) float smem_f[];
     float* lse_s = smem_f + 2 * C::STAGE;        // [2][32]  LSE*log2(e) of the unit's queries
     float* dsum_s = lse_s + 2 * 32;              // [2][32]
@@ -572,20 +616,20 @@ void f32_bwd_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __r
     const int N = p.N, w1 = p.w1, w2 = p.w2;
     const int j0 = jb * XJ, jw = j0 + 32 * wave, j = jw + ln, jc = j < N ? j : N - 1;
 
-    const float* qp = (const float*)p.q.p + p.q.off(b, 0, h);
-    const float* k1p = (const float*)p.k1.p + p.k1.off(b, 0, h);
-    const float* k2p = (const float*)p.k2.p + p.k2.off(b, 0, h);
-    const float* v1p = (const float*)p.v1.p + p.v1.off(b, 0, h);
-    const float* v2p = (const float*)p.v2.p + p.v2.off(b, 0, h);
-    const float* dop = (const float*)p.dout.p + p.dout.off(b, 0, h);
+    const EL* qp = (const EL*)p.q.p + p.q.off(b, 0, h);
+    const EL* k1p = (const EL*)p.k1.p + p.k1.off(b, 0, h);
+    const EL* k2p = (const EL*)p.k2.p + p.k2.off(b, 0, h);
+    const EL* v1p = (const EL*)p.v1.p + p.v1.off(b, 0, h);
+    const EL* v2p = (const EL*)p.v2.p + p.v2.off(b, 0, h);
+    const EL* dop = (const EL*)p.dout.p + p.dout.off(b, 0, h);
     const float qscale = p.scale * LOG2E;
 
     // this wavefront's K and V rows as resident B operands (column = key j, slots d = 8g + 4hf + t)
     float kf[D / 2], vf[D / 2];
 #pragma unroll
     for (int gg = 0; gg < C::DG; ++gg) {
-        const float4 ka = *(const float4*)(k1p + (int64_t)jc * p.k1.sn + 8 * gg + 4 * hf);
-        const float4 va = *(const float4*)(v1p + (int64_t)jc * p.v1.sn + 8 * gg + 4 * hf);
+        const float4 ka = cols4<T, PAD>(k1p + (int64_t)jc * p.k1.sn, 8 * gg + 4 * hf, p.D);
+        const float4 va = cols4<T, PAD>(v1p + (int64_t)jc * p.v1.sn, 8 * gg + 4 * hf, p.D);
         kf[4 * gg] = ka.x; kf[4 * gg + 1] = ka.y; kf[4 * gg + 2] = ka.z; kf[4 * gg + 3] = ka.w;
         vf[4 * gg] = va.x; vf[4 * gg + 1] = va.y; vf[4 * gg + 2] = va.z; vf[4 * gg + 3] = va.w;
     }
@@ -630,7 +674,7 @@ void f32_bwd_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __r
     }
 
     // ---- forming a unit: Q~ and dO~ tiles (32 rows), LSE and D of its queries ----
-    float4 fq[C::KR], fk[C::KR], fd[C::KR], fv[C::KR];
+    typename T::Raw fq[C::KR], fk[C::KR], fd[C::KR], fv[C::KR];
     float f_lse = 0.f, f_dsum = 0.f;
     auto fetch_unit = [&](int ib, int delta) {
 #pragma unroll
@@ -640,10 +684,10 @@ void f32_bwd_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __r
             int i = ib * BQ + row;
             i = i < N ? i : N - 1;
             const int k = i - delta > 0 ? i - delta : 0;
-            fq[u] = *(const float4*)(qp + (int64_t)i * p.q.sn + col * 4);
-            fk[u] = *(const float4*)(k2p + (int64_t)k * p.k2.sn + col * 4);
-            fd[u] = *(const float4*)(dop + (int64_t)i * p.dout.sn + col * 4);
-            fv[u] = *(const float4*)(v2p + (int64_t)k * p.v2.sn + col * 4);
+            fq[u] = raw4<T, PAD>(qp + (int64_t)i * p.q.sn, col * 4, p.D);
+            fk[u] = raw4<T, PAD>(k2p + (int64_t)k * p.k2.sn, col * 4, p.D);
+            fd[u] = raw4<T, PAD>(dop + (int64_t)i * p.dout.sn, col * 4, p.D);
+            fv[u] = raw4<T, PAD>(v2p + (int64_t)k * p.v2.sn, col * 4, p.D);
         }
         if (tid < 32) {
             int i = ib * BQ + tid;
@@ -660,10 +704,11 @@ void f32_bwd_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __r
             const int c = tid + XT * u;
             const int row = c / (D / 4), col = c - row * (D / 4);
             const float kb = p.k2_bias, vb = p.v2_bias;
-            *(float4*)(Qs + row * C::RS + col * 4) = make_float4(fq[u].x * qscale * (fk[u].x + kb), fq[u].y * qscale * (fk[u].y + kb),
-                                                                 fq[u].z * qscale * (fk[u].z + kb), fq[u].w * qscale * (fk[u].w + kb));
-            *(float4*)(Ds + row * C::RS + col * 4) = make_float4(fd[u].x * (fv[u].x + vb), fd[u].y * (fv[u].y + vb),
-                                                                 fd[u].z * (fv[u].z + vb), fd[u].w * (fv[u].w + vb));
+            const fx4 q4 = T::widen(fq[u]), k4 = T::widen(fk[u]), d4 = T::widen(fd[u]), v4 = T::widen(fv[u]);
+            *(float4*)(Qs + row * C::RS + col * 4) = make_float4(q4[0] * qscale * (k4[0] + kb), q4[1] * qscale * (k4[1] + kb),
+                                                                 q4[2] * qscale * (k4[2] + kb), q4[3] * qscale * (k4[3] + kb));
+            *(float4*)(Ds + row * C::RS + col * 4) = make_float4(d4[0] * (v4[0] + vb), d4[1] * (v4[1] + vb), d4[2] * (v4[2] + vb),
+                                                                 d4[3] * (v4[3] + vb));
         }
         if (tid < 32) {
             lse_s[buf * 32 + tid] = f_lse;
@@ -742,32 +787,35 @@ void f32_bwd_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __r
     }
 
     if (j < N) {
-        float* dkp = p.dk1.p ? (float*)p.dk1.p + p.dk1.off(b, j, h) + 4 * hf : nullptr;
-        float* dvp = p.dv1.p ? (float*)p.dv1.p + p.dv1.off(b, j, h) + 4 * hf : nullptr;
-        if constexpr (SPLIT) {
-            const int64_t BH = (int64_t)p.B * p.H;
-            if (dkp) dkp = part + (((0 * (int64_t)nsplit + sp) * BH + bh) * N + j) * D + 4 * hf;
-            if (dvp) dvp = part + (((1 * (int64_t)nsplit + sp) * BH + bh) * N + j) * D + 4 * hf;
+        // Q~ carries scale*log2(e): dK = ln2 * sum dS * Q~
+#pragma unroll
+        for (int which = 0; which < 2; ++which) {
+            const Tensor& t = which ? p.dv1 : p.dk1;
+            if (!t.p) continue;
+            const floatx16(&acc)[C::DT] = which ? dvacc : dkacc;
+            const float sc = which ? 1.f : LN2;
+#pragma unroll
+            for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+                for (int g4 = 0; g4 < 4; ++g4) {
+                    const int col = dt * 32 + 8 * g4 + 4 * hf;
+                    const float x0 = acc[dt][4 * g4] * sc, x1 = acc[dt][4 * g4 + 1] * sc, x2 = acc[dt][4 * g4 + 2] * sc, x3 = acc[dt][4 * g4 + 3] * sc;
+                    if constexpr (SPLIT)
+                        *(float4*)(part + (((which * (int64_t)nsplit + sp) * p.B * p.H + bh) * N + j) * D + col) = make_float4(x0, x1, x2, x3);
+                    else if (!PAD || col < p.D)
+                        T::store((EL*)t.p + t.off(b, j, h) + col, x0, x1, x2, x3);
+                }
         }
-#pragma unroll
-        for (int dt = 0; dt < C::DT; ++dt)
-#pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4) {
-                // Q~ carries scale*log2(e): dK = ln2 * sum dS * Q~
-                if (dkp) *(float4*)(dkp + dt * 32 + 8 * g4) = make_float4(dkacc[dt][4 * g4] * LN2, dkacc[dt][4 * g4 + 1] * LN2,
-                                                                           dkacc[dt][4 * g4 + 2] * LN2, dkacc[dt][4 * g4 + 3] * LN2);
-                if (dvp) *(float4*)(dvp + dt * 32 + 8 * g4) = make_float4(dvacc[dt][4 * g4], dvacc[dt][4 * g4 + 1], dvacc[dt][4 * g4 + 2],
-                                                                           dvacc[dt][4 * g4 + 3]);
-            }
     }
 }
 
 // dK and dV from the partial sums of a split launch, shares added in their order
-template <int D>
+template <class T, int D>
 __global__ __launch_bounds__(256) void f32_kv_sum_kernel(Problem p, int nsplit, const float* __restrict__ part, int64_t chunks) {
     const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (c >= chunks) return;
     const int col = (int)(c % (D / 4));
+    if (col * 4 >= p.D) return;
     const int64_t rowid = c / (D / 4);
     const int j = (int)(rowid % p.N);
     const int bh = (int)(rowid / p.N);
@@ -782,7 +830,7 @@ __global__ __launch_bounds__(256) void f32_kv_sum_kernel(Problem p, int nsplit, 
             const float4 y = *(const float4*)(part + (((which * (int64_t)nsplit + s) * BH + bh) * p.N + j) * D + col * 4);
             acc.x += y.x; acc.y += y.y; acc.z += y.z; acc.w += y.w;
         }
-        *(float4*)((float*)t.p + t.off(b, j, h) + col * 4) = acc;
+        T::store((typename T::T*)t.p + t.off(b, j, h) + col * 4, acc.x, acc.y, acc.z, acc.w);
     }
 }
 
@@ -801,21 +849,21 @@ size_t f32_dq_part_bytes(int B, int N, int H, int D, int w2) {
 }
 
 // ------------------------------------------------------------------ launchers ----
-template <int D>
+template <class T, int D, bool PAD>
 int launch_f32_fwd(const Problem& p, hipStream_t st) {
     using C = F32Cfg<D>;
     const int nqb = (p.N + BQ - 1) / BQ;
     const int64_t total = (int64_t)nqb * p.B * p.H;
     if (total > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
-    if (!allow_full_lds((const void*)f32_fwd_kernel<D>)) return SA2_ERR_LAUNCH_FAILED;
-    hipLaunchKernelGGL((f32_fwd_kernel<D>), dim3((unsigned)total), dim3(XT), C::FWD_LDS, st, p, nqb, (int)total);
+    if (!allow_full_lds((const void*)f32_fwd_kernel<T, D, PAD>)) return SA2_ERR_LAUNCH_FAILED;
+    hipLaunchKernelGGL((f32_fwd_kernel<T, D, PAD>), dim3((unsigned)total), dim3(XT), C::FWD_LDS, st, p, nqb, (int)total);
     return hipGetLastError() == hipSuccess ? SA2_OK : SA2_ERR_LAUNCH_FAILED;
 }
 
-template <int D>
+template <class T, int D, bool PAD>
 int launch_f32_bwd(const Problem& p, hipStream_t st) {
     using C = F32Cfg<D>;
-    int rc = launch_rowdot(p.out, p.dout, p.dsum, p.B, p.N, p.H, p.D, SA2_F32, st);
+    int rc = launch_rowdot(p.out, p.dout, p.dsum, p.B, p.N, p.H, p.D, T::DTYPE, st);
     if (rc != SA2_OK) return rc;
     if (p.dq.p || p.dk2.p || p.dv2.p) {
         const int nkb = (p.N + BQ - 1) / BQ;
@@ -824,16 +872,16 @@ int launch_f32_bwd(const Problem& p, hipStream_t st) {
         if (p.scratch_bytes < f32_dq_part_bytes(p.B, p.N, p.H, D, p.w2)) return SA2_ERR_WORKSPACE_TOO_SMALL;
         float* part = (float*)p.scratch;
         const int segw = C::kp_segment(p.w2);
-        if (!allow_full_lds((const void*)f32_bwd_kp_kernel<D, false>) || !allow_full_lds((const void*)f32_bwd_kp_kernel<D, true>))
+        if (!allow_full_lds((const void*)f32_bwd_kp_kernel<T, D, false, PAD>) || !allow_full_lds((const void*)f32_bwd_kp_kernel<T, D, true, PAD>))
             return SA2_ERR_LAUNCH_FAILED;
         if (segw < p.w2 + 1)
-            hipLaunchKernelGGL((f32_bwd_kp_kernel<D, true>), dim3((unsigned)total), dim3(XT), C::kp_lds(segw - 1), st, p, nkb, (int)total, part, segw);
+            hipLaunchKernelGGL((f32_bwd_kp_kernel<T, D, true, PAD>), dim3((unsigned)total), dim3(XT), C::kp_lds(segw - 1), st, p, nkb, (int)total, part, segw);
         else
-            hipLaunchKernelGGL((f32_bwd_kp_kernel<D, false>), dim3((unsigned)total), dim3(XT), C::kp_lds(segw - 1), st, p, nkb, (int)total, part, segw);
+            hipLaunchKernelGGL((f32_bwd_kp_kernel<T, D, false, PAD>), dim3((unsigned)total), dim3(XT), C::kp_lds(segw - 1), st, p, nkb, (int)total, part, segw);
         if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
         if (p.dq.p) {
             const int64_t chunks = (int64_t)p.B * p.H * p.N * (D / 4);
-            hipLaunchKernelGGL((f32_dq_sum_kernel<D>), dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, p, nkb, part, chunks);
+            hipLaunchKernelGGL((f32_dq_sum_kernel<T, D>), dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, p, nkb, part, chunks);
             if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
         }
     }
@@ -847,60 +895,97 @@ int launch_f32_bwd(const Problem& p, hipStream_t st) {
             if (p.scratch_bytes < f32_mfma_bwd_scratch_bytes(p.B, p.N, p.H, D, p.w1, p.w2)) return SA2_ERR_WORKSPACE_TOO_SMALL;
             kv_part = (float*)((char*)p.scratch + f32_dq_part_bytes(p.B, p.N, p.H, D, p.w2));
         }
-        if (!allow_full_lds((const void*)f32_bwd_kv_kernel<D, false>) || !allow_full_lds((const void*)f32_bwd_kv_kernel<D, true>))
+        if (!allow_full_lds((const void*)f32_bwd_kv_kernel<T, D, false, PAD>) || !allow_full_lds((const void*)f32_bwd_kv_kernel<T, D, true, PAD>))
             return SA2_ERR_LAUNCH_FAILED;
         if (nsplit > 1)
-            hipLaunchKernelGGL((f32_bwd_kv_kernel<D, true>), dim3((unsigned)total), dim3(XT), C::KV_LDS, st, p, njb, (int)total, nsplit, kv_part);
+            hipLaunchKernelGGL((f32_bwd_kv_kernel<T, D, true, PAD>), dim3((unsigned)total), dim3(XT), C::KV_LDS, st, p, njb, (int)total, nsplit, kv_part);
         else
-            hipLaunchKernelGGL((f32_bwd_kv_kernel<D, false>), dim3((unsigned)total), dim3(XT), C::KV_LDS, st, p, njb, (int)total, 1, kv_part);
+            hipLaunchKernelGGL((f32_bwd_kv_kernel<T, D, false, PAD>), dim3((unsigned)total), dim3(XT), C::KV_LDS, st, p, njb, (int)total, 1, kv_part);
         if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
         if (nsplit > 1) {
             const int64_t chunks = (int64_t)p.B * p.H * p.N * (D / 4);
-            hipLaunchKernelGGL((f32_kv_sum_kernel<D>), dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, p, nsplit, kv_part, chunks);
+            hipLaunchKernelGGL((f32_kv_sum_kernel<T, D>), dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, p, nsplit, kv_part, chunks);
             if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
         }
     }
     return SA2_OK;
 }
 
+// rows on a 16-byte grid
+template <int PER_CHUNK>
 bool rows16(const Tensor& t, int B, int N, int H) {
+    constexpr int M = PER_CHUNK - 1;
     if (!t.p) return true;
     if ((uintptr_t)t.p & 15u) return false;
-    return !((B > 1 && (t.sb & 3)) || (N > 1 && (t.sn & 3)) || (H > 1 && (t.sh & 3)));
+    return !((B > 1 && (t.sb & M)) || (N > 1 && (t.sn & M)) || (H > 1 && (t.sh & M)));
+}
+
+// Kernel width of a head_dim, and the call f(memory type, width, PAD) for it.  16-bit tensors come here only with head
+// dims that the 16-bit kernels do not have, always padded or 96 columns wide.
+int f32_width(int D) { return D <= 32 ? 32 : D <= 64 ? 64 : D <= 96 ? 96 : 128; }
+template <class F>
+int for_f32_width(int D, int dtype, F&& f) {
+    auto of_type = [&](auto m) {
+        constexpr bool F32 = decltype(m)::DTYPE == SA2_F32;
+        const bool exact = F32 && D == f32_width(D);
+        auto of_pad = [&](auto width) {
+            if constexpr (F32) {
+                if (exact) return f(m, width, std::false_type{});
+            }
+            return f(m, width, std::true_type{});
+        };
+        switch (f32_width(D)) {
+            case 32: return of_pad(std::integral_constant<int, 32>{});
+            case 64: return of_pad(std::integral_constant<int, 64>{});
+            case 96: return f(m, std::integral_constant<int, 96>{}, std::true_type{});
+            default: return of_pad(std::integral_constant<int, 128>{});
+        }
+    };
+    return dtype == SA2_F32 ? of_type(MemF32{}) : dtype == SA2_F16 ? of_type(Mem16<ElemF16>{}) : of_type(Mem16<ElemBF16>{});
 }
 
 }  // namespace
 
-bool f32_mfma_supported(int D, int dtype) { return dtype == SA2_F32 && (D == 32 || D == 64 || D == 128); }
+// fp32: any multiple of four columns.  16 bits: multiples of eight that the 16-bit kernels do not take.
+bool f32_mfma_supported(int D, int dtype) {
+    if (D < 4 || D > 128) return false;
+    return dtype == SA2_F32 ? D % 4 == 0 : D % 8 == 0 && D != 16 && D != 32 && D != 64 && D != 128;
+}
 
 bool f32_mfma_bwd_supported(int D, int w2, int dtype) {
     (void)w2;                // any K' window: wide ones are walked in segments
     return f32_mfma_supported(D, dtype);
 }
 
-bool f32_mfma_layout_ok(const Problem& p, bool backward) {
+bool f32_mfma_layout_ok(const Problem& p, int dtype, bool backward) {
+    auto ok = [&](const Tensor& t) { return dtype == SA2_F32 ? rows16<4>(t, p.B, p.N, p.H) : rows16<8>(t, p.B, p.N, p.H); };
     const Tensor* fwd[] = {&p.q, &p.k1, &p.k2, &p.v1, &p.v2, &p.out};
     for (const Tensor* t : fwd)
-        if (!rows16(*t, p.B, p.N, p.H)) return false;
+        if (!ok(*t)) return false;
     if (backward) {
         const Tensor* bwd[] = {&p.dout, &p.dq, &p.dk1, &p.dk2, &p.dv1, &p.dv2};
         for (const Tensor* t : bwd)
-            if (!rows16(*t, p.B, p.N, p.H)) return false;
+            if (!ok(*t)) return false;
     }
     return true;
 }
 
-size_t f32_mfma_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2) {
+size_t f32_mfma_bwd_scratch_bytes(int B, int N, int H, int head_dim, int w1, int w2) {
+    const int D = f32_width(head_dim);
     const int ns = f32_kv_nsplit(B, N, H, D, w1, w2);
     return f32_dq_part_bytes(B, N, H, D, w2) + (ns > 1 ? (size_t)2 * ns * B * H * (size_t)N * D * sizeof(float) : 0);
 }
 
-int launch_f32_mfma_fwd(const Problem& p, hipStream_t st) {
-    return p.D == 128 ? launch_f32_fwd<128>(p, st) : p.D == 64 ? launch_f32_fwd<64>(p, st) : launch_f32_fwd<32>(p, st);
+int launch_f32_mfma_fwd(const Problem& p, int dtype, hipStream_t st) {
+    return for_f32_width(p.D, dtype, [&](auto m, auto width, auto pad) {
+        return launch_f32_fwd<decltype(m), decltype(width)::value, decltype(pad)::value>(p, st);
+    });
 }
 
-int launch_f32_mfma_bwd(const Problem& p, hipStream_t st) {
-    return p.D == 128 ? launch_f32_bwd<128>(p, st) : p.D == 64 ? launch_f32_bwd<64>(p, st) : launch_f32_bwd<32>(p, st);
+int launch_f32_mfma_bwd(const Problem& p, int dtype, hipStream_t st) {
+    return for_f32_width(p.D, dtype, [&](auto m, auto width, auto pad) {
+        return launch_f32_bwd<decltype(m), decltype(width)::value, decltype(pad)::value>(p, st);
+    });
 }
 
 }  // namespace sa2

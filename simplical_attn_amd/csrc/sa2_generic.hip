@@ -363,18 +363,18 @@ __global__ __launch_bounds__(256) void rowdot_kernel(Tensor out, Tensor dout, fl
     if (lane == 0) dsum[row] = s;
 }
 
-// The same for 16-bit elements with 16-byte aligned rows and D = 8 << n: a lane takes eight
-// consecutive elements of a row in one 16-byte load per tensor, D / 8 lanes share a row, a
-// wavefront covers 512 / D rows.
+// The same for 16-bit elements with 16-byte aligned rows and D a multiple of 8: a lane takes eight
+// consecutive elements of a row in one 16-byte load per tensor, the next power of two of D / 8 lanes
+// share a row (at head_dim 96: 12 of 16 lanes work).
 template <typename T>
-__global__ __launch_bounds__(256) void rowdot_vec_kernel(Tensor out, Tensor dout, float* dsum, int N, int H, int lpr_log2,
+__global__ __launch_bounds__(256) void rowdot_vec_kernel(Tensor out, Tensor dout, float* dsum, int N, int H, int D, int lpr_log2,
                                                          int64_t rows) {
     const int lane = threadIdx.x & 63;
     const int lpr = 1 << lpr_log2;                        // lanes per row
     const int64_t row = (((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) << (6 - lpr_log2)) + (lane >> lpr_log2);
     const int sub = lane & (lpr - 1);
     float s = 0.f;
-    if (row < rows) {
+    if (row < rows && sub * 8 < D) {
         const int i = (int)(row % N);
         const int bh = (int)(row / N);
         const int b = bh / H, h = bh - b * H;
@@ -418,14 +418,13 @@ int launch_rowdot(const Tensor& out, const Tensor& dout, float* dsum, int B, int
     const int64_t rows = (int64_t)B * H * N;
     const int64_t blocks = (rows + 3) / 4;
     if (blocks > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
-    // 16-bit elements, D = 8, 16, .. 256 and 16-byte aligned rows: the vector kernel
+    // 16-bit elements, D a multiple of 8 up to 256 and 16-byte aligned rows: the vector kernel
     auto aligned = [&](const Tensor& t) {
         return ((uintptr_t)t.p & 15u) == 0 && (B == 1 || t.sb % 8 == 0) && (N == 1 || t.sn % 8 == 0) && (H == 1 || t.sh % 8 == 0);
     };
-    int lpr_log2 = -1;
-    for (int n = 0; n <= 5; ++n)
-        if (D == (8 << n)) lpr_log2 = n;
-    const bool vec = dtype != SA2_F32 && lpr_log2 >= 0 && aligned(out) && aligned(dout);
+    int lpr_log2 = 0;
+    while ((8 << lpr_log2) < D) ++lpr_log2;
+    const bool vec = dtype != SA2_F32 && D % 8 == 0 && aligned(out) && aligned(dout);
     return dispatch_dtype(dtype, [&](auto* tag) {
         using T = std::remove_pointer_t<decltype(tag)>;
         if constexpr (sizeof(T) == 2) {
@@ -433,7 +432,7 @@ int launch_rowdot(const Tensor& out, const Tensor& dout, float* dsum, int B, int
                 const int64_t per_block = (int64_t)4 << (6 - lpr_log2);           // rows per workgroup
                 const int64_t vblocks = (rows + per_block - 1) / per_block;
                 hipLaunchKernelGGL(rowdot_vec_kernel<T>, dim3((unsigned)vblocks), dim3(256), 0, st, out, dout, dsum, N, H,
-                                   lpr_log2, rows);
+                                   D, lpr_log2, rows);
                 return check_launch();
             }
         }

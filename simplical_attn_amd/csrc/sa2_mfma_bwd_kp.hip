@@ -93,7 +93,9 @@ struct KpCfg {
 // SEG = true: a K' window too wide for the dQ accumulator in LDS is cut into nseg runs of segw deltas, one
 // workgroup per (K' block, segment); a kernel of its own so that the common case carries none of it.  Each writes its own dQ partial (rows k0 + seg*segw ..) and, when
 // nseg > 1, fp32 partial dK' and dV' to `kpart` ([dV' | dK'][nseg][B*H][N][D]) for kp_sum_kernel.
-template <class E, int D, bool RAW, bool LEFT, int U, bool SEG = false>
+//
+// PAD: the tensors have p.D <= D columns (see load_cols8).
+template <class E, int D, bool RAW, bool LEFT, int U, bool SEG, bool PAD>
 __global__ __launch_bounds__(KT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_part, int left, int nseg_arg, int segw_arg,
                         float* __restrict__ kpart) {
@@ -181,6 +183,7 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
     // ---- staging of one K/V tile: wavefront w requests group w of both tiles, straight into LDS
     const bool t_owner = wave < C::NGROUP;
     const int t_row = wave * C::RPW + (lane % C::RPW), t_col = lane / C::RPW;
+    const bool t_inside = t_col * 8 < p.D;                    // (used when PAD)
     const uint32_t k_off = ((uint32_t)t_row * (uint32_t)p.k1.sn + t_col * 8) * 2u;
     const uint32_t v_off = ((uint32_t)t_row * (uint32_t)p.v1.sn + t_col * 8) * 2u;
     typedef __attribute__((address_space(3))) void* lds_ptr;
@@ -197,8 +200,13 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
         const char* kbp = (const char*)(k1p + (int64_t)j0 * p.k1.sn);
         const char* vbp = (const char*)(v1p + (int64_t)j0 * p.v1.sn);
         unsigned char* dst = smem_raw + (size_t)stage * (C::STAGE * 2) + wave * C::GROUP;
-        __builtin_amdgcn_global_load_lds((glb_ptr)(kbp + ko), (lds_ptr)dst, 16, 0, 0);
-        __builtin_amdgcn_global_load_lds((glb_ptr)(vbp + vo), (lds_ptr)(dst + C::TILE_BYTES), 16, 0, 0);
+        const char *ks = kbp + ko, *vs = vbp + vo;
+        if constexpr (PAD) {
+            ks = t_inside ? ks : (const char*)zero_chunk;
+            vs = t_inside ? vs : (const char*)zero_chunk;
+        }
+        __builtin_amdgcn_global_load_lds((glb_ptr)ks, (lds_ptr)dst, 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((glb_ptr)vs, (lds_ptr)(dst + C::TILE_BYTES), 16, 0, 0);
     };
 
     // ---- raw rows, LSE, D and the dQ accumulator -------------------------------------
@@ -208,15 +216,15 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
             const int row = c / CPR, col = c - row * CPR;
             int r = kq + row;
             r = r < N ? r : N - 1;
-            *(uint4*)(q_s + row * C::RS + col * 8) = *(const uint4*)(qp + (int64_t)r * p.q.sn + col * 8);
-            *(uint4*)(do_s + row * C::RS + col * 8) = *(const uint4*)(dop + (int64_t)r * p.dout.sn + col * 8);
+            *(uint4*)(q_s + row * C::RS + col * 8) = load_cols8<PAD>(qp + (int64_t)r * p.q.sn, col * 8, p.D);
+            *(uint4*)(do_s + row * C::RS + col * 8) = load_cols8<PAD>(dop + (int64_t)r * p.dout.sn, col * 8, p.D);
         }
         for (int c = tid; c < BQ * CPR; c += KT) {
             const int row = c / CPR, col = c - row * CPR;
             int r = k0 + row;
             r = r < N ? r : N - 1;
-            *(uint4*)(k2_s + row * C::RS + col * 8) = *(const uint4*)(k2p + (int64_t)r * p.k2.sn + col * 8);
-            *(uint4*)(v2_s + row * C::RS + col * 8) = *(const uint4*)(v2p + (int64_t)r * p.v2.sn + col * 8);
+            *(uint4*)(k2_s + row * C::RS + col * 8) = load_cols8<PAD>(k2p + (int64_t)r * p.k2.sn, col * 8, p.D);
+            *(uint4*)(v2_s + row * C::RS + col * 8) = load_cols8<PAD>(v2p + (int64_t)r * p.v2.sn, col * 8, p.D);
         }
         for (int c = tid; c < RQ; c += KT) {
             int r = kq + c;
@@ -343,13 +351,13 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
                     for (int v = 0; v < 16; ++v) racc[u][dt][v] = 0.f;
                 float lse2 = 0.f;
                 {
-                    const uint16_t* qrow = q_row(ln + delta[u]) + hf * 8;
-                    const uint16_t* krow = k2_row() + hf * 8;
+                    const uint16_t* qrow = q_row(ln + delta[u]);
+                    const uint16_t* krow = k2_row();
                     uint4 qav[C::DK], kxv[C::DK];       // all reads of the two rows first
 #pragma unroll
-                    for (int kk = 0; kk < C::DK; ++kk) qav[kk] = *(const uint4*)(qrow + kk * 16);
+                    for (int kk = 0; kk < C::DK; ++kk) qav[kk] = load_cols8<PAD && !RAW>(qrow, kk * 16 + hf * 8, p.D);
 #pragma unroll
-                    for (int kk = 0; kk < C::DK; ++kk) kxv[kk] = *(const uint4*)(krow + kk * 16);
+                    for (int kk = 0; kk < C::DK; ++kk) kxv[kk] = load_cols8<PAD && LEFT>(krow, kk * 16 + hf * 8, p.D);
 #pragma unroll
                     for (int kk = 0; kk < C::DK; ++kk) {
                         const uint4 qa = qav[kk];
@@ -442,10 +450,10 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 if (!ok[u]) continue;
-                const uint16_t* drow = do_row(ln + delta[u]) + 4 * hf;
+                const uint16_t* drow = do_row(ln + delta[u]);
                 uint2 dx[4 * C::DT];               // the dO row, read in one batch
 #pragma unroll
-                for (int e = 0; e < 4 * C::DT; ++e) dx[e] = *(const uint2*)(drow + (e >> 2) * 32 + 8 * (e & 3));
+                for (int e = 0; e < 4 * C::DT; ++e) dx[e] = load_cols4<PAD && !RAW>(drow, (e >> 2) * 32 + 8 * (e & 3) + 4 * hf, p.D);
 #pragma unroll
                 for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
@@ -465,6 +473,7 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
                     for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
                         for (int g4 = 0; g4 < 4; ++g4) {
+                            if (PAD && dt * 32 + 8 * g4 >= p.D) continue;
                             union { EL hh[4]; uint2 u; } o;
 #pragma unroll
                             for (int x = 0; x < 4; ++x) o.hh[x] = (EL)pacc[dt][4 * g4 + x];
@@ -502,13 +511,13 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
                     for (int v = 0; v < 16; ++v) gacc[u][dt][v] = 0.f;
                 float dsum = 0.f;
                 {
-                    const uint16_t* drow = do_row(ln + delta[u]) + hf * 8;
-                    const uint16_t* vrow = v2_row() + hf * 8;
+                    const uint16_t* drow = do_row(ln + delta[u]);
+                    const uint16_t* vrow = v2_row();
                     uint4 dav[C::DK], vxv[C::DK];       // all reads of the two rows first
 #pragma unroll
-                    for (int kk = 0; kk < C::DK; ++kk) dav[kk] = *(const uint4*)(drow + kk * 16);
+                    for (int kk = 0; kk < C::DK; ++kk) dav[kk] = load_cols8<PAD && !RAW>(drow, kk * 16 + hf * 8, p.D);
 #pragma unroll
-                    for (int kk = 0; kk < C::DK; ++kk) vxv[kk] = *(const uint4*)(vrow + kk * 16);
+                    for (int kk = 0; kk < C::DK; ++kk) vxv[kk] = load_cols8<PAD && LEFT>(vrow, kk * 16 + hf * 8, p.D);
 #pragma unroll
                     for (int kk = 0; kk < C::DK; ++kk) {
                         const uint4 da = dav[kk];
@@ -595,10 +604,10 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 if (!ok[u]) continue;
-                const uint16_t* qrow = q_row(ln + delta[u]) + 4 * hf;
+                const uint16_t* qrow = q_row(ln + delta[u]);
                 uint2 qx[4 * C::DT];               // the q row, read in one batch
 #pragma unroll
-                for (int e = 0; e < 4 * C::DT; ++e) qx[e] = *(const uint2*)(qrow + (e >> 2) * 32 + 8 * (e & 3));
+                for (int e = 0; e < 4 * C::DT; ++e) qx[e] = load_cols4<PAD && !RAW>(qrow, (e >> 2) * 32 + 8 * (e & 3) + 4 * hf, p.D);
 #pragma unroll
                 for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
@@ -620,6 +629,7 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
                         for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
                             for (int g4 = 0; g4 < 4; ++g4) {
+                                if (PAD && dt * 32 + 8 * g4 >= p.D) continue;
                                 union { EL hh[4]; uint2 u; } o;
 #pragma unroll
                                 for (int x = 0; x < 4; ++x) o.hh[x] = (EL)(p.scale * pacc[dt][4 * g4 + x]);
@@ -630,10 +640,10 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
                 if (ok[0] && want_dq) {
                     // (rows of keys past the end of the sequence carry zeros: their G is zero)
                     float* dst = dq_part + (((int64_t)bh * nkb_all + kb) * RQ + w2 + ln) * D + 4 * hf;
-                    const uint16_t* krow = k2_row() + 4 * hf;
+                    const uint16_t* krow = k2_row();
                     uint2 kx[4 * C::DT];           // the K' row, read in one batch
 #pragma unroll
-                    for (int e = 0; e < 4 * C::DT; ++e) kx[e] = *(const uint2*)(krow + (e >> 2) * 32 + 8 * (e & 3));
+                    for (int e = 0; e < 4 * C::DT; ++e) kx[e] = load_cols4<PAD>(krow, (e >> 2) * 32 + 8 * (e & 3) + 4 * hf, p.D);
 #pragma unroll
                     for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
@@ -746,7 +756,7 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
             const int rem = it - which * BQ * CHF;
             const int row = rem / CHF, c0 = (rem - row * CHF) * 8;
             const Tensor& t = which ? p.dk2 : p.dv2;
-            if (k0 + row < N && t.p) pre[j] = *(const uint4*)((const uint16_t*)t.p + t.off(b, k0 + row, h) + c0);
+            if (k0 + row < N && t.p && (!PAD || c0 < p.D)) pre[j] = *(const uint4*)((const uint16_t*)t.p + t.off(b, k0 + row, h) + c0);
         }
     }
     {
@@ -794,6 +804,7 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
                 *(float4*)(dst + 4) = make_float4(acc[4] * sc, acc[5] * sc, acc[6] * sc, acc[7] * sc);
                 continue;
             }
+            if (PAD && c0 >= p.D) continue;
             uint16_t* dst = (uint16_t*)t.p + t.off(b, k, h) + c0;
             const uint4 x = pre[j];                                 // zeros where the pre-pass did not run
             const float part[8] = {E::lo(x.x), E::hi(x.x), E::lo(x.y), E::hi(x.y),
@@ -815,6 +826,7 @@ __global__ __launch_bounds__(256) void mfma_bwd_dq_sum_kernel(Problem p, const f
     const int64_t it = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (it >= items) return;
     const int c0 = (int)(it % CH) * 8;
+    if (c0 >= p.D) return;                   // (the partials' rows have the kernel's width)
     const int64_t row = it / CH;
     const int N = p.N, RQ = BQ + p.w2;       // queries a K' block reaches
     const int RS = BQ + segw - 1;            // rows of one segment's partial
@@ -855,11 +867,11 @@ __global__ __launch_bounds__(256) void mfma_bwd_dq_sum_kernel(Problem p, const f
 
 // dK' and dV' from the fp32 partial sums of a segmented launch, segments added in their order
 template <class E>
-__global__ __launch_bounds__(256) void kp_sum_kernel(Problem p, int nseg, const float* __restrict__ kpart, int64_t chunks) {
+__global__ __launch_bounds__(256) void kp_sum_kernel(Problem p, int D, int nseg, const float* __restrict__ kpart, int64_t chunks) {
     const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (c >= chunks) return;
-    const int D = p.D;
     const int col = (int)(c % (D / 4));
+    if (col * 4 >= p.D) return;
     const int64_t rowid = c / (D / 4);
     const int k = (int)(rowid % p.N);
     const int bh = (int)(rowid / p.N);
@@ -901,7 +913,7 @@ size_t kp_dq_part_bytes(int B, int N, int H, int D, const KpPlan& pl) {
     return ((size_t)B * H * nkb * pl.nseg * (size_t)(BQ + pl.segw - 1) * D * sizeof(float) + 255) / 256 * 256;
 }
 
-template <class E, int D>
+template <class E, int D, bool PAD>
 int launch_kp(const Problem& p, hipStream_t st) {
     constexpr int U = kp_units<D>();
     using C = KpCfg<D, U>;
@@ -922,20 +934,20 @@ int launch_kp(const Problem& p, hipStream_t st) {
         const size_t lds_left = (size_t)C::NSTAGE * C::STAGE * 2 + KpCfg<D, 1>::PX_BYTES;
         const int ngrp = (nkb + NPAIR - 1) / NPAIR;
         const int64_t total_left = (int64_t)ngrp * p.B * p.H;
-        if (!allow_full_lds((const void*)mfma_bwd_kp_kernel<E, D, false, true, 1>)) return SA2_ERR_LAUNCH_FAILED;
-        hipLaunchKernelGGL((mfma_bwd_kp_kernel<E, D, false, true, 1>), dim3((unsigned)total_left), dim3(KT), lds_left, st, p, ngrp,
+        if (!allow_full_lds((const void*)mfma_bwd_kp_kernel<E, D, false, true, 1, false, PAD>)) return SA2_ERR_LAUNCH_FAILED;
+        hipLaunchKernelGGL((mfma_bwd_kp_kernel<E, D, false, true, 1, false, PAD>), dim3((unsigned)total_left), dim3(KT), lds_left, st, p, ngrp,
                            (int)total_left, part, 0, 1, p.w2 + 1, (float*)nullptr);
         if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
     }
     if (pl.nseg > 1) {
-        if (!allow_full_lds((const void*)mfma_bwd_kp_kernel<E, D, false, false, U, true>)) return SA2_ERR_LAUNCH_FAILED;
-        hipLaunchKernelGGL((mfma_bwd_kp_kernel<E, D, false, false, U, true>), dim3((unsigned)total), dim3(KT), lds, st, p, nkb,
+        if (!allow_full_lds((const void*)mfma_bwd_kp_kernel<E, D, false, false, U, true, PAD>)) return SA2_ERR_LAUNCH_FAILED;
+        hipLaunchKernelGGL((mfma_bwd_kp_kernel<E, D, false, false, U, true, PAD>), dim3((unsigned)total), dim3(KT), lds, st, p, nkb,
                            (int)total, part, left, pl.nseg, pl.segw, kpart);
     } else {
-        const void* fn = raw ? (const void*)mfma_bwd_kp_kernel<E, D, true, false, U> : (const void*)mfma_bwd_kp_kernel<E, D, false, false, U>;
+        const void* fn = raw ? (const void*)mfma_bwd_kp_kernel<E, D, true, false, U, false, PAD> : (const void*)mfma_bwd_kp_kernel<E, D, false, false, U, false, PAD>;
         if (!allow_full_lds(fn)) return SA2_ERR_LAUNCH_FAILED;
-        if (raw) hipLaunchKernelGGL((mfma_bwd_kp_kernel<E, D, true, false, U>), dim3((unsigned)total), dim3(KT), lds, st, p, nkb, (int)total, part, left, 1, p.w2 + 1, kpart);
-        else hipLaunchKernelGGL((mfma_bwd_kp_kernel<E, D, false, false, U>), dim3((unsigned)total), dim3(KT), lds, st, p, nkb, (int)total, part, left, 1, p.w2 + 1, kpart);
+        if (raw) hipLaunchKernelGGL((mfma_bwd_kp_kernel<E, D, true, false, U, false, PAD>), dim3((unsigned)total), dim3(KT), lds, st, p, nkb, (int)total, part, left, 1, p.w2 + 1, kpart);
+        else hipLaunchKernelGGL((mfma_bwd_kp_kernel<E, D, false, false, U, false, PAD>), dim3((unsigned)total), dim3(KT), lds, st, p, nkb, (int)total, part, left, 1, p.w2 + 1, kpart);
     }
     if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
     if (p.dq.p) {
@@ -946,7 +958,7 @@ int launch_kp(const Problem& p, hipStream_t st) {
     }
     if (pl.nseg > 1 && (p.dk2.p || p.dv2.p)) {
         const int64_t chunks = (int64_t)p.B * p.H * p.N * (D / 4);
-        hipLaunchKernelGGL((kp_sum_kernel<E>), dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, p, pl.nseg, kpart, chunks);
+        hipLaunchKernelGGL((kp_sum_kernel<E>), dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, p, D, pl.nseg, kpart, chunks);
         if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
     }
     return SA2_OK;
@@ -955,15 +967,16 @@ int launch_kp(const Problem& p, hipStream_t st) {
 }  // namespace
 
 // workspace of the K'-side kernel: the dQ partials, then (segmented launches) the dK' and dV' partials
-size_t kp_scratch_bytes(int B, int N, int H, int D, int w2) {
+size_t kp_scratch_bytes(int B, int N, int H, int head_dim, int w2) {
+    const int D = mfma_width(head_dim);
     const KpPlan pl = kp_plan(D, w2);
     return kp_dq_part_bytes(B, N, H, D, pl) + (pl.nseg > 1 ? (size_t)2 * pl.nseg * B * H * (size_t)N * D * sizeof(float) : 0);
 }
 
 int launch_mfma_bwd_kp(const Problem& p, int dtype, hipStream_t st) {
-    if (dtype == SA2_F16)
-        return p.D == 128 ? launch_kp<ElemF16, 128>(p, st) : p.D == 64 ? launch_kp<ElemF16, 64>(p, st) : launch_kp<ElemF16, 32>(p, st);
-    return p.D == 128 ? launch_kp<ElemBF16, 128>(p, st) : p.D == 64 ? launch_kp<ElemBF16, 64>(p, st) : launch_kp<ElemBF16, 32>(p, st);
+    return for_mfma_width(p.D, dtype, [&](auto e, auto width, auto pad) {
+        return launch_kp<decltype(e), decltype(width)::value, decltype(pad)::value>(p, st);
+    });
 }
 
 }  // namespace sa2

@@ -67,7 +67,8 @@ struct KvCfg {
 // SEG = true: a K' window too wide for LDS is walked in segments of ws_arg + 1 deltas; LDS holds the K'/V'
 // rows of one segment of a query block and they are reloaded at every segment.  (A kernel of its own, so that
 // the common case carries none of it.)
-template <class E, int D, bool BIAS, int KB, bool SEG, bool SPLIT>
+// PAD: the tensors have p.D <= D columns (see load_cols8).
+template <class E, int D, bool BIAS, int KB, bool SEG, bool SPLIT, bool PAD>
 __global__ __launch_bounds__(VT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __restrict__ part, int ws_arg) {
     const int nsplit = nsplit_arg;           // (1 unless SPLIT; kept a run-time value: the compiler's code for the sweep is better that way)
@@ -112,9 +113,13 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __
     for (int sb = 0; sb < KB; ++sb) {
         const Tensor& t = role ? p.v1 : p.k1;
         const int j = jw + 32 * sb + ln;
-        const uint16_t* src = (const uint16_t*)t.p + t.off(b, j < N ? j : N - 1, h) + hf * 8;
+        const uint16_t* src = (const uint16_t*)t.p + t.off(b, j < N ? j : N - 1, h);
 #pragma unroll
-        for (int kk = 0; kk < C::DK; ++kk) kvf[sb][kk] = *(const X8*)(src + kk * 16);
+        for (int kk = 0; kk < C::DK; ++kk) {
+            union { uint4 u; X8 v; } x;
+            x.u = load_cols8<PAD>(src, kk * 16 + hf * 8, p.D);
+            kvf[sb][kk] = x.v;
+        }
     }
     floatx16 oacc[KB][C::DT];                    // dV^T (P wavefront) or dK^T (dS wavefront)
 #pragma unroll
@@ -165,8 +170,8 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __
             const int row = c / CPR, col = c - row * CPR;
             int i = i0 + row;
             i = i < N ? i : N - 1;
-            const uint4 qa = *(const uint4*)(qp + (int64_t)i * p.q.sn + col * 8);
-            const uint4 da = *(const uint4*)(dop + (int64_t)i * p.dout.sn + col * 8);
+            const uint4 qa = load_cols8<PAD>(qp + (int64_t)i * p.q.sn, col * 8, p.D);
+            const uint4 da = load_cols8<PAD>(dop + (int64_t)i * p.dout.sn, col * 8, p.D);
             float* qd = q_s + row * C::FS + col * 8;
             float* dd = do_s + row * C::FS + col * 8;
             *(float4*)qd = make_float4(E::lo(qa.x) * qscale, E::hi(qa.x) * qscale, E::lo(qa.y) * qscale, E::hi(qa.y) * qscale);
@@ -178,8 +183,8 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __
             const int row = c / CPR, col = c - row * CPR;
             int k = i0 - dbase - ws + row;
             k = k < 0 ? 0 : (k < N ? k : N - 1);
-            *(uint4*)(k2_s + row * C::RS + col * 8) = *(const uint4*)(k2p + (int64_t)k * p.k2.sn + col * 8);
-            *(uint4*)(v2_s + row * C::RS + col * 8) = *(const uint4*)(v2p + (int64_t)k * p.v2.sn + col * 8);
+            *(uint4*)(k2_s + row * C::RS + col * 8) = load_cols8<PAD>(k2p + (int64_t)k * p.k2.sn, col * 8, p.D);
+            *(uint4*)(v2_s + row * C::RS + col * 8) = load_cols8<PAD>(v2p + (int64_t)k * p.v2.sn, col * 8, p.D);
         }
         if (tid < BQ) {
             int i = i0 + tid;
@@ -452,6 +457,7 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __
             for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
                 for (int g4 = 0; g4 < 4; ++g4) {
+                    if (PAD && dt * 32 + 8 * g4 >= p.D) continue;
                     union { EL hh[4]; uint2 u; } a;
 #pragma unroll
                     for (int x = 0; x < 4; ++x) a.hh[x] = (EL)(oacc[sb][dt][4 * g4 + x] * sc);
@@ -472,12 +478,13 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __
 }
 
 // dK and dV from the partial sums of a split launch, shares added in their order
+// (the partials' rows have the kernel's width D, of which p.D columns are stored)
 template <class E>
-__global__ __launch_bounds__(256) void kv_sum_kernel(Problem p, int nsplit, const float* __restrict__ part, int64_t chunks) {
+__global__ __launch_bounds__(256) void kv_sum_kernel(Problem p, int D, int nsplit, const float* __restrict__ part, int64_t chunks) {
     const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (c >= chunks) return;
-    const int D = p.D;
     const int col = (int)(c % (D / 4));
+    if (col * 4 >= p.D) return;
     const int64_t rowid = c / (D / 4);
     const int j = (int)(rowid % p.N);
     const int bh = (int)(rowid / p.N);
@@ -518,7 +525,7 @@ KvPlan kv_plan(int B, int N, int H, int D, int w1, int w2) {
     return pl;
 }
 
-template <class E, int D, int KB>
+template <class E, int D, int KB, bool PAD>
 int launch_kv_geometry(const Problem& p, int nsplit, hipStream_t st) {
     using C = KvCfg<D, KB>;
     const int njb = (p.N + C::VJ - 1) / C::VJ;
@@ -543,43 +550,44 @@ int launch_kv_geometry(const Problem& p, int nsplit, hipStream_t st) {
     };
     bool ok;
     if (nsplit > 1)
-        ok = seg    ? go(mfma_bwd_kv_kernel<E, D, true, KB, true, true>)
-             : bias ? go(mfma_bwd_kv_kernel<E, D, true, KB, false, true>)
-                    : go(mfma_bwd_kv_kernel<E, D, false, KB, false, true>);
+        ok = seg    ? go(mfma_bwd_kv_kernel<E, D, true, KB, true, true, PAD>)
+             : bias ? go(mfma_bwd_kv_kernel<E, D, true, KB, false, true, PAD>)
+                    : go(mfma_bwd_kv_kernel<E, D, false, KB, false, true, PAD>);
     else
-        ok = seg    ? go(mfma_bwd_kv_kernel<E, D, true, KB, true, false>)
-             : bias ? go(mfma_bwd_kv_kernel<E, D, true, KB, false, false>)
-                    : go(mfma_bwd_kv_kernel<E, D, false, KB, false, false>);
+        ok = seg    ? go(mfma_bwd_kv_kernel<E, D, true, KB, true, false, PAD>)
+             : bias ? go(mfma_bwd_kv_kernel<E, D, true, KB, false, false, PAD>)
+                    : go(mfma_bwd_kv_kernel<E, D, false, KB, false, false, PAD>);
     if (!ok) return SA2_ERR_LAUNCH_FAILED;
     if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
     if (nsplit > 1) {
         const int64_t chunks = (int64_t)p.B * p.H * p.N * (D / 4);
-        hipLaunchKernelGGL((kv_sum_kernel<E>), dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, p, nsplit, part, chunks);
+        hipLaunchKernelGGL((kv_sum_kernel<E>), dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, p, D, nsplit, part, chunks);
         if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
     }
     return SA2_OK;
 }
 
-template <class E, int D>
+template <class E, int D, bool PAD>
 int launch_kv(const Problem& p, hipStream_t st) {
     const KvPlan pl = kv_plan(p.B, p.N, p.H, D, p.w1, p.w2);
     if constexpr (D == 64) {
-        if (pl.kb == 2) return launch_kv_geometry<E, D, 2>(p, pl.nsplit, st);
+        if (pl.kb == 2) return launch_kv_geometry<E, D, 2, PAD>(p, pl.nsplit, st);
     }
-    return launch_kv_geometry<E, D, 1>(p, pl.nsplit, st);
+    return launch_kv_geometry<E, D, 1, PAD>(p, pl.nsplit, st);
 }
 
 }  // namespace
 
-size_t kv_split_scratch_bytes(int B, int N, int H, int D, int w1, int w2) {
+size_t kv_split_scratch_bytes(int B, int N, int H, int head_dim, int w1, int w2) {
+    const int D = mfma_width(head_dim);
     const KvPlan pl = kv_plan(B, N, H, D, w1, w2);
     return pl.nsplit > 1 ? (size_t)2 * pl.nsplit * B * H * (size_t)N * D * sizeof(float) : 0;
 }
 
 int launch_mfma_bwd_kv(const Problem& p, int dtype, hipStream_t st) {
-    if (dtype == SA2_F16)
-        return p.D == 128 ? launch_kv<ElemF16, 128>(p, st) : p.D == 64 ? launch_kv<ElemF16, 64>(p, st) : launch_kv<ElemF16, 32>(p, st);
-    return p.D == 128 ? launch_kv<ElemBF16, 128>(p, st) : p.D == 64 ? launch_kv<ElemBF16, 64>(p, st) : launch_kv<ElemBF16, 32>(p, st);
+    return for_mfma_width(p.D, dtype, [&](auto e, auto width, auto pad) {
+        return launch_kv<decltype(e), decltype(width)::value, decltype(pad)::value>(p, st);
+    });
 }
 
 }  // namespace sa2

@@ -1,6 +1,8 @@
 // Types and device helpers shared by the gfx950 MFMA kernels (bf16 and fp16 elements).
 #pragma once
 
+#include <type_traits>
+
 #include "sa2_common.h"
 
 namespace sa2 {
@@ -78,6 +80,40 @@ struct ElemF16 {
         return __builtin_amdgcn_fdot2(a, b, c, false);
     }
 };
+
+// head_dim 16 runs in the 32-column kernels, compiled with PAD = true: columns from p.D on read as zeros (they add
+// nothing to a logit and give zero output and gradient columns) and are not written.  No copies: register loads are
+// guarded by these helpers, and a lane of a direct global->LDS load whose 16-byte chunk lies past the row reads the
+// zero chunk below instead.  Rows are multiples of 8 elements, so a chunk is inside or outside as a whole.
+__device__ __attribute__((aligned(16))) unsigned zero_chunk[4];
+template <bool PAD>
+__device__ __forceinline__ uint4 load_cols8(const uint16_t* row, int col, int width) {
+    if constexpr (PAD) {
+        if (col >= width) return make_uint4(0, 0, 0, 0);
+    }
+    return *(const uint4*)(row + col);
+}
+template <bool PAD>
+__device__ __forceinline__ uint2 load_cols4(const uint16_t* row, int col, int width) {
+    if constexpr (PAD) {
+        if (col >= width) return make_uint2(0, 0);
+    }
+    return *(const uint2*)(row + col);
+}
+// The width of the tuned 16-bit kernels a head_dim runs in, and the call f(element type, width, PAD) for it
+inline int mfma_width(int D) { return D <= 32 ? 32 : D; }
+template <class F>
+int for_mfma_width(int D, int dtype, F&& f) {
+    auto of_type = [&](auto e) {
+        switch (D) {
+            case 128: return f(e, std::integral_constant<int, 128>{}, std::false_type{});
+            case 64: return f(e, std::integral_constant<int, 64>{}, std::false_type{});
+            case 32: return f(e, std::integral_constant<int, 32>{}, std::false_type{});
+            default: return f(e, std::integral_constant<int, 32>{}, std::true_type{});
+        }
+    };
+    return dtype == SA2_F16 ? of_type(ElemF16{}) : of_type(ElemBF16{});
+}
 
 // Exchange between lane l and lane l^32 (one VALU op): returns the partner's value.
 __device__ __forceinline__ float other_half(float x) {

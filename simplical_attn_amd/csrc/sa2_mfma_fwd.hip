@@ -123,7 +123,8 @@ __device__ __forceinline__ void issue_v_all(uint32_t addr, lds_half_operand (&vh
 
 // SIDE: the K' and V' rows the block's deltas reach are copied to LDS (they fit); otherwise
 // they are read from global memory where they are needed.
-template <class E, int D, int MODE, bool SIDE>
+// PAD: the tensors have p.D <= D columns (see load_cols8).
+template <class E, int D, int MODE, bool SIDE, bool PAD>
 __global__ __launch_bounds__(FT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void mfma_fwd_kernel(Problem p, int nqb, int total, int left) {
     typedef typename E::scalar EL;
@@ -191,6 +192,7 @@ void mfma_fwd_kernel(Problem p, int nqb, int total, int left) {
     // when D = 64).  Tiles are requested strictly in sweep order into consecutive ring stages.
     const bool t_owner = wave < C::NGROUP;
     const int t_row = wave * C::RPW + (lane % C::RPW), t_col = lane / C::RPW;
+    const bool t_inside = t_col * 8 < p.D;                      // (used when PAD)
     const uint32_t k_off = ((uint32_t)t_row * (uint32_t)p.k1.sn + t_col * 8) * 2u;
     const uint32_t v_off = ((uint32_t)t_row * (uint32_t)p.v1.sn + t_col * 8) * 2u;
     // the same for the tile that holds the end of the sequence: rows past it are clamped to the
@@ -212,8 +214,13 @@ void mfma_fwd_kernel(Problem p, int nqb, int total, int left) {
             const char* kb = (const char*)(k1p + (int64_t)j0 * p.k1.sn);
             const char* vb = (const char*)(v1p + (int64_t)j0 * p.v1.sn);
             unsigned char* dst = smem_raw + (size_t)dma_stage * (C::STAGE * 2) + wave * C::GROUP;
-            __builtin_amdgcn_global_load_lds((glb_ptr)(kb + ko), (lds_ptr)dst, 16, 0, 0);
-            __builtin_amdgcn_global_load_lds((glb_ptr)(vb + vo), (lds_ptr)(dst + C::TILE_BYTES), 16, 0, 0);
+            const char *ks = kb + ko, *vs = vb + vo;
+            if constexpr (PAD) {
+                ks = t_inside ? ks : (const char*)zero_chunk;
+                vs = t_inside ? vs : (const char*)zero_chunk;
+            }
+            __builtin_amdgcn_global_load_lds((glb_ptr)ks, (lds_ptr)dst, 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((glb_ptr)vs, (lds_ptr)(dst + C::TILE_BYTES), 16, 0, 0);
         }
         dma_tile = dma_tile + 1 == nt ? 0 : dma_tile + 1;
         dma_stage = (dma_stage + 1) & (C::NSTAGE - 1);
@@ -233,7 +240,12 @@ void mfma_fwd_kernel(Problem p, int nqb, int total, int left) {
         if (has_left && !SAFE) {
             const uint16_t* prow = (const uint16_t*)p.out.p + p.out.off(b, io, h) + ac;
             uint32_t pw[ACN / 2];
-            load_words(prow, pw);
+            if constexpr (PAD) {
+#pragma unroll
+                for (int c = 0; c < ACN / 2; ++c) pw[c] = ac + 2 * c < p.D ? *(const uint32_t*)(prow + 2 * c) : 0u;
+            } else {
+                load_words(prow, pw);
+            }
             float* o = oacc + aq * C::OS + ac;
 #pragma unroll
             for (int c = 0; c < ACN / 2; ++c) {
@@ -270,15 +282,15 @@ void mfma_fwd_kernel(Problem p, int nqb, int total, int left) {
             const int row = c / CPR, col = c - row * CPR;
             int r = i0 + row;
             r = r < N ? r : N - 1;
-            *(uint4*)(q_s + row * C::KS + col * 8) = *(const uint4*)(qp + (int64_t)r * p.q.sn + col * 8);
+            *(uint4*)(q_s + row * C::KS + col * 8) = load_cols8<PAD>(qp + (int64_t)r * p.q.sn, col * 8, p.D);
         }
         if constexpr (SIDE) {
             for (int c = tid; c < side_rows * CPR; c += FT) {
                 const int row = c / CPR, col = c - row * CPR;
                 int r = i0 - w2 + row;
                 r = r < 0 ? 0 : (r < N ? r : N - 1);
-                *(uint4*)(k2_s + row * C::KS + col * 8) = *(const uint4*)(k2p + (int64_t)r * p.k2.sn + col * 8);
-                *(uint4*)(v2_s + row * C::KS + col * 8) = *(const uint4*)(v2p + (int64_t)r * p.v2.sn + col * 8);
+                *(uint4*)(k2_s + row * C::KS + col * 8) = load_cols8<PAD>(k2p + (int64_t)r * p.k2.sn, col * 8, p.D);
+                *(uint4*)(v2_s + row * C::KS + col * 8) = load_cols8<PAD>(v2p + (int64_t)r * p.v2.sn, col * 8, p.D);
             }
         }
     }
@@ -360,16 +372,16 @@ void mfma_fwd_kernel(Problem p, int nqb, int total, int left) {
             // ---- new unit: Q~ operand, fresh softmax state ----------------------
             X8 qf[C::DK];
             {
-                const uint16_t* krow = k2_row(delta) + hf * 8;
+                const uint16_t* krow = k2_row(delta);
                 const uint16_t* qrow;
-                if constexpr (LEFT) qrow = qp + (int64_t)ic * p.q.sn + hf * 8;
-                else qrow = q_s + ln * C::KS + hf * 8;
+                if constexpr (LEFT) qrow = qp + (int64_t)ic * p.q.sn;
+                else qrow = q_s + ln * C::KS;
                 // (all reads of the two rows first: from global memory they overlap)
                 uint4 qav[C::DK], kbv[C::DK];
 #pragma unroll
-                for (int kk = 0; kk < C::DK; ++kk) kbv[kk] = *(const uint4*)(krow + kk * 16);
+                for (int kk = 0; kk < C::DK; ++kk) kbv[kk] = load_cols8<PAD && !SIDE>(krow, kk * 16 + hf * 8, p.D);
 #pragma unroll
-                for (int kk = 0; kk < C::DK; ++kk) qav[kk] = *(const uint4*)(qrow + kk * 16);
+                for (int kk = 0; kk < C::DK; ++kk) qav[kk] = load_cols8<PAD && LEFT>(qrow, kk * 16 + hf * 8, p.D);
                 auto form_q = [&](auto BIASED) {
                     const float kbias = decltype(BIASED)::value ? p.k2_bias : 0.f;
 #pragma unroll
@@ -677,15 +689,16 @@ void mfma_fwd_kernel(Problem p, int nqb, int total, int left) {
             if (ok && i < N) {
                 const float inv = lt > 0.f ? 1.f / lt : 0.f;
                 const int kr = i - delta > 0 ? i - delta : 0;
-                const uint16_t* vrow = v2p + (int64_t)kr * p.v2.sn + 4 * hf;
+                const uint16_t* vrow = v2p + (int64_t)kr * p.v2.sn;
                 uint16_t* orow = (uint16_t*)p.out.p + p.out.off(b, i, h) + 4 * hf;
                 uint2 vx[4 * C::DT];               // the V' row, read in one batch
 #pragma unroll
-                for (int e = 0; e < 4 * C::DT; ++e) vx[e] = *(const uint2*)(vrow + (e >> 2) * 32 + 8 * (e & 3));
+                for (int e = 0; e < 4 * C::DT; ++e) vx[e] = load_cols4<PAD>(vrow, (e >> 2) * 32 + 8 * (e & 3) + 4 * hf, p.D);
 #pragma unroll
                 for (int dt = 0; dt < C::DT; ++dt)
 #pragma unroll
                     for (int g4 = 0; g4 < 4; ++g4) {
+                        if (PAD && dt * 32 + 8 * g4 >= p.D) continue;
                         const uint2 x = vx[4 * dt + g4];
                         union { EL h[4]; uint2 u; } o;
                         o.h[0] = (EL)(inv * racc[dt][4 * g4 + 0] * (E::lo(x.x) + p.v2_bias));
@@ -709,14 +722,14 @@ void mfma_fwd_kernel(Problem p, int nqb, int total, int left) {
                 const int ln_u = tid_u & 31, hf_u = (tid_u >> 5) & 1;
                 const uint16_t* vrow;
                 if constexpr (SIDE) {
-                    vrow = v2_s + (ln_u + w2 - delta) * C::KS + 4 * hf_u;
+                    vrow = v2_s + (ln_u + w2 - delta) * C::KS;
                 } else {
                     const int iq = i0 + ln_u < N ? i0 + ln_u : N - 1;
-                    vrow = v2p + (int64_t)(iq - delta > 0 ? iq - delta : 0) * p.v2.sn + 4 * hf_u;
+                    vrow = v2p + (int64_t)(iq - delta > 0 ? iq - delta : 0) * p.v2.sn;
                 }
                 uint2 vx[4 * C::DT];
 #pragma unroll
-                for (int e = 0; e < 4 * C::DT; ++e) vx[e] = *(const uint2*)(vrow + (e >> 2) * 32 + 8 * (e & 3));
+                for (int e = 0; e < 4 * C::DT; ++e) vx[e] = load_cols4<PAD && !SIDE>(vrow, (e >> 2) * 32 + 8 * (e & 3) + 4 * hf_u, p.D);
                 const float lt = l + other_half(l);
                 const bool row_has = (i0 + ln_u < N) & (i0 + ln_u >= delta);
                 // The fast kernel keeps a unit's reference point fixed, and every unit after the wavefront's
@@ -762,15 +775,15 @@ void mfma_fwd_kernel(Problem p, int nqb, int total, int left) {
         // the V' row of this lane's query, read in one batch before the exchange below
         const uint16_t* vrow;
         if constexpr (SIDE) {
-            vrow = v2_s + (ok ? ln_m + w2 - delta : 0) * C::KS + 4 * hf_m;
+            vrow = v2_s + (ok ? ln_m + w2 - delta : 0) * C::KS;
         } else {
             const int iq = i0 + ln_m < N ? i0 + ln_m : N - 1;
             const int vr = ok && iq - delta > 0 ? iq - delta : 0;
-            vrow = v2p + (int64_t)vr * p.v2.sn + 4 * hf_m;
+            vrow = v2p + (int64_t)vr * p.v2.sn;
         }
         uint2 vx[4 * C::DT];
 #pragma unroll
-        for (int e = 0; e < 4 * C::DT; ++e) vx[e] = *(const uint2*)(vrow + (e >> 2) * 32 + 8 * (e & 3));
+        for (int e = 0; e < 4 * C::DT; ++e) vx[e] = load_cols4<PAD && !SIDE>(vrow, (e >> 2) * 32 + 8 * (e & 3) + 4 * hf_m, p.D);
         const float lt = l + other_half(l);
         if (hf_m == 0) {
             xch_m[wave * BQ + ln_m] = m;
@@ -960,7 +973,13 @@ void mfma_fwd_kernel(Problem p, int nqb, int total, int left) {
         union { EL h[ACN]; uint32_t w[ACN / 2]; } o;
 #pragma unroll
         for (int c = 0; c < ACN; ++c) o.h[c] = (EL)(oacc[aq * C::OS + ac + c] * inv);
-        store_words(orow, o.w);
+        if constexpr (PAD) {
+#pragma unroll
+            for (int c = 0; c < ACN / 2; ++c)
+                if (ac + 2 * c < p.D) *(uint32_t*)(orow + 2 * c) = o.w[c];
+        } else {
+            store_words(orow, o.w);
+        }
         if ((tid_f & 15) == 0) {
             float lse;
             if (Ms > LOG2_EPS) lse = LN2 * (Ms + __log2f(L + 1e-8f * fast_exp2(-Ms)));
@@ -970,34 +989,34 @@ void mfma_fwd_kernel(Problem p, int nqb, int total, int left) {
     }
 }
 
-template <class E, int D, bool SIDE>
+template <class E, int D, bool SIDE, bool PAD>
 int launch_fwd_kernels(const Problem& p, int nqb, int total, hipStream_t st) {
     using C = Cfg<D>;
     const size_t lds = C::lds_bytes(p.w2);
     // one unit left over after the rounds of eight: the pre-pass takes it, unless the grid is so
     // small that a further launch costs more than the lone round
     const int left = (p.w2 >= FW && p.w2 % FW == 0 && (p.force_prepass || total >= PREPASS_MIN_WORKGROUPS)) ? 1 : 0;
-    if (!allow_full_lds((const void*)mfma_fwd_kernel<E, D, MODE_FAST, SIDE>) ||
-        !allow_full_lds((const void*)mfma_fwd_kernel<E, D, MODE_SAFE, SIDE>) ||
-        !allow_full_lds((const void*)mfma_fwd_kernel<E, D, MODE_LEFT, false>))
+    if (!allow_full_lds((const void*)mfma_fwd_kernel<E, D, MODE_FAST, SIDE, PAD>) ||
+        !allow_full_lds((const void*)mfma_fwd_kernel<E, D, MODE_SAFE, SIDE, PAD>) ||
+        !allow_full_lds((const void*)mfma_fwd_kernel<E, D, MODE_LEFT, false, PAD>))
         return SA2_ERR_LAUNCH_FAILED;
     if (left) {
         const int ngrp = (nqb + FW - 1) / FW;
         const int total_left = ngrp * (total / nqb);
-        hipLaunchKernelGGL((mfma_fwd_kernel<E, D, MODE_LEFT, false>), dim3((unsigned)total_left), dim3(FT), C::STAGE_BYTES, st, p,
+        hipLaunchKernelGGL((mfma_fwd_kernel<E, D, MODE_LEFT, false, PAD>), dim3((unsigned)total_left), dim3(FT), C::STAGE_BYTES, st, p,
                            ngrp, total_left, 0);
         if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
     }
-    hipLaunchKernelGGL((mfma_fwd_kernel<E, D, MODE_FAST, SIDE>), dim3((unsigned)total), dim3(FT), lds, st, p, nqb, total, left);
+    hipLaunchKernelGGL((mfma_fwd_kernel<E, D, MODE_FAST, SIDE, PAD>), dim3((unsigned)total), dim3(FT), lds, st, p, nqb, total, left);
     if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
-    hipLaunchKernelGGL((mfma_fwd_kernel<E, D, MODE_SAFE, SIDE>), dim3((unsigned)total), dim3(FT), lds, st, p, nqb, total, left);
+    hipLaunchKernelGGL((mfma_fwd_kernel<E, D, MODE_SAFE, SIDE, PAD>), dim3((unsigned)total), dim3(FT), lds, st, p, nqb, total, left);
     return hipGetLastError() == hipSuccess ? SA2_OK : SA2_ERR_LAUNCH_FAILED;
 }
 
-template <class E, int D>
+template <class E, int D, bool PAD>
 int launch_fwd_pair(const Problem& p, int nqb, int total, hipStream_t st) {
-    return Cfg<D>::side_fits(p.w2) ? launch_fwd_kernels<E, D, true>(p, nqb, total, st)
-                                   : launch_fwd_kernels<E, D, false>(p, nqb, total, st);
+    return Cfg<D>::side_fits(p.w2) ? launch_fwd_kernels<E, D, true, PAD>(p, nqb, total, st)
+                                   : launch_fwd_kernels<E, D, false, PAD>(p, nqb, total, st);
 }
 
 bool aligned16(const Tensor& t, int B, int N, int H) {
@@ -1015,7 +1034,7 @@ bool aligned16(const Tensor& t, int B, int N, int H) {
 
 bool mfma_supported(int B, int N, int H, int D, int w1, int w2, int dtype) {
     (void)B; (void)H; (void)w1; (void)w2; (void)N;
-    return (dtype == SA2_BF16 || dtype == SA2_F16) && (D == 32 || D == 64 || D == 128);
+    return (dtype == SA2_BF16 || dtype == SA2_F16) && (D == 16 || D == 32 || D == 64 || D == 128);
 }
 
 bool mfma_layout_ok(const Problem& p, bool backward) {
@@ -1034,13 +1053,9 @@ int launch_mfma_fwd(const Problem& p, int dtype, hipStream_t st) {
     const int nqb = (p.N + BQ - 1) / BQ;
     const int64_t total = (int64_t)nqb * p.B * p.H;
     if (total > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
-    if (dtype == SA2_F16)
-        return p.D == 128 ? launch_fwd_pair<ElemF16, 128>(p, nqb, (int)total, st)
-               : p.D == 64 ? launch_fwd_pair<ElemF16, 64>(p, nqb, (int)total, st)
-                           : launch_fwd_pair<ElemF16, 32>(p, nqb, (int)total, st);
-    return p.D == 128 ? launch_fwd_pair<ElemBF16, 128>(p, nqb, (int)total, st)
-           : p.D == 64 ? launch_fwd_pair<ElemBF16, 64>(p, nqb, (int)total, st)
-                       : launch_fwd_pair<ElemBF16, 32>(p, nqb, (int)total, st);
+    return for_mfma_width(p.D, dtype, [&](auto e, auto width, auto pad) {
+        return launch_fwd_pair<decltype(e), decltype(width)::value, decltype(pad)::value>(p, nqb, (int)total, st);
+    });
 }
 
 }  // namespace sa2
