@@ -3,6 +3,7 @@ import ctypes
 import os
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
+HOST_PATH = os.path.join(_PKG, "lib", "_sa2_torch.so")
 LIB_PATH = os.environ.get("SA2_LIBRARY", os.path.join(_PKG, "lib", "libsa2_hip.so"))
 
 # Symbols include/sa2.h declares; the ABI test checks that all of them resolve.
@@ -61,6 +62,29 @@ def load():
     lib.sa2_rowdot.argtypes = [c_void_p] * 3 + [c_int] * 4 + [i64p, c_int, c_void_p]
     _lib = lib
     return lib
+
+
+_host = None
+
+
+def host():
+    """The native host path (csrc/host/sa2_torch.cpp) over the library of load(); raises if it has not been built."""
+    global _host
+    if _host is None:
+        lib = load()
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError("_sa2_torch.so not found at %s; build it with `python -m simplical_attn_amd.build`" % HOST_PATH)
+        import importlib.util
+
+        from . import simplicial_attn
+        spec = importlib.util.spec_from_file_location("_sa2_torch", HOST_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        address = lambda f: ctypes.cast(f, ctypes.c_void_p).value
+        module.bind(address(lib.sa2_forward), address(lib.sa2_backward), address(lib.sa2_bwd_workspace_bytes),
+                    address(lib.sa2_strerror), simplicial_attn._check_inputs, simplicial_attn._check_saved, Sa2Error)
+        _host = module
+    return _host
 
 
 def check(status):

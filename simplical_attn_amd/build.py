@@ -1,9 +1,10 @@
-"""Builds the HIP library in-tree with hipcc for gfx950.
+"""Builds the HIP library and the native host path in-tree.
 
-    python -m simplical_attn_amd.build        # compile every source, link libsa2_hip.so
+    python -m simplical_attn_amd.build        # compile every source, link libsa2_hip.so and _sa2_torch.so
 
-One object per .hip file (compiled in parallel), linked into
-simplical_attn_amd/lib/libsa2_hip.so.  Cross-compiles without a GPU.
+One object per .hip file (hipcc for gfx950, compiled in parallel), linked into
+simplical_attn_amd/lib/libsa2_hip.so, and csrc/host/sa2_torch.cpp (host code against torch's C++ API) into
+simplical_attn_amd/lib/_sa2_torch.so.  Cross-compiles without a GPU.
 """
 import concurrent.futures
 import glob
@@ -16,6 +17,8 @@ ROOT = os.path.dirname(PKG)
 CSRC = os.path.join(PKG, "csrc")
 LIB_DIR = os.path.join(PKG, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libsa2_hip.so")
+HOST_SRC = os.path.join(CSRC, "host", "sa2_torch.cpp")
+HOST_PATH = os.path.join(LIB_DIR, "_sa2_torch.so")
 OBJ_DIR = os.path.join(LIB_DIR, "obj")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -40,11 +43,32 @@ def _compile(src, extra):
     return obj, err
 
 
+def _build_host():
+    """The torch extension: no device code, so the host compiler builds it."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    inc = [x for d in cpp_extension.include_paths("cuda") if os.path.isdir(d) for x in ("-isystem", d)]
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    tmp = HOST_PATH + ".tmp"
+    cmd = ["g++", "-O2", "-fPIC", "-shared", "-std=c++17", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-DTORCH_EXTENSION_NAME=_sa2_torch", "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch.compiled_with_cxx11_abi()),
+           "-I", os.path.join(ROOT, "include"), *inc, "-isystem", sysconfig.get_paths()["include"], HOST_SRC, "-o", tmp,
+           "-L", lib, "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_python"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("building the host extension failed:\n" + res.stderr)
+    os.replace(tmp, HOST_PATH)
+
+
 def build_library(verbose=True, extra_flags=()):
     os.makedirs(OBJ_DIR, exist_ok=True)
     sources = sorted(glob.glob(os.path.join(CSRC, "*.hip")))
-    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(sources))) as ex:
+    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(sources) + 1)) as ex:
+        host = ex.submit(_build_host)
         results = list(ex.map(lambda s: _compile(s, list(extra_flags)), sources))
+        host.result()
     for (obj, err), src in zip(results, sources):
         if verbose and err.strip():
             print("[%s]\n%s" % (os.path.basename(src), err), file=sys.stderr)

@@ -5,8 +5,8 @@ Same operator interface as the reference's wrapper (simplicial/triton_impl.py):
 k2_bias, v2_bias)`` (triton_impl.py:15-158) and the module
 ``TwoSimplicialAttention(head_dim, w1, w2, scale, k2_bias, v2_bias)``
 (triton_impl.py:161-186).  The kernels behind it are the HIP library's, reached
-through the C ABI in include/sa2.h; torch only owns the device buffers and the
-stream.  There is no CPU or eager fallback: tensors must live on the GPU and
+through the C ABI in include/sa2.h by the native host path (csrc/host/sa2_torch.cpp); torch only owns the device
+buffers and the stream.  There is no CPU or eager fallback: tensors must live on the GPU and
 the library must have been built.
 """
 import math
@@ -72,21 +72,8 @@ def simplicial_forward(q, k1, k2, v1, v2, w1, w2, scale=None, k2_bias=0.0, v2_bi
                        window_inclusive=True):
     """Runs the forward kernel; returns (output like q, LSE [B,H,N] fp32).
     Replaces the launch in triton_impl.py:23-51."""
-    _check_inputs(q, k1, k2, v1, v2)
-    lib = _lib.load()
-    B, N, H, D = q.shape
-    if scale is None:
-        scale = 1.0 / math.sqrt(D)
-    q, k1, k2, v1, v2 = (_rows(t) for t in (q, k1, k2, v1, v2))
-    with torch.cuda.device(q.device):
-        out = torch.empty((B, N, H, D), dtype=q.dtype, device=q.device)
-        lse = torch.empty((B, H, N), dtype=torch.float32, device=q.device)
-        _lib.check(lib.sa2_forward(
-            q.data_ptr(), k1.data_ptr(), k2.data_ptr(), v1.data_ptr(), v2.data_ptr(),
-            out.data_ptr(), lse.data_ptr(), B, N, H, D, _strides(q, k1, k2, v1, v2, out),
-            int(w1), int(w2), float(scale), float(k2_bias), float(v2_bias),
-            _DTYPES[q.dtype], int(bool(window_inclusive)), int(flags), _stream(q)))
-    return out, lse
+    return _lib.host().forward(q, k1, k2, v1, v2, int(w1), int(w2), scale, k2_bias, v2_bias, bool(window_inclusive),
+                               int(flags))
 
 
 def simplicial_backward(q, k1, k2, v1, v2, out, lse, dout, w1, w2, scale=None, k2_bias=0.0, v2_bias=0.0,
@@ -94,34 +81,11 @@ def simplicial_backward(q, k1, k2, v1, v2, out, lse, dout, w1, w2, scale=None, k
     """Runs the backward kernels; returns (dq, dk1, dk2, dv1, dv2) in the input
     dtype, None where ``needs`` is False.  Replaces triton_impl.py:61-158.
     ``out`` and ``lse`` are what simplicial_forward returned for the same inputs and arguments."""
-    _check_inputs(q, k1, k2, v1, v2)
-    _check_saved(q, out, lse, dout)
     if len(needs) != 5:
         raise ValueError("needs must have five entries (dq, dk1, dk2, dv1, dv2), got %d" % len(needs))
-    lib = _lib.load()
-    B, N, H, D = q.shape
-    if scale is None:
-        scale = 1.0 / math.sqrt(D)
-    q, k1, k2, v1, v2, out, dout = (_rows(t) for t in (q, k1, k2, v1, v2, out, dout))
-    dt = _DTYPES[q.dtype]
-    reach1 = int(w1) if window_inclusive else int(w1) - 1
-    reach2 = int(w2) if window_inclusive else int(w2) - 1
-    with torch.cuda.device(q.device):
-        grads = [torch.empty((B, N, H, D), dtype=q.dtype, device=q.device) if need else None for need in needs]
-        ws_bytes = lib.sa2_bwd_workspace_bytes(B, N, H, D, reach1, reach2, dt, int(flags))
-        workspace = torch.empty(max(int(ws_bytes), 256), dtype=torch.uint8, device=q.device)
-        like = grads[0] if grads[0] is not None else q
-        stride_src = [g if g is not None else like for g in grads]
-        ptr = lambda g: g.data_ptr() if g is not None else None
-        _lib.check(lib.sa2_backward(
-            q.data_ptr(), k1.data_ptr(), k2.data_ptr(), v1.data_ptr(), v2.data_ptr(),
-            out.data_ptr(), dout.data_ptr(), lse.data_ptr(),
-            ptr(grads[0]), ptr(grads[1]), ptr(grads[2]), ptr(grads[3]), ptr(grads[4]),
-            workspace.data_ptr(), workspace.numel(), B, N, H, D,
-            _strides(q, k1, k2, v1, v2, out, dout, *stride_src),
-            int(w1), int(w2), float(scale), float(k2_bias), float(v2_bias),
-            dt, int(bool(window_inclusive)), int(flags), _stream(q)))
-    return tuple(grads)
+    mask = sum(1 << t for t, need in enumerate(needs) if need)
+    return _lib.host().backward(q, k1, k2, v1, v2, out, lse, dout, int(w1), int(w2), scale, k2_bias, v2_bias, mask,
+                                bool(window_inclusive), int(flags))
 
 
 def simplicial_rowdot(dO, O):
@@ -227,5 +191,6 @@ class TwoSimplicialAttention(torch.nn.Module):
         self.window_inclusive = bool(window_inclusive)
 
     def forward(self, q, k1, k2, v1, v2):
-        return TwoSimplicialAttentionFunction.apply(q, k1, k2, v1, v2, self.w1, self.w2, self.scale,
-                                                    self.k2_bias, self.v2_bias, self.window_inclusive)
+        # the autograd formula of TwoSimplicialAttentionFunction, in native code
+        return _lib.host().attention(q, k1, k2, v1, v2, int(self.w1), int(self.w2), self.scale, self.k2_bias,
+                                     self.v2_bias, self.window_inclusive, _lib.FLAG_AUTO)
