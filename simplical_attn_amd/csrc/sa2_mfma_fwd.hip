@@ -94,12 +94,11 @@ struct Cfg {
     static size_t lds_bytes(int w2) { return BASE_BYTES + (side_fits(w2) ? side_bytes(w2) : 0); }
 };
 
-// SAFE = false: the fast kernel.  A weight that overflows (logits growing by more
-// than ~100 octaves along the window after the reference point was fixed) only marks
-// the block by storing NaN in its first LSE slot.
-// SAFE = true: the repair kernel, launched right after: a block that finds the mark
-// recomputes itself refreshing the reference point on every tile; every other block
-// exits at once.
+// MODE_FAST: a weight that overflows (logits growing by more than ~100 octaves along the
+// window after the reference point was fixed) is only noted; the workgroup then computes its
+// block once more as MODE_SAFE, which refreshes the reference point on every tile.  (A launch of
+// its own for the second pass cost every call 4 us at small sizes and 7.6 us at B1 H16 N8192 for
+// workgroups that found nothing to do.)
 // MODE_LEFT: the pre-pass for window sizes that leave one unit over after the rounds of
 // eight (w2 + 1 = 8n + 1).  A workgroup takes eight consecutive query blocks, one per
 // wavefront, and computes the unit delta = w2 of each while sharing one sweep of K/V tiles.
@@ -125,8 +124,7 @@ __device__ __forceinline__ void issue_v_all(uint32_t addr, lds_half_operand (&vh
 // they are read from global memory where they are needed.
 // PAD: the tensors have p.D <= D columns (see load_cols8).
 template <class E, int D, int MODE, bool SIDE, bool PAD>
-__global__ __launch_bounds__(FT) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void mfma_fwd_kernel(Problem p, int nqb, int total, int left) {
+__device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, int left, int tid) {
     typedef typename E::scalar EL;
     typedef typename E::x8 X8;
     typedef typename E::x2 X2;
@@ -145,7 +143,6 @@ void mfma_fwd_kernel(Problem p, int nqb, int total, int left) {
     uint16_t* q_s = (uint16_t*)(fin_l + BQ);    // [BQ][KS] q rows of the block
     uint16_t* k2_s = q_s + BQ * C::KS;          // [BQ + w2][KS] K' rows i0-w2 .. i0+31 (when SIDE)
 
-    const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63, ln = lane & 31, hf = lane >> 5;
 
@@ -163,10 +160,6 @@ void mfma_fwd_kernel(Problem p, int nqb, int total, int left) {
     const int i = i0 + ln;
     const int ic = i < N ? i : N - 1;
     const int i_last = (i0 + BQ - 1 < N ? i0 + BQ - 1 : N - 1);
-    if (SAFE) {
-        const float mark = p.lse[(int64_t)bh * N + i0];
-        if (mark == mark) return;                 // not NaN: the fast kernel's result stands
-    }
 
     const uint16_t* qp = (const uint16_t*)p.q.p + p.q.off(b, 0, h);
     const uint16_t* k1p = (const uint16_t*)p.k1.p + p.k1.off(b, 0, h);
@@ -709,10 +702,10 @@ void mfma_fwd_kernel(Problem p, int nqb, int total, int left) {
                     }
                 if (hf == 0) {
                     const float lam = lt > 0.f ? m + __log2f(lt) : -INFINITY;
-                    p.lse[(int64_t)bh * N + i] = any_bad ? __builtin_nanf("") : lam;
+                    p.lse[(int64_t)bh * N + i] = any_bad ? __builtin_nanf("") : lam;     // (the main kernel then takes its second pass)
                 }
             }
-            return;
+            return false;
         }
 
         if constexpr (C::NOFOLD) {
@@ -984,7 +977,27 @@ void mfma_fwd_kernel(Problem p, int nqb, int total, int left) {
             float lse;
             if (Ms > LOG2_EPS) lse = LN2 * (Ms + __log2f(L + 1e-8f * fast_exp2(-Ms)));
             else lse = LN_EPS + log1pf(L * fast_exp2(Ms - LOG2_EPS));
-            p.lse[(int64_t)bh * N + io] = (any_bad && aq == 0) ? __builtin_nanf("") : lse;
+            p.lse[(int64_t)bh * N + io] = lse;
+        }
+    }
+    return any_bad;
+}
+
+template <class E, int D, int MODE, bool SIDE, bool PAD>
+__global__ __launch_bounds__(FT) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void mfma_fwd_kernel(Problem p, int nqb, int total, int left) {
+    const bool again = fwd_block<E, D, MODE, SIDE, PAD>(p, nqb, total, left, threadIdx.x);
+    if constexpr (MODE == MODE_FAST) {
+        if (again) {                              // (uniform over the workgroup)
+            __syncthreads();
+            // (the arguments are read again from the kernel argument segment, so that none of them stays in a
+            // register for this pass while the first one runs)
+            typedef const __attribute__((address_space(4))) Problem* arg_ptr;
+            arg_ptr args = (arg_ptr)__builtin_amdgcn_kernarg_segment_ptr();
+            asm volatile("" : "+s"(args));
+            const Problem* again_p = (const Problem*)args;
+            const int* rest = (const int*)(again_p + 1);
+            fwd_block<E, D, MODE_SAFE, SIDE, PAD>(*again_p, rest[0], rest[1], 0, recompute_here(threadIdx.x));
         }
     }
 }
@@ -997,7 +1010,6 @@ int launch_fwd_kernels(const Problem& p, int nqb, int total, hipStream_t st) {
     // small that a further launch costs more than the lone round
     const int left = (p.w2 >= FW && p.w2 % FW == 0 && (p.force_prepass || total >= PREPASS_MIN_WORKGROUPS)) ? 1 : 0;
     if (!allow_full_lds((const void*)mfma_fwd_kernel<E, D, MODE_FAST, SIDE, PAD>) ||
-        !allow_full_lds((const void*)mfma_fwd_kernel<E, D, MODE_SAFE, SIDE, PAD>) ||
         !allow_full_lds((const void*)mfma_fwd_kernel<E, D, MODE_LEFT, false, PAD>))
         return SA2_ERR_LAUNCH_FAILED;
     if (left) {
@@ -1008,8 +1020,6 @@ int launch_fwd_kernels(const Problem& p, int nqb, int total, hipStream_t st) {
         if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
     }
     hipLaunchKernelGGL((mfma_fwd_kernel<E, D, MODE_FAST, SIDE, PAD>), dim3((unsigned)total), dim3(FT), lds, st, p, nqb, total, left);
-    if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
-    hipLaunchKernelGGL((mfma_fwd_kernel<E, D, MODE_SAFE, SIDE, PAD>), dim3((unsigned)total), dim3(FT), lds, st, p, nqb, total, left);
     return hipGetLastError() == hipSuccess ? SA2_OK : SA2_ERR_LAUNCH_FAILED;
 }
 
