@@ -92,8 +92,9 @@ int sa2_forward(const void* q, const void* k1, const void* k2, const void* v1, c
                 int w1, int w2, float scale, float k2_bias, float v2_bias,
                 int dtype, int window_inclusive, unsigned flags, void* hip_stream);
 
-/* Bytes of device workspace sa2_backward needs for this problem (0 is never
- * returned for a valid problem; returns 0 for an invalid one). */
+/* Bytes of device workspace sa2_backward needs for this problem, whichever of the two window
+ * conventions the call then uses with these w1 and w2 (0 is never returned for a valid problem;
+ * returns 0 for an invalid one). */
 size_t sa2_bwd_workspace_bytes(int B, int N, int H, int D, int w1, int w2, int dtype, unsigned flags);
 
 /*

@@ -124,6 +124,26 @@ KernelPath pick_path(const Problem& p, int dtype, unsigned flags, bool backward,
     return path;
 }
 
+// Bytes one call needs, for inclusive reaches w1 and w2.  Not monotone in them (the plans of the backward kernels cut
+// the work where the grid asks for it): the exported function covers both window conventions of the same numbers.
+size_t bwd_need(int B, int N, int H, int D, int w1, int w2, int dtype, unsigned flags) {
+    if (check_dims(B, N, H, D, w1, w2, dtype, 1) != SA2_OK) return 0;
+    size_t scratch = generic_bwd_scratch_bytes(B, N, H, D, w1, w2);
+    if (!(flags & SA2_FLAG_FORCE_GENERIC) && mfma_bwd_supported(B, N, H, D, reach(w1, 1, N), reach(w2, 1, N), dtype)) {
+        const size_t m = mfma_bwd_scratch_bytes(B, N, H, D, reach(w1, 1, N), reach(w2, 1, N));
+        if (m > scratch) scratch = m;
+    }
+    if (!(flags & SA2_FLAG_FORCE_GENERIC) && wide_bwd_supported(D, reach(w2, 1, N), dtype)) {
+        const size_t m = wide_bwd_scratch_bytes(B, N, H, D, reach(w1, 1, N), reach(w2, 1, N));
+        if (m > scratch) scratch = m;
+    }
+    if (!(flags & SA2_FLAG_FORCE_GENERIC) && f32_mfma_bwd_supported(D, reach(w2, 1, N), dtype)) {
+        const size_t m = f32_mfma_bwd_scratch_bytes(B, N, H, D, reach(w1, 1, N), reach(w2, 1, N));
+        if (m > scratch) scratch = m;
+    }
+    return dsum_bytes(B, N, H) + align_up(scratch, 256) + 256;
+}
+
 }  // namespace
 
 extern "C" {
@@ -189,21 +209,9 @@ int sa2_forward(const void* q, const void* k1, const void* k2, const void* v1, c
 }
 
 size_t sa2_bwd_workspace_bytes(int B, int N, int H, int D, int w1, int w2, int dtype, unsigned flags) {
-    if (check_dims(B, N, H, D, w1, w2, dtype, 1) != SA2_OK) return 0;
-    size_t scratch = generic_bwd_scratch_bytes(B, N, H, D, w1, w2);
-    if (!(flags & SA2_FLAG_FORCE_GENERIC) && mfma_bwd_supported(B, N, H, D, reach(w1, 1, N), reach(w2, 1, N), dtype)) {
-        const size_t m = mfma_bwd_scratch_bytes(B, N, H, D, reach(w1, 1, N), reach(w2, 1, N));
-        if (m > scratch) scratch = m;
-    }
-    if (!(flags & SA2_FLAG_FORCE_GENERIC) && wide_bwd_supported(D, reach(w2, 1, N), dtype)) {
-        const size_t m = wide_bwd_scratch_bytes(B, N, H, D, reach(w1, 1, N), reach(w2, 1, N));
-        if (m > scratch) scratch = m;
-    }
-    if (!(flags & SA2_FLAG_FORCE_GENERIC) && f32_mfma_bwd_supported(D, reach(w2, 1, N), dtype)) {
-        const size_t m = f32_mfma_bwd_scratch_bytes(B, N, H, D, reach(w1, 1, N), reach(w2, 1, N));
-        if (m > scratch) scratch = m;
-    }
-    return dsum_bytes(B, N, H) + align_up(scratch, 256) + 256;
+    const size_t closed = bwd_need(B, N, H, D, w1, w2, dtype, flags);
+    const size_t open = closed && w1 > 0 && w2 > 0 ? bwd_need(B, N, H, D, w1 - 1, w2 - 1, dtype, flags) : 0;
+    return closed > open ? closed : open;
 }
 
 int sa2_backward(const void* q, const void* k1, const void* k2, const void* v1, const void* v2,
@@ -218,7 +226,7 @@ int sa2_backward(const void* q, const void* k1, const void* k2, const void* v1, 
     if (rc != SA2_OK) return rc;
     if (!strides_ok(strides, SA2_BWD_TENSORS, B, N, H)) return SA2_ERR_BAD_STRIDE;
     // The half-open convention with window w has the reach of the closed one with w-1.
-    const size_t need = sa2_bwd_workspace_bytes(B, N, H, D, window_inclusive ? w1 : w1 - 1,
+    const size_t need = bwd_need(B, N, H, D, window_inclusive ? w1 : w1 - 1,
                                                 window_inclusive ? w2 : w2 - 1, dtype, flags);
     if (workspace_bytes < need || ((uintptr_t)workspace & 255u)) return SA2_ERR_WORKSPACE_TOO_SMALL;
     if (!dq && !dk1 && !dk2 && !dv1 && !dv2) return SA2_OK;
@@ -264,7 +272,7 @@ int sa2_backward_static_workspace(const void* q, const void* k1, const void* k2,
                                   int dtype, int window_inclusive, unsigned flags, void* hip_stream) {
     int rc = check_dims(B, N, H, D, w1, w2, dtype, window_inclusive);
     if (rc != SA2_OK) return rc;
-    const size_t need = sa2_bwd_workspace_bytes(B, N, H, D, window_inclusive ? w1 : w1 - 1,
+    const size_t need = bwd_need(B, N, H, D, window_inclusive ? w1 : w1 - 1,
                                                 window_inclusive ? w2 : w2 - 1, dtype, flags);
     if (need == 0 || need > (size_t)SA2_STATIC_WORKSPACE_BYTES) return SA2_ERR_STATIC_WORKSPACE;
     void* ws = static_workspace();

@@ -101,13 +101,20 @@ int launch_wide_fwd(const Problem& p, int dtype, hipStream_t st);
 int launch_wide_bwd(const Problem& p, int dtype, hipStream_t st);
 // K'-side backward kernel (dQ, dK', dV') that keeps its partial sums on chip (K' windows too wide for
 // that are cut into segments of deltas, one workgroup each)
-size_t kp_scratch_bytes(int B, int N, int H, int D, int w2);
-int launch_mfma_bwd_kp(const Problem& p, int dtype, hipStream_t st);
+size_t kp_scratch_bytes(int B, int N, int H, int D, int w1, int w2);
+// Where the two kernels leave fp32 partial sums, rows of the kernel's width: the dQ partials of (K' block, segment)
+// workgroups, [dV' | dK'][kp_n][B*H][N][width] of a segmented K'-side launch and [dK | dV][kv_n][B*H][N][width] of a split
+// K-side launch.  NULL: that kernel wrote its results itself (dQ: not wanted).
+struct BwdSums {
+    const float *dq, *kp, *kv;
+    int nkb, nseg, segw, kp_n, kv_n;
+};
+int launch_mfma_bwd_kp(const Problem& p, int dtype, hipStream_t st, BwdSums* sums);
 // K-side backward kernel (dK, dV) with paired wavefronts; for small grids it splits a key block's
 // query blocks over several workgroups, whose fp32 partial sums lie in the workspace behind the
 // K'-side part (kp_side_scratch_bytes); K' windows too wide for its LDS rows are walked in segments
 size_t kv_split_scratch_bytes(int B, int N, int H, int D, int w1, int w2);
-size_t kp_side_scratch_bytes(int B, int N, int H, int D, int w2);
-int launch_mfma_bwd_kv(const Problem& p, int dtype, hipStream_t st);
+size_t kp_side_scratch_bytes(int B, int N, int H, int D, int w1, int w2);
+int launch_mfma_bwd_kv(const Problem& p, int dtype, hipStream_t st, BwdSums* sums);
 
 }  // namespace sa2

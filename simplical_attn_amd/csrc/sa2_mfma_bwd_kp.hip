@@ -10,11 +10,11 @@
 //
 // dK' and dV' are aligned with the unit's rows, so they accumulate in registers over the
 // deltas a wavefront handles; dQ is shifted by delta and goes through an fp32 accumulator
-// in LDS (rows k0 .. k0+31+w2), written once per workgroup as a partial that a small
-// kernel adds up (a query gets partials from at most 2 + w2/32 workgroups, summed in a
-// fixed order: bitwise reproducible).  A K' window too wide for that accumulator is cut into
-// segments of deltas, one workgroup per (K' block, segment); their fp32 partial dK' and dV' are
-// added by kp_sum_kernel in segment order.
+// in LDS (rows k0 .. k0+31+w2), written once per workgroup as a partial that bwd_sum_kernel
+// adds up (a query gets partials from at most 2 + w2/32 workgroups, summed in a
+// fixed order: bitwise reproducible).  A K' window too wide for that accumulator, or one whose K' blocks alone leave the
+// chip idle (kp_plan), is cut into segments of deltas, one workgroup per (K' block, segment); their fp32
+// partial dK' and dV' are added by bwd_sum_kernel in segment order.
 //
 // Eight wavefronts, two per SIMD, form four pairs that each hold one unit per round (two
 // consecutive deltas at head_dim 32 and 64, where the registers allow it: every K and V operand
@@ -90,9 +90,9 @@ struct KpCfg {
 // U = 2 (head_dim 32 and 64, where the registers allow it): a pair holds two consecutive deltas per round, so
 // that every K and V operand read, every tile request and every step barrier serves twice the MFMAs.
 //
-// SEG = true: a K' window too wide for the dQ accumulator in LDS is cut into nseg runs of segw deltas, one
-// workgroup per (K' block, segment); a kernel of its own so that the common case carries none of it.  Each writes its own dQ partial (rows k0 + seg*segw ..) and, when
-// nseg > 1, fp32 partial dK' and dV' to `kpart` ([dV' | dK'][nseg][B*H][N][D]) for kp_sum_kernel.
+// SEG = true: the K' window is cut into nseg runs of segw deltas, one workgroup per (K' block, segment); a kernel of its
+// own so that the common case carries none of it.  Each writes its own dQ partial (rows k0 + seg*segw ..) and, when
+// nseg > 1, fp32 partial dK' and dV' to `kpart` ([dV' | dK'][nseg][B*H][N][D]) for bwd_sum_kernel.
 //
 // PAD: the tensors have p.D <= D columns (see load_cols8).
 template <class E, int D, bool RAW, bool LEFT, int U, bool SEG, bool PAD>
@@ -104,7 +104,7 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
     constexpr bool raw = RAW;
     static_assert(!(RAW && LEFT), "the pre-pass keeps no row copies in LDS");
     static_assert(!LEFT || U == 1, "the pre-pass holds one unit per pair");
-    static_assert(!SEG || (!LEFT && !RAW), "segments: main kernel, rows from global memory");
+    static_assert(!SEG || !LEFT, "segments: main kernel only");
     using C = KpCfg<D, U>;
     constexpr int UPR = NPAIR * U;                            // units per round
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -817,96 +817,58 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
     }
 }
 
-// dQ[i] = sum of the partials of the K' blocks that reach query i, in block order.
-template <class E, int D>
-__global__ __launch_bounds__(256) void mfma_bwd_dq_sum_kernel(Problem p, const float* __restrict__ dq_part, int nkb,
-                                                             int64_t items, int nseg, int segw) {
-    typedef typename E::scalar EL;
-    constexpr int CH = D / 8;
-    const int64_t it = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (it >= items) return;
-    const int c0 = (int)(it % CH) * 8;
-    if (c0 >= p.D) return;                   // (the partials' rows have the kernel's width)
-    const int64_t row = it / CH;
-    const int N = p.N, RQ = BQ + p.w2;       // queries a K' block reaches
-    const int RS = BQ + segw - 1;            // rows of one segment's partial
-    const int i = (int)(row % N);
-    const int bh = (int)(row / N);
-    const int b = bh / p.H, h = bh - b * p.H;
-    const int kb_hi = i / BQ;
-    int kb_lo = (i - RQ + BQ) / BQ;              // smallest kb with i - 32*kb <= RQ-1
-    kb_lo = (i - RQ + 1 <= 0) ? 0 : kb_lo;
-    float acc[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) acc[c] = 0.f;
-    if (nseg == 1) {
-        for (int kb = kb_lo; kb <= kb_hi; ++kb) {
-            const float* src = dq_part + (((int64_t)bh * nkb + kb) * RQ + (i - kb * BQ)) * D + c0;
-            const float4 a = *(const float4*)src, c4 = *(const float4*)(src + 4);
-            acc[0] += a.x; acc[1] += a.y; acc[2] += a.z; acc[3] += a.w;
-            acc[4] += c4.x; acc[5] += c4.y; acc[6] += c4.z; acc[7] += c4.w;
-        }
-        kb_lo = kb_hi + 1;
-    }
-    for (int kb = kb_lo; kb <= kb_hi; ++kb) {
-        const int rel = i - kb * BQ;             // row of the block's reach; segment s holds rel - s*segw in [0, RS)
-        const int s_hi = rel / segw < nseg - 1 ? rel / segw : nseg - 1;
-        const int s_lo = rel - RS + 1 <= 0 ? 0 : (rel - RS + segw) / segw;
-        for (int sg = s_lo; sg <= s_hi; ++sg) {
-            const float* src = dq_part + ((((int64_t)bh * nkb + kb) * nseg + sg) * RS + (rel - sg * segw)) * D + c0;
-            const float4 a = *(const float4*)src, c4 = *(const float4*)(src + 4);
-            acc[0] += a.x; acc[1] += a.y; acc[2] += a.z; acc[3] += a.w;
-            acc[4] += c4.x; acc[5] += c4.y; acc[6] += c4.z; acc[7] += c4.w;
-        }
-    }
-    union { EL hh[8]; uint4 u; } o;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) o.hh[c] = (EL)acc[c];
-    *(uint4*)((uint16_t*)p.dq.p + p.dq.off(b, i, h) + c0) = o.u;
-}
-
-// dK' and dV' from the fp32 partial sums of a segmented launch, segments added in their order
-template <class E>
-__global__ __launch_bounds__(256) void kp_sum_kernel(Problem p, int D, int nseg, const float* __restrict__ kpart, int64_t chunks) {
-    const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (c >= chunks) return;
-    const int col = (int)(c % (D / 4));
-    if (col * 4 >= p.D) return;
-    const int64_t rowid = c / (D / 4);
-    const int k = (int)(rowid % p.N);
-    const int bh = (int)(rowid / p.N);
-    const int b = bh / p.H, h = bh - b * p.H;
-    const int64_t BH = (int64_t)p.B * p.H;
-#pragma unroll
-    for (int which = 0; which < 2; ++which) {
-        const Tensor& t = which ? p.dk2 : p.dv2;
-        if (!t.p) continue;
-        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int sg = 0; sg < nseg; ++sg) {
-            const float4 y = *(const float4*)(kpart + (((which * (int64_t)nseg + sg) * BH + bh) * p.N + k) * D + col * 4);
-            acc.x += y.x; acc.y += y.y; acc.z += y.z; acc.w += y.w;
-        }
-        *(uint2*)((uint16_t*)t.p + t.off(b, k, h) + col * 4) = make_uint2(E::pack(acc.x, acc.y), E::pack(acc.z, acc.w));
-    }
-}
-
-// Geometry of a launch: deltas per segment and number of segments (one while the dQ accumulator of the
-// whole K' window fits LDS).  A pair holds two deltas per round at head_dim 32 and 64, one at 128.
+// Geometry of a launch: deltas per segment and number of segments.  A pair holds two deltas per round at head_dim 32
+// and 64, one at 128; a segment is a whole number of rounds.
 struct KpPlan {
     int segw, nseg;
 };
 template <int D>
 constexpr int kp_units() { return D <= 64 ? 2 : 1; }
-template <int D>
-KpPlan kp_plan_of(int w2) {
-    using C = KpCfg<D, kp_units<D>()>;
-    if (C::fits(w2)) return KpPlan{w2 + 1, 1};
-    constexpr int UPR = NPAIR * kp_units<D>();
-    int segw = UPR;
-    while (C::fits(segw + UPR - 1)) segw += UPR;           // whole rounds per segment
-    return KpPlan{segw, (w2 + segw) / segw};
+
+size_t kp_dq_part_bytes(int B, int N, int H, int D, const KpPlan& pl);
+size_t kp_part_bytes(int B, int N, int H, int D, const KpPlan& pl) {
+    return pl.nseg > 1 ? (size_t)2 * pl.nseg * B * H * (size_t)N * D * sizeof(float) : 0;
 }
-KpPlan kp_plan(int D, int w2) { return D == 128 ? kp_plan_of<128>(w2) : D == 64 ? kp_plan_of<64>(w2) : kp_plan_of<32>(w2); }
+
+// One workgroup fills a CU.  A segment costs its rounds (each the tiles of the K window plus the work between two
+// sweeps, about two tiles' time) and about six tiles' time of prologue and epilogue; its partial sums are written once
+// and read once (5 MB take about a tile's time).  The plan is the cut of the K' window for which waves of workgroups x
+// cost of one is least, among those whose dQ accumulator fits LDS; grids of four waves and more are cut only where
+// LDS asks for it (the tail of the last wave is below what a cut costs), and partial sums never push a problem over
+// SA2_STATIC_WORKSPACE_BYTES.
+// Measured on the K'-side kernel: B2 H4 N512 D64 w 256/256 (128 blocks) 625 -> 330 us with two segments,
+// B2 H4 N256 D64 w 32/32 (64 blocks) 40 -> 21 us with three.
+template <int D>
+KpPlan kp_plan_of(int B, int N, int H, int w1, int w2) {
+    using C = KpCfg<D, kp_units<D>()>;
+    constexpr int UPR = NPAIR * kp_units<D>(), CUS = 256;
+    KpPlan lds{w2 + 1, 1};
+    if (!C::fits(w2)) {
+        int segw = UPR;
+        while (C::fits(segw + UPR - 1)) segw += UPR;
+        lds = KpPlan{segw, (w2 + segw) / segw};
+    }
+    const int64_t base = (int64_t)B * H * ((N + BQ - 1) / BQ);
+    if (base * lds.nseg >= 4 * CUS) return lds;
+    const int rounds = (w2 + UPR) / UPR, tiles = ((w1 < N ? w1 : N) + BQ + UPR + TJ - 1) / TJ + 2;
+    KpPlan best = lds;
+    double least = 0;
+    for (int per = (lds.segw + UPR - 1) / UPR; per >= 1; --per) {                // rounds per segment
+        const int nseg = (rounds + per - 1) / per;
+        const KpPlan pl = nseg == 1 ? lds : KpPlan{per * UPR, nseg};
+        const double bytes = 2.0 * (double)(kp_dq_part_bytes(B, N, H, D, pl) + kp_part_bytes(B, N, H, D, pl));
+        const double cost = (double)((base * pl.nseg + CUS - 1) / CUS) * (per * tiles + 6) + bytes / 5e6;
+        if (per == (lds.segw + UPR - 1) / UPR) least = cost;
+        else if (cost < 0.95 * least && bytes / 2 <= (double)(SA2_STATIC_WORKSPACE_BYTES / 4)) {
+            least = cost;
+            best = pl;
+        }
+    }
+    return best;
+}
+KpPlan kp_plan(int B, int N, int H, int D, int w1, int w2) {
+    return D == 128 ? kp_plan_of<128>(B, N, H, w1, w2) : D == 64 ? kp_plan_of<64>(B, N, H, w1, w2) : kp_plan_of<32>(B, N, H, w1, w2);
+}
 
 size_t kp_dq_part_bytes(int B, int N, int H, int D, const KpPlan& pl) {
     const size_t nkb = (size_t)(N + BQ - 1) / BQ;
@@ -914,16 +876,16 @@ size_t kp_dq_part_bytes(int B, int N, int H, int D, const KpPlan& pl) {
 }
 
 template <class E, int D, bool PAD>
-int launch_kp(const Problem& p, hipStream_t st) {
+int launch_kp(const Problem& p, hipStream_t st, BwdSums* sums) {
     constexpr int U = kp_units<D>();
     using C = KpCfg<D, U>;
-    const KpPlan pl = kp_plan(D, p.w2);
+    const KpPlan pl = kp_plan(p.B, p.N, p.H, D, p.w1, p.w2);
     const int nkb = (p.N + BQ - 1) / BQ;
     const int64_t total = (int64_t)nkb * p.B * p.H * pl.nseg;
     if (total > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
-    if ((p.dq.p || pl.nseg > 1) && p.scratch_bytes < kp_scratch_bytes(p.B, p.N, p.H, D, p.w2)) return SA2_ERR_WORKSPACE_TOO_SMALL;
+    if ((p.dq.p || pl.nseg > 1) && p.scratch_bytes < kp_scratch_bytes(p.B, p.N, p.H, D, p.w1, p.w2)) return SA2_ERR_WORKSPACE_TOO_SMALL;
     const int w2s = pl.segw - 1;
-    const bool raw = pl.nseg == 1 && C::raw_fits(w2s);
+    const bool raw = C::raw_fits(w2s);
     const size_t lds = C::lds_bytes(w2s, raw);
     float* part = (float*)p.scratch;
     float* kpart = (float*)((char*)p.scratch + kp_dq_part_bytes(p.B, p.N, p.H, D, pl));
@@ -939,43 +901,35 @@ int launch_kp(const Problem& p, hipStream_t st) {
                            (int)total_left, part, 0, 1, p.w2 + 1, (float*)nullptr);
         if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
     }
-    if (pl.nseg > 1) {
-        if (!allow_full_lds((const void*)mfma_bwd_kp_kernel<E, D, false, false, U, true, PAD>)) return SA2_ERR_LAUNCH_FAILED;
-        hipLaunchKernelGGL((mfma_bwd_kp_kernel<E, D, false, false, U, true, PAD>), dim3((unsigned)total), dim3(KT), lds, st, p, nkb,
-                           (int)total, part, left, pl.nseg, pl.segw, kpart);
-    } else {
-        const void* fn = raw ? (const void*)mfma_bwd_kp_kernel<E, D, true, false, U, false, PAD> : (const void*)mfma_bwd_kp_kernel<E, D, false, false, U, false, PAD>;
-        if (!allow_full_lds(fn)) return SA2_ERR_LAUNCH_FAILED;
-        if (raw) hipLaunchKernelGGL((mfma_bwd_kp_kernel<E, D, true, false, U, false, PAD>), dim3((unsigned)total), dim3(KT), lds, st, p, nkb, (int)total, part, left, 1, p.w2 + 1, kpart);
-        else hipLaunchKernelGGL((mfma_bwd_kp_kernel<E, D, false, false, U, false, PAD>), dim3((unsigned)total), dim3(KT), lds, st, p, nkb, (int)total, part, left, 1, p.w2 + 1, kpart);
-    }
-    if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
-    if (p.dq.p) {
-        const int64_t items = (int64_t)p.B * p.H * p.N * (D / 8);
-        hipLaunchKernelGGL((mfma_bwd_dq_sum_kernel<E, D>), dim3((unsigned)((items + 255) / 256)), dim3(256), 0, st, p, part,
-                           nkb, items, pl.nseg, pl.segw);
-        if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
-    }
-    if (pl.nseg > 1 && (p.dk2.p || p.dv2.p)) {
-        const int64_t chunks = (int64_t)p.B * p.H * p.N * (D / 4);
-        hipLaunchKernelGGL((kp_sum_kernel<E>), dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, p, D, pl.nseg, kpart, chunks);
-        if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
-    }
+    auto go = [&](auto kernel) {
+        if (!allow_full_lds((const void*)kernel)) return false;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(KT), lds, st, p, nkb, (int)total, part, left, pl.nseg, pl.segw, kpart);
+        return hipGetLastError() == hipSuccess;
+    };
+    const bool ok = pl.nseg > 1 ? (raw ? go(mfma_bwd_kp_kernel<E, D, true, false, U, true, PAD>) : go(mfma_bwd_kp_kernel<E, D, false, false, U, true, PAD>))
+                                : (raw ? go(mfma_bwd_kp_kernel<E, D, true, false, U, false, PAD>) : go(mfma_bwd_kp_kernel<E, D, false, false, U, false, PAD>));
+    if (!ok) return SA2_ERR_LAUNCH_FAILED;
+    sums->dq = p.dq.p ? part : nullptr;
+    sums->nkb = nkb;
+    sums->nseg = pl.nseg;
+    sums->segw = pl.segw;
+    sums->kp = pl.nseg > 1 ? kpart : nullptr;
+    sums->kp_n = pl.nseg;
     return SA2_OK;
 }
 
 }  // namespace
 
 // workspace of the K'-side kernel: the dQ partials, then (segmented launches) the dK' and dV' partials
-size_t kp_scratch_bytes(int B, int N, int H, int head_dim, int w2) {
+size_t kp_scratch_bytes(int B, int N, int H, int head_dim, int w1, int w2) {
     const int D = mfma_width(head_dim);
-    const KpPlan pl = kp_plan(D, w2);
-    return kp_dq_part_bytes(B, N, H, D, pl) + (pl.nseg > 1 ? (size_t)2 * pl.nseg * B * H * (size_t)N * D * sizeof(float) : 0);
+    const KpPlan pl = kp_plan(B, N, H, D, w1, w2);
+    return kp_dq_part_bytes(B, N, H, D, pl) + kp_part_bytes(B, N, H, D, pl);
 }
 
-int launch_mfma_bwd_kp(const Problem& p, int dtype, hipStream_t st) {
+int launch_mfma_bwd_kp(const Problem& p, int dtype, hipStream_t st, BwdSums* sums) {
     return for_mfma_width(p.D, dtype, [&](auto e, auto width, auto pad) {
-        return launch_kp<decltype(e), decltype(width)::value, decltype(pad)::value>(p, st);
+        return launch_kp<decltype(e), decltype(width)::value, decltype(pad)::value>(p, st, sums);
     });
 }
 

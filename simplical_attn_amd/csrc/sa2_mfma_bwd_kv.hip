@@ -17,7 +17,7 @@
 //
 // Small grids (fewer workgroups than the chip holds) split a key block's stream of units over up to
 // sixteen workgroups (shares of whole units, at least eight each); each writes its fp32 partial dK and
-// dV to the workspace and kv_sum_kernel adds the partials in split order.
+// dV to the workspace and bwd_sum_kernel adds the partials in split order.
 #include <type_traits>
 
 #include "sa2_mfma_common.h"
@@ -477,32 +477,6 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __
     }
 }
 
-// dK and dV from the partial sums of a split launch, shares added in their order
-// (the partials' rows have the kernel's width D, of which p.D columns are stored)
-template <class E>
-__global__ __launch_bounds__(256) void kv_sum_kernel(Problem p, int D, int nsplit, const float* __restrict__ part, int64_t chunks) {
-    const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (c >= chunks) return;
-    const int col = (int)(c % (D / 4));
-    if (col * 4 >= p.D) return;
-    const int64_t rowid = c / (D / 4);
-    const int j = (int)(rowid % p.N);
-    const int bh = (int)(rowid / p.N);
-    const int b = bh / p.H, h = bh - b * p.H;
-    const int64_t BH = (int64_t)p.B * p.H;
-#pragma unroll
-    for (int which = 0; which < 2; ++which) {
-        const Tensor& t = which ? p.dv1 : p.dk1;
-        if (!t.p) continue;
-        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int s = 0; s < nsplit; ++s) {
-            const float4 y = *(const float4*)(part + (((which * (int64_t)nsplit + s) * BH + bh) * p.N + j) * D + col * 4);
-            acc.x += y.x; acc.y += y.y; acc.z += y.z; acc.w += y.w;
-        }
-        *(uint2*)((uint16_t*)t.p + t.off(b, j, h) + col * 4) = make_uint2(E::pack(acc.x, acc.y), E::pack(acc.z, acc.w));
-    }
-}
-
 // Geometry of a launch: 32-row K blocks per wavefront pair, and the number of shares a key block's
 // stream of units is split into.  Both depend on the problem's sizes only.
 struct KvPlan {
@@ -526,7 +500,7 @@ KvPlan kv_plan(int B, int N, int H, int D, int w1, int w2) {
 }
 
 template <class E, int D, int KB, bool PAD>
-int launch_kv_geometry(const Problem& p, int nsplit, hipStream_t st) {
+int launch_kv_geometry(const Problem& p, int nsplit, hipStream_t st, BwdSums* sums) {
     using C = KvCfg<D, KB>;
     const int njb = (p.N + C::VJ - 1) / C::VJ;
     const int64_t total = (int64_t)njb * p.B * p.H * nsplit;
@@ -537,7 +511,7 @@ int launch_kv_geometry(const Problem& p, int nsplit, hipStream_t st) {
     // the partial sums of a split launch lie behind the K'-side kernel's part of the workspace
     float* part = nullptr;
     if (nsplit > 1) {
-        const size_t off = kp_side_scratch_bytes(p.B, p.N, p.H, D, p.w2);
+        const size_t off = kp_side_scratch_bytes(p.B, p.N, p.H, D, p.w1, p.w2);
         if (p.scratch_bytes < off + kv_split_scratch_bytes(p.B, p.N, p.H, D, p.w1, p.w2)) return SA2_ERR_WORKSPACE_TOO_SMALL;
         part = (float*)((char*)p.scratch + off);
     }
@@ -559,21 +533,18 @@ int launch_kv_geometry(const Problem& p, int nsplit, hipStream_t st) {
                     : go(mfma_bwd_kv_kernel<E, D, false, KB, false, false, PAD>);
     if (!ok) return SA2_ERR_LAUNCH_FAILED;
     if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
-    if (nsplit > 1) {
-        const int64_t chunks = (int64_t)p.B * p.H * p.N * (D / 4);
-        hipLaunchKernelGGL((kv_sum_kernel<E>), dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, p, D, nsplit, part, chunks);
-        if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
-    }
+    sums->kv = part;
+    sums->kv_n = nsplit;
     return SA2_OK;
 }
 
 template <class E, int D, bool PAD>
-int launch_kv(const Problem& p, hipStream_t st) {
+int launch_kv(const Problem& p, hipStream_t st, BwdSums* sums) {
     const KvPlan pl = kv_plan(p.B, p.N, p.H, D, p.w1, p.w2);
     if constexpr (D == 64) {
-        if (pl.kb == 2) return launch_kv_geometry<E, D, 2, PAD>(p, pl.nsplit, st);
+        if (pl.kb == 2) return launch_kv_geometry<E, D, 2, PAD>(p, pl.nsplit, st, sums);
     }
-    return launch_kv_geometry<E, D, 1, PAD>(p, pl.nsplit, st);
+    return launch_kv_geometry<E, D, 1, PAD>(p, pl.nsplit, st, sums);
 }
 
 }  // namespace
@@ -584,9 +555,9 @@ size_t kv_split_scratch_bytes(int B, int N, int H, int head_dim, int w1, int w2)
     return pl.nsplit > 1 ? (size_t)2 * pl.nsplit * B * H * (size_t)N * D * sizeof(float) : 0;
 }
 
-int launch_mfma_bwd_kv(const Problem& p, int dtype, hipStream_t st) {
+int launch_mfma_bwd_kv(const Problem& p, int dtype, hipStream_t st, BwdSums* sums) {
     return for_mfma_width(p.D, dtype, [&](auto e, auto width, auto pad) {
-        return launch_kv<decltype(e), decltype(width)::value, decltype(pad)::value>(p, st);
+        return launch_kv<decltype(e), decltype(width)::value, decltype(pad)::value>(p, st, sums);
     });
 }
 
