@@ -72,6 +72,39 @@ __device__ __forceinline__ float lse_with_eps(float m, float l) {
 constexpr int LDS_BYTES_PER_CU = 160 * 1024;
 bool allow_full_lds(const void* kernel);
 
+// How a K'-side launch cuts the K' window: segw deltas per segment, nseg segments, one workgroup per (K' block, segment).
+struct KpPlan {
+    int segw, nseg;
+};
+// One workgroup fills a CU.  A segment costs its rounds of `upr` deltas (each the tiles of the K window plus the work
+// between two sweeps, about two tiles' time) and about six tiles' time of prologue and epilogue; its partial sums
+// (bytes(plan)) are written once and read once (5 MB take about a tile's time).  The plan is the cut for which waves of
+// workgroups x cost of one is least, among segments of at most `most` deltas (what LDS holds); grids of four waves and
+// more are cut only where LDS asks for it (the tail of the last wave is below what a cut costs), and a cut for the
+// grid's sake never takes more than a quarter of SA2_STATIC_WORKSPACE_BYTES.
+// Measured on the 16-bit kernel: B2 H4 N512 D64 w 256/256 (128 blocks) 625 -> 349 us with two segments,
+// B2 H4 N256 D64 w 32/32 (64 blocks) 40 -> 23 us with three.
+template <class F>
+KpPlan plan_segments(int B, int N, int H, int w1, int w2, int upr, int most, F&& bytes) {
+    constexpr int CUS = 256, ROWS = 32;
+    const int64_t base = (int64_t)B * H * ((N + ROWS - 1) / ROWS);
+    KpPlan best = most > w2 ? KpPlan{w2 + 1, 1} : KpPlan{most, (w2 + most) / most};
+    if (base * best.nseg >= 4 * CUS) return best;
+    const int rounds = (w2 + upr) / upr, tiles = ((w1 < N ? w1 : N) + 2 * ROWS + upr - 1) / ROWS + 2, longest = (best.segw + upr - 1) / upr;
+    double least = 0;
+    for (int per = longest; per >= 1; --per) {                                   // rounds per segment
+        const KpPlan pl = per == longest ? best : KpPlan{per * upr, (rounds + per - 1) / per};
+        const double part = (double)bytes(pl);
+        const double cost = (double)((base * pl.nseg + CUS - 1) / CUS) * (per * tiles + 6) + 2 * part / 5e6;
+        if (per == longest) least = cost;
+        else if (cost < 0.95 * least && part <= (double)(SA2_STATIC_WORKSPACE_BYTES / 4)) {
+            least = cost;
+            best = pl;
+        }
+    }
+    return best;
+}
+
 // ---- launchers (each returns a sa2_status) ----------------------------------
 int launch_rowdot(const Tensor& out, const Tensor& dout, float* dsum, int B, int N, int H, int D,
                   int dtype, hipStream_t st);
@@ -90,7 +123,7 @@ size_t mfma_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2);
 bool f32_mfma_supported(int D, int dtype);
 bool f32_mfma_bwd_supported(int D, int w2, int dtype);
 bool f32_mfma_layout_ok(const Problem& p, int dtype, bool backward);
-size_t f32_mfma_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2);
+size_t f32_mfma_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2, int dtype);
 int launch_f32_mfma_fwd(const Problem& p, int dtype, hipStream_t st);
 int launch_f32_mfma_bwd(const Problem& p, int dtype, hipStream_t st);
 // 16-bit tensors with head_dim 256 on the 16-bit MFMA (rows 16-byte aligned)
@@ -109,6 +142,7 @@ struct BwdSums {
     const float *dq, *kp, *kv;
     int nkb, nseg, segw, kp_n, kv_n;
 };
+int launch_bwd_sums(const Problem& p, const BwdSums& sums, int width, int dtype, hipStream_t st);
 int launch_mfma_bwd_kp(const Problem& p, int dtype, hipStream_t st, BwdSums* sums);
 // K-side backward kernel (dK, dV) with paired wavefronts; for small grids it splits a key block's
 // query blocks over several workgroups, whose fp32 partial sums lie in the workspace behind the

@@ -13,6 +13,7 @@
 namespace sa2 {
 namespace {
 
+// E: the gradients' element type (float or a 16-bit one).
 // The gradients that the two kernels left as fp32 partial sums, one launch for all of them (grid dimension y).
 // Four columns of one row per thread; what bounds it is reading the partials once.  (A kernel per kind, as before, cost
 // three launches of 5-10 us each at small sizes, most of it latency: the partials of a row were read one after the
@@ -59,7 +60,8 @@ __global__ __launch_bounds__(256) void bwd_sum_kernel(Problem p, BwdSums s, int 
     }
     const Tensor& t = kind == SUM_DQ ? p.dq : kind == SUM_DK1 ? p.dk1 : kind == SUM_DV1 ? p.dv1 : kind == SUM_DV2 ? p.dv2 : p.dk2;
     const int b = bh / p.H, h = bh - b * p.H;
-    *(uint2*)((uint16_t*)t.p + t.off(b, i, h) + col) = make_uint2(E::pack(acc.x, acc.y), E::pack(acc.z, acc.w));
+    if constexpr (std::is_same<E, float>::value) *(float4*)((float*)t.p + t.off(b, i, h) + col) = acc;
+    else *(uint2*)((uint16_t*)t.p + t.off(b, i, h) + col) = make_uint2(E::pack(acc.x, acc.y), E::pack(acc.z, acc.w));
 }
 
 }  // namespace
@@ -78,16 +80,7 @@ size_t mfma_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2) {
     return kp_side_scratch_bytes(B, N, H, D, w1, w2) + kv_split_scratch_bytes(B, N, H, D, w1, w2);
 }
 
-int launch_mfma_bwd(const Problem& p, int dtype, hipStream_t st) {
-    int rc = launch_rowdot(p.out, p.dout, p.dsum, p.B, p.N, p.H, p.D, dtype, st);
-    if (rc != SA2_OK) return rc;
-    BwdSums sums = {};
-    if (p.dq.p || p.dk2.p || p.dv2.p) {
-        rc = launch_mfma_bwd_kp(p, dtype, st, &sums);
-        if (rc != SA2_OK) return rc;
-    }
-    if (p.dk1.p || p.dv1.p) rc = launch_mfma_bwd_kv(p, dtype, st, &sums);
-    if (rc != SA2_OK) return rc;
+int launch_bwd_sums(const Problem& p, const BwdSums& sums, int width, int dtype, hipStream_t st) {
     unsigned kinds = 0;
     int n = 0;
     auto want = [&](int kind, const float* part, const Tensor& t) {
@@ -99,12 +92,25 @@ int launch_mfma_bwd(const Problem& p, int dtype, hipStream_t st) {
     want(SUM_DV2, sums.kp, p.dv2);
     want(SUM_DK2, sums.kp, p.dk2);
     if (n == 0) return SA2_OK;
-    const int D = mfma_width(p.D);
-    const int64_t items = (int64_t)p.B * p.H * p.N * (D / 4);
+    const int64_t items = (int64_t)p.B * p.H * p.N * (width / 4);
     const dim3 grid((unsigned)((items + 255) / 256), (unsigned)n);
-    if (dtype == SA2_F16) hipLaunchKernelGGL((bwd_sum_kernel<ElemF16>), grid, dim3(256), 0, st, p, sums, D, kinds, items);
-    else hipLaunchKernelGGL((bwd_sum_kernel<ElemBF16>), grid, dim3(256), 0, st, p, sums, D, kinds, items);
+    if (dtype == SA2_F32) hipLaunchKernelGGL((bwd_sum_kernel<float>), grid, dim3(256), 0, st, p, sums, width, kinds, items);
+    else if (dtype == SA2_F16) hipLaunchKernelGGL((bwd_sum_kernel<ElemF16>), grid, dim3(256), 0, st, p, sums, width, kinds, items);
+    else hipLaunchKernelGGL((bwd_sum_kernel<ElemBF16>), grid, dim3(256), 0, st, p, sums, width, kinds, items);
     return hipGetLastError() == hipSuccess ? SA2_OK : SA2_ERR_LAUNCH_FAILED;
+}
+
+int launch_mfma_bwd(const Problem& p, int dtype, hipStream_t st) {
+    int rc = launch_rowdot(p.out, p.dout, p.dsum, p.B, p.N, p.H, p.D, dtype, st);
+    if (rc != SA2_OK) return rc;
+    BwdSums sums = {};
+    if (p.dq.p || p.dk2.p || p.dv2.p) {
+        rc = launch_mfma_bwd_kp(p, dtype, st, &sums);
+        if (rc != SA2_OK) return rc;
+    }
+    if (p.dk1.p || p.dv1.p) rc = launch_mfma_bwd_kv(p, dtype, st, &sums);
+    if (rc != SA2_OK) return rc;
+    return launch_bwd_sums(p, sums, mfma_width(p.D), dtype, st);
 }
 
 }  // namespace sa2

@@ -13,7 +13,7 @@
 // in LDS (rows k0 .. k0+31+w2), written once per workgroup as a partial that bwd_sum_kernel
 // adds up (a query gets partials from at most 2 + w2/32 workgroups, summed in a
 // fixed order: bitwise reproducible).  A K' window too wide for that accumulator, or one whose K' blocks alone leave the
-// chip idle (kp_plan), is cut into segments of deltas, one workgroup per (K' block, segment); their fp32
+// chip idle (plan_segments), is cut into segments of deltas, one workgroup per (K' block, segment); their fp32
 // partial dK' and dV' are added by bwd_sum_kernel in segment order.
 //
 // Eight wavefronts, two per SIMD, form four pairs that each hold one unit per round (two
@@ -817,62 +817,31 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
     }
 }
 
-// Geometry of a launch: deltas per segment and number of segments.  A pair holds two deltas per round at head_dim 32
-// and 64, one at 128; a segment is a whole number of rounds.
-struct KpPlan {
-    int segw, nseg;
-};
+// A pair holds two deltas per round at head_dim 32 and 64, one at 128; a segment is a whole number of rounds.
 template <int D>
 constexpr int kp_units() { return D <= 64 ? 2 : 1; }
-
-size_t kp_dq_part_bytes(int B, int N, int H, int D, const KpPlan& pl);
-size_t kp_part_bytes(int B, int N, int H, int D, const KpPlan& pl) {
-    return pl.nseg > 1 ? (size_t)2 * pl.nseg * B * H * (size_t)N * D * sizeof(float) : 0;
-}
-
-// One workgroup fills a CU.  A segment costs its rounds (each the tiles of the K window plus the work between two
-// sweeps, about two tiles' time) and about six tiles' time of prologue and epilogue; its partial sums are written once
-// and read once (5 MB take about a tile's time).  The plan is the cut of the K' window for which waves of workgroups x
-// cost of one is least, among those whose dQ accumulator fits LDS; grids of four waves and more are cut only where
-// LDS asks for it (the tail of the last wave is below what a cut costs), and partial sums never push a problem over
-// SA2_STATIC_WORKSPACE_BYTES.
-// Measured on the K'-side kernel: B2 H4 N512 D64 w 256/256 (128 blocks) 625 -> 330 us with two segments,
-// B2 H4 N256 D64 w 32/32 (64 blocks) 40 -> 21 us with three.
-template <int D>
-KpPlan kp_plan_of(int B, int N, int H, int w1, int w2) {
-    using C = KpCfg<D, kp_units<D>()>;
-    constexpr int UPR = NPAIR * kp_units<D>(), CUS = 256;
-    KpPlan lds{w2 + 1, 1};
-    if (!C::fits(w2)) {
-        int segw = UPR;
-        while (C::fits(segw + UPR - 1)) segw += UPR;
-        lds = KpPlan{segw, (w2 + segw) / segw};
-    }
-    const int64_t base = (int64_t)B * H * ((N + BQ - 1) / BQ);
-    if (base * lds.nseg >= 4 * CUS) return lds;
-    const int rounds = (w2 + UPR) / UPR, tiles = ((w1 < N ? w1 : N) + BQ + UPR + TJ - 1) / TJ + 2;
-    KpPlan best = lds;
-    double least = 0;
-    for (int per = (lds.segw + UPR - 1) / UPR; per >= 1; --per) {                // rounds per segment
-        const int nseg = (rounds + per - 1) / per;
-        const KpPlan pl = nseg == 1 ? lds : KpPlan{per * UPR, nseg};
-        const double bytes = 2.0 * (double)(kp_dq_part_bytes(B, N, H, D, pl) + kp_part_bytes(B, N, H, D, pl));
-        const double cost = (double)((base * pl.nseg + CUS - 1) / CUS) * (per * tiles + 6) + bytes / 5e6;
-        if (per == (lds.segw + UPR - 1) / UPR) least = cost;
-        else if (cost < 0.95 * least && bytes / 2 <= (double)(SA2_STATIC_WORKSPACE_BYTES / 4)) {
-            least = cost;
-            best = pl;
-        }
-    }
-    return best;
-}
-KpPlan kp_plan(int B, int N, int H, int D, int w1, int w2) {
-    return D == 128 ? kp_plan_of<128>(B, N, H, w1, w2) : D == 64 ? kp_plan_of<64>(B, N, H, w1, w2) : kp_plan_of<32>(B, N, H, w1, w2);
-}
 
 size_t kp_dq_part_bytes(int B, int N, int H, int D, const KpPlan& pl) {
     const size_t nkb = (size_t)(N + BQ - 1) / BQ;
     return ((size_t)B * H * nkb * pl.nseg * (size_t)(BQ + pl.segw - 1) * D * sizeof(float) + 255) / 256 * 256;
+}
+
+size_t kp_part_bytes(int B, int N, int H, int D, const KpPlan& pl) {
+    return pl.nseg > 1 ? (size_t)2 * pl.nseg * B * H * (size_t)N * D * sizeof(float) : 0;
+}
+template <int D>
+KpPlan kp_plan_of(int B, int N, int H, int w1, int w2) {
+    using C = KpCfg<D, kp_units<D>()>;
+    constexpr int UPR = NPAIR * kp_units<D>();
+    int most = UPR;
+    if (C::fits(w2)) most = w2 + 1;
+    else
+        while (C::fits(most + UPR - 1)) most += UPR;
+    return plan_segments(B, N, H, w1, w2, UPR, most,
+                         [&](const KpPlan& pl) { return kp_dq_part_bytes(B, N, H, D, pl) + kp_part_bytes(B, N, H, D, pl); });
+}
+KpPlan kp_plan(int B, int N, int H, int D, int w1, int w2) {
+    return D == 128 ? kp_plan_of<128>(B, N, H, w1, w2) : D == 64 ? kp_plan_of<64>(B, N, H, w1, w2) : kp_plan_of<32>(B, N, H, w1, w2);
 }
 
 template <class E, int D, bool PAD>

@@ -1,0 +1,1134 @@
+// fp32 arithmetic on the 16-bit matrix pipes of gfx950: fp32 tensors of head dims up to 128, and 16-bit tensors of
+// the head dims the 16-bit kernels do not have, in kernels 32, 64, 96 and 128 columns wide.
+//
+// Every operand is carried as a sum of bf16 planes: x = h + m + l with h = bf16(x), m = bf16(x - h), l = bf16(x - h - m),
+// which holds all 24 bits of an fp32 value (bf16 has fp32's exponent range).  A product of two such sums is taken as
+// the MFMAs h*h, h*m, m*h, h*l, l*h, m*m (v_mfma_f32_32x32x16_bf16: exact 16-bit products, fp32 accumulation); what is
+// left out, m*l + l*m + l*l, is below 2^-26 of |x*y|, less than the rounding of an fp32 product.  bf16 tensors are one
+// plane and fp16 tensors two, exactly, so that with a three-plane partner they take three and five MFMAs.
+//
+// Why: v_mfma_f32_32x32x2_f32 runs at a sixteenth of the bf16 rate; six bf16 MFMAs do the same work in 6/16 of its
+// time.  The price is vector work (about 5.5 instructions to split a value), which runs beside the MFMAs.
+//
+// Same expanded-row view as the 16-bit kernels: rows r = (i, delta), Q~[r] = q[i] * (k2[i-delta] + k2_bias) *
+// scale*log2(e), dO~[r] = dO[i] * (v2[i-delta] + v2_bias), formed in fp32 and then split.  With the logits computed
+// transposed (S^T = K1 . Q~^T) a lane's accumulator registers are, once split, the B operand of R^T += V1^T . P^T.
+//
+// K/V (or unit) tiles go through LDS as planes, row-major with a row stride of D + 16 elements: row operands are 16-byte
+// reads of a row, transposed operands ds_read_b64_tr_b16 reads of the same tile, both free of bank conflicts.  A tile
+// is read from global memory into registers a step ahead, split on its way into LDS, one barrier per tile.
+//
+//   split_fwd_kernel    32 queries per workgroup; wavefront w takes delta = w, w+W, ... and keeps one
+//                       online softmax and one output accumulator across its units; the W are
+//                       merged once at the end.
+//   split_kp_kernel     32 K' rows per workgroup and every delta (or a segment of them).  After a unit's
+//                       sweep its three reductions go to fp32 accumulators in LDS in column-rotated
+//                       phases: dK' and dV' rows are aligned with the unit's rows, dQ rows are shifted by
+//                       delta; the dQ accumulator is written once per workgroup as a partial.
+//   split_kv_kernel     128 K/V rows per workgroup (32 per wavefront pair, resident in registers as B
+//                       operands), streaming every unit (query block, delta) that can see them.
+// The backward kernels pair their eight wavefronts as the 16-bit kernels do (one P and one dS wavefront per SIMD, so that
+// each holds the planes of one operand and one accumulator in 256 registers: four wavefronts that did both needed 350 and
+// moved 136 of them between the two register files per tile).  A step has two halves.  In the first the P wavefront
+// computes S and, beside the other's dP MFMAs, the exponentials and the split of P; in the second it adds P's product
+// while the dS wavefront multiplies and splits dS, whose product follows.
+// Every output element has one writer and a fixed summation order: no atomics, bitwise reproducible.
+#include "sa2_mfma_common.h"
+
+namespace sa2 {
+namespace {
+
+constexpr int NPAIR = 4;               // wavefront pairs per workgroup of the backward kernels
+constexpr int XT = NPAIR * 2 * 64;     // threads per workgroup
+constexpr int XJ = NPAIR * 32;         // K rows per workgroup of the K-side kernel
+
+template <class T, int D>
+struct SplitCfg {
+    static constexpr int NK = T::PLANES;       // planes of a K or V tile
+    static constexpr int DK = D / 16;          // k-steps of a contraction over head_dim
+    static constexpr int DT = D / 32;          // 32-column blocks of an output contraction
+    static constexpr int RS = D + 16;          // row stride of a plane (elements)
+    static constexpr int RSB = RS * 2;         // ... in bytes
+    static constexpr int PLANE = 32 * RS;      // elements
+    static constexpr int AS = D + 4;           // row stride of fp32 accumulators in LDS
+    static constexpr size_t LDS_LIMIT = 160 * 1024;
+    // Forward: eight wavefronts (two per SIMD) where operands and accumulators fit 256 registers, else four.
+    static constexpr int FW = D <= 64 ? 8 : 4;
+    static constexpr int KV_TILE = NK * PLANE;             // a K or V tile
+    static constexpr int KV_STAGE = 2 * KV_TILE;           // K tile, then V tile
+    static constexpr size_t FWD_TILES = (size_t)2 * KV_STAGE * 2;
+    static constexpr size_t FWD_MERGE = (size_t)FW * 32 * AS * 4;
+    static constexpr size_t FWD_LDS = (FWD_TILES > FWD_MERGE ? FWD_TILES : FWD_MERGE) + 2 * FW * 32 * 4;
+    // K'-side: two stages, or one (a barrier more per tile) where two would leave no room for the dQ accumulator
+    static constexpr int KP_STAGES = D == 128 && NK == 3 ? 1 : 2;
+    static constexpr size_t KP_TILES = (size_t)KP_STAGES * KV_STAGE * 2;
+    static constexpr size_t PX_BYTES = (size_t)NPAIR * 4096;           // P on its way to the dS wavefront: fp32, a tile per pair
+    // the stages, P, the dQ accumulator (32 + w2 rows) and the dK' and dV' accumulators (32 rows each)
+    static size_t kp_lds(int w2) { return KP_TILES + PX_BYTES + (size_t)(32 + w2 + 64) * AS * 4; }
+    static bool kp_fits(int w2) { return kp_lds(w2) <= LDS_LIMIT; }
+    // K-side: a unit is the Q~ and dO~ tiles of three planes
+    static constexpr int UNIT_TILE = 3 * PLANE;
+    static constexpr int UNIT_STAGE = 2 * UNIT_TILE;
+    static constexpr size_t KV_LDS = (size_t)2 * UNIT_STAGE * 2 + PX_BYTES + 2 * 2 * 32 * 4;
+};
+
+__device__ __forceinline__ floatx16 zero16() {
+    floatx16 z;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) z[v] = 0.f;
+    return z;
+}
+__device__ __forceinline__ int xcd_order(int pid, int total) {
+    // workgroups are dealt round-robin to the 8 XCDs: neighbours in the problem share an L2
+    return (total & 7) == 0 ? (pid & 7) * (total >> 3) + (pid >> 3) : pid;
+}
+
+typedef float fx4 __attribute__((ext_vector_type(4)));      // 16 bytes in flight (plain vectors: stay in registers)
+typedef unsigned ux2 __attribute__((ext_vector_type(2)));
+
+// The element type of the tensors: four columns as they lie in memory (Raw), their fp32 values, and fp32 values rounded
+// to the type.  Everything between the loads and the stores is fp32.
+struct MemF32 {
+    typedef float T;
+    typedef fx4 Raw;
+    static constexpr int DTYPE = SA2_F32;
+    static constexpr int PLANES = 3;
+    static __device__ __forceinline__ fx4 widen(Raw x) { return x; }
+    static __device__ __forceinline__ void store(T* p, float a, float b, float c, float d) { *(float4*)p = make_float4(a, b, c, d); }
+};
+template <class E>
+struct Mem16 {
+    typedef uint16_t T;
+    typedef ux2 Raw;
+    static constexpr int DTYPE = E::DTYPE;
+    static constexpr int PLANES = E::DTYPE == SA2_BF16 ? 1 : 2;      // bf16 planes that hold a value exactly
+    static __device__ __forceinline__ fx4 widen(Raw x) { return fx4{E::lo(x[0]), E::hi(x[0]), E::lo(x[1]), E::hi(x[1])}; }
+    static __device__ __forceinline__ void store(T* p, float a, float b, float c, float d) {
+        *(uint2*)p = make_uint2(E::pack(a, b), E::pack(c, d));
+    }
+};
+
+// Four columns of a row.  PAD: the tensors have width <= D columns; the kernel's columns from there on read as zeros
+// and are not written (rows are multiples of four elements, so four columns are inside or outside together).
+template <class T, bool PAD>
+__device__ __forceinline__ typename T::Raw raw4(const typename T::T* row, int col, int width) {
+    if constexpr (PAD) {
+        if (col >= width) return (typename T::Raw)(0);
+    }
+    return *(const typename T::Raw*)(row + col);
+}
+template <class T, bool PAD>
+__device__ __forceinline__ float4 cols4(const typename T::T* row, int col, int width) {
+    const fx4 x = T::widen(raw4<T, PAD>(row, col, width));
+    return make_float4(x[0], x[1], x[2], x[3]);
+}
+
+// ---- planes ----
+__device__ __forceinline__ uint32_t pack2(float a, float b) {          // one v_cvt_pk_bf16_f32
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    union { bf16x2 v; uint32_t u; } r;
+    r.v = __builtin_convertvector((f32x2{a, b}), bf16x2);
+    return r.u;
+}
+// The first N planes of two values (packed pairs)
+template <int N>
+__device__ __forceinline__ void split2(float a, float b, uint32_t (&o)[N]) {
+    o[0] = pack2(a, b);
+#pragma unroll
+    for (int n = 1; n < N; ++n) {
+        a -= bf16_lo(o[n - 1]);
+        b -= bf16_hi(o[n - 1]);
+        o[n] = pack2(a, b);
+    }
+}
+// Eight values (two groups of four) as an MFMA operand per plane
+template <int N>
+__device__ __forceinline__ void split8(const float (&x)[8], bf16x8 (&o)[N]) {
+    union { uint32_t u[4]; bf16x8 v; } r[N];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        uint32_t w[N];
+        split2<N>(x[2 * t], x[2 * t + 1], w);
+#pragma unroll
+        for (int n = 0; n < N; ++n) r[n].u[t] = w[n];
+    }
+#pragma unroll
+    for (int n = 0; n < N; ++n) o[n] = r[n].v;
+}
+// Four columns to the planes of a tile (`dst`: plane 0; planes lie `plane` elements apart)
+template <class T, int N>
+__device__ __forceinline__ void store_planes(const fx4& x, uint16_t* dst, int plane) {
+    uint32_t a[N], b[N];
+    split2<N>(x[0], x[1], a);
+    split2<N>(x[2], x[3], b);
+#pragma unroll
+    for (int n = 0; n < N; ++n) *(uint2*)(dst + n * plane) = make_uint2(a[n], b[n]);
+}
+// c += a * b over the planes whose product counts, the small ones first
+template <int NA, int NB>
+__device__ __forceinline__ floatx16 mma(const bf16x8 (&a)[NA], const bf16x8 (&b)[NB], floatx16 c) {
+#pragma unroll
+    for (int sum = 2; sum >= 0; --sum)
+#pragma unroll
+        for (int x = 0; x < NA; ++x)
+            if (sum - x >= 0 && sum - x < NB) c = ElemBF16::mfma(a[x], b[sum - x], c, 0, 0, 0);
+    return c;
+}
+constexpr int mma_count(int na, int nb = 3) {
+    int n = 0;
+    for (int x = 0; x < na; ++x)
+        for (int y = 0; y < nb; ++y) n += x + y <= 2;
+    return n;
+}
+// Spreads VALU instructions over the MFMAs of the block it closes
+template <int MFMAS, int VALUS>
+__device__ __forceinline__ void interleave() {
+    constexpr int PER = (VALUS + MFMAS - 1) / MFMAS;
+#pragma unroll
+    for (int x = 0; x < MFMAS; ++x) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x402, PER, 0);
+    }
+}
+// Row operand (rows of the tile as MFMA rows) of k-step kk and transposed operand (rows as the contraction index) of
+// k-step ks and 32-column block dt, all planes.  `addr`: LDS byte address of plane 0 plus the lane part.
+template <int N, int RSB>
+__device__ __forceinline__ void row_operand(uint32_t addr, int kk, bf16x8 (&o)[N]) {
+#pragma unroll
+    for (int n = 0; n < N; ++n) o[n] = lds_read_x8(addr + (uint32_t)(n * 32 * RSB + kk * 32));
+}
+// Lane part of a transposed read: within 16 lanes, lane s supplies the address of row s/4, columns 4*(s%4)..+3, and lane
+// i receives column i of those four rows; the four 16-lane groups take the rows 0-3 / 4-7 (by half) of the 16-column
+// halves of a 32-column block, so that the eight values are the k-slots of a 32x32 accumulator handed on.
+template <int RSB>
+__device__ __forceinline__ uint32_t column_lane(int lane) {
+    const int grp = lane >> 4, s = lane & 15;
+    return (uint32_t)((4 * (grp >> 1) + (s >> 2)) * RSB + (16 * (grp & 1) + 4 * (s & 3)) * 2);
+}
+template <int N, int RSB>
+__device__ __forceinline__ void column_operand(uint32_t addr, int ks, int dt, bf16x8 (&o)[N]) {
+    typedef short v4s __attribute__((ext_vector_type(4)));
+    typedef v4s __attribute__((address_space(3)))* lds_v4s;
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+        union { v4s h[2]; bf16x8 v; } u;
+        const uint32_t a = addr + (uint32_t)(n * 32 * RSB + 16 * ks * RSB + dt * 64);
+        u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(uintptr_t)a);
+        u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(uintptr_t)(a + 8 * RSB));
+        o[n] = u.v;
+    }
+}
+
+// Rows [j0, j0+32) of two tensors (clamped to the sequence) from global memory to registers, and
+// from there, split, to the two tiles of a stage.  NT threads.
+template <class T, int D, int NT>
+struct TileRegs {
+    static constexpr int ALL = 32 * D / 4, KR = (ALL + NT - 1) / NT;       // groups of four columns: of a tile, per thread
+    typename T::Raw a[KR], b[KR];
+    template <bool PAD>
+    __device__ __forceinline__ void load(const typename T::T* ap, int64_t as, const typename T::T* bp, int64_t bs, int j0, int N, int tid, int width) {
+#pragma unroll
+        for (int u = 0; u < KR; ++u) {
+            const int c = tid + NT * u;
+            if (ALL % NT != 0 && c >= ALL) break;
+            const int row = c / (D / 4), col = c - row * (D / 4);
+            int j = j0 + row;
+            j = j < N ? j : N - 1;
+            a[u] = raw4<T, PAD>(ap + (int64_t)j * as, col * 4, width);
+            b[u] = raw4<T, PAD>(bp + (int64_t)j * bs, col * 4, width);
+        }
+    }
+    __device__ __forceinline__ void store(uint16_t* stage, int tid) const {
+        using C = SplitCfg<T, D>;
+#pragma unroll
+        for (int u = 0; u < KR; ++u) {
+            const int c = tid + NT * u;
+            if (ALL % NT != 0 && c >= ALL) break;
+            const int row = c / (D / 4), col = c - row * (D / 4);
+            store_planes<T, C::NK>(T::widen(a[u]), stage + row * C::RS + col * 4, C::PLANE);
+            store_planes<T, C::NK>(T::widen(b[u]), stage + C::KV_TILE + row * C::RS + col * 4, C::PLANE);
+        }
+    }
+};
+// The product row x * (y + bias) * mul of eight columns from `col` on, split into three planes
+template <class T, bool PAD>
+__device__ __forceinline__ void product_planes(const typename T::T* xrow, const typename T::T* yrow, int col, int width, float bias, float mul,
+                                               bf16x8 (&o)[3]) {
+    const float4 x0 = cols4<T, PAD>(xrow, col, width), x1 = cols4<T, PAD>(xrow, col + 4, width);
+    const float4 y0 = cols4<T, PAD>(yrow, col, width), y1 = cols4<T, PAD>(yrow, col + 4, width);
+    const float r[8] = {x0.x * mul * (y0.x + bias), x0.y * mul * (y0.y + bias), x0.z * mul * (y0.z + bias), x0.w * mul * (y0.w + bias),
+                        x1.x * mul * (y1.x + bias), x1.y * mul * (y1.y + bias), x1.z * mul * (y1.z + bias), x1.w * mul * (y1.w + bias)};
+    split8<3>(r, o);
+}
+
+// ================================================================== forward =====
+template <class T, int D, bool PAD>
+__global__ __launch_bounds__((SplitCfg<T, D>::FW * 64)) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 2 : 1, D <= 64 ? 2 : 1)))
+void split_fwd_kernel(Problem p, int nqb, int total) {
+    using C = SplitCfg<T, D>;
+    constexpr int W = C::FW, NT = W * 64;
+    typedef typename T::T EL;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_f[];
+    uint16_t* tiles = (uint16_t*)smem_f;                                             // two stages
+    float* mrg_m = (float*)(smem_f + (C::FWD_LDS - (size_t)2 * W * 32 * 4));         // [W][32]
+    float* mrg_l = mrg_m + W * 32;                                                   // [W][32]
+
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63, ln = lane & 31, hf = lane >> 5;
+    const int pid = xcd_order(blockIdx.x, total);
+    const int bh = pid / nqb, qb = pid - bh * nqb;
+    const int b = bh / p.H, h = bh - b * p.H;
+    const int N = p.N, w1 = p.w1, w2 = p.w2;
+    const int i0 = qb * BQ, i = i0 + ln, ic = i < N ? i : N - 1;
+    const int i_last = i0 + BQ - 1 < N ? i0 + BQ - 1 : N - 1;
+
+    const EL* qp = (const EL*)p.q.p + p.q.off(b, 0, h);
+    const EL* k1p = (const EL*)p.k1.p + p.k1.off(b, 0, h);
+    const EL* k2p = (const EL*)p.k2.p + p.k2.off(b, 0, h);
+    const EL* v1p = (const EL*)p.v1.p + p.v1.off(b, 0, h);
+    const EL* v2p = (const EL*)p.v2.p + p.v2.off(b, 0, h);
+
+    const int jt_lo = (i0 - w1 > 0 ? i0 - w1 : 0) / TJ, jt_hi = i_last / TJ;
+    const int nt = jt_hi - jt_lo + 1;
+    const int n_units = (w2 < i_last ? w2 : i_last) + 1;
+    const int nrounds = (n_units + W - 1) / W;
+    const float qscale = p.scale * LOG2E;
+
+    const uint32_t tiles_addr = lds_address(tiles);
+    const uint32_t row_lane = (uint32_t)(ln * C::RSB + hf * 16), col_lane = column_lane<C::RSB>(lane);
+
+    TileRegs<T, D, NT> next;                     // the tile on its way from global memory to LDS
+    auto request = [&](int s) { next.template load<PAD>(k1p, p.k1.sn, v1p, p.v1.sn, (jt_lo + s) * TJ, N, tid, p.D); };
+    request(0);
+    next.store(tiles, tid);
+    request(1 % nt);
+    __syncthreads();
+
+    // the wavefront's running softmax over its units: reference exponent, sum, weighted output
+    float M = -INFINITY, L = 0.f;
+    floatx16 oacc[C::DT];
+#pragma unroll
+    for (int dt = 0; dt < C::DT; ++dt) oacc[dt] = zero16();
+
+    int g = 0;
+    for (int round = 0; round < nrounds; ++round) {
+        const int delta = round * W + wave;
+        const bool ok = delta < n_units;
+        const int kr = ic - delta > 0 ? ic - delta : 0;
+        const bool row_ok = ok && i < N && i >= delta;
+        const bool rows_full = i0 >= delta && i0 + BQ - 1 < N;
+
+        bf16x8 qf[C::DK][3];
+        if (ok) {
+#pragma unroll
+            for (int kk = 0; kk < C::DK; ++kk)
+                product_planes<T, PAD>(qp + (int64_t)ic * p.q.sn, k2p + (int64_t)kr * p.k2.sn, kk * 16 + hf * 8, p.D, p.k2_bias, qscale, qf[kk]);
+        }
+        float m = -INFINITY, l = 0.f;
+        floatx16 racc[C::DT];
+#pragma unroll
+        for (int dt = 0; dt < C::DT; ++dt) racc[dt] = zero16();
+
+        for (int s = 0; s < nt; ++s, ++g) {
+            if (ok) {
+                const int j0 = (jt_lo + s) * TJ;
+                const uint32_t Ks = tiles_addr + (uint32_t)((g & 1) * C::KV_STAGE * 2);
+                const uint32_t Vt = Ks + (uint32_t)(C::KV_TILE * 2) + col_lane;
+                floatx16 sacc = zero16();
+#pragma unroll
+                for (int kk = 0; kk < C::DK; ++kk) {
+                    bf16x8 ka[C::NK];
+                    row_operand<C::NK, C::RSB>(Ks + row_lane, kk, ka);
+                    sacc = mma(ka, qf[kk], sacc);
+                }
+                // register v of this lane: key j0 + 8*(v/4) + 4*hf + v%4
+                const bool interior = rows_full && (j0 + TJ - 1 <= i0) && (j0 >= i0 + BQ - 1 - w1);
+                if (!interior) {
+                    const int hi = i - j0 - 4 * hf, lo = hi - w1;
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) {
+                        const int c = 8 * (v >> 2) + (v & 3);
+                        sacc[v] = (row_ok && c <= hi && c >= lo) ? sacc[v] : -INFINITY;
+                    }
+                }
+                float mx = sacc[0];
+#pragma unroll
+                for (int v = 1; v < 16; ++v) mx = fmaxf(mx, sacc[v]);
+                mx = fmaxf(mx, other_half(mx));
+                const float m_new = fmaxf(m, mx);
+                const float m_use = m_new == -INFINITY ? 0.f : m_new;
+                const float alpha = fast_exp2(m - m_use);
+                m = m_new;
+                if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
+                    l *= alpha;
+#pragma unroll
+                    for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) racc[dt][v] *= alpha;
+                }
+                bf16x8 pb[2][3];
+                float rs = 0.f;
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks) {
+                    float pv[8];
+#pragma unroll
+                    for (int t = 0; t < 8; ++t) {
+                        pv[t] = fast_exp2(sacc[8 * ks + t] - m_use);
+                        rs += pv[t];
+                    }
+                    split8<3>(pv, pb[ks]);
+                }
+                l += rs;
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                    for (int dt = 0; dt < C::DT; ++dt) {
+                        bf16x8 va[C::NK];
+                        column_operand<C::NK, C::RSB>(Vt, ks, dt, va);
+                        racc[dt] = mma(va, pb[ks], racc[dt]);
+                    }
+            }
+            // (unconditional: past the last step this moves a tile nobody reads, which is cheaper than a branch
+            // around register arrays)
+            next.store(tiles + ((g + 1) & 1) * C::KV_STAGE, tid);
+            request((s + 2) % nt);
+            __syncthreads();
+        }
+
+        if (ok) {
+            // fold the unit into the wavefront's running result: O += e^(m-M) * (v2 + bias) * R
+            const float lt = l + other_half(l);
+            const float M_new = fmaxf(M, m);
+            const float Mu = M_new == -INFINITY ? 0.f : M_new;
+            const float a = fast_exp2(M - Mu), c = fast_exp2(m - Mu);
+            L = L * a + lt * c;
+            M = M_new;
+            const EL* vrow = v2p + (int64_t)kr * p.v2.sn;
+#pragma unroll
+            for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+                for (int g4 = 0; g4 < 4; ++g4) {
+                    const float4 x = cols4<T, PAD>(vrow, dt * 32 + 8 * g4 + 4 * hf, p.D);
+                    oacc[dt][4 * g4 + 0] = oacc[dt][4 * g4 + 0] * a + c * racc[dt][4 * g4 + 0] * (x.x + p.v2_bias);
+                    oacc[dt][4 * g4 + 1] = oacc[dt][4 * g4 + 1] * a + c * racc[dt][4 * g4 + 1] * (x.y + p.v2_bias);
+                    oacc[dt][4 * g4 + 2] = oacc[dt][4 * g4 + 2] * a + c * racc[dt][4 * g4 + 2] * (x.z + p.v2_bias);
+                    oacc[dt][4 * g4 + 3] = oacc[dt][4 * g4 + 3] * a + c * racc[dt][4 * g4 + 3] * (x.w + p.v2_bias);
+                }
+        }
+    }
+
+    // ---- merge the wavefronts (the tile stages are free: the sweep's last barrier is behind us) ----
+    float* mrg = (float*)smem_f;                           // [W][32][AS]
+    {
+        float* row = mrg + (wave * 32 + ln) * C::AS + 4 * hf;
+#pragma unroll
+        for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4)
+                *(float4*)(row + dt * 32 + 8 * g4) = make_float4(oacc[dt][4 * g4], oacc[dt][4 * g4 + 1], oacc[dt][4 * g4 + 2],
+                                                                 oacc[dt][4 * g4 + 3]);
+        if (hf == 0) {
+            mrg_m[wave * 32 + ln] = M;
+            mrg_l[wave * 32 + ln] = L;
+        }
+    }
+    __syncthreads();
+    constexpr int TPR = NT / 32;                           // threads per row
+    const int row = tid / TPR, io = i0 + row;
+    if (io < N) {
+        float Mx = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < W; ++w) Mx = fmaxf(Mx, mrg_m[w * 32 + row]);
+        const float Mu = Mx == -INFINITY ? 0.f : Mx;
+        float wgt[W], Ls = 0.f;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            wgt[w] = fast_exp2(mrg_m[w * 32 + row] - Mu);
+            Ls += mrg_l[w * 32 + row] * wgt[w];
+        }
+        // sum_w + 1e-8 in units of 2^Mu (reference.py:74); for a tiny Mu the epsilon dominates
+        const bool big = Mu > LOG2_EPS;
+        const float denom = big ? Ls + 1e-8f * fast_exp2(-Mu) : Ls * fast_exp2(Mu - LOG2_EPS) + 1.f;
+        const float inv = big ? 1.f / denom : fast_exp2(Mu - LOG2_EPS) / denom;
+        EL* orow = (EL*)p.out.p + p.out.off(b, io, h);
+#pragma unroll
+        for (int col = 4 * (tid % TPR); col < D; col += 4 * TPR) {
+            if (PAD && col >= p.D) continue;
+            float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                const float4 y = *(const float4*)(mrg + (w * 32 + row) * C::AS + col);
+                acc.x += wgt[w] * y.x; acc.y += wgt[w] * y.y; acc.z += wgt[w] * y.z; acc.w += wgt[w] * y.w;
+            }
+            T::store(orow + col, acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+        }
+        if (tid % TPR == 0)
+            p.lse[(int64_t)bh * N + io] = big ? LN2 * Mu + logf(denom) : LN_EPS + logf(denom);
+    }
+}
+
+// ============================================== backward, K' side: dQ, dK', dV' =====
+// P between the wavefronts of a pair: 16 values per lane as four 16-byte chunks, chunk-major (no bank conflicts)
+__device__ __forceinline__ void px_put(float* px, int lane, const float (&p)[16]) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) *(fx4*)(px + c * 256 + lane * 4) = fx4{p[4 * c], p[4 * c + 1], p[4 * c + 2], p[4 * c + 3]};
+}
+__device__ __forceinline__ void px_get(const float* px, int lane, float (&p)[16]) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const fx4 x = *(const fx4*)(px + c * 256 + lane * 4);
+        p[4 * c] = x[0]; p[4 * c + 1] = x[1]; p[4 * c + 2] = x[2]; p[4 * c + 3] = x[3];
+    }
+}
+template <int N>
+__device__ __forceinline__ void split16(const float (&x)[16], bf16x8 (&o)[2][N]) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+        float h[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) h[t] = x[8 * ks + t];
+        split8<N>(h, o[ks]);
+    }
+}
+
+// The K' window in nseg segments of segw deltas, one workgroup per (segment, K' block): segment-major launch order.
+// nseg > 1: fp32 partial dK', dV' to `kpart` ([dV' | dK'][nseg][B*H][N][D]).
+template <class T, int D, bool PAD>
+__global__ __launch_bounds__(XT) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void split_kp_kernel(Problem p, int nkb, int per_seg, float* __restrict__ dq_part, int nseg, int segw, float* __restrict__ kpart) {
+    using C = SplitCfg<T, D>;
+    typedef typename T::T EL;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_f[];
+    uint16_t* tiles = (uint16_t*)smem_f;
+    float* px_all = (float*)(smem_f + C::KP_TILES);
+    float* dk_s = px_all + NPAIR * 1024;         // [32][AS]: dK' rows k0 .. k0+31 (before the scale)
+    float* dv_s = dk_s + 32 * C::AS;             // [32][AS]: dV' rows
+    float* dq_s = dv_s + 32 * C::AS;             // [32 + segw - 1][AS]: dQ rows k0 + first delta .. (before the scale)
+
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int role = wave >> 2, pr = wave & 3;   // role 0: P wavefront, 1: dS wavefront
+    const int lane = tid & 63, ln = lane & 31, hf = lane >> 5;
+    const int seg = (int)blockIdx.x / per_seg;
+    const int pid = xcd_order((int)blockIdx.x - seg * per_seg, per_seg);
+    const int bh = pid / nkb, kb = pid - bh * nkb;
+    const int b = bh / p.H, h = bh - b * p.H;
+    const int N = p.N, w1 = p.w1, w2 = p.w2;
+    const int k0 = kb * BQ, k = k0 + ln, kc = k < N ? k : N - 1;
+    const int dlo = seg * segw;                  // first delta of the segment
+    const int RQ = 32 + segw - 1;                // rows of the dQ accumulator
+
+    const EL* qp = (const EL*)p.q.p + p.q.off(b, 0, h);
+    const EL* k1p = (const EL*)p.k1.p + p.k1.off(b, 0, h);
+    const EL* k2p = (const EL*)p.k2.p + p.k2.off(b, 0, h);
+    const EL* v1p = (const EL*)p.v1.p + p.v1.off(b, 0, h);
+    const EL* v2p = (const EL*)p.v2.p + p.v2.off(b, 0, h);
+    const EL* dop = (const EL*)p.dout.p + p.dout.off(b, 0, h);
+    const bool want_dq = p.dq.p != nullptr;
+
+    const int nu_all = (w2 < N - 1 - k0 ? w2 : N - 1 - k0) + 1;        // deltas with k0 + delta < N
+    const int n_units = nu_all - dlo < segw ? nu_all - dlo : segw;     // of this segment (may be <= 0)
+    const int nrounds = (n_units + NPAIR - 1) / NPAIR;
+    const float qscale = p.scale * LOG2E;
+    const uint32_t tiles_addr = lds_address(tiles);
+    const uint32_t row_lane = (uint32_t)(ln * C::RSB + hf * 16), col_lane = column_lane<C::RSB>(lane);
+    float* px = px_all + pr * 1024;
+
+    for (int c = tid; c < (RQ + 64) * C::AS; c += XT) dk_s[c] = 0.f;       // all three accumulators
+
+    TileRegs<T, D, XT> next;                     // the tile on its way from global memory to LDS
+    auto rounds = [&](auto ROLE_TAG) {
+        constexpr int ROLE = decltype(ROLE_TAG)::value;
+        const int d_end = dlo + n_units - 1;
+        auto first_tile = [&](int round) {                    // of the round's smallest delta
+            const int i_min = k0 + dlo + round * NPAIR;
+            return (i_min - w1 > 0 ? i_min - w1 : 0) / TJ;
+        };
+        auto request = [&](int jt) { next.template load<PAD>(k1p, p.k1.sn, v1p, p.v1.sn, jt * TJ, N, tid, p.D); };
+        if (nrounds > 0) request(first_tile(0));
+        for (int round = 0; round < nrounds; ++round) {
+            // tiles of the round's units (within the sequence)
+            const int d_first = dlo + round * NPAIR;
+            const int d_last = d_first + NPAIR - 1 < d_end ? d_first + NPAIR - 1 : d_end;
+            const int i_max = k0 + 31 + d_last < N - 1 ? k0 + 31 + d_last : N - 1;
+            const int jt_lo = first_tile(round), jt_hi = i_max / TJ;
+            const int nt = jt_hi - jt_lo + 1;
+
+            const int delta = d_first + pr;
+            const bool ok = delta <= d_end;
+            const int i = k + delta, ic = i < N ? i : N - 1;
+            const bool row_ok = ok && i < N;                  // (k <= i < N)
+            const int iw_lo = k0 + delta, iw_hi = k0 + 31 + delta < N - 1 ? k0 + 31 + delta : N - 1;   // this unit's queries
+            const bool rows_full = k0 + 31 + delta < N;
+
+            bf16x8 xf[C::DK][3];                              // Q~ (P wavefront) or dO~ (dS wavefront)
+            float c0 = 0.f;                                   // the C operand of the first chain: -LSE or -D
+            if (ok) {
+#pragma unroll
+                for (int kk = 0; kk < C::DK; ++kk) {
+                    const int col = kk * 16 + hf * 8;
+                    if constexpr (ROLE == 0)
+                        product_planes<T, PAD>(qp + (int64_t)ic * p.q.sn, k2p + (int64_t)kc * p.k2.sn, col, p.D, p.k2_bias, qscale, xf[kk]);
+                    else
+                        product_planes<T, PAD>(dop + (int64_t)ic * p.dout.sn, v2p + (int64_t)kc * p.v2.sn, col, p.D, p.v2_bias, 1.f, xf[kk]);
+                }
+                c0 = ROLE == 0 ? -p.lse[(int64_t)bh * N + ic] * LOG2E : -p.dsum[(int64_t)bh * N + ic];
+            }
+            floatx16 acc[C::DT];                              // R or G
+#pragma unroll
+            for (int dt = 0; dt < C::DT; ++dt) acc[dt] = zero16();
+
+            // (the previous round's last barrier has passed: the stages are free)
+            auto put_next = [&](int s) {                      // tile s + 1 to its stage, tile s + 2 requested
+                if (s + 1 < nt) next.store(tiles + (C::KP_STAGES == 2 ? (s + 1) & 1 : 0) * C::KV_STAGE, tid);
+                if (s + 2 < nt) request(jt_lo + s + 2);
+            };
+            next.store(tiles, tid);
+            if (nt > 1) request(jt_lo + 1);
+            __syncthreads();
+            for (int s = 0; s < nt; ++s) {
+                const int j0 = (jt_lo + s) * TJ;
+                // tiles that hold no key of this unit's windows are skipped by the pair
+                const bool in = ok && j0 <= iw_hi && j0 + TJ - 1 >= iw_lo - w1;
+                const uint32_t Ks = tiles_addr + (uint32_t)((C::KP_STAGES == 2 ? s & 1 : 0) * C::KV_STAGE * 2);
+                const uint32_t Vs = Ks + (uint32_t)(C::KV_TILE * 2);
+                bf16x8 pb[2][3];
+                floatx16 chain;
+                if (ROLE == 1 && C::KP_STAGES == 2) put_next(s);
+                if (in) {
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) chain[v] = c0;
+                    if (ROLE == 0 && !(rows_full && (j0 + TJ - 1 <= iw_lo) && (j0 >= iw_lo + 31 - w1))) {
+                        const int hi = i - j0 - 4 * hf, lo = hi - w1;
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) {
+                            const int c = 8 * (v >> 2) + (v & 3);
+                            chain[v] = row_ok && c <= hi && c >= lo ? c0 : -INFINITY;
+                        }
+                    }
+                    if (ROLE == 0) __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+                    for (int kk = 0; kk < C::DK; ++kk) {
+                        bf16x8 a[C::NK];
+                        row_operand<C::NK, C::RSB>((ROLE == 0 ? Ks : Vs) + row_lane, kk, a);
+                        chain = mma(a, xf[kk], chain);
+                    }
+                    if (ROLE == 0) {
+                        __builtin_amdgcn_s_setprio(0);
+                        float pv[16];
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) pv[v] = fast_exp2(chain[v]);
+                        px_put(px, lane, pv);
+                        split16<3>(pv, pb);
+                    }
+                }
+                __syncthreads();
+                if (in) {
+                    if (ROLE == 1) {
+                        float pv[16];
+                        px_get(px, lane, pv);
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) pv[v] *= chain[v];
+                        split16<3>(pv, pb);
+                    }
+#pragma unroll
+                    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                        for (int dt = 0; dt < C::DT; ++dt) {
+                            bf16x8 a[C::NK];
+                            column_operand<C::NK, C::RSB>((ROLE == 0 ? Vs : Ks) + col_lane, ks, dt, a);
+                            acc[dt] = mma(a, pb[ks], acc[dt]);
+                        }
+                }
+                if (C::KP_STAGES == 1) __syncthreads();       // everyone is done with the only stage
+                if (ROLE == 0 || C::KP_STAGES == 1) put_next(s);
+                __syncthreads();
+            }
+
+            // ---- the unit's reductions into the workgroup's LDS accumulators: dV'[k] += R*dO[i] (P wavefronts),
+            //      dK'[k] += G*q[i] (rows ln) and dQ[i] += G*k2~[k] (rows ln + delta; dS wavefronts).  Four phases; in phase
+            //      ph pair pr owns column group (pr + ph) % 4 of every row, so no two wavefronts touch an element at
+            //      once and every element sums in a fixed order.  The rows are read once, before the phases. ----
+            typename T::Raw x[4 * C::DT], y[ROLE == 1 ? 4 * C::DT : 1];
+            {
+                const EL* xrow = ROLE == 0 ? dop + (int64_t)ic * p.dout.sn : qp + (int64_t)ic * p.q.sn;
+                const EL* krow = k2p + (int64_t)kc * p.k2.sn;
+#pragma unroll
+                for (int e = 0; e < 4 * C::DT; ++e) {
+                    const int col = (e >> 2) * 32 + 8 * (e & 3) + 4 * hf;
+                    x[e] = raw4<T, PAD>(xrow, col, p.D);
+                    if (ROLE == 1) y[ROLE == 1 ? e : 0] = raw4<T, PAD>(krow, col, p.D);
+                }
+            }
+            if (round + 1 < nrounds) request(first_tile(round + 1));
+            auto reduce = [&](auto PR_TAG) {
+                constexpr int PR = decltype(PR_TAG)::value;
+                float* arow = (ROLE == 0 ? dv_s : dk_s) + ln * C::AS + 4 * hf;
+                float* dqrow = dq_s + (ln + delta - dlo) * C::AS + 4 * hf;
+#pragma unroll
+                for (int ph = 0; ph < 4; ++ph) {
+                    constexpr int G4S[4] = {PR, (PR + 1) & 3, (PR + 2) & 3, (PR + 3) & 3};
+                    const int g4 = G4S[ph];
+                    if (row_ok) {
+#pragma unroll
+                        for (int dt = 0; dt < C::DT; ++dt) {
+                            const int col = dt * 32 + 8 * g4;
+                            const fx4 xv = T::widen(x[4 * dt + g4]);
+                            fx4 a = *(fx4*)(arow + col);
+#pragma unroll
+                            for (int t = 0; t < 4; ++t) a[t] += acc[dt][4 * g4 + t] * xv[t];
+                            *(fx4*)(arow + col) = a;
+                            if (ROLE == 1 && want_dq) {
+                                const fx4 yv = T::widen(y[ROLE == 1 ? 4 * dt + g4 : 0]);
+                                fx4 o = *(fx4*)(dqrow + col);
+#pragma unroll
+                                for (int t = 0; t < 4; ++t) o[t] += acc[dt][4 * g4 + t] * (yv[t] + p.k2_bias);
+                                *(fx4*)(dqrow + col) = o;
+                            }
+                        }
+                    }
+                    __syncthreads();
+                }
+            };
+            switch (pr) {
+                case 0: reduce(std::integral_constant<int, 0>{}); break;
+                case 1: reduce(std::integral_constant<int, 1>{}); break;
+                case 2: reduce(std::integral_constant<int, 2>{}); break;
+                default: reduce(std::integral_constant<int, 3>{}); break;
+            }
+        }
+    };
+    if (role == 0) rounds(std::integral_constant<int, 0>{});
+    else rounds(std::integral_constant<int, 1>{});
+    __syncthreads();
+
+    // ---- dK' and dV' rows of the block ----
+    for (int c = tid; c < 2 * 32 * (D / 4); c += XT) {
+        const int which = c / (32 * (D / 4)), rem = c - which * 32 * (D / 4);     // 0: dV', 1: dK'
+        const int row = rem / (D / 4), col = (rem - row * (D / 4)) * 4, ko = k0 + row;
+        const Tensor& t = which ? p.dk2 : p.dv2;
+        if (ko >= N || !t.p) continue;
+        const float sc = which ? p.scale : 1.f;
+        const fx4 a = *(const fx4*)((which ? dk_s : dv_s) + row * C::AS + col) * sc;
+        if (nseg > 1) *(fx4*)(kpart + ((((int64_t)which * nseg + seg) * p.B * p.H + bh) * N + ko) * D + col) = a;
+        else if (!PAD || col < p.D) T::store((EL*)t.p + t.off(b, ko, h) + col, a[0], a[1], a[2], a[3]);
+    }
+    // ---- dQ partial: rows k0 + dlo .. (rows of deltas beyond the end of the sequence hold zeros) ----
+    if (want_dq) {
+        float* part = dq_part + (((int64_t)bh * nkb + kb) * nseg + seg) * (int64_t)RQ * D;
+        for (int c = tid; c < RQ * (D / 4); c += XT) {
+            const int r = c / (D / 4), col = (c - r * (D / 4)) * 4;
+            *(fx4*)(part + (int64_t)r * D + col) = *(const fx4*)(dq_s + r * C::AS + col) * p.scale;
+        }
+    }
+}
+
+// =================================================== backward, K side: dK, dV =====
+// nsplit > 1 (grids smaller than the chip): the workgroup takes the sp-th share of the key block's stream
+// of units and writes fp32 partial sums to `part` ([dK | dV][nsplit][B*H][N][D]) for bwd_sum_kernel.
+template <class T, int D, bool SPLIT, bool PAD>
+__global__ __launch_bounds__(XT) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void split_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __restrict__ part) {
+    const int nsplit = SPLIT ? nsplit_arg : 1;
+    using C = SplitCfg<T, D>;
+    typedef typename T::T EL;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_f[];
+    uint16_t* tiles = (uint16_t*)smem_f;
+    float* px_all = (float*)(tiles + 2 * C::UNIT_STAGE);
+    float* lse_s = px_all + NPAIR * 1024;        // [2][32]  -LSE*log2(e) of the unit's queries
+    float* dsum_s = lse_s + 2 * 32;              // [2][32]  -D
+
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int role = wave >> 2, pr = wave & 3;   // role 0: P wavefront (K rows, dV), 1: dS wavefront (V rows, dK)
+    const int lane = tid & 63, ln = lane & 31, hf = lane >> 5;
+    const int pid = xcd_order(blockIdx.x, total);
+    const int sp = pid % nsplit, pj = pid / nsplit;
+    const int bh = pj / njb, jb = pj - bh * njb;
+    const int b = bh / p.H, h = bh - b * p.H;
+    const int N = p.N, w1 = p.w1, w2 = p.w2;
+    const int j0 = jb * XJ, jw = j0 + 32 * pr, j = jw + ln, jc = j < N ? j : N - 1;
+
+    const EL* qp = (const EL*)p.q.p + p.q.off(b, 0, h);
+    const EL* k1p = (const EL*)p.k1.p + p.k1.off(b, 0, h);
+    const EL* k2p = (const EL*)p.k2.p + p.k2.off(b, 0, h);
+    const EL* v1p = (const EL*)p.v1.p + p.v1.off(b, 0, h);
+    const EL* v2p = (const EL*)p.v2.p + p.v2.off(b, 0, h);
+    const EL* dop = (const EL*)p.dout.p + p.dout.off(b, 0, h);
+    const float qscale = p.scale * LOG2E;
+
+    const uint32_t tiles_addr = lds_address(tiles);
+    const uint32_t row_lane = (uint32_t)(ln * C::RSB + hf * 16), col_lane = column_lane<C::RSB>(lane);
+
+    float* px = px_all + pr * 1024;
+
+    // the pair's K rows (P wavefront) or V rows (dS wavefront) as resident B operands (column = key j)
+    bf16x8 kf[C::DK][C::NK];
+    {
+        const EL* row = role ? v1p + (int64_t)jc * p.v1.sn : k1p + (int64_t)jc * p.k1.sn;
+#pragma unroll
+        for (int kk = 0; kk < C::DK; ++kk) {
+            const int col = kk * 16 + hf * 8;
+            const float4 x0 = cols4<T, PAD>(row, col, p.D), x1 = cols4<T, PAD>(row, col + 4, p.D);
+            const float r[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+            split8<C::NK>(r, kf[kk]);
+        }
+    }
+    floatx16 acc[C::DT];                         // dV^T or dK^T
+#pragma unroll
+    for (int dt = 0; dt < C::DT; ++dt) acc[dt] = zero16();
+
+    const int j_last = j0 + XJ - 1 < N ? j0 + XJ - 1 : N - 1;
+    const int i_max = (int)((int64_t)j_last + w1 < N - 1 ? j_last + w1 : N - 1);
+    auto units_of = [&](int ib) {
+        const int il = ib * BQ + BQ - 1 < N ? ib * BQ + BQ - 1 : N - 1;
+        return (w2 < il ? w2 : il) + 1;
+    };
+    // The units (query block, delta) that see the key block, in stream order, and this workgroup's share of
+    // them: from delta d_first of block ib_lo to delta d_last of block ib_hi.  The shares cut the stream
+    // counted with w2 + 1 slots per block (a block near the start of the sequence has fewer units: the slots
+    // beyond are skipped).
+    int ib_lo = j0 / BQ, ib_hi = i_max / BQ, d_first = 0, d_last = w2;
+    bool empty_share = ib_lo > ib_hi;
+    if constexpr (SPLIT) {
+        const int per = w2 + 1, ib0 = ib_lo;
+        const int slots = (ib_hi - ib_lo + 1) * per;
+        const int chunk = (slots + nsplit - 1) / nsplit;
+        const int v_lo = sp * chunk, v_hi = (v_lo + chunk < slots ? v_lo + chunk : slots) - 1;
+        empty_share = v_lo > v_hi;
+        if (!empty_share) {
+            ib_lo = ib0 + v_lo / per;
+            d_first = v_lo - (ib_lo - ib0) * per;
+            ib_hi = ib0 + v_hi / per;
+            d_last = v_hi - (ib_hi - ib0) * per;
+            if (d_first >= units_of(ib_lo)) {        // the share starts in the slots a short block does not have
+                ++ib_lo;
+                d_first = 0;
+            }
+            empty_share = !(ib_lo < ib_hi || (ib_lo == ib_hi && d_first <= d_last));
+        }
+    }
+    // (a share of a split launch may be empty: it walks one unit without touching it and writes zeros)
+    if (empty_share) {
+        ib_lo = ib_hi = j0 / BQ;
+        d_first = d_last = 0;
+    }
+
+    // ---- forming a unit: Q~ and dO~ tiles (32 rows), LSE and D of its queries ----
+    constexpr int ALL = 32 * D / 4, KR = (ALL + XT - 1) / XT;      // groups of four columns: of a tile, per thread
+    typename T::Raw fq[KR], fk[KR], fd[KR], fv[KR];
+    float f_lse = 0.f, f_dsum = 0.f;
+    auto fetch_unit = [&](int ib, int delta) {
+#pragma unroll
+        for (int u = 0; u < KR; ++u) {
+            const int c = tid + XT * u;
+            if (ALL % XT != 0 && c >= ALL) break;
+            const int row = c / (D / 4), col = c - row * (D / 4);
+            int i = ib * BQ + row;
+            i = i < N ? i : N - 1;
+            const int k = i - delta > 0 ? i - delta : 0;
+            fq[u] = raw4<T, PAD>(qp + (int64_t)i * p.q.sn, col * 4, p.D);
+            fk[u] = raw4<T, PAD>(k2p + (int64_t)k * p.k2.sn, col * 4, p.D);
+            fd[u] = raw4<T, PAD>(dop + (int64_t)i * p.dout.sn, col * 4, p.D);
+            fv[u] = raw4<T, PAD>(v2p + (int64_t)k * p.v2.sn, col * 4, p.D);
+        }
+        if (tid < 32) {
+            int i = ib * BQ + tid;
+            i = i < N ? i : N - 1;
+            f_lse = -p.lse[(int64_t)bh * N + i] * LOG2E;
+            f_dsum = -p.dsum[(int64_t)bh * N + i];
+        }
+    };
+    auto store_unit = [&](int buf) {
+        uint16_t* Qs = tiles + buf * C::UNIT_STAGE;
+        uint16_t* Ds = Qs + C::UNIT_TILE;
+#pragma unroll
+        for (int u = 0; u < KR; ++u) {
+            const int c = tid + XT * u;
+            if (ALL % XT != 0 && c >= ALL) break;
+            const int row = c / (D / 4), col = c - row * (D / 4);
+            const float kb = p.k2_bias, vb = p.v2_bias;
+            const fx4 q4 = T::widen(fq[u]), k4 = T::widen(fk[u]), d4 = T::widen(fd[u]), v4 = T::widen(fv[u]);
+            const fx4 qt = {q4[0] * qscale * (k4[0] + kb), q4[1] * qscale * (k4[1] + kb), q4[2] * qscale * (k4[2] + kb), q4[3] * qscale * (k4[3] + kb)};
+            const fx4 dt = {d4[0] * (v4[0] + vb), d4[1] * (v4[1] + vb), d4[2] * (v4[2] + vb), d4[3] * (v4[3] + vb)};
+            store_planes<T, 3>(qt, Qs + row * C::RS + col * 4, C::PLANE);
+            store_planes<T, 3>(dt, Ds + row * C::RS + col * 4, C::PLANE);
+        }
+        if (tid < 32) {
+            lse_s[buf * 32 + tid] = f_lse;
+            dsum_s[buf * 32 + tid] = f_dsum;
+        }
+    };
+
+    fetch_unit(ib_lo, d_first);
+    store_unit(0);
+    __syncthreads();
+    auto stream = [&](auto ROLE_TAG) {
+        constexpr int ROLE = decltype(ROLE_TAG)::value;
+        int ib = ib_lo, delta = d_first, nu = units_of(ib_lo), buf = 0;
+        while (true) {
+            int nib = ib, ndelta = delta + 1;
+            if (ndelta >= nu) {
+                nib = ib + 1;
+                ndelta = 0;
+            }
+            const bool more = SPLIT ? (nib < ib_hi || (nib == ib_hi && ndelta <= d_last)) : nib <= ib_hi;
+            if (more) fetch_unit(nib, ndelta);
+
+            const int i0 = ib * BQ;
+            const bool touches = (i0 + BQ - 1 >= jw) && ((int64_t)i0 <= (int64_t)jw + 31 + w1) && jw < N && !empty_share;
+            const uint32_t Qs = tiles_addr + (uint32_t)(buf * C::UNIT_STAGE * 2);
+            const uint32_t Ds = Qs + (uint32_t)(C::UNIT_TILE * 2);
+            bf16x8 pb[2][3];
+            floatx16 chain;
+            if (touches) {
+                // register v of this lane: query i0 + 8*(v/4) + 4*hf + v%4, key j; -LSE (-inf outside the window) or -D
+                const float* c0 = (ROLE == 0 ? lse_s : dsum_s) + buf * 32 + 4 * hf;
+#pragma unroll
+                for (int g4 = 0; g4 < 4; ++g4) {
+                    const fx4 x = *(const fx4*)(c0 + 8 * g4);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) chain[4 * g4 + t] = x[t];
+                }
+                if (ROLE == 0 && !((i0 >= jw + 31) && ((int64_t)i0 + 31 <= (int64_t)jw + w1) && (i0 + BQ - 1 < N) && (i0 >= delta))) {
+                    const int lo = j - i0 - 4 * hf;                                    // c >= lo  <=>  j <= i
+                    const int hi = (int)((int64_t)j + w1 - i0 < (1 << 20) ? j + w1 - i0 : (1 << 20)) - 4 * hf;   // i <= j + w1
+                    const int dlo = delta - i0 - 4 * hf, nhi = N - 1 - i0 - 4 * hf;
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) {
+                        const int c = 8 * (v >> 2) + (v & 3);
+                        chain[v] = (j < N) && (c >= lo) && (c <= hi) && (c >= dlo) && (c <= nhi) ? chain[v] : -INFINITY;
+                    }
+                }
+                if (ROLE == 0) __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+                for (int kk = 0; kk < C::DK; ++kk) {
+                    bf16x8 a[3];
+                    row_operand<3, C::RSB>((ROLE == 0 ? Qs : Ds) + row_lane, kk, a);
+                    chain = mma(a, kf[kk], chain);
+                }
+                if (ROLE == 0) {
+                    __builtin_amdgcn_s_setprio(0);
+                    float pv[16];
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) pv[v] = fast_exp2(chain[v]);
+                    px_put(px, lane, pv);
+                    split16<3>(pv, pb);
+                }
+            }
+            __syncthreads();
+            if (touches) {
+                if (ROLE == 1) {
+                    float pv[16];
+                    px_get(px, lane, pv);
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) pv[v] *= chain[v];
+                    split16<3>(pv, pb);
+                }
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                    for (int dt = 0; dt < C::DT; ++dt) {
+                        bf16x8 a[3];
+                        column_operand<3, C::RSB>((ROLE == 0 ? Ds : Qs) + col_lane, ks, dt, a);
+                        acc[dt] = mma(a, pb[ks], acc[dt]);
+                    }
+            }
+            if (!more) break;
+            store_unit(buf ^ 1);          // (the other buffer was last read one step ago, before that step's barrier)
+            __syncthreads();
+            if (nib != ib) nu = units_of(nib);
+            ib = nib;
+            delta = ndelta;
+            buf ^= 1;
+        }
+    };
+    if (role == 0) stream(std::integral_constant<int, 0>{});
+    else stream(std::integral_constant<int, 1>{});
+
+    if (j < N) {
+        // Q~ carries scale*log2(e): dK = ln2 * sum dS * Q~
+        const int which = role ? 0 : 1;
+        const Tensor& t = which ? p.dv1 : p.dk1;
+        if (t.p) {
+            const float sc = which ? 1.f : LN2;
+#pragma unroll
+            for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+                for (int g4 = 0; g4 < 4; ++g4) {
+                    const int col = dt * 32 + 8 * g4 + 4 * hf;
+                    const float x0 = acc[dt][4 * g4] * sc, x1 = acc[dt][4 * g4 + 1] * sc, x2 = acc[dt][4 * g4 + 2] * sc, x3 = acc[dt][4 * g4 + 3] * sc;
+                    if constexpr (SPLIT)
+                        *(float4*)(part + (((which * (int64_t)nsplit + sp) * p.B * p.H + bh) * N + j) * D + col) = make_float4(x0, x1, x2, x3);
+                    else if (!PAD || col < p.D)
+                        T::store((EL*)t.p + t.off(b, j, h) + col, x0, x1, x2, x3);
+                }
+        }
+    }
+}
+
+// Shares a key block's query blocks are split into when the K-side grid is smaller than the chip
+int split_kv_nsplit(int B, int N, int H, int D, int w1, int w2) {
+    const int64_t bh = (int64_t)B * H, base = bh * ((N + XJ - 1) / XJ);
+    const int blocks = (XJ + (w1 < N ? w1 : N) + BQ - 1) / BQ + 1;
+    const int64_t units = (int64_t)blocks * ((w2 < N - 1 ? w2 : N - 1) + 1);     // of a key block's stream, at most
+    int ns = 1;                                                                  // shares of at least 8 units
+    while (ns < 16 && base * ns * 2 <= 512 && (int64_t)ns * 2 * 8 <= units && (int64_t)2 * ns * 2 * bh * N * D * 4 <= ((int64_t)32 << 20))
+        ns *= 2;
+    return ns;
+}
+size_t split_kv_bytes(int B, int N, int H, int D, int nsplit) { return nsplit > 1 ? (size_t)2 * nsplit * B * H * (size_t)N * D * sizeof(float) : 0; }
+size_t split_dq_part_bytes(int B, int N, int H, int D, const KpPlan& pl) {
+    return ((size_t)B * H * ((N + BQ - 1) / BQ) * pl.nseg * (size_t)(31 + pl.segw) * D * sizeof(float) + 255) / 256 * 256;
+}
+size_t split_kp_bytes(int B, int N, int H, int D, const KpPlan& pl) {
+    return split_dq_part_bytes(B, N, H, D, pl) + (pl.nseg > 1 ? (size_t)2 * pl.nseg * B * H * (size_t)N * D * sizeof(float) : 0);
+}
+// Deltas per segment: what the dQ accumulator in LDS holds, or fewer where the grid asks for it
+template <class T, int D>
+KpPlan split_kp_plan(int B, int N, int H, int w1, int w2) {
+    using C = SplitCfg<T, D>;
+    int most = NPAIR;
+    while (most < w2 + 1 && C::kp_fits(most + NPAIR - 1)) most += NPAIR;
+    return plan_segments(B, N, H, w1, w2, NPAIR, most, [&](const KpPlan& pl) { return split_kp_bytes(B, N, H, D, pl); });
+}
+
+// ------------------------------------------------------------------ launchers ----
+template <class T, int D, bool PAD>
+int launch_split_fwd(const Problem& p, hipStream_t st) {
+    using C = SplitCfg<T, D>;
+    const int nqb = (p.N + BQ - 1) / BQ;
+    const int64_t total = (int64_t)nqb * p.B * p.H;
+    if (total > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
+    if (!allow_full_lds((const void*)split_fwd_kernel<T, D, PAD>)) return SA2_ERR_LAUNCH_FAILED;
+    hipLaunchKernelGGL((split_fwd_kernel<T, D, PAD>), dim3((unsigned)total), dim3(C::FW * 64), C::FWD_LDS, st, p, nqb, (int)total);
+    return hipGetLastError() == hipSuccess ? SA2_OK : SA2_ERR_LAUNCH_FAILED;
+}
+
+template <class T, int D, bool PAD>
+int launch_split_bwd(const Problem& p, hipStream_t st) {
+    using C = SplitCfg<T, D>;
+    int rc = launch_rowdot(p.out, p.dout, p.dsum, p.B, p.N, p.H, p.D, T::DTYPE, st);
+    if (rc != SA2_OK) return rc;
+    BwdSums sums = {};
+    const KpPlan pl = split_kp_plan<T, D>(p.B, p.N, p.H, p.w1, p.w2);
+    const size_t kp_bytes = (split_kp_bytes(p.B, p.N, p.H, D, pl) + 255) / 256 * 256;
+    const int nsplit = split_kv_nsplit(p.B, p.N, p.H, D, p.w1, p.w2);
+    if (p.scratch_bytes < kp_bytes + split_kv_bytes(p.B, p.N, p.H, D, nsplit)) return SA2_ERR_WORKSPACE_TOO_SMALL;
+    if (p.dq.p || p.dk2.p || p.dv2.p) {
+        const int nkb = (p.N + BQ - 1) / BQ;
+        const int64_t per_seg = (int64_t)nkb * p.B * p.H, total = per_seg * pl.nseg;
+        if (total > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
+        float* part = (float*)p.scratch;
+        float* kpart = (float*)((char*)p.scratch + split_dq_part_bytes(p.B, p.N, p.H, D, pl));
+        if (!allow_full_lds((const void*)split_kp_kernel<T, D, PAD>)) return SA2_ERR_LAUNCH_FAILED;
+        hipLaunchKernelGGL((split_kp_kernel<T, D, PAD>), dim3((unsigned)total), dim3(XT), C::kp_lds(pl.segw - 1), st, p, nkb, (int)per_seg, part,
+                           pl.nseg, pl.segw, kpart);
+        if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
+        sums.dq = p.dq.p ? part : nullptr;
+        sums.nkb = nkb;
+        sums.nseg = sums.kp_n = pl.nseg;
+        sums.segw = pl.segw;
+        sums.kp = pl.nseg > 1 ? kpart : nullptr;
+    }
+    if (p.dk1.p || p.dv1.p) {
+        const int njb = (p.N + XJ - 1) / XJ;
+        const int64_t total = (int64_t)njb * p.B * p.H * nsplit;
+        if (total > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
+        float* part = nsplit > 1 ? (float*)((char*)p.scratch + kp_bytes) : nullptr;
+        auto go = [&](auto kernel) {
+            if (!allow_full_lds((const void*)kernel)) return false;
+            hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(XT), C::KV_LDS, st, p, njb, (int)total, nsplit, part);
+            return hipGetLastError() == hipSuccess;
+        };
+        if (!(nsplit > 1 ? go(split_kv_kernel<T, D, true, PAD>) : go(split_kv_kernel<T, D, false, PAD>))) return SA2_ERR_LAUNCH_FAILED;
+        sums.kv = part;
+        sums.kv_n = nsplit;
+    }
+    return launch_bwd_sums(p, sums, D, T::DTYPE, st);
+}
+
+// rows on a 16-byte grid
+template <int PER_CHUNK>
+bool rows16(const Tensor& t, int B, int N, int H) {
+    constexpr int M = PER_CHUNK - 1;
+    if (!t.p) return true;
+    if ((uintptr_t)t.p & 15u) return false;
+    return !((B > 1 && (t.sb & M)) || (N > 1 && (t.sn & M)) || (H > 1 && (t.sh & M)));
+}
+
+// Kernel width of a head_dim, and the call f(memory type, width, PAD) for it.  16-bit tensors come here only with head
+// dims that the 16-bit kernels do not have, always padded or 96 columns wide.
+int split_width(int D) { return D <= 32 ? 32 : D <= 64 ? 64 : D <= 96 ? 96 : 128; }
+template <class F>
+int for_split_width(int D, int dtype, F&& f) {
+    auto of_type = [&](auto m) {
+        constexpr bool F32 = decltype(m)::DTYPE == SA2_F32;
+        const bool exact = F32 && D == split_width(D);
+        auto of_pad = [&](auto width) {
+            if constexpr (F32) {
+                if (exact) return f(m, width, std::false_type{});
+            }
+            return f(m, width, std::true_type{});
+        };
+        switch (split_width(D)) {
+            case 32: return of_pad(std::integral_constant<int, 32>{});
+            case 64: return of_pad(std::integral_constant<int, 64>{});
+            case 96: return f(m, std::integral_constant<int, 96>{}, std::true_type{});
+            default: return of_pad(std::integral_constant<int, 128>{});
+        }
+    };
+    return dtype == SA2_F32 ? of_type(MemF32{}) : dtype == SA2_F16 ? of_type(Mem16<ElemF16>{}) : of_type(Mem16<ElemBF16>{});
+}
+
+}  // namespace
+
+// fp32: any multiple of four columns.  16 bits: multiples of eight that the 16-bit kernels do not take.
+bool f32_mfma_supported(int D, int dtype) {
+    if (D < 4 || D > 128) return false;
+    return dtype == SA2_F32 ? D % 4 == 0 : D % 8 == 0 && D != 16 && D != 32 && D != 64 && D != 128;
+}
+
+bool f32_mfma_bwd_supported(int D, int w2, int dtype) {
+    (void)w2;                // any K' window: wide ones are walked in segments
+    return f32_mfma_supported(D, dtype);
+}
+
+bool f32_mfma_layout_ok(const Problem& p, int dtype, bool backward) {
+    auto ok = [&](const Tensor& t) { return dtype == SA2_F32 ? rows16<4>(t, p.B, p.N, p.H) : rows16<8>(t, p.B, p.N, p.H); };
+    const Tensor* fwd[] = {&p.q, &p.k1, &p.k2, &p.v1, &p.v2, &p.out};
+    for (const Tensor* t : fwd)
+        if (!ok(*t)) return false;
+    if (backward) {
+        const Tensor* bwd[] = {&p.dout, &p.dq, &p.dk1, &p.dk2, &p.dv1, &p.dv2};
+        for (const Tensor* t : bwd)
+            if (!ok(*t)) return false;
+    }
+    return true;
+}
+
+size_t f32_mfma_bwd_scratch_bytes(int B, int N, int H, int head_dim, int w1, int w2, int dtype) {
+    size_t bytes = 0;
+    for_split_width(head_dim, dtype, [&](auto m, auto width, auto) {
+        constexpr int D = decltype(width)::value;
+        bytes = (split_kp_bytes(B, N, H, D, split_kp_plan<decltype(m), D>(B, N, H, w1, w2)) + 255) / 256 * 256 +
+                split_kv_bytes(B, N, H, D, split_kv_nsplit(B, N, H, D, w1, w2));
+        return 0;
+    });
+    return bytes;
+}
+
+int launch_f32_mfma_fwd(const Problem& p, int dtype, hipStream_t st) {
+    return for_split_width(p.D, dtype, [&](auto m, auto width, auto pad) {
+        return launch_split_fwd<decltype(m), decltype(width)::value, decltype(pad)::value>(p, st);
+    });
+}
+
+int launch_f32_mfma_bwd(const Problem& p, int dtype, hipStream_t st) {
+    return for_split_width(p.D, dtype, [&](auto m, auto width, auto pad) {
+        return launch_split_bwd<decltype(m), decltype(width)::value, decltype(pad)::value>(p, st);
+    });
+}
+
+}  // namespace sa2
