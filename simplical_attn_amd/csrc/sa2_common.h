@@ -27,6 +27,7 @@ struct Problem {
     float* dsum;                     // [B,H,N]  sum_d dout*out
     void* scratch;                   // remaining workspace (path specific)
     size_t scratch_bytes;
+    int nsplit;                      // forward: shares of the rounds (partial outputs in `scratch` when more than one)
     int force_prepass;               // take the pre-pass kernels whenever the window allows, whatever the size
 };
 
@@ -59,6 +60,14 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
+// Workgroups are dealt round-robin to the 8 XCDs, each with its own L2: gives every XCD a run of consecutive work items,
+// so that neighbours in the problem (which share most of their K/V window) meet in one L2.  A permutation of
+// 0 .. total-1 for every total.
+__device__ __forceinline__ int xcd_order(int pid, int total) {
+    const int x = pid & 7, each = total >> 3, more = total & 7;
+    return x * each + (x < more ? x : more) + (pid >> 3);
+}
+
 // log(sum_w + 1e-8) from the running maximum m and l = sum exp(s-m), for any m.
 __device__ __forceinline__ float lse_with_eps(float m, float l) {
     const float log_eps = -18.420680743952367f;   // log(1e-8)
@@ -72,37 +81,91 @@ __device__ __forceinline__ float lse_with_eps(float m, float l) {
 constexpr int LDS_BYTES_PER_CU = 160 * 1024;
 bool allow_full_lds(const void* kernel);
 
-// How a K'-side launch cuts the K' window: segw deltas per segment, nseg segments, one workgroup per (K' block, segment).
+// ---- how a launch divides its work ------------------------------------------
+// The kernels keep one workgroup per CU, so a grid runs in waves of 256 workgroups: every whole wave takes the mean
+// workgroup's time, what is left over mostly the longest's, and the grid ends no sooner than that one.  Where a grid is
+// smaller than the chip, or its last wave nearly empty, or its workgroups uneven (short ones at the ends of the
+// sequence), the plans below cut the work of a workgroup into shares with fp32 partial sums, which cost their write and
+// read (2.5 MB per unit of time, a sweep step of about 1 us) and a summation launch.  The constants are the ones whose
+// choices lost least against the best of up to sixteen measured cuts at nineteen sizes (1.0 % for the K-side kernel,
+// 2.6 % for the K'-side one).  All plans depend on the problem's sizes only.
+constexpr int CUS = 256;
+inline double grid_time(int64_t workgroups, double longest, double mean) {
+    const int64_t waves = workgroups / CUS;
+    const double t = (double)waves * mean + (workgroups - waves * CUS > 2 ? 0.7 * longest + 0.3 * mean : 0.0);
+    return t > longest ? t : longest;
+}
+// mean over the sequence of min(i, w) / w
+inline double window_fill(int w, int N) { return w < N ? 1.0 - 0.5 * w / N : 0.5 * N / w; }
+constexpr double PART_BYTES_PER_STEP = 2.5e6, SUM_LAUNCH_STEPS = 8;
+
+// The K' window in nseg segments of segw deltas, one workgroup per (K' block, segment)
 struct KpPlan {
     int segw, nseg;
 };
-// One workgroup fills a CU.  A segment costs its rounds of `upr` deltas (each the tiles of the K window plus the work
-// between two sweeps, about two tiles' time) and about six tiles' time of prologue and epilogue; its partial sums
-// (bytes(plan)) are written once and read once (5 MB take about a tile's time).  The plan is the cut for which waves of
-// workgroups x cost of one is least, among segments of at most `most` deltas (what LDS holds); grids of four waves and
-// more are cut only where LDS asks for it (the tail of the last wave is below what a cut costs), and a cut for the
-// grid's sake never takes more than a quarter of SA2_STATIC_WORKSPACE_BYTES.
-// Measured on the 16-bit kernel: B2 H4 N512 D64 w 256/256 (128 blocks) 625 -> 349 us with two segments,
-// B2 H4 N256 D64 w 32/32 (64 blocks) 40 -> 23 us with three.
-template <class F>
-KpPlan plan_segments(int B, int N, int H, int w1, int w2, int upr, int most, F&& bytes) {
-    constexpr int CUS = 256, ROWS = 32;
+// Segments are whole rounds of `upr` deltas, at most `most` deltas (what LDS holds).  A round sweeps the tiles of the K
+// window; the work between two sweeps takes about two tiles' time, or five and a half where the rows of q and dO do not
+// fit LDS beside the accumulator (raw(segment)), prologue and epilogue about eight.  bytes(plan): all partial sums; a cut may
+// take 32 MiB, or three times what the uncut launch needs.
+// Measured on the 16-bit kernel (us, uncut -> planned): B2 H4 N512 D64 w 256/256 607 -> 234 (seven segments),
+// B3 H21 N282 D128 w 176/48 488 -> 303 (three), B1 H8 N4096 D128 w 128/64 862 -> 655 (two: the rows then fit LDS),
+// B2 H4 N256 D64 w 32/32 43 -> 29 (three).
+template <class Raw, class Bytes>
+KpPlan plan_segments(int B, int N, int H, int w1, int w2, int upr, int most, Raw&& raw, Bytes&& bytes) {
+    constexpr int ROWS = 32, MOST_SEGMENTS = 16;
     const int64_t base = (int64_t)B * H * ((N + ROWS - 1) / ROWS);
+    const int rounds = (w2 + upr) / upr;
+    const double tiles = ((w1 < N ? w1 : N) + ROWS + upr) / (double)ROWS + 1, fill = window_fill(w1, N) * window_fill(w2, N);
     KpPlan best = most > w2 ? KpPlan{w2 + 1, 1} : KpPlan{most, (w2 + most) / most};
-    if (base * best.nseg >= 4 * CUS) return best;
-    const int rounds = (w2 + upr) / upr, tiles = ((w1 < N ? w1 : N) + 2 * ROWS + upr - 1) / ROWS + 2, longest = (best.segw + upr - 1) / upr;
+    const double first_bytes = (double)bytes(best), cap = 3 * first_bytes > 33554432.0 ? 3 * first_bytes : 33554432.0;
     double least = 0;
-    for (int per = longest; per >= 1; --per) {                                   // rounds per segment
-        const KpPlan pl = per == longest ? best : KpPlan{per * upr, (rounds + per - 1) / per};
+    for (int nseg = best.nseg, last = 0; nseg <= MOST_SEGMENTS || least == 0; ++nseg) {
+        const int per = (rounds + nseg - 1) / nseg;                                  // rounds per segment
+        if (per == last || per < 1) continue;
+        last = per;
+        const KpPlan pl = least == 0 ? best : KpPlan{per * upr, (rounds + per - 1) / per};
         const double part = (double)bytes(pl);
-        const double cost = (double)((base * pl.nseg + CUS - 1) / CUS) * (per * tiles + 6) + 2 * part / 5e6;
-        if (per == longest) least = cost;
-        else if (cost < 0.95 * least && part <= (double)(SA2_STATIC_WORKSPACE_BYTES / 4)) {
+        if (least != 0 && part > cap) break;
+        const double sweep = per * (tiles + (raw(pl.segw) ? 2.0 : 5.5));
+        const double cost = grid_time(base * pl.nseg, sweep + 8, sweep * fill + 8) + part / PART_BYTES_PER_STEP;
+        if (least == 0 || cost < least) {
             least = cost;
             best = pl;
         }
+        if (per == 1) break;
     }
     return best;
+}
+
+// A forward launch in nsplit shares of the rounds of `upr` deltas: fp32 partial outputs in the workspace.  A round takes
+// about three tiles' time beside its sweep, prologue and epilogue about eight.  Fewer than four rounds are not worth a
+// summation launch.
+inline int plan_forward(int B, int N, int H, int width, int w1, int w2, int upr) {
+    constexpr int ROWS = 32, MOST = 16;
+    const int64_t rows = (int64_t)B * H * N, base = (int64_t)B * H * ((N + ROWS - 1) / ROWS);
+    const int rounds = ((w2 < N - 1 ? w2 : N - 1) + upr) / upr;
+    if (rounds < 4 || base >= 4 * CUS) return 1;
+    const double tiles = ((w1 < N ? w1 : N) + ROWS) / (double)ROWS + 1, fill = window_fill(w1, N) * window_fill(w2, N);
+    int best = 1;
+    double least = 0;
+    for (int ns = 1, last = 0; ns <= MOST && ns <= rounds; ++ns) {
+        const int per = (rounds + ns - 1) / ns;
+        if (per == last) continue;
+        last = per;
+        const int shares = (rounds + per - 1) / per;
+        const double part = shares > 1 ? (double)shares * rows * (width + 2) * 4 : 0;
+        if (part > 67108864.0) break;
+        const double sweep = per * (tiles + 3);
+        const double cost = grid_time(base * shares, sweep + 8, sweep * fill + 8) + (shares > 1 ? SUM_LAUNCH_STEPS + part / PART_BYTES_PER_STEP : 0);
+        if (least == 0 || cost < 0.95 * least) {
+            least = cost;
+            best = shares;
+        }
+    }
+    return best;
+}
+inline size_t fwd_part_bytes(int B, int N, int H, int width, int nsplit) {
+    return nsplit > 1 ? (size_t)nsplit * B * H * (size_t)N * (width + 2) * sizeof(float) : 0;
 }
 
 // ---- launchers (each returns a sa2_status) ----------------------------------
@@ -116,6 +179,8 @@ bool mfma_supported(int B, int N, int H, int D, int w1, int w2, int dtype);
 bool mfma_bwd_supported(int B, int N, int H, int D, int w1, int w2, int dtype);
 bool mfma_layout_ok(const Problem& p, bool backward);
 int launch_mfma_fwd(const Problem& p, int dtype, hipStream_t st);
+int mfma_fwd_nsplit(int B, int N, int H, int D, int w1, int w2);
+size_t mfma_fwd_part_bytes(int B, int N, int H, int D, int nsplit);
 int launch_mfma_bwd(const Problem& p, int dtype, hipStream_t st);
 size_t mfma_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2);
 // fp32 arithmetic on the fp32 MFMA: fp32 tensors of any head_dim up to 128 that is a multiple of 4, and 16-bit tensors
@@ -125,6 +190,8 @@ bool f32_mfma_bwd_supported(int D, int w2, int dtype);
 bool f32_mfma_layout_ok(const Problem& p, int dtype, bool backward);
 size_t f32_mfma_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2, int dtype);
 int launch_f32_mfma_fwd(const Problem& p, int dtype, hipStream_t st);
+int f32_mfma_fwd_nsplit(int B, int N, int H, int D, int w1, int w2);
+size_t f32_mfma_fwd_part_bytes(int B, int N, int H, int D, int nsplit);
 int launch_f32_mfma_bwd(const Problem& p, int dtype, hipStream_t st);
 // 16-bit tensors with head_dim 256 on the 16-bit MFMA (rows 16-byte aligned)
 bool wide_supported(int D, int dtype);
@@ -132,6 +199,9 @@ bool wide_bwd_supported(int D, int w2, int dtype);
 size_t wide_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2);
 int launch_wide_fwd(const Problem& p, int dtype, hipStream_t st);
 int launch_wide_bwd(const Problem& p, int dtype, hipStream_t st);
+// Partial outputs of a split forward, [nsplit][B*H*N] pairs (reference exponent M, sum L) and then
+// [nsplit][B*H*N][width] sums at that reference, merged into out and lse in share order
+int launch_fwd_merge(const Problem& p, int width, int dtype, hipStream_t st);
 // K'-side backward kernel (dQ, dK', dV') that keeps its partial sums on chip (K' windows too wide for
 // that are cut into segments of deltas, one workgroup each)
 size_t kp_scratch_bytes(int B, int N, int H, int D, int w1, int w2);

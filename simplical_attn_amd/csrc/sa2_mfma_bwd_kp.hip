@@ -134,8 +134,7 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
     // to the same XCD.
     const int per_seg = SEG ? total / nseg : total;
     const int seg = SEG ? (int)blockIdx.x / per_seg : 0;
-    int pb = SEG ? (int)blockIdx.x - seg * per_seg : (int)blockIdx.x;
-    if ((per_seg & 7) == 0) pb = (pb & 7) * (per_seg >> 3) + (pb >> 3);
+    const int pb = xcd_order(SEG ? (int)blockIdx.x - seg * per_seg : (int)blockIdx.x, per_seg);
     // (in the pre-pass nkb counts groups of four K' blocks and k0 belongs to the pair)
     const int bh = pb / nkb, kb = LEFT ? (pb - bh * nkb) * NPAIR + pr : pb - bh * nkb;
     const int b = bh / p.H, h = bh - b * p.H;
@@ -837,7 +836,7 @@ KpPlan kp_plan_of(int B, int N, int H, int w1, int w2) {
     if (C::fits(w2)) most = w2 + 1;
     else
         while (C::fits(most + UPR - 1)) most += UPR;
-    return plan_segments(B, N, H, w1, w2, UPR, most,
+    return plan_segments(B, N, H, w1, w2, UPR, most, [](int segw) { return C::raw_fits(segw - 1); },
                          [&](const KpPlan& pl) { return kp_dq_part_bytes(B, N, H, D, pl) + kp_part_bytes(B, N, H, D, pl); });
 }
 KpPlan kp_plan(int B, int N, int H, int D, int w1, int w2) {

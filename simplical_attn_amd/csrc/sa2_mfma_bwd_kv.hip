@@ -1,6 +1,6 @@
 // MFMA backward for gfx950 (bf16 or fp16 elements), the K-side kernel: dK and dV.
 //
-// A workgroup owns 128 consecutive K/V rows, 32 per wavefront pair (at head_dim 64, where the
+// A workgroup owns 128 consecutive K/V rows, 32 per wavefront pair (at head_dim 32 and 64, where the
 // registers allow it and the grid stays large enough: 256 rows, two 32-row blocks per pair, so
 // that a unit's forming, its operand reads and the step's barrier serve twice the MFMAs),
 // resident in registers as MFMA B operands.  It streams every unit of expanded rows that can see them: unit
@@ -16,7 +16,7 @@
 // Every output element has one writer and a fixed summation order.
 //
 // Small grids (fewer workgroups than the chip holds) split a key block's stream of units over up to
-// sixteen workgroups (shares of whole units, at least eight each); each writes its fp32 partial dK and
+// sixteen workgroups (shares of whole units, at least four each); each writes its fp32 partial dK and
 // dV to the workspace and bwd_sum_kernel adds the partials in split order.
 #include <type_traits>
 
@@ -29,8 +29,7 @@ constexpr int VW = 8;                  // wavefronts per workgroup
 constexpr int VT = VW * 64;            // threads per workgroup
 constexpr int VPAIR = 4;
 constexpr int KV_MAX_SPLIT = 16;       // workgroups a key block's stream of units is split over, at most
-constexpr int KV_MIN_SHARE = 8;        // units a share holds at least
-constexpr int KV_GRID_TARGET = 512;    // a split stops once the grid holds this many workgroups
+constexpr int KV_MIN_SHARE = 4;        // units a share holds at least
 
 // KB: 32-row blocks of K/V rows per wavefront pair
 template <int D, int KB>
@@ -94,8 +93,7 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __
     const int role = wave >> 2, pr = wave & 3;
     const int lane = tid & 63, ln = lane & 31, hf = lane >> 5;
 
-    int pid = blockIdx.x;
-    if ((total & 7) == 0) pid = (pid & 7) * (total >> 3) + (pid >> 3);
+    const int pid = xcd_order(blockIdx.x, total);
     const int sp = pid % nsplit, pj = pid / nsplit;
     const int bh = pj / njb, jb = pj - bh * njb;
     const int b = bh / p.H, h = bh - b * p.H;
@@ -477,26 +475,48 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __
     }
 }
 
-// Geometry of a launch: 32-row K blocks per wavefront pair, and the number of shares a key block's
-// stream of units is split into.  Both depend on the problem's sizes only.
+// Geometry of a launch: 32-row K blocks per wavefront pair, and the number of shares a key block's stream of units is split
+// into, by grid_time.  A unit (about a step's time) costs 1.55 times as much with two K blocks per pair, whose operand
+// reads and barriers then serve twice the MFMAs, 1.1 times with one in a split launch; prologue and epilogue take about 16.  The partial sums stay under what
+// SA2_STATIC_WORKSPACE_BYTES leaves beside the K'-side kernel's, or 128 MiB where those alone exceed it.
+// Measured on this kernel (us, one K block unsplit -> planned): B2 H4 N512 D64 w 256/256 2259 -> 257, B3 H6 N777 D64 w 100/20
+// 164 -> 99, B2 H8 N2048 D64 w 512/32 508 -> 457, B5 H29 N448 D32 w 816/96 2386 -> 1183, B1 H4 N2048 D128 w 512/32 667 -> 199.
 struct KvPlan {
     int kb, nsplit;
 };
 KvPlan kv_plan(int B, int N, int H, int D, int w1, int w2) {
-    KvPlan pl{1, 1};
+    KvPlan best{1, 1};
     const int64_t bh = (int64_t)B * H;
-    // two K blocks per pair at head_dim 64 when that still leaves a grid worth splitting no further than in two
-    if (D == 64 && bh * ((N + 255) / 256) * 2 >= KV_GRID_TARGET / 2) pl.kb = 2;
-    const int vj = VPAIR * 32 * pl.kb;
-    const int64_t base = bh * ((N + vj - 1) / vj);
-    const int blocks = (vj + (w1 < N ? w1 : N) + BQ - 1) / BQ + 1;          // query blocks a key block streams, at most
-    // (the partial sums of a split launch stay under 32 MiB)
-    auto part_bytes = [&](int ns) { return (int64_t)2 * ns * bh * N * D * 4; };
-    const int64_t units = (int64_t)blocks * ((w2 < N - 1 ? w2 : N - 1) + 1);     // of a key block's stream, at most
-    while (pl.nsplit < KV_MAX_SPLIT && base * pl.nsplit * 2 <= KV_GRID_TARGET && (int64_t)pl.nsplit * 2 * KV_MIN_SHARE <= units &&
-           part_bytes(pl.nsplit * 2) <= ((int64_t)32 << 20))
-        pl.nsplit *= 2;
-    return pl;
+    const int per = (w2 < N - 1 ? w2 : N - 1) + 1;                                   // units of a query block, at most
+    const double other = (double)kp_side_scratch_bytes(B, N, H, D, w1, w2) + (double)bh * N * 4 + 1024;
+    const double cap = other < (double)SA2_STATIC_WORKSPACE_BYTES ? (double)SA2_STATIC_WORKSPACE_BYTES - other : 134217728.0;
+    double least = 0;
+    for (int kb = 1; kb <= (D <= 64 ? 2 : 1); ++kb) {
+        const int vj = VPAIR * 32 * kb, njb = (N + vj - 1) / vj;
+        const int64_t base = bh * njb;
+        // query blocks a key block streams: at most, and on average (fewer at the end of the sequence)
+        const int nqb = (N + BQ - 1) / BQ;
+        int blocks = (vj + (w1 < N ? w1 : N) + BQ - 1) / BQ + 1;
+        blocks = blocks < nqb ? blocks : nqb;
+        double mean_blocks = 0;
+        const int sampled = njb < 64 ? njb : 64;
+        for (int x = 0; x < sampled; ++x) {
+            const int64_t jb = (int64_t)x * njb / sampled, last = jb * vj + vj - 1 + w1;
+            mean_blocks += (double)((last < N - 1 ? last : N - 1) / BQ - jb * vj / BQ + 1) / sampled;
+        }
+        const double longest = (double)blocks * per, mean = mean_blocks * per * window_fill(w2, N);
+        for (int ns = 1; ns <= KV_MAX_SPLIT; ++ns) {
+            const double part = ns > 1 ? 2.0 * ns * bh * N * D * 4 : 0;
+            if (ns > 1 && (base * ns > 16 * CUS || (int64_t)blocks * per / ns < KV_MIN_SHARE || part > cap)) break;
+            const double unit = kb == 2 ? 1.55 : ns > 1 ? 1.1 : 1.0;
+            const double cost = grid_time(base * ns, longest * unit / ns + 16, mean * unit / ns + 16) + (ns > 1 ? SUM_LAUNCH_STEPS + part / PART_BYTES_PER_STEP : 0);
+            if (least == 0 || cost < least) {
+                least = cost;
+                best = KvPlan{kb, ns};
+            }
+        }
+    }
+    return best;
 }
 
 template <class E, int D, int KB, bool PAD>
@@ -541,7 +561,7 @@ int launch_kv_geometry(const Problem& p, int nsplit, hipStream_t st, BwdSums* su
 template <class E, int D, bool PAD>
 int launch_kv(const Problem& p, hipStream_t st, BwdSums* sums) {
     const KvPlan pl = kv_plan(p.B, p.N, p.H, D, p.w1, p.w2);
-    if constexpr (D == 64) {
+    if constexpr (D <= 64) {
         if (pl.kb == 2) return launch_kv_geometry<E, D, 2, PAD>(p, pl.nsplit, st, sums);
     }
     return launch_kv_geometry<E, D, 1, PAD>(p, pl.nsplit, st, sums);

@@ -146,11 +146,7 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63, ln = lane & 31, hf = lane >> 5;
 
-    // Workgroups are dealt round-robin to the 8 XCDs; remap so that the
-    // neighbouring query blocks of one head (which share almost all of their
-    // K/V window) run on the same XCD and meet in its L2.
-    int pid = blockIdx.x;
-    if ((total & 7) == 0) pid = (pid & 7) * (total >> 3) + (pid >> 3);
+    const int pid = xcd_order(blockIdx.x, total);
     // (in the pre-pass nqb counts groups of eight query blocks)
     const int bh = pid / nqb, qb = LEFT ? (pid - bh * nqb) * FW + wave : pid - bh * nqb;
     const int b = bh / p.H, h = bh - b * p.H;

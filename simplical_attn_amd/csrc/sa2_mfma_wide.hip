@@ -70,11 +70,6 @@ __device__ __forceinline__ floatx16 zeros16() {
     for (int v = 0; v < 16; ++v) z[v] = 0.f;
     return z;
 }
-__device__ __forceinline__ int xcd_neighbours(int pid, int total) {
-    // workgroups are dealt round-robin to the 8 XCDs: neighbours in the problem share an L2
-    return (total & 7) == 0 ? (pid & 7) * (total >> 3) + (pid >> 3) : pid;
-}
-
 // Rows [j0, j0+32) of two tensors (clamped to the sequence) from global memory to registers, and
 // from there to the two tiles of a stage.
 template <int D, int DV, int KR>
@@ -151,7 +146,7 @@ void wide_fwd_kernel(Problem p, int nqb, int total) {
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63, ln = lane & 31, hf = lane >> 5;
-    const int pid = xcd_neighbours(blockIdx.x, total);
+    const int pid = xcd_order(blockIdx.x, total);
     const int c0 = blockIdx.y * DV;                          // this pass's output columns
     const int bh = pid / nqb, qb = pid - bh * nqb;
     const int b = bh / p.H, h = bh - b * p.H;
@@ -356,7 +351,7 @@ void wide_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_part, 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63, ln = lane & 31, hf = lane >> 5;
-    const int pid = xcd_neighbours(blockIdx.x, total);
+    const int pid = xcd_order(blockIdx.x, total);
     const int c0 = blockIdx.y * DV;
     const int bh = pid / nkb, kb = pid - bh * nkb;
     const int b = bh / p.H, h = bh - b * p.H;
@@ -603,7 +598,7 @@ void wide_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __rest
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63, ln = lane & 31, hf = lane >> 5;
-    const int pid = xcd_neighbours(blockIdx.x, total);
+    const int pid = xcd_order(blockIdx.x, total);
     const int c0 = blockIdx.y * DV;
     const int sp = pid % nsplit, pj = pid / nsplit;
     const int bh = pj / njb, jb = pj - bh * njb;

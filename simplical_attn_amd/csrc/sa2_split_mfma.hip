@@ -78,11 +78,6 @@ __device__ __forceinline__ floatx16 zero16() {
     for (int v = 0; v < 16; ++v) z[v] = 0.f;
     return z;
 }
-__device__ __forceinline__ int xcd_order(int pid, int total) {
-    // workgroups are dealt round-robin to the 8 XCDs: neighbours in the problem share an L2
-    return (total & 7) == 0 ? (pid & 7) * (total >> 3) + (pid >> 3) : pid;
-}
-
 typedef float fx4 __attribute__((ext_vector_type(4)));      // 16 bytes in flight (plain vectors: stay in registers)
 typedef unsigned ux2 __attribute__((ext_vector_type(2)));
 
@@ -991,7 +986,7 @@ KpPlan split_kp_plan(int B, int N, int H, int w1, int w2) {
     using C = SplitCfg<T, D>;
     int most = NPAIR;
     while (most < w2 + 1 && C::kp_fits(most + NPAIR - 1)) most += NPAIR;
-    return plan_segments(B, N, H, w1, w2, NPAIR, most, [&](const KpPlan& pl) { return split_kp_bytes(B, N, H, D, pl); });
+    return plan_segments(B, N, H, w1, w2, NPAIR, most, [](int) { return false; }, [&](const KpPlan& pl) { return split_kp_bytes(B, N, H, D, pl); });
 }
 
 // ------------------------------------------------------------------ launchers ----
