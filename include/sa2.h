@@ -92,6 +92,20 @@ int sa2_forward(const void* q, const void* k1, const void* k2, const void* v1, c
                 int w1, int w2, float scale, float k2_bias, float v2_bias,
                 int dtype, int window_inclusive, unsigned flags, void* hip_stream);
 
+/*
+ * sa2_forward with device workspace.  Where the query blocks alone leave the chip idle (short sequences, few
+ * heads, wide K' windows) the rounds of a block are then shared by several workgroups, whose partial outputs go
+ * through the workspace; elsewhere it is not touched.  workspace: sa2_fwd_workspace_bytes(...) bytes, 256-byte
+ * aligned, contents on entry ignored; NULL: as sa2_forward.  sa2_fwd_workspace_bytes returns 0 where none is used.
+ */
+int sa2_forward_ws(const void* q, const void* k1, const void* k2, const void* v1, const void* v2,
+                   void* out, float* lse, void* workspace, size_t workspace_bytes,
+                   int B, int N, int H, int D,
+                   const int64_t* strides,
+                   int w1, int w2, float scale, float k2_bias, float v2_bias,
+                   int dtype, int window_inclusive, unsigned flags, void* hip_stream);
+size_t sa2_fwd_workspace_bytes(int B, int N, int H, int D, int w1, int w2, int dtype, int window_inclusive, unsigned flags);
+
 /* Bytes of device workspace sa2_backward needs for this problem, whichever of the two window
  * conventions the call then uses with these w1 and w2 (0 is never returned for a valid problem;
  * returns 0 for an invalid one). */

@@ -8,7 +8,7 @@ LIB_PATH = os.environ.get("SA2_LIBRARY", os.path.join(_PKG, "lib", "libsa2_hip.s
 
 # Symbols include/sa2.h declares; the ABI test checks that all of them resolve.
 EXPORTED_SYMBOLS = (
-    "sa2_version", "sa2_strerror", "sa2_uses_mfma", "sa2_forward",
+    "sa2_version", "sa2_strerror", "sa2_uses_mfma", "sa2_forward", "sa2_forward_ws", "sa2_fwd_workspace_bytes",
     "sa2_bwd_workspace_bytes", "sa2_backward", "sa2_backward_static_workspace", "sa2_rowdot",
 )
 STATIC_WORKSPACE_BYTES = 64 << 20
@@ -49,6 +49,11 @@ def load():
     lib.sa2_forward.restype = c_int
     lib.sa2_forward.argtypes = ([c_void_p] * 7 + [c_int] * 4 + [i64p] + [c_int, c_int, c_float, c_float, c_float]
                                 + [c_int, c_int, c_uint, c_void_p])
+    lib.sa2_forward_ws.restype = c_int
+    lib.sa2_forward_ws.argtypes = ([c_void_p] * 8 + [c_size_t] + [c_int] * 4 + [i64p] + [c_int, c_int, c_float, c_float, c_float]
+                                   + [c_int, c_int, c_uint, c_void_p])
+    lib.sa2_fwd_workspace_bytes.restype = c_size_t
+    lib.sa2_fwd_workspace_bytes.argtypes = [c_int] * 8 + [c_uint]
     lib.sa2_bwd_workspace_bytes.restype = c_size_t
     lib.sa2_bwd_workspace_bytes.argtypes = [c_int] * 7 + [c_uint]
     lib.sa2_backward.restype = c_int
@@ -81,8 +86,8 @@ def host():
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)
         address = lambda f: ctypes.cast(f, ctypes.c_void_p).value
-        module.bind(address(lib.sa2_forward), address(lib.sa2_backward), address(lib.sa2_bwd_workspace_bytes),
-                    address(lib.sa2_strerror), simplicial_attn._check_inputs, simplicial_attn._check_saved, Sa2Error)
+        module.bind(address(lib.sa2_forward_ws), address(lib.sa2_fwd_workspace_bytes), address(lib.sa2_backward),
+                    address(lib.sa2_bwd_workspace_bytes), address(lib.sa2_strerror), simplicial_attn._check_inputs, simplicial_attn._check_saved, Sa2Error)
         _host = module
     return _host
 

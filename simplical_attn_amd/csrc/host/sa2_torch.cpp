@@ -22,7 +22,8 @@ using at::Tensor;
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
-decltype(&sa2_forward) fwd_fn = nullptr;
+decltype(&sa2_forward_ws) fwd_fn = nullptr;
+decltype(&sa2_fwd_workspace_bytes) fwd_ws_fn = nullptr;
 decltype(&sa2_backward) bwd_fn = nullptr;
 decltype(&sa2_bwd_workspace_bytes) ws_fn = nullptr;
 decltype(&sa2_strerror) err_fn = nullptr;
@@ -81,11 +82,13 @@ std::pair<Tensor, Tensor> run_forward(const Tensor& q_, const Tensor& k1_, const
     const int64_t B = q.size(0), N = q.size(1), H = q.size(2), D = q.size(3);
     Tensor out = at::empty({B, N, H, D}, q.options().requires_grad(false));
     Tensor lse = at::empty({B, H, N}, q.options().dtype(at::kFloat).requires_grad(false));
+    const size_t bytes = fwd_ws_fn((int)B, (int)N, (int)H, (int)D, (int)a.w1, (int)a.w2, dtype_code(q), a.inclusive ? 1 : 0, a.flags);
+    const Tensor ws = bytes ? at::empty({(int64_t)bytes}, lse.options().dtype(at::kByte)) : Tensor();
     int64_t s[3 * SA2_FWD_TENSORS];
     const Tensor* const t[SA2_FWD_TENSORS] = {&q, &k1, &k2, &v1, &v2, &out};
     for (int i = 0; i < SA2_FWD_TENSORS; ++i) put_strides(s + 3 * i, *t[i]);
-    check(fwd_fn(q.data_ptr(), k1.data_ptr(), k2.data_ptr(), v1.data_ptr(), v2.data_ptr(), out.data_ptr(), (float*)lse.data_ptr(), (int)B, (int)N,
-                 (int)H, (int)D, s, (int)a.w1, (int)a.w2, (float)a.scale, (float)a.k2_bias, (float)a.v2_bias, dtype_code(q), a.inclusive ? 1 : 0,
+    check(fwd_fn(q.data_ptr(), k1.data_ptr(), k2.data_ptr(), v1.data_ptr(), v2.data_ptr(), out.data_ptr(), (float*)lse.data_ptr(),
+                 bytes ? ws.data_ptr() : nullptr, bytes, (int)B, (int)N, (int)H, (int)D, s, (int)a.w1, (int)a.w2, (float)a.scale, (float)a.k2_bias, (float)a.v2_bias, dtype_code(q), a.inclusive ? 1 : 0,
                  a.flags, (void*)c10::hip::getCurrentHIPStream(q.device().index()).stream()));
     return {out, lse};
 }
@@ -199,8 +202,9 @@ py::tuple backward(const Tensor& q, const Tensor& k1, const Tensor& k2, const Te
 
 PYBIND11_MODULE(_sa2_torch, m) {
     m.doc() = "Native host path of the 2-simplicial attention operator";
-    m.def("bind", [](uintptr_t fwd, uintptr_t bwd, uintptr_t ws, uintptr_t err, py::object check_inputs, py::object check_saved, py::object error) {
+    m.def("bind", [](uintptr_t fwd, uintptr_t fwd_ws, uintptr_t bwd, uintptr_t ws, uintptr_t err, py::object check_inputs, py::object check_saved, py::object error) {
         fwd_fn = (decltype(fwd_fn))fwd;
+        fwd_ws_fn = (decltype(fwd_ws_fn))fwd_ws;
         bwd_fn = (decltype(bwd_fn))bwd;
         ws_fn = (decltype(ws_fn))ws;
         err_fn = (decltype(err_fn))err;

@@ -179,10 +179,30 @@ int sa2_forward(const void* q, const void* k1, const void* k2, const void* v1, c
                 void* out, float* lse, int B, int N, int H, int D, const int64_t* strides,
                 int w1, int w2, float scale, float k2_bias, float v2_bias,
                 int dtype, int window_inclusive, unsigned flags, void* hip_stream) {
+    return sa2_forward_ws(q, k1, k2, v1, v2, out, lse, nullptr, 0, B, N, H, D, strides, w1, w2, scale, k2_bias, v2_bias, dtype,
+                          window_inclusive, flags, hip_stream);
+}
+
+size_t sa2_fwd_workspace_bytes(int B, int N, int H, int D, int w1, int w2, int dtype, int window_inclusive, unsigned flags) {
+    if (check_dims(B, N, H, D, w1, w2, dtype, window_inclusive) != SA2_OK || (flags & SA2_FLAG_FORCE_GENERIC)) return 0;
+    w1 = reach(w1, window_inclusive, N);
+    w2 = reach(w2, window_inclusive, N);
+    if (f32_mfma_supported(D, dtype)) return f32_mfma_fwd_part_bytes(B, N, H, D, f32_mfma_fwd_nsplit(B, N, H, D, w1, w2));
+    if (mfma_supported(B, N, H, D, w1, w2, dtype))
+        return mfma_fwd_part_bytes(B, N, H, D, mfma_fwd_nsplit(B, N, H, D, w1, w2, (flags & SA2_FLAG_FORCE_MFMA) != 0));
+    return 0;
+}
+
+int sa2_forward_ws(const void* q, const void* k1, const void* k2, const void* v1, const void* v2,
+                   void* out, float* lse, void* workspace, size_t workspace_bytes,
+                   int B, int N, int H, int D, const int64_t* strides,
+                   int w1, int w2, float scale, float k2_bias, float v2_bias,
+                   int dtype, int window_inclusive, unsigned flags, void* hip_stream) {
     if (!q || !k1 || !k2 || !v1 || !v2 || !out || !lse || !strides) return SA2_ERR_NULL_POINTER;
     int rc = check_dims(B, N, H, D, w1, w2, dtype, window_inclusive);
     if (rc != SA2_OK) return rc;
     if (!strides_ok(strides, SA2_FWD_TENSORS, B, N, H)) return SA2_ERR_BAD_STRIDE;
+    if ((uintptr_t)workspace & 255u) return SA2_ERR_WORKSPACE_TOO_SMALL;
 
     Problem p;
     memset(&p, 0, sizeof(p));
@@ -203,6 +223,18 @@ int sa2_forward(const void* q, const void* k1, const void* k2, const void* v1, c
     hipStream_t st = (hipStream_t)hip_stream;
     const KernelPath path = pick_path(p, dtype, flags, false, &rc);
     if (rc != SA2_OK) return rc;
+    // shares of the rounds, where the caller brought room for their partial outputs
+    p.nsplit = 1;
+    if (workspace) {
+        const int ns = path == PATH_MFMA16   ? mfma_fwd_nsplit(B, N, H, D, p.w1, p.w2, p.force_prepass != 0)
+                       : path == PATH_MFMA32 ? f32_mfma_fwd_nsplit(B, N, H, D, p.w1, p.w2)
+                                             : 1;
+        const size_t need = path == PATH_MFMA32 ? f32_mfma_fwd_part_bytes(B, N, H, D, ns) : mfma_fwd_part_bytes(B, N, H, D, ns);
+        if (ns > 1 && workspace_bytes < need) return SA2_ERR_WORKSPACE_TOO_SMALL;
+        p.nsplit = ns;
+        p.scratch = workspace;
+        p.scratch_bytes = workspace_bytes;
+    }
     return path == PATH_MFMA16 ? launch_mfma_fwd(p, dtype, st)
            : path == PATH_WIDE16 ? launch_wide_fwd(p, dtype, st)
            : path == PATH_MFMA32 ? launch_f32_mfma_fwd(p, dtype, st) : launch_generic_fwd(p, dtype, st);

@@ -144,7 +144,7 @@ inline int plan_forward(int B, int N, int H, int width, int w1, int w2, int upr)
     constexpr int ROWS = 32, MOST = 16;
     const int64_t rows = (int64_t)B * H * N, base = (int64_t)B * H * ((N + ROWS - 1) / ROWS);
     const int rounds = ((w2 < N - 1 ? w2 : N - 1) + upr) / upr;
-    if (rounds < 4 || base >= 4 * CUS) return 1;
+    if (rounds < 4 || base >= 3 * CUS) return 1;
     const double tiles = ((w1 < N ? w1 : N) + ROWS) / (double)ROWS + 1, fill = window_fill(w1, N) * window_fill(w2, N);
     int best = 1;
     double least = 0;
@@ -179,7 +179,7 @@ bool mfma_supported(int B, int N, int H, int D, int w1, int w2, int dtype);
 bool mfma_bwd_supported(int B, int N, int H, int D, int w1, int w2, int dtype);
 bool mfma_layout_ok(const Problem& p, bool backward);
 int launch_mfma_fwd(const Problem& p, int dtype, hipStream_t st);
-int mfma_fwd_nsplit(int B, int N, int H, int D, int w1, int w2);
+int mfma_fwd_nsplit(int B, int N, int H, int D, int w1, int w2, bool force_prepass);
 size_t mfma_fwd_part_bytes(int B, int N, int H, int D, int nsplit);
 int launch_mfma_bwd(const Problem& p, int dtype, hipStream_t st);
 size_t mfma_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2);

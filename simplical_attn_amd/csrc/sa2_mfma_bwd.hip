@@ -64,7 +64,54 @@ __global__ __launch_bounds__(256) void bwd_sum_kernel(Problem p, BwdSums s, int 
     else *(uint2*)((uint16_t*)t.p + t.off(b, i, h) + col) = make_uint2(E::pack(acc.x, acc.y), E::pack(acc.z, acc.w));
 }
 
+// out and LSE of a split forward: the shares' sums brought to a common reference exponent, in share order.  One
+// thread per four columns, four shares' reads in flight; bound by reading the partial outputs once.
+template <class E>
+__global__ __launch_bounds__(256) void fwd_merge_kernel(Problem p, int D, int64_t items) {
+    const int64_t it = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (it >= items) return;
+    const int col = (int)(it % (D / 4)) * 4;
+    if (col >= p.D) return;
+    const int64_t row = it / (D / 4), rows = (int64_t)p.B * p.H * p.N;
+    const float2* ml = (const float2*)p.scratch;                       // (M, L) of [share][row]
+    const float* part = (const float*)p.scratch + 2 * rows * p.nsplit;
+    float M = -INFINITY;
+#pragma unroll 4
+    for (int x = 0; x < p.nsplit; ++x) M = fmaxf(M, ml[x * rows + row].x);
+    const float Mu = M == -INFINITY ? 0.f : M;
+    float L = 0.f;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+    for (int x = 0; x < p.nsplit; ++x) {
+        const float2 s = ml[x * rows + row];
+        if (s.x == -INFINITY) continue;                                // (an empty share left no sums)
+        const float w = fast_exp2(s.x - Mu);
+        const float4 y = *(const float4*)(part + (x * rows + row) * D + col);
+        L += w * s.y;
+        acc.x += w * y.x; acc.y += w * y.y; acc.z += w * y.z; acc.w += w * y.w;
+    }
+    // sum + 1e-8 in units of 2^Mu; for a tiny Mu the epsilon dominates
+    const bool big = Mu > LOG2_EPS;
+    const float denom = big ? L + 1e-8f * fast_exp2(-Mu) : L * fast_exp2(Mu - LOG2_EPS) + 1.f;
+    const float inv = big ? 1.f / denom : fast_exp2(Mu - LOG2_EPS) / denom;
+    const int i = (int)(row % p.N), bh = (int)(row / p.N), b = bh / p.H, h = bh - b * p.H;
+    if constexpr (std::is_same<E, float>::value)
+        *(float4*)((float*)p.out.p + p.out.off(b, i, h) + col) = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+    else
+        *(uint2*)((uint16_t*)p.out.p + p.out.off(b, i, h) + col) = make_uint2(E::pack(acc.x * inv, acc.y * inv), E::pack(acc.z * inv, acc.w * inv));
+    if (col == 0) p.lse[row] = big ? LN2 * Mu + logf(denom) : LN_EPS + logf(denom);
+}
+
 }  // namespace
+
+int launch_fwd_merge(const Problem& p, int width, int dtype, hipStream_t st) {
+    const int64_t items = (int64_t)p.B * p.H * p.N * (width / 4);
+    const dim3 grid((unsigned)((items + 255) / 256));
+    if (dtype == SA2_F32) hipLaunchKernelGGL((fwd_merge_kernel<float>), grid, dim3(256), 0, st, p, width, items);
+    else if (dtype == SA2_F16) hipLaunchKernelGGL((fwd_merge_kernel<ElemF16>), grid, dim3(256), 0, st, p, width, items);
+    else hipLaunchKernelGGL((fwd_merge_kernel<ElemBF16>), grid, dim3(256), 0, st, p, width, items);
+    return hipGetLastError() == hipSuccess ? SA2_OK : SA2_ERR_LAUNCH_FAILED;
+}
 
 bool mfma_bwd_supported(int B, int N, int H, int D, int w1, int w2, int dtype) {
     return mfma_supported(B, N, H, D, w1, w2, dtype);

@@ -123,7 +123,9 @@ __device__ __forceinline__ void issue_v_all(uint32_t addr, lds_half_operand (&vh
 // SIDE: the K' and V' rows the block's deltas reach are copied to LDS (they fit); otherwise
 // they are read from global memory where they are needed.
 // PAD: the tensors have p.D <= D columns (see load_cols8).
-template <class E, int D, int MODE, bool SIDE, bool PAD>
+// SPLIT: the workgroup takes the rounds of one of nsplit shares of its query block and leaves its sums unnormalised in the
+// workspace (see launch_fwd_merge).
+template <class E, int D, int MODE, bool SIDE, bool PAD, bool SPLIT>
 __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, int left, int tid) {
     typedef typename E::scalar EL;
     typedef typename E::x8 X8;
@@ -146,7 +148,11 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63, ln = lane & 31, hf = lane >> 5;
 
-    const int pid = xcd_order(blockIdx.x, total);
+    int pid = xcd_order(blockIdx.x, total), share = 0;
+    if constexpr (SPLIT) {
+        share = pid % p.nsplit;
+        pid /= p.nsplit;
+    }
     // (in the pre-pass nqb counts groups of eight query blocks)
     const int bh = pid / nqb, qb = LEFT ? (pid - bh * nqb) * FW + wave : pid - bh * nqb;
     const int b = bh / p.H, h = bh - b * p.H;
@@ -170,8 +176,20 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
     // delta = 0 .. n_units-1; the fast kernel leaves delta = w2 to the pre-pass where that ran
     const bool has_left = left && i_last >= w2;
     const int n_units = LEFT ? 1 : (w2 < i_last ? w2 : i_last) + 1 - (has_left && !SAFE ? 1 : 0);
-    const int nrounds = (n_units + FW - 1) / FW;
-    const int total_steps = nrounds * nt;
+    const int all_rounds = (n_units + FW - 1) / FW;
+    const int per_share = SPLIT ? ((w2 + FW) / FW + p.nsplit - 1) / p.nsplit : all_rounds;
+    const int round0 = SPLIT ? share * per_share : 0;
+    const int round1 = round0 + per_share < all_rounds ? round0 + per_share : all_rounds;
+    const int total_steps = (round1 - round0) * nt;
+    if constexpr (SPLIT) {
+        if (round0 >= round1) {                  // a block near the start of the sequence has fewer rounds
+            if (tid < BQ && i0 + tid < N) {
+                const int64_t rows = (int64_t)p.B * p.H * N;
+                ((float2*)p.scratch)[share * rows + (int64_t)bh * N + i0 + tid] = make_float2(-INFINITY, 0.f);
+            }
+            return false;
+        }
+    }
     // tiles of the sweep that hold keys of this wavefront's rows (the whole sweep outside the pre-pass)
     const int ws0 = LEFT ? (i0 - w1 > 0 ? i0 - w1 : 0) / TJ - jt_lo : 0;
     const int ws1 = LEFT ? (i_last < 0 ? 0 : i_last) / TJ - jt_lo : nt - 1;
@@ -263,7 +281,9 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
     if (total_steps > 1) dma_next();
 
     // ---- q rows of the block and the K'/V' rows its deltas reach, once, to LDS ----
-    const int side_rows = BQ + w2;
+    // (rows i0 - dtop .. of the deltas of this workgroup's rounds)
+    const int dtop = SPLIT ? (round1 * FW - 1 < w2 ? round1 * FW - 1 : w2) : w2;
+    const int side_rows = BQ + (SPLIT ? dtop - round0 * FW : w2);
     uint16_t* v2_s = k2_s + side_rows * C::KS;
     if constexpr (!LEFT) {
         constexpr int CPR = D / 8;                 // 16-byte chunks per row
@@ -276,7 +296,7 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
         if constexpr (SIDE) {
             for (int c = tid; c < side_rows * CPR; c += FT) {
                 const int row = c / CPR, col = c - row * CPR;
-                int r = i0 - w2 + row;
+                int r = i0 - dtop + row;
                 r = r < 0 ? 0 : (r < N ? r : N - 1);
                 *(uint4*)(k2_s + row * C::KS + col * 8) = load_cols8<PAD>(k2p + (int64_t)r * p.k2.sn, col * 8, p.D);
                 *(uint4*)(v2_s + row * C::KS + col * 8) = load_cols8<PAD>(v2p + (int64_t)r * p.v2.sn, col * 8, p.D);
@@ -286,7 +306,7 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
     // K'/V' row of this lane's query for a given delta: LDS copy or global memory
     auto k2_row = [&](int delta) {
         if constexpr (SIDE) {
-            return (const uint16_t*)(k2_s + (ln + w2 - delta) * C::KS);       // row (i0 + ln - delta) - (i0 - w2)
+            return (const uint16_t*)(k2_s + (ln + dtop - delta) * C::KS);       // row (i0 + ln - delta) - (i0 - dtop)
         } else {
             const int k = ic - delta;
             return k2p + (int64_t)(k > 0 ? k : 0) * p.k2.sn;
@@ -338,7 +358,7 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
             for (int v = 0; v < 16; ++v) wacc[dt][v] = 0.f;
     }
 
-    for (int round = 0; round < nrounds; ++round) {
+    for (int round = round0; round < round1; ++round) {
         const int delta = LEFT ? w2 : round * FW + wave;
         const bool ok = LEFT ? (i0 < N && i_last >= w2) : delta < n_units;
         // The unit starts from the query's running reference point (finite from the second
@@ -711,7 +731,7 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
                 const int ln_u = tid_u & 31, hf_u = (tid_u >> 5) & 1;
                 const uint16_t* vrow;
                 if constexpr (SIDE) {
-                    vrow = v2_s + (ln_u + w2 - delta) * C::KS;
+                    vrow = v2_s + (ln_u + dtop - delta) * C::KS;
                 } else {
                     const int iq = i0 + ln_u < N ? i0 + ln_u : N - 1;
                     vrow = v2p + (int64_t)(iq - delta > 0 ? iq - delta : 0) * p.v2.sn;
@@ -764,7 +784,7 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
         // the V' row of this lane's query, read in one batch before the exchange below
         const uint16_t* vrow;
         if constexpr (SIDE) {
-            vrow = v2_s + (ok ? ln_m + w2 - delta : 0) * C::KS;
+            vrow = v2_s + (ok ? ln_m + dtop - delta : 0) * C::KS;
         } else {
             const int iq = i0 + ln_m < N ? i0 + ln_m : N - 1;
             const int vr = ok && iq - delta > 0 ? iq - delta : 0;
@@ -957,6 +977,14 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
     const int io = i0 + aq;
     if (io < N) {
         const float Ms = fin_m[aq], L = fin_l[aq];
+        if constexpr (SPLIT) {
+            const int64_t rows = (int64_t)p.B * p.H * N, row = share * rows + (int64_t)bh * N + io;
+            float* part = (float*)p.scratch + 2 * rows * p.nsplit + row * D + ac;
+#pragma unroll
+            for (int c = 0; c < ACN; c += 2) *(float2*)(part + c) = make_float2(oacc[aq * C::OS + ac + c], oacc[aq * C::OS + ac + c + 1]);
+            if ((tid_f & 15) == 0) ((float2*)p.scratch)[row] = make_float2(Ms, L);
+            return any_bad;
+        }
         const float inv = 1.f / (L + 1e-8f * fast_exp2(-Ms));
         uint16_t* orow = (uint16_t*)p.out.p + p.out.off(b, io, h) + ac;
         union { EL h[ACN]; uint32_t w[ACN / 2]; } o;
@@ -979,10 +1007,10 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
     return any_bad;
 }
 
-template <class E, int D, int MODE, bool SIDE, bool PAD>
+template <class E, int D, int MODE, bool SIDE, bool PAD, bool SPLIT>
 __global__ __launch_bounds__(FT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void mfma_fwd_kernel(Problem p, int nqb, int total, int left) {
-    const bool again = fwd_block<E, D, MODE, SIDE, PAD>(p, nqb, total, left, threadIdx.x);
+    const bool again = fwd_block<E, D, MODE, SIDE, PAD, SPLIT>(p, nqb, total, left, threadIdx.x);
     if constexpr (MODE == MODE_FAST) {
         if (again) {                              // (uniform over the workgroup)
             __syncthreads();
@@ -993,35 +1021,48 @@ void mfma_fwd_kernel(Problem p, int nqb, int total, int left) {
             asm volatile("" : "+s"(args));
             const Problem* again_p = (const Problem*)args;
             const int* rest = (const int*)(again_p + 1);
-            fwd_block<E, D, MODE_SAFE, SIDE, PAD>(*again_p, rest[0], rest[1], 0, recompute_here(threadIdx.x));
+            fwd_block<E, D, MODE_SAFE, SIDE, PAD, SPLIT>(*again_p, rest[0], rest[1], 0, recompute_here(threadIdx.x));
         }
     }
+}
+
+// deltas (minus one) whose K'/V' rows a workgroup needs: all of them, or those of a share's rounds
+inline int fwd_side_span(const Problem& p) {
+    if (p.nsplit <= 1) return p.w2;
+    const int deltas = ((p.w2 + FW) / FW + p.nsplit - 1) / p.nsplit * FW;
+    return deltas - 1 < p.w2 ? deltas - 1 : p.w2;
 }
 
 template <class E, int D, bool SIDE, bool PAD>
 int launch_fwd_kernels(const Problem& p, int nqb, int total, hipStream_t st) {
     using C = Cfg<D>;
-    const size_t lds = C::lds_bytes(p.w2);
+    const size_t lds = C::lds_bytes(fwd_side_span(p));
     // one unit left over after the rounds of eight: the pre-pass takes it, unless the grid is so
     // small that a further launch costs more than the lone round
-    const int left = (p.w2 >= FW && p.w2 % FW == 0 && (p.force_prepass || total >= PREPASS_MIN_WORKGROUPS)) ? 1 : 0;
-    if (!allow_full_lds((const void*)mfma_fwd_kernel<E, D, MODE_FAST, SIDE, PAD>) ||
-        !allow_full_lds((const void*)mfma_fwd_kernel<E, D, MODE_LEFT, false, PAD>))
-        return SA2_ERR_LAUNCH_FAILED;
+    const int left = (p.nsplit <= 1 && p.w2 >= FW && p.w2 % FW == 0 && (p.force_prepass || total >= PREPASS_MIN_WORKGROUPS)) ? 1 : 0;
     if (left) {
         const int ngrp = (nqb + FW - 1) / FW;
         const int total_left = ngrp * (total / nqb);
-        hipLaunchKernelGGL((mfma_fwd_kernel<E, D, MODE_LEFT, false, PAD>), dim3((unsigned)total_left), dim3(FT), C::STAGE_BYTES, st, p,
+        if (!allow_full_lds((const void*)mfma_fwd_kernel<E, D, MODE_LEFT, false, PAD, false>)) return SA2_ERR_LAUNCH_FAILED;
+        hipLaunchKernelGGL((mfma_fwd_kernel<E, D, MODE_LEFT, false, PAD, false>), dim3((unsigned)total_left), dim3(FT), C::STAGE_BYTES, st, p,
                            ngrp, total_left, 0);
         if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
     }
-    hipLaunchKernelGGL((mfma_fwd_kernel<E, D, MODE_FAST, SIDE, PAD>), dim3((unsigned)total), dim3(FT), lds, st, p, nqb, total, left);
-    return hipGetLastError() == hipSuccess ? SA2_OK : SA2_ERR_LAUNCH_FAILED;
+    auto go = [&](auto kernel, int64_t grid) {
+        if (!allow_full_lds((const void*)kernel)) return false;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(FT), lds, st, p, nqb, (int)grid, left);
+        return hipGetLastError() == hipSuccess;
+    };
+    if (p.nsplit <= 1) return go(mfma_fwd_kernel<E, D, MODE_FAST, SIDE, PAD, false>, total) ? SA2_OK : SA2_ERR_LAUNCH_FAILED;
+    const int64_t grid = (int64_t)total * p.nsplit;
+    if (grid > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
+    if (!go(mfma_fwd_kernel<E, D, MODE_FAST, SIDE, PAD, true>, grid)) return SA2_ERR_LAUNCH_FAILED;
+    return launch_fwd_merge(p, D, E::DTYPE, st);
 }
 
 template <class E, int D, bool PAD>
 int launch_fwd_pair(const Problem& p, int nqb, int total, hipStream_t st) {
-    return Cfg<D>::side_fits(p.w2) ? launch_fwd_kernels<E, D, true, PAD>(p, nqb, total, st)
+    return Cfg<D>::side_fits(fwd_side_span(p)) ? launch_fwd_kernels<E, D, true, PAD>(p, nqb, total, st)
                                    : launch_fwd_kernels<E, D, false, PAD>(p, nqb, total, st);
 }
 
@@ -1054,6 +1095,12 @@ bool mfma_layout_ok(const Problem& p, bool backward) {
     }
     return true;
 }
+
+// Shares of a forward given workspace for their partial outputs: none where the pre-pass is to take the odd unit
+int mfma_fwd_nsplit(int B, int N, int H, int D, int w1, int w2, bool force_prepass) {
+    return force_prepass && w2 >= FW && w2 % FW == 0 ? 1 : plan_forward(B, N, H, mfma_width(D), w1, w2, FW);
+}
+size_t mfma_fwd_part_bytes(int B, int N, int H, int D, int nsplit) { return fwd_part_bytes(B, N, H, mfma_width(D), nsplit); }
 
 int launch_mfma_fwd(const Problem& p, int dtype, hipStream_t st) {
     const int nqb = (p.N + BQ - 1) / BQ;

@@ -257,7 +257,8 @@ __device__ __forceinline__ void product_planes(const typename T::T* xrow, const 
 }
 
 // ================================================================== forward =====
-template <class T, int D, bool PAD>
+// SPLIT: one of nsplit shares of the rounds, unnormalised sums to the workspace (see launch_fwd_merge).
+template <class T, int D, bool PAD, bool SPLIT>
 __global__ __launch_bounds__((SplitCfg<T, D>::FW * 64)) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 2 : 1, D <= 64 ? 2 : 1)))
 void split_fwd_kernel(Problem p, int nqb, int total) {
     using C = SplitCfg<T, D>;
@@ -271,7 +272,11 @@ void split_fwd_kernel(Problem p, int nqb, int total) {
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63, ln = lane & 31, hf = lane >> 5;
-    const int pid = xcd_order(blockIdx.x, total);
+    int pid = xcd_order(blockIdx.x, total), share = 0;
+    if constexpr (SPLIT) {
+        share = pid % p.nsplit;
+        pid /= p.nsplit;
+    }
     const int bh = pid / nqb, qb = pid - bh * nqb;
     const int b = bh / p.H, h = bh - b * p.H;
     const int N = p.N, w1 = p.w1, w2 = p.w2;
@@ -287,7 +292,15 @@ void split_fwd_kernel(Problem p, int nqb, int total) {
     const int jt_lo = (i0 - w1 > 0 ? i0 - w1 : 0) / TJ, jt_hi = i_last / TJ;
     const int nt = jt_hi - jt_lo + 1;
     const int n_units = (w2 < i_last ? w2 : i_last) + 1;
-    const int nrounds = (n_units + W - 1) / W;
+    const int all_rounds = (n_units + W - 1) / W;
+    const int per_share = SPLIT ? ((w2 + W) / W + p.nsplit - 1) / p.nsplit : all_rounds;
+    const int round0 = SPLIT ? share * per_share : 0;
+    const int round1 = round0 + per_share < all_rounds ? round0 + per_share : all_rounds;
+    if (SPLIT && round0 >= round1) {             // a block near the start of the sequence has fewer rounds
+        if (tid < 32 && i0 + tid < N)
+            ((float2*)p.scratch)[(int64_t)share * p.B * p.H * N + (int64_t)bh * N + i0 + tid] = make_float2(-INFINITY, 0.f);
+        return;
+    }
     const float qscale = p.scale * LOG2E;
 
     const uint32_t tiles_addr = lds_address(tiles);
@@ -307,7 +320,7 @@ void split_fwd_kernel(Problem p, int nqb, int total) {
     for (int dt = 0; dt < C::DT; ++dt) oacc[dt] = zero16();
 
     int g = 0;
-    for (int round = 0; round < nrounds; ++round) {
+    for (int round = round0; round < round1; ++round) {
         const int delta = round * W + wave;
         const bool ok = delta < n_units;
         const int kr = ic - delta > 0 ? ic - delta : 0;
@@ -442,6 +455,8 @@ void split_fwd_kernel(Problem p, int nqb, int total) {
             wgt[w] = fast_exp2(mrg_m[w * 32 + row] - Mu);
             Ls += mrg_l[w * 32 + row] * wgt[w];
         }
+        const int64_t rows = (int64_t)p.B * p.H * N, prow = share * rows + (int64_t)bh * N + io;
+        if (SPLIT && tid % TPR == 0) ((float2*)p.scratch)[prow] = make_float2(Mx, Ls);
         // sum_w + 1e-8 in units of 2^Mu (reference.py:74); for a tiny Mu the epsilon dominates
         const bool big = Mu > LOG2_EPS;
         const float denom = big ? Ls + 1e-8f * fast_exp2(-Mu) : Ls * fast_exp2(Mu - LOG2_EPS) + 1.f;
@@ -449,16 +464,17 @@ void split_fwd_kernel(Problem p, int nqb, int total) {
         EL* orow = (EL*)p.out.p + p.out.off(b, io, h);
 #pragma unroll
         for (int col = 4 * (tid % TPR); col < D; col += 4 * TPR) {
-            if (PAD && col >= p.D) continue;
+            if (PAD && !SPLIT && col >= p.D) continue;
             float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
             for (int w = 0; w < W; ++w) {
                 const float4 y = *(const float4*)(mrg + (w * 32 + row) * C::AS + col);
                 acc.x += wgt[w] * y.x; acc.y += wgt[w] * y.y; acc.z += wgt[w] * y.z; acc.w += wgt[w] * y.w;
             }
-            T::store(orow + col, acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+            if constexpr (SPLIT) *(float4*)((float*)p.scratch + 2 * rows * p.nsplit + prow * D + col) = acc;
+            else T::store(orow + col, acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
         }
-        if (tid % TPR == 0)
+        if (!SPLIT && tid % TPR == 0)
             p.lse[(int64_t)bh * N + io] = big ? LN2 * Mu + logf(denom) : LN_EPS + logf(denom);
     }
 }
@@ -996,9 +1012,16 @@ int launch_split_fwd(const Problem& p, hipStream_t st) {
     const int nqb = (p.N + BQ - 1) / BQ;
     const int64_t total = (int64_t)nqb * p.B * p.H;
     if (total > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
-    if (!allow_full_lds((const void*)split_fwd_kernel<T, D, PAD>)) return SA2_ERR_LAUNCH_FAILED;
-    hipLaunchKernelGGL((split_fwd_kernel<T, D, PAD>), dim3((unsigned)total), dim3(C::FW * 64), C::FWD_LDS, st, p, nqb, (int)total);
-    return hipGetLastError() == hipSuccess ? SA2_OK : SA2_ERR_LAUNCH_FAILED;
+    auto go = [&](auto kernel, int64_t grid) {
+        if (!allow_full_lds((const void*)kernel)) return false;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(C::FW * 64), C::FWD_LDS, st, p, nqb, (int)grid);
+        return hipGetLastError() == hipSuccess;
+    };
+    if (p.nsplit <= 1) return go(split_fwd_kernel<T, D, PAD, false>, total) ? SA2_OK : SA2_ERR_LAUNCH_FAILED;
+    const int64_t grid = total * p.nsplit;
+    if (grid > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
+    if (!go(split_fwd_kernel<T, D, PAD, true>, grid)) return SA2_ERR_LAUNCH_FAILED;
+    return launch_fwd_merge(p, D, T::DTYPE, st);
 }
 
 template <class T, int D, bool PAD>
@@ -1113,6 +1136,12 @@ size_t f32_mfma_bwd_scratch_bytes(int B, int N, int H, int head_dim, int w1, int
     });
     return bytes;
 }
+
+int f32_mfma_fwd_nsplit(int B, int N, int H, int head_dim, int w1, int w2) {
+    const int D = split_width(head_dim);
+    return plan_forward(B, N, H, D, w1, w2, D <= 64 ? SplitCfg<MemF32, 64>::FW : SplitCfg<MemF32, 128>::FW);
+}
+size_t f32_mfma_fwd_part_bytes(int B, int N, int H, int head_dim, int nsplit) { return fwd_part_bytes(B, N, H, split_width(head_dim), nsplit); }
 
 int launch_f32_mfma_fwd(const Problem& p, int dtype, hipStream_t st) {
     return for_split_width(p.D, dtype, [&](auto m, auto width, auto pad) {

@@ -1,0 +1,41 @@
+"""Forward launches whose rounds are shared by several workgroups (short sequences with wide K' windows): the partial
+outputs, their merge and the second pass of an overflowed block, against the CPU oracle; sa2_forward without a workspace
+computes the same problem in one workgroup per query block."""
+import pytest
+import torch
+
+from simplical_attn_amd import _lib
+from tests.util import assert_close_rel, make_inputs, oracle_all
+
+pytestmark = pytest.mark.gpu
+CODE = {torch.float32: _lib.SA2_F32, torch.bfloat16: _lib.SA2_BF16, torch.float16: _lib.SA2_F16}
+BAR = {torch.bfloat16: 2e-2, torch.float16: 1e-2, torch.float32: 1e-5}
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("case", [(1, 130, 2, 64, 40, 60, True), (2, 97, 1, 128, 200, 47, False), (1, 256, 1, 32, 33, 255, True),
+                                  (1, 77, 3, 16, 20, 33, True), (1, 33, 1, 96, 8, 40, True)])
+@pytest.mark.parametrize("scale", [None, 6.0])
+def test_shares_of_the_rounds_merge_to_the_oracle(dtype, case, scale):
+    """scale 6: logits of hundreds, so that blocks overflow their first reference point and take the second pass."""
+    import simplical_attn_amd as sa
+    lib = _lib.load()
+    B, N, H, D, w1, w2, inclusive = case
+    assert lib.sa2_fwd_workspace_bytes(B, N, H, D, w1, w2, CODE[dtype], int(inclusive), 0) > 0
+    host = make_inputs(B, N, H, D, seed=N, dtype=dtype)
+    x = [t.cuda() for t in host[:5]]
+    out, lse = sa.simplicial_forward(*x, w1, w2, scale, 0.1, -0.2, window_inclusive=inclusive)
+    want = oracle_all(host, w1, w2, scale, 0.1, -0.2, inclusive=inclusive)
+    # (16-bit logits of hundreds carry absolute errors of their rounding: the largest weight may change hands)
+    if scale is None or dtype == torch.float32:
+        assert_close_rel(out, want["out"], BAR[dtype] if scale is None else 2e-4, "out")
+    assert torch.isfinite(out.float()).all()
+    assert_close_rel(lse, want["lse"], BAR[dtype] if scale is None or dtype != torch.float32 else 1e-5, "lse")
+    o1, l1 = torch.empty_like(out), torch.empty_like(lse)
+    strides = _lib.stride_array([(t.stride(0), t.stride(1), t.stride(2)) for t in (*x, o1)])
+    _lib.check(lib.sa2_forward(*[t.data_ptr() for t in x], o1.data_ptr(), l1.data_ptr(), B, N, H, D, strides, w1, w2,
+                               D ** -0.5 if scale is None else scale, 0.1, -0.2, CODE[dtype], int(inclusive), 0,
+                               torch.cuda.current_stream().cuda_stream))
+    assert_close_rel(out, o1.float().cpu(), {torch.float32: 1e-5 if scale is None else 2e-4}.get(dtype, 1e-2), "out, shared against whole")
+    assert_close_rel(lse, l1.cpu(), 1e-5 if dtype == torch.float32 else 1e-3, "lse, shared against whole")
+    torch.cuda.synchronize()
