@@ -197,6 +197,7 @@ int launch_f32_mfma_bwd(const Problem& p, int dtype, hipStream_t st);
 bool wide_supported(int D, int dtype);
 bool wide_bwd_supported(int D, int w2, int dtype);
 size_t wide_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2);
+int wide_fwd_nsplit(int B, int N, int H, int w1, int w2);
 int launch_wide_fwd(const Problem& p, int dtype, hipStream_t st);
 int launch_wide_bwd(const Problem& p, int dtype, hipStream_t st);
 // Partial outputs of a split forward, [nsplit][B*H*N] pairs (reference exponent M, sum L) and then

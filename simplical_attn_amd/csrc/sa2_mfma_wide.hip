@@ -10,10 +10,10 @@
 // stride that keeps both kinds of read free of bank conflicts.
 //
 // A head_dim of 256 does not leave room for the operands of the logit contraction (64 registers) next
-// to accumulators for all 256 output columns of two contractions, so every kernel takes the output
+// to accumulators for all 256 output columns of two contractions, so the backward kernels take the output
 // columns in passes of DV = 128 (grid dimension y): a pass contracts the logits over the whole
 // head_dim and accumulates its own 128 columns of R, G, dK, dV.  The logits (and dP) are computed
-// once per pass: 1.5x the forward's and 1.33x the backward's algorithmic MFMA work.
+// once per pass: 1.33x the backward's algorithmic MFMA work.
 //
 //   wide_fwd_kernel   32 queries per workgroup; wavefront w takes delta = w, w+4, ... with one online
 //                     softmax and one output accumulator across its units, merged once at the end.
@@ -32,6 +32,8 @@ namespace {
 constexpr int WW = 4;                  // wavefronts per workgroup
 constexpr int WT = WW * 64;            // threads per workgroup
 constexpr int WJ = WW * 32;            // K rows per workgroup of the K-side kernel
+
+constexpr int WSIDE = 36;              // K' and V' rows the forward keeps in LDS: the 35 of a round, and one to make pairs
 
 typedef unsigned ux4 __attribute__((ext_vector_type(4)));     // 16 bytes in flight (a plain vector: stays in registers)
 
@@ -131,27 +133,96 @@ __device__ __forceinline__ typename E::x8 product8(const ux4& a, const ux4& b, f
     return r;
 }
 
+template <class E>
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    union { typename E::x2 h; uint32_t u; } v;
+    v.h = __builtin_convertvector((f2){a, b}, typename E::x2);
+    return v.u;
+}
+// ---- tiles -----------------------------------------------------------------------
+// A 32-row tile of a 256-column tensor in LDS: sixteen groups of two rows, each written by one direct
+// global->LDS load of a wavefront (1 KB; lane L puts the 16-byte chunk L / 2 of row L % 2 at byte 16 * L)
+// and GROUP bytes apart.  Row operand reads are free of bank conflicts, transposed ones take two passes.  (A swizzle of the
+// chunks that frees both measured the same or slower, forward 889 -> 915 us and K-side 1526 -> 1537 us at B1 H8 N4096
+// w 512/32: LDS is not what the kernels wait for, and its addresses cost vector instructions.)
+struct WT256 {
+    static constexpr int RPW = 2, GROUP = 1024 + 32, NGROUP = 16;
+    static constexpr int BYTES = NGROUP * GROUP;
+    static constexpr int row_off(int r) { return (r / RPW) * GROUP + (r % RPW) * 16; }
+};
+constexpr size_t WIDE_FWD_LDS = (size_t)7 * WT256::BYTES + 2 * (WSIDE / 2) * WT256::GROUP;
+static_assert(WIDE_FWD_LDS >= (size_t)WW * 32 * 260 * 4 + 2 * WW * 32 * 4 && WIDE_FWD_LDS <= 160 * 1024, "the merge lies over the tiles");
+typedef __attribute__((address_space(3))) void* wide_lds_ptr;
+typedef const __attribute__((address_space(1))) void* wide_glb_ptr;
+
+// The four groups of wavefront `wave` of the tile of rows j0 .. j0+31 (rows past the end of the sequence read the
+// last one): `lane_off` is the byte offset of the lane's chunk in the wavefront's first group.
+__device__ __forceinline__ void wide_request(const uint16_t* base, int64_t sn, int j0, int N, int wave, int lane, uint32_t lane_off,
+                                             unsigned char* dst) {
+    const char* g = (const char*)(base + (int64_t)j0 * sn);
+    if (__builtin_expect(j0 + 32 <= N, 1)) {
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+            __builtin_amdgcn_global_load_lds((wide_glb_ptr)(g + (lane_off + (uint32_t)x * ((uint32_t)sn * 4u))), (wide_lds_ptr)(dst + (4 * wave + x) * WT256::GROUP), 16, 0, 0);
+    } else {
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            const int row = 8 * wave + 2 * x + (lane & 1), r = row < N - 1 - j0 ? row : N - 1 - j0;
+            __builtin_amdgcn_global_load_lds((wide_glb_ptr)(g + ((uint32_t)r * (uint32_t)sn + (uint32_t)(lane >> 1) * 8) * 2u),
+                                             (wide_lds_ptr)(dst + (4 * wave + x) * WT256::GROUP), 16, 0, 0);
+        }
+    }
+}
+// Transposed operands of k-step KS (rows 16*KS .. +15) of the column blocks DT0 .. DT0+N-1, as opaque reads
+template <int KS, int DT0, int N, int I = 0, int M>
+__device__ __forceinline__ void wide_tr_issue(uint32_t addr, lds_half_operand (&h)[M]) {
+    if constexpr (I < N) {
+        constexpr int o = (DT0 + I) * 64 * WT256::RPW + WT256::row_off(16 * KS);
+        lds_tr_issue<o, o + WT256::row_off(8)>(addr, h[2 * I], h[2 * I + 1]);
+        wide_tr_issue<KS, DT0, N, I + 1>(addr, h);
+    }
+}
+// Row operands of the k-steps K0 .. K0+7
+template <int K0, int I = 0, class X8>
+__device__ __forceinline__ void wide_row_issue(uint32_t addr, X8 (&r)[8]) {
+    if constexpr (I < 8) {
+        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(r[I]) : "v"(addr), "n"((K0 + I) * 32 * WT256::RPW));
+        wide_row_issue<K0, I + 1>(addr, r);
+    }
+}
+
 // ================================================================== forward =====
-template <class E, int D, int DV>
-__global__ __launch_bounds__(WT) __attribute__((amdgpu_waves_per_eu(1, 1)))
-void wide_fwd_kernel(Problem p, int nqb, int total) {
+// What bounds it: in the sweep the matrix pipe at the rate that power allows (1.09 us per step of 32 MFMAs per wavefront,
+// 1.0 PFLOP/s), and between two sweeps the forming of Q~ and the sum over the unit, 6 us per round.  The logits of tile t
+// run under the softmax arithmetic of tile t-1, operand reads are one block of eight MFMAs ahead of their use, and the
+// last eight value MFMAs of a tile run behind the step's barrier, under the next tile's operand reads.
+// B1 H8 N4096 w 512/32 bf16: 2215 us in two column passes, 890 now; B1 H3 N700 w 500/100 949 -> 233 (shares of the rounds).
+// SAFE: the second pass of a block in which a weight overflowed (logits growing by tens of octaves along the window after
+// the reference point was fixed): the reference point follows the maxima on every tile, nothing is pipelined.
+// Returns whether that pass is needed.
+template <class E, bool SPLIT, bool SAFE>
+__device__ __forceinline__ bool wide_fwd_block(const Problem& p, int nqb, int total, unsigned char* smem_w) {
     typedef typename E::scalar EL;
     typedef typename E::x8 X8;
-    using C = WideCfg<D, DV>;
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem_w[];
-    uint16_t* tiles = (uint16_t*)smem_w;
-    float* mrg_m = (float*)(smem_w + (C::TILES_BYTES > C::MERGE_BYTES ? C::TILES_BYTES : C::MERGE_BYTES));   // [WW][32]
-    float* mrg_l = mrg_m + WW * 32;
-
+    typedef typename E::x2 X2;
+    constexpr int D = 256, DK = 16, DT = 8, TB = WT256::BYTES;
     const int tid = threadIdx.x;
+    unsigned char* q_s = smem_w + 6 * TB;                    // q rows of the block
+    unsigned char* k2_s = q_s + TB;                          // ring of WSIDE K' rows
+    unsigned char* v2_s = k2_s + WSIDE / 2 * WT256::GROUP;   // ... and V' rows
+
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63, ln = lane & 31, hf = lane >> 5;
-    const int pid = xcd_order(blockIdx.x, total);
-    const int c0 = blockIdx.y * DV;                          // this pass's output columns
+    int pid = xcd_order(blockIdx.x, total), share = 0;
+    if constexpr (SPLIT) {
+        share = pid % p.nsplit;
+        pid /= p.nsplit;
+    }
     const int bh = pid / nqb, qb = pid - bh * nqb;
     const int b = bh / p.H, h = bh - b * p.H;
     const int N = p.N, w1 = p.w1, w2 = p.w2;
-    const int i0 = qb * BQ, i = i0 + ln, ic = i < N ? i : N - 1;
+    const int i0 = qb * BQ, i = i0 + ln;
     const int i_last = i0 + BQ - 1 < N ? i0 + BQ - 1 : N - 1;
 
     const uint16_t* qp = (const uint16_t*)p.q.p + p.q.off(b, 0, h);
@@ -160,143 +231,305 @@ void wide_fwd_kernel(Problem p, int nqb, int total) {
     const uint16_t* v1p = (const uint16_t*)p.v1.p + p.v1.off(b, 0, h);
     const uint16_t* v2p = (const uint16_t*)p.v2.p + p.v2.off(b, 0, h);
 
-    const int jt_lo = (i0 - w1 > 0 ? i0 - w1 : 0) / TJ, jt_hi = i_last / TJ;
+    // The sweep goes from the diagonal tile down: every row has a key in its first tile, which fixes its reference point.
+    const int jt_lo = (i0 - w1 > 0 ? i0 - w1 : 0) / TJ, jt_hi = i0 / TJ;
     const int nt = jt_hi - jt_lo + 1;
     const int n_units = (w2 < i_last ? w2 : i_last) + 1;
-    const int nrounds = (n_units + WW - 1) / WW;
+    const int all_rounds = (n_units + WW - 1) / WW;
+    const int per_share = SPLIT ? ((w2 + WW) / WW + p.nsplit - 1) / p.nsplit : all_rounds;
+    const int round0 = SPLIT ? share * per_share : 0;
+    const int round1 = round0 + per_share < all_rounds ? round0 + per_share : all_rounds;
+    if constexpr (SPLIT) {
+        if (round0 >= round1) {                  // a block near the start of the sequence has fewer rounds
+            if (tid < BQ && i0 + tid < N)
+                ((float2*)p.scratch)[share * (int64_t)p.B * p.H * N + (int64_t)bh * N + i0 + tid] = make_float2(-INFINITY, 0.f);
+            return false;
+        }
+    }
+    const int total_steps = (round1 - round0) * nt;
     const float qscale = p.scale * LOG2E;
-    const uint32_t tiles_addr = lds_address(tiles);
-    const uint32_t tr_lane = tr_lane_offset<C::RSB>(lane);
 
-    ux4 tk[C::KR], tv[C::KR];                    // the tile on its way from global memory to LDS
-    wide_load<D, DV>(tk, tv, k1p, p.k1.sn, v1p, p.v1.sn, jt_lo * TJ, N, tid);
-    wide_store<D, DV>(tk, tv, tiles, tid);
-    wide_load<D, DV>(tk, tv, k1p, p.k1.sn, v1p, p.v1.sn, (jt_lo + 1 % nt) * TJ, N, tid);
-    __syncthreads();
+    // ---- requests: step g asks for the K tile of step g+2 and the V tile of step g+1, in rings of three ----
+    const uint32_t k_off = ((uint32_t)(8 * wave + (lane & 1)) * (uint32_t)p.k1.sn + (uint32_t)(lane >> 1) * 8) * 2u;
+    const uint32_t v_off = ((uint32_t)(8 * wave + (lane & 1)) * (uint32_t)p.v1.sn + (uint32_t)(lane >> 1) * 8) * 2u;
+    int kt = 0, kstage = 0, kleft = total_steps, vt = 0, vstage = 0, vleft = total_steps;
+    auto request_k = [&]() {
+        wide_request(k1p, p.k1.sn, (jt_hi - kt) * TJ, N, wave, lane, k_off, smem_w + kstage * TB);
+        kt = kt + 1 == nt ? 0 : kt + 1;
+        kstage = kstage == 2 ? 0 : kstage + 1;
+        --kleft;
+    };
+    auto request_v = [&]() {
+        wide_request(v1p, p.v1.sn, (jt_hi - vt) * TJ, N, wave, lane, v_off, smem_w + (3 + vstage) * TB);
+        vt = vt + 1 == nt ? 0 : vt + 1;
+        vstage = vstage == 2 ? 0 : vstage + 1;
+        --vleft;
+    };
+    // K'/V' row u counts back from row i0 + 31 of share's first round; it sits at place u % WSIDE of its ring.  A round
+    // needs rows 4r .. 4r+34; `pair` is a pair of rows (u = 2 * pair, 2 * pair + 1).
+    auto request_side = [&](const uint16_t* base, int64_t sn, int pair, unsigned char* ring) {
+        int k = i0 + BQ - 1 - round0 * WW - 2 * pair - (lane & 1);
+        k = k < 0 ? 0 : (k < N ? k : N - 1);
+        __builtin_amdgcn_global_load_lds((wide_glb_ptr)(base + (int64_t)k * sn + (lane >> 1) * 8),
+                                         (wide_lds_ptr)(ring + (pair % (WSIDE / 2)) * WT256::GROUP), 16, 0, 0);
+    };
+    request_k();
+    request_v();
+    wide_request(qp, p.q.sn, i0, N, wave, lane, ((uint32_t)(8 * wave + (lane & 1)) * (uint32_t)p.q.sn + (uint32_t)(lane >> 1) * 8) * 2u, q_s);
+    for (int x = wave; x < WSIDE / 2; x += WW) {
+        request_side(k2p, p.k2.sn, x, k2_s);
+        request_side(v2p, p.v2.sn, x, v2_s);
+    }
+    if (kleft > 0) request_k();
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
 
-    // the wavefront's running softmax over its units: reference exponent, sum, weighted output
-    float M = -INFINITY, L = 0.f;
-    floatx16 oacc[C::DT];
+    const uint32_t smem_addr = lds_address(smem_w);
+    const uint32_t row_lane = (uint32_t)((ln / 2) * WT256::GROUP + (hf * 2 + (ln & 1)) * 16);
+    const uint32_t col_lane = lds_group_column_lane_offset<WT256::RPW, WT256::GROUP>(lane);
+
+    // the wavefront's running softmax over its units: reference exponent (one per row for all units), sum, weighted output
+    float m = -INFINITY, L = 0.f;
+    floatx16 wacc[DT], racc[DT];
 #pragma unroll
-    for (int dt = 0; dt < C::DT; ++dt) oacc[dt] = zeros16();
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) wacc[dt][v] = 0.f;
 
-    int g = 0;
-    for (int round = 0; round < nrounds; ++round) {
+    bool bad = false;
+    int buf = 0;                                             // ring stage of the current step's K tile
+    for (int round = round0; round < round1; ++round) {
+        const int rr = round - round0;
         const int delta = round * WW + wave;
         const bool ok = delta < n_units;
-        const int kr = ic - delta > 0 ? ic - delta : 0;
-        const bool row_ok = ok && i < N && i >= delta;
-        const bool rows_full = i0 >= delta && i0 + BQ - 1 < N;
-
-        X8 qf[C::DK];
-        if (ok) {
+        const bool row_ok = i < N && i >= delta;
+        const bool rows_full = ok && i0 >= delta && i0 + BQ - 1 < N;
+        const int place = (BQ - 1 - ln + rr * WW + wave) % WSIDE;
+        const uint32_t side = (uint32_t)((place / 2) * WT256::GROUP + (place & 1) * 16);
+        X8 qf[DK];
 #pragma unroll
-            for (int kk = 0; kk < C::DK; ++kk) {
-                const ux4 qa = *(const ux4*)(qp + (int64_t)ic * p.q.sn + kk * 16 + hf * 8);
-                const ux4 kb = *(const ux4*)(k2p + (int64_t)kr * p.k2.sn + kk * 16 + hf * 8);
-                qf[kk] = product8<E>(qa, kb, p.k2_bias, qscale);
-            }
+        for (int kk = 0; kk < DK; ++kk) {
+            const ux4 qa = *(const ux4*)(q_s + row_lane + kk * 64);
+            const ux4 kb = *(const ux4*)(k2_s + side + hf * 32 + kk * 64);
+            qf[kk] = product8<E>(qa, kb, p.k2_bias, qscale);
         }
-        float m = -INFINITY, l = 0.f;
-        floatx16 racc[C::DT];
+        float l = 0.f, mu = -INFINITY;            // (mu: the unit's own reference point in the second pass)
 #pragma unroll
-        for (int dt = 0; dt < C::DT; ++dt) racc[dt] = zeros16();
+        for (int dt = 0; dt < DT; ++dt) racc[dt] = zeros16();
+        // -inf where the key lies outside the window of the row.  Element v of this lane is key j0 + 8*(v/4) + 4*hf + v%4.
+        auto mask = [&](floatx16& s, int j0) {
+            int hi = i - j0 - 4 * hf;
+            asm volatile("" : "+v"(hi));          // (compared here, not kept from one round to the next)
+            const int lo = hi - w1;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int c = 8 * (v >> 2) + (v & 3);
+                s[v] = (row_ok && c <= hi && c >= lo) ? s[v] : -INFINITY;
+            }
+        };
+        auto tile_plain = [&](int j0) { return rows_full && j0 + TJ - 1 <= i0 && j0 >= i0 + BQ - 1 - w1; };
+        if (!SAFE && ok && __builtin_amdgcn_ballot_w64(m == -INFINITY) != 0) {
+            // the reference point of the wavefront's rows: the maximum of the first tile (0 for a row that has no key at all)
+            floatx16 t = zeros16();
+#pragma unroll
+            for (int kk = 0; kk < DK; ++kk) t = E::mfma(lds_read_x8<X8>(smem_addr + buf * TB + row_lane + kk * 64), qf[kk], t, 0, 0, 0);
+            mask(t, jt_hi * TJ);
+            float mx = t[0];
+#pragma unroll
+            for (int v = 1; v < 16; ++v) mx = fmaxf(mx, t[v]);
+            mx = fmaxf(mx, other_half(mx));
+            if (m == -INFINITY) m = mx == -INFINITY ? 0.f : mx;
+        }
 
-        for (int s = 0; s < nt; ++s, ++g) {
-            if (ok) {
-                const int j0 = (jt_lo + s) * TJ;
-                const uint16_t* Ks = tiles + (g & 1) * C::STAGE;
-                const uint32_t Vt = tiles_addr + (uint32_t)(((g & 1) * C::STAGE + C::TILE) * 2) + tr_lane + (uint32_t)(c0 * 2);
-                floatx16 sacc = zeros16();
+        floatx16 cur, prev;
+        X8 pb[2], pb1;                            // weights of the tile before; of the one before that, second k-step
+        lds_half_operand va[16], vb[16];
+        // weights of the logits `s` and their row sum (this lane's half of the keys)
+        auto weights = [&](const floatx16& s, float ref) {
 #pragma unroll
-                for (int kk = 0; kk < C::DK; ++kk) {
-                    const X8 ka = *(const X8*)(Ks + ln * C::RS + kk * 16 + hf * 8);
-                    sacc = E::mfma(ka, qf[kk], sacc, 0, 0, 0);
-                }
-                // register v of this lane: key j0 + 8*(v/4) + 4*hf + v%4
-                const bool interior = rows_full && (j0 + TJ - 1 <= i0) && (j0 >= i0 + BQ - 1 - w1);
-                if (!interior) {
-                    const int hi = i - j0 - 4 * hf, lo = hi - w1;
+            for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) {
-                        const int c = 8 * (v >> 2) + (v & 3);
-                        sacc[v] = (row_ok && c <= hi && c >= lo) ? sacc[v] : -INFINITY;
-                    }
-                }
-                float mx = sacc[0];
+                for (int t = 0; t < 8; ++t) pb[ks][t] = (EL)fast_exp2(s[ks * 8 + t] - ref);
+            const X2 ones = {(EL)1.f, (EL)1.f};
+            float r = 0.f;
 #pragma unroll
-                for (int v = 1; v < 16; ++v) mx = fmaxf(mx, sacc[v]);
-                mx = fmaxf(mx, other_half(mx));
-                const float m_new = fmaxf(m, mx);
-                const float m_use = m_new == -INFINITY ? 0.f : m_new;
-                const float alpha = fast_exp2(m - m_use);
-                m = m_new;
-                if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
+            for (int ks = 0; ks < 2; ++ks) {
+                r = E::dot2(__builtin_shufflevector(pb[ks], pb[ks], 0, 1), ones, r, false);
+                r = E::dot2(__builtin_shufflevector(pb[ks], pb[ks], 2, 3), ones, r, false);
+                r = E::dot2(__builtin_shufflevector(pb[ks], pb[ks], 4, 5), ones, r, false);
+                r = E::dot2(__builtin_shufflevector(pb[ks], pb[ks], 6, 7), ones, r, false);
+            }
+            return r;
+        };
+        auto value_mfmas = [&](const lds_half_operand (&x)[16], const X8& w) {
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) racc[dt] = E::mfma(lds_join<X8>(x[2 * dt], x[2 * dt + 1]), w, racc[dt], 0, 0, 0);
+        };
+        auto logit_mfmas = [&](const X8 (&k)[8], int k0, floatx16 c) {
+#pragma unroll
+            for (int x = 0; x < 8; ++x) c = E::mfma(k[x], qf[k0 + x], c, 0, 0, 0);
+            return c;
+        };
+        auto end_step = [&](bool both) {
+            if (both) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            buf = buf == 2 ? 0 : buf + 1;
+        };
+        auto begin_step = [&]() {
+            const bool both = kleft > 0;
+            if (vleft > 0) request_v();
+            if (both) request_k();
+            return both;
+        };
+
+        auto side_rows = [&]() {
+            // (every wavefront has formed its Q~ and is done with the round before)
+            if (wave < 2) request_side(k2p, p.k2.sn, 2 * rr + WSIDE / 2 + wave, k2_s);
+            else if (rr > 0) request_side(v2p, p.v2.sn, 2 * rr + WSIDE / 2 - 4 + wave, v2_s);
+            if (nt == 1) asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+        };
+        if constexpr (SAFE) {
+            for (int s = 0; s < nt; ++s) {
+                const bool both = begin_step();
+                if (ok) {
+                    const int j0 = (jt_hi - s) * TJ;
+                    cur = zeros16();
+#pragma unroll
+                    for (int kk = 0; kk < DK; ++kk) cur = E::mfma(lds_read_x8<X8>(smem_addr + buf * TB + row_lane + kk * 64), qf[kk], cur, 0, 0, 0);
+                    if (!tile_plain(j0)) mask(cur, j0);
+                    float mx = cur[0];
+#pragma unroll
+                    for (int v = 1; v < 16; ++v) mx = fmaxf(mx, cur[v]);
+                    const float m_new = fmaxf(mu, fmaxf(mx, other_half(mx))), m_use = m_new == -INFINITY ? 0.f : m_new;
+                    const float alpha = fast_exp2(mu - m_use);
+                    mu = m_new;
                     l *= alpha;
 #pragma unroll
-                    for (int dt = 0; dt < C::DT; ++dt)
+                    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
                         for (int v = 0; v < 16; ++v) racc[dt][v] *= alpha;
+                    l += weights(cur, m_use);
                 }
-                // the weights as the MFMA sees them (rounded), and their sum
-                X8 pb[2];
-                float rs = 0.f;
+                end_step(both);                  // (the V tile of a step is complete behind its barrier)
+                if (s == 0) side_rows();
+                if (ok) {
+                    const uint32_t vt_addr = smem_addr + (3 + (buf == 0 ? 2 : buf - 1)) * TB + col_lane;
 #pragma unroll
-                for (int ks = 0; ks < 2; ++ks)
+                    for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-                    for (int t = 0; t < 8; ++t) {
-                        pb[ks][t] = (EL)fast_exp2(sacc[ks * 8 + t] - m_use);
-                        rs += (float)pb[ks][t];
-                    }
-                l += rs;
-#pragma unroll
-                for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-                    for (int dt = 0; dt < C::DT; ++dt) {
-                        const X8 va = tr_operand<X8, C::RSB>(Vt + (uint32_t)(16 * ks * C::RSB + dt * 64));
-                        racc[dt] = E::mfma(va, pb[ks], racc[dt], 0, 0, 0);
-                    }
+                        for (int dt = 0; dt < DT; ++dt)
+                            racc[dt] = E::mfma(lds_group_column_operand_at<WT256, X8>(vt_addr + dt * 64 * WT256::RPW, ks), pb[ks], racc[dt], 0, 0, 0);
+                }
             }
-            // (unconditional: past the last step this moves a tile nobody reads)
-            wide_store<D, DV>(tk, tv, tiles + ((g + 1) & 1) * C::STAGE, tid);
-            wide_load<D, DV>(tk, tv, k1p, p.k1.sn, v1p, p.v1.sn, (jt_lo + (g + 2) % nt) * TJ, N, tid);
-            __syncthreads();
+        } else {
+        // ---- first step: logits only ----
+        {
+            const bool both = begin_step();
+            if (ok) {
+                X8 k0[8], k1[8];
+                const uint32_t a = smem_addr + buf * TB + row_lane;
+                wide_row_issue<0>(a, k0);
+                wide_row_issue<8>(a, k1);
+                lds_wait<8>(k0);
+                prev = logit_mfmas(k0, 0, zeros16());
+                lds_wait<0>(k1);
+                prev = logit_mfmas(k1, 8, prev);
+                mask(prev, jt_hi * TJ);          // (the diagonal tile)
+            }
+            end_step(both);
         }
-
+        side_rows();
+        for (int s = 1; s < nt; ++s) {
+            const bool both = begin_step();
+            if (ok) {
+                const int j0 = (jt_hi - s) * TJ;
+                X8 k0[8], k1[8];
+                const uint32_t a = smem_addr + buf * TB + row_lane;
+                const uint32_t vt_addr = smem_addr + (3 + (buf == 0 ? 2 : buf - 1)) * TB + col_lane;
+                wide_row_issue<0>(a, k0);
+                wide_row_issue<8>(a, k1);
+                __builtin_amdgcn_sched_barrier(0);
+                if (s > 1) value_mfmas(vb, pb1);
+                lds_wait<8>(k0);
+                cur = logit_mfmas(k0, 0, zeros16());
+                lds_wait<0>(k1);
+                wide_tr_issue<0, 0, 8>(vt_addr, va);
+                cur = logit_mfmas(k1, 8, cur);
+                const float rs = weights(prev, m);
+                l += rs;
+                bad |= !(rs < E::WEIGHT_LIMIT);
+                pb1 = pb[1];
+                lds_settle(va);
+                wide_tr_issue<1, 0, 8>(vt_addr, vb);
+                value_mfmas(va, pb[0]);
+                lds_settle(vb);
+                prev = cur;
+                if (!tile_plain(j0)) mask(prev, j0);
+            }
+            end_step(both);
+        }
+        // ---- last tile's values ----
         if (ok) {
-            // fold the unit into the wavefront's running result: O += e^(m-M) * (v2 + bias) * R
+            const uint32_t vt_addr = smem_addr + (3 + (buf == 0 ? 2 : buf - 1)) * TB + col_lane;
+            wide_tr_issue<0, 0, 8>(vt_addr, va);
+            if (nt > 1) value_mfmas(vb, pb1);
+            const float rs = weights(prev, m);
+            l += rs;
+            bad |= !(rs < E::WEIGHT_LIMIT);
+            lds_settle(va);
+            wide_tr_issue<1, 0, 8>(vt_addr, vb);
+            value_mfmas(va, pb[0]);
+            lds_settle(vb);
+            value_mfmas(vb, pb[1]);
+        }
+        }
+        // ---- the unit joins the running result: O += (v2 + bias) * R ----
+        if (ok) {
             const float lt = l + other_half(l);
-            const float M_new = fmaxf(M, m);
-            const float Mu = M_new == -INFINITY ? 0.f : M_new;
-            const float a = fast_exp2(M - Mu), c = fast_exp2(m - Mu);
-            L = L * a + lt * c;
-            M = M_new;
-            const uint16_t* vrow = v2p + (int64_t)kr * p.v2.sn + c0 + 4 * hf;
+            float a = 1.f, c = 1.f;
+            if constexpr (SAFE) {
+                const float M_new = fmaxf(m, mu), Mu = M_new == -INFINITY ? 0.f : M_new;
+                a = fast_exp2(m - Mu);
+                c = fast_exp2(mu - Mu);
+                m = M_new;
+                L *= a;
+            }
+            L += c * lt;
+            const unsigned char* vrow = v2_s + side + hf * 8;
 #pragma unroll
-            for (int dt = 0; dt < C::DT; ++dt)
+            for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
                 for (int g4 = 0; g4 < 4; ++g4) {
-                    const uint2 x = *(const uint2*)(vrow + dt * 32 + 8 * g4);
-                    oacc[dt][4 * g4 + 0] = oacc[dt][4 * g4 + 0] * a + c * racc[dt][4 * g4 + 0] * (E::lo(x.x) + p.v2_bias);
-                    oacc[dt][4 * g4 + 1] = oacc[dt][4 * g4 + 1] * a + c * racc[dt][4 * g4 + 1] * (E::hi(x.x) + p.v2_bias);
-                    oacc[dt][4 * g4 + 2] = oacc[dt][4 * g4 + 2] * a + c * racc[dt][4 * g4 + 2] * (E::lo(x.y) + p.v2_bias);
-                    oacc[dt][4 * g4 + 3] = oacc[dt][4 * g4 + 3] * a + c * racc[dt][4 * g4 + 3] * (E::hi(x.y) + p.v2_bias);
+                    const uint2 x = *(const uint2*)(vrow + (4 * dt + g4) * 32);
+                    const float y[4] = {E::lo(x.x), E::hi(x.x), E::lo(x.y), E::hi(x.y)};
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        const int v = 4 * g4 + t;
+                        if constexpr (SAFE) wacc[dt][v] = wacc[dt][v] * a + c * racc[dt][v] * (y[t] + p.v2_bias);
+                        else wacc[dt][v] += racc[dt][v] * (y[t] + p.v2_bias);
+                    }
                 }
         }
     }
 
-    // ---- merge the four wavefronts (the tile stages are free: the sweep's last barrier is behind us) ----
+    // ---- merge the four wavefronts ----
+    if constexpr (!SAFE) {
+        if (__syncthreads_or(bad ? 1 : 0)) return true;
+    }
+    else __syncthreads();
+    constexpr int AS = D + 4;
     float* mrg = (float*)smem_w;                           // [WW][32][AS]
+    float* mrg_m = mrg + WW * 32 * AS;                     // [WW][32]
+    float* mrg_l = mrg_m + WW * 32;
     {
-        float* row = mrg + (wave * 32 + ln) * C::AS + 4 * hf;
+        float* row = mrg + (wave * 32 + ln) * AS + 4 * hf;
 #pragma unroll
-        for (int dt = 0; dt < C::DT; ++dt)
+        for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4)
-                *(float4*)(row + dt * 32 + 8 * g4) = make_float4(oacc[dt][4 * g4], oacc[dt][4 * g4 + 1], oacc[dt][4 * g4 + 2],
-                                                                 oacc[dt][4 * g4 + 3]);
+                *(float4*)(row + dt * 32 + 8 * g4) = make_float4(wacc[dt][4 * g4], wacc[dt][4 * g4 + 1], wacc[dt][4 * g4 + 2],
+                                                                 wacc[dt][4 * g4 + 3]);
         if (hf == 0) {
-            mrg_m[wave * 32 + ln] = M;
+            mrg_m[wave * 32 + ln] = L > 0.f || L != L ? m : -INFINITY;         // (a row without a key has no say in the reference)
             mrg_l[wave * 32 + ln] = L;
         }
     }
@@ -313,25 +546,46 @@ void wide_fwd_kernel(Problem p, int nqb, int total) {
             wgt[w] = fast_exp2(mrg_m[w * 32 + row] - Mu);
             Ls += mrg_l[w * 32 + row] * wgt[w];
         }
-        // sum_w + 1e-8 in units of 2^Mu (reference.py:74); for a tiny Mu the epsilon dominates
+        const int64_t rows = (int64_t)p.B * p.H * N, prow = share * rows + (int64_t)bh * N + io;
+        float* part = (float*)p.scratch + 2 * rows * p.nsplit + prow * D;      // (SPLIT)
+        // sum_w + 1e-8 in units of 2^Mu; for a tiny Mu the epsilon dominates
         const bool big = Mu > LOG2_EPS;
         const float denom = big ? Ls + 1e-8f * fast_exp2(-Mu) : Ls * fast_exp2(Mu - LOG2_EPS) + 1.f;
         const float inv = big ? 1.f / denom : fast_exp2(Mu - LOG2_EPS) / denom;
-        uint16_t* orow = (uint16_t*)p.out.p + p.out.off(b, io, h) + c0;
+        uint16_t* orow = (uint16_t*)p.out.p + p.out.off(b, io, h);
 #pragma unroll
-        for (int x = 0; x < C::DT; ++x) {
+        for (int x = 0; x < DT; ++x) {
             const int col = 32 * x + 4 * (tid & 7);
             float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
             for (int w = 0; w < WW; ++w) {
-                const float4 y = *(const float4*)(mrg + (w * 32 + row) * C::AS + col);
+                const float4 y = *(const float4*)(mrg + (w * 32 + row) * AS + col);
                 acc.x += wgt[w] * y.x; acc.y += wgt[w] * y.y; acc.z += wgt[w] * y.z; acc.w += wgt[w] * y.w;
             }
-            *(uint2*)(orow + col) = make_uint2(E::pack(acc.x * inv, acc.y * inv), E::pack(acc.z * inv, acc.w * inv));
+            if constexpr (SPLIT) *(float4*)(part + col) = acc;
+            else *(uint2*)(orow + col) = make_uint2(E::pack(acc.x * inv, acc.y * inv), E::pack(acc.z * inv, acc.w * inv));
         }
-        if ((tid & 7) == 0 && blockIdx.y == 0)
-            p.lse[(int64_t)bh * N + io] = big ? LN2 * Mu + logf(denom) : LN_EPS + logf(denom);
+        if ((tid & 7) == 0) {
+            if constexpr (SPLIT) ((float2*)p.scratch)[prow] = make_float2(Mx, Ls);
+            else p.lse[(int64_t)bh * N + io] = big ? LN2 * Mu + logf(denom) : LN_EPS + logf(denom);
+        }
     }
+    return false;
+}
+
+// (A function of its own, so that its registers do not count where the first pass allocates its: inlined, it pushed the
+// output accumulator of the first pass to scratch memory.)
+template <class E, bool SPLIT>
+__device__ __attribute__((noinline))
+void wide_fwd_again(const Problem __attribute__((address_space(4))) * p, int nqb, int total, uint32_t lds) {
+    wide_fwd_block<E, SPLIT, true>(*(const Problem*)p, nqb, total, (unsigned char*)(__attribute__((address_space(3))) unsigned char*)(uintptr_t)lds);
+}
+template <class E, bool SPLIT>
+__global__ __launch_bounds__(WT) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void wide_fwd_kernel(Problem p, int nqb, int total) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_w[];
+    if (wide_fwd_block<E, SPLIT, false>(p, nqb, total, smem_w))              // (uniform over the workgroup)
+        wide_fwd_again<E, SPLIT>((const Problem __attribute__((address_space(4)))*)__builtin_amdgcn_kernarg_segment_ptr(), nqb, total, lds_address(smem_w));
 }
 
 // ============================================== backward, K' side: dQ, dK', dV' =====
@@ -836,15 +1090,18 @@ size_t wide_dq_part_bytes(int B, int N, int H, int D, int w2) {
 }
 
 // ------------------------------------------------------------------ launchers ----
-template <class E, int D, int DV>
-int launch_wide_fwd(const Problem& p, hipStream_t st) {
-    using C = WideCfg<D, DV>;
-    const int nqb = (p.N + BQ - 1) / BQ;
-    const int64_t total = (int64_t)nqb * p.B * p.H;
+template <class E>
+int launch_wide_fwd_of(const Problem& p, hipStream_t st) {
+    const int nqb = (p.N + BQ - 1) / BQ, nsplit = p.nsplit > 1 ? p.nsplit : 1;
+    const int64_t total = (int64_t)nqb * p.B * p.H * nsplit;
     if (total > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
-    if (!allow_full_lds((const void*)wide_fwd_kernel<E, D, DV>)) return SA2_ERR_LAUNCH_FAILED;
-    hipLaunchKernelGGL((wide_fwd_kernel<E, D, DV>), dim3((unsigned)total, C::NPASS), dim3(WT), C::FWD_LDS, st, p, nqb, (int)total);
-    return hipGetLastError() == hipSuccess ? SA2_OK : SA2_ERR_LAUNCH_FAILED;
+    auto go = [&](auto kernel) {
+        if (!allow_full_lds((const void*)kernel)) return false;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(WT), WIDE_FWD_LDS, st, p, nqb, (int)total);
+        return hipGetLastError() == hipSuccess;
+    };
+    if (!(nsplit > 1 ? go(wide_fwd_kernel<E, true>) : go(wide_fwd_kernel<E, false>))) return SA2_ERR_LAUNCH_FAILED;
+    return nsplit > 1 ? launch_fwd_merge(p, 256, E::DTYPE, st) : SA2_OK;
 }
 
 template <class E, int D, int DV>
@@ -916,8 +1173,10 @@ size_t wide_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2) {
     return wide_dq_part_bytes(B, N, H, D, w2) + (ns > 1 ? (size_t)2 * ns * B * H * (size_t)N * D * sizeof(float) : 0);
 }
 
+int wide_fwd_nsplit(int B, int N, int H, int w1, int w2) { return plan_forward(B, N, H, 256, w1, w2, WW); }
+
 int launch_wide_fwd(const Problem& p, int dtype, hipStream_t st) {
-    return dtype == SA2_F16 ? launch_wide_fwd<ElemF16, 256, 128>(p, st) : launch_wide_fwd<ElemBF16, 256, 128>(p, st);
+    return dtype == SA2_F16 ? launch_wide_fwd_of<ElemF16>(p, st) : launch_wide_fwd_of<ElemBF16>(p, st);
 }
 
 int launch_wide_bwd(const Problem& p, int dtype, hipStream_t st) {
