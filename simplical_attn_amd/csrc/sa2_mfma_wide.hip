@@ -2,27 +2,23 @@
 // (bf16 or fp16), forward and backward, on v_mfma_f32_32x32x16_bf16 / _f16.
 //
 // Same expanded-row view as the tuned kernels (rows r = (i, delta), Q~[r] = q[i] * k2~[i-delta] *
-// scale*log2(e), dO~[r] = dO[i] * v2~[i-delta], both rounded to the element type), in the simple
-// arrangement of the fp32 MFMA kernels: four wavefronts per workgroup, one per SIMD with the whole
-// register file, 32-row tiles row-major in a double-buffered LDS stage written from registers, one
-// barrier per tile.  Row operands are 16-byte reads of a tile row; transposed operands (the tile's
-// rows as the contraction index) come from the same tile through ds_read_b64_tr_b16, with a row
-// stride that keeps both kinds of read free of bank conflicts.
-//
-// A head_dim of 256 does not leave room for the operands of the logit contraction (64 registers) next
-// to accumulators for all 256 output columns of two contractions, so the backward kernels take the output
-// columns in passes of DV = 128 (grid dimension y): a pass contracts the logits over the whole
-// head_dim and accumulates its own 128 columns of R, G, dK, dV.  The logits (and dP) are computed
-// once per pass: 1.33x the backward's algorithmic MFMA work.
+// scale*log2(e), dO~[r] = dO[i] * v2~[i-delta], both rounded to the element type).  Four wavefronts per
+// workgroup, one per SIMD with all 512 registers: that is room for a row operand of 256 columns and for
+// the accumulators of all 256 output columns of two contractions, so that nothing is computed twice.
+// (The arrangement before took the output columns in two passes of 128, each with the logits over the
+// whole head_dim: 1.5x the forward's and 1.33x the backward's MFMA work, and left the matrix pipe idle
+// under every wait and every piece of vector arithmetic.)  A lone wavefront hides its latencies itself:
+// operand reads are opaque instructions issued one or two blocks of MFMAs ahead of their use, waits count
+// outstanding LDS operations, vector arithmetic stands between the MFMAs, and accumulators that live
+// through a sweep are pinned to accumulation registers.
 //
 //   wide_fwd_kernel   32 queries per workgroup; wavefront w takes delta = w, w+4, ... with one online
 //                     softmax and one output accumulator across its units, merged once at the end.
-//   wide_kp_kernel    32 K' rows per workgroup and every delta; the unit's reductions (dK', dV' rows
-//                     aligned with the unit's rows, dQ rows shifted by delta) go to fp32 accumulators
-//                     in LDS in column-rotated phases; dQ leaves as a per-workgroup partial that
-//                     wide_dq_sum_kernel adds up in block order.
+//   wide_kp_kernel    32 K' rows per workgroup and a run of deltas, two pairs of wavefronts.
 //   wide_kv_kernel    128 K/V rows per workgroup (32 per wavefront, resident in registers as B
 //                     operands), streaming every unit (query block, delta) that can see them.
+// Measured at B1 H8 N4096 w 512/32, bf16 (us, two column passes -> now): 2215 -> 890, 3860 -> 2170, 4900 -> 1530; the MFMAs'
+// rate inside the sweeps is 0.9 to 1.0 PFLOP/s, where a large matrix product reaches 1.2 on this card.
 // Every output element has one writer and a fixed summation order: no atomics, bitwise reproducible.
 #include "sa2_mfma_common.h"
 
@@ -32,39 +28,12 @@ namespace {
 constexpr int WW = 4;                  // wavefronts per workgroup
 constexpr int WT = WW * 64;            // threads per workgroup
 constexpr int WJ = WW * 32;            // K rows per workgroup of the K-side kernel
-
+constexpr int WKV_SIDE = 40;           // K' and V' rows the K-side kernel keeps in LDS: the 32 of a unit, and eight to come or past
+constexpr int WKP_DQ = 34;             // dQ rows the K'-side kernel keeps in LDS: the 33 of a round, and one to make pairs
 constexpr int WSIDE = 36;              // K' and V' rows the forward keeps in LDS: the 35 of a round, and one to make pairs
 
+typedef float fx4 __attribute__((ext_vector_type(4)));
 typedef unsigned ux4 __attribute__((ext_vector_type(4)));     // 16 bytes in flight (a plain vector: stays in registers)
-
-template <int D, int DV>
-struct WideCfg {
-    static_assert(D % 32 == 0 && DV % 32 == 0 && D % DV == 0, "32-column blocks");
-    static constexpr int DK = D / 16;          // k-steps of a contraction over head_dim
-    static constexpr int DT = DV / 32;         // 32-column blocks of a pass's output columns
-    static constexpr int NPASS = D / DV;
-    static constexpr int RS = D + 16;          // tile row stride (elements): rows lie 8 banks apart
-    static constexpr int RSB = RS * 2;         // ... in bytes
-    static constexpr int TILE = 32 * RS;       // elements
-    static constexpr int STAGE = 2 * TILE;     // two tiles (K and V, or Q~ and dO~)
-    static constexpr int KR = 32 * D / 8 / WT; // 16-byte chunks per thread and tile
-    static constexpr int AS = DV + 4;          // row stride of the fp32 accumulators in LDS
-    static constexpr size_t TILES_BYTES = (size_t)2 * STAGE * 2;
-    static constexpr size_t MERGE_BYTES = (size_t)WW * 32 * AS * 4;
-    static constexpr size_t FWD_LDS = (TILES_BYTES > MERGE_BYTES ? TILES_BYTES : MERGE_BYTES) + 2 * WW * 32 * 4;
-    static constexpr size_t LDS_LIMIT = 160 * 1024;
-    static size_t kp_lds(int w2) { return TILES_BYTES + (size_t)(32 + w2 + 64) * AS * 4; }
-    static bool kp_fits(int w2) { return kp_lds(w2) <= LDS_LIMIT; }
-    // deltas whose dQ rows the accumulator holds at once: all w2 + 1 of them, or (wider K' windows) the largest
-    // multiple of four that fits; the kernel then walks the window in segments of that many deltas
-    static int kp_segment(int w2) {
-        if (kp_fits(w2)) return w2 + 1;
-        int segw = 32;
-        while (kp_fits(segw + WW - 1)) segw += WW;
-        return segw;
-    }
-    static constexpr size_t KV_LDS = TILES_BYTES + 2 * 2 * 32 * 4;
-};
 
 __device__ __forceinline__ floatx16 zeros16() {
     floatx16 z;
@@ -72,67 +41,6 @@ __device__ __forceinline__ floatx16 zeros16() {
     for (int v = 0; v < 16; ++v) z[v] = 0.f;
     return z;
 }
-// Rows [j0, j0+32) of two tensors (clamped to the sequence) from global memory to registers, and
-// from there to the two tiles of a stage.
-template <int D, int DV, int KR>
-__device__ __forceinline__ void wide_load(ux4 (&a)[KR], ux4 (&b)[KR], const uint16_t* ap, int64_t as,
-                                          const uint16_t* bp, int64_t bs, int j0, int N, int tid) {
-#pragma unroll
-    for (int u = 0; u < KR; ++u) {
-        const int c = tid + WT * u;
-        const int row = c / (D / 8), col = c - row * (D / 8);
-        int j = j0 + row;
-        j = j < N ? j : N - 1;
-        a[u] = *(const ux4*)(ap + (int64_t)j * as + col * 8);
-        b[u] = *(const ux4*)(bp + (int64_t)j * bs + col * 8);
-    }
-}
-template <int D, int DV, int KR>
-__device__ __forceinline__ void wide_store(const ux4 (&a)[KR], const ux4 (&b)[KR], uint16_t* stage, int tid) {
-    using C = WideCfg<D, DV>;
-#pragma unroll
-    for (int u = 0; u < KR; ++u) {
-        const int c = tid + WT * u;
-        const int row = c / (D / 8), col = c - row * (D / 8);
-        *(ux4*)(stage + row * C::RS + col * 8) = a[u];
-        *(ux4*)(stage + C::TILE + row * C::RS + col * 8) = b[u];
-    }
-}
-
-// Lane part of a transposed operand read out of a row-major tile: within 16 lanes, lane s supplies the
-// address of row s/4, columns 4*(s%4)..+3, and lane i receives column i of those four rows; the four
-// 16-lane groups of a wavefront take the rows 0-3 / 4-7 (by half) of the 16-column halves of a 32-column
-// block.  The operand of k-step ks and column block c is then the reads at
-//   tile + lane part + (16*ks) * row stride + 2*c     and     ... + (16*ks + 8) * row stride ...
-// whose eight values are, in order, the k-slots of a 32x32 accumulator handed on as the other operand.
-template <int RSB>
-__device__ __forceinline__ uint32_t tr_lane_offset(int lane) {
-    const int grp = lane >> 4, s = lane & 15;
-    return (uint32_t)((4 * (grp >> 1) + (s >> 2)) * RSB + (16 * (grp & 1) + 4 * (s & 3)) * 2);
-}
-template <class X8, int RSB>
-__device__ __forceinline__ X8 tr_operand(uint32_t addr) {
-    typedef short v4s __attribute__((ext_vector_type(4)));
-    typedef v4s __attribute__((address_space(3)))* lds_v4s;
-    union { v4s h[2]; X8 v; } u;
-    u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(uintptr_t)addr);
-    u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(uintptr_t)(addr + 8 * RSB));
-    return u.v;
-}
-
-// a[r] * (b[r] + bias) [* mul] of two 16-byte chunks (8 elements), rounded to the element type
-template <class E>
-__device__ __forceinline__ typename E::x8 product8(const ux4& a, const ux4& b, float bias, float mul) {
-    typedef typename E::scalar EL;
-    typename E::x8 r;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        r[2 * t] = (EL)(E::lo(a[t]) * mul * (E::lo(b[t]) + bias));
-        r[2 * t + 1] = (EL)(E::hi(a[t]) * mul * (E::hi(b[t]) + bias));
-    }
-    return r;
-}
-
 template <class E>
 __device__ __forceinline__ uint32_t pack2(float a, float b) {
     typedef float f2 __attribute__((ext_vector_type(2)));
@@ -140,6 +48,17 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
     v.h = __builtin_convertvector((f2){a, b}, typename E::x2);
     return v.u;
 }
+// a[r] * mul * (b[r] + bias) of two 16-byte chunks (8 elements), rounded to the element type
+template <class E, bool BIASED = true>
+__device__ __forceinline__ typename E::x8 product8(const ux4& a, const ux4& b, float bias, float mul) {
+    union { uint32_t w[4]; typename E::x8 v; } r;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+        r.w[t] = BIASED ? pack2<E>(E::lo(a[t]) * mul * (E::lo(b[t]) + bias), E::hi(a[t]) * mul * (E::hi(b[t]) + bias))
+                        : pack2<E>(E::lo(a[t]) * mul * E::lo(b[t]), E::hi(a[t]) * mul * E::hi(b[t]));
+    return r.v;
+}
+
 // ---- tiles -----------------------------------------------------------------------
 // A 32-row tile of a 256-column tensor in LDS: sixteen groups of two rows, each written by one direct
 // global->LDS load of a wavefront (1 KB; lane L puts the 16-byte chunk L / 2 of row L % 2 at byte 16 * L)
@@ -151,6 +70,9 @@ struct WT256 {
     static constexpr int BYTES = NGROUP * GROUP;
     static constexpr int row_off(int r) { return (r / RPW) * GROUP + (r % RPW) * 16; }
 };
+constexpr size_t WIDE_KP_LDS = (size_t)4 * WT256::BYTES + 2 * 6144 + 2 * (WSIDE / 2) * WT256::GROUP + (size_t)WKP_DQ * 260 * 4;
+static_assert(WIDE_KP_LDS >= (size_t)WW * 32 * 260 * 4 && WIDE_KP_LDS <= 160 * 1024, "the last sums lie over everything");
+constexpr size_t WIDE_KV_LDS = (size_t)6 * WT256::BYTES + 2 * (WKV_SIDE / 2) * WT256::GROUP + 2 * 2 * 32 * 4;
 constexpr size_t WIDE_FWD_LDS = (size_t)7 * WT256::BYTES + 2 * (WSIDE / 2) * WT256::GROUP;
 static_assert(WIDE_FWD_LDS >= (size_t)WW * 32 * 260 * 4 + 2 * WW * 32 * 4 && WIDE_FWD_LDS <= 160 * 1024, "the merge lies over the tiles");
 typedef __attribute__((address_space(3))) void* wide_lds_ptr;
@@ -181,6 +103,86 @@ __device__ __forceinline__ void wide_tr_issue(uint32_t addr, lds_half_operand (&
         constexpr int o = (DT0 + I) * 64 * WT256::RPW + WT256::row_off(16 * KS);
         lds_tr_issue<o, o + WT256::row_off(8)>(addr, h[2 * I], h[2 * I + 1]);
         wide_tr_issue<KS, DT0, N, I + 1>(addr, h);
+    }
+}
+// acc += a * b with the accumulator in accumulation registers.  Opaque: beside 256 registers of accumulators that live
+// through a whole sweep the compiler's own placement moves some of them to scratch memory in every step.  Operands that
+// the vector ALU writes pass through settle_operand first; results are read behind settle_acc.
+template <class X8>
+__device__ __forceinline__ void mfma_acc(floatx16& acc, const X8& a, const X8& b) {
+    if constexpr (std::is_same<X8, bf16x8>::value) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+    else asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+}
+// The same into vector registers, for results that the vector ALU reads: at least four more MFMAs are issued before it
+// does (see wait_acc), which outlasts the matrix pipe's latency.
+template <class X8>
+__device__ __forceinline__ void mfma_vec(floatx16& acc, const X8& a, const X8& b) {
+    if constexpr (std::is_same<X8, bf16x8>::value) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+    else asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+}
+template <class X8>
+__device__ __forceinline__ void mfma_vec_zero(floatx16& acc, const X8& a, const X8& b) {          // acc = a * b
+    if constexpr (std::is_same<X8, bf16x8>::value) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "v"(b));
+    else asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "v"(b));
+}
+// Accumulators start from here rather than from a constant, and every loop over MFMAs keeps them out of its branches:
+// a value that meets another one of vector registers is copied between the two files in every step.
+template <int N>
+__device__ __forceinline__ void zero_acc(floatx16 (&acc)[N]) {
+    bf16x8 z;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) z[t] = (__bf16)0.f;
+    asm volatile("s_nop 3" : "+v"(z));
+#pragma unroll
+    for (int x = 0; x < N; ++x) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %1, 0" : "=a"(acc[x]) : "v"(z));
+}
+__device__ __forceinline__ void settle_c(floatx16& acc) { asm volatile("s_nop 3" : "+v"(acc)); }
+__device__ __forceinline__ void wait_acc(floatx16& acc) { asm volatile("s_nop 7" : "+v"(acc)); }
+template <class X8>
+__device__ __forceinline__ void settle_operand(X8 (&x)[2]) { asm volatile("s_nop 3" : "+v"(x[0]), "+v"(x[1])); }
+__device__ __forceinline__ void settle_halves(lds_half_operand (&x)[8]) {
+    asm volatile("s_nop 3" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]));
+}
+template <int N>
+__device__ __forceinline__ void settle_acc(floatx16 (&acc)[N]) {
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+    for (int x = 0; x < N; ++x) asm volatile("" : "+a"(acc[x]));
+}
+// 16 bytes from / to LDS as opaque operations, in the order of the program
+template <int OFF, class V>
+__device__ __forceinline__ void lds_read16(uint32_t addr, V& v) { asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(v) : "v"(addr), "n"(OFF)); }
+template <int OFF, class V>
+__device__ __forceinline__ void lds_write16(uint32_t addr, const V& v) { asm volatile("ds_write_b128 %0, %1 offset:%2" ::"v"(addr), "v"(v), "n"(OFF) : "memory"); }
+__device__ __forceinline__ void opaque(int& x) { asm volatile("" : "+v"(x)); }
+template <class V>
+__device__ __forceinline__ void arrived(V& a, V& b) { asm volatile("" : "+v"(a), "+v"(b)); }          // (behind the wait for them)
+// keeps values that the vector ALU updates between two sweeps in accumulation registers during them
+template <int N>
+__device__ __forceinline__ void stay_acc(floatx16 (&acc)[N]) {
+#pragma unroll
+    for (int x = 0; x < N; ++x) asm volatile("" : "+a"(acc[x]));
+}
+// Row operands of the k-steps K0 .. K0+3
+template <int K0, int I = 0, class X8>
+__device__ __forceinline__ void wide_rows4(uint32_t addr, X8 (&r)[4]) {
+    if constexpr (I < 4) {
+        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(r[I]) : "v"(addr), "n"((K0 + I) * 32 * WT256::RPW));
+        wide_rows4<K0, I + 1>(addr, r);
+    }
+}
+// at most PENDING LDS operations issued so far are outstanding; the halves named here may be used from here on
+template <int PENDING>
+__device__ __forceinline__ void lds_wait_halves(lds_half_operand (&x)[8]) {
+    asm volatile("s_waitcnt lgkmcnt(%8)"
+                 : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7])
+                 : "n"(PENDING));
+}
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for<N, I + 1>(f);
     }
 }
 // Row operands of the k-steps K0 .. K0+7
@@ -589,276 +591,405 @@ void wide_fwd_kernel(Problem p, int nqb, int total) {
 }
 
 // ============================================== backward, K' side: dQ, dK', dV' =====
-// SEG: the K' window is walked in segments of segw deltas (a kernel of its own; segw = w2 + 1 otherwise)
-template <class E, int D, int DV, bool SEG>
+// A workgroup owns 32 consecutive K' rows k0 .. k0+31 and a run of deltas (all of them, or a segment where the K' blocks
+// alone leave the chip idle); unit delta is the 32 expanded rows (i = k + delta, k).  Two pairs of wavefronts hold one
+// unit each per round and sweep the K/V window in 32-key tiles, two tiles of each in LDS.  In a pair one wavefront works
+// on the K tile only, S^T = K1.Q~^T and G^T += K1^T.dS^T, the other on the V tile only, dP^T = V1.dO~^T and
+// R^T += V1^T.P^T; half way through a step they exchange P (16 bit, as the MFMA takes it) and dP - D (fp32).  So each holds
+// one row operand and one output of all 256 columns, and beside them the sum over its deltas of G*q (dK') or R*dO (dV'),
+// which are aligned with the K' rows.  dQ rows are shifted by delta: a ring of fp32 rows in LDS, whose two oldest rows
+// leave for the workgroup's partial after every round.
+// What bounds it: in the sweep the matrix pipe (1.25 us per step of 32 MFMAs per wavefront), and between two sweeps the sums
+// over the unit (9 us per round, 30 % of the time at a K window of 512).  The second half of a step's last contraction runs
+// in the next step, from registers: it covers that step's first LDS reads and the exponentials.  The K' row stays in
+// registers although some of it is pushed to scratch memory in the sweep: reading it from the tensor again in every round
+// measured 2340 against 2200 us.  B1 H8 N4096 w 512/32 bf16: 3860 us in two column passes, 2170 now.
+template <class E, bool BIASED>
 __global__ __launch_bounds__(WT) __attribute__((amdgpu_waves_per_eu(1, 1)))
-void wide_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_part, int segw) {
+void wide_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_part, int nseg, int segw, float* __restrict__ kpart) {
     typedef typename E::scalar EL;
     typedef typename E::x8 X8;
-    using C = WideCfg<D, DV>;
+    constexpr int D = 256, DK = 16, DT = 8, TB = WT256::BYTES, AS = D + 4;
+    constexpr int RING = WSIDE / 2;                          // pairs of rows in the rings of q and dO rows
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_w[];
-    uint16_t* tiles = (uint16_t*)smem_w;
-    float* dk_s = (float*)(smem_w + C::TILES_BYTES);     // [32][AS]: dK' rows k0 .. k0+31 (before the scale)
-    float* dv_s = dk_s + 32 * C::AS;                     // [32][AS]: dV' rows
-    float* dq_s = dv_s + 32 * C::AS;                     // [32 + segw - 1][AS]: dQ rows k0 + dbase .. of the current segment (before the scale)
+    unsigned char* px = smem_w + 4 * TB;                     // (K tiles, then V tiles)  [pair][P: 2 KB, dP: 4 KB]
+    unsigned char* q_s = px + 2 * 6144;
+    unsigned char* do_s = q_s + RING * WT256::GROUP;
+    float* dq_s = (float*)(do_s + RING * WT256::GROUP);      // [WKP_DQ][AS]
 
-    const int tid = threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lane = tid & 63, ln = lane & 31, hf = lane >> 5;
-    const int pid = xcd_order(blockIdx.x, total);
-    const int c0 = blockIdx.y * DV;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int role = wave >> 1, pair = wave & 1;             // role 0: K tile, 1: V tile
+    // (segments one after the other in launch order: the last one is the short one)
+    const int per_seg = total / nseg, seg = (int)blockIdx.x / per_seg;
+    const int pid = xcd_order((int)blockIdx.x - seg * per_seg, per_seg);
     const int bh = pid / nkb, kb = pid - bh * nkb;
     const int b = bh / p.H, h = bh - b * p.H;
     const int N = p.N, w1 = p.w1, w2 = p.w2;
-    const int k0 = kb * BQ, k = k0 + ln, kc = k < N ? k : N - 1;
-    const int NR = 32 + w2;                      // rows of the block's dQ partial
-    const int NRS = 32 + segw - 1;               // rows of the accumulator
-    int dbase = 0;                               // first delta of the current segment
-
-    const uint16_t* qp = (const uint16_t*)p.q.p + p.q.off(b, 0, h);
-    const uint16_t* k1p = (const uint16_t*)p.k1.p + p.k1.off(b, 0, h);
-    const uint16_t* k2p = (const uint16_t*)p.k2.p + p.k2.off(b, 0, h);
-    const uint16_t* v1p = (const uint16_t*)p.v1.p + p.v1.off(b, 0, h);
-    const uint16_t* v2p = (const uint16_t*)p.v2.p + p.v2.off(b, 0, h);
-    const uint16_t* dop = (const uint16_t*)p.dout.p + p.dout.off(b, 0, h);
+    const int k0 = kb * BQ, kq = k0 + seg * segw;            // query of K' row k0 at the first delta
+    const int nu_all = (w2 < N - 1 - k0 ? w2 : N - 1 - k0) + 1 - seg * segw;
+    const int n_units = nu_all < segw ? nu_all : segw;       // (may be <= 0)
+    const int nrounds = n_units > 0 ? (n_units + 1) / 2 : 0;
+    const int RQ = BQ + segw - 1;                            // rows of the dQ partial
     const bool want_dq = p.dq.p != nullptr;
 
-    const int n_units = (w2 < N - 1 - k0 ? w2 : N - 1 - k0) + 1;       // delta with k0 + delta < N
-    const int nrounds = (n_units + WW - 1) / WW;
-    const float qscale = p.scale * LOG2E;
-    const uint32_t tiles_addr = lds_address(tiles);
-    const uint32_t tr_lane = tr_lane_offset<C::RSB>(lane);
+    const uint16_t* k1p = (const uint16_t*)p.k1.p + p.k1.off(b, 0, h);
+    const uint16_t* v1p = (const uint16_t*)p.v1.p + p.v1.off(b, 0, h);
+    const uint16_t* qp = (const uint16_t*)p.q.p + p.q.off(b, 0, h);
+    const uint16_t* dop = (const uint16_t*)p.dout.p + p.dout.off(b, 0, h);
 
-    for (int c = tid; c < (NRS + 64) * C::AS; c += WT) dk_s[c] = 0.f;      // all three accumulators
-
-    ux4 tk[C::KR], tv[C::KR];
-    for (int round = 0; round < nrounds; ++round) {
-        // queries of the round's units: k0 + 4*round .. k0 + 31 + 4*round + 3 (within the sequence)
-        const int d_first = round * WW, d_last = d_first + WW - 1 < n_units - 1 ? d_first + WW - 1 : n_units - 1;
-        const int i_min = k0 + d_first, i_max = k0 + 31 + d_last < N - 1 ? k0 + 31 + d_last : N - 1;
-        const int jt_lo = (i_min - w1 > 0 ? i_min - w1 : 0) / TJ, jt_hi = i_max / TJ;
-        const int nt = jt_hi - jt_lo + 1;
-
-        const int delta = d_first + wave;
-        const bool ok = delta < n_units;
-        const int i = k + delta, ic = i < N ? i : N - 1;
-        const bool row_ok = ok && i < N;
-        const int iw_lo = k0 + delta, iw_hi = k0 + 31 + delta < N - 1 ? k0 + 31 + delta : N - 1;   // this unit's queries
-        const bool rows_full = k0 + 31 + delta < N;
-
-        X8 qf[C::DK], dof[C::DK];
-        float lse2 = 0.f, dsum = 0.f;
-        if (ok) {
-#pragma unroll
-            for (int kk = 0; kk < C::DK; ++kk) {
-                const int col = kk * 16 + hf * 8;
-                const ux4 qa = *(const ux4*)(qp + (int64_t)ic * p.q.sn + col);
-                const ux4 ka = *(const ux4*)(k2p + (int64_t)kc * p.k2.sn + col);
-                const ux4 da = *(const ux4*)(dop + (int64_t)ic * p.dout.sn + col);
-                const ux4 va = *(const ux4*)(v2p + (int64_t)kc * p.v2.sn + col);
-                qf[kk] = product8<E>(qa, ka, p.k2_bias, qscale);
-                dof[kk] = product8<E>(da, va, p.v2_bias, 1.f);
-            }
-            lse2 = p.lse[(int64_t)bh * N + ic] * LOG2E;
-            dsum = p.dsum[(int64_t)bh * N + ic];
+    auto here = [&]() {                                      // (lane parts are computed where they are used)
+        int t = threadIdx.x;
+        opaque(t);
+        return t & 63;
+    };
+    // ---- tiles: step g works on slot g & 1 and asks for the tile of step g + 1 (of this round or the next) ----
+    auto round_first = [&](int r) {
+        const int i_min = kq + 2 * r;
+        return (i_min - w1 > 0 ? i_min - w1 : 0) / TJ;
+    };
+    auto round_last = [&](int r) {
+        const int d = 2 * r + 1 < n_units - 1 ? 2 * r + 1 : n_units - 1;
+        const int i_max = kq + d + BQ - 1 < N - 1 ? kq + d + BQ - 1 : N - 1;
+        return i_max / TJ;
+    };
+    int slot = 0, next_round = 0, next_tile = round_first(0), next_last = round_last(0);
+    auto request_tile = [&](int to) {
+        if (next_round < nrounds) {
+            const int lane = here();
+            const uint32_t r2 = 8 * wave + (lane & 1), c2 = (lane >> 1) * 8;
+            wide_request(k1p, p.k1.sn, next_tile * TJ, N, wave, lane, (r2 * (uint32_t)p.k1.sn + c2) * 2u, smem_w + to * TB);
+            wide_request(v1p, p.v1.sn, next_tile * TJ, N, wave, lane, (r2 * (uint32_t)p.v1.sn + c2) * 2u, smem_w + (2 + to) * TB);
         }
-        floatx16 racc[C::DT], gacc[C::DT];
-#pragma unroll
-        for (int dt = 0; dt < C::DT; ++dt) racc[dt] = gacc[dt] = zeros16();
-
-        // (the previous round's last barrier has passed: both stages are free)
-        wide_load<D, DV>(tk, tv, k1p, p.k1.sn, v1p, p.v1.sn, jt_lo * TJ, N, tid);
-        wide_store<D, DV>(tk, tv, tiles, tid);
-        wide_load<D, DV>(tk, tv, k1p, p.k1.sn, v1p, p.v1.sn, (jt_lo + 1 % nt) * TJ, N, tid);
-        __syncthreads();
-        for (int s = 0; s < nt; ++s) {
-            const int j0 = (jt_lo + s) * TJ;
-            // tiles that hold no key of this unit's windows are skipped by the wavefront
-            if (ok && j0 <= iw_hi && j0 + TJ - 1 >= iw_lo - w1) {
-                const uint16_t* Ks = tiles + (s & 1) * C::STAGE;
-                const uint16_t* Vs = Ks + C::TILE;
-                const uint32_t Kt = tiles_addr + (uint32_t)((s & 1) * C::STAGE * 2) + tr_lane + (uint32_t)(c0 * 2);
-                const uint32_t Vt = Kt + (uint32_t)(C::TILE * 2);
-                floatx16 sacc = zeros16(), dpacc = zeros16();
-#pragma unroll
-                for (int kk = 0; kk < C::DK; ++kk) {
-                    const X8 ka = *(const X8*)(Ks + ln * C::RS + kk * 16 + hf * 8);
-                    const X8 va = *(const X8*)(Vs + ln * C::RS + kk * 16 + hf * 8);
-                    sacc = E::mfma(ka, qf[kk], sacc, 0, 0, 0);
-                    dpacc = E::mfma(va, dof[kk], dpacc, 0, 0, 0);
-                }
-                const bool interior = rows_full && (j0 + TJ - 1 <= iw_lo) && (j0 >= iw_lo + 31 - w1);
-                const int hi = i - j0 - 4 * hf, lo = hi - w1;
-                X8 pb[2], dsb[2];
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int c = 8 * (v >> 2) + (v & 3);
-                    const bool valid = interior || (row_ok && c <= hi && c >= lo);
-                    const float pv = valid ? fast_exp2(sacc[v] - lse2) : 0.f;
-                    pb[v >> 3][v & 7] = (EL)pv;
-                    dsb[v >> 3][v & 7] = (EL)(pv * (dpacc[v] - dsum));
-                }
-#pragma unroll
-                for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-                    for (int dt = 0; dt < C::DT; ++dt) {
-                        const uint32_t o = (uint32_t)(16 * ks * C::RSB + dt * 64);
-                        racc[dt] = E::mfma(tr_operand<X8, C::RSB>(Vt + o), pb[ks], racc[dt], 0, 0, 0);
-                        gacc[dt] = E::mfma(tr_operand<X8, C::RSB>(Kt + o), dsb[ks], gacc[dt], 0, 0, 0);
-                    }
-            }
-            wide_store<D, DV>(tk, tv, tiles + ((s + 1) & 1) * C::STAGE, tid);
-            wide_load<D, DV>(tk, tv, k1p, p.k1.sn, v1p, p.v1.sn, (jt_lo + (s + 2) % nt) * TJ, N, tid);
-            __syncthreads();
+        if (next_tile == next_last) {
+            ++next_round;
+            next_tile = round_first(next_round);
+            next_last = round_last(next_round);
+        } else {
+            ++next_tile;
         }
-
-        // ---- the unit's reductions into the workgroup's LDS accumulators:
-        //      dK'[k] += G*q[i], dV'[k] += R*dO[i] (rows ln), dQ[i] += G*k2~[k] (rows ln + delta).
-        //      Four phases; in phase ph wavefront w owns column group (w + ph) % 4 of every row, so no
-        //      two wavefronts touch an element at once and every element sums in a fixed order. ----
-#pragma unroll
-        for (int ph = 0; ph < 4; ++ph) {
-            if (row_ok) {
-                const int g4 = (wave + ph) & 3;
-                const int col = 8 * g4 + 4 * hf;
-                const uint16_t* qrow = qp + (int64_t)ic * p.q.sn + c0 + col;
-                const uint16_t* drow = dop + (int64_t)ic * p.dout.sn + c0 + col;
-                const uint16_t* krow = k2p + (int64_t)kc * p.k2.sn + c0 + col;
-                float* dkrow = dk_s + ln * C::AS + col;
-                float* dvrow = dv_s + ln * C::AS + col;
-                float* dqrow = dq_s + (ln + delta - dbase) * C::AS + col;
-#pragma unroll
-                for (int dt = 0; dt < C::DT; ++dt) {
-                    // (g4 is uniform over the wavefront: pick this group's four registers)
-                    float gv[4], rv[4];
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) {
-                        gv[t] = g4 == 0 ? gacc[dt][t] : g4 == 1 ? gacc[dt][4 + t] : g4 == 2 ? gacc[dt][8 + t] : gacc[dt][12 + t];
-                        rv[t] = g4 == 0 ? racc[dt][t] : g4 == 1 ? racc[dt][4 + t] : g4 == 2 ? racc[dt][8 + t] : racc[dt][12 + t];
-                    }
-                    const uint2 qx = *(const uint2*)(qrow + dt * 32);
-                    const uint2 dx = *(const uint2*)(drow + dt * 32);
-                    float4 a = *(float4*)(dkrow + dt * 32);
-                    a.x += gv[0] * E::lo(qx.x); a.y += gv[1] * E::hi(qx.x); a.z += gv[2] * E::lo(qx.y); a.w += gv[3] * E::hi(qx.y);
-                    *(float4*)(dkrow + dt * 32) = a;
-                    float4 c = *(float4*)(dvrow + dt * 32);
-                    c.x += rv[0] * E::lo(dx.x); c.y += rv[1] * E::hi(dx.x); c.z += rv[2] * E::lo(dx.y); c.w += rv[3] * E::hi(dx.y);
-                    *(float4*)(dvrow + dt * 32) = c;
-                    if (want_dq) {
-                        const uint2 kx = *(const uint2*)(krow + dt * 32);
-                        float4 o = *(float4*)(dqrow + dt * 32);
-                        o.x += gv[0] * (E::lo(kx.x) + p.k2_bias); o.y += gv[1] * (E::hi(kx.x) + p.k2_bias);
-                        o.z += gv[2] * (E::lo(kx.y) + p.k2_bias); o.w += gv[3] * (E::hi(kx.y) + p.k2_bias);
-                        *(float4*)(dqrow + dt * 32) = o;
-                    }
-                }
-            }
-            __syncthreads();
-        }
-        // ---- end of a segment: its first segw dQ rows are complete and go to the partial; the 31 rows the next
-        //      segment shares with it move to the front of the accumulator ----
-        if (SEG && round + 1 < nrounds && (round + 1) * WW - dbase >= segw) {
-            if (want_dq) {
-                float* part = dq_part + (((int64_t)bh * nkb + kb) * (int64_t)NR + dbase) * D + c0;
-                for (int c = tid; c < segw * (DV / 4); c += WT) {
-                    const int r = c / (DV / 4), col = c - r * (DV / 4);
-                    *(float4*)(part + (int64_t)r * D + col * 4) = *(const float4*)(dq_s + r * C::AS + col * 4);
-                }
-                __syncthreads();
-                for (int c = tid; c < 31 * (DV / 4); c += WT) {         // (segw >= 32: source and destination are disjoint)
-                    const int r = c / (DV / 4), col = c - r * (DV / 4);
-                    *(float4*)(dq_s + r * C::AS + col * 4) = *(const float4*)(dq_s + (segw + r) * C::AS + col * 4);
-                }
-                __syncthreads();
-                for (int c = tid; c < (NRS - 31) * (DV / 4); c += WT) {
-                    const int r = 31 + c / (DV / 4), col = c % (DV / 4);
-                    *(float4*)(dq_s + r * C::AS + col * 4) = make_float4(0.f, 0.f, 0.f, 0.f);
-                }
-                __syncthreads();
-            }
-            dbase += segw;
-        }
+    };
+    // ---- q and dO rows kq + u, u in [2r, 2r+32] in round r: pair u / 2 at place (u / 2) % RING ----
+    auto request_rows = [&](const uint16_t* base, int64_t sn, int at, unsigned char* ring) {
+        const int lane = here();
+        const int i = kq + 2 * at + (lane & 1) < N ? kq + 2 * at + (lane & 1) : N - 1;
+        __builtin_amdgcn_global_load_lds((wide_glb_ptr)(base + (int64_t)i * sn + (lane >> 1) * 8),
+                                         (wide_lds_ptr)(ring + (at % RING) * WT256::GROUP), 16, 0, 0);
+    };
+    request_tile(0);
+    for (int x = wave; x < RING; x += WW) {
+        request_rows(qp, p.q.sn, x, q_s);
+        request_rows(dop, p.dout.sn, x, do_s);
     }
+    for (int c = threadIdx.x; c < WKP_DQ * AS; c += WT) dq_s[c] = 0.f;
 
-    // ---- dK' and dV' rows of the block (this pass's columns) ----
+    const Tensor& rt = role ? p.v2 : p.k2;                   // the wavefront's K' or V' row, as a row operand holds it
+    ux4 raw[DK];
     {
-        const int row = tid >> 3, ko = k0 + row;
-        if (ko < N) {
+        const int lane = here(), k = k0 + (lane & 31) < N ? k0 + (lane & 31) : N - 1;
+        const uint16_t* src = (const uint16_t*)rt.p + rt.off(b, k, h) + (lane >> 5) * 8;
 #pragma unroll
-            for (int x = 0; x < C::DT; ++x) {
-                const int col = 32 * x + 4 * (tid & 7);
-                if (p.dk2.p) {
-                    const float4 a = *(const float4*)(dk_s + row * C::AS + col);
-                    *(uint2*)((uint16_t*)p.dk2.p + p.dk2.off(b, ko, h) + c0 + col) =
-                        make_uint2(E::pack(a.x * p.scale, a.y * p.scale), E::pack(a.z * p.scale, a.w * p.scale));
+        for (int kk = 0; kk < DK; ++kk) raw[kk] = *(const ux4*)(src + kk * 16);
+    }
+#pragma unroll
+    for (int kk = 0; kk < DK; ++kk) asm volatile("" : "+v"(raw[kk]));
+    // LSE * log2(e) (role 0) or D (role 1) of the lane's row, one round ahead
+    auto row_value = [&](int r) {
+        const int i = kq + (here() & 31) + 2 * r + pair, ic = i < N ? i : N - 1;
+        return role ? p.dsum[(int64_t)bh * N + ic] : p.lse[(int64_t)bh * N + ic] * LOG2E;
+    };
+    float value_next = row_value(0);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+
+    const uint32_t lds0 = lds_address(smem_w);
+    auto k2_of = [&](float x) { return BIASED ? x + p.k2_bias : x; };
+    floatx16 pacc[DT];                                       // dK' before the scale (role 0), dV' (role 1)
+    zero_acc(pacc);
+
+    // dQ rows [u0, u1) of the ring to the partial, their places to zero
+    auto flush = [&](int u0, int u1, int t, int threads) {
+        float* part = dq_part + (((int64_t)bh * nkb + kb) * nseg + seg) * (int64_t)RQ * D;
+        for (int c = t; c < (u1 - u0) * (D / 4); c += threads) {
+            const int u = u0 + c / (D / 4), col = (c % (D / 4)) * 4;
+            float4* src = (float4*)(dq_s + (u % WKP_DQ) * AS + col);
+            float4 a = u < 2 * nrounds + 32 ? *src : make_float4(0.f, 0.f, 0.f, 0.f);
+            *(float4*)(part + (int64_t)u * D + col) = make_float4(a.x * p.scale, a.y * p.scale, a.z * p.scale, a.w * p.scale);
+            if (u < 2 * nrounds + 32) *src = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    };
+    auto sweep = [&](auto ROLE) {
+        constexpr int R = decltype(ROLE)::value;
+        unsigned char* rows_s = R ? do_s : q_s;
+        for (int round = 0; round < nrounds; ++round) {
+            const int delta = 2 * round + pair;              // relative to the segment
+            float value = value_next;
+            asm volatile("" : "+v"(value));
+            if (round + 1 < nrounds) value_next = row_value(round + 1);
+            X8 rf[DK];                                       // Q~ or dO~
+            {
+#pragma unroll
+                for (int kk = 0; kk < DK; ++kk) asm volatile("" : "+v"(raw[kk]));     // (unpacked here, not once for all rounds)
+                const int lane = here(), u = (lane & 31) + delta;
+                const unsigned char* src = rows_s + ((u >> 1) % RING) * WT256::GROUP + (u & 1) * 16 + (lane >> 5) * 32;
+#pragma unroll
+                for (int kk = 0; kk < DK; ++kk)
+                    rf[kk] = product8<E, BIASED>(*(const ux4*)(src + kk * 64), raw[kk], R ? p.v2_bias : p.k2_bias, R ? 1.f : p.scale * LOG2E);
+            }
+#pragma unroll
+            for (int kk = 0; kk < DK; ++kk) asm volatile("s_nop 1" : "+v"(rf[kk]));
+            floatx16 acc[DT];                                // G or R
+            zero_acc(acc);
+            stay_acc(pacc);
+            X8 ro[4][4];                                     // row operands of a chunk of four MFMAs
+            lds_half_operand ta[8], tb[8], pa[8], pc[8];     // transposed operands; pa, pc: of the half that runs in the next step
+            X8 wb[2];                                        // dS or P
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                pa[t] = pc[t] = lds_half_operand{0, 0, 0, 0};
+                wb[0][t] = wb[1][t] = (EL)0.f;
+            }
+            settle_operand(wb);
+            settle_halves(pa);
+            settle_halves(pc);
+            auto second = [&](lds_half_operand (&x)[8], int dt0, int ks, int y) { mfma_acc(acc[dt0 + y], lds_join<X8>(x[2 * y], x[2 * y + 1]), wb[ks]); };
+
+            const int tile_first = round_first(round), tile_last = round_last(round);
+            for (int jt = tile_first; jt <= tile_last; ++jt) {
+                const int lane = here(), ln = lane & 31, hf = lane >> 5;
+                const uint32_t tile = lds0 + (uint32_t)((2 * R + slot) * TB);
+                const uint32_t row_a = tile + (uint32_t)((ln / 2) * WT256::GROUP + (hf * 2 + (ln & 1)) * 16);
+                const uint32_t col_a = tile + lds_group_column_lane_offset<WT256::RPW, WT256::GROUP>(lane);
+                const uint32_t px_a = lds0 + (uint32_t)(4 * TB + pair * 6144 + lane * 16);
+                request_tile(slot ^ 1);
+                // ---- S or dP ----
+                wide_rows4<0>(row_a, ro[0]);
+                wide_rows4<4>(row_a, ro[1]);
+#pragma unroll
+                for (int y = 0; y < 4; ++y) second(pa, 0, 1, y);
+                wide_rows4<8>(row_a, ro[2]);
+                floatx16 s;
+                lds_wait<8>(ro[0]);
+                mfma_vec_zero(s, ro[0][0], rf[0]);
+#pragma unroll
+                for (int y = 1; y < 4; ++y) mfma_vec(s, ro[0][y], rf[y]);
+                wide_rows4<12>(row_a, ro[3]);
+                lds_wait<8>(ro[1]);
+#pragma unroll
+                for (int y = 0; y < 4; ++y) mfma_vec(s, ro[1][y], rf[4 + y]);
+                lds_wait<4>(ro[2]);
+#pragma unroll
+                for (int y = 0; y < 4; ++y) mfma_vec(s, ro[2][y], rf[8 + y]);
+                lds_wait<0>(ro[3]);
+#pragma unroll
+                for (int y = 0; y < 4; ++y) mfma_vec(s, ro[3][y], rf[12 + y]);
+                second(pc, 4, 1, 0);
+                second(pc, 4, 1, 1);
+                wait_acc(s);
+                if constexpr (R == 0) {
+                    // element v of this lane is key 32 * jt + 8*(v/4) + 4*hf + v%4, the row's query is kq + ln + delta
+                    const int j0 = jt * TJ, i_min = kq + delta;
+                    if (!(i_min + BQ - 1 < N && delta < n_units && j0 + TJ - 1 <= i_min && j0 >= i_min + BQ - 1 - w1)) {
+                        int hi = i_min + ln - j0 - 4 * hf;
+                        opaque(hi);
+                        const int lo = hi - w1;
+                        const bool row_ok = i_min + ln < N && delta < n_units;
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) {
+                            const int c = 8 * (v >> 2) + (v & 3);
+                            s[v] = row_ok && c <= hi && c >= lo ? s[v] : -INFINITY;
+                        }
+                    }
+                    X8 pw[2];
+#pragma unroll
+                    for (int g = 0; g < 2; ++g) {
+#pragma unroll
+                        for (int t = 0; t < 8; ++t) {
+                            s[8 * g + t] = fast_exp2(s[8 * g + t] - value);
+                            pw[g][t] = (EL)s[8 * g + t];
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                        second(pc, 4, 1, 2 + g);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    lds_write16<0>(px_a, pw[0]);
+                    lds_write16<1024>(px_a, pw[1]);
+                } else {
+                    fx4 d[4];
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) d[v >> 2][v & 3] = s[v] - value;
+                    second(pc, 4, 1, 2);
+                    second(pc, 4, 1, 3);
+                    lds_write16<2048>(px_a, d[0]);
+                    lds_write16<3072>(px_a, d[1]);
+                    lds_write16<4096>(px_a, d[2]);
+                    lds_write16<5120>(px_a, d[3]);
                 }
-                if (p.dv2.p) {
-                    const float4 a = *(const float4*)(dv_s + row * C::AS + col);
-                    *(uint2*)((uint16_t*)p.dv2.p + p.dv2.off(b, ko, h) + c0 + col) = make_uint2(E::pack(a.x, a.y), E::pack(a.z, a.w));
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                // (both pairs are past the rows of the round before: the places of its first two take the next ones)
+                if (round > 0 && jt == tile_first && pair == 0) {
+                    if constexpr (R == 0) request_rows(qp, p.q.sn, round + RING - 1, q_s);
+                    else request_rows(dop, p.dout.sn, round + RING - 1, do_s);
+                }
+                // ---- G or R: first half here, second half in the next step ----
+                if constexpr (R == 0) {
+                    fx4 d[4];
+                    lds_read16<2048>(px_a, d[0]);
+                    lds_read16<3072>(px_a, d[1]);
+                    lds_read16<4096>(px_a, d[2]);
+                    lds_read16<5120>(px_a, d[3]);
+                    wide_tr_issue<0, 0, 4>(col_a, ta);
+                    asm volatile("s_waitcnt lgkmcnt(8)" : "+v"(d[0]), "+v"(d[1]), "+v"(d[2]), "+v"(d[3]));
+                    wide_tr_issue<0, 4, 4>(col_a, tb);
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) wb[v >> 3][v & 7] = (EL)(s[v] * d[v >> 2][v & 3]);
+                    settle_operand(wb);
+                } else {
+                    lds_read16<0>(px_a, wb[0]);
+                    lds_read16<1024>(px_a, wb[1]);
+                    wide_tr_issue<0, 0, 4>(col_a, ta);
+                    asm volatile("s_waitcnt lgkmcnt(8)" : "+v"(wb[0]), "+v"(wb[1]));
+                    wide_tr_issue<0, 4, 4>(col_a, tb);
+                }
+                lds_wait_halves<8>(ta);
+#pragma unroll
+                for (int y = 0; y < 4; ++y) second(ta, 0, 0, y);
+                wide_tr_issue<1, 0, 4>(col_a, pa);
+                lds_wait_halves<8>(tb);
+#pragma unroll
+                for (int y = 0; y < 4; ++y) second(tb, 4, 0, y);
+                wide_tr_issue<1, 4, 4>(col_a, pc);
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                lds_wait_halves<0>(pa);
+                lds_wait_halves<0>(pc);
+                asm volatile("s_barrier" ::: "memory");
+                slot ^= 1;
+            }
+#pragma unroll
+            for (int y = 0; y < 4; ++y) second(pa, 0, 1, y);
+#pragma unroll
+            for (int y = 0; y < 4; ++y) second(pc, 4, 1, y);
+            settle_acc(acc);
+            // ---- sums over the unit's rows: dK'[k] += G * q[i] or dV'[k] += R * dO[i] ... ----
+            {
+                const int lane = here(), hf = lane >> 5, u = (lane & 31) + delta;
+                const unsigned char* src = rows_s + ((u >> 1) % RING) * WT256::GROUP + (u & 1) * 16 + hf * 8;
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int g4 = 0; g4 < 4; ++g4) {
+                        const uint2 x = *(const uint2*)(src + (4 * dt + g4) * 32);
+                        pacc[dt][4 * g4 + 0] += acc[dt][4 * g4 + 0] * E::lo(x.x);
+                        pacc[dt][4 * g4 + 1] += acc[dt][4 * g4 + 1] * E::hi(x.x);
+                        pacc[dt][4 * g4 + 2] += acc[dt][4 * g4 + 2] * E::lo(x.y);
+                        pacc[dt][4 * g4 + 3] += acc[dt][4 * g4 + 3] * E::hi(x.y);
+                    }
+                stay_acc(pacc);
+            }
+            // ... and dQ[k + delta] += G * k2~[k]: the two pairs' rows overlap, so each takes one half of the columns at a time ----
+            if (want_dq) {
+                if constexpr (R == 0) {
+                    auto add_dq = [&](auto HALF) {
+                        constexpr int dt0 = decltype(HALF)::value * 4;
+                        const int lane = here();
+                        float* row = dq_s + (((lane & 31) + delta) % WKP_DQ) * AS + (lane >> 5) * 4;
+#pragma unroll
+                        for (int kk = 2 * dt0; kk < 2 * dt0 + 8; ++kk) {
+                            // the row operand's 16-byte chunks as the accumulators' columns: 16*kk + 4*hf .. and 16*kk + 8 + 4*hf ..
+                            const auto e0 = __builtin_amdgcn_permlane32_swap(raw[kk][0], raw[kk][2], false, false);
+                            const auto e1 = __builtin_amdgcn_permlane32_swap(raw[kk][1], raw[kk][3], false, false);
+#pragma unroll
+                            for (int g = 0; g < 2; ++g) {
+                                const int dt = kk / 2, g4 = 2 * (kk & 1) + g;
+                                float4 a = *(float4*)(row + dt * 32 + 8 * g4);
+                                a.x += acc[dt][4 * g4 + 0] * k2_of(E::lo(e0[g]));
+                                a.y += acc[dt][4 * g4 + 1] * k2_of(E::hi(e0[g]));
+                                a.z += acc[dt][4 * g4 + 2] * k2_of(E::lo(e1[g]));
+                                a.w += acc[dt][4 * g4 + 3] * k2_of(E::hi(e1[g]));
+                                *(float4*)(row + dt * 32 + 8 * g4) = a;
+                            }
+                        }
+                    };
+                    if (pair) add_dq(std::integral_constant<int, 1>{});
+                    else add_dq(std::integral_constant<int, 0>{});
+                    __syncthreads();
+                    if (pair) add_dq(std::integral_constant<int, 0>{});
+                    else add_dq(std::integral_constant<int, 1>{});
+                    __syncthreads();
+                } else {
+                    __syncthreads();
+                    __syncthreads();
+                    flush(2 * round, 2 * round + 2, here() + pair * 64, 128);
                 }
             }
         }
-    }
-    // ---- dQ partial of this block: rows k0 .. k0+31+w2, this pass's columns ----
-    //      (those from dbase on are still here; rows past the accumulator belong to deltas beyond the end of the
-    //      sequence: zeros)
-    if (want_dq) {
-        float* part = dq_part + (((int64_t)bh * nkb + kb) * (int64_t)NR + dbase) * D + c0;
-        for (int c = tid; c < (NR - dbase) * (DV / 4); c += WT) {
-            const int r = c / (DV / 4), col = c - r * (DV / 4);
-            *(float4*)(part + (int64_t)r * D + col * 4) =
-                r < NRS ? *(const float4*)(dq_s + r * C::AS + col * 4) : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-    }
-}
+    };
+    if (role == 0) sweep(std::integral_constant<int, 0>{});
+    else sweep(std::integral_constant<int, 1>{});
 
-// dQ[i] = scale * sum over the K' blocks kb with 32*kb <= i <= 32*kb + 31 + w2, in block order
-template <class E, int D>
-__global__ __launch_bounds__(256) void wide_dq_sum_kernel(Problem p, int nkb, const float* __restrict__ dq_part, int64_t chunks) {
-    const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (c >= chunks) return;
-    const int col = (int)(c % (D / 4));
-    const int64_t rowid = c / (D / 4);
-    const int i = (int)(rowid % p.N);
-    const int bh = (int)(rowid / p.N);
-    const int b = bh / p.H, h = bh - b * p.H;
-    const int NR = 32 + p.w2;
-    const int kb_lo = (i - 31 - p.w2) <= 0 ? 0 : (i - p.w2) / 32;      // smallest kb with 32*kb + 31 + w2 >= i
-    const int kb_hi = i / 32;
-    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int kb = kb_lo; kb <= kb_hi; ++kb) {
-        const float4 y = *(const float4*)(dq_part + (((int64_t)bh * nkb + kb) * NR + (i - 32 * kb)) * D + col * 4);
-        acc.x += y.x; acc.y += y.y; acc.z += y.z; acc.w += y.w;
+    // ---- what is left of the dQ partial, then dK' and dV' (two wavefronts each) through LDS ----
+    __syncthreads();
+    if (want_dq) {
+        flush(2 * nrounds, RQ, threadIdx.x, WT);
+        __syncthreads();
     }
-    *(uint2*)((uint16_t*)p.dq.p + p.dq.off(b, i, h) + col * 4) =
-        make_uint2(E::pack(acc.x * p.scale, acc.y * p.scale), E::pack(acc.z * p.scale, acc.w * p.scale));
+    float* sums = (float*)smem_w;                            // [WW][32][AS]
+    {
+        const int lane = here();
+        float* row = sums + (wave * 32 + (lane & 31)) * AS + 4 * (lane >> 5);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4)
+                *(float4*)(row + dt * 32 + 8 * g4) = make_float4(pacc[dt][4 * g4], pacc[dt][4 * g4 + 1], pacc[dt][4 * g4 + 2], pacc[dt][4 * g4 + 3]);
+    }
+    __syncthreads();
+    for (int it = threadIdx.x; it < 2 * BQ * (D / 4); it += WT) {
+        const int which = it / (BQ * (D / 4));               // 0: dV', 1: dK'
+        const int r = it / (D / 4) % BQ, col = it % (D / 4) * 4, k = k0 + r;
+        const Tensor& t = which ? p.dk2 : p.dv2;
+        if (k >= N || !t.p) continue;
+        const float* src = sums + ((which ? 0 : 2) * 32 + r) * AS + col;
+        const float4 x = *(const float4*)src, y = *(const float4*)(src + 32 * AS);
+        const float sc = which ? p.scale : 1.f;
+        const float4 o = make_float4((x.x + y.x) * sc, (x.y + y.y) * sc, (x.z + y.z) * sc, (x.w + y.w) * sc);
+        if (nseg > 1) *(float4*)(kpart + ((((int64_t)which * nseg + seg) * p.B * p.H + bh) * N + k) * D + col) = o;
+        else *(uint2*)((uint16_t*)t.p + t.off(b, k, h) + col) = make_uint2(pack2<E>(o.x, o.y), pack2<E>(o.z, o.w));
+    }
 }
 
 // =================================================== backward, K side: dK, dV =====
-// nsplit > 1 (grids smaller than the chip): the workgroup takes the sp-th share of the key block's stream
-// of units and writes fp32 partial sums to `part` ([dK | dV][nsplit][B*H][N][D]) for wide_kv_sum_kernel.
-template <class E, int D, int DV, bool SPLIT>
+// A workgroup owns 128 K/V rows, 32 per wavefront, resident in registers as B operands beside the accumulators of all
+// 256 columns of dK and dV (384 of the 512 registers of the one wavefront per SIMD), and streams every unit (query
+// block, delta) that sees them.  The unit's Q~ and dO~ tiles are formed by all wavefronts from the block's q and dO rows
+// and a ring of K' and V' rows in LDS, one unit ahead.
+// What bounds it: power; without the forming the units run at the 1.2 PFLOP/s of a large matrix product, and the forming's
+// LDS traffic and arithmetic add a quarter.  B1 H8 N4096 w 512/32 bf16: 4900 us in two column passes, 1530 now.  A unit is
+// sixteen chunks of four MFMAs; the operands of a chunk are requested two chunks before, an eighth of the forming rides
+// on every second one, and the last two chunks run behind the unit's barrier, under the first operand reads of the next.
+// nsplit > 1 (grids smaller than the chip): the workgroup takes the sp-th share of the key block's stream of units and
+// writes fp32 partial sums to `part` ([dK | dV][nsplit][B*H][N][D]).
+template <class E, bool SPLIT, bool BIASED>
 __global__ __launch_bounds__(WT) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void wide_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __restrict__ part) {
     const int nsplit = SPLIT ? nsplit_arg : 1;
     typedef typename E::scalar EL;
     typedef typename E::x8 X8;
-    using C = WideCfg<D, DV>;
+    constexpr int D = 256, DK = 16, DT = 8, TB = WT256::BYTES;
+    constexpr int RING = WKV_SIDE / 2;                       // pairs of rows in a K'/V' ring
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_w[];
-    uint16_t* tiles = (uint16_t*)smem_w;
-    float* lse_s = (float*)(smem_w + C::TILES_BYTES);    // [2][32]  LSE*log2(e) of the unit's queries
-    float* dsum_s = lse_s + 2 * 32;                      // [2][32]
+    unsigned char* q_s = smem_w + 4 * TB;                    // (0 .. 3: the Q~ and dO~ tiles of two units)
+    unsigned char* do_s = q_s + TB;
+    unsigned char* k2_s = do_s + TB;
+    unsigned char* v2_s = k2_s + RING * WT256::GROUP;
+    float* lse_s = (float*)(v2_s + RING * WT256::GROUP);     // [2][32]  -LSE*log2(e) of the block's queries
+    float* dsum_s = lse_s + 2 * 32;                          // [2][32]  -D_i
 
-    const int tid = threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lane = tid & 63, ln = lane & 31, hf = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int pid = xcd_order(blockIdx.x, total);
-    const int c0 = blockIdx.y * DV;
     const int sp = pid % nsplit, pj = pid / nsplit;
     const int bh = pj / njb, jb = pj - bh * njb;
     const int b = bh / p.H, h = bh - b * p.H;
     const int N = p.N, w1 = p.w1, w2 = p.w2;
-    const int j0 = jb * WJ, jw = j0 + 32 * wave, j = jw + ln, jc = j < N ? j : N - 1;
+    const int j0 = jb * WJ, jw = j0 + 32 * wave;
 
     const uint16_t* qp = (const uint16_t*)p.q.p + p.q.off(b, 0, h);
     const uint16_t* k1p = (const uint16_t*)p.k1.p + p.k1.off(b, 0, h);
@@ -867,20 +998,17 @@ void wide_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __rest
     const uint16_t* v2p = (const uint16_t*)p.v2.p + p.v2.off(b, 0, h);
     const uint16_t* dop = (const uint16_t*)p.dout.p + p.dout.off(b, 0, h);
     const float qscale = p.scale * LOG2E;
-    const uint32_t tiles_addr = lds_address(tiles);
-    const uint32_t tr_lane = tr_lane_offset<C::RSB>(lane);
 
     // this wavefront's K and V rows as resident B operands (column = key j)
-    X8 kf[C::DK], vf[C::DK];
+    X8 kf[DK], vf[DK];
+    const int ln = threadIdx.x & 31, hf = (threadIdx.x >> 5) & 1, jc = jw + ln < N ? jw + ln : N - 1;
 #pragma unroll
-    for (int kk = 0; kk < C::DK; ++kk) {
+    for (int kk = 0; kk < DK; ++kk) {
         kf[kk] = *(const X8*)(k1p + (int64_t)jc * p.k1.sn + kk * 16 + hf * 8);
         vf[kk] = *(const X8*)(v1p + (int64_t)jc * p.v1.sn + kk * 16 + hf * 8);
     }
-    floatx16 dkacc[C::DT], dvacc[C::DT];
 #pragma unroll
-    for (int dt = 0; dt < C::DT; ++dt) dkacc[dt] = dvacc[dt] = zeros16();
-
+    for (int kk = 0; kk < DK; ++kk) asm volatile("" : "+v"(kf[kk]), "+v"(vf[kk]));     // (here, so that nothing waits for them in the stream)
     const int j_last = j0 + WJ - 1 < N ? j0 + WJ - 1 : N - 1;
     const int i_max = (int)((int64_t)j_last + w1 < N - 1 ? j_last + w1 : N - 1);
     auto units_of = [&](int ib) {
@@ -917,117 +1045,284 @@ void wide_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __rest
         d_first = d_last = 0;
     }
 
-    // ---- forming a unit: Q~ and dO~ tiles (32 rows), LSE and D of its queries ----
-    ux4 fq[C::KR], fk[C::KR], fd[C::KR], fv[C::KR];
-    float f_lse = 0.f, f_dsum = 0.f;
-    auto fetch_unit = [&](int ib, int delta) {
-#pragma unroll
-        for (int u = 0; u < C::KR; ++u) {
-            const int c = tid + WT * u;
-            const int row = c / (D / 8), col = c - row * (D / 8);
-            int i = ib * BQ + row;
-            i = i < N ? i : N - 1;
-            const int k = i - delta > 0 ? i - delta : 0;
-            fq[u] = *(const ux4*)(qp + (int64_t)i * p.q.sn + col * 8);
-            fk[u] = *(const ux4*)(k2p + (int64_t)k * p.k2.sn + col * 8);
-            fd[u] = *(const ux4*)(dop + (int64_t)i * p.dout.sn + col * 8);
-            fv[u] = *(const ux4*)(v2p + (int64_t)k * p.v2.sn + col * 8);
-        }
-        if (tid < 32) {
-            int i = ib * BQ + tid;
-            i = i < N ? i : N - 1;
-            f_lse = p.lse[(int64_t)bh * N + i] * LOG2E;
-            f_dsum = p.dsum[(int64_t)bh * N + i];
-        }
+    // ---- rows of a query block: q and dO, and the first rows of the K'/V' rings.  Row u of a ring counts back from row
+    //      i0 + 31 - d0 (d0: the first delta of the block's run); unit delta takes the rows delta - d0 .. delta - d0 + 31 ----
+    // (what derives from the lane is computed where it is used: kept in registers through the stream it costs the operands theirs)
+    auto here = [&]() {
+        int t = threadIdx.x;
+        opaque(t);
+        return t & 63;
     };
-    auto store_unit = [&](int buf) {
-        uint16_t* Qs = tiles + buf * C::STAGE;
-        uint16_t* Ds = Qs + C::TILE;
-#pragma unroll
-        for (int u = 0; u < C::KR; ++u) {
-            const int c = tid + WT * u;
-            const int row = c / (D / 8), col = c - row * (D / 8);
-            *(X8*)(Qs + row * C::RS + col * 8) = product8<E>(fq[u], fk[u], p.k2_bias, qscale);
-            *(X8*)(Ds + row * C::RS + col * 8) = product8<E>(fd[u], fv[u], p.v2_bias, 1.f);
+    auto request_side = [&](const uint16_t* base, int64_t sn, int top, int pair, unsigned char* ring) {
+        const int lane = here();
+        int k = top - 2 * pair - (lane & 1);
+        k = k < 0 ? 0 : (k < N ? k : N - 1);
+        __builtin_amdgcn_global_load_lds((wide_glb_ptr)(base + (int64_t)k * sn + (lane >> 1) * 8),
+                                         (wide_lds_ptr)(ring + (pair % RING) * WT256::GROUP), 16, 0, 0);
+    };
+    auto request_block = [&](int ib, int d0, int par) {
+        const int lane = here();
+        int i = ib * BQ + (lane & 31);
+        i = i < N ? i : N - 1;
+        const float lse = p.lse[(int64_t)bh * N + i], dsum = p.dsum[(int64_t)bh * N + i];
+        const uint32_t r2 = 8 * wave + (lane & 1), c2 = (lane >> 1) * 8;
+        wide_request(qp, p.q.sn, ib * BQ, N, wave, lane, (r2 * (uint32_t)p.q.sn + c2) * 2u, q_s);
+        wide_request(dop, p.dout.sn, ib * BQ, N, wave, lane, (r2 * (uint32_t)p.dout.sn + c2) * 2u, do_s);
+        for (int x = wave; x < RING; x += WW) {
+            request_side(k2p, p.k2.sn, ib * BQ + BQ - 1 - d0, x, k2_s);
+            request_side(v2p, p.v2.sn, ib * BQ + BQ - 1 - d0, x, v2_s);
         }
-        if (tid < 32) {
-            lse_s[buf * 32 + tid] = f_lse;
-            dsum_s[buf * 32 + tid] = f_dsum;
+        if (wave == 0 && lane < 32) {
+            lse_s[par * 32 + lane] = -lse * LOG2E;
+            dsum_s[par * 32 + lane] = -dsum;
         }
     };
 
-    int ib = ib_lo, delta = d_first, nu = units_of(ib_lo), buf = 0;
-    fetch_unit(ib, delta);
-    store_unit(0);
+    // ---- forming: this wavefront's groups wave + 4x of the tiles, one 16-byte chunk per lane, tensor and x ----
+    const uint32_t lds0 = lds_address(smem_w);
+    constexpr uint32_t XG = 4 * WT256::GROUP;
+    int du = 0;                                              // unit to form: delta - d0
+    auto place_of = [&](int lane) { return (BQ - 1 - 2 * wave - (lane & 1) + du) % WKV_SIDE; };      // of the row that goes with group `wave`
+    auto ring_at = [&](int lane, int place, int x) {         // byte offset of the row that goes with group wave + 4x
+        int g = (place >> 1) - 4 * x;
+        g = g < 0 ? g + RING : g;
+        return (uint32_t)(g * WT256::GROUP + (place & 1) * 16 + (lane >> 1) * 32);
+    };
+    auto form_plain = [&](int buf) {
+        const int lane = here(), place = place_of(lane);
+        const uint32_t form_lane = (uint32_t)(wave * WT256::GROUP + lane * 16);
+#pragma unroll 1
+        for (int x = 0; x < 4; ++x) {
+            const uint32_t r = ring_at(lane, place, x);
+            const ux4 qa = *(const ux4*)(q_s + form_lane + x * XG), ka = *(const ux4*)(k2_s + r);
+            const ux4 da = *(const ux4*)(do_s + form_lane + x * XG), va = *(const ux4*)(v2_s + r);
+            *(X8*)(smem_w + (2 * buf) * TB + form_lane + x * XG) = product8<E>(qa, ka, p.k2_bias, qscale);
+            *(X8*)(smem_w + (2 * buf + 1) * TB + form_lane + x * XG) = product8<E>(da, va, p.v2_bias, 1.f);
+        }
+    };
+
+    int ib = ib_lo, delta = d_first, d0 = d_first, nu = units_of(ib_lo), buf = 0, par = 0;
+    request_block(ib, d0, par);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    form_plain(0);
     __syncthreads();
-    while (true) {
+
+    X8 ro[4][4];                                             // row operands and (halves of) transposed operands of
+    lds_half_operand to[4][8];                               // the chunks c, by c % 4
+    X8 pb[2], dsb[2];
+    floatx16 dkacc[DT], dvacc[DT];
+    // (the last two chunks of a unit run at the start of the wavefront's next one: none outstanding yet)
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            dsb[x][t] = (EL)0.f;
+            to[2 + x][t] = lds_half_operand{0, 0, 0, 0};
+        }
+    settle_operand(dsb);
+    settle_halves(to[2]);
+    settle_halves(to[3]);
+    // chunk c of a unit: 0-3 S, 4-7 dP, 8-11 dV, 12-15 dK
+    auto issue = [&](auto C, uint32_t row_a, uint32_t col_a) {
+        constexpr int c = decltype(C)::value;
+        if constexpr (c < 8) wide_rows4<(c & 3) * 4>(row_a + (c < 4 ? 0u : (uint32_t)TB), ro[c & 3]);
+        else wide_tr_issue<(c >> 1) & 1, (c & 1) * 4, 4>(col_a + (c < 12 ? (uint32_t)TB : 0u), to[c & 3]);
+    };
+    auto tail_mfma = [&](auto C, int x) {                    // dV and dK
+        constexpr int c = decltype(C)::value;
+        const X8 a = lds_join<X8>(to[c & 3][2 * x], to[c & 3][2 * x + 1]);
+        constexpr int dt0 = (c & 1) * 4, ks = (c >> 1) & 1;
+        if constexpr (c < 12) mfma_acc(dvacc[dt0 + x], a, pb[ks]);
+        else mfma_acc(dkacc[dt0 + x], a, dsb[ks]);
+    };
+    auto tail_chunk = [&](auto C) {
+#pragma unroll
+        for (int x = 0; x < 4; ++x) tail_mfma(C, x);
+    };
+    // One unit, and beside it the forming of the next one of the query block (after the last one: of nothing that is used).
+    // LDS operations return in order: a wait for n outstanding ones is a wait for everything issued before the last n.
+    // The vector ALU's work sits between the MFMAs one by one: a wavefront issues in order, and alone on its SIMD it
+    // would leave the matrix pipe idle for as long as a longer piece takes.
+    auto unit = [&]() {
+        const int lane = here(), ln = lane & 31, hf = lane >> 5, j = jw + ln;
+        const uint32_t form_lane = (uint32_t)(wave * WT256::GROUP + lane * 16);
+        const uint32_t row_lane = (uint32_t)((ln / 2) * WT256::GROUP + (hf * 2 + (ln & 1)) * 16);
+        const uint32_t col_lane = lds_group_column_lane_offset<WT256::RPW, WT256::GROUP>(lane);
+        const int place = place_of(lane);
+        const uint32_t tile = lds0 + (uint32_t)(buf * 2 * TB), row_a = tile + row_lane, col_a = tile + col_lane;
+        const uint32_t next = lds0 + (uint32_t)((buf ^ 1) * 2 * TB) + form_lane;
+        const uint32_t raw_a = lds0 + 4 * TB + form_lane, ring_a = lds0 + 6 * TB;
+        const uint32_t per_query = lds0 + (uint32_t)(6 * TB + 2 * RING * WT256::GROUP + par * 128 + hf * 16);
+        const int i0 = ib * BQ;
+        // register v of this lane: query i0 + 8*(v/4) + 4*hf + v%4, key j
+        const bool interior = (i0 >= jw + 31) && ((int64_t)i0 + 31 <= (int64_t)jw + w1) && (i0 + BQ - 1 < N) && (i0 >= delta);
+        // The forming in eight slices of one 16-byte chunk each (group wave + 4 * (k / 2), Q~ for even k and dO~ for odd):
+        // slice 0 beside the tail of the unit before, slice k beside the chunks 2k-2 and 2k-1, a pair of elements after
+        // every second MFMA.
+        ux4 fa[2], fb[2];
+        auto form_read = [&](auto K) {
+            constexpr int k = decltype(K)::value, x = k >> 1, which = k & 1;
+            lds_read16<which * TB + x * (int)XG>(raw_a, fa[which]);
+            lds_read16<which * RING * WT256::GROUP>(ring_a + ring_at(lane, place, x), fb[which]);
+        };
+        auto form_pair = [&](auto K, int y) {
+            constexpr int which = decltype(K)::value & 1;
+            const float bias = which ? p.v2_bias : p.k2_bias, mul = which ? 1.f : qscale;
+            const uint32_t u = fa[which][y], v = fb[which][y];
+            if constexpr (BIASED) fa[which][y] = pack2<E>(E::lo(u) * mul * (E::lo(v) + bias), E::hi(u) * mul * (E::hi(v) + bias));
+            else fa[which][y] = pack2<E>(E::lo(u) * mul * E::lo(v), E::hi(u) * mul * E::hi(v));
+        };
+        auto form_write = [&](auto K) {
+            constexpr int k = decltype(K)::value;
+            lds_write16<(k & 1) * TB + (k >> 1) * (int)XG>(next, fa[k & 1]);
+        };
+        fx4 lp[4], dp[4];
+        lds_read16<0>(per_query, lp[0]);
+        lds_read16<32>(per_query, lp[1]);
+        lds_read16<64>(per_query, lp[2]);
+        lds_read16<96>(per_query, lp[3]);
+        form_read(std::integral_constant<int, 0>{});
+        issue(std::integral_constant<int, 0>{}, row_a, col_a);
+        tail_chunk(std::integral_constant<int, 14>{});
+        form_read(std::integral_constant<int, 1>{});
+        issue(std::integral_constant<int, 1>{}, row_a, col_a);
+        asm volatile("s_waitcnt lgkmcnt(10)" : "+v"(fa[0]), "+v"(fb[0]));
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+            tail_mfma(std::integral_constant<int, 15>{}, y);
+            __builtin_amdgcn_sched_barrier(0);
+            form_pair(std::integral_constant<int, 0>{}, y);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        form_write(std::integral_constant<int, 0>{});
+        floatx16 sacc, dpacc;
+        static_for<16>([&](auto CC) {
+            constexpr int c = decltype(CC)::value;
+            if constexpr ((c & 1) == 1 && c < 13) form_read(std::integral_constant<int, (c + 3) / 2>{});
+            if constexpr (c == 3) {
+                lds_read16<256>(per_query, dp[0]);
+                lds_read16<288>(per_query, dp[1]);
+                lds_read16<320>(per_query, dp[2]);
+                lds_read16<352>(per_query, dp[3]);
+            }
+            if constexpr (c < 14) issue(std::integral_constant<int, c + 2>{}, row_a, col_a);
+            // what may be outstanding: the operands of the next two chunks, and the forming's accesses beside them
+            constexpr int len1 = c + 1 > 15 ? 0 : c + 1 < 8 ? 4 : 8, len2 = c + 2 > 15 ? 0 : c + 2 < 8 ? 4 : 8;
+            constexpr int want = len1 + len2 + ((c & 1) ? (c < 13 ? 2 : 0) + (c == 3 ? 4 : 0) : c < 14 ? 1 : 0);
+            constexpr int n = want > 15 ? 15 : want;
+            if constexpr (c < 8) lds_wait<n>(ro[c & 3]);
+            else lds_wait_halves<n>(to[c & 3]);
+            if constexpr (c == 0) {
+                arrived(lp[0], lp[1]);
+                arrived(lp[2], lp[3]);
+#pragma unroll
+                for (int v = 0; v < 16; ++v) sacc[v] = lp[v >> 2][v & 3];
+                settle_c(sacc);
+            }
+            if constexpr (c == 4) {
+                arrived(dp[0], dp[1]);
+                arrived(dp[2], dp[3]);
+#pragma unroll
+                for (int v = 0; v < 16; ++v) dpacc[v] = dp[v >> 2][v & 3];
+                settle_c(dpacc);
+            }
+            if constexpr ((c & 1) == 0 && c < 14) arrived(fa[(c / 2 + 1) & 1], fb[(c / 2 + 1) & 1]);
+            if constexpr (c == 6) {
+                wait_acc(sacc);
+                if (!interior) {
+                    int lo = j - i0 - 4 * hf;                                          // c >= lo  <=>  j <= i
+                    opaque(lo);                           // (a branch: few units need the mask)
+                    const int hi = lo < (1 << 20) - w1 ? lo + w1 : (1 << 20);          // i <= j + w1
+                    const int dlo = delta - j + lo, nhi = N - 1 - j + lo;
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) {
+                        const int y = 8 * (v >> 2) + (v & 3);
+                        sacc[v] = (j < N) && (y >= lo) && (y <= hi) && (y >= dlo) && (y <= nhi) ? sacc[v] : -INFINITY;
+                    }
+                }
+            }
+            if constexpr (c == 10) wait_acc(dpacc);
+            if constexpr (c < 14) {
+#pragma unroll
+                for (int y = 0; y < 4; ++y) {
+                    if constexpr (c < 4) mfma_vec(sacc, ro[c & 3][y], kf[4 * c + y]);
+                    else if constexpr (c < 8) mfma_vec(dpacc, ro[c & 3][y], vf[4 * (c - 4) + y]);
+                    else tail_mfma(CC, y);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if ((y & 1) == 0) form_pair(std::integral_constant<int, c / 2 + 1>{}, 2 * (c & 1) + y / 2);
+                    if constexpr (c == 6 || c == 7) {                    // the weights P
+#pragma unroll
+                        for (int v = 8 * (c - 6) + 2 * y; v < 8 * (c - 6) + 2 * y + 2; ++v) {
+                            sacc[v] = fast_exp2(sacc[v]);
+                            pb[v >> 3][v & 7] = (EL)sacc[v];
+                        }
+                    }
+                    if constexpr (c == 10 || c == 11) {                  // dS
+#pragma unroll
+                        for (int v = 8 * (c - 10) + 2 * y; v < 8 * (c - 10) + 2 * y + 2; ++v) dsb[v >> 3][v & 7] = (EL)(sacc[v] * dpacc[v]);
+                    }
+                    if ((c & 1) == 1 && y == 2) form_write(std::integral_constant<int, c / 2 + 1>{});
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if constexpr (c == 7) settle_operand(pb);
+                if constexpr (c == 11) settle_operand(dsb);
+            }
+        });
+    };
+
+    bool more = true;
+    // one unit of the stream: requests and forming of what comes next, with the wavefront's own work on it or without
+    auto step = [&](auto WORK) {
         int nib = ib, ndelta = delta + 1;
         if (ndelta >= nu) {
             nib = ib + 1;
             ndelta = 0;
         }
-        const bool more = SPLIT ? (nib < ib_hi || (nib == ib_hi && ndelta <= d_last)) : nib <= ib_hi;
-        if (more) fetch_unit(nib, ndelta);
-
-        const int i0 = ib * BQ;
-        const bool touches = (i0 + BQ - 1 >= jw) && ((int64_t)i0 <= (int64_t)jw + 31 + w1) && jw < N && !empty_share;
-        if (touches) {
-            const uint16_t* Qs = tiles + buf * C::STAGE;
-            const uint16_t* Ds = Qs + C::TILE;
-            const uint32_t Qt = tiles_addr + (uint32_t)(buf * C::STAGE * 2) + tr_lane + (uint32_t)(c0 * 2);
-            const uint32_t Dt = Qt + (uint32_t)(C::TILE * 2);
-            floatx16 sacc = zeros16(), dpacc = zeros16();
-#pragma unroll
-            for (int kk = 0; kk < C::DK; ++kk) {
-                const X8 qa = *(const X8*)(Qs + ln * C::RS + kk * 16 + hf * 8);
-                const X8 da = *(const X8*)(Ds + ln * C::RS + kk * 16 + hf * 8);
-                sacc = E::mfma(qa, kf[kk], sacc, 0, 0, 0);
-                dpacc = E::mfma(da, vf[kk], dpacc, 0, 0, 0);
+        more = SPLIT ? (nib < ib_hi || (nib == ib_hi && ndelta <= d_last)) : nib <= ib_hi;
+        const bool form = more && nib == ib;                 // the next unit belongs to the same query block
+        du = form ? ndelta - d0 : 0;
+        if (form) {
+            if ((du & 3) == 0) {                             // four more rows for each ring, where four are no longer needed
+                const int pair = (du + WKV_SIDE - 4) / 2 + (wave & 1), top = ib * BQ + BQ - 1 - d0;
+                if (wave < 2) request_side(k2p, p.k2.sn, top, pair, k2_s);
+                else request_side(v2p, p.v2.sn, top, pair, v2_s);
             }
-            // register v of this lane: query i0 + 8*(v/4) + 4*hf + v%4, key j
-            const bool interior = (i0 >= jw + 31) && ((int64_t)i0 + 31 <= (int64_t)jw + w1) && (i0 + BQ - 1 < N) && (i0 >= delta);
-            const int lo = j - i0 - 4 * hf;                                    // c >= lo  <=>  j <= i
-            const int hi = (int)((int64_t)j + w1 - i0 < (1 << 20) ? j + w1 - i0 : (1 << 20)) - 4 * hf;   // i <= j + w1
-            const int dlo = delta - i0 - 4 * hf, nhi = N - 1 - i0 - 4 * hf;
-            X8 pb[2], dsb[2];
-#pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4) {
-                const float4 ls = *(const float4*)(lse_s + buf * 32 + 8 * g4 + 4 * hf);
-                const float4 dm = *(const float4*)(dsum_s + buf * 32 + 8 * g4 + 4 * hf);
-                const float lsv[4] = {ls.x, ls.y, ls.z, ls.w}, dmv[4] = {dm.x, dm.y, dm.z, dm.w};
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const int v = 4 * g4 + t, c = 8 * g4 + t;
-                    const bool valid = interior || ((j < N) && (c >= lo) && (c <= hi) && (c >= dlo) && (c <= nhi));
-                    const float pv = valid ? fast_exp2(sacc[v] - lsv[t]) : 0.f;
-                    pb[v >> 3][v & 7] = (EL)pv;
-                    dsb[v >> 3][v & 7] = (EL)(pv * (dpacc[v] - dmv[t]));
-                }
-            }
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-                for (int dt = 0; dt < C::DT; ++dt) {
-                    const uint32_t o = (uint32_t)(16 * ks * C::RSB + dt * 64);
-                    dvacc[dt] = E::mfma(tr_operand<X8, C::RSB>(Dt + o), pb[ks], dvacc[dt], 0, 0, 0);
-                    dkacc[dt] = E::mfma(tr_operand<X8, C::RSB>(Qt + o), dsb[ks], dkacc[dt], 0, 0, 0);
-                }
+        } else if (more) {
+            request_block(nib, 0, par ^ 1);
         }
-        if (!more) break;
-        store_unit(buf ^ 1);          // (the other buffer was last read one step ago, before that step's barrier)
-        __syncthreads();
-        if (nib != ib) nu = units_of(nib);
+        if constexpr (decltype(WORK)::value) unit();
+        else if (form) form_plain(buf ^ 1);
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (more && nib != ib) {
+            nu = units_of(nib);
+            d0 = 0;
+            par ^= 1;
+            form_plain(buf ^ 1);
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        }
         ib = nib;
         delta = ndelta;
         buf ^= 1;
-    }
+    };
+    // the wavefront's keys are seen by a run of query blocks (none: keys past the end of the sequence, or an empty share)
+    const int t_lo = jw / BQ, t_hi = jw < N && !empty_share ? (int)(((int64_t)jw + 31 + w1) / BQ < (1 << 26) ? ((int64_t)jw + 31 + w1) / BQ : (1 << 26)) : -1;
+    zero_acc(dkacc);
+    zero_acc(dvacc);
+    while (more && (ib < t_lo || t_hi < 0)) step(std::false_type{});
+    while (more && ib <= t_hi) step(std::true_type{});
+    tail_chunk(std::integral_constant<int, 14>{});
+    tail_chunk(std::integral_constant<int, 15>{});
+    while (more) step(std::false_type{});
+    settle_acc(dkacc);
+    settle_acc(dvacc);
 
+    const int lane_f = here(), hf_f = lane_f >> 5, j = jw + (lane_f & 31);
     if (j < N && SPLIT) {
         const int64_t BH = (int64_t)p.B * p.H;
-        float* dkp = p.dk1.p ? part + (((0 * (int64_t)nsplit + sp) * BH + bh) * N + j) * D + c0 + 4 * hf : nullptr;
-        float* dvp = p.dv1.p ? part + (((1 * (int64_t)nsplit + sp) * BH + bh) * N + j) * D + c0 + 4 * hf : nullptr;
+        float* dkp = p.dk1.p ? part + (((0 * (int64_t)nsplit + sp) * BH + bh) * N + j) * D + 4 * hf_f : nullptr;
+        float* dvp = p.dv1.p ? part + (((1 * (int64_t)nsplit + sp) * BH + bh) * N + j) * D + 4 * hf_f : nullptr;
 #pragma unroll
-        for (int dt = 0; dt < C::DT; ++dt)
+        for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4) {
                 if (dkp) *(float4*)(dkp + dt * 32 + 8 * g4) = make_float4(dkacc[dt][4 * g4] * LN2, dkacc[dt][4 * g4 + 1] * LN2,
@@ -1036,10 +1331,10 @@ void wide_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __rest
                                                                            dvacc[dt][4 * g4 + 3]);
             }
     } else if (j < N) {
-        uint16_t* dkp = p.dk1.p ? (uint16_t*)p.dk1.p + p.dk1.off(b, j, h) + c0 + 4 * hf : nullptr;
-        uint16_t* dvp = p.dv1.p ? (uint16_t*)p.dv1.p + p.dv1.off(b, j, h) + c0 + 4 * hf : nullptr;
+        uint16_t* dkp = p.dk1.p ? (uint16_t*)p.dk1.p + p.dk1.off(b, j, h) + 4 * hf_f : nullptr;
+        uint16_t* dvp = p.dv1.p ? (uint16_t*)p.dv1.p + p.dv1.off(b, j, h) + 4 * hf_f : nullptr;
 #pragma unroll
-        for (int dt = 0; dt < C::DT; ++dt)
+        for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4) {
                 // Q~ carries scale*log2(e): dK = ln2 * sum dS * Q~
@@ -1051,42 +1346,37 @@ void wide_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __rest
     }
 }
 
-// dK and dV from the partial sums of a split launch, shares added in their order
-template <class E, int D>
-__global__ __launch_bounds__(256) void wide_kv_sum_kernel(Problem p, int nsplit, const float* __restrict__ part, int64_t chunks) {
-    const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (c >= chunks) return;
-    const int col = (int)(c % (D / 4));
-    const int64_t rowid = c / (D / 4);
-    const int j = (int)(rowid % p.N);
-    const int bh = (int)(rowid / p.N);
-    const int b = bh / p.H, h = bh - b * p.H;
-    const int64_t BH = (int64_t)p.B * p.H;
-#pragma unroll
-    for (int which = 0; which < 2; ++which) {
-        const Tensor& t = which ? p.dv1 : p.dk1;
-        if (!t.p) continue;
-        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int s = 0; s < nsplit; ++s) {
-            const float4 y = *(const float4*)(part + (((which * (int64_t)nsplit + s) * BH + bh) * p.N + j) * D + col * 4);
-            acc.x += y.x; acc.y += y.y; acc.z += y.z; acc.w += y.w;
+// Shares of a key block's stream of units: the least time by grid_time with about 2.3 us per unit and the time of a dozen
+// units around them.  Partial sums may take 64 MiB.
+int wide_kv_nsplit(int B, int N, int H, int D, int w1, int w2) {
+    constexpr double UNIT = 2.3, AROUND = 12;
+    const int64_t bh = (int64_t)B * H, base = bh * ((N + WJ - 1) / WJ);
+    const int64_t units = (int64_t)((WJ + (w1 < N ? w1 : N)) / BQ + 1) * ((w2 < N - 1 ? w2 : N - 1) + 1);      // of a key block's stream, at most
+    const double fill = window_fill(w1, N) * window_fill(w2, N);
+    int best = 1;
+    double least = 0;
+    for (int ns = 1; ns <= 16 && units / ns >= 4; ++ns) {
+        const double part = ns > 1 ? 2.0 * ns * bh * N * D * 4 : 0, per = (double)((units + ns - 1) / ns);
+        if (part > 67108864.0) break;
+        const double cost = UNIT * grid_time(base * ns, per + AROUND, per * fill + AROUND) + (ns > 1 ? SUM_LAUNCH_STEPS + part / PART_BYTES_PER_STEP : 0);
+        if (least == 0 || cost < 0.97 * least) {
+            least = cost;
+            best = ns;
         }
-        *(uint2*)((uint16_t*)t.p + t.off(b, j, h) + col * 4) = make_uint2(E::pack(acc.x, acc.y), E::pack(acc.z, acc.w));
     }
+    return best;
 }
-
-// Shares a key block's query blocks are split into when the K-side grid is smaller than the chip
-int wide_kv_nsplit(int B, int N, int H, int D, int w1, int w2, int npass) {
-    const int64_t bh = (int64_t)B * H, base = bh * ((N + WJ - 1) / WJ) * npass;
-    const int blocks = (WJ + (w1 < N ? w1 : N) + BQ - 1) / BQ + 1;
-    const int64_t units = (int64_t)blocks * ((w2 < N - 1 ? w2 : N - 1) + 1);     // of a key block's stream, at most
-    int ns = 1;                                                                  // shares of at least 8 units
-    while (ns < 16 && base * ns * 2 <= 512 && (int64_t)ns * 2 * 8 <= units && (int64_t)2 * ns * 2 * bh * N * D * 4 <= ((int64_t)32 << 20))
-        ns *= 2;
-    return ns;
+size_t wide_dq_part_bytes(int B, int N, int H, const KpPlan& pl) {
+    return ((size_t)B * H * ((N + BQ - 1) / BQ) * pl.nseg * (size_t)(BQ + pl.segw - 1) * 256 * sizeof(float) + 255) / 256 * 256;
 }
-size_t wide_dq_part_bytes(int B, int N, int H, int D, int w2) {
-    return ((size_t)B * H * ((N + BQ - 1) / BQ) * (size_t)(32 + w2) * D * sizeof(float) + 255) / 256 * 256;
+size_t wide_kp_part_bytes(int B, int N, int H, const KpPlan& pl) { return pl.nseg > 1 ? (size_t)2 * pl.nseg * B * H * (size_t)N * 256 * sizeof(float) : 0; }
+KpPlan wide_kp_plan(int B, int N, int H, int w1, int w2) {
+    return plan_segments(B, N, H, w1, w2, 2, w2 + 1, [](int) { return false; },      // (the work between two sweeps takes long here)
+                         [&](const KpPlan& pl) { return wide_dq_part_bytes(B, N, H, pl) + wide_kp_part_bytes(B, N, H, pl); });
+}
+size_t wide_kp_bytes(int B, int N, int H, int w1, int w2) {
+    const KpPlan pl = wide_kp_plan(B, N, H, w1, w2);
+    return (wide_dq_part_bytes(B, N, H, pl) + wide_kp_part_bytes(B, N, H, pl) + 255) / 256 * 256;
 }
 
 // ------------------------------------------------------------------ launchers ----
@@ -1104,59 +1394,51 @@ int launch_wide_fwd_of(const Problem& p, hipStream_t st) {
     return nsplit > 1 ? launch_fwd_merge(p, 256, E::DTYPE, st) : SA2_OK;
 }
 
-template <class E, int D, int DV>
-int launch_wide_bwd(const Problem& p, hipStream_t st) {
-    using C = WideCfg<D, DV>;
+template <class E>
+int launch_wide_bwd_of(const Problem& p, hipStream_t st) {
+    constexpr int D = 256;
     int rc = launch_rowdot(p.out, p.dout, p.dsum, p.B, p.N, p.H, p.D, E::DTYPE, st);
     if (rc != SA2_OK) return rc;
+    const bool biased = p.k2_bias != 0.f || p.v2_bias != 0.f;           // (the common case pays for none of it)
+    BwdSums sums = {};
+    const KpPlan pl = wide_kp_plan(p.B, p.N, p.H, p.w1, p.w2);
+    const int nsplit = wide_kv_nsplit(p.B, p.N, p.H, D, p.w1, p.w2);
+    if (((p.dq.p || pl.nseg > 1) || nsplit > 1) && p.scratch_bytes < wide_bwd_scratch_bytes(p.B, p.N, p.H, D, p.w1, p.w2)) return SA2_ERR_WORKSPACE_TOO_SMALL;
     if (p.dq.p || p.dk2.p || p.dv2.p) {
         const int nkb = (p.N + BQ - 1) / BQ;
-        const int64_t total = (int64_t)nkb * p.B * p.H;
+        const int64_t total = (int64_t)nkb * p.B * p.H * pl.nseg;
         if (total > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
-        if (p.scratch_bytes < wide_dq_part_bytes(p.B, p.N, p.H, D, p.w2)) return SA2_ERR_WORKSPACE_TOO_SMALL;
         float* part = (float*)p.scratch;
-        if (!allow_full_lds((const void*)wide_kp_kernel<E, D, DV, false>) || !allow_full_lds((const void*)wide_kp_kernel<E, D, DV, true>))
-            return SA2_ERR_LAUNCH_FAILED;
-        const int segw = C::kp_segment(p.w2);
-        if (segw < p.w2 + 1)
-            hipLaunchKernelGGL((wide_kp_kernel<E, D, DV, true>), dim3((unsigned)total, C::NPASS), dim3(WT), C::kp_lds(segw - 1), st, p, nkb,
-                               (int)total, part, segw);
-        else
-            hipLaunchKernelGGL((wide_kp_kernel<E, D, DV, false>), dim3((unsigned)total, C::NPASS), dim3(WT), C::kp_lds(segw - 1), st, p, nkb,
-                               (int)total, part, segw);
-        if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
-        if (p.dq.p) {
-            const int64_t chunks = (int64_t)p.B * p.H * p.N * (D / 4);
-            hipLaunchKernelGGL((wide_dq_sum_kernel<E, D>), dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, p, nkb, part, chunks);
-            if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
-        }
+        float* kpart = (float*)((char*)p.scratch + wide_dq_part_bytes(p.B, p.N, p.H, pl));
+        auto go = [&](auto kernel) {
+            if (!allow_full_lds((const void*)kernel)) return false;
+            hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(WT), WIDE_KP_LDS, st, p, nkb, (int)total, part, pl.nseg, pl.segw, kpart);
+            return hipGetLastError() == hipSuccess;
+        };
+        if (!(biased ? go(wide_kp_kernel<E, true>) : go(wide_kp_kernel<E, false>))) return SA2_ERR_LAUNCH_FAILED;
+        sums.dq = p.dq.p ? part : nullptr;
+        sums.nkb = nkb;
+        sums.nseg = pl.nseg;
+        sums.segw = pl.segw;
+        sums.kp = pl.nseg > 1 ? kpart : nullptr;
+        sums.kp_n = pl.nseg;
     }
     if (p.dk1.p || p.dv1.p) {
         const int njb = (p.N + WJ - 1) / WJ;
-        const int nsplit = wide_kv_nsplit(p.B, p.N, p.H, D, p.w1, p.w2, C::NPASS);
         const int64_t total = (int64_t)njb * p.B * p.H * nsplit;
         if (total > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
-        float* kv_part = nullptr;
-        if (nsplit > 1) {
-            if (p.scratch_bytes < wide_bwd_scratch_bytes(p.B, p.N, p.H, D, p.w1, p.w2)) return SA2_ERR_WORKSPACE_TOO_SMALL;
-            kv_part = (float*)((char*)p.scratch + wide_dq_part_bytes(p.B, p.N, p.H, D, p.w2));
-        }
-        if (!allow_full_lds((const void*)wide_kv_kernel<E, D, DV, false>) || !allow_full_lds((const void*)wide_kv_kernel<E, D, DV, true>))
-            return SA2_ERR_LAUNCH_FAILED;
-        if (nsplit > 1)
-            hipLaunchKernelGGL((wide_kv_kernel<E, D, DV, true>), dim3((unsigned)total, C::NPASS), dim3(WT), C::KV_LDS, st, p, njb, (int)total,
-                               nsplit, kv_part);
-        else
-            hipLaunchKernelGGL((wide_kv_kernel<E, D, DV, false>), dim3((unsigned)total, C::NPASS), dim3(WT), C::KV_LDS, st, p, njb, (int)total,
-                               1, kv_part);
-        if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
-        if (nsplit > 1) {
-            const int64_t chunks = (int64_t)p.B * p.H * p.N * (D / 4);
-            hipLaunchKernelGGL((wide_kv_sum_kernel<E, D>), dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, p, nsplit, kv_part, chunks);
-            if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
-        }
+        float* part = (float*)((char*)p.scratch + wide_kp_bytes(p.B, p.N, p.H, p.w1, p.w2));
+        auto go = [&](auto kernel) {
+            if (!allow_full_lds((const void*)kernel)) return false;
+            hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(WT), WIDE_KV_LDS, st, p, njb, (int)total, nsplit, part);
+            return hipGetLastError() == hipSuccess;
+        };
+        if (!(nsplit > 1 ? (biased ? go(wide_kv_kernel<E, true, true>) : go(wide_kv_kernel<E, true, false>))
+                         : (biased ? go(wide_kv_kernel<E, false, true>) : go(wide_kv_kernel<E, false, false>)))) return SA2_ERR_LAUNCH_FAILED;
+        sums.kv = nsplit > 1 ? part : nullptr;
+        sums.kv_n = nsplit;
     }
-    return SA2_OK;
+    return launch_bwd_sums(p, sums, D, E::DTYPE, st);
 }
 
 }  // namespace
@@ -1169,8 +1451,8 @@ bool wide_bwd_supported(int D, int w2, int dtype) {
 }
 
 size_t wide_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2) {
-    const int ns = wide_kv_nsplit(B, N, H, D, w1, w2, 2);
-    return wide_dq_part_bytes(B, N, H, D, w2) + (ns > 1 ? (size_t)2 * ns * B * H * (size_t)N * D * sizeof(float) : 0);
+    const int ns = wide_kv_nsplit(B, N, H, D, w1, w2);
+    return wide_kp_bytes(B, N, H, w1, w2) + (ns > 1 ? (size_t)2 * ns * B * H * (size_t)N * D * sizeof(float) : 0);
 }
 
 int wide_fwd_nsplit(int B, int N, int H, int w1, int w2) { return plan_forward(B, N, H, 256, w1, w2, WW); }
@@ -1180,7 +1462,7 @@ int launch_wide_fwd(const Problem& p, int dtype, hipStream_t st) {
 }
 
 int launch_wide_bwd(const Problem& p, int dtype, hipStream_t st) {
-    return dtype == SA2_F16 ? launch_wide_bwd<ElemF16, 256, 128>(p, st) : launch_wide_bwd<ElemBF16, 256, 128>(p, st);
+    return dtype == SA2_F16 ? launch_wide_bwd_of<ElemF16>(p, st) : launch_wide_bwd_of<ElemBF16>(p, st);
 }
 
 }  // namespace sa2
