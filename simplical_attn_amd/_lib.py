@@ -87,7 +87,8 @@ def host():
         spec.loader.exec_module(module)
         address = lambda f: ctypes.cast(f, ctypes.c_void_p).value
         module.bind(address(lib.sa2_forward_ws), address(lib.sa2_fwd_workspace_bytes), address(lib.sa2_backward),
-                    address(lib.sa2_bwd_workspace_bytes), address(lib.sa2_strerror), simplicial_attn._check_inputs, simplicial_attn._check_saved, Sa2Error)
+                    address(lib.sa2_bwd_workspace_bytes), address(lib.sa2_strerror), simplicial_attn._check_inputs, simplicial_attn._check_saved, Sa2Error,
+                    simplicial_attn.TwoSimplicialAttentionFunction.apply)
         _host = module
     return _host
 

@@ -157,9 +157,17 @@ void refuse_inputs(const Tensor& q, const Tensor& k1, const Tensor& k2, const Te
     throw std::invalid_argument("q, k1, k2, v1 and v2 must be GPU tensors of one shape [batch, seq_len, num_heads, head_dim], dtype and device");
 }
 
+// Calls that need more of autograd than the native formula gives go through the Python autograd function (set by bind):
+// a tensor with a forward-mode tangent, for which the Python function raises (the native path below would drop the
+// tangent where no input requires grad, which reads as a zero derivative).
+PyObject* general_py = nullptr;
+bool plain(const Tensor& t) { return !t._fw_grad(0).defined(); }
+
 Tensor attention(const Tensor& q, const Tensor& k1, const Tensor& k2, const Tensor& v1, const Tensor& v2, int64_t w1, int64_t w2,
                  std::optional<double> scale, double k2_bias, double v2_bias, bool inclusive, unsigned flags) {
     if (!inputs_ok(q, k1, k2, v1, v2)) refuse_inputs(q, k1, k2, v1, v2);
+    if (!(plain(q) && plain(k1) && plain(k2) && plain(v1) && plain(v2)))
+        return py::handle{general_py}(q, k1, k2, v1, v2, w1, w2, scale, k2_bias, v2_bias, inclusive, flags).cast<Tensor>();
     const Args a{w1, w2, scale_of(scale, q), k2_bias, v2_bias, inclusive, flags};
     py::gil_scoped_release nogil;
     if (at::GradMode::is_enabled() &&
@@ -202,7 +210,8 @@ py::tuple backward(const Tensor& q, const Tensor& k1, const Tensor& k2, const Te
 
 PYBIND11_MODULE(_sa2_torch, m) {
     m.doc() = "Native host path of the 2-simplicial attention operator";
-    m.def("bind", [](uintptr_t fwd, uintptr_t fwd_ws, uintptr_t bwd, uintptr_t ws, uintptr_t err, py::object check_inputs, py::object check_saved, py::object error) {
+    m.def("bind", [](uintptr_t fwd, uintptr_t fwd_ws, uintptr_t bwd, uintptr_t ws, uintptr_t err, py::object check_inputs, py::object check_saved, py::object error,
+                     py::object general) {
         fwd_fn = (decltype(fwd_fn))fwd;
         fwd_ws_fn = (decltype(fwd_ws_fn))fwd_ws;
         bwd_fn = (decltype(bwd_fn))bwd;
@@ -210,6 +219,7 @@ PYBIND11_MODULE(_sa2_torch, m) {
         err_fn = (decltype(err_fn))err;
         check_inputs_py = check_inputs.release().ptr();         // kept for the process
         check_saved_py = check_saved.release().ptr();
+        general_py = general.release().ptr();
         static PyObject* error_class = nullptr;
         error_class = error.release().ptr();
         py::register_exception_translator([](std::exception_ptr p) {

@@ -62,3 +62,28 @@ def test_side_streams_and_threads():
         t.join()
     for g in got:
         assert all(torch.equal(a, b) for a, b in zip(g, want))
+
+
+def _raised(call):
+    try:
+        call()
+    except Exception as e:          # noqa: BLE001 - the kind is what is compared
+        return type(e)
+    return None
+
+
+@pytest.mark.parametrize("which", [0, 3])
+@pytest.mark.parametrize("grad", [True, False])
+def test_forward_mode_derivatives_are_refused_not_dropped(which, grad):
+    """There is no forward-mode formula: the module raises for a dual tensor, as the autograd function does, also where
+    no input requires grad."""
+    import torch.autograd.forward_ad as fwd
+
+    import simplical_attn_amd as sa
+    x = [t.cuda() for t in make_inputs(1, 64, 1, 64, seed=5, with_dout=False)]
+    module, fn = _both(sa, 64)
+    with fwd.dual_level(), torch.set_grad_enabled(grad):
+        duals = list(x)
+        duals[which] = fwd.make_dual(x[which], torch.ones_like(x[which]))
+        assert _raised(lambda: module(*duals)) is _raised(lambda: fn(*duals)) is NotImplementedError
+    assert torch.equal(module(*x), fn(*x))
