@@ -7,8 +7,10 @@
 //
 // The C ABI functions are handed over as addresses by bind(), so that the library is whichever one Python loaded.
 // A call whose arguments this file does not accept goes to the Python checks, which raise the error that names them.
+#include <ATen/TensorSubclassLikeUtils.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/extension.h>
 
 #include <cmath>
@@ -157,16 +159,20 @@ void refuse_inputs(const Tensor& q, const Tensor& k1, const Tensor& k2, const Te
     throw std::invalid_argument("q, k1, k2, v1 and v2 must be GPU tensors of one shape [batch, seq_len, num_heads, head_dim], dtype and device");
 }
 
-// Calls that need more of autograd than the native formula gives go through the Python autograd function (set by bind):
-// a tensor with a forward-mode tangent, for which the Python function raises (the native path below would drop the
-// tangent where no input requires grad, which reads as a zero derivative).
+// Calls that need more of autograd or of the dispatcher than the native formula gives go through the Python autograd
+// function (set by bind):
+//  - a tensor with a forward-mode tangent, for which the Python function raises (the native path below would drop the
+//    tangent where no input requires grad, which reads as a zero derivative);
+//  - a call under torch.jit.trace, which records the Python function as one operation (of the native path it would see
+//    the allocation of the output only, and a replay would return uninitialised memory);
+//  - tensors of torch.func transforms and other wrappers, and active dispatch modes.
 PyObject* general_py = nullptr;
-bool plain(const Tensor& t) { return !t._fw_grad(0).defined(); }
+bool plain(const Tensor& t) { return !t._fw_grad(0).defined() && !at::isTensorSubclassLike(t); }
 
 Tensor attention(const Tensor& q, const Tensor& k1, const Tensor& k2, const Tensor& v1, const Tensor& v2, int64_t w1, int64_t w2,
                  std::optional<double> scale, double k2_bias, double v2_bias, bool inclusive, unsigned flags) {
     if (!inputs_ok(q, k1, k2, v1, v2)) refuse_inputs(q, k1, k2, v1, v2);
-    if (!(plain(q) && plain(k1) && plain(k2) && plain(v1) && plain(v2)))
+    if (torch::jit::tracer::isTracing() || !(plain(q) && plain(k1) && plain(k2) && plain(v1) && plain(v2)))
         return py::handle{general_py}(q, k1, k2, v1, v2, w1, w2, scale, k2_bias, v2_bias, inclusive, flags).cast<Tensor>();
     const Args a{w1, w2, scale_of(scale, q), k2_bias, v2_bias, inclusive, flags};
     py::gil_scoped_release nogil;

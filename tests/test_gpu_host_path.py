@@ -1,6 +1,7 @@
 """The module's native host path against TwoSimplicialAttentionFunction (same kernels, autograd formula in Python): every
 subset of inputs that need gradients, broadcast inputs and upstream gradients, no_grad, a side stream and threads."""
 import threading
+import warnings
 
 import pytest
 import torch
@@ -87,3 +88,41 @@ def test_forward_mode_derivatives_are_refused_not_dropped(which, grad):
         duals[which] = fwd.make_dual(x[which], torch.ones_like(x[which]))
         assert _raised(lambda: module(*duals)) is _raised(lambda: fn(*duals)) is NotImplementedError
     assert torch.equal(module(*x), fn(*x))
+
+
+@pytest.mark.parametrize("grad", [True, False])
+def test_traced_module_computes_on_new_inputs(grad):
+    import simplical_attn_amd as sa
+    x, y = ([t.cuda().requires_grad_(grad) for t in make_inputs(1, 96, 2, 64, seed=s, with_dout=False)] for s in (6, 7))
+    module, fn = _both(sa, 64)
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore")
+        traced = torch.jit.trace(module, x, check_trace=False)
+    assert any(n.kind() == "prim::PythonOp" for n in traced.graph.nodes())
+    assert torch.equal(traced(*y), fn(*y)) and torch.equal(traced(*x), fn(*x))
+
+
+@pytest.mark.parametrize("transform", ["grad", "vmap", "jvp"])
+def test_function_transforms_raise_as_the_autograd_function_does(transform):
+    import simplical_attn_amd as sa
+    x = [t.cuda() for t in make_inputs(2, 64, 1, 64, seed=8, with_dout=False)]
+    module, fn = _both(sa, 64)
+
+    def outcome(call):
+        if transform == "grad":
+            return _raised(lambda: torch.func.grad(lambda q: call(q, *x[1:]).sum())(x[0]))
+        if transform == "jvp":
+            return _raised(lambda: torch.func.jvp(lambda q: call(q, *x[1:]), (x[0],), (x[0],)))
+        return _raised(lambda: torch.func.vmap(call)(*[t[:, None] for t in x]))
+
+    assert outcome(module) is outcome(fn) is not None
+
+
+def test_saved_tensor_hooks_see_what_the_backward_needs():
+    import simplical_attn_amd as sa
+    *x, dout = [t.cuda() for t in make_inputs(1, 100, 2, 64, seed=9, dtype=torch.bfloat16)]
+    module, fn = _both(sa, 64)
+    want = _grads(fn, x, dout, (True,) * 5)
+    with torch.autograd.graph.save_on_cpu():
+        got = _grads(module, x, dout, (True,) * 5)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
