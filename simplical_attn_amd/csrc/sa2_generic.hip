@@ -365,7 +365,9 @@ __global__ __launch_bounds__(256) void rowdot_kernel(Tensor out, Tensor dout, fl
 
 // The same for rows on a 16-byte grid: a lane takes the 16-byte chunk of a row (8 or 4 elements) in one load per tensor,
 // the next power of two of the chunks of a row share it (at head_dim 96 in 16 bits: 12 of 16 lanes work).  Bound by
-// reading both tensors: fp32 B4 N7559 H8 D64 (124 MB) 53 us with a wavefront per row, 27 us so.
+// reading both tensors: fp32 B4 N7559 H8 D64 (124 MB) 53 us with a wavefront per row, 27 us so.  A lane adds its products
+// in pairs, which makes the sum as deep as the kernel above makes it, with the same error (a chain of the eight products
+// of 16-bit rows: 6 % more at head_dim 96).
 template <typename T>
 __global__ __launch_bounds__(256) void rowdot_vec_kernel(Tensor out, Tensor dout, float* dsum, int N, int H, int D, int lpr_log2,
                                                          int64_t rows) {
@@ -382,8 +384,15 @@ __global__ __launch_bounds__(256) void rowdot_vec_kernel(Tensor out, Tensor dout
         union { uint4 v; T e[PER]; } o, g;
         o.v = *(const uint4*)((const T*)out.p + out.off(b, i, h) + sub * PER);
         g.v = *(const uint4*)((const T*)dout.p + dout.off(b, i, h) + sub * PER);
+        float x[PER / 2];
 #pragma unroll
-        for (int t = 0; t < PER; ++t) s = fmaf(to_float(o.e[t]), to_float(g.e[t]), s);
+        for (int t = 0; t < PER / 2; ++t)
+            x[t] = fmaf(to_float(o.e[t + PER / 2]), to_float(g.e[t + PER / 2]), to_float(o.e[t]) * to_float(g.e[t]));
+#pragma unroll
+        for (int half = PER / 4; half > 0; half >>= 1)
+#pragma unroll
+            for (int t = 0; t < half; ++t) x[t] += x[t + half];
+        s = x[0];
     }
     for (int off = lpr >> 1; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
     if (row < rows && sub == 0) dsum[row] = s;

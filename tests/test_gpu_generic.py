@@ -249,6 +249,21 @@ def test_rowdot_kernels(D, dtype):
     assert torch.allclose(simplicial_rowdot(av, b).double(), want, rtol=1e-5, atol=1e-4)
 
 
+@pytest.mark.parametrize("D,dtype", [(64, torch.float32), (96, torch.float32), (96, torch.float16), (80, torch.bfloat16),
+                                     (128, torch.bfloat16)])
+def test_rowdot_kernels_are_equally_precise(D, dtype):
+    """The 16-byte-per-lane kernel against the element-wise one, which views off the 16-byte grid take: root mean square
+    errors against fp64 over 32768 rows, a figure that varies by under 1 % from seed to seed."""
+    from simplical_attn_amd import simplicial_rowdot
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(D)
+    a, b = (torch.randn(1, 16384, 2, D, generator=g).to(dtype).to(dev) for _ in range(2))
+    off = torch.zeros(1, 16384, 2, D + 4, dtype=dtype, device=dev)[..., 2:D + 2].copy_(a)
+    want = (a.double() * b.double()).sum(-1).permute(0, 2, 1)
+    vec, wave = ((simplicial_rowdot(t, b).double() - want).square().mean().sqrt().item() for t in (a, off))
+    assert vec <= 1.03 * wave
+
+
 def test_broadcast_views_are_accepted():
     """Losses that hand backward an expanded gradient (stride 0 along a summed axis) and keys
     expanded over heads (stride 0 on H) run, as the reference's stride-generic launch lets them
