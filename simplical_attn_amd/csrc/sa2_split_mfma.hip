@@ -2,10 +2,16 @@
 // the head dims the 16-bit kernels do not have, in kernels 32, 64, 96 and 128 columns wide.
 //
 // Every operand is carried as a sum of bf16 planes: x = h + m + l with h = bf16(x), m = bf16(x - h), l = bf16(x - h - m),
-// which holds all 24 bits of an fp32 value (bf16 has fp32's exponent range).  A product of two such sums is taken as
-// the MFMAs h*h, h*m, m*h, h*l, l*h, m*m (v_mfma_f32_32x32x16_bf16: exact 16-bit products, fp32 accumulation); what is
-// left out, m*l + l*m + l*l, is below 2^-26 of |x*y|, less than the rounding of an fp32 product.  bf16 tensors are one
-// plane and fp16 tensors two, exactly, so that with a three-plane partner they take three and five MFMAs.
+// which holds all 24 bits of an fp32 value.  A product of two such sums is taken as the MFMAs h*h, h*m, m*h, h*l, l*h, m*m
+// (v_mfma_f32_32x32x16_bf16: exact 16-bit products, a sum rounded to nearest once per eight of them); what is left out,
+// m*l + l*m + l*l, is below 2^-25 of |x*y| and below 2^-27 in the mean.  bf16 tensors are one plane and fp16 tensors two,
+// exactly, so that with a three-plane partner they take three and five MFMAs.
+//
+// Errors against fp64 (relative 2-norm, N(0,1) inputs; dq, dk1, dv1, dv2 in units of 1e-7), here and before:
+//   B1 H2 N128 D64 w 32/16     4.1 4.7 3.7 2.4   v_mfma_f32_32x32x2_f32 5.1 5.8 4.5 2.7, fp32 FMA kernels 3.3 3.6 2.3 2.1
+//   B1 H1 N2048 D64 w 512/32   5.5 7.5 6.3 3.2   v_mfma_f32_32x32x2_f32 6.6 9.2 7.4 4.0, fp32 FMA kernels 5.0 7.7 7.3 3.3
+//   B1 H1 N1024 D96 w 512/32   4.6 4.9 3.4 2.6   fp32 FMA kernels 4.7 8.0 7.3 3.0
+// (the outputs of 32, 64 and 128 columns stood on the fp32 MFMA before, the others on the FMA kernels).
 //
 // Why: v_mfma_f32_32x32x2_f32 runs at a sixteenth of the bf16 rate; six bf16 MFMAs do the same work in 6/16 of its
 // time.  The price is vector work (about 5.5 instructions to split a value), which runs beside the MFMAs.
@@ -69,7 +75,7 @@ struct SplitCfg {
     // K-side: a unit is the Q~ and dO~ tiles of three planes
     static constexpr int UNIT_TILE = 3 * PLANE;
     static constexpr int UNIT_STAGE = 2 * UNIT_TILE;
-    static constexpr size_t KV_LDS = (size_t)2 * UNIT_STAGE * 2 + PX_BYTES + 2 * 2 * 32 * 4;
+    static constexpr size_t KV_LDS = (size_t)2 * UNIT_STAGE * 2 + PX_BYTES + 2 * 2 * 32 * 16;
 };
 
 __device__ __forceinline__ floatx16 zero16() {
@@ -102,6 +108,10 @@ struct Mem16 {
         *(uint2*)p = make_uint2(E::pack(a, b), E::pack(c, d));
     }
 };
+
+// fp32 tensors of the padded head dims (and 96): finer sums, see Chain and accumulate
+template <class T, bool PAD>
+constexpr bool fine() { return T::DTYPE == SA2_F32 && PAD; }
 
 // Four columns of a row.  PAD: the tensors have width <= D columns; the kernel's columns from there on read as zeros
 // and are not written (rows are multiples of four elements, so four columns are inside or outside together).
@@ -159,15 +169,96 @@ __device__ __forceinline__ void store_planes(const fx4& x, uint16_t* dst, int pl
 #pragma unroll
     for (int n = 0; n < N; ++n) *(uint2*)(dst + n * plane) = make_uint2(a[n], b[n]);
 }
-// c += a * b over the planes whose product counts, the small ones first
-template <int NA, int NB>
-__device__ __forceinline__ floatx16 mma(const bf16x8 (&a)[NA], const bf16x8 (&b)[NB], floatx16 c) {
+// c += a * b over the plane products m*m, h*l, l*h (sum 2), h*m, m*h (1) and h*h (0) with LO <= sum <= HI, the small ones
+// first
+template <int LO, int HI, int NA, int NB>
+__device__ __forceinline__ floatx16 mma_sums(const bf16x8 (&a)[NA], const bf16x8 (&b)[NB], floatx16 c) {
 #pragma unroll
-    for (int sum = 2; sum >= 0; --sum)
+    for (int sum = HI; sum >= LO; --sum)
 #pragma unroll
         for (int x = 0; x < NA; ++x)
             if (sum - x >= 0 && sum - x < NB) c = ElemBF16::mfma(a[x], b[sum - x], c, 0, 0, 0);
     return c;
+}
+template <int NA, int NB>
+__device__ __forceinline__ floatx16 mma(const bf16x8 (&a)[NA], const bf16x8 (&b)[NB], floatx16 c) {
+    return mma_sums<0, 2>(a, b, c);
+}
+// A contraction over head_dim.  An MFMA rounds its sum once per eight products, so a chain of all plane products rounds
+// 0.75 D times at the size of the result.  FINE: the small products have a chain of their own, which leaves D / 8.  With
+// accumulate() below it costs B1 H8 N1024 D96 w 256/32 fp32 1.14 -> 1.32 ms a step and takes its errors from 1.3 times the
+// FMA kernels' to theirs.
+template <bool FINE>
+struct Chain {
+    floatx16 main, small;
+    __device__ __forceinline__ void clear() {
+        main = zero16();
+        if constexpr (FINE) small = zero16();
+    }
+    template <int NA, int NB>
+    __device__ __forceinline__ void add(const bf16x8 (&a)[NA], const bf16x8 (&b)[NB]) {
+        if constexpr (FINE) {
+            small = mma_sums<1, 2>(a, b, small);
+            main = mma_sums<0, 0>(a, b, main);
+        } else {
+            main = mma(a, b, main);
+        }
+    }
+    __device__ __forceinline__ floatx16 sum() const {
+        if constexpr (FINE) return main + small;
+        else return main;
+    }
+};
+// LSE*log2(e) or D is taken off a finished chain by one more MFMA: an operand of its planes against ones (in the lanes of
+// the first eight slots).  Subtracted last and exactly, it costs one rounding; a chain that starts from it rounds every
+// step at its size, which doubled the error of the gradients.
+__device__ __forceinline__ bf16x8 lead_planes(float x, float rest) {
+    union { uint32_t u[4]; bf16x8 v; } r;
+    uint32_t w[3];
+    split2<3>(-x, -rest, w);
+    r.u[0] = w[0]; r.u[1] = w[1]; r.u[2] = w[2]; r.u[3] = 0;
+    return r.v;
+}
+__device__ __forceinline__ bf16x8 lse_planes(float lse) {
+    constexpr float LOG2E_REST = 1.9259629911e-8f;       // log2(e) - LOG2E
+    const float x = lse * LOG2E;
+    return lead_planes(x, fmaf(lse, LOG2E, -x) + lse * LOG2E_REST);
+}
+__device__ __forceinline__ bf16x8 lead_ones(int hf) {
+    uint32_t w = hf ? 0u : 0x3f803f80u;
+    asm volatile("" : "+v"(w));                          // (made where it is used: four registers less to keep)
+    union { uint32_t u[4]; bf16x8 v; } r;
+    r.u[0] = r.u[1] = r.u[2] = r.u[3] = w;
+    return r.v;
+}
+// acc += the product of a 32-row tile; `operand(ks, dt, a)` reads its transposed operand.  FINE: the tile is summed by
+// itself, so that the accumulator over all tiles is rounded once per tile instead of 24 times.
+template <bool FINE, int NA, int DT, class Read>
+__device__ __forceinline__ void accumulate(floatx16 (&acc)[DT], const bf16x8 (&b)[2][3], Read&& operand) {
+    if constexpr (FINE) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+            bf16x8 a[2][NA];
+            floatx16 t = zero16();
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                operand(ks, dt, a[ks]);
+                t = mma_sums<1, 2>(a[ks], b[ks], t);
+            }
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) t = mma_sums<0, 0>(a[ks], b[ks], t);
+            acc[dt] += t;
+        }
+    } else {
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) {
+                bf16x8 a[NA];
+                operand(ks, dt, a);
+                acc[dt] = mma(a, b[ks], acc[dt]);
+            }
+    }
 }
 constexpr int mma_count(int na, int nb = 3) {
     int n = 0;
@@ -263,6 +354,7 @@ __global__ __launch_bounds__((SplitCfg<T, D>::FW * 64)) __attribute__((amdgpu_wa
 void split_fwd_kernel(Problem p, int nqb, int total) {
     using C = SplitCfg<T, D>;
     constexpr int W = C::FW, NT = W * 64;
+    constexpr bool FINE = fine<T, PAD>();
     typedef typename T::T EL;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_f[];
     uint16_t* tiles = (uint16_t*)smem_f;                                             // two stages
@@ -343,13 +435,15 @@ void split_fwd_kernel(Problem p, int nqb, int total) {
                 const int j0 = (jt_lo + s) * TJ;
                 const uint32_t Ks = tiles_addr + (uint32_t)((g & 1) * C::KV_STAGE * 2);
                 const uint32_t Vt = Ks + (uint32_t)(C::KV_TILE * 2) + col_lane;
-                floatx16 sacc = zero16();
+                Chain<FINE> logits;
+                logits.clear();
 #pragma unroll
                 for (int kk = 0; kk < C::DK; ++kk) {
                     bf16x8 ka[C::NK];
                     row_operand<C::NK, C::RSB>(Ks + row_lane, kk, ka);
-                    sacc = mma(ka, qf[kk], sacc);
+                    logits.add(ka, qf[kk]);
                 }
+                floatx16 sacc = logits.sum();
                 // register v of this lane: key j0 + 8*(v/4) + 4*hf + v%4
                 const bool interior = rows_full && (j0 + TJ - 1 <= i0) && (j0 >= i0 + BQ - 1 - w1);
                 if (!interior) {
@@ -388,14 +482,7 @@ void split_fwd_kernel(Problem p, int nqb, int total) {
                     split8<3>(pv, pb[ks]);
                 }
                 l += rs;
-#pragma unroll
-                for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-                    for (int dt = 0; dt < C::DT; ++dt) {
-                        bf16x8 va[C::NK];
-                        column_operand<C::NK, C::RSB>(Vt, ks, dt, va);
-                        racc[dt] = mma(va, pb[ks], racc[dt]);
-                    }
+                accumulate<FINE, C::NK>(racc, pb, [&](int ks, int dt, bf16x8 (&va)[C::NK]) { column_operand<C::NK, C::RSB>(Vt, ks, dt, va); });
             }
             // (unconditional: past the last step this moves a tile nobody reads, which is cheaper than a branch
             // around register arrays)
@@ -509,6 +596,7 @@ template <class T, int D, bool PAD>
 __global__ __launch_bounds__(XT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void split_kp_kernel(Problem p, int nkb, int per_seg, float* __restrict__ dq_part, int nseg, int segw, float* __restrict__ kpart) {
     using C = SplitCfg<T, D>;
+    constexpr bool FINE = fine<T, PAD>();
     typedef typename T::T EL;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_f[];
     uint16_t* tiles = (uint16_t*)smem_f;
@@ -574,7 +662,7 @@ void split_kp_kernel(Problem p, int nkb, int per_seg, float* __restrict__ dq_par
             const bool rows_full = k0 + 31 + delta < N;
 
             bf16x8 xf[C::DK][3];                              // Q~ (P wavefront) or dO~ (dS wavefront)
-            float c0 = 0.f;                                   // the C operand of the first chain: -LSE or -D
+            float lead = 0.f;                                 // LSE or D, to be taken off the first chain
             if (ok) {
 #pragma unroll
                 for (int kk = 0; kk < C::DK; ++kk) {
@@ -584,7 +672,7 @@ void split_kp_kernel(Problem p, int nkb, int per_seg, float* __restrict__ dq_par
                     else
                         product_planes<T, PAD>(dop + (int64_t)ic * p.dout.sn, v2p + (int64_t)kc * p.v2.sn, col, p.D, p.v2_bias, 1.f, xf[kk]);
                 }
-                c0 = ROLE == 0 ? -p.lse[(int64_t)bh * N + ic] * LOG2E : -p.dsum[(int64_t)bh * N + ic];
+                lead = (ROLE == 0 ? p.lse : p.dsum)[(int64_t)bh * N + ic];
             }
             floatx16 acc[C::DT];                              // R or G
 #pragma unroll
@@ -605,31 +693,34 @@ void split_kp_kernel(Problem p, int nkb, int per_seg, float* __restrict__ dq_par
                 const uint32_t Ks = tiles_addr + (uint32_t)((C::KP_STAGES == 2 ? s & 1 : 0) * C::KV_STAGE * 2);
                 const uint32_t Vs = Ks + (uint32_t)(C::KV_TILE * 2);
                 bf16x8 pb[2][3];
-                floatx16 chain;
+                floatx16 first;                               // logits less LSE, or dP less D
                 if (ROLE == 1 && C::KP_STAGES == 2) put_next(s);
                 if (in) {
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) chain[v] = c0;
-                    if (ROLE == 0 && !(rows_full && (j0 + TJ - 1 <= iw_lo) && (j0 >= iw_lo + 31 - w1))) {
-                        const int hi = i - j0 - 4 * hf, lo = hi - w1;
-#pragma unroll
-                        for (int v = 0; v < 16; ++v) {
-                            const int c = 8 * (v >> 2) + (v & 3);
-                            chain[v] = row_ok && c <= hi && c >= lo ? c0 : -INFINITY;
-                        }
-                    }
+                    Chain<FINE> chain;
+                    chain.clear();
                     if (ROLE == 0) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
                     for (int kk = 0; kk < C::DK; ++kk) {
                         bf16x8 a[C::NK];
                         row_operand<C::NK, C::RSB>((ROLE == 0 ? Ks : Vs) + row_lane, kk, a);
-                        chain = mma(a, xf[kk], chain);
+                        chain.add(a, xf[kk]);
                     }
+                    float x = lead;
+                    asm volatile("" : "+v"(x));               // (planes made where they are used: one register to keep)
+                    first = ElemBF16::mfma(lead_ones(hf), ROLE == 0 ? lse_planes(x) : lead_planes(x, 0.f), chain.sum(), 0, 0, 0);
                     if (ROLE == 0) {
                         __builtin_amdgcn_s_setprio(0);
                         float pv[16];
 #pragma unroll
-                        for (int v = 0; v < 16; ++v) pv[v] = fast_exp2(chain[v]);
+                        for (int v = 0; v < 16; ++v) pv[v] = fast_exp2(first[v]);
+                        if (!(rows_full && (j0 + TJ - 1 <= iw_lo) && (j0 >= iw_lo + 31 - w1))) {
+                            const int hi = i - j0 - 4 * hf, lo = hi - w1;
+#pragma unroll
+                            for (int v = 0; v < 16; ++v) {
+                                const int c = 8 * (v >> 2) + (v & 3);
+                                pv[v] = row_ok && c <= hi && c >= lo ? pv[v] : 0.f;
+                            }
+                        }
                         px_put(px, lane, pv);
                         split16<3>(pv, pb);
                     }
@@ -640,17 +731,12 @@ void split_kp_kernel(Problem p, int nkb, int per_seg, float* __restrict__ dq_par
                         float pv[16];
                         px_get(px, lane, pv);
 #pragma unroll
-                        for (int v = 0; v < 16; ++v) pv[v] *= chain[v];
+                        for (int v = 0; v < 16; ++v) pv[v] *= first[v];
                         split16<3>(pv, pb);
                     }
-#pragma unroll
-                    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-                        for (int dt = 0; dt < C::DT; ++dt) {
-                            bf16x8 a[C::NK];
-                            column_operand<C::NK, C::RSB>((ROLE == 0 ? Vs : Ks) + col_lane, ks, dt, a);
-                            acc[dt] = mma(a, pb[ks], acc[dt]);
-                        }
+                    accumulate<FINE, C::NK>(acc, pb, [&](int ks, int dt, bf16x8 (&a)[C::NK]) {
+                        column_operand<C::NK, C::RSB>((ROLE == 0 ? Vs : Ks) + col_lane, ks, dt, a);
+                    });
                 }
                 if (C::KP_STAGES == 1) __syncthreads();       // everyone is done with the only stage
                 if (ROLE == 0 || C::KP_STAGES == 1) put_next(s);
@@ -743,12 +829,12 @@ __global__ __launch_bounds__(XT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void split_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __restrict__ part) {
     const int nsplit = SPLIT ? nsplit_arg : 1;
     using C = SplitCfg<T, D>;
+    constexpr bool FINE = fine<T, PAD>();
     typedef typename T::T EL;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_f[];
     uint16_t* tiles = (uint16_t*)smem_f;
     float* px_all = (float*)(tiles + 2 * C::UNIT_STAGE);
-    float* lse_s = px_all + NPAIR * 1024;        // [2][32]  -LSE*log2(e) of the unit's queries
-    float* dsum_s = lse_s + 2 * 32;              // [2][32]  -D
+    unsigned char* lead_s = (unsigned char*)(px_all + NPAIR * 1024);     // [2][LSE, D][32 queries] lead_planes
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -847,8 +933,8 @@ void split_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __res
         if (tid < 32) {
             int i = ib * BQ + tid;
             i = i < N ? i : N - 1;
-            f_lse = -p.lse[(int64_t)bh * N + i] * LOG2E;
-            f_dsum = -p.dsum[(int64_t)bh * N + i];
+            f_lse = p.lse[(int64_t)bh * N + i];
+            f_dsum = p.dsum[(int64_t)bh * N + i];
         }
     };
     auto store_unit = [&](int buf) {
@@ -867,8 +953,8 @@ void split_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __res
             store_planes<T, 3>(dt, Ds + row * C::RS + col * 4, C::PLANE);
         }
         if (tid < 32) {
-            lse_s[buf * 32 + tid] = f_lse;
-            dsum_s[buf * 32 + tid] = f_dsum;
+            *(bf16x8*)(lead_s + (buf * 64 + tid) * 16) = lse_planes(f_lse);
+            *(bf16x8*)(lead_s + (buf * 64 + 32 + tid) * 16) = lead_planes(f_dsum, 0.f);
         }
     };
 
@@ -892,38 +978,34 @@ void split_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __res
             const uint32_t Qs = tiles_addr + (uint32_t)(buf * C::UNIT_STAGE * 2);
             const uint32_t Ds = Qs + (uint32_t)(C::UNIT_TILE * 2);
             bf16x8 pb[2][3];
-            floatx16 chain;
+            floatx16 first;                   // logits less LSE, or dP less D: register v is query i0 + 8*(v/4) + 4*hf + v%4
             if (touches) {
-                // register v of this lane: query i0 + 8*(v/4) + 4*hf + v%4, key j; -LSE (-inf outside the window) or -D
-                const float* c0 = (ROLE == 0 ? lse_s : dsum_s) + buf * 32 + 4 * hf;
-#pragma unroll
-                for (int g4 = 0; g4 < 4; ++g4) {
-                    const fx4 x = *(const fx4*)(c0 + 8 * g4);
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) chain[4 * g4 + t] = x[t];
-                }
-                if (ROLE == 0 && !((i0 >= jw + 31) && ((int64_t)i0 + 31 <= (int64_t)jw + w1) && (i0 + BQ - 1 < N) && (i0 >= delta))) {
-                    const int lo = j - i0 - 4 * hf;                                    // c >= lo  <=>  j <= i
-                    const int hi = (int)((int64_t)j + w1 - i0 < (1 << 20) ? j + w1 - i0 : (1 << 20)) - 4 * hf;   // i <= j + w1
-                    const int dlo = delta - i0 - 4 * hf, nhi = N - 1 - i0 - 4 * hf;
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) {
-                        const int c = 8 * (v >> 2) + (v & 3);
-                        chain[v] = (j < N) && (c >= lo) && (c <= hi) && (c >= dlo) && (c <= nhi) ? chain[v] : -INFINITY;
-                    }
-                }
+                Chain<FINE> chain;
+                chain.clear();
                 if (ROLE == 0) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
                 for (int kk = 0; kk < C::DK; ++kk) {
                     bf16x8 a[3];
                     row_operand<3, C::RSB>((ROLE == 0 ? Qs : Ds) + row_lane, kk, a);
-                    chain = mma(a, kf[kk], chain);
+                    chain.add(a, kf[kk]);
                 }
+                const bf16x8 lead = *(const bf16x8*)(lead_s + (buf * 64 + ROLE * 32 + ln) * 16);
+                first = ElemBF16::mfma(lead, lead_ones(hf), chain.sum(), 0, 0, 0);
                 if (ROLE == 0) {
                     __builtin_amdgcn_s_setprio(0);
                     float pv[16];
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) pv[v] = fast_exp2(chain[v]);
+                    for (int v = 0; v < 16; ++v) pv[v] = fast_exp2(first[v]);
+                    if (!((i0 >= jw + 31) && ((int64_t)i0 + 31 <= (int64_t)jw + w1) && (i0 + BQ - 1 < N) && (i0 >= delta))) {
+                        const int lo = j - i0 - 4 * hf;                                    // c >= lo  <=>  j <= i
+                        const int hi = (int)((int64_t)j + w1 - i0 < (1 << 20) ? j + w1 - i0 : (1 << 20)) - 4 * hf;   // i <= j + w1
+                        const int dlo = delta - i0 - 4 * hf, nhi = N - 1 - i0 - 4 * hf;
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) {
+                            const int c = 8 * (v >> 2) + (v & 3);
+                            pv[v] = (j < N) && (c >= lo) && (c <= hi) && (c >= dlo) && (c <= nhi) ? pv[v] : 0.f;
+                        }
+                    }
                     px_put(px, lane, pv);
                     split16<3>(pv, pb);
                 }
@@ -934,17 +1016,12 @@ void split_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __res
                     float pv[16];
                     px_get(px, lane, pv);
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) pv[v] *= chain[v];
+                    for (int v = 0; v < 16; ++v) pv[v] *= first[v];
                     split16<3>(pv, pb);
                 }
-#pragma unroll
-                for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-                    for (int dt = 0; dt < C::DT; ++dt) {
-                        bf16x8 a[3];
-                        column_operand<3, C::RSB>((ROLE == 0 ? Ds : Qs) + col_lane, ks, dt, a);
-                        acc[dt] = mma(a, pb[ks], acc[dt]);
-                    }
+                accumulate<FINE, 3>(acc, pb, [&](int ks, int dt, bf16x8 (&a)[3]) {
+                    column_operand<3, C::RSB>((ROLE == 0 ? Ds : Qs) + col_lane, ks, dt, a);
+                });
             }
             if (!more) break;
             store_unit(buf ^ 1);          // (the other buffer was last read one step ago, before that step's barrier)
