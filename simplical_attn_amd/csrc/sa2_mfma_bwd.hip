@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(Problem p, int D, int64_
 #pragma unroll 4
     for (int x = 0; x < p.nsplit; ++x) {
         const float2 s = ml[x * rows + row];
-        if (s.x == -INFINITY) continue;                                // (an empty share left no sums)
+        if (s.x == -INFINITY && s.y == 0.f) continue;                  // (an empty share left no sums; NaN logits leave L NaN)
         const float w = fast_exp2(s.x - Mu);
         const float4 y = *(const float4*)(part + (x * rows + row) * D + col);
         L += w * s.y;

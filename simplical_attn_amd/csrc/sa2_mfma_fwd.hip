@@ -932,7 +932,7 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
 #pragma unroll
         for (int w = 0; w < FW; ++w) {
             const float mw = xch_m[w * BQ + aq];
-            Ln += mw == -INFINITY ? 0.f : xch_l[w * BQ + aq] * fast_exp2(mw - Mq_use);
+            Ln += xch_l[w * BQ + aq] * (mw == -INFINITY ? 0.f : fast_exp2(mw - Mq_use));      // (NaN logits: Mw -inf, Lw NaN)
         }
         float acc[ACN];
         {

@@ -39,3 +39,15 @@ def test_shares_of_the_rounds_merge_to_the_oracle(dtype, case, scale):
     assert_close_rel(out, o1.float().cpu(), {torch.float32: 1e-5 if scale is None else 2e-4}.get(dtype, 1e-2), "out, shared against whole")
     assert_close_rel(lse, l1.cpu(), 1e-5 if dtype == torch.float32 else 1e-3, "lse, shared against whole")
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 32), (torch.bfloat16, 64), (torch.float16, 128), (torch.bfloat16, 96),
+                                     (torch.bfloat16, 256), (torch.float32, 64), (torch.float32, 96)])
+def test_a_query_that_is_not_a_number_stays_one_through_the_merge(dtype, D):
+    import simplical_attn_amd as sa
+    assert _lib.load().sa2_fwd_workspace_bytes(1, 160, 1, D, 40, 60, CODE[dtype], 1, 0) > 0
+    x = [t.cuda() for t in make_inputs(1, 160, 1, D, seed=2, dtype=dtype, with_dout=False)]
+    x[0][:, 70] = float("nan")
+    out, _ = sa.simplicial_forward(*x, 40, 60)
+    rows = out[0, :, 0].isnan()
+    assert rows[70].all() and rows.sum().item() == D
