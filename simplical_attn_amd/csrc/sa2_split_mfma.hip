@@ -39,6 +39,7 @@
 // computes S and, beside the other's dP MFMAs, the exponentials and the split of P; in the second it adds P's product
 // while the dS wavefront multiplies and splits dS, whose product follows.
 // Every output element has one writer and a fixed summation order: no atomics, bitwise reproducible.
+#include "sa2_fma_rows.h"
 #include "sa2_mfma_common.h"
 
 namespace sa2 {
@@ -47,10 +48,12 @@ namespace {
 constexpr int NPAIR = 4;               // wavefront pairs per workgroup of the backward kernels
 constexpr int XT = NPAIR * 2 * 64;     // threads per workgroup
 constexpr int XJ = NPAIR * 32;         // K rows per workgroup of the K-side kernel
+constexpr float TINY = 7.888609052210118e-31f;     // 2^-100
 
 template <class T, int D>
 struct SplitCfg {
     static constexpr int NK = T::PLANES;       // planes of a K or V tile
+    static constexpr bool LIMIT = T::DTYPE == SA2_F32;
     static constexpr int DK = D / 16;          // k-steps of a contraction over head_dim
     static constexpr int DT = D / 32;          // 32-column blocks of an output contraction
     static constexpr int RS = D + 16;          // row stride of a plane (elements)
@@ -64,7 +67,9 @@ struct SplitCfg {
     static constexpr int KV_STAGE = 2 * KV_TILE;           // K tile, then V tile
     static constexpr size_t FWD_TILES = (size_t)2 * KV_STAGE * 2;
     static constexpr size_t FWD_MERGE = (size_t)FW * 32 * AS * 4;
-    static constexpr size_t FWD_LDS = (FWD_TILES > FWD_MERGE ? FWD_TILES : FWD_MERGE) + 2 * FW * 32 * 4;
+    static constexpr size_t FWD_FMA = smem_bytes(D, FW);
+    static constexpr size_t larger(size_t a, size_t b) { return a > b ? a : b; }
+    static constexpr size_t FWD_LDS = larger(FWD_FMA, larger(FWD_TILES, FWD_MERGE)) + 2 * FW * 32 * 4;
     // K'-side: two stages, or one (a barrier more per tile) where two would leave no room for the dQ accumulator
     static constexpr int KP_STAGES = D == 128 && NK == 3 ? 1 : 2;
     static constexpr size_t KP_TILES = (size_t)KP_STAGES * KV_STAGE * 2;
@@ -92,6 +97,7 @@ typedef unsigned ux2 __attribute__((ext_vector_type(2)));
 struct MemF32 {
     typedef float T;
     typedef fx4 Raw;
+    typedef float Fma;                             // the type's name in sa2_fma_rows.h
     static constexpr int DTYPE = SA2_F32;
     static constexpr int PLANES = 3;
     static __device__ __forceinline__ fx4 widen(Raw x) { return x; }
@@ -101,6 +107,7 @@ template <class E>
 struct Mem16 {
     typedef uint16_t T;
     typedef ux2 Raw;
+    typedef typename std::conditional<E::DTYPE == SA2_BF16, bf16_t, f16_t>::type Fma;
     static constexpr int DTYPE = E::DTYPE;
     static constexpr int PLANES = E::DTYPE == SA2_BF16 ? 1 : 2;      // bf16 planes that hold a value exactly
     static __device__ __forceinline__ fx4 widen(Raw x) { return fx4{E::lo(x[0]), E::hi(x[0]), E::lo(x[1]), E::hi(x[1])}; }
@@ -135,10 +142,12 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {          // one v_
     r.v = __builtin_convertvector((f32x2{a, b}), bf16x2);
     return r.u;
 }
-// The first N planes of two values (packed pairs)
-template <int N>
+// The first N planes of two values (packed pairs).  LIMIT: values above the largest bf16 (fp32's lowest values, which mask
+// keys, among them) are split from there on; without it their first plane would be infinite.
+template <int N, bool LIMIT = false>
 __device__ __forceinline__ void split2(float a, float b, uint32_t (&o)[N]) {
-    o[0] = pack2(a, b);
+    constexpr float MOST = 3.3895313892515355e38f;
+    o[0] = LIMIT ? pack2(__builtin_amdgcn_fmed3f(a, -MOST, MOST), __builtin_amdgcn_fmed3f(b, -MOST, MOST)) : pack2(a, b);
 #pragma unroll
     for (int n = 1; n < N; ++n) {
         a -= bf16_lo(o[n - 1]);
@@ -147,13 +156,13 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t (&o)[N]) {
     }
 }
 // Eight values (two groups of four) as an MFMA operand per plane
-template <int N>
+template <int N, bool LIMIT = false>
 __device__ __forceinline__ void split8(const float (&x)[8], bf16x8 (&o)[N]) {
     union { uint32_t u[4]; bf16x8 v; } r[N];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
         uint32_t w[N];
-        split2<N>(x[2 * t], x[2 * t + 1], w);
+        split2<N, LIMIT>(x[2 * t], x[2 * t + 1], w);
 #pragma unroll
         for (int n = 0; n < N; ++n) r[n].u[t] = w[n];
     }
@@ -161,11 +170,11 @@ __device__ __forceinline__ void split8(const float (&x)[8], bf16x8 (&o)[N]) {
     for (int n = 0; n < N; ++n) o[n] = r[n].v;
 }
 // Four columns to the planes of a tile (`dst`: plane 0; planes lie `plane` elements apart)
-template <class T, int N>
+template <int N, bool LIMIT>
 __device__ __forceinline__ void store_planes(const fx4& x, uint16_t* dst, int plane) {
     uint32_t a[N], b[N];
-    split2<N>(x[0], x[1], a);
-    split2<N>(x[2], x[3], b);
+    split2<N, LIMIT>(x[0], x[1], a);
+    split2<N, LIMIT>(x[2], x[3], b);
 #pragma unroll
     for (int n = 0; n < N; ++n) *(uint2*)(dst + n * plane) = make_uint2(a[n], b[n]);
 }
@@ -331,8 +340,8 @@ struct TileRegs {
             const int c = tid + NT * u;
             if (ALL % NT != 0 && c >= ALL) break;
             const int row = c / (D / 4), col = c - row * (D / 4);
-            store_planes<T, C::NK>(T::widen(a[u]), stage + row * C::RS + col * 4, C::PLANE);
-            store_planes<T, C::NK>(T::widen(b[u]), stage + C::KV_TILE + row * C::RS + col * 4, C::PLANE);
+            store_planes<C::NK, C::LIMIT>(T::widen(a[u]), stage + row * C::RS + col * 4, C::PLANE);
+            store_planes<C::NK, C::LIMIT>(T::widen(b[u]), stage + C::KV_TILE + row * C::RS + col * 4, C::PLANE);
         }
     }
 };
@@ -531,6 +540,7 @@ void split_fwd_kernel(Problem p, int nqb, int total) {
     __syncthreads();
     constexpr int TPR = NT / 32;                           // threads per row
     const int row = tid / TPR, io = i0 + row;
+    bool nan = false, tiny = false, usual = T::DTYPE != SA2_F32;      // of the results (see below)
     if (io < N) {
         float Mx = -INFINITY;
 #pragma unroll
@@ -558,13 +568,45 @@ void split_fwd_kernel(Problem p, int nqb, int total) {
                 const float4 y = *(const float4*)(mrg + (w * 32 + row) * C::AS + col);
                 acc.x += wgt[w] * y.x; acc.y += wgt[w] * y.y; acc.z += wgt[w] * y.z; acc.w += wgt[w] * y.w;
             }
+            const float r[4] = {acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv};
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                nan |= r[t] != r[t];
+                if (T::DTYPE == SA2_F32) {
+                    usual |= fabsf(r[t]) >= TINY;
+                    tiny |= r[t] != 0.f && fabsf(r[t]) < TINY;
+                }
+            }
             if constexpr (SPLIT) *(float4*)((float*)p.scratch + 2 * rows * p.nsplit + prow * D + col) = acc;
-            else T::store(orow + col, acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+            else T::store(orow + col, r[0], r[1], r[2], r[3]);
         }
         if (!SPLIT && tid % TPR == 0)
             p.lse[(int64_t)bh * N + io] = big ? LN2 * Mu + logf(denom) : LN_EPS + logf(denom);
+        nan |= Ls != Ls;
     }
+
+    // ---- what the planes do not cover: the block again, by rows, in fp32 FMA arithmetic ----
+    // Infinite operands (their lower planes are NaN) and NaN in rows that the windows leave out (a weight of zero times
+    // NaN) both show as NaN in the results.  fp32 values under 2^-110 have lost their last plane; a block whose results
+    // all lie under TINY may come from such.
+    if (!__syncthreads_or(nan || tiny)) return;
+    const bool any_nan = __syncthreads_or(nan), any_usual = __syncthreads_or(usual);
+    if (!any_nan && any_usual) return;
+    const int d_lo = round0 * W, d_hi = round1 * W - 1 < w2 ? round1 * W - 1 : w2;
+    for (int r0 = 0; r0 < BQ && i0 + r0 < N; r0 += W)
+        fma_fwd_rows<typename T::Fma>(p, bh, i0 + r0, d_lo, d_hi, (float*)smem_f, [&](int ir, int ln_r, float m, float l, const float (&acc)[MAXC]) {
+            if constexpr (SPLIT) {
+                const int64_t rows = (int64_t)p.B * p.H * N, prow = share * rows + (int64_t)bh * N + ir;
+                if (ln_r == 0) ((float2*)p.scratch)[prow] = make_float2(m * LOG2E, l);
+#pragma unroll
+                for (int c = 0; c < MAXC; ++c)
+                    if (ln_r + 64 * c < p.D) ((float*)p.scratch)[2 * rows * p.nsplit + prow * D + ln_r + 64 * c] = acc[c];
+            } else {
+                fma_store_row<typename T::Fma>(p, bh, ir, ln_r, m, l, acc);
+            }
+        });
 }
+
 
 // ============================================== backward, K' side: dQ, dK', dV' =====
 // P between the wavefronts of a pair: 16 values per lane as four 16-byte chunks, chunk-major (no bank conflicts)
@@ -869,7 +911,7 @@ void split_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __res
             const int col = kk * 16 + hf * 8;
             const float4 x0 = cols4<T, PAD>(row, col, p.D), x1 = cols4<T, PAD>(row, col + 4, p.D);
             const float r[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-            split8<C::NK>(r, kf[kk]);
+            split8<C::NK, C::LIMIT>(r, kf[kk]);
         }
     }
     floatx16 acc[C::DT];                         // dV^T or dK^T
@@ -949,8 +991,8 @@ void split_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __res
             const fx4 q4 = T::widen(fq[u]), k4 = T::widen(fk[u]), d4 = T::widen(fd[u]), v4 = T::widen(fv[u]);
             const fx4 qt = {q4[0] * qscale * (k4[0] + kb), q4[1] * qscale * (k4[1] + kb), q4[2] * qscale * (k4[2] + kb), q4[3] * qscale * (k4[3] + kb)};
             const fx4 dt = {d4[0] * (v4[0] + vb), d4[1] * (v4[1] + vb), d4[2] * (v4[2] + vb), d4[3] * (v4[3] + vb)};
-            store_planes<T, 3>(qt, Qs + row * C::RS + col * 4, C::PLANE);
-            store_planes<T, 3>(dt, Ds + row * C::RS + col * 4, C::PLANE);
+            store_planes<3, false>(qt, Qs + row * C::RS + col * 4, C::PLANE);
+            store_planes<3, false>(dt, Ds + row * C::RS + col * 4, C::PLANE);
         }
         if (tid < 32) {
             *(bf16x8*)(lead_s + (buf * 64 + tid) * 16) = lse_planes(f_lse);

@@ -1,0 +1,64 @@
+"""Values that the plane-split kernels (fp32 tensors, and 16-bit tensors of head dims without kernels of their own) do not
+carry as sums of bf16 planes: infinities, NaN in rows that the windows leave out, fp32's lowest values as masks, and tensors
+so small that their last plane is lost.  All must come out as on the fp32 FMA kernels, which sum valid pairs only."""
+import pytest
+import torch
+
+from tests.util import make_inputs
+
+pytestmark = pytest.mark.gpu
+AUTO, GENERIC = 0, 1
+BAR = {torch.float32: 3e-6, torch.float16: 2e-3, torch.bfloat16: 1.5e-2}      # relative 2-norm, two roundings apart
+LAYOUTS = [(torch.float32, 64, 20), (torch.float32, 64, 3), (torch.float32, 128, 40), (torch.float32, 96, 20), (torch.float32, 16, 3),
+           (torch.bfloat16, 96, 40), (torch.float16, 80, 3)]                  # few and many deltas: whole blocks and shares
+
+
+def _inputs(dtype, D, what):
+    x = [t.cuda() for t in make_inputs(1, 200, 2, D, seed=D, dtype=dtype)]
+    inf, nan = float("inf"), float("nan")
+    if what == "infinity in a value":
+        x[4] = x[4].abs()
+        x[3][:, 90, :, 5] = inf
+    elif what == "minus infinity in a key":
+        x[0], x[2] = x[0].abs(), x[2].abs()
+        x[1][:, 90] = -inf
+    elif what == "NaN value":
+        x[3][:, 90] = nan
+    elif what == "NaN query":
+        x[0][:, 90, :, 1] = nan
+    elif what == "infinity in V'":
+        x[4][:, 90, :, 0] = inf
+    elif what == "mask":
+        x[0], x[2] = x[0].abs(), x[2].abs()
+        x[1][:, 80:90] = torch.finfo(dtype).min
+    elif what == "small values":
+        x[3] = x[3] * 1e-36
+    elif what == "small keys":
+        x[1] = x[1] * 1e-36
+    return x
+
+
+def _same(got, want, bar, name):
+    got, want = got.double(), want.double()
+    assert torch.equal(got.isnan(), want.isnan()), name
+    assert torch.equal(got.isinf(), want.isinf()), name
+    assert torch.equal(got[want.isinf()] > 0, want[want.isinf()] > 0), name
+    ok = want.isfinite()
+    diff, size = (got[ok] - want[ok]).norm().item(), want[ok].norm().item()
+    assert diff <= bar * size, (name, diff, size)
+
+
+FORWARD = ["infinity in a value", "minus infinity in a key", "NaN value", "NaN query", "infinity in V'", "mask", "small values", "small keys"]
+
+
+def _cases(kinds):         # (the small tensors are an fp32 range)
+    return [(*layout, what) for layout in LAYOUTS for what in kinds if layout[0] == torch.float32 or not what.startswith("small")]
+
+
+@pytest.mark.parametrize("dtype,D,w2,what", _cases(FORWARD))
+def test_forward(dtype, D, w2, what):
+    import simplical_attn_amd as sa
+    x = _inputs(dtype, D, what)
+    got, want = (sa.simplicial_forward(*x[:5], 40, w2, flags=flags) for flags in (AUTO, GENERIC))
+    _same(got[0], want[0], BAR[dtype], "out")
+    _same(got[1], want[1], 1e-6, "lse")
