@@ -2,7 +2,8 @@
 // the head dims the 16-bit kernels do not have, in kernels 32, 64, 96 and 128 columns wide.
 //
 // Every operand is carried as a sum of bf16 planes: x = h + m + l with h = bf16(x), m = bf16(x - h), l = bf16(x - h - m),
-// which holds all 24 bits of an fp32 value.  A product of two such sums is taken as the MFMAs h*h, h*m, m*h, h*l, l*h, m*m
+// which holds all 24 bits of an fp32 value (under 2^-110 those down to 2^-133; blocks of such values, and infinities, are
+// computed by rows, see the end of split_fwd_kernel and split_guard_kernel).  A product of two such sums is taken as the MFMAs h*h, h*m, m*h, h*l, l*h, m*m
 // (v_mfma_f32_32x32x16_bf16: exact 16-bit products, a sum rounded to nearest once per eight of them); what is left out,
 // m*l + l*m + l*l, is below 2^-25 of |x*y| and below 2^-27 in the mean.  bf16 tensors are one plane and fp16 tensors two,
 // exactly, so that with a three-plane partner they take three and five MFMAs.
@@ -608,6 +609,102 @@ void split_fwd_kernel(Problem p, int nqb, int total) {
 }
 
 
+// ============================================== backward: which arithmetic =====
+// The row term, and whether the planes cover the operands: they do not where one is infinite or NaN, where products of q
+// and K' or of dO and V' may overflow, and (fp32) where all of a tensor's values in a workgroup's rows are so small, and
+// not zero, that products of them come under 2^-110.  Each workgroup takes a run of consecutive rows and leaves its
+// verdict in guard[blockIdx.x].  The two kernels below run whatever it says; if any is set, split_fma_bwd_kernel computes all
+// gradients again by rows.  Bound by reading the seven tensors once: fp32 B2 H8 N2048 D64 (59 MB) 16 us, the row term alone
+// 9; the launch that looks at the verdicts 5.
+constexpr int GUARD_MOST = 1024, GUARD_ROWS = 64;      // workgroups at most, rows per workgroup at least
+inline int guard_blocks(int64_t rows) {
+    const int64_t n = (rows + GUARD_ROWS - 1) / GUARD_ROWS;
+    return (int)(n < GUARD_MOST ? n : GUARD_MOST);
+}
+size_t guard_bytes(int B, int N, int H) { return ((size_t)guard_blocks((int64_t)B * H * N) * sizeof(int) + 255) / 256 * 256; }
+constexpr float GUARD_HIGH = 1.152921504606847e18f;    // 2^60: twice that is an exponent short of fp32's largest
+constexpr float GUARD_LOW = 8.881784197001252e-16f;    // 2^-50; dO: 2^-60
+constexpr float GUARD_LOW_DO = 8.673617379884035e-19f;
+template <class T>
+__global__ __launch_bounds__(256) void split_guard_kernel(Problem p, int lpr_log2, int64_t rows, int64_t per_block, int* __restrict__ guard) {
+    constexpr int PER = 16 / sizeof(typename T::T), SETS = 7;
+    constexpr bool F32 = T::DTYPE == SA2_F32;
+    const int lane = threadIdx.x & 63, lpr = 1 << lpr_log2, sub = lane & (lpr - 1);       // lanes per row
+    const int step = 4 << (6 - lpr_log2);
+    const int64_t first = (int64_t)blockIdx.x * per_block, last = first + per_block < rows ? first + per_block : rows;
+    const Tensor* const set[SETS] = {&p.dout, &p.q, &p.k2, &p.v2, &p.k1, &p.v1, &p.out};  // the first four enter products
+    bool bad = false;
+    unsigned seen = 0;                       // bit t: tensor t has a usual value here, bit 8 + t: one that is small but not zero
+    for (int64_t r0 = first; r0 < last; r0 += step) {
+        const int64_t row = r0 + ((int)(threadIdx.x >> 6) << (6 - lpr_log2)) + (lane >> lpr_log2);
+        float s = 0.f;
+        if (row < last && sub * PER < p.D) {
+            const int i = (int)(row % p.N), bh = (int)(row / p.N), b = bh / p.H, h = bh - b * p.H;
+            union { uint4 v; typename T::Fma e[PER]; } x[SETS];
+#pragma unroll
+            for (int t = 0; t < SETS; ++t) x[t].v = *(const uint4*)((const typename T::T*)set[t]->p + set[t]->off(b, i, h) + sub * PER);
+            float y[PER / 2];
+#pragma unroll
+            for (int e = 0; e < PER / 2; ++e)
+                y[e] = fmaf(to_float(x[6].e[e + PER / 2]), to_float(x[0].e[e + PER / 2]), to_float(x[6].e[e]) * to_float(x[0].e[e]));
+#pragma unroll
+            for (int half = PER / 4; half > 0; half >>= 1)
+#pragma unroll
+                for (int e = 0; e < half; ++e) y[e] += y[e + half];
+            s = y[0];
+#pragma unroll
+            for (int t = 0; t < SETS; ++t) {
+                float most = 0.f;
+#pragma unroll
+                for (int e = 0; e < PER; ++e) {
+                    const float a = fabsf(to_float(x[t].e[e]));
+                    bad |= !(a < INFINITY);
+                    most = fmaxf(most, a);
+                }
+                if (t < 4) bad |= most >= GUARD_HIGH;
+                if (F32 && t < 6) {
+                    const bool usual = most >= (t == 0 ? GUARD_LOW_DO : GUARD_LOW);
+                    seen |= (usual ? 1u : most > 0.f ? 256u : 0u) << t;
+                }
+            }
+            if (sub == 0) {
+                const float lse = p.lse[row];
+                bad |= !(fabsf(lse) < INFINITY);
+            }
+        }
+        for (int off = lpr >> 1; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+        bad |= s != s;
+        if (row < last && sub == 0) p.dsum[row] = s;
+    }
+    if constexpr (F32) {
+        for (int t = 0; t < 6; ++t) {
+            const bool usual = __syncthreads_or(seen >> t & 1), small = __syncthreads_or(seen >> (8 + t) & 1);
+            bad |= small && !usual;
+        }
+    }
+    const int verdict = __syncthreads_or(bad);
+    if (threadIdx.x == 0) guard[blockIdx.x] = verdict;
+}
+__device__ __forceinline__ bool guarded(const int* __restrict__ guard, int n) {
+    int any = 0;
+    for (int c = threadIdx.x; c < n; c += blockDim.x) any |= guard[c];
+    return __syncthreads_or(any);
+}
+// All gradients by rows, where the guard says so (launched last: it overwrites what the sums left)
+constexpr int FMA_ROWS = 4, FMA_BLOCKS = 512;
+template <class E>
+__global__ __launch_bounds__(FMA_ROWS * 64) void split_fma_bwd_kernel(Problem p, const int* __restrict__ guard, int nguard, int nblk, int64_t blocks) {
+    extern __shared__ float smem[];
+    if (!guarded(guard, nguard)) return;
+    const OwnerArgs k = owner_k(p), k2 = owner_k2(p);
+    for (int64_t x = blockIdx.x; x < blocks; x += gridDim.x) {
+        const int bh = (int)(x / nblk), first = (int)(x - (int64_t)bh * nblk) * FMA_ROWS;
+        if (p.dq.p) fma_dq_rows<E>(p, bh, first, smem);
+        if (p.dk1.p || p.dv1.p) fma_owner_rows<E>(p, k, bh, first, smem);
+        if (p.dk2.p || p.dv2.p) fma_owner_rows<E>(p, k2, bh, first, smem);
+    }
+}
+
 // ============================================== backward, K' side: dQ, dK', dV' =====
 // P between the wavefronts of a pair: 16 values per lane as four 16-byte chunks, chunk-major (no bank conflicts)
 __device__ __forceinline__ void px_put(float* px, int lane, const float (&p)[16]) {
@@ -1146,13 +1243,21 @@ int launch_split_fwd(const Problem& p, hipStream_t st) {
 template <class T, int D, bool PAD>
 int launch_split_bwd(const Problem& p, hipStream_t st) {
     using C = SplitCfg<T, D>;
-    int rc = launch_rowdot(p.out, p.dout, p.dsum, p.B, p.N, p.H, p.D, T::DTYPE, st);
-    if (rc != SA2_OK) return rc;
     BwdSums sums = {};
     const KpPlan pl = split_kp_plan<T, D>(p.B, p.N, p.H, p.w1, p.w2);
     const size_t kp_bytes = (split_kp_bytes(p.B, p.N, p.H, D, pl) + 255) / 256 * 256;
     const int nsplit = split_kv_nsplit(p.B, p.N, p.H, D, p.w1, p.w2);
-    if (p.scratch_bytes < kp_bytes + split_kv_bytes(p.B, p.N, p.H, D, nsplit)) return SA2_ERR_WORKSPACE_TOO_SMALL;
+    const size_t part_bytes = kp_bytes + split_kv_bytes(p.B, p.N, p.H, D, nsplit);
+    if (p.scratch_bytes < part_bytes + guard_bytes(p.B, p.N, p.H)) return SA2_ERR_WORKSPACE_TOO_SMALL;
+    int* guard = (int*)((char*)p.scratch + part_bytes);
+    const int64_t rows = (int64_t)p.B * p.H * p.N;
+    const int nguard = guard_blocks(rows);
+    {
+        int lpr_log2 = 0;
+        while ((int)(16 / sizeof(typename T::T)) << lpr_log2 < p.D) ++lpr_log2;
+        hipLaunchKernelGGL(split_guard_kernel<T>, dim3((unsigned)nguard), dim3(256), 0, st, p, lpr_log2, rows, (rows + nguard - 1) / nguard, guard);
+        if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
+    }
     if (p.dq.p || p.dk2.p || p.dv2.p) {
         const int nkb = (p.N + BQ - 1) / BQ;
         const int64_t per_seg = (int64_t)nkb * p.B * p.H, total = per_seg * pl.nseg;
@@ -1183,7 +1288,14 @@ int launch_split_bwd(const Problem& p, hipStream_t st) {
         sums.kv = part;
         sums.kv_n = nsplit;
     }
-    return launch_bwd_sums(p, sums, D, T::DTYPE, st);
+    const int rc = launch_bwd_sums(p, sums, D, T::DTYPE, st);
+    if (rc != SA2_OK) return rc;
+    const int nblk = (p.N + FMA_ROWS - 1) / FMA_ROWS;
+    const int64_t blocks = (int64_t)nblk * p.B * p.H;
+    if (!allow_full_lds((const void*)split_fma_bwd_kernel<typename T::Fma>)) return SA2_ERR_LAUNCH_FAILED;
+    hipLaunchKernelGGL(split_fma_bwd_kernel<typename T::Fma>, dim3((unsigned)(blocks < FMA_BLOCKS ? blocks : FMA_BLOCKS)), dim3(FMA_ROWS * 64),
+                       smem_bytes(p.D, FMA_ROWS), st, p, guard, nguard, nblk, blocks);
+    return hipGetLastError() == hipSuccess ? SA2_OK : SA2_ERR_LAUNCH_FAILED;
 }
 
 // rows on a 16-byte grid
@@ -1250,7 +1362,7 @@ size_t f32_mfma_bwd_scratch_bytes(int B, int N, int H, int head_dim, int w1, int
     for_split_width(head_dim, dtype, [&](auto m, auto width, auto) {
         constexpr int D = decltype(width)::value;
         bytes = (split_kp_bytes(B, N, H, D, split_kp_plan<decltype(m), D>(B, N, H, w1, w2)) + 255) / 256 * 256 +
-                split_kv_bytes(B, N, H, D, split_kv_nsplit(B, N, H, D, w1, w2));
+                split_kv_bytes(B, N, H, D, split_kv_nsplit(B, N, H, D, w1, w2)) + guard_bytes(B, N, H);
         return 0;
     });
     return bytes;

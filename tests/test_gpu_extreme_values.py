@@ -33,6 +33,12 @@ def _inputs(dtype, D, what):
         x[1][:, 80:90] = torch.finfo(dtype).min
     elif what == "small values":
         x[3] = x[3] * 1e-36
+    elif what == "NaN gradient":
+        x[5][:, 90] = nan
+    elif what == "small gradient":
+        x[5] = x[5] * 1e-36
+    elif what == "product above the range":
+        x[4][:, 90], x[5][:, 95] = 1e30, 1e30
     elif what == "small keys":
         x[1] = x[1] * 1e-36
     return x
@@ -62,3 +68,29 @@ def test_forward(dtype, D, w2, what):
     got, want = (sa.simplicial_forward(*x[:5], 40, w2, flags=flags) for flags in (AUTO, GENERIC))
     _same(got[0], want[0], BAR[dtype], "out")
     _same(got[1], want[1], 1e-6, "lse")
+
+
+BACKWARD = FORWARD + ["NaN gradient", "small gradient"]
+
+
+@pytest.mark.parametrize("dtype,D,w2,what", _cases(BACKWARD) + [(torch.float32, 64, 20, "product above the range")])
+def test_backward(dtype, D, w2, what):
+    import simplical_attn_amd as sa
+    x = _inputs(dtype, D, what)
+    out, lse = sa.simplicial_forward(*x[:5], 40, w2, flags=GENERIC)
+    got, want = (sa.simplicial_backward(*x[:5], out, lse, x[5], 40, w2, flags=flags) for flags in (AUTO, GENERIC))
+    for name, a, b in zip(("dq", "dk1", "dk2", "dv1", "dv2"), got, want):
+        _same(a, b, BAR[dtype], name)
+
+
+def test_backward_of_a_subset_of_the_gradients():
+    """The repaired launch writes what was asked for and nothing else."""
+    import simplical_attn_amd as sa
+    x = _inputs(torch.float32, 64, "NaN value")
+    out, lse = sa.simplicial_forward(*x[:5], 40, 20)
+    full = sa.simplicial_backward(*x[:5], out, lse, x[5], 40, 20)
+    for needs in ((True, False, False, False, True), (False, True, False, False, False)):
+        part = sa.simplicial_backward(*x[:5], out, lse, x[5], 40, 20, needs=needs)
+        for need, a, b in zip(needs, part, full):
+            assert (a is None) == (not need)
+            assert a is None or torch.equal(a.nan_to_num(), b.nan_to_num())
