@@ -117,9 +117,9 @@ struct Mem16 {
     }
 };
 
-// fp32 tensors of the padded head dims (and 96): finer sums, see Chain and accumulate
-template <class T, bool PAD>
-constexpr bool fine() { return T::DTYPE == SA2_F32 && PAD; }
+// MODE of a kernel: tensors as wide as the kernel, or narrower (PAD below); PADDED_FINE: with finer sums (Chain and
+// accumulate) for the fp32 head dims that ran on the FMA kernels before (16, which was padded onto the fp32 MFMA, did not)
+constexpr int EXACT = 0, PADDED = 1, PADDED_FINE = 2;
 
 // Four columns of a row.  PAD: the tensors have width <= D columns; the kernel's columns from there on read as zeros
 // and are not written (rows are multiples of four elements, so four columns are inside or outside together).
@@ -359,12 +359,12 @@ __device__ __forceinline__ void product_planes(const typename T::T* xrow, const 
 
 // ================================================================== forward =====
 // SPLIT: one of nsplit shares of the rounds, unnormalised sums to the workspace (see launch_fwd_merge).
-template <class T, int D, bool PAD, bool SPLIT>
+template <class T, int D, int MODE, bool SPLIT>
 __global__ __launch_bounds__((SplitCfg<T, D>::FW * 64)) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 2 : 1, D <= 64 ? 2 : 1)))
 void split_fwd_kernel(Problem p, int nqb, int total) {
     using C = SplitCfg<T, D>;
     constexpr int W = C::FW, NT = W * 64;
-    constexpr bool FINE = fine<T, PAD>();
+    constexpr bool PAD = MODE != EXACT, FINE = MODE == PADDED_FINE;
     typedef typename T::T EL;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_f[];
     uint16_t* tiles = (uint16_t*)smem_f;                                             // two stages
@@ -731,11 +731,11 @@ __device__ __forceinline__ void split16(const float (&x)[16], bf16x8 (&o)[2][N])
 
 // The K' window in nseg segments of segw deltas, one workgroup per (segment, K' block): segment-major launch order.
 // nseg > 1: fp32 partial dK', dV' to `kpart` ([dV' | dK'][nseg][B*H][N][D]).
-template <class T, int D, bool PAD>
+template <class T, int D, int MODE>
 __global__ __launch_bounds__(XT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void split_kp_kernel(Problem p, int nkb, int per_seg, float* __restrict__ dq_part, int nseg, int segw, float* __restrict__ kpart) {
     using C = SplitCfg<T, D>;
-    constexpr bool FINE = fine<T, PAD>();
+    constexpr bool PAD = MODE != EXACT, FINE = MODE == PADDED_FINE;
     typedef typename T::T EL;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_f[];
     uint16_t* tiles = (uint16_t*)smem_f;
@@ -963,12 +963,12 @@ void split_kp_kernel(Problem p, int nkb, int per_seg, float* __restrict__ dq_par
 // =================================================== backward, K side: dK, dV =====
 // nsplit > 1 (grids smaller than the chip): the workgroup takes the sp-th share of the key block's stream
 // of units and writes fp32 partial sums to `part` ([dK | dV][nsplit][B*H][N][D]) for bwd_sum_kernel.
-template <class T, int D, bool SPLIT, bool PAD>
+template <class T, int D, bool SPLIT, int MODE>
 __global__ __launch_bounds__(XT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void split_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __restrict__ part) {
     const int nsplit = SPLIT ? nsplit_arg : 1;
     using C = SplitCfg<T, D>;
-    constexpr bool FINE = fine<T, PAD>();
+    constexpr bool PAD = MODE != EXACT, FINE = MODE == PADDED_FINE;
     typedef typename T::T EL;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_f[];
     uint16_t* tiles = (uint16_t*)smem_f;
@@ -1196,12 +1196,13 @@ void split_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __res
 }
 
 // Shares a key block's query blocks are split into when the K-side grid is smaller than the chip
-int split_kv_nsplit(int B, int N, int H, int D, int w1, int w2) {
+int split_kv_nsplit(int B, int N, int H, int D, int w1, int w2, size_t room) {
     const int64_t bh = (int64_t)B * H, base = bh * ((N + XJ - 1) / XJ);
     const int blocks = (XJ + (w1 < N ? w1 : N) + BQ - 1) / BQ + 1;
     const int64_t units = (int64_t)blocks * ((w2 < N - 1 ? w2 : N - 1) + 1);     // of a key block's stream, at most
     int ns = 1;                                                                  // shares of at least 8 units
-    while (ns < 16 && base * ns * 2 <= 512 && (int64_t)ns * 2 * 8 <= units && (int64_t)2 * ns * 2 * bh * N * D * 4 <= ((int64_t)32 << 20))
+    while (ns < 16 && base * ns * 2 <= 512 && (int64_t)ns * 2 * 8 <= units && (int64_t)2 * ns * 2 * bh * N * D * 4 <= ((int64_t)32 << 20) &&
+           (size_t)2 * ns * 2 * bh * N * D * 4 <= room)
         ns *= 2;
     return ns;
 }
@@ -1214,15 +1215,15 @@ size_t split_kp_bytes(int B, int N, int H, int D, const KpPlan& pl) {
 }
 // Deltas per segment: what the dQ accumulator in LDS holds, or fewer where the grid asks for it
 template <class T, int D>
-KpPlan split_kp_plan(int B, int N, int H, int w1, int w2) {
+KpPlan split_kp_plan(int B, int N, int H, int w1, int w2, size_t room) {
     using C = SplitCfg<T, D>;
     int most = NPAIR;
     while (most < w2 + 1 && C::kp_fits(most + NPAIR - 1)) most += NPAIR;
-    return plan_segments(B, N, H, w1, w2, NPAIR, most, [](int) { return false; }, [&](const KpPlan& pl) { return split_kp_bytes(B, N, H, D, pl); });
+    return plan_segments(B, N, H, w1, w2, NPAIR, most, room, [](int) { return false; }, [&](const KpPlan& pl) { return split_kp_bytes(B, N, H, D, pl); });
 }
 
 // ------------------------------------------------------------------ launchers ----
-template <class T, int D, bool PAD>
+template <class T, int D, int MODE>
 int launch_split_fwd(const Problem& p, hipStream_t st) {
     using C = SplitCfg<T, D>;
     const int nqb = (p.N + BQ - 1) / BQ;
@@ -1233,20 +1234,21 @@ int launch_split_fwd(const Problem& p, hipStream_t st) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(C::FW * 64), C::FWD_LDS, st, p, nqb, (int)grid);
         return hipGetLastError() == hipSuccess;
     };
-    if (p.nsplit <= 1) return go(split_fwd_kernel<T, D, PAD, false>, total) ? SA2_OK : SA2_ERR_LAUNCH_FAILED;
+    if (p.nsplit <= 1) return go(split_fwd_kernel<T, D, MODE, false>, total) ? SA2_OK : SA2_ERR_LAUNCH_FAILED;
     const int64_t grid = total * p.nsplit;
     if (grid > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
-    if (!go(split_fwd_kernel<T, D, PAD, true>, grid)) return SA2_ERR_LAUNCH_FAILED;
+    if (!go(split_fwd_kernel<T, D, MODE, true>, grid)) return SA2_ERR_LAUNCH_FAILED;
     return launch_fwd_merge(p, D, T::DTYPE, st);
 }
 
-template <class T, int D, bool PAD>
+template <class T, int D, int MODE>
 int launch_split_bwd(const Problem& p, hipStream_t st) {
     using C = SplitCfg<T, D>;
     BwdSums sums = {};
-    const KpPlan pl = split_kp_plan<T, D>(p.B, p.N, p.H, p.w1, p.w2);
+    const size_t room = room_left(p.room, guard_bytes(p.B, p.N, p.H));
+    const KpPlan pl = split_kp_plan<T, D>(p.B, p.N, p.H, p.w1, p.w2, room);
     const size_t kp_bytes = (split_kp_bytes(p.B, p.N, p.H, D, pl) + 255) / 256 * 256;
-    const int nsplit = split_kv_nsplit(p.B, p.N, p.H, D, p.w1, p.w2);
+    const int nsplit = split_kv_nsplit(p.B, p.N, p.H, D, p.w1, p.w2, room_left(room, kp_bytes));
     const size_t part_bytes = kp_bytes + split_kv_bytes(p.B, p.N, p.H, D, nsplit);
     if (p.scratch_bytes < part_bytes + guard_bytes(p.B, p.N, p.H)) return SA2_ERR_WORKSPACE_TOO_SMALL;
     int* guard = (int*)((char*)p.scratch + part_bytes);
@@ -1264,8 +1266,8 @@ int launch_split_bwd(const Problem& p, hipStream_t st) {
         if (total > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
         float* part = (float*)p.scratch;
         float* kpart = (float*)((char*)p.scratch + split_dq_part_bytes(p.B, p.N, p.H, D, pl));
-        if (!allow_full_lds((const void*)split_kp_kernel<T, D, PAD>)) return SA2_ERR_LAUNCH_FAILED;
-        hipLaunchKernelGGL((split_kp_kernel<T, D, PAD>), dim3((unsigned)total), dim3(XT), C::kp_lds(pl.segw - 1), st, p, nkb, (int)per_seg, part,
+        if (!allow_full_lds((const void*)split_kp_kernel<T, D, MODE>)) return SA2_ERR_LAUNCH_FAILED;
+        hipLaunchKernelGGL((split_kp_kernel<T, D, MODE>), dim3((unsigned)total), dim3(XT), C::kp_lds(pl.segw - 1), st, p, nkb, (int)per_seg, part,
                            pl.nseg, pl.segw, kpart);
         if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
         sums.dq = p.dq.p ? part : nullptr;
@@ -1284,7 +1286,7 @@ int launch_split_bwd(const Problem& p, hipStream_t st) {
             hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(XT), C::KV_LDS, st, p, njb, (int)total, nsplit, part);
             return hipGetLastError() == hipSuccess;
         };
-        if (!(nsplit > 1 ? go(split_kv_kernel<T, D, true, PAD>) : go(split_kv_kernel<T, D, false, PAD>))) return SA2_ERR_LAUNCH_FAILED;
+        if (!(nsplit > 1 ? go(split_kv_kernel<T, D, true, MODE>) : go(split_kv_kernel<T, D, false, MODE>))) return SA2_ERR_LAUNCH_FAILED;
         sums.kv = part;
         sums.kv_n = nsplit;
     }
@@ -1307,25 +1309,31 @@ bool rows16(const Tensor& t, int B, int N, int H) {
     return !((B > 1 && (t.sb & M)) || (N > 1 && (t.sn & M)) || (H > 1 && (t.sh & M)));
 }
 
-// Kernel width of a head_dim, and the call f(memory type, width, PAD) for it.  16-bit tensors come here only with head
+// Kernel width of a head_dim, and the call f(memory type, width, MODE) for it.  16-bit tensors come here only with head
 // dims that the 16-bit kernels do not have, always padded or 96 columns wide.
 int split_width(int D) { return D <= 32 ? 32 : D <= 64 ? 64 : D <= 96 ? 96 : 128; }
 template <class F>
 int for_split_width(int D, int dtype, F&& f) {
-    auto of_type = [&](auto m) {
-        constexpr bool F32 = decltype(m)::DTYPE == SA2_F32;
-        const bool exact = F32 && D == split_width(D);
-        auto of_pad = [&](auto width) {
-            if constexpr (F32) {
-                if (exact) return f(m, width, std::false_type{});
+    auto of_width = [&](auto m, auto width) {
+        constexpr int W = decltype(width)::value;
+        if constexpr (decltype(m)::DTYPE == SA2_F32) {
+            if constexpr (W != 96) {
+                if (D == W) return f(m, width, std::integral_constant<int, EXACT>{});
             }
-            return f(m, width, std::true_type{});
-        };
+            if constexpr (W == 32) {
+                if (D == 16) return f(m, width, std::integral_constant<int, PADDED>{});
+            }
+            return f(m, width, std::integral_constant<int, PADDED_FINE>{});
+        } else {
+            return f(m, width, std::integral_constant<int, PADDED>{});
+        }
+    };
+    auto of_type = [&](auto m) {
         switch (split_width(D)) {
-            case 32: return of_pad(std::integral_constant<int, 32>{});
-            case 64: return of_pad(std::integral_constant<int, 64>{});
-            case 96: return f(m, std::integral_constant<int, 96>{}, std::true_type{});
-            default: return of_pad(std::integral_constant<int, 128>{});
+            case 32: return of_width(m, std::integral_constant<int, 32>{});
+            case 64: return of_width(m, std::integral_constant<int, 64>{});
+            case 96: return of_width(m, std::integral_constant<int, 96>{});
+            default: return of_width(m, std::integral_constant<int, 128>{});
         }
     };
     return dtype == SA2_F32 ? of_type(MemF32{}) : dtype == SA2_F16 ? of_type(Mem16<ElemF16>{}) : of_type(Mem16<ElemBF16>{});
@@ -1357,12 +1365,14 @@ bool f32_mfma_layout_ok(const Problem& p, int dtype, bool backward) {
     return true;
 }
 
-size_t f32_mfma_bwd_scratch_bytes(int B, int N, int H, int head_dim, int w1, int w2, int dtype) {
+size_t f32_mfma_bwd_scratch_bytes(int B, int N, int H, int head_dim, int w1, int w2, int dtype, size_t room) {
+    const size_t guard = guard_bytes(B, N, H);
     size_t bytes = 0;
+    room = room_left(room, guard);
     for_split_width(head_dim, dtype, [&](auto m, auto width, auto) {
         constexpr int D = decltype(width)::value;
-        bytes = (split_kp_bytes(B, N, H, D, split_kp_plan<decltype(m), D>(B, N, H, w1, w2)) + 255) / 256 * 256 +
-                split_kv_bytes(B, N, H, D, split_kv_nsplit(B, N, H, D, w1, w2)) + guard_bytes(B, N, H);
+        const size_t kp = (split_kp_bytes(B, N, H, D, split_kp_plan<decltype(m), D>(B, N, H, w1, w2, room)) + 255) / 256 * 256;
+        bytes = kp + split_kv_bytes(B, N, H, D, split_kv_nsplit(B, N, H, D, w1, w2, room_left(room, kp))) + guard;
         return 0;
     });
     return bytes;
@@ -1375,14 +1385,14 @@ int f32_mfma_fwd_nsplit(int B, int N, int H, int head_dim, int w1, int w2) {
 size_t f32_mfma_fwd_part_bytes(int B, int N, int H, int head_dim, int nsplit) { return fwd_part_bytes(B, N, H, split_width(head_dim), nsplit); }
 
 int launch_f32_mfma_fwd(const Problem& p, int dtype, hipStream_t st) {
-    return for_split_width(p.D, dtype, [&](auto m, auto width, auto pad) {
-        return launch_split_fwd<decltype(m), decltype(width)::value, decltype(pad)::value>(p, st);
+    return for_split_width(p.D, dtype, [&](auto m, auto width, auto mode) {
+        return launch_split_fwd<decltype(m), decltype(width)::value, decltype(mode)::value>(p, st);
     });
 }
 
 int launch_f32_mfma_bwd(const Problem& p, int dtype, hipStream_t st) {
-    return for_split_width(p.D, dtype, [&](auto m, auto width, auto pad) {
-        return launch_split_bwd<decltype(m), decltype(width)::value, decltype(pad)::value>(p, st);
+    return for_split_width(p.D, dtype, [&](auto m, auto width, auto mode) {
+        return launch_split_bwd<decltype(m), decltype(width)::value, decltype(mode)::value>(p, st);
     });
 }
 

@@ -55,10 +55,11 @@ def test_config1_fp32_gradients():
 
 @pytest.mark.parametrize("shape,w,times", [((1, 128, 2, 64), (32, 16), 1.8), ((1, 260, 2, 32), (64, 16), 1.8),
                                            ((1, 200, 1, 128), (128, 8), 1.8), ((1, 300, 2, 96), (128, 24), 1.2),
-                                           ((2, 260, 1, 48), (64, 64), 1.2), ((1, 300, 2, 16), (128, 24), 1.2)])
+                                           ((2, 260, 1, 48), (64, 64), 1.2), ((1, 300, 2, 24), (128, 24), 1.2),
+                                           ((1, 300, 2, 16), (128, 24), 1.8)])
 def test_errors_in_units_of_the_fma_kernels(shape, w, times):
     """Root mean square errors against fp64, as multiples of those the fp32 FMA kernels make on the same inputs.  Head
-    dims with a kernel of their own ran on v_mfma_f32_32x32x2_f32 before, with up to 1.9 times the FMA kernels' errors
+    dims with a kernel of their own, and 16, ran on v_mfma_f32_32x32x2_f32 before, with up to 1.9 times the FMA kernels' errors
     (1.6 at most here, measured); the others ran on the FMA kernels and may not be worse (1.0, and what varies from
     seed to seed)."""
     def errors(flags):
