@@ -41,7 +41,7 @@ typedef enum sa2_status {
     SA2_ERR_LAUNCH_FAILED = -7,  /* hipGetLastError() after a launch */
     SA2_ERR_UNSUPPORTED = -8,    /* a forced kernel path does not support the shape/dtype */
     SA2_ERR_TOO_LARGE = -9,      /* an index would overflow the kernels' 32-bit grid */
-    SA2_ERR_STATIC_WORKSPACE = -10 /* sa2_backward_static_workspace: the problem needs more than
+    SA2_ERR_STATIC_WORKSPACE = -10 /* sa2_backward_static_workspace: the problem does not fit
                                       SA2_STATIC_WORKSPACE_BYTES, or the array's address is unavailable */
 } sa2_status;
 
@@ -138,10 +138,14 @@ int sa2_backward(const void* q, const void* k1, const void* k2, const void* v1, 
 /*
  * sa2_backward for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart
- * in the reference.  Same arguments, kernels and results as sa2_backward, minus the
- * workspace: that is a file-scope device array of SA2_STATIC_WORKSPACE_BYTES inside the
- * library, one copy per GPU, held until the process ends.  The call itself allocates and
- * frees nothing.  A problem with sa2_bwd_workspace_bytes(...) > SA2_STATIC_WORKSPACE_BYTES
+ * in the reference.  Same arguments as sa2_backward, minus the workspace: that is a
+ * file-scope device array of SA2_STATIC_WORKSPACE_BYTES inside the library, one copy per
+ * GPU, held until the process ends.  The call itself allocates and frees nothing.  Where
+ * sa2_bwd_workspace_bytes(...) <= SA2_STATIC_WORKSPACE_BYTES it runs sa2_backward's kernels
+ * with the same results, bit for bit.  Otherwise it runs them with fewer partial sums (added
+ * in another order), and where even the fewest do not fit and the head_dim has no kernels of
+ * its own (see sa2_uses_mfma), or the fp32 K' window would fit in one piece, the fp32-FMA
+ * kernels.  A problem that fits in none of these ways
  * returns SA2_ERR_STATIC_WORKSPACE and launches nothing.  All calls on one GPU share the
  * array (the kernels overwrite what they read from it, so nothing needs clearing between
  * calls): calls that overlap on one GPU - different streams, or host threads - race;

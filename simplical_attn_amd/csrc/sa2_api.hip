@@ -126,22 +126,93 @@ KernelPath pick_path(const Problem& p, int dtype, unsigned flags, bool backward,
 
 // Bytes one call needs, for inclusive reaches w1 and w2.  Not monotone in them (the plans of the backward kernels cut
 // the work where the grid asks for it): the exported function covers both window conventions of the same numbers.
-size_t bwd_need(int B, int N, int H, int D, int w1, int w2, int dtype, unsigned flags) {
+size_t bwd_need(int B, int N, int H, int D, int w1, int w2, int dtype, unsigned flags, size_t room) {
     if (check_dims(B, N, H, D, w1, w2, dtype, 1) != SA2_OK) return 0;
     size_t scratch = generic_bwd_scratch_bytes(B, N, H, D, w1, w2);
     if (!(flags & SA2_FLAG_FORCE_GENERIC) && mfma_bwd_supported(B, N, H, D, reach(w1, 1, N), reach(w2, 1, N), dtype)) {
-        const size_t m = mfma_bwd_scratch_bytes(B, N, H, D, reach(w1, 1, N), reach(w2, 1, N));
+        const size_t m = mfma_bwd_scratch_bytes(B, N, H, D, reach(w1, 1, N), reach(w2, 1, N), room);
         if (m > scratch) scratch = m;
     }
     if (!(flags & SA2_FLAG_FORCE_GENERIC) && wide_bwd_supported(D, reach(w2, 1, N), dtype)) {
-        const size_t m = wide_bwd_scratch_bytes(B, N, H, D, reach(w1, 1, N), reach(w2, 1, N));
+        const size_t m = wide_bwd_scratch_bytes(B, N, H, D, reach(w1, 1, N), reach(w2, 1, N), room);
         if (m > scratch) scratch = m;
     }
     if (!(flags & SA2_FLAG_FORCE_GENERIC) && f32_mfma_bwd_supported(D, reach(w2, 1, N), dtype)) {
-        const size_t m = f32_mfma_bwd_scratch_bytes(B, N, H, D, reach(w1, 1, N), reach(w2, 1, N), dtype);
+        const size_t m = f32_mfma_bwd_scratch_bytes(B, N, H, D, reach(w1, 1, N), reach(w2, 1, N), dtype, room);
         if (m > scratch) scratch = m;
     }
     return dsum_bytes(B, N, H) + align_up(scratch, 256) + 256;
+}
+
+// How sa2_backward_static_workspace takes a problem into its array (inclusive reaches w1 and w2): as sa2_backward does
+// where that fits, else with plans that cut less, else - for head dims without kernels of their own, and for fp32 K'
+// windows that fit in one piece but not as the segments the kernels' LDS asks for - on the fp32 FMA kernels, which need
+// the row term only.  false: refused.
+bool static_plan(int B, int N, int H, int D, int w1, int w2, int dtype, unsigned* flags, size_t* room) {
+    const size_t all = SA2_STATIC_WORKSPACE_BYTES;
+    auto fits = [&] {
+        const size_t need = bwd_need(B, N, H, D, w1, w2, dtype, *flags, *room);
+        return need != 0 && need <= all;
+    };
+    *room = ROOM_ANY;
+    if (fits()) return true;
+    *room = room_left(all, dsum_bytes(B, N, H) + 512);
+    if (fits()) return true;
+    const double whole = ((double)B * H * ((N + 31) / 32) * (32 + reach(w2, 1, N)) * D + (double)B * H * N) * sizeof(float);
+    if ((*flags & SA2_FLAG_FORCE_MFMA) || (own_width(D, dtype) && (dtype != SA2_F32 || (D != 96 && whole > (double)all)))) return false;
+    *flags |= SA2_FLAG_FORCE_GENERIC;
+    return fits();
+}
+
+int run_backward(size_t room, const void* q, const void* k1, const void* k2, const void* v1, const void* v2,
+                 const void* out, const void* dout, const float* lse,
+                 void* dq, void* dk1, void* dk2, void* dv1, void* dv2,
+                 void* workspace, size_t workspace_bytes,
+                 int B, int N, int H, int D, const int64_t* strides,
+                 int w1, int w2, float scale, float k2_bias, float v2_bias,
+                 int dtype, int window_inclusive, unsigned flags, void* hip_stream) {
+    if (!q || !k1 || !k2 || !v1 || !v2 || !out || !dout || !lse || !strides || !workspace) return SA2_ERR_NULL_POINTER;
+    int rc = check_dims(B, N, H, D, w1, w2, dtype, window_inclusive);
+    if (rc != SA2_OK) return rc;
+    if (!strides_ok(strides, SA2_BWD_TENSORS, B, N, H)) return SA2_ERR_BAD_STRIDE;
+    // The half-open convention with window w has the reach of the closed one with w-1.
+    const size_t need = bwd_need(B, N, H, D, window_inclusive ? w1 : w1 - 1,
+                                                window_inclusive ? w2 : w2 - 1, dtype, flags, room);
+    if (workspace_bytes < need || ((uintptr_t)workspace & 255u)) return SA2_ERR_WORKSPACE_TOO_SMALL;
+    if (!dq && !dk1 && !dk2 && !dv1 && !dv2) return SA2_OK;
+
+    Problem p;
+    memset(&p, 0, sizeof(p));
+    p.B = B; p.N = N; p.H = H; p.D = D;
+    p.w1 = reach(w1, window_inclusive, N);
+    p.w2 = reach(w2, window_inclusive, N);
+    p.scale = scale; p.k2_bias = k2_bias; p.v2_bias = v2_bias;
+    p.q = make_tensor(q, strides, SA2_T_Q);
+    p.k1 = make_tensor(k1, strides, SA2_T_K1);
+    p.k2 = make_tensor(k2, strides, SA2_T_K2);
+    p.v1 = make_tensor(v1, strides, SA2_T_V1);
+    p.v2 = make_tensor(v2, strides, SA2_T_V2);
+    p.out = make_tensor(out, strides, SA2_T_OUT);
+    p.dout = make_tensor(dout, strides, SA2_T_DOUT);
+    p.dq = make_tensor(dq, strides, SA2_T_DQ);
+    p.dk1 = make_tensor(dk1, strides, SA2_T_DK1);
+    p.dk2 = make_tensor(dk2, strides, SA2_T_DK2);
+    p.dv1 = make_tensor(dv1, strides, SA2_T_DV1);
+    p.dv2 = make_tensor(dv2, strides, SA2_T_DV2);
+    p.lse = const_cast<float*>(lse);
+    p.dsum = (float*)workspace;
+    p.scratch = (char*)workspace + dsum_bytes(B, N, H);
+    p.scratch_bytes = workspace_bytes - dsum_bytes(B, N, H);
+
+    p.room = room;
+    p.force_prepass = (flags & SA2_FLAG_FORCE_MFMA) ? 1 : 0;
+
+    hipStream_t st = (hipStream_t)hip_stream;
+    const KernelPath path = pick_path(p, dtype, flags, true, &rc);
+    if (rc != SA2_OK) return rc;
+    return path == PATH_MFMA16 ? launch_mfma_bwd(p, dtype, st)
+           : path == PATH_WIDE16 ? launch_wide_bwd(p, dtype, st)
+           : path == PATH_MFMA32 ? launch_f32_mfma_bwd(p, dtype, st) : launch_generic_bwd(p, dtype, st);
 }
 
 }  // namespace
@@ -245,8 +316,8 @@ int sa2_forward_ws(const void* q, const void* k1, const void* k2, const void* v1
 }
 
 size_t sa2_bwd_workspace_bytes(int B, int N, int H, int D, int w1, int w2, int dtype, unsigned flags) {
-    const size_t closed = bwd_need(B, N, H, D, w1, w2, dtype, flags);
-    const size_t open = closed && w1 > 0 && w2 > 0 ? bwd_need(B, N, H, D, w1 - 1, w2 - 1, dtype, flags) : 0;
+    const size_t closed = bwd_need(B, N, H, D, w1, w2, dtype, flags, ROOM_ANY);
+    const size_t open = closed && w1 > 0 && w2 > 0 ? bwd_need(B, N, H, D, w1 - 1, w2 - 1, dtype, flags, ROOM_ANY) : 0;
     return closed > open ? closed : open;
 }
 
@@ -257,47 +328,8 @@ int sa2_backward(const void* q, const void* k1, const void* k2, const void* v1, 
                  int B, int N, int H, int D, const int64_t* strides,
                  int w1, int w2, float scale, float k2_bias, float v2_bias,
                  int dtype, int window_inclusive, unsigned flags, void* hip_stream) {
-    if (!q || !k1 || !k2 || !v1 || !v2 || !out || !dout || !lse || !strides || !workspace) return SA2_ERR_NULL_POINTER;
-    int rc = check_dims(B, N, H, D, w1, w2, dtype, window_inclusive);
-    if (rc != SA2_OK) return rc;
-    if (!strides_ok(strides, SA2_BWD_TENSORS, B, N, H)) return SA2_ERR_BAD_STRIDE;
-    // The half-open convention with window w has the reach of the closed one with w-1.
-    const size_t need = bwd_need(B, N, H, D, window_inclusive ? w1 : w1 - 1,
-                                                window_inclusive ? w2 : w2 - 1, dtype, flags);
-    if (workspace_bytes < need || ((uintptr_t)workspace & 255u)) return SA2_ERR_WORKSPACE_TOO_SMALL;
-    if (!dq && !dk1 && !dk2 && !dv1 && !dv2) return SA2_OK;
-
-    Problem p;
-    memset(&p, 0, sizeof(p));
-    p.B = B; p.N = N; p.H = H; p.D = D;
-    p.w1 = reach(w1, window_inclusive, N);
-    p.w2 = reach(w2, window_inclusive, N);
-    p.scale = scale; p.k2_bias = k2_bias; p.v2_bias = v2_bias;
-    p.q = make_tensor(q, strides, SA2_T_Q);
-    p.k1 = make_tensor(k1, strides, SA2_T_K1);
-    p.k2 = make_tensor(k2, strides, SA2_T_K2);
-    p.v1 = make_tensor(v1, strides, SA2_T_V1);
-    p.v2 = make_tensor(v2, strides, SA2_T_V2);
-    p.out = make_tensor(out, strides, SA2_T_OUT);
-    p.dout = make_tensor(dout, strides, SA2_T_DOUT);
-    p.dq = make_tensor(dq, strides, SA2_T_DQ);
-    p.dk1 = make_tensor(dk1, strides, SA2_T_DK1);
-    p.dk2 = make_tensor(dk2, strides, SA2_T_DK2);
-    p.dv1 = make_tensor(dv1, strides, SA2_T_DV1);
-    p.dv2 = make_tensor(dv2, strides, SA2_T_DV2);
-    p.lse = const_cast<float*>(lse);
-    p.dsum = (float*)workspace;
-    p.scratch = (char*)workspace + dsum_bytes(B, N, H);
-    p.scratch_bytes = workspace_bytes - dsum_bytes(B, N, H);
-
-    p.force_prepass = (flags & SA2_FLAG_FORCE_MFMA) ? 1 : 0;
-
-    hipStream_t st = (hipStream_t)hip_stream;
-    const KernelPath path = pick_path(p, dtype, flags, true, &rc);
-    if (rc != SA2_OK) return rc;
-    return path == PATH_MFMA16 ? launch_mfma_bwd(p, dtype, st)
-           : path == PATH_WIDE16 ? launch_wide_bwd(p, dtype, st)
-           : path == PATH_MFMA32 ? launch_f32_mfma_bwd(p, dtype, st) : launch_generic_bwd(p, dtype, st);
+    return run_backward(ROOM_ANY, q, k1, k2, v1, v2, out, dout, lse, dq, dk1, dk2, dv1, dv2, workspace, workspace_bytes,
+                        B, N, H, D, strides, w1, w2, scale, k2_bias, v2_bias, dtype, window_inclusive, flags, hip_stream);
 }
 
 int sa2_backward_static_workspace(const void* q, const void* k1, const void* k2, const void* v1, const void* v2,
@@ -308,12 +340,12 @@ int sa2_backward_static_workspace(const void* q, const void* k1, const void* k2,
                                   int dtype, int window_inclusive, unsigned flags, void* hip_stream) {
     int rc = check_dims(B, N, H, D, w1, w2, dtype, window_inclusive);
     if (rc != SA2_OK) return rc;
-    const size_t need = bwd_need(B, N, H, D, window_inclusive ? w1 : w1 - 1,
-                                                window_inclusive ? w2 : w2 - 1, dtype, flags);
-    if (need == 0 || need > (size_t)SA2_STATIC_WORKSPACE_BYTES) return SA2_ERR_STATIC_WORKSPACE;
+    size_t room;
+    if (!static_plan(B, N, H, D, window_inclusive ? w1 : w1 - 1, window_inclusive ? w2 : w2 - 1, dtype, &flags, &room))
+        return SA2_ERR_STATIC_WORKSPACE;
     void* ws = static_workspace();
     if (!ws) return SA2_ERR_STATIC_WORKSPACE;
-    return sa2_backward(q, k1, k2, v1, v2, out, dout, lse, dq, dk1, dk2, dv1, dv2, ws, SA2_STATIC_WORKSPACE_BYTES,
+    return run_backward(room, q, k1, k2, v1, v2, out, dout, lse, dq, dk1, dk2, dv1, dv2, ws, SA2_STATIC_WORKSPACE_BYTES,
                         B, N, H, D, strides, w1, w2, scale, k2_bias, v2_bias, dtype, window_inclusive, flags, hip_stream);
 }
 

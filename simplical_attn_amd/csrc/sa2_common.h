@@ -27,6 +27,7 @@ struct Problem {
     float* dsum;                     // [B,H,N]  sum_d dout*out
     void* scratch;                   // remaining workspace (path specific)
     size_t scratch_bytes;
+    size_t room;                     // backward: bytes the plans may spend on partial sums (ROOM_ANY: what they think best)
     int nsplit;                      // forward: shares of the rounds (partial outputs in `scratch` when more than one)
     int force_prepass;               // take the pre-pass kernels whenever the window allows, whatever the size
 };
@@ -99,6 +100,10 @@ inline double grid_time(int64_t workgroups, double longest, double mean) {
 inline double window_fill(int w, int N) { return w < N ? 1.0 - 0.5 * w / N : 0.5 * N / w; }
 constexpr double PART_BYTES_PER_STEP = 2.5e6, SUM_LAUNCH_STEPS = 8;
 
+// All partial sums of a call that has to make do with `room` bytes: the plans cut less, down to the uncut launch
+constexpr size_t ROOM_ANY = ~(size_t)0;
+inline size_t room_left(size_t room, size_t taken) { return room == ROOM_ANY ? room : room > taken ? room - taken : 0; }
+
 // The K' window in nseg segments of segw deltas, one workgroup per (K' block, segment)
 struct KpPlan {
     int segw, nseg;
@@ -111,13 +116,14 @@ struct KpPlan {
 // B3 H21 N282 D128 w 176/48 488 -> 303 (three), B1 H8 N4096 D128 w 128/64 862 -> 655 (two: the rows then fit LDS),
 // B2 H4 N256 D64 w 32/32 43 -> 29 (three).
 template <class Raw, class Bytes>
-KpPlan plan_segments(int B, int N, int H, int w1, int w2, int upr, int most, Raw&& raw, Bytes&& bytes) {
+KpPlan plan_segments(int B, int N, int H, int w1, int w2, int upr, int most, size_t room, Raw&& raw, Bytes&& bytes) {
     constexpr int ROWS = 32, MOST_SEGMENTS = 16;
     const int64_t base = (int64_t)B * H * ((N + ROWS - 1) / ROWS);
     const int rounds = (w2 + upr) / upr;
     const double tiles = ((w1 < N ? w1 : N) + ROWS + upr) / (double)ROWS + 1, fill = window_fill(w1, N) * window_fill(w2, N);
     KpPlan best = most > w2 ? KpPlan{w2 + 1, 1} : KpPlan{most, (w2 + most) / most};
-    const double first_bytes = (double)bytes(best), cap = 3 * first_bytes > 33554432.0 ? 3 * first_bytes : 33554432.0;
+    const double first_bytes = (double)bytes(best), likes = 3 * first_bytes > 33554432.0 ? 3 * first_bytes : 33554432.0;
+    const double cap = likes < (double)room ? likes : (double)room;
     double least = 0;
     for (int nseg = best.nseg, last = 0; nseg <= MOST_SEGMENTS || least == 0; ++nseg) {
         const int per = (rounds + nseg - 1) / nseg;                                  // rounds per segment
@@ -182,13 +188,13 @@ int launch_mfma_fwd(const Problem& p, int dtype, hipStream_t st);
 int mfma_fwd_nsplit(int B, int N, int H, int D, int w1, int w2, bool force_prepass);
 size_t mfma_fwd_part_bytes(int B, int N, int H, int D, int nsplit);
 int launch_mfma_bwd(const Problem& p, int dtype, hipStream_t st);
-size_t mfma_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2);
+size_t mfma_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2, size_t room);
 // fp32 arithmetic on the fp32 MFMA: fp32 tensors of any head_dim up to 128 that is a multiple of 4, and 16-bit tensors
 // of the head dims the 16-bit kernels do not have (multiples of 8 up to 120); rows 16-byte aligned
 bool f32_mfma_supported(int D, int dtype);
 bool f32_mfma_bwd_supported(int D, int w2, int dtype);
 bool f32_mfma_layout_ok(const Problem& p, int dtype, bool backward);
-size_t f32_mfma_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2, int dtype);
+size_t f32_mfma_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2, int dtype, size_t room);
 int launch_f32_mfma_fwd(const Problem& p, int dtype, hipStream_t st);
 int f32_mfma_fwd_nsplit(int B, int N, int H, int D, int w1, int w2);
 size_t f32_mfma_fwd_part_bytes(int B, int N, int H, int D, int nsplit);
@@ -196,7 +202,7 @@ int launch_f32_mfma_bwd(const Problem& p, int dtype, hipStream_t st);
 // 16-bit tensors with head_dim 256 on the 16-bit MFMA (rows 16-byte aligned)
 bool wide_supported(int D, int dtype);
 bool wide_bwd_supported(int D, int w2, int dtype);
-size_t wide_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2);
+size_t wide_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2, size_t room);
 int wide_fwd_nsplit(int B, int N, int H, int w1, int w2);
 int launch_wide_fwd(const Problem& p, int dtype, hipStream_t st);
 int launch_wide_bwd(const Problem& p, int dtype, hipStream_t st);
@@ -205,7 +211,7 @@ int launch_wide_bwd(const Problem& p, int dtype, hipStream_t st);
 int launch_fwd_merge(const Problem& p, int width, int dtype, hipStream_t st);
 // K'-side backward kernel (dQ, dK', dV') that keeps its partial sums on chip (K' windows too wide for
 // that are cut into segments of deltas, one workgroup each)
-size_t kp_scratch_bytes(int B, int N, int H, int D, int w1, int w2);
+size_t kp_scratch_bytes(int B, int N, int H, int D, int w1, int w2, size_t room);
 // Where the two kernels leave fp32 partial sums, rows of the kernel's width: the dQ partials of (K' block, segment)
 // workgroups, [dV' | dK'][kp_n][B*H][N][width] of a segmented K'-side launch and [dK | dV][kv_n][B*H][N][width] of a split
 // K-side launch.  NULL: that kernel wrote its results itself (dQ: not wanted).
@@ -218,8 +224,8 @@ int launch_mfma_bwd_kp(const Problem& p, int dtype, hipStream_t st, BwdSums* sum
 // K-side backward kernel (dK, dV) with paired wavefronts; for small grids it splits a key block's
 // query blocks over several workgroups, whose fp32 partial sums lie in the workspace behind the
 // K'-side part (kp_side_scratch_bytes); K' windows too wide for its LDS rows are walked in segments
-size_t kv_split_scratch_bytes(int B, int N, int H, int D, int w1, int w2);
-size_t kp_side_scratch_bytes(int B, int N, int H, int D, int w1, int w2);
+size_t kv_split_scratch_bytes(int B, int N, int H, int D, int w1, int w2, size_t room);
+size_t kp_side_scratch_bytes(int B, int N, int H, int D, int w1, int w2, size_t room);
 int launch_mfma_bwd_kv(const Problem& p, int dtype, hipStream_t st, BwdSums* sums);
 
 }  // namespace sa2

@@ -119,12 +119,12 @@ bool mfma_bwd_supported(int B, int N, int H, int D, int w1, int w2, int dtype) {
 
 // Workspace of the K'-side kernel (dQ partials, and the dK', dV' partials of a segmented launch),
 // rounded up so that what follows it stays 256-byte aligned
-size_t kp_side_scratch_bytes(int B, int N, int H, int D, int w1, int w2) {
-    return (kp_scratch_bytes(B, N, H, D, w1, w2) + 255) / 256 * 256;
+size_t kp_side_scratch_bytes(int B, int N, int H, int D, int w1, int w2, size_t room) {
+    return (kp_scratch_bytes(B, N, H, D, w1, w2, room) + 255) / 256 * 256;
 }
 
-size_t mfma_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2) {
-    return kp_side_scratch_bytes(B, N, H, D, w1, w2) + kv_split_scratch_bytes(B, N, H, D, w1, w2);
+size_t mfma_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2, size_t room) {
+    return kp_side_scratch_bytes(B, N, H, D, w1, w2, room) + kv_split_scratch_bytes(B, N, H, D, w1, w2, room);
 }
 
 int launch_bwd_sums(const Problem& p, const BwdSums& sums, int width, int dtype, hipStream_t st) {

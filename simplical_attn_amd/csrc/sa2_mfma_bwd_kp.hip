@@ -829,29 +829,29 @@ size_t kp_part_bytes(int B, int N, int H, int D, const KpPlan& pl) {
     return pl.nseg > 1 ? (size_t)2 * pl.nseg * B * H * (size_t)N * D * sizeof(float) : 0;
 }
 template <int D>
-KpPlan kp_plan_of(int B, int N, int H, int w1, int w2) {
+KpPlan kp_plan_of(int B, int N, int H, int w1, int w2, size_t room) {
     using C = KpCfg<D, kp_units<D>()>;
     constexpr int UPR = NPAIR * kp_units<D>();
     int most = UPR;
     if (C::fits(w2)) most = w2 + 1;
     else
         while (C::fits(most + UPR - 1)) most += UPR;
-    return plan_segments(B, N, H, w1, w2, UPR, most, [](int segw) { return C::raw_fits(segw - 1); },
+    return plan_segments(B, N, H, w1, w2, UPR, most, room, [](int segw) { return C::raw_fits(segw - 1); },
                          [&](const KpPlan& pl) { return kp_dq_part_bytes(B, N, H, D, pl) + kp_part_bytes(B, N, H, D, pl); });
 }
-KpPlan kp_plan(int B, int N, int H, int D, int w1, int w2) {
-    return D == 128 ? kp_plan_of<128>(B, N, H, w1, w2) : D == 64 ? kp_plan_of<64>(B, N, H, w1, w2) : kp_plan_of<32>(B, N, H, w1, w2);
+KpPlan kp_plan(int B, int N, int H, int D, int w1, int w2, size_t room) {
+    return D == 128 ? kp_plan_of<128>(B, N, H, w1, w2, room) : D == 64 ? kp_plan_of<64>(B, N, H, w1, w2, room) : kp_plan_of<32>(B, N, H, w1, w2, room);
 }
 
 template <class E, int D, bool PAD>
 int launch_kp(const Problem& p, hipStream_t st, BwdSums* sums) {
     constexpr int U = kp_units<D>();
     using C = KpCfg<D, U>;
-    const KpPlan pl = kp_plan(p.B, p.N, p.H, D, p.w1, p.w2);
+    const KpPlan pl = kp_plan(p.B, p.N, p.H, D, p.w1, p.w2, p.room);
     const int nkb = (p.N + BQ - 1) / BQ;
     const int64_t total = (int64_t)nkb * p.B * p.H * pl.nseg;
     if (total > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
-    if ((p.dq.p || pl.nseg > 1) && p.scratch_bytes < kp_scratch_bytes(p.B, p.N, p.H, D, p.w1, p.w2)) return SA2_ERR_WORKSPACE_TOO_SMALL;
+    if ((p.dq.p || pl.nseg > 1) && p.scratch_bytes < kp_scratch_bytes(p.B, p.N, p.H, D, p.w1, p.w2, p.room)) return SA2_ERR_WORKSPACE_TOO_SMALL;
     const int w2s = pl.segw - 1;
     const bool raw = C::raw_fits(w2s);
     const size_t lds = C::lds_bytes(w2s, raw);
@@ -889,9 +889,9 @@ int launch_kp(const Problem& p, hipStream_t st, BwdSums* sums) {
 }  // namespace
 
 // workspace of the K'-side kernel: the dQ partials, then (segmented launches) the dK' and dV' partials
-size_t kp_scratch_bytes(int B, int N, int H, int head_dim, int w1, int w2) {
+size_t kp_scratch_bytes(int B, int N, int H, int head_dim, int w1, int w2, size_t room) {
     const int D = mfma_width(head_dim);
-    const KpPlan pl = kp_plan(B, N, H, D, w1, w2);
+    const KpPlan pl = kp_plan(B, N, H, D, w1, w2, room);
     return kp_dq_part_bytes(B, N, H, D, pl) + kp_part_bytes(B, N, H, D, pl);
 }
 

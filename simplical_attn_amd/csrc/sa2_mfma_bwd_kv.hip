@@ -484,12 +484,13 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __
 struct KvPlan {
     int kb, nsplit;
 };
-KvPlan kv_plan(int B, int N, int H, int D, int w1, int w2) {
+KvPlan kv_plan(int B, int N, int H, int D, int w1, int w2, size_t room) {
     KvPlan best{1, 1};
     const int64_t bh = (int64_t)B * H;
     const int per = (w2 < N - 1 ? w2 : N - 1) + 1;                                   // units of a query block, at most
-    const double other = (double)kp_side_scratch_bytes(B, N, H, D, w1, w2) + (double)bh * N * 4 + 1024;
-    const double cap = other < (double)SA2_STATIC_WORKSPACE_BYTES ? (double)SA2_STATIC_WORKSPACE_BYTES - other : 134217728.0;
+    const double kp = (double)kp_side_scratch_bytes(B, N, H, D, w1, w2, room), other = kp + (double)bh * N * 4 + 1024;
+    double cap = other < (double)SA2_STATIC_WORKSPACE_BYTES ? (double)SA2_STATIC_WORKSPACE_BYTES - other : 134217728.0;
+    if (cap > (double)room - kp) cap = (double)room - kp;
     double least = 0;
     for (int kb = 1; kb <= (D <= 64 ? 2 : 1); ++kb) {
         const int vj = VPAIR * 32 * kb, njb = (N + vj - 1) / vj;
@@ -531,8 +532,8 @@ int launch_kv_geometry(const Problem& p, int nsplit, hipStream_t st, BwdSums* su
     // the partial sums of a split launch lie behind the K'-side kernel's part of the workspace
     float* part = nullptr;
     if (nsplit > 1) {
-        const size_t off = kp_side_scratch_bytes(p.B, p.N, p.H, D, p.w1, p.w2);
-        if (p.scratch_bytes < off + kv_split_scratch_bytes(p.B, p.N, p.H, D, p.w1, p.w2)) return SA2_ERR_WORKSPACE_TOO_SMALL;
+        const size_t off = kp_side_scratch_bytes(p.B, p.N, p.H, D, p.w1, p.w2, p.room);
+        if (p.scratch_bytes < off + kv_split_scratch_bytes(p.B, p.N, p.H, D, p.w1, p.w2, p.room)) return SA2_ERR_WORKSPACE_TOO_SMALL;
         part = (float*)((char*)p.scratch + off);
     }
     const bool seg = ws < p.w2;
@@ -560,7 +561,7 @@ int launch_kv_geometry(const Problem& p, int nsplit, hipStream_t st, BwdSums* su
 
 template <class E, int D, bool PAD>
 int launch_kv(const Problem& p, hipStream_t st, BwdSums* sums) {
-    const KvPlan pl = kv_plan(p.B, p.N, p.H, D, p.w1, p.w2);
+    const KvPlan pl = kv_plan(p.B, p.N, p.H, D, p.w1, p.w2, p.room);
     if constexpr (D <= 64) {
         if (pl.kb == 2) return launch_kv_geometry<E, D, 2, PAD>(p, pl.nsplit, st, sums);
     }
@@ -569,9 +570,9 @@ int launch_kv(const Problem& p, hipStream_t st, BwdSums* sums) {
 
 }  // namespace
 
-size_t kv_split_scratch_bytes(int B, int N, int H, int head_dim, int w1, int w2) {
+size_t kv_split_scratch_bytes(int B, int N, int H, int head_dim, int w1, int w2, size_t room) {
     const int D = mfma_width(head_dim);
-    const KvPlan pl = kv_plan(B, N, H, D, w1, w2);
+    const KvPlan pl = kv_plan(B, N, H, D, w1, w2, room);
     return pl.nsplit > 1 ? (size_t)2 * pl.nsplit * B * H * (size_t)N * D * sizeof(float) : 0;
 }
 

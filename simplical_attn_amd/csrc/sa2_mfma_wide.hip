@@ -1347,8 +1347,8 @@ void wide_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __rest
 }
 
 // Shares of a key block's stream of units: the least time by grid_time with about 2.3 us per unit and the time of a dozen
-// units around them.  Partial sums may take 64 MiB.
-int wide_kv_nsplit(int B, int N, int H, int D, int w1, int w2) {
+// units around them.  Partial sums may take 64 MiB, or `room`.
+int wide_kv_nsplit(int B, int N, int H, int D, int w1, int w2, size_t room) {
     constexpr double UNIT = 2.3, AROUND = 12;
     const int64_t bh = (int64_t)B * H, base = bh * ((N + WJ - 1) / WJ);
     const int64_t units = (int64_t)((WJ + (w1 < N ? w1 : N)) / BQ + 1) * ((w2 < N - 1 ? w2 : N - 1) + 1);      // of a key block's stream, at most
@@ -1357,7 +1357,7 @@ int wide_kv_nsplit(int B, int N, int H, int D, int w1, int w2) {
     double least = 0;
     for (int ns = 1; ns <= 16 && units / ns >= 4; ++ns) {
         const double part = ns > 1 ? 2.0 * ns * bh * N * D * 4 : 0, per = (double)((units + ns - 1) / ns);
-        if (part > 67108864.0) break;
+        if (part > 67108864.0 || part > (double)room) break;
         const double cost = UNIT * grid_time(base * ns, per + AROUND, per * fill + AROUND) + (ns > 1 ? SUM_LAUNCH_STEPS + part / PART_BYTES_PER_STEP : 0);
         if (least == 0 || cost < 0.97 * least) {
             least = cost;
@@ -1370,12 +1370,12 @@ size_t wide_dq_part_bytes(int B, int N, int H, const KpPlan& pl) {
     return ((size_t)B * H * ((N + BQ - 1) / BQ) * pl.nseg * (size_t)(BQ + pl.segw - 1) * 256 * sizeof(float) + 255) / 256 * 256;
 }
 size_t wide_kp_part_bytes(int B, int N, int H, const KpPlan& pl) { return pl.nseg > 1 ? (size_t)2 * pl.nseg * B * H * (size_t)N * 256 * sizeof(float) : 0; }
-KpPlan wide_kp_plan(int B, int N, int H, int w1, int w2) {
-    return plan_segments(B, N, H, w1, w2, 2, w2 + 1, [](int) { return false; },      // (the work between two sweeps takes long here)
+KpPlan wide_kp_plan(int B, int N, int H, int w1, int w2, size_t room) {
+    return plan_segments(B, N, H, w1, w2, 2, w2 + 1, room, [](int) { return false; },      // (the work between two sweeps takes long here)
                          [&](const KpPlan& pl) { return wide_dq_part_bytes(B, N, H, pl) + wide_kp_part_bytes(B, N, H, pl); });
 }
-size_t wide_kp_bytes(int B, int N, int H, int w1, int w2) {
-    const KpPlan pl = wide_kp_plan(B, N, H, w1, w2);
+size_t wide_kp_bytes(int B, int N, int H, int w1, int w2, size_t room) {
+    const KpPlan pl = wide_kp_plan(B, N, H, w1, w2, room);
     return (wide_dq_part_bytes(B, N, H, pl) + wide_kp_part_bytes(B, N, H, pl) + 255) / 256 * 256;
 }
 
@@ -1401,9 +1401,10 @@ int launch_wide_bwd_of(const Problem& p, hipStream_t st) {
     if (rc != SA2_OK) return rc;
     const bool biased = p.k2_bias != 0.f || p.v2_bias != 0.f;           // (the common case pays for none of it)
     BwdSums sums = {};
-    const KpPlan pl = wide_kp_plan(p.B, p.N, p.H, p.w1, p.w2);
-    const int nsplit = wide_kv_nsplit(p.B, p.N, p.H, D, p.w1, p.w2);
-    if (((p.dq.p || pl.nseg > 1) || nsplit > 1) && p.scratch_bytes < wide_bwd_scratch_bytes(p.B, p.N, p.H, D, p.w1, p.w2)) return SA2_ERR_WORKSPACE_TOO_SMALL;
+    const KpPlan pl = wide_kp_plan(p.B, p.N, p.H, p.w1, p.w2, p.room);
+    const size_t kp_bytes = wide_kp_bytes(p.B, p.N, p.H, p.w1, p.w2, p.room);
+    const int nsplit = wide_kv_nsplit(p.B, p.N, p.H, D, p.w1, p.w2, room_left(p.room, kp_bytes));
+    if (((p.dq.p || pl.nseg > 1) || nsplit > 1) && p.scratch_bytes < wide_bwd_scratch_bytes(p.B, p.N, p.H, D, p.w1, p.w2, p.room)) return SA2_ERR_WORKSPACE_TOO_SMALL;
     if (p.dq.p || p.dk2.p || p.dv2.p) {
         const int nkb = (p.N + BQ - 1) / BQ;
         const int64_t total = (int64_t)nkb * p.B * p.H * pl.nseg;
@@ -1427,7 +1428,7 @@ int launch_wide_bwd_of(const Problem& p, hipStream_t st) {
         const int njb = (p.N + WJ - 1) / WJ;
         const int64_t total = (int64_t)njb * p.B * p.H * nsplit;
         if (total > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
-        float* part = (float*)((char*)p.scratch + wide_kp_bytes(p.B, p.N, p.H, p.w1, p.w2));
+        float* part = (float*)((char*)p.scratch + kp_bytes);
         auto go = [&](auto kernel) {
             if (!allow_full_lds((const void*)kernel)) return false;
             hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(WT), WIDE_KV_LDS, st, p, njb, (int)total, nsplit, part);
@@ -1450,9 +1451,10 @@ bool wide_bwd_supported(int D, int w2, int dtype) {
     return wide_supported(D, dtype);
 }
 
-size_t wide_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2) {
-    const int ns = wide_kv_nsplit(B, N, H, D, w1, w2);
-    return wide_kp_bytes(B, N, H, w1, w2) + (ns > 1 ? (size_t)2 * ns * B * H * (size_t)N * D * sizeof(float) : 0);
+size_t wide_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2, size_t room) {
+    const size_t kp_bytes = wide_kp_bytes(B, N, H, w1, w2, room);
+    const int ns = wide_kv_nsplit(B, N, H, D, w1, w2, room_left(room, kp_bytes));
+    return kp_bytes + (ns > 1 ? (size_t)2 * ns * B * H * (size_t)N * D * sizeof(float) : 0);
 }
 
 int wide_fwd_nsplit(int B, int N, int H, int w1, int w2) { return plan_forward(B, N, H, 256, w1, w2, WW); }

@@ -86,6 +86,32 @@ def test_static_workspace_backward_with_null_gradients(needs):
                 assert (b == 7.0).all() and (a == -3.0).all(), name          # the fill values: untouched
 
 
+@pytest.mark.parametrize("dtype,shape,w", [
+    (torch.bfloat16, (1, 512, 4, 256), (512, 32)),       # the planned cuts of the K' window take more than the array: fewer
+    (torch.bfloat16, (4, 971, 9, 128), (78, 55)),
+    (torch.float32, (5, 1670, 4, 64), (466, 184)),
+    (torch.float32, (1, 700, 16, 96), (24, 300)),        # head dims without 16-bit or fp32 MFMA kernels of their own: the
+    (torch.bfloat16, (2, 1024, 8, 80), (16, 250)),       # fp32 FMA kernels, which need the row term only
+])
+def test_static_workspace_takes_problems_whose_plans_want_more(dtype, shape, w):
+    import simplical_attn_amd as sa
+    lib = _lib.load()
+    code = DT[dtype]
+    assert lib.sa2_bwd_workspace_bytes(*shape, *w, code, 0) > _lib.STATIC_WORKSPACE_BYTES
+    q, k1, k2, v1, v2, dout = [t.cuda() for t in make_inputs(*shape, 4, dtype)]
+    out, lse = sa.simplicial_forward(q, k1, k2, v1, v2, *w)
+    want = sa.simplicial_backward(q, k1, k2, v1, v2, out, lse, dout, *w)
+    grads = [torch.full_like(q, 7.0) for _ in range(5)]
+    strides = _lib.stride_array([(t.stride(0), t.stride(1), t.stride(2)) for t in (q, k1, k2, v1, v2, out, dout, *grads)])
+    _lib.check(lib.sa2_backward_static_workspace(*[t.data_ptr() for t in (q, k1, k2, v1, v2, out, dout, lse, *grads)], *shape, strides,
+                                                 *w, shape[3] ** -0.5, 0.0, 0.0, code, 1, 0, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    for name, a, b in zip(("dq", "dk1", "dk2", "dv1", "dv2"), grads, want):
+        # other plans and kernels of the same arithmetic: both are within the bar of their type
+        err = ((a.float() - b.float()).norm() / b.float().norm()).item()
+        assert err <= (2e-2 if dtype == torch.bfloat16 else 3e-6), (name, err)
+
+
 def test_static_workspace_rejects_what_does_not_fit():
     lib = _lib.load()
     dev = torch.device("cuda:0")
