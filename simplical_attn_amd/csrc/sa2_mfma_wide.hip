@@ -692,9 +692,13 @@ void wide_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_part, 
     }
 #pragma unroll
     for (int kk = 0; kk < DK; ++kk) asm volatile("" : "+v"(raw[kk]));
+    // The pair's unit in a round.  A last round of one unit: the second pair takes the same one with weights of zero, so that
+    // a NaN it meets belongs to rows inside the windows (behind them it would reach rows that have no part in it).
+    const int last_unit = n_units > 0 ? n_units - 1 : 0;
+    auto unit_of = [&](int r) { return 2 * r + pair < last_unit ? 2 * r + pair : last_unit; };
     // LSE * log2(e) (role 0) or D (role 1) of the lane's row, one round ahead
     auto row_value = [&](int r) {
-        const int i = kq + (here() & 31) + 2 * r + pair, ic = i < N ? i : N - 1;
+        const int i = kq + (here() & 31) + unit_of(r), ic = i < N ? i : N - 1;
         return role ? p.dsum[(int64_t)bh * N + ic] : p.lse[(int64_t)bh * N + ic] * LOG2E;
     };
     float value_next = row_value(0);
@@ -720,7 +724,8 @@ void wide_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_part, 
         constexpr int R = decltype(ROLE)::value;
         unsigned char* rows_s = R ? do_s : q_s;
         for (int round = 0; round < nrounds; ++round) {
-            const int delta = 2 * round + pair;              // relative to the segment
+            const int delta = unit_of(round);                // relative to the segment
+            const bool has_unit = 2 * round + pair < n_units;
             float value = value_next;
             asm volatile("" : "+v"(value));
             if (round + 1 < nrounds) value_next = row_value(round + 1);
@@ -787,11 +792,11 @@ void wide_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_part, 
                 if constexpr (R == 0) {
                     // element v of this lane is key 32 * jt + 8*(v/4) + 4*hf + v%4, the row's query is kq + ln + delta
                     const int j0 = jt * TJ, i_min = kq + delta;
-                    if (!(i_min + BQ - 1 < N && delta < n_units && j0 + TJ - 1 <= i_min && j0 >= i_min + BQ - 1 - w1)) {
+                    if (!(i_min + BQ - 1 < N && has_unit && j0 + TJ - 1 <= i_min && j0 >= i_min + BQ - 1 - w1)) {
                         int hi = i_min + ln - j0 - 4 * hf;
                         opaque(hi);
                         const int lo = hi - w1;
-                        const bool row_ok = i_min + ln < N && delta < n_units;
+                        const bool row_ok = i_min + ln < N && has_unit;
 #pragma unroll
                         for (int v = 0; v < 16; ++v) {
                             const int c = 8 * (v >> 2) + (v & 3);

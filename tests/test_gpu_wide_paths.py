@@ -50,3 +50,16 @@ def test_weights_that_overflow_take_the_second_pass(dtype, N, w2):
     out, lse = sa.simplicial_forward(*[t.cuda() for t in x], N, w2)
     assert_close_rel(out, want["out"], 2e-2 if dtype == torch.bfloat16 else 1e-2, "out")
     assert_close_rel(lse, want["lse"], 4e-3, "lse")                            # (the rounding of q * k2~ * scale, times 200)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("w2", [20, 21])
+def test_a_query_that_is_not_a_number_stays_in_its_window(dtype, w2):
+    """An even K' window has an odd number of deltas: the last round's second unit lies behind the window."""
+    import simplical_attn_amd as sa
+    x = [t.cuda() for t in make_inputs(1, 160, 1, 256, seed=3, dtype=dtype)]
+    x[0][:, 50] = float("nan")
+    out, lse = sa.simplicial_forward(*x[:5], 40, w2)
+    dq, _, dk2, _, dv2 = sa.simplicial_backward(*x[:5], out, lse, x[5], 40, w2)
+    rows = lambda t: t[0, :, 0].isnan().any(-1).nonzero()[:, 0].tolist()
+    assert rows(dq) == [50] and rows(dk2) == rows(dv2) == list(range(50 - w2, 51))
