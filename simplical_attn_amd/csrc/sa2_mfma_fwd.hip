@@ -1007,21 +1007,25 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
     return any_bad;
 }
 
+// The kernel's only argument: it starts the kernel argument segment, from which the second pass reads it again.
+struct FwdArgs {
+    Problem p;
+    int nqb, total, left;
+};
 template <class E, int D, int MODE, bool SIDE, bool PAD, bool SPLIT>
 __global__ __launch_bounds__(FT) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void mfma_fwd_kernel(Problem p, int nqb, int total, int left) {
-    const bool again = fwd_block<E, D, MODE, SIDE, PAD, SPLIT>(p, nqb, total, left, threadIdx.x);
+void mfma_fwd_kernel(FwdArgs args) {
+    const bool again = fwd_block<E, D, MODE, SIDE, PAD, SPLIT>(args.p, args.nqb, args.total, args.left, threadIdx.x);
     if constexpr (MODE == MODE_FAST) {
         if (again) {                              // (uniform over the workgroup)
             __syncthreads();
             // (the arguments are read again from the kernel argument segment, so that none of them stays in a
             // register for this pass while the first one runs)
-            typedef const __attribute__((address_space(4))) Problem* arg_ptr;
-            arg_ptr args = (arg_ptr)__builtin_amdgcn_kernarg_segment_ptr();
-            asm volatile("" : "+s"(args));
-            const Problem* again_p = (const Problem*)args;
-            const int* rest = (const int*)(again_p + 1);
-            fwd_block<E, D, MODE_SAFE, SIDE, PAD, SPLIT>(*again_p, rest[0], rest[1], 0, recompute_here(threadIdx.x));
+            typedef const __attribute__((address_space(4))) FwdArgs* arg_ptr;
+            arg_ptr segment = (arg_ptr)__builtin_amdgcn_kernarg_segment_ptr();
+            asm volatile("" : "+s"(segment));
+            const FwdArgs* again_args = (const FwdArgs*)segment;
+            fwd_block<E, D, MODE_SAFE, SIDE, PAD, SPLIT>(again_args->p, again_args->nqb, again_args->total, 0, recompute_here(threadIdx.x));
         }
     }
 }
@@ -1044,13 +1048,13 @@ int launch_fwd_kernels(const Problem& p, int nqb, int total, hipStream_t st) {
         const int ngrp = (nqb + FW - 1) / FW;
         const int total_left = ngrp * (total / nqb);
         if (!allow_full_lds((const void*)mfma_fwd_kernel<E, D, MODE_LEFT, false, PAD, false>)) return SA2_ERR_LAUNCH_FAILED;
-        hipLaunchKernelGGL((mfma_fwd_kernel<E, D, MODE_LEFT, false, PAD, false>), dim3((unsigned)total_left), dim3(FT), C::STAGE_BYTES, st, p,
-                           ngrp, total_left, 0);
+        hipLaunchKernelGGL((mfma_fwd_kernel<E, D, MODE_LEFT, false, PAD, false>), dim3((unsigned)total_left), dim3(FT), C::STAGE_BYTES, st,
+                           (FwdArgs{p, ngrp, total_left, 0}));
         if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
     }
     auto go = [&](auto kernel, int64_t grid) {
         if (!allow_full_lds((const void*)kernel)) return false;
-        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(FT), lds, st, p, nqb, (int)grid, left);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(FT), lds, st, (FwdArgs{p, nqb, (int)grid, left}));
         return hipGetLastError() == hipSuccess;
     };
     if (p.nsplit <= 1) return go(mfma_fwd_kernel<E, D, MODE_FAST, SIDE, PAD, false>, total) ? SA2_OK : SA2_ERR_LAUNCH_FAILED;
