@@ -7,15 +7,15 @@ A step is one forward + backward pass of the operator over one batch of
 synthetic input that is already resident in HBM (iid normal, seeded, bf16).
 The default workload is the headline configuration: bf16, B=1 H=16 N=8192 D=128,
 w1=512 w2=32.  Workloads c1 (fp32 B=1 H=2 N=128 D=64 w 32/16, the forward-only plumbing
-configuration) and c2f32 (fp32 tensors at the shape of c2) run on the fp32 MFMA kernels and are
-priced against the fp32 matrix peak.  Prints ONE JSON line:
+configuration) and c2f32 (fp32 tensors at the shape of c2) run on the plane-split kernels, six bf16
+MFMAs per product, and are priced against a sixth of the bf16 dense peak.  Prints ONE JSON line:
 
   metric/value   forward+backward algorithmic TFLOP/s: 16*D*T flops per step,
                  T = number of valid (i,j,k) triples (matmul flops only, 2 per
                  MAC: 4*D*T forward, 12*D*T backward)
   roofline       the kernel group that takes the longest in the step (whichever of the
                  forward, the K-side and the K'-side backward measures longest in this
-                 run), against the bf16 dense MFMA peak (achieved = that group's
+                 run), against the dense MFMA peak (achieved = that group's
                  algorithmic flops / its duration, measured here with events on the
                  launch stream); `groups` lists all three; `mfma_busy` and
                  `traffic` are rocprofv3 counter results read from profiles/
@@ -45,7 +45,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 PEAK_BF16_TFLOPS = 2516.6     # published: 256 CU x 2.4 GHz x 4096 flop/clk/CU, dense
-PEAK_FP32_TFLOPS = 157.3
+PEAK_FP32_TFLOPS = PEAK_BF16_TFLOPS / 6      # fp32 tensors: six bf16 MFMAs per product (v_mfma_f32_32x32x2_f32: 157.3)
 PEAK_HBM_GBS = 8000.0
 BF16_FLOP_PER_CLK_PER_CU = 4096
 
@@ -362,12 +362,17 @@ def main():
     half_bwd = bwd_flops / 2
     keys, key_sources = profile_keys()
     wl = args.workload
+    # launches of each group at this workload: pre-passes (a single unit left over after the rounds), main kernels, sums.
+    # Beside them a backward launches the row-term kernel and, in fp32, the one that looks at its verdicts.
+    launches = {"c4": (2, 1, 3), "c2": (2, 2, 3), "c5": (2, 1, 2), "c1": (1, 2, 2), "c2f32": (1, 2, 2)}[wl]
     if fp32:
-        labels = ("f32_fwd_kernel<%d> (v_mfma_f32_32x32x2_f32)" % D, 1, "f32_bwd_kv_kernel<%d> (dK, dV)" % D, 1,
-                  "f32_bwd_kp_kernel<%d> + f32_dq_sum_kernel (dQ, dK', dV')" % D, 2)
+        labels = ("split_fwd_kernel<fp32, %d> (six v_mfma_f32_32x32x16_bf16 per product)" % D, launches[0],
+                  "split_kv_kernel<fp32, %d> + sum (dK, dV)" % D, launches[1],
+                  "split_kp_kernel<fp32, %d> + sum (dQ, dK', dV')" % D, launches[2])
     else:
-        labels = ("mfma_fwd_kernel<%d> (pre-pass + fast kernel + repair launch)" % D, 3, "mfma_bwd_kv_kernel<%d> (dK, dV)" % D, 1,
-                  "mfma_bwd_kp_kernel<%d> (pre-pass + main) + dq_sum (dQ, dK', dV')" % D, 3)
+        labels = ("mfma_fwd_kernel<%d> (pre-pass + main)" % D, launches[0],
+                  "mfma_bwd_kv_kernel<%d>%s (dK, dV)" % (D, " + sum" if launches[1] > 1 else ""), launches[1],
+                  "mfma_bwd_kp_kernel<%d> (%smain) + sum (dQ, dK', dV')" % (D, "pre-pass + " if launches[2] > 2 else ""), launches[2])
     kernels = {
         "forward": {"kernel": labels[0], "ms": fwd_ms, "flops": fwd_flops, "launches": labels[1]},
         "backward_k_side": {"kernel": labels[2], "ms": bwd_k1_ms, "flops": half_bwd, "launches": labels[3]},
@@ -375,7 +380,7 @@ def main():
     }
     for name, k in kernels.items():
         k["tflops"] = k["flops"] / k["ms"] / 1e9
-        k["frac_bf16_peak"] = k["tflops"] / PEAK_TFLOPS              # (of the fp32 matrix peak for the fp32 workloads)
+        k["frac_bf16_peak"] = k["tflops"] / PEAK_TFLOPS              # (of a sixth of it for the fp32 workloads)
         k["mfma_busy"] = keys.get((wl, name, "mfma_busy"))          # rocprofv3, from profiles/
         k["traffic"] = keys.get((wl, name, "traffic_bytes"))
     kernels["forward"]["hbm_gbs"] = fwd_bytes / fwd_ms / 1e6
@@ -393,20 +398,19 @@ def main():
     for cname, call, ms_call in (("forward", fwd_call, fwd_ms), ("backward", bwd_call, bwd_all_ms), ("step", step, ms_per_step)):
         clocks[cname] = observed_clock_mhz(call, ms_call)
     cus = props.multi_processor_count
-    flop_per_clk_per_cu = int(round(BF16_FLOP_PER_CLK_PER_CU * PEAK_TFLOPS / PEAK_BF16_TFLOPS))      # 4096 bf16, 256 fp32
+    flop_per_clk_per_cu = BF16_FLOP_PER_CLK_PER_CU * PEAK_TFLOPS / PEAK_BF16_TFLOPS      # 4096 bf16, a sixth of it fp32
     peak_at = lambda mhz: cus * flop_per_clk_per_cu * mhz * 1e6 / 1e12
     clock = {"mhz": clocks, "method": "device cycle counter (60 ms spin kernel on a second stream) / event time",
              "peak_bf16_tflops_at_observed_clock": {k: peak_at(v) for k, v in clocks.items()},
              "published_peak_bf16_tflops": PEAK_TFLOPS,
-             "published_peak_is": "%d CU x 2400 MHz x %d flop/clk/CU (%s matrix)" % (cus, flop_per_clk_per_cu, dtype_name)}
+             "published_peak_is": "%d CU x 2400 MHz x %.0f flop/clk/CU (%s tensors)" % (cus, flop_per_clk_per_cu, dtype_name)}
     kernels["forward"]["frac_at_observed_clock"] = kernels["forward"]["tflops"] / peak_at(clocks["forward"])
     for name in ("backward_k_side", "backward_kprime_side", "backward"):
         kernels[name]["frac_at_observed_clock"] = kernels[name]["tflops"] / peak_at(clocks["backward"])
 
-    # The dominant kernel group: the one that takes the longest in the step.  The K-side kernel is a
-    # single launch (its duration here: the call that requests only dK and dV, minus the row-dot
-    # kernel); the forward and the K'-side group hold three launches each (a pre-pass and a short
-    # epilogue kernel beside the main one), of which the main kernel is more than nine tenths.
+    # The dominant kernel group: the one that takes the longest in the step.  (A backward group's duration is
+    # that of a call that requests its gradients only, minus the row-term kernel; of a group's launches the main
+    # kernel is more than nine tenths.)
     dominant = max(("forward", "backward_k_side", "backward_kprime_side"), key=lambda k: kernels[k]["ms"])
     roofline = {
         "bound": "mfma", "kernel": kernels[dominant]["kernel"], "group": dominant,
