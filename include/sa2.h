@@ -69,7 +69,7 @@ const char* sa2_strerror(int status);
 /* 1 if head_dim is one that MFMA kernels of the element type have a width of their own for (the ones
  * SA2_FLAG_FORCE_MFMA accepts, given 16-byte aligned rows), 0 otherwise.  Under SA2_FLAG_AUTO head_dim 16
  * and other head dims up to 128 (multiples of 4 in fp32, of 8 in 16 bits) also run on the matrix pipes, in a wider
- * kernel or, in 16 bits, in the fp32 MFMA kernels.  sa2_backward makes the same choice: its MFMA
+ * kernel; 16-bit tensors of those other than 16 in the kernels that carry fp32 operands as sums of bf16 planes.  sa2_backward makes the same choice: its MFMA
  * kernels take any K' window (one wider than their on-chip accumulators hold is walked in segments). */
 int sa2_uses_mfma(int B, int N, int H, int D, int w1, int w2, int dtype);
 

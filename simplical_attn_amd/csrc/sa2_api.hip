@@ -97,11 +97,11 @@ void* static_workspace() {
 size_t dsum_bytes(int B, int N, int H) { return align_up((size_t)B * H * N * sizeof(float), 256); }
 
 // Which kernels a call takes: the fp32 FMA kernels, the tuned 16-bit MFMA kernels (head_dim 32, 64, 128), the
-// 16-bit MFMA kernels for head_dim 256, or the fp32 MFMA kernels.
+// 16-bit MFMA kernels for head_dim 256, or the plane-split kernels (fp32 arithmetic on the 16-bit MFMA).
 enum KernelPath { PATH_GENERIC, PATH_MFMA16, PATH_WIDE16, PATH_MFMA32 };
 
 // Head dims the matrix-pipe kernels of the element type have a width of their own for.  The others run in the next
-// wider kernel (head_dim 16) or in the fp32 MFMA kernels, which SA2_FLAG_AUTO chooses; a forced call asks for these.
+// wider kernel (head_dim 16) or in the plane-split kernels, which SA2_FLAG_AUTO chooses; a forced call asks for these.
 bool own_width(int D, int dtype) { return D == 32 || D == 64 || D == 128 || D == (dtype == SA2_F32 ? 96 : 256); }
 
 KernelPath pick_path(const Problem& p, int dtype, unsigned flags, bool backward, int* status) {
@@ -229,7 +229,7 @@ const char* sa2_strerror(int status) {
         case SA2_ERR_BAD_SHAPE: return "bad shape: B, N, H, D must be >= 1 and D <= 256";
         case SA2_ERR_BAD_STRIDE: return "bad stride: batch/sequence/head strides must be positive (D stride is 1)";
         case SA2_ERR_BAD_WINDOW: return "bad window: w1 and w2 must be >= 0 (>= 1 for the half-open convention)";
-        case SA2_ERR_WORKSPACE_TOO_SMALL: return "workspace is smaller than sa2_bwd_workspace_bytes() or not 256-byte aligned";
+        case SA2_ERR_WORKSPACE_TOO_SMALL: return "workspace is smaller than sa2_bwd_workspace_bytes() (forward: sa2_fwd_workspace_bytes()) or not 256-byte aligned";
         case SA2_ERR_LAUNCH_FAILED: return "a HIP kernel launch failed";
         case SA2_ERR_UNSUPPORTED: return "the forced kernel path does not support this shape, dtype or layout";
         case SA2_ERR_TOO_LARGE: return "problem too large for the kernels' 32-bit grid (B*H*N must be < 2^31)";

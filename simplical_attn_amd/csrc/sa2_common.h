@@ -108,13 +108,18 @@ inline size_t room_left(size_t room, size_t taken) { return room == ROOM_ANY ? r
 struct KpPlan {
     int segw, nseg;
 };
+// The uncut launch's pre-pass (the single delta over of w2 = 4n) is charged as the round it saves: at B1 H16 N8192 D128
+// w 512/32 eight rounds and the pre-pass take 2826 us, nine rounds (w 512/33) 2895.
 // Segments are whole rounds of `upr` deltas, at most `most` deltas (what LDS holds).  A round sweeps the tiles of the K
 // window; the work between two sweeps takes about two tiles' time, or five and a half where the rows of q and dO do not
 // fit LDS beside the accumulator (raw(segment)), prologue and epilogue about eight.  bytes(plan): all partial sums; a cut may
 // take 32 MiB, or three times what the uncut launch needs.
 // Measured on the 16-bit kernel (us, uncut -> planned): B2 H4 N512 D64 w 256/256 607 -> 234 (seven segments),
 // B3 H21 N282 D128 w 176/48 488 -> 303 (three), B1 H8 N4096 D128 w 128/64 862 -> 655 (two: the rows then fit LDS),
-// B2 H4 N256 D64 w 32/32 43 -> 29 (three).
+// B2 H4 N256 D64 w 32/32 43 -> 29 (three), B1 H8 N32768 D128 w 1024/64 19809 -> 19385 (two; 0.66 GB more of partial sums).
+// Against every cut (profiles/plan_cuts.md): the plane-split kernels within 3.0 % of the best at ten sizes, head_dim 256
+// within 3.2 % at seven of eight (27 % off at B1 H3 N700 w 500/100, where the bytes bind), the 16-bit kernels within 0.2 % at
+// ten of twelve (30 % off at B4 H8 N2048 D128 w 64/48, 6 % at B4 H16 N2048 D128 w 1024/96).
 template <class Raw, class Bytes>
 KpPlan plan_segments(int B, int N, int H, int w1, int w2, int upr, int most, size_t room, Raw&& raw, Bytes&& bytes) {
     constexpr int ROWS = 32, MOST_SEGMENTS = 16;
@@ -144,8 +149,10 @@ KpPlan plan_segments(int B, int N, int H, int w1, int w2, int upr, int most, siz
 }
 
 // A forward launch in nsplit shares of the rounds of `upr` deltas: fp32 partial outputs in the workspace.  A round takes
-// about three tiles' time beside its sweep, prologue and epilogue about eight.  Fewer than four rounds are not worth a
-// summation launch.
+// about three tiles' time beside its sweep, prologue and epilogue about eight.  Fewer than four rounds are not shared: at
+// B3 H6 N777 D64 w 100/20 two shares take 66 us against 41 (a grid smaller still would gain: fp32 B1 H2 N128 D64 w 32/16
+// 28 us, 19 in three shares).  Against every cut: the best or within 2 % at eight of fifteen sizes, 5 - 25 % off at the
+// others, where a grid a little under a whole wave would take more shares.
 inline int plan_forward(int B, int N, int H, int width, int w1, int w2, int upr) {
     constexpr int ROWS = 32, MOST = 16;
     const int64_t rows = (int64_t)B * H * N, base = (int64_t)B * H * ((N + ROWS - 1) / ROWS);
@@ -189,7 +196,7 @@ int mfma_fwd_nsplit(int B, int N, int H, int D, int w1, int w2, bool force_prepa
 size_t mfma_fwd_part_bytes(int B, int N, int H, int D, int nsplit);
 int launch_mfma_bwd(const Problem& p, int dtype, hipStream_t st);
 size_t mfma_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2, size_t room);
-// fp32 arithmetic on the fp32 MFMA: fp32 tensors of any head_dim up to 128 that is a multiple of 4, and 16-bit tensors
+// fp32 arithmetic on the 16-bit MFMA, operands as sums of bf16 planes (sa2_split_mfma.hip): fp32 tensors of any head_dim up to 128 that is a multiple of 4, and 16-bit tensors
 // of the head dims the 16-bit kernels do not have (multiples of 8 up to 120); rows 16-byte aligned
 bool f32_mfma_supported(int D, int dtype);
 bool f32_mfma_bwd_supported(int D, int w2, int dtype);

@@ -28,7 +28,7 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 
 // The 16-bit element type of a call: how its pairs unpack to fp32, its MFMA and its
 // two-element dot product.  WEIGHT_LIMIT bounds the row sum of one tile of softmax weights
-// in the forward's fast kernel: above it the block is recomputed by the repair kernel (bf16
+// in the forward's first pass: above it the block is computed again with a moving reference point (bf16
 // shares fp32's exponent range; an fp16 weight must stay below 65504).
 struct ElemBF16 {
     typedef __bf16 scalar;

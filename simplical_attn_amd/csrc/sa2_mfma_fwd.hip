@@ -262,7 +262,7 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
             if (tid < BQ) {
                 const int it = i0 + tid < N ? i0 + tid : N - 1;
                 const float lam = p.lse[(int64_t)bh * N + it];
-                bad = !(lam == lam);                           // the pre-pass overflowed: repair the block
+                bad = !(lam == lam);                           // the pre-pass overflowed: the block takes its second pass
                 lam_s[tid] = lam;
             }
         } else {
@@ -491,7 +491,7 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
             };
 
             if (SAFE) {
-                // ---- repair pass: the reference point follows the maxima on every tile ----
+                // ---- second pass: the reference point follows the maxima on every tile ----
                 for (int s = 0; s < nt; ++s) {
                     begin_step(s);
                     const uint32_t Ks = stage_addr(buf);
@@ -742,7 +742,7 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
                 const float lt = l + other_half(l);
                 const bool row_has = (i0 + ln_u < N) & (i0 + ln_u >= delta);
                 // The fast kernel keeps a unit's reference point fixed, and every unit after the wavefront's
-                // first starts from the running one: all weights are 1.  The repair kernel moves it.
+                // first starts from the running one: all weights are 1.  The second pass moves it.
                 float a = 1.f, c = 1.f;
                 if (SAFE) {
                     const float Mn = fmaxf(Mw, m), Mu = Mn == -INFINITY ? 0.f : Mn;

@@ -36,7 +36,8 @@
 //                       operands), streaming every unit (query block, delta) that can see them.
 // The backward kernels pair their eight wavefronts as the 16-bit kernels do (one P and one dS wavefront per SIMD, so that
 // each holds the planes of one operand and one accumulator in 256 registers: four wavefronts that did both needed 350 and
-// moved 136 of them between the two register files per tile).  A step has two halves.  In the first the P wavefront
+// moved 136 of them between the two register files per tile; at 128 columns in fp32 they do not fit all the same, and 470
+// bytes per lane of the K'-side kernel and 300 of the K-side one go through scratch memory).  A step has two halves.  In the first the P wavefront
 // computes S and, beside the other's dP MFMAs, the exponentials and the split of P; in the second it adds P's product
 // while the dS wavefront multiplies and splits dS, whose product follows.
 // Every output element has one writer and a fixed summation order: no atomics, bitwise reproducible.
@@ -1195,7 +1196,9 @@ void split_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __res
     }
 }
 
-// Shares a key block's query blocks are split into when the K-side grid is smaller than the chip
+// Shares a key block's query blocks are split into when the K-side grid is smaller than the chip: doubled until the grid
+// holds two waves.  Against every number of shares (profiles/plan_cuts.md): within 11 % of the best at seven of ten sizes,
+// 22 - 37 % off at small ones whose best is no power of two (bf16 B2 H3 N777 D40 w 100/20: 140 us in eight, 102 in six).
 int split_kv_nsplit(int B, int N, int H, int D, int w1, int w2, size_t room) {
     const int64_t bh = (int64_t)B * H, base = bh * ((N + XJ - 1) / XJ);
     const int blocks = (XJ + (w1 < N ? w1 : N) + BQ - 1) / BQ + 1;

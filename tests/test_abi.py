@@ -70,7 +70,7 @@ def test_argument_validation_needs_no_gpu(lib):
     assert lib.sa2_backward(one, one, one, one, one, one, one, one, one, one, one, one, one, one, 16,
                             1, 8, 2, 64, strides, 4, 4, 0.125, 0.0, 0.0, 0, 1, 0, None) == -6
     assert lib.sa2_uses_mfma(1, 8192, 16, 128, 512, 32, _lib.SA2_BF16) == 1
-    assert lib.sa2_uses_mfma(1, 8192, 16, 128, 512, 32, _lib.SA2_F32) == 1      # the fp32 MFMA kernels
+    assert lib.sa2_uses_mfma(1, 8192, 16, 128, 512, 32, _lib.SA2_F32) == 1      # the plane-split kernels
     assert lib.sa2_uses_mfma(1, 8192, 16, 256, 512, 32, _lib.SA2_F32) == 0
     assert lib.sa2_uses_mfma(1, 8192, 16, 256, 512, 32, _lib.SA2_BF16) == 1     # the head_dim 256 MFMA kernels
     assert lib.sa2_uses_mfma(1, 8192, 16, 192, 512, 32, _lib.SA2_BF16) == 0

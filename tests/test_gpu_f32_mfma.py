@@ -86,7 +86,7 @@ def test_forward_backward_vs_oracle(shape):
     want = oracle_all(inp, 16, 16)
     for name in NAMES:
         # (N = 1: dq, dk1, dk2 vanish by cancellation, a relative error of noise says nothing)
-        assert_close_rel(got[name], want[name], 1e-5, name, label="fp32 MFMA shapes" if N > 1 else None)
+        assert_close_rel(got[name], want[name], 1e-5, name, label="fp32 shapes, matrix pipes" if N > 1 else None)
 
 
 @pytest.mark.parametrize("w", [(1, 1), (4, 4), (8, 3), (0, 5), (5, 0), (0, 0), (64, 64), (100, 7), (70, 200), (31, 32),

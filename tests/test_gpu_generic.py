@@ -234,8 +234,7 @@ def test_rowdot():
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("D", [16, 32, 64, 128, 256, 40])
 def test_rowdot_kernels(D, dtype):
-    """The 16-byte-per-lane kernel (16-bit elements, D = 8 << n, aligned rows), the element-wise one
-    (everything else), and views whose rows are not 16-byte aligned."""
+    """The 16-byte-per-lane kernel (rows on the 16-byte grid), the element-wise one (everything else), and views whose rows are not 16-byte aligned."""
     from simplical_attn_amd import simplicial_rowdot
     dev = torch.device("cuda:0")
     g = torch.Generator().manual_seed(D)

@@ -1,5 +1,5 @@
 """Head dims between the kernels' own widths run in the next wider kernel (16-bit tensors other than head_dim 16: on the
-fp32 MFMA kernels), whose columns from head_dim on read as zeros and are not written.  Against the CPU oracle, on views
+plane-split kernels), whose columns from head_dim on read as zeros and are not written.  Against the CPU oracle, on views
 into wider rows whose columns past head_dim hold NaN (a read past a row's end would poison the result), and on
 contiguous tensors with the same bits."""
 import pytest

@@ -273,8 +273,8 @@ def test_packed_projection_views_take_the_mfma_kernels():
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_head_dim_16_is_padded_onto_the_mfma_kernels(dtype):
-    """head_dim 16 (simplicial/test_correctness.py:32): tensors are zero-padded to 32 columns
-    by the host wrapper and run on the MFMA kernels of their element type; results equal those of the MFMA
+    """head_dim 16 (simplicial/test_correctness.py:32) runs in the 32-column kernels of its
+    element type, whose other columns read as zeros; results equal those of the MFMA
     kernels on the hand-padded tensors bit for bit (same scale) and meet the oracle at the type's parity bar."""
     import simplical_attn_amd as sa
     B, N, H, D, w1, w2 = 2, 150, 3, 16, 40, 9

@@ -100,7 +100,7 @@ def test_auto_dispatch_takes_mfma_for_bf16_d64_d128():
     assert lib.sa2_uses_mfma(2, 2048, 8, 64, 512, 32, _lib.SA2_BF16) == 1
     assert lib.sa2_uses_mfma(1, 8192, 16, 128, 512, 32, _lib.SA2_BF16) == 1
     assert lib.sa2_uses_mfma(1, 8192, 16, 128, 512, 32, _lib.SA2_F16) == 1
-    assert lib.sa2_uses_mfma(1, 128, 2, 64, 32, 16, _lib.SA2_F32) == 1      # (the fp32 MFMA kernels)
+    assert lib.sa2_uses_mfma(1, 128, 2, 64, 32, 16, _lib.SA2_F32) == 1      # (the plane-split kernels)
     assert lib.sa2_uses_mfma(1, 128, 2, 256, 32, 16, _lib.SA2_F32) == 0
     assert lib.sa2_uses_mfma(1, 128, 2, 32, 32, 16, _lib.SA2_BF16) == 1
     assert lib.sa2_uses_mfma(1, 128, 2, 48, 32, 16, _lib.SA2_BF16) == 0
@@ -162,7 +162,7 @@ def test_extreme_and_zero_inputs():
 def test_repair_pass_when_logits_outgrow_the_first_reference_point():
     """The fast kernel fixes a unit's softmax reference at its first tile; logits that
     later grow by hundreds of octaves overflow its weights, the block is marked and the
-    repair kernel redoes it with a moving reference.  The result must still match."""
+    second pass redoes it with a moving reference.  The result must still match."""
     B, N, H, D, w1, w2 = 1, 160, 2, 64, 100, 5
     q = torch.full((B, N, H, D), 0.5)
     k2 = torch.full((B, N, H, D), 0.5)
