@@ -94,3 +94,29 @@ def test_backward_of_a_subset_of_the_gradients():
         for need, a, b in zip(needs, part, full):
             assert (a is None) == (not need)
             assert a is None or torch.equal(a.nan_to_num(), b.nan_to_num())
+
+
+def test_captured_step_follows_its_inputs():
+    """A step captured on usual values, replayed on others: the verdict is the device's, at every replay."""
+    import simplical_attn_amd as sa
+    static = _inputs(torch.float32, 64, "")
+
+    def step(x):
+        out, lse = sa.simplicial_forward(*x[:5], 40, 40)
+        return (out, lse, *sa.simplicial_backward(*x[:5], out, lse, x[5], 40, 40))
+
+    step(static)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = step(static)
+    for what in ("NaN value", "", "infinity in a value", ""):
+        new = _inputs(torch.float32, 64, what)
+        for s, n in zip(static, new):
+            s.copy_(n)
+        graph.replay()
+        torch.cuda.synchronize()
+        got = [t.clone() for t in captured]
+        for a, b in zip(got, step(new)):
+            assert torch.equal(a.nan_to_num(7.0, 8.0, 9.0), b.nan_to_num(7.0, 8.0, 9.0)), what
+        assert torch.isfinite(got[2]).all() == (what == "")
