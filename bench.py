@@ -328,7 +328,7 @@ def main():
     ms_per_step = e0.elapsed_time(e1) / args.steps
 
     # ---- the forward's and the backward's share of a step (events inside further steps) ----
-    # Back-to-back forwards draw more power than the step's mix; on some boxes the forward runs up
+    # Back-to-back forwards draw more power than the step's mix; on some machines the forward runs up
     # to 5 % faster between two backwards than in a loop of its own.  Both figures are reported.
     marks = []
     for _ in range(max(5, args.steps)):

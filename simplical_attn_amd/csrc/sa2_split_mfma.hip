@@ -594,6 +594,17 @@ void split_fwd_kernel(Problem p, int nqb, int total) {
     if (!__syncthreads_or(nan || tiny)) return;
     const bool any_nan = __syncthreads_or(nan), any_usual = __syncthreads_or(usual);
     if (!any_nan && any_usual) return;
+    {
+        // (a row whose q holds a NaN is NaN as it stands: a block of such rows, as a run that has diverged sends them, is done)
+        bool q_nan = false;
+        for (int col = 4 * (tid % TPR); io < N && col < p.D; col += 4 * TPR) {
+            const float4 x = cols4<T, PAD>((const EL*)p.q.p + p.q.off(b, io, h), col, p.D);
+            q_nan |= x.x != x.x || x.y != x.y || x.z != x.z || x.w != x.w;
+        }
+        const uint64_t row_lanes = (((uint64_t)1 << TPR) - 1) << (lane / TPR * TPR);
+        const bool row_nan = (__builtin_amdgcn_ballot_w64(q_nan) & row_lanes) != 0;
+        if (!__syncthreads_or(io < N && !row_nan)) return;
+    }
     const int d_lo = round0 * W, d_hi = round1 * W - 1 < w2 ? round1 * W - 1 : w2;
     for (int r0 = 0; r0 < BQ && i0 + r0 < N; r0 += W)
         fma_fwd_rows<typename T::Fma>(p, bh, i0 + r0, d_lo, d_hi, (float*)smem_f, [&](int ir, int ln_r, float m, float l, const float (&acc)[MAXC]) {
@@ -614,8 +625,9 @@ void split_fwd_kernel(Problem p, int nqb, int total) {
 // The row term, and whether the planes cover the operands: they do not where one is infinite or NaN, where products of q
 // and K' or of dO and V' may overflow, and (fp32) where all of a tensor's values in a workgroup's rows are so small, and
 // not zero, that products of them come under 2^-110.  Each workgroup takes a run of consecutive rows and leaves its
-// verdict in guard[blockIdx.x].  The two kernels below run whatever it says; if any is set, split_fma_bwd_kernel computes all
-// gradients again by rows.  Bound by reading the seven tensors once: fp32 B2 H8 N2048 D64 (59 MB) 16 us, the row term alone
+// verdict in guard[blockIdx.x]: 0 covered, 1 not, 2 not but every row has a NaN in q or nothing else in dO, which makes
+// everything that such rows reach NaN as it stands.  The two kernels below run whatever it says; where it is 1, or 2 for some
+// rows only, split_fma_bwd_kernel computes all gradients again by rows (not where a run that has diverged sends nothing but NaN).  Bound by reading the seven tensors once: fp32 B2 H8 N2048 D64 (59 MB) 16 us, the row term alone
 // 9; the launch that looks at the verdicts 5.
 constexpr int GUARD_MOST = 1024, GUARD_ROWS = 64;      // workgroups at most, rows per workgroup at least
 inline int guard_blocks(int64_t rows) {
@@ -634,11 +646,12 @@ __global__ __launch_bounds__(256) void split_guard_kernel(Problem p, int lpr_log
     const int step = 4 << (6 - lpr_log2);
     const int64_t first = (int64_t)blockIdx.x * per_block, last = first + per_block < rows ? first + per_block : rows;
     const Tensor* const set[SETS] = {&p.dout, &p.q, &p.k2, &p.v2, &p.k1, &p.v1, &p.out};  // the first four enter products
-    bool bad = false;
+    bool bad = false, all_nan = true;
     unsigned seen = 0;                       // bit t: tensor t has a usual value here, bit 8 + t: one that is small but not zero
     for (int64_t r0 = first; r0 < last; r0 += step) {
         const int64_t row = r0 + ((int)(threadIdx.x >> 6) << (6 - lpr_log2)) + (lane >> lpr_log2);
         float s = 0.f;
+        bool q_nan = false, do_some = false;
         if (row < last && sub * PER < p.D) {
             const int i = (int)(row % p.N), bh = (int)(row / p.N), b = bh / p.H, h = bh - b * p.H;
             union { uint4 v; typename T::Fma e[PER]; } x[SETS];
@@ -660,6 +673,8 @@ __global__ __launch_bounds__(256) void split_guard_kernel(Problem p, int lpr_log
                 for (int e = 0; e < PER; ++e) {
                     const float a = fabsf(to_float(x[t].e[e]));
                     bad |= !(a < INFINITY);
+                    if (t == 0) do_some |= a == a;
+                    if (t == 1) q_nan |= a != a;
                     most = fmaxf(most, a);
                 }
                 if (t < 4) bad |= most >= GUARD_HIGH;
@@ -676,6 +691,9 @@ __global__ __launch_bounds__(256) void split_guard_kernel(Problem p, int lpr_log
         for (int off = lpr >> 1; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
         bad |= s != s;
         if (row < last && sub == 0) p.dsum[row] = s;
+        const uint64_t row_lanes = (lpr < 64 ? ((uint64_t)1 << lpr) - 1 : ~(uint64_t)0) << (lane & ~(lpr - 1));
+        const bool row_nan = (__builtin_amdgcn_ballot_w64(q_nan) & row_lanes) != 0 || (__builtin_amdgcn_ballot_w64(do_some) & row_lanes) == 0;
+        all_nan &= row >= last || row_nan;
     }
     if constexpr (F32) {
         for (int t = 0; t < 6; ++t) {
@@ -683,13 +701,14 @@ __global__ __launch_bounds__(256) void split_guard_kernel(Problem p, int lpr_log
             bad |= small && !usual;
         }
     }
-    const int verdict = __syncthreads_or(bad);
-    if (threadIdx.x == 0) guard[blockIdx.x] = verdict;
+    const bool verdict = __syncthreads_or(bad), some = __syncthreads_or(!all_nan);
+    if (threadIdx.x == 0) guard[blockIdx.x] = verdict ? (some ? 1 : 2) : 0;
 }
 __device__ __forceinline__ bool guarded(const int* __restrict__ guard, int n) {
-    int any = 0;
-    for (int c = threadIdx.x; c < n; c += blockDim.x) any |= guard[c];
-    return __syncthreads_or(any);
+    int seen = 0;
+    for (int c = threadIdx.x; c < n; c += blockDim.x) seen |= 1 << guard[c];
+    if (!__syncthreads_or(seen & 6)) return false;
+    return __syncthreads_or(seen & 3);                       // (verdicts of 2 throughout: nothing to do)
 }
 // All gradients by rows, where the guard says so (launched last: it overwrites what the sums left)
 constexpr int FMA_ROWS = 4, FMA_BLOCKS = 512;

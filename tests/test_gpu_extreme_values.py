@@ -26,6 +26,12 @@ def _inputs(dtype, D, what):
         x[3][:, 90] = nan
     elif what == "NaN query":
         x[0][:, 90, :, 1] = nan
+    elif what == "NaN in every query":
+        x[0][:, :, :, 2] = nan
+    elif what == "nothing but NaN in the gradient":
+        x[5][:] = nan
+    elif what == "NaN in the queries of one head":
+        x[0][:, :, 0, 2] = nan
     elif what == "infinity in V'":
         x[4][:, 90, :, 0] = inf
     elif what == "mask":
@@ -54,7 +60,7 @@ def _same(got, want, bar, name):
     assert diff <= bar * size, (name, diff, size)
 
 
-FORWARD = ["infinity in a value", "minus infinity in a key", "NaN value", "NaN query", "infinity in V'", "mask", "small values", "small keys"]
+FORWARD = ["NaN in every query", "NaN in the queries of one head", "infinity in a value", "minus infinity in a key", "NaN value", "NaN query", "infinity in V'", "mask", "small values", "small keys"]
 
 
 def _cases(kinds):         # (the small tensors are an fp32 range)
@@ -70,7 +76,7 @@ def test_forward(dtype, D, w2, what):
     _same(got[1], want[1], 1e-6, "lse")
 
 
-BACKWARD = FORWARD + ["NaN gradient", "small gradient"]
+BACKWARD = FORWARD + ["nothing but NaN in the gradient", "NaN gradient", "small gradient"]
 
 
 @pytest.mark.parametrize("dtype,D,w2,what", _cases(BACKWARD) + [(torch.float32, 64, 20, "product above the range")])
