@@ -230,11 +230,11 @@ __device__ __forceinline__ bf16x8 lead_planes(float x, float rest) {
     r.u[0] = w[0]; r.u[1] = w[1]; r.u[2] = w[2]; r.u[3] = 0;
     return r.v;
 }
-__device__ __forceinline__ bf16x8 lse_planes(float lse) {
+__device__ __forceinline__ float lse_rest(float lse, float x) {        // what x = LSE*log2(e) lost when it was rounded
     constexpr float LOG2E_REST = 1.9259629911e-8f;       // log2(e) - LOG2E
-    const float x = lse * LOG2E;
-    return lead_planes(x, fmaf(lse, LOG2E, -x) + lse * LOG2E_REST);
+    return fmaf(lse, LOG2E, -x) + lse * LOG2E_REST;
 }
+__device__ __forceinline__ bf16x8 lse_planes(float lse) { return lead_planes(lse * LOG2E, lse_rest(lse, lse * LOG2E)); }
 __device__ __forceinline__ bf16x8 lead_ones(int hf) {
     uint32_t w = hf ? 0u : 0x3f803f80u;
     asm volatile("" : "+v"(w));                          // (made where it is used: four registers less to keep)
@@ -1074,7 +1074,9 @@ void split_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __res
     // ---- forming a unit: Q~ and dO~ tiles (32 rows), LSE and D of its queries ----
     constexpr int ALL = 32 * D / 4, KR = (ALL + XT - 1) / XT;      // groups of four columns: of a tile, per thread
     typename T::Raw fq[KR], fk[KR], fd[KR], fv[KR];
-    float f_lse = 0.f, f_dsum = 0.f;
+    float f_lead = 0.f;                       // LSE (threads 0-31) or D (32-63) of a query
+    // (LSE and D of a unit by the two halves of wavefront 0: by one half, one after the other, the kernel took 4 % longer at
+    // 128 columns, where that wavefront is on the step's critical path)
     auto fetch_unit = [&](int ib, int delta) {
 #pragma unroll
         for (int u = 0; u < KR; ++u) {
@@ -1089,11 +1091,10 @@ void split_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __res
             fd[u] = raw4<T, PAD>(dop + (int64_t)i * p.dout.sn, col * 4, p.D);
             fv[u] = raw4<T, PAD>(v2p + (int64_t)k * p.v2.sn, col * 4, p.D);
         }
-        if (tid < 32) {
-            int i = ib * BQ + tid;
+        if (tid < 64) {
+            int i = ib * BQ + ln;
             i = i < N ? i : N - 1;
-            f_lse = p.lse[(int64_t)bh * N + i];
-            f_dsum = p.dsum[(int64_t)bh * N + i];
+            f_lead = (hf ? p.dsum : p.lse)[(int64_t)bh * N + i];
         }
     };
     auto store_unit = [&](int buf) {
@@ -1111,9 +1112,9 @@ void split_kv_kernel(Problem p, int njb, int total, int nsplit_arg, float* __res
             store_planes<3, false>(qt, Qs + row * C::RS + col * 4, C::PLANE);
             store_planes<3, false>(dt, Ds + row * C::RS + col * 4, C::PLANE);
         }
-        if (tid < 32) {
-            *(bf16x8*)(lead_s + (buf * 64 + tid) * 16) = lse_planes(f_lse);
-            *(bf16x8*)(lead_s + (buf * 64 + 32 + tid) * 16) = lead_planes(f_dsum, 0.f);
+        if (tid < 64) {
+            const float x = hf ? f_lead : f_lead * LOG2E;
+            *(bf16x8*)(lead_s + (buf * 64 + tid) * 16) = lead_planes(x, hf ? 0.f : lse_rest(f_lead, x));
         }
     };
 
