@@ -702,7 +702,7 @@ __global__ __launch_bounds__(256) void split_guard_kernel(Problem p, int lpr_log
         }
     }
     const bool verdict = __syncthreads_or(bad), some = __syncthreads_or(!all_nan);
-    if (threadIdx.x == 0) guard[blockIdx.x] = verdict ? (some ? 1 : 2) : 0;
+    if (threadIdx.x == 0) guard[blockIdx.x] = first >= last ? 3 : verdict ? (some ? 1 : 2) : 0;      // (3: no rows, no say)
 }
 __device__ __forceinline__ bool guarded(const int* __restrict__ guard, int n) {
     int seen = 0;
