@@ -144,8 +144,8 @@ int sa2_backward(const void* q, const void* k1, const void* k2, const void* v1, 
  * sa2_bwd_workspace_bytes(...) <= SA2_STATIC_WORKSPACE_BYTES it runs sa2_backward's kernels
  * with the same results, bit for bit.  Otherwise it runs them with fewer partial sums (added
  * in another order), and where even the fewest do not fit and the head_dim has no kernels of
- * its own (see sa2_uses_mfma), or the fp32 K' window would fit in one piece, the fp32-FMA
- * kernels.  A problem that fits in none of these ways
+ * its own (see sa2_uses_mfma; fp32 96 counts as one without), or the fp32 K' window would
+ * fit in one piece, the fp32-FMA kernels.  A problem that fits in none of these ways
  * returns SA2_ERR_STATIC_WORKSPACE and launches nothing.  All calls on one GPU share the
  * array (the kernels overwrite what they read from it, so nothing needs clearing between
  * calls): calls that overlap on one GPU - different streams, or host threads - race;

@@ -145,9 +145,9 @@ size_t bwd_need(int B, int N, int H, int D, int w1, int w2, int dtype, unsigned 
 }
 
 // How sa2_backward_static_workspace takes a problem into its array (inclusive reaches w1 and w2): as sa2_backward does
-// where that fits, else with plans that cut less, else - for head dims without kernels of their own, and for fp32 K'
-// windows that fit in one piece but not as the segments the kernels' LDS asks for - on the fp32 FMA kernels, which need
-// the row term only.  false: refused.
+// where that fits, else with plans that cut less, else on the fp32 FMA kernels, which need the row term only: head dims
+// without kernels of their own and fp32 96, which ran on them before, and fp32 K' windows that fit in one piece but not
+// as the segments the kernels' LDS asks for.  false: refused.
 bool static_plan(int B, int N, int H, int D, int w1, int w2, int dtype, unsigned* flags, size_t* room) {
     const size_t all = SA2_STATIC_WORKSPACE_BYTES;
     auto fits = [&] {
