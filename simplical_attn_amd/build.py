@@ -12,6 +12,8 @@ import os
 import subprocess
 import sys
 
+from . import listing_check
+
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
 CSRC = os.path.join(PKG, "csrc")
@@ -30,6 +32,8 @@ FLAGS = [
     "-Wno-unused-command-line-argument",
     "-I", os.path.join(ROOT, "include"), "-I", CSRC,
 ]
+# sources with hand-placed MFMAs -> their kernels, whose code is checked (see listing_check.py)
+HAND_PLACED = {"sa2_mfma_bwd_kv_bf16.hip": "mfma_bwd_kv_kernel", "sa2_mfma_bwd_kv_fp16.hip": "mfma_bwd_kv_kernel"}
 
 
 def _compile(src, extra):
@@ -40,6 +44,9 @@ def _compile(src, extra):
     err = "\n".join(l for l in res.stderr.splitlines() if noise not in l)
     if res.returncode != 0:
         raise RuntimeError("hipcc failed on %s:\n%s" % (src, err))
+    kernels = HAND_PLACED.get(os.path.basename(src))
+    if kernels:
+        listing_check.check_object(obj, kernels)
     return obj, err
 
 

@@ -88,12 +88,12 @@ bool allow_full_lds(const void* kernel);
 // smaller than the chip, or its last wave nearly empty, or its workgroups uneven (short ones at the ends of the
 // sequence), the plans below cut the work of a workgroup into shares with fp32 partial sums, which cost their write and
 // read (2.5 MB per unit of time, a sweep step of about 1 us) and a summation launch.  The constants are the ones whose
-// choices lost least against the best of up to sixteen measured cuts at nineteen sizes (1.0 % for the K-side kernel,
-// 2.6 % for the K'-side one).  All plans depend on the problem's sizes only.
+// choices lost least against the best of up to sixteen measured cuts (2.6 % on average for the K'-side kernel at nineteen
+// sizes; the 16-bit K-side kernel has its own, see kv_plan).  All plans depend on the problem's sizes only.
 constexpr int CUS = 256;
-inline double grid_time(int64_t workgroups, double longest, double mean) {
+inline double grid_time(int64_t workgroups, double longest, double mean, double tail = 0.7) {
     const int64_t waves = workgroups / CUS;
-    const double t = (double)waves * mean + (workgroups - waves * CUS > 2 ? 0.7 * longest + 0.3 * mean : 0.0);
+    const double t = (double)waves * mean + (workgroups - waves * CUS > 2 ? tail * longest + (1 - tail) * mean : 0.0);
     return t > longest ? t : longest;
 }
 // mean over the sequence of min(i, w) / w

@@ -1,0 +1,8 @@
+// The K-side backward kernel for bf16 tensors.
+#include "sa2_mfma_bwd_kv.h"
+
+namespace sa2 {
+
+int launch_mfma_bwd_kv_bf16(const Problem& p, int kb, int nsplit, hipStream_t st, BwdSums* sums) { return launch_kv<ElemBF16>(p, kb, nsplit, st, sums); }
+
+}  // namespace sa2
