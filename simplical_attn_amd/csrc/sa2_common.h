@@ -91,9 +91,9 @@ bool allow_full_lds(const void* kernel);
 // choices lost least against the best of up to sixteen measured cuts (2.6 % on average for the K'-side kernel at nineteen
 // sizes; the 16-bit K-side kernel has its own, see kv_plan).  All plans depend on the problem's sizes only.
 constexpr int CUS = 256;
-inline double grid_time(int64_t workgroups, double longest, double mean, double tail = 0.7) {
+inline double grid_time(int64_t workgroups, double longest, double mean) {
     const int64_t waves = workgroups / CUS;
-    const double t = (double)waves * mean + (workgroups - waves * CUS > 2 ? tail * longest + (1 - tail) * mean : 0.0);
+    const double t = (double)waves * mean + (workgroups - waves * CUS > 2 ? 0.7 * longest + 0.3 * mean : 0.0);
     return t > longest ? t : longest;
 }
 // mean over the sequence of min(i, w) / w

@@ -9,47 +9,25 @@
 // Transposed operands come from the same unit tiles through ds_read_b64_tr_b16; the tiles are laid out in row groups so
 // that both kinds of read are free of bank conflicts.  Every output element has one writer and a fixed summation order.
 //
-// One wavefront per SIMD with all 512 registers does A, B and C itself, so it hides its latencies itself: B(t) and the
-// forming of unit t+2 stand between the MFMAs of A(t+1) and C(t), operand reads eight MFMAs ahead of their use, in an order
-// that the source fixes (a sched_barrier behind every MFMA).  What this costs and where it ends was measured on the
-// instructions alone: an MFMA takes 33 cycles, under which five more vector instructions are free; a read of LDS takes 4 to 7
-// of its own, right behind an MFMA (14 behind vector instructions), and an s_nop up to 9, which is why no instruction here
-// reads the result of an exponential or the operand of an MFMA just written.
+// One wavefront per SIMD with all 512 registers does A, B and C itself (sa2_mfma_lone.h): B(t) and the forming of unit t+2
+// stand between the MFMAs of A(t+1) and C(t), operand reads eight MFMAs ahead of their use.
 // The arrangement before it (two wavefronts per SIMD, one with S, P and dV, one with dP, dS and dK, P handed over in LDS, a
 // barrier per unit) ran matrix pipe, vector ALU and LDS one after the other, 2500 cycles per unit of 1024 MFMA cycles; here
-// it is 1700 to 1800.  With the row-term kernel, us: B2 H8 N2048 D64 w 512/32 458 -> 315, B1 H16 N8192 D128 w 512/32
-// 2714 -> 2247 (there the board's power is the next limit).
+// it is 1700 to 1800.  With the row-term kernel, us: B2 H8 N2048 D64 w 512/32 458 -> 309, B1 H16 N8192 D128 w 512/32
+// 2714 -> 2260 (there the board's power is the next limit).
 //
 // Small grids (fewer workgroups than the chip holds) split a key block's stream of units over up to sixteen workgroups
 // (shares of whole units, at least four each); each writes its fp32 partial dK and dV to the workspace and bwd_sum_kernel
 // adds the partials in split order.
 #pragma once
 
-#include <type_traits>
-
-#include "sa2_mfma_common.h"
+#include "sa2_mfma_lone.h"
 
 namespace sa2 {
 namespace {
 
 constexpr int VW = 4;                  // wavefronts per workgroup, one per SIMD
 constexpr int VT = VW * 64;            // threads per workgroup
-
-template <int N, int I = 0, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<N, I + 1>(f);
-    }
-}
-
-template <class E>
-__device__ __forceinline__ uint32_t pack2(float a, float b) {
-    typedef float f2 __attribute__((ext_vector_type(2)));
-    union { typename E::x2 h; uint32_t u; } v;
-    v.h = __builtin_convertvector((f2){a, b}, typename E::x2);
-    return v.u;
-}
 
 // KB: 32-row blocks of K/V rows per wavefront
 template <int D, int KB>
@@ -78,62 +56,6 @@ struct KvCfg {
     static constexpr int max_segment() { return (int)((LDS_LIMIT - BASE_BYTES) / (2 * D * 2)) / RPW * RPW - BQ - RPW; }
 };
 
-// Accumulation registers 0 .. 191 belong to the kernel, not to the compiler: the sums that live through the kernel and the
-// resident operands are named by number in the instructions below, and each of these says that it destroys them all, so
-// that nothing else is ever kept there.  (Left to the compiler, beside 300 other registers of the sweep, sums and operands
-// move between the two files or to scratch memory in every step.)  Their order: dV^T tiles, dK^T tiles, K operands, V operands.
-#define KV_SUMS_AND_OPERANDS \
-    "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", "a10", "a11", "a12", "a13", "a14", "a15", \
-    "a16", "a17", "a18", "a19", "a20", "a21", "a22", "a23", "a24", "a25", "a26", "a27", "a28", "a29", "a30", "a31", \
-    "a32", "a33", "a34", "a35", "a36", "a37", "a38", "a39", "a40", "a41", "a42", "a43", "a44", "a45", "a46", "a47", \
-    "a48", "a49", "a50", "a51", "a52", "a53", "a54", "a55", "a56", "a57", "a58", "a59", "a60", "a61", "a62", "a63", \
-    "a64", "a65", "a66", "a67", "a68", "a69", "a70", "a71", "a72", "a73", "a74", "a75", "a76", "a77", "a78", "a79", \
-    "a80", "a81", "a82", "a83", "a84", "a85", "a86", "a87", "a88", "a89", "a90", "a91", "a92", "a93", "a94", "a95", \
-    "a96", "a97", "a98", "a99", "a100", "a101", "a102", "a103", "a104", "a105", "a106", "a107", "a108", "a109", "a110", "a111", \
-    "a112", "a113", "a114", "a115", "a116", "a117", "a118", "a119", "a120", "a121", "a122", "a123", "a124", "a125", "a126", "a127", \
-    "a128", "a129", "a130", "a131", "a132", "a133", "a134", "a135", "a136", "a137", "a138", "a139", "a140", "a141", "a142", "a143", \
-    "a144", "a145", "a146", "a147", "a148", "a149", "a150", "a151", "a152", "a153", "a154", "a155", "a156", "a157", "a158", "a159", \
-    "a160", "a161", "a162", "a163", "a164", "a165", "a166", "a167", "a168", "a169", "a170", "a171", "a172", "a173", "a174", "a175", \
-    "a176", "a177", "a178", "a179", "a180", "a181", "a182", "a183", "a184", "a185", "a186", "a187", "a188", "a189", "a190", "a191"
-// d = a * operand B + c, d += a * operand B: tiles in vector registers, whose first reader comes at least four MFMAs later
-template <int B, class X8>
-__device__ __forceinline__ void tile_start(floatx16& d, const X8& a, const floatx16& c) {
-    if constexpr (std::is_same<X8, bf16x8>::value)
-        asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, a[%3:%4], %2" : "=&v"(d) : "v"(a), "v"(c), "n"(B), "n"(B + 3) : KV_SUMS_AND_OPERANDS);
-    else asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, a[%3:%4], %2" : "=&v"(d) : "v"(a), "v"(c), "n"(B), "n"(B + 3) : KV_SUMS_AND_OPERANDS);
-}
-template <int B, class X8>
-__device__ __forceinline__ void tile_more(floatx16& d, const X8& a) {
-    if constexpr (std::is_same<X8, bf16x8>::value)
-        asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, a[%2:%3], %0" : "+v"(d) : "v"(a), "n"(B), "n"(B + 3) : KV_SUMS_AND_OPERANDS);
-    else asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, a[%2:%3], %0" : "+v"(d) : "v"(a), "n"(B), "n"(B + 3) : KV_SUMS_AND_OPERANDS);
-}
-// sum S += a * b
-template <int S, class X8>
-__device__ __forceinline__ void sum_more(const X8& a, const X8& b) {
-    if constexpr (std::is_same<X8, bf16x8>::value)
-        asm volatile("v_mfma_f32_32x32x16_bf16 a[%2:%3], %0, %1, a[%2:%3]" ::"v"(a), "v"(b), "n"(S), "n"(S + 15) : KV_SUMS_AND_OPERANDS);
-    else asm volatile("v_mfma_f32_32x32x16_f16 a[%2:%3], %0, %1, a[%2:%3]" ::"v"(a), "v"(b), "n"(S), "n"(S + 15) : KV_SUMS_AND_OPERANDS);
-}
-// (a value that is read between two of these instructions only could still be given one of the registers)
-__device__ __forceinline__ void keep_out() { asm volatile("" ::: KV_SUMS_AND_OPERANDS); }
-template <int R>
-__device__ __forceinline__ void set_reg(uint32_t x) {
-    asm volatile("v_accvgpr_write_b32 a[%1:%1], %0" ::"v"(x), "n"(R) : KV_SUMS_AND_OPERANDS);
-}
-template <int R>
-__device__ __forceinline__ float get_reg() {
-    float x;
-    asm volatile("v_accvgpr_read_b32 %0, a[%1:%1]" : "=v"(x) : "n"(R) : KV_SUMS_AND_OPERANDS);
-    return x;
-}
-
-// 16 bytes per lane from global memory straight to LDS, lane L to `to` + 16 * L.  Opaque: the compiler would wait for it
-// before every read of LDS.
-__device__ __forceinline__ void lds_request(const void* src, uint32_t to) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(__builtin_amdgcn_readfirstlane(to)), "v"(src) : "memory");
-}
-
 // BIAS = false: k2_bias and v2_bias are both zero (the reference's default), the adds drop out.
 // nsplit > 1: the workgroup takes the sp-th share of the key block's units and writes fp32 partial sums to `part`
 // ([2][nsplit][B*H][N][D]: dK before its scale, then dV).
@@ -145,6 +67,7 @@ __global__ __launch_bounds__(VT) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit, float* __restrict__ part, int ws_arg) {
     typedef typename E::x8 X8;
     using C = KvCfg<D, KB>;
+    using L = Lone<false>;
     constexpr int VJ = C::VJ, DK = C::DK, DT = C::DT, NCH = C::NCH, RPW = C::RPW;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     const int N = p.N, w1 = p.w1, w2 = p.w2;
@@ -181,28 +104,6 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit, float* __rest
     // registers (see above) of the sums and of the resident operands
     constexpr int DV0 = 0, DK0 = KB * DT * 16, K0 = 2 * KB * DT * 16, V0 = K0 + KB * DK * 4;
     static_assert(V0 + KB * DK * 4 <= 192, "");
-    static_for<K0>([&](auto X) __attribute__((always_inline)) { set_reg<decltype(X)::value>(0u); });
-    {
-        uint4 kr[KB][DK], vr[KB][DK];
-#pragma unroll
-        for (int sb = 0; sb < KB; ++sb) {
-            const int j = jw + 32 * sb + ln, jc = j < N ? j : N - 1;
-            const uint16_t* ks = (const uint16_t*)p.k1.p + p.k1.off(b, jc, h);
-            const uint16_t* vs = (const uint16_t*)p.v1.p + p.v1.off(b, jc, h);
-#pragma unroll
-            for (int kk = 0; kk < DK; ++kk) {
-                kr[sb][kk] = load_cols8<PAD>(ks, kk * 16 + hf * 8, p.D);
-                vr[sb][kk] = load_cols8<PAD>(vs, kk * 16 + hf * 8, p.D);
-            }
-        }
-        static_for<KB * DK>([&](auto X) __attribute__((always_inline)) {
-            constexpr int x = decltype(X)::value;
-            const uint4 k = kr[x / DK][x % DK], v = vr[x / DK][x % DK];
-            set_reg<K0 + 4 * x>(k.x); set_reg<K0 + 4 * x + 1>(k.y); set_reg<K0 + 4 * x + 2>(k.z); set_reg<K0 + 4 * x + 3>(k.w);
-            set_reg<V0 + 4 * x>(v.x); set_reg<V0 + 4 * x + 1>(v.y); set_reg<V0 + 4 * x + 2>(v.z); set_reg<V0 + 4 * x + 3>(v.w);
-        });
-    }
-
     const float qscale = p.scale * LOG2E;
     const int j_last = (j0 + VJ - 1 < N ? j0 + VJ - 1 : N - 1);
     const int i_max = (int)((int64_t)j_last + w1 < N - 1 ? j_last + w1 : N - 1);
@@ -326,15 +227,14 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit, float* __rest
     const uint32_t form_lane = (uint32_t)(wave * C::GROUP + lane * 16);
     constexpr uint32_t KKB = 32 * RPW, DTB = 64 * RPW;
 
-    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
     u4 kx[NCH], vx[NCH];
     u4 fw[NCH][2];                               // Q~ and dO~ chunks of the unit in work
     auto form_read = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
             const uint32_t a = f_lane + f_at[c] / RPW * 1024 + f_at[c] % RPW * 16;
-            kx[c] = *(const u4 __attribute__((address_space(3)))*)(uintptr_t)a;
-            vx[c] = *(const u4 __attribute__((address_space(3)))*)(uintptr_t)(a + side);
+            kx[c] = *(lds_u4)(uintptr_t)a;
+            vx[c] = *(lds_u4)(uintptr_t)(a + side);
         }
     };
     // item f: word f % 8 / 2 of Q~ or dO~ (in turn) of chunk f / 8
@@ -427,16 +327,16 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit, float* __rest
     auto a_mfma = [&](auto XP, auto SB, auto I) __attribute__((always_inline)) {
         constexpr int x = decltype(XP)::value, sb = decltype(SB)::value, i = decltype(I)::value, kk = i % DK;
         constexpr int at = (sb * DK + kk) * 4;
-        if constexpr (i == 0) tile_start<K0 + at>(s[x], qa[0], nl[sb]);
-        else if constexpr (i < DK) tile_more<K0 + at>(s[x], qa[kk]);
-        else if constexpr (i == DK) tile_start<V0 + at>(dp[x], da[0], nd);
-        else tile_more<V0 + at>(dp[x], da[kk]);
+        if constexpr (i == 0) L::tile_start<K0 + at>(s[x], qa[0], nl[sb]);
+        else if constexpr (i < DK) L::tile_more<K0 + at>(s[x], qa[kk]);
+        else if constexpr (i == DK) L::tile_start<V0 + at>(dp[x], da[0], nd);
+        else L::tile_more<V0 + at>(dp[x], da[kk]);
     };
     auto c_mfma = [&](auto XP, auto SB, auto I) __attribute__((always_inline)) {
         constexpr int x = decltype(XP)::value, sb = decltype(SB)::value, i = decltype(I)::value;
         constexpr int which = i / (2 * DT), ks = i / DT % 2, dt = i % DT;
-        if constexpr (which == 0) sum_more<DV0 + (sb * DT + dt) * 16>(dot[dt][ks], __builtin_bit_cast(X8, pw[x][ks]));
-        else sum_more<DK0 + (sb * DT + dt) * 16>(qt[dt][ks], __builtin_bit_cast(X8, dw[x][ks]));
+        if constexpr (which == 0) L::sum_more<DV0 + (sb * DT + dt) * 16>(dot[dt][ks], __builtin_bit_cast(X8, pw[x][ks]));
+        else L::sum_more<DK0 + (sb * DT + dt) * 16>(qt[dt][ks], __builtin_bit_cast(X8, dw[x][ks]));
     };
     // (an exponential's result may not be read by the next instruction: a pair is rounded behind the next pair's exponentials)
     auto round_p = [&](auto XP, auto I) __attribute__((always_inline)) {
@@ -455,13 +355,6 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit, float* __rest
         dw[x][ks][t] = pack2<E>(s[x][e] * dp[x][e], s[x][e + 1] * dp[x][e + 1]);
     };
     auto unit_barrier = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-#define KVC(n) std::integral_constant<int, (n)>{}
-    // runs f for the items of N that fall to slot SLOT of SLOTS
-    auto deal = [&](auto N, auto SLOT, auto SLOTS, auto f) __attribute__((always_inline)) {
-        constexpr int n = decltype(N)::value, s0 = decltype(SLOT)::value, ss = decltype(SLOTS)::value;
-        constexpr int a = s0 < 0 ? 0 : s0 < ss ? s0 : ss, z = s0 + 1 < 0 ? 0 : s0 + 1 < ss ? s0 + 1 : ss, lo = n * a / ss, hi = n * z / ss;
-        static_for<hi - lo>([&](auto Y) __attribute__((always_inline)) { f(std::integral_constant<int, lo + decltype(Y)::value>{}); });
-    };
     // One K block per unit.  A(t), under the forming of unit t+2; then C(t-1), whose four groups of MFMAs (dV^T and dK^T, each
     // from the rows' first and second half) free the halves of P and dS one after the other for B(t).
     constexpr int BAR = LONG ? 2 * DT : 0;                    // MFMA of phase C that the unit's barrier stands before
@@ -470,36 +363,36 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit, float* __rest
         form_read();
         static_for<NE>([&](auto I) __attribute__((always_inline)) {
             constexpr int i = decltype(I)::value;
-            a_mfma(KVC(0), KVC(0), I);
-            if constexpr (LONG && i < DK) read_row(KVC(1), I, ua);
+            a_mfma(LONE_C(0), LONE_C(0), I);
+            if constexpr (LONG && i < DK) read_row(LONE_C(1), I, ua);
             if constexpr (CC) {
-                if constexpr (LONG) deal(KVC(12), KVC(i - 4), KVC(12), [&](auto X) __attribute__((always_inline)) { read_column(X, uc); });
-                else deal(KVC(4 * DT), I, KVC(NE - 2), [&](auto X) __attribute__((always_inline)) { read_column(X, uc); });
+                if constexpr (LONG) deal<12, i - 4, 12>([&](auto X) __attribute__((always_inline)) { read_column(X, uc); });
+                else deal<4 * DT, decltype(I)::value, NE - 2>([&](auto X) __attribute__((always_inline)) { read_column(X, uc); });
             }
-            deal(KVC(NF), I, KVC(NE + DT), form_item);
+            deal<NF, decltype(I)::value, NE + DT>(form_item);
             __builtin_amdgcn_sched_barrier(0);
         });
         static_for<NE>([&](auto I) __attribute__((always_inline)) {
             constexpr int i = decltype(I)::value, group = i / DT;
             if constexpr (i == BAR) unit_barrier();
             if constexpr (CC) {
-                c_mfma(KVC(0), KVC(0), I);
-                if constexpr (LONG && i < 4) read_column(KVC(12 + i), uc);
+                c_mfma(LONE_C(0), LONE_C(0), I);
+                if constexpr (LONG && i < 4) read_column(LONE_C(12 + i), uc);
             }
-            if constexpr (LONG && i >= BAR) read_row(KVC(0), KVC(i - BAR), ub);
-            if constexpr (!LONG) read_row(KVC(i / DK), KVC(i % DK), ub);
-            if constexpr (group == 0) deal(KVC(NF), KVC(NE + i), KVC(NE + DT), form_item);
-            deal(KVC(2 * NCH), KVC(i - 2 * DT), KVC(DT), [&](auto X) __attribute__((always_inline)) { form_store(X, uc); });
-            if constexpr (group == 1 || group == 2) deal(KVC(8), KVC(i - DT), KVC(2 * DT), [&](auto X) __attribute__((always_inline)) { p_item(KVC(0), X); });
-            if constexpr (group == 3) deal(KVC(4), KVC(i - 3 * DT), KVC(DT), [&](auto X) __attribute__((always_inline)) { ds_item(KVC(0), X); });
+            if constexpr (LONG && i >= BAR) read_row(LONE_C(0), LONE_C(i - BAR), ub);
+            if constexpr (!LONG) read_row(LONE_C(i / DK), LONE_C(i % DK), ub);
+            if constexpr (group == 0) deal<NF, NE + i, NE + DT>(form_item);
+            deal<2 * NCH, i - 2 * DT, DT>([&](auto X) __attribute__((always_inline)) { form_store(X, uc); });
+            if constexpr (group == 1 || group == 2) deal<8, i - DT, 2 * DT>([&](auto X) __attribute__((always_inline)) { p_item(LONE_C(0), X); });
+            if constexpr (group == 3) deal<4, i - 3 * DT, DT>([&](auto X) __attribute__((always_inline)) { ds_item(LONE_C(0), X); });
             __builtin_amdgcn_sched_barrier(0);
         });
-        static_for<4>([&](auto X) __attribute__((always_inline)) { ds_item(KVC(0), KVC(4 + decltype(X)::value)); });
+        static_for<4>([&](auto X) __attribute__((always_inline)) { ds_item(LONE_C(0), LONE_C(4 + decltype(X)::value)); });
         aim_next();
     };
     auto single_last = [&]() __attribute__((always_inline)) {                       // C of unit t-1 alone
         static_for<4 * DT>([&](auto X) __attribute__((always_inline)) { read_column(X, uc); });
-        static_for<NE>([&](auto I) __attribute__((always_inline)) { c_mfma(KVC(0), KVC(0), I); });
+        static_for<NE>([&](auto I) __attribute__((always_inline)) { c_mfma(LONE_C(0), LONE_C(0), I); });
     };
     // Two K blocks per unit: A(t, 0), C(t-1, 1), A(t, 1), C(t, 0); the transposed operands of unit t serve C(t, 0) and C(t, 1).
     // The weights and dS of a block are formed from the end of its phase A to the beginning of its phase C, the unit t+2 throughout.
@@ -507,58 +400,73 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit, float* __rest
         constexpr bool CC = decltype(DO_C)::value;
         constexpr int EARLY = 6;                              // weights (of eight pairs) formed before the other block's phase A
         auto later = [&](auto XP, auto I) __attribute__((always_inline)) {
-            deal(KVC(16 - EARLY), I, KVC(NE), [&](auto X) __attribute__((always_inline)) {
+            deal<16 - EARLY, decltype(I)::value, NE>([&](auto X) __attribute__((always_inline)) {
                 constexpr int x = decltype(X)::value;
-                if constexpr (x < 8 - EARLY) p_item(XP, KVC(EARLY + x));
-                else ds_item(XP, KVC(x - (8 - EARLY)));
+                if constexpr (x < 8 - EARLY) p_item(XP, LONE_C(EARLY + x));
+                else ds_item(XP, LONE_C(x - (8 - EARLY)));
             });
         };
         auto early = [&](auto XP, auto I) __attribute__((always_inline)) {
-            deal(KVC(EARLY), I, KVC(NE), [&](auto X) __attribute__((always_inline)) { p_item(XP, X); });
+            deal<EARLY, decltype(I)::value, NE>([&](auto X) __attribute__((always_inline)) { p_item(XP, X); });
         };
-        auto form = [&](auto PHASE, auto I) __attribute__((always_inline)) { deal(KVC(NF), KVC(decltype(PHASE)::value * NE + decltype(I)::value), KVC(4 * NE - 2), form_item); };
+        auto form = [&](auto PHASE, auto I) __attribute__((always_inline)) { deal<NF, decltype(PHASE)::value * NE + decltype(I)::value, 4 * NE - 2>(form_item); };
         form_read();
         static_for<NE>([&](auto I) __attribute__((always_inline)) {
-            a_mfma(KVC(0), KVC(0), I);
-            if constexpr (CC) later(KVC(1), I);
-            form(KVC(0), I);
+            a_mfma(LONE_C(0), LONE_C(0), I);
+            if constexpr (CC) later(LONE_C(1), I);
+            form(LONE_C(0), I);
             __builtin_amdgcn_sched_barrier(0);
         });
         static_for<NE>([&](auto I) __attribute__((always_inline)) {
-            if constexpr (CC) c_mfma(KVC(1), KVC(KB - 1), I);
-            early(KVC(0), I);
-            form(KVC(1), I);
+            if constexpr (CC) c_mfma(LONE_C(1), LONE_C(KB - 1), I);
+            early(LONE_C(0), I);
+            form(LONE_C(1), I);
             __builtin_amdgcn_sched_barrier(0);
         });
         static_for<NE>([&](auto I) __attribute__((always_inline)) {
-            a_mfma(KVC(1), KVC(KB - 1), I);
-            deal(KVC(4 * DT), I, KVC(NE - 2), [&](auto X) __attribute__((always_inline)) { read_column(X, ua); });
-            later(KVC(0), I);
-            form(KVC(2), I);
+            a_mfma(LONE_C(1), LONE_C(KB - 1), I);
+            deal<4 * DT, decltype(I)::value, NE - 2>([&](auto X) __attribute__((always_inline)) { read_column(X, ua); });
+            later(LONE_C(0), I);
+            form(LONE_C(2), I);
             __builtin_amdgcn_sched_barrier(0);
         });
         unit_barrier();
         static_for<NE>([&](auto I) __attribute__((always_inline)) {
             constexpr int i = decltype(I)::value;
-            c_mfma(KVC(0), KVC(0), I);
-            read_row(KVC(i / DK), KVC(i % DK), ub);
-            early(KVC(1), I);
-            form(KVC(3), I);
+            c_mfma(LONE_C(0), LONE_C(0), I);
+            read_row(LONE_C(i / DK), LONE_C(i % DK), ub);
+            early(LONE_C(1), I);
+            form(LONE_C(3), I);
             __builtin_amdgcn_sched_barrier(0);
         });
         static_for<2 * NCH>([&](auto X) __attribute__((always_inline)) { form_store(X, uc); });
         aim_next();
     };
     auto pair_last = [&]() __attribute__((always_inline)) {                         // C(t-1, 1) alone
-        static_for<2>([&](auto X) __attribute__((always_inline)) { p_item(KVC(1), KVC(6 + decltype(X)::value)); });
-        static_for<8>([&](auto X) __attribute__((always_inline)) { ds_item(KVC(1), X); });
-        static_for<NE>([&](auto I) __attribute__((always_inline)) { c_mfma(KVC(1), KVC(KB - 1), I); });
+        static_for<2>([&](auto X) __attribute__((always_inline)) { p_item(LONE_C(1), LONE_C(6 + decltype(X)::value)); });
+        static_for<8>([&](auto X) __attribute__((always_inline)) { ds_item(LONE_C(1), X); });
+        static_for<NE>([&](auto I) __attribute__((always_inline)) { c_mfma(LONE_C(1), LONE_C(KB - 1), I); });
     };
 
+    {
+        X8 z;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) z[t] = (typename E::scalar)0.f;
+        asm volatile("s_nop 3" : "+v"(z));
+        static_for<2 * KB * DT>([&](auto X) __attribute__((always_inline)) { L::sum_zero<16 * decltype(X)::value>(z); });
+    }
     if (has_work) {
         // ---- prologue: rows of the first block, units 0 and 1 ----
         request_block(ib_lo);
         load_side(ib_lo * BQ - (SEG ? d_first : 0) - ws);
+        static_for<KB * DK>([&](auto X) __attribute__((always_inline)) {       // K and V rows as resident B operands
+            constexpr int x = decltype(X)::value, sb = x / DK, col = x % DK * 16;
+            const int j = jw + 32 * sb + ln, jc = j < N ? j : N - 1, c = col + hf * 8;
+            const uint16_t* ks = (const uint16_t*)p.k1.p + p.k1.off(b, jc, h) + c;
+            const uint16_t* vs = (const uint16_t*)p.v1.p + p.v1.off(b, jc, h) + c;
+            L::load_regs<K0 + 4 * x>(PAD && c >= p.D ? (const void*)zero_chunk : (const void*)ks);
+            L::load_regs<V0 + 4 * x>(PAD && c >= p.D ? (const void*)zero_chunk : (const void*)vs);
+        });
         f_stop = run_end(f_ib, f_delta);
         asm volatile("s_waitcnt vmcnt(0)" : "+v"(row_raw) :: "memory");
         take_block(ib_lo);
@@ -625,7 +533,7 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit, float* __rest
             }
         };
         auto rotate = [&]() __attribute__((always_inline)) {
-            keep_out();
+            L::keep_out();
             const uint32_t u = uc;
             uc = ua;
             ua = ub;
@@ -644,7 +552,7 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit, float* __rest
         // behind n units
         auto advance = [&](int n) __attribute__((always_inline)) {
             form_advance(n);
-            keep_out();
+            L::keep_out();
             delta += n;
             if (delta > stop) {
                 ++ib;
@@ -656,10 +564,10 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit, float* __rest
                 }
                 stop = last_unit_of(ib);
                 enter_block();
-                keep_out();
+                L::keep_out();
             }
             enter_unit();
-            keep_out();
+            L::keep_out();
         };
         constexpr std::true_type yes{};
         constexpr std::false_type no{};
@@ -722,7 +630,7 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit, float* __rest
         float* pdst = nsplit > 1 ? part + ((((role ? 0 : 1) * (int64_t)nsplit + sp) * BH + bh) * N + (j < N ? j : N - 1)) * D + 4 * hf : nullptr;
         static_for<4 * DT>([&](auto Y) __attribute__((always_inline)) {
             constexpr int dt = decltype(Y)::value / 4, g4 = decltype(Y)::value % 4, at = (role ? DK0 : DV0) + (sb * DT + dt) * 16 + 4 * g4;
-            const float x0 = get_reg<at>() * sc, x1 = get_reg<at + 1>() * sc, x2 = get_reg<at + 2>() * sc, x3 = get_reg<at + 3>() * sc;
+            const float x0 = L::get_reg<at>() * sc, x1 = L::get_reg<at + 1>() * sc, x2 = L::get_reg<at + 2>() * sc, x3 = L::get_reg<at + 3>() * sc;
             if (j >= N) return;
             if (nsplit > 1) {
                 *(float4*)(pdst + dt * 32 + 8 * g4) = make_float4(x0, x1, x2, x3);

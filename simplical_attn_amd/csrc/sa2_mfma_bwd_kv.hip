@@ -10,17 +10,24 @@ namespace {
 constexpr int KV_MAX_SPLIT = 16;       // workgroups a key block's stream of units is split over, at most
 constexpr int KV_MIN_SHARE = 4;        // units a share holds at least
 
-// Geometry of a launch: 32-row K blocks per wavefront, and the number of shares a key block's stream of units is split into,
-// by grid_time in microseconds: a unit's time by head_dim and blocks, what a change of the query block costs beside it, and
-// prologue and epilogue, fitted to 290 measured cuts at seventeen sizes (profiles/plan_cuts.md): the choice is the best cut at
-// seven of them, 2.6 % off on average and 11 % at most.  A finer cut has to promise 5 %: it costs workspace.  The partial sums
+// Geometry of a launch: 32-row K blocks per wavefront, and the number of shares a key block's stream of units is split into:
+// the cut that ends first by a model in microseconds: a unit's time by head_dim and blocks, what a change of the query block
+// costs beside it, prologue and epilogue, the partial sums' bytes and their summation launch.  Workgroups that all start at once
+// take as long as the longest; more of them fill the chip one behind the other, which ends behind the mean load by 0.6 of the
+// longest, or in whole waves if that is sooner (workgroups of one length).  Fitted to 290 measured cuts at seventeen sizes
+// (profiles/plan_cuts.md): the choice is the best cut at fifteen of them, 4 % and 10 % off at the others.  The partial sums
 // stay under what SA2_STATIC_WORKSPACE_BYTES leaves beside the K'-side kernel's, or 128 MiB where those alone exceed it.
-// Measured with the row term and the sums (us, this plan's kernel before -> now): B2 H4 N512 D64 w 256/256 256 -> 168,
-// B3 H6 N777 D64 w 100/20 102 -> 70, B2 H8 N2048 D64 w 512/32 458 -> 315, B5 H29 N448 D32 w 816/96 1183 -> 750,
+// Measured with the row term and the sums (us, the kernel with two wavefronts per SIMD -> now): B2 H4 N512 D64 w 256/256
+// 256 -> 175, B3 H6 N777 D64 w 100/20 102 -> 67, B2 H8 N2048 D64 w 512/32 458 -> 325, B5 H29 N448 D32 w 816/96 1183 -> 850,
 // B1 H4 N2048 D128 w 512/32 199 -> 160.
 struct KvPlan {
     int kb, nsplit;
 };
+double kv_time(int64_t workgroups, double longest, double mean) {
+    if (workgroups <= CUS) return longest;
+    const double waves = (double)((workgroups + CUS - 1) / CUS) * longest, filled = (double)workgroups / CUS * mean + 0.6 * longest;
+    return waves < filled ? waves : filled;
+}
 KvPlan kv_plan(int B, int N, int H, int D, int w1, int w2, size_t room) {
     KvPlan best{1, 1};
     const int64_t bh = (int64_t)B * H;
@@ -42,13 +49,13 @@ KvPlan kv_plan(int B, int N, int H, int D, int w1, int w2, size_t room) {
             const int64_t jb = (int64_t)x * njb / sampled, last = jb * vj + vj - 1 + w1;
             mean_blocks += (double)((last < N - 1 ? last : N - 1) / BQ - jb * vj / BQ + 1) / sampled;
         }
-        const double unit = D == 128 ? 0.805 : D == 64 ? (kb == 2 ? 0.71 : 0.475) : kb == 2 ? 0.585 : 0.455, change = 0.68;
+        const double unit = D == 128 ? 0.77 : D == 64 ? (kb == 2 ? 0.69 : 0.433) : kb == 2 ? 0.558 : 0.417, change = 0.56;
         const double longest = blocks * (per * unit + change), mean = mean_blocks * (per * window_fill(w2, N) * unit + change);
         for (int ns = 1; ns <= KV_MAX_SPLIT; ++ns) {
             const double part = ns > 1 ? 2.0 * ns * bh * N * D * 4 : 0;
             if (ns > 1 && (base * ns > 16 * CUS || (int64_t)blocks * per / ns < KV_MIN_SHARE || part > cap)) break;
-            const double cost = grid_time(base * ns, longest / ns + 2.6, mean / ns + 2.6, 0.38) + (ns > 1 ? 5.9 + part / 2.4e6 : 0);
-            if (least == 0 || cost < 0.95 * least) {
+            const double cost = kv_time(base * ns, longest / ns + 3.8, mean / ns + 3.8) + (ns > 1 ? 6.5 + part / 3.3e6 : 0);
+            if (least == 0 || cost < least) {
                 least = cost;
                 best = KvPlan{kb, ns};
             }

@@ -3,27 +3,30 @@ import pytest
 
 from simplical_attn_amd import listing_check
 
-CLEAN = """0000 <k_kernel>:
-\tv_accvgpr_write_b32 a3, v9   // 00
+CLEAN = """k_kernel:
+\tv_accvgpr_write_b32 a192, v9
 \tds_read_b128 v[4:7], v9
 \tv_mul_f32_e32 v1, v2, v3
 \ts_waitcnt lgkmcnt(0)
 \tv_mov_b32_e32 v8, 0
-\tv_mfma_f32_32x32x16_bf16 v[16:31], v[4:7], a[128:131], v[32:47]
+\t;;#ASMSTART
+\tv_mfma_f32_32x32x16_bf16 v[16:31], v[4:7], a[0x80:0x83], v[32:47]
 \tv_mfma_f32_32x32x16_bf16 a[0:15], v[4:7], v[0:3], a[0:15]
 \tv_mfma_f32_32x32x16_bf16 a[16:31], v[4:7], v[0:3], a[16:31]
+\tv_accvgpr_read_b32 v9, a[40:40]
+\t;;#ASMEND
 \tv_exp_f32_e32 v16, v16
-\tv_accvgpr_read_b32 v9, a3
 """
 
 
 @pytest.mark.parametrize("old,new,rule", [
     ("", "", None),
     ("ds_read_b128 v[4:7]", "ds_read_b128 a[4:7]", 1),
-    ("v_accvgpr_read_b32 v9, a3", "v_accvgpr_read_b32 v9, a3\n\tv_accvgpr_read_b32 v9, a3", 1),
+    ("v_accvgpr_write_b32 a192", "v_accvgpr_write_b32 a191", 1),
     ("v_mov_b32_e32 v8, 0", "v_mov_b32_e32 v4, 0", 2),
     ("\tv_mfma_f32_32x32x16_bf16 a[16:31], v[4:7], v[0:3], a[16:31]\n", "", 3),
 ])
 def test_planted_breaks(old, new, rule):
-    bad = listing_check.violations(CLEAN.replace(old, new, 1).splitlines(), "k_kernel")
+    bad, found = listing_check.violations(CLEAN.replace(old, new, 1).splitlines(), "k_kernel", 192)
+    assert found == 1
     assert {b[0] for b in bad} == (set() if rule is None else {rule})
