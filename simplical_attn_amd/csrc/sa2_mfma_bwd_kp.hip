@@ -47,15 +47,8 @@ template <int D, int U = 1>
 struct KpCfg {
     static constexpr int DK = D / 16;
     static constexpr int DT = D / 32;
-    // K and V tiles are written by direct global->LDS loads: one wavefront instruction fills a
-    // group of RPW rows (1 KB), lane L putting the 16-byte chunk L / RPW of row L % RPW at byte
-    // 16 * L; groups lie GROUP bytes apart.  Row and transposed operand reads are conflict free.
-    static constexpr int RPW = 512 / D;
-    // byte offset of row r of a tile (chunk 0)
-    static constexpr int row_off(int r) { return (r / RPW) * GROUP + (r % RPW) * 16; }
-    static constexpr int GROUP = 1024 + 16 * RPW;
-    static constexpr int NGROUP = TJ / RPW;
-    static constexpr int TILE_BYTES = NGROUP * GROUP;
+    using Tile = QuadTile<D>;                  // K and V tiles in LDS
+    static constexpr int NGROUP = Tile::NGROUP, TILE_BYTES = Tile::BYTES;
     static constexpr int STAGE = TILE_BYTES;   // bf16 elements of a stage: K tile, then V tile
     static constexpr int NSTAGE = 3;
     static constexpr int RS = D + 8;           // raw row / slab row stride (bf16)
@@ -181,7 +174,7 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
 
     // ---- staging of one K/V tile: wavefront w requests group w of both tiles, straight into LDS
     const bool t_owner = wave < C::NGROUP;
-    const int t_row = wave * C::RPW + (lane % C::RPW), t_col = lane / C::RPW;
+    const int t_row = wave * C::Tile::RPW + C::Tile::dma_row(lane), t_col = C::Tile::dma_chunk(lane);
     const bool t_inside = t_col * 8 < p.D;                    // (used when PAD)
     const uint32_t k_off = ((uint32_t)t_row * (uint32_t)p.k1.sn + t_col * 8) * 2u;
     const uint32_t v_off = ((uint32_t)t_row * (uint32_t)p.v1.sn + t_col * 8) * 2u;
@@ -198,7 +191,7 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
         }
         const char* kbp = (const char*)(k1p + (int64_t)j0 * p.k1.sn);
         const char* vbp = (const char*)(v1p + (int64_t)j0 * p.v1.sn);
-        unsigned char* dst = smem_raw + (size_t)stage * (C::STAGE * 2) + wave * C::GROUP;
+        unsigned char* dst = smem_raw + (size_t)stage * (C::STAGE * 2) + wave * C::Tile::GROUP;
         const char *ks = kbp + ko, *vs = vbp + vo;
         if constexpr (PAD) {
             ks = t_inside ? ks : (const char*)zero_chunk;
@@ -274,25 +267,9 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
     const float qscale = p.scale * LOG2E;
     const uint32_t smem_addr = lds_address(smem);
     const uint32_t px_addr = lds_address(px) + (uint32_t)(pr * 2 * U * 64 * 32 + lane * 32);
-    const uint32_t row_lane = (uint32_t)((ln / C::RPW) * C::GROUP + (hf * C::RPW + ln % C::RPW) * 16);   // row operand
-    const uint32_t col_lane = lds_group_column_lane_offset<C::RPW, C::GROUP>(lane);                      // transposed operand
-    constexpr uint32_t KKB = 32 * C::RPW, DTB = 64 * C::RPW;      // operand strides of a k-step / a 32-column block
-    constexpr uint32_t GA = C::row_off(16), GB = C::row_off(8);
+    const uint32_t row_lane = C::Tile::row_lane(lane), col_lane = C::Tile::column_lane(lane);     // row, transposed operand
     // all transposed operand reads of a tile (opaque reads, settled before use)
-    auto issue_tr = [&](uint32_t a, lds_half_operand (&h)[4 * C::DT]) {
-        lds_tr_issue<0, GB>(a, h[0], h[1]);
-        lds_tr_issue<GA, GA + GB>(a, h[2], h[3]);
-        if constexpr (C::DT >= 2) {
-            lds_tr_issue<DTB, DTB + GB>(a, h[4], h[5]);
-            lds_tr_issue<DTB + GA, DTB + GA + GB>(a, h[6], h[7]);
-        }
-        if constexpr (C::DT == 4) {
-            lds_tr_issue<2 * DTB, 2 * DTB + GB>(a, h[8], h[9]);
-            lds_tr_issue<2 * DTB + GA, 2 * DTB + GA + GB>(a, h[10], h[11]);
-            lds_tr_issue<3 * DTB, 3 * DTB + GB>(a, h[12], h[13]);
-            lds_tr_issue<3 * DTB + GA, 3 * DTB + GA + GB>(a, h[14], h[15]);
-        }
-    };
+    auto issue_tr = [&](uint32_t tile, lds_half_operand (&h)[4 * C::DT]) { quad_tile_issue_blocks<D, 0, C::DT>(tile, col_lane, h); };
 
     // Step g works on ring stage g % 3 (the dS wavefronts also on the one before).  The tile of
     // step g+1 (the next one of this round, or the first one of the next round) is requested at
@@ -393,7 +370,7 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
                     const uint32_t ks_addr = smem_addr + (uint32_t)(buf * C::STAGE) * 2u;
                     X8 ka[C::DK];
 #pragma unroll
-                    for (int kk = 0; kk < C::DK; ++kk) ka[kk] = lds_read_x8<X8>(ks_addr + row_lane + kk * KKB);
+                    for (int kk = 0; kk < C::DK; ++kk) ka[kk] = lds_read_x8<X8>(C::Tile::row_at(ks_addr, row_lane, kk));
                     X8 pb[U][2];
 #pragma unroll
                     for (int u = 0; u < U; ++u) {
@@ -423,7 +400,7 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
                             for (int t = 0; t < 8; ++t) pb[u][ks][t] = (EL)fast_exp2(sh[ks * 8 + t]);
                     }
                     lds_half_operand vh[4 * C::DT];
-                    issue_tr(ks_addr + (uint32_t)C::TILE_BYTES + col_lane, vh);
+                    issue_tr(ks_addr + (uint32_t)C::TILE_BYTES, vh);
 #pragma unroll
                     for (int u = 0; u < U; ++u) {
                         if (!in[u]) continue;
@@ -549,7 +526,7 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
                 }
                 const int pb = buf == 0 ? C::NSTAGE - 1 : buf - 1;
                 lds_half_operand kh[4 * C::DT];
-                issue_tr(smem_addr + (uint32_t)(pb * C::STAGE) * 2u + col_lane, kh);
+                issue_tr(smem_addr + (uint32_t)(pb * C::STAGE) * 2u, kh);
                 lds_settle(kh);
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
@@ -582,7 +559,7 @@ void mfma_bwd_kp_kernel(Problem p, int nkb, int total, float* __restrict__ dq_pa
                     const uint32_t vs_addr = smem_addr + (uint32_t)(buf * C::STAGE) * 2u + (uint32_t)C::TILE_BYTES;
                     X8 va[C::DK];
 #pragma unroll
-                    for (int kk = 0; kk < C::DK; ++kk) va[kk] = lds_read_x8<X8>(vs_addr + row_lane + kk * KKB);
+                    for (int kk = 0; kk < C::DK; ++kk) va[kk] = lds_read_x8<X8>(C::Tile::row_at(vs_addr, row_lane, kk));
 #pragma unroll
                     for (int u = 0; u < U; ++u) {
                         if (!(s >= sa[u] && s <= sb[u])) continue;

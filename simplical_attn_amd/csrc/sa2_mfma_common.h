@@ -123,7 +123,7 @@ __device__ __forceinline__ float other_half(float x) {
     return __uint_as_float((threadIdx.x & 32) ? r[0] : r[1]);
 }
 
-// Tiles in LDS (written by direct global->LDS loads, or by wavefronts in the same order) keep
+// The tiles of 256 columns (written by direct global->LDS loads, or by wavefronts in the same order) keep
 // groups of RPW rows together: within a group the 16-byte chunk c of row q sits at byte
 // (c * RPW + q) * 16, groups lie GROUP bytes apart.  Row operand reads (16 bytes per lane) and the
 // transposed reads below are both free of bank conflicts in this layout.
@@ -189,6 +189,73 @@ __device__ __forceinline__ X8 lds_join(const lds_half_operand& a, const lds_half
     u.h[0] = a;
     u.h[1] = b;
     return u.v;
+}
+// A 32-row K, V, Q or dO tile in LDS as direct global->LDS loads write it.  One wavefront instruction brings a group of RPW
+// rows (1 KB); four neighbouring lanes bring the four 16-byte chunks of 64 consecutive bytes of one row, so that chunk c of row r
+// lies at (c / 4) * 64 * RPW + (r % RPW) * 64 + (c % 4 ^ flip(r)) * 16 of its group.  The 64 bytes are what the loads need:
+// such an instruction takes a CU 17 cycles (37 TB/s over the chip), with pairs of lanes 33, and 65 (9.7 TB/s) where each lane
+// reads another row; whole rows one behind the other need an exchange of chunks that costs an address computation per operand
+// read (VALU instructions of the forward +20 %, its time +3 %).  flip and the distance of the groups make row operand reads (16
+// bytes of one chunk of 16 rows) and transposed operand reads (four rows by 64 bytes) free of bank conflicts.
+// Same results; B1 H16 N8192 D128 w 512/32 bf16: forward 1263 -> 1250 us, K' side 2820 -> 2816; B2 H8 N2048 D64: 211.4 -> 209.5, 426.4 -> 425.6.
+template <int D>
+struct QuadTile {
+    static constexpr int RPW = 512 / D, NGROUP = 32 / RPW;
+    static constexpr int GROUP = 1024 + (D == 128 ? 16 : D == 64 ? 32 : 0), BYTES = NGROUP * GROUP;
+    static constexpr int BLOCK = 64 * RPW;                       // from a 32-column block to the next
+    static __device__ __forceinline__ int flip(int r) { return D == 128 ? 0 : D == 64 ? r >> 2 & 1 : r >> 2 & 3; }
+    static constexpr int row_off(int r) { return (r / RPW) * GROUP + (r % RPW) * 64; }     // (flip aside)
+    // row of its group, and chunk, that a lane brings
+    static __device__ __forceinline__ int dma_row(int lane) { return lane / 4 % RPW; }
+    static __device__ __forceinline__ int dma_chunk(int lane) { return 4 * (lane / (4 * RPW)) + (lane % 4 ^ flip(dma_row(lane))); }
+    // a lane's part of the row operand (row lane % 32, the k-slots of its half) and the address of k-step kk
+    static __device__ __forceinline__ uint32_t row_lane(int lane) {
+        const int r = lane & 31;
+        return (uint32_t)(row_off(r) + ((lane >> 5) ^ flip(r)) * 16);
+    }
+    static __device__ __forceinline__ uint32_t row_at(uint32_t tile, uint32_t row_lane, int kk) {
+        if constexpr (D == 32) return tile + (row_lane ^ (uint32_t)(kk * 32));             // flip moves chunk pairs as well
+        else return tile + row_lane + (uint32_t)(kk / 2 * BLOCK + kk % 2 * 32);
+    }
+    // a lane's part of the transposed operand of the columns 0 .. 31 and the rows 0 .. 7, and the address of rows 8*a .. 8*a+7;
+    // column block dt lies dt * BLOCK further
+    static __device__ __forceinline__ uint32_t column_lane(int lane) {
+        const int grp = lane >> 4, s = lane & 15, r = 4 * (grp >> 1) + (s >> 2), c = 2 * (grp & 1) + ((s & 3) >> 1);
+        return (uint32_t)(row_off(r) + (c ^ flip(r)) * 16 + (s & 1) * 8);
+    }
+    static __device__ __forceinline__ uint32_t column_at(uint32_t tile, uint32_t column_lane, int a) {
+        if constexpr (D == 32) return tile + (column_lane ^ (uint32_t)((a & 1) * 32)) + (uint32_t)row_off(8 * a);
+        else return tile + column_lane + (uint32_t)row_off(8 * a);
+    }
+};
+// The transposed operand of rows 16*ks .. 16*ks+15 and column block dt out of such a tile (compiler-visible reads)
+template <int D, class X8>
+__device__ __forceinline__ X8 quad_tile_column(uint32_t tile, uint32_t column_lane, int dt, int ks) {
+    typedef short v4s __attribute__((ext_vector_type(4)));
+    typedef v4s __attribute__((address_space(3)))* lds_v4s;
+    using T = QuadTile<D>;
+    union { v4s h[2]; X8 v; } u;
+    u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(uintptr_t)(T::column_at(tile, column_lane, 2 * ks) + dt * T::BLOCK));
+    u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(uintptr_t)(T::column_at(tile, column_lane, 2 * ks + 1) + dt * T::BLOCK));
+    return u.v;
+}
+// The same for both k-steps as opaque reads (see lds_tr_issue): h[0..1] = k-step 0, h[2..3] = k-step 1
+template <int D, int DT>
+__device__ __forceinline__ void quad_tile_issue(uint32_t tile, uint32_t column_lane, lds_half_operand* h) {
+    using T = QuadTile<D>;
+    const uint32_t a = tile + column_lane, b = D == 32 ? tile + (column_lane ^ 32u) : a;
+    asm volatile("ds_read_b64_tr_b16 %0, %4 offset:%6\n\tds_read_b64_tr_b16 %1, %5 offset:%7\n\t"
+                 "ds_read_b64_tr_b16 %2, %4 offset:%8\n\tds_read_b64_tr_b16 %3, %5 offset:%9"
+                 : "=&v"(h[0]), "=&v"(h[1]), "=&v"(h[2]), "=&v"(h[3])
+                 : "v"(a), "v"(b), "n"(DT * T::BLOCK), "n"(DT * T::BLOCK + T::row_off(8)), "n"(DT * T::BLOCK + T::row_off(16)),
+                   "n"(DT * T::BLOCK + T::row_off(24)));
+}
+template <int D, int DT0, int DT1>      // column blocks DT0 .. DT1-1
+__device__ __forceinline__ void quad_tile_issue_blocks(uint32_t tile, uint32_t column_lane, lds_half_operand* h) {
+    if constexpr (DT0 < DT1) {
+        quad_tile_issue<D, DT0>(tile, column_lane, h);
+        quad_tile_issue_blocks<D, DT0 + 1, DT1>(tile, column_lane, h + 4);
+    }
 }
 // NW consecutive 32-bit words (2*NW 16-bit elements) from / to a NW*4-byte aligned address
 template <int NW>

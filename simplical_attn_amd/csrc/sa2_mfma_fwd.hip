@@ -14,8 +14,8 @@
 // queries of one (batch, head).  A "unit" is (delta, those 32 queries) = one
 // 32-row MFMA N-tile; each wavefront holds one unit at a time and sweeps the K
 // window [i0-w1, i0+31] in 32-key tiles that go straight from global memory into a
-// four-stage LDS ring (global_load_lds, two steps ahead of their use) in a grouped
-// layout that both the 16-byte K operand reads and the transposed V operand reads
+// four-stage LDS ring (global_load_lds, two steps ahead of their use) in a
+// layout (QuadTile) that both the 16-byte K operand reads and the transposed V operand reads
 // (ds_read_b64_tr_b16) take without bank conflicts.  The q rows of the block and the
 // K'/V' rows its deltas reach are copied to LDS once.  A step issues the logit MFMAs
 // of tile t between the softmax instructions of tile t-1, then the step's barrier (every
@@ -65,18 +65,12 @@ struct Cfg {
     // of its units in registers (32 more at head_dim 64) and the eight are merged once at the end,
     // instead of a fold through LDS with three barriers after every round of eight units.
     static constexpr bool NOFOLD = D <= 64;
-    // A K or V tile in LDS is written by direct global->LDS loads: one wavefront instruction
-    // fills a group of RPW rows (1 KB), lane L putting the 16-byte chunk L / RPW of row
-    // L % RPW at byte 16 * L.  Groups lie GROUP bytes apart.  Row operand reads and
-    // transposed operand reads are both bank-conflict free in this layout.
-    static constexpr int RPW = 512 / D;                     // rows per group: 4 (D = 128), 8 (D = 64), 16 (D = 32)
-    // byte offset of row r of a tile (chunk 0)
-    static constexpr int row_off(int r) { return (r / RPW) * GROUP + (r % RPW) * 16; }
-    static constexpr int GROUP = 1024 + 16 * RPW;           // bytes
-    static constexpr int NGROUP = TK / RPW;
-    static constexpr int TILE_BYTES = NGROUP * GROUP;
-    static constexpr int STAGE = TILE_BYTES;                // bf16 elements of one stage = K tile + V tile
+    using Tile = QuadTile<D>;                                // K and V tiles in LDS
+    static constexpr int NGROUP = Tile::NGROUP;
     static constexpr int SS = D + 8;                        // slab row stride (bf16)
+    // (room behind a tile: two slabs lie over a free stage at the end of a round)
+    static constexpr int TILE_BYTES = Tile::BYTES > 2 * BQ * SS ? Tile::BYTES : 2 * BQ * SS;
+    static constexpr int STAGE = TILE_BYTES;                // bf16 elements of one stage = K tile + V tile
     static constexpr int OS = D + 4;                        // accumulator row stride (fp32)
     // LDS carve-up (bytes)
     static constexpr int NSTAGE = 4;
@@ -107,18 +101,6 @@ struct Cfg {
 // left = 1, starts its accumulator from that pair and handles delta < w2 in full rounds.
 constexpr int MODE_FAST = 0, MODE_SAFE = 1, MODE_LEFT = 2;
 constexpr int PREPASS_MIN_WORKGROUPS = 768;      // three workgroups per CU
-
-// Transposed V operand reads of a whole tile, item I of N = (32-key half h, 32-column block dt,
-// k-step ks): rows 32h + 16ks + {0..7, 8..15} of columns 32dt .. 32dt+31, into vh[2I], vh[2I+1].
-template <class C, int I, int N, int M>
-__device__ __forceinline__ void issue_v_all(uint32_t addr, lds_half_operand (&vh)[M]) {
-    if constexpr (I < N) {
-        constexpr int h = I / (2 * C::DT), dt = (I / 2) % C::DT, ks = I % 2;
-        constexpr int base = dt * 64 * C::RPW;
-        lds_tr_issue<base + C::row_off(32 * h + 16 * ks), base + C::row_off(32 * h + 16 * ks + 8)>(addr, vh[2 * I], vh[2 * I + 1]);
-        issue_v_all<C, I + 1, N>(addr, vh);
-    }
-}
 
 // SIDE: the K' and V' rows the block's deltas reach are copied to LDS (they fit); otherwise
 // they are read from global memory where they are needed.
@@ -198,7 +180,7 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
     // Wavefront w fills group w of the K tile and of the V tile (the first NGROUP wavefronts
     // when D = 64).  Tiles are requested strictly in sweep order into consecutive ring stages.
     const bool t_owner = wave < C::NGROUP;
-    const int t_row = wave * C::RPW + (lane % C::RPW), t_col = lane / C::RPW;
+    const int t_row = wave * C::Tile::RPW + C::Tile::dma_row(lane), t_col = C::Tile::dma_chunk(lane);
     const bool t_inside = t_col * 8 < p.D;                      // (used when PAD)
     const uint32_t k_off = ((uint32_t)t_row * (uint32_t)p.k1.sn + t_col * 8) * 2u;
     const uint32_t v_off = ((uint32_t)t_row * (uint32_t)p.v1.sn + t_col * 8) * 2u;
@@ -220,7 +202,7 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
             const uint32_t ko = at_end ? k_off_c : k_off, vo = at_end ? v_off_c : v_off;
             const char* kb = (const char*)(k1p + (int64_t)j0 * p.k1.sn);
             const char* vb = (const char*)(v1p + (int64_t)j0 * p.v1.sn);
-            unsigned char* dst = smem_raw + (size_t)dma_stage * (C::STAGE * 2) + wave * C::GROUP;
+            unsigned char* dst = smem_raw + (size_t)dma_stage * (C::STAGE * 2) + wave * C::Tile::GROUP;
             const char *ks = kb + ko, *vs = vb + vo;
             if constexpr (PAD) {
                 ks = t_inside ? ks : (const char*)zero_chunk;
@@ -317,8 +299,8 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
     // LDS byte addresses: the stage ring, this lane's part of a K operand read (row ln, k-slots of
     // its half) and of a transposed V operand read
     const uint32_t smem_addr = lds_address(smem);
-    const uint32_t k_lane = (uint32_t)((ln / C::RPW) * C::GROUP + (hf * C::RPW + ln % C::RPW) * 16);
-    const uint32_t v_lane = lds_group_column_lane_offset<C::RPW, C::GROUP>(lane);
+    const uint32_t k_lane = C::Tile::row_lane(lane);
+    const uint32_t v_lane = C::Tile::column_lane(lane);
 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -437,14 +419,13 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
                 }
                 rsum = r;
             };
-            constexpr uint32_t KKB = 32 * C::RPW, DTB = 64 * C::RPW;      // operand strides of a k-step / a 32-column block
             auto stage_addr = [&](int st) { return smem_addr + (uint32_t)st * (uint32_t)(C::STAGE * 2); };
-            constexpr uint32_t SUBB = C::row_off(32 % C::TK);                   // byte offset of a tile's second 32-key half
+            static_assert(C::NSUB == 1, "one 32-row tile per step");
             // logits of the 32-key half `h` of the tile at ks_addr
             auto logit_mfmas = [&](uint32_t ks_addr, int h, floatx16 c) -> floatx16 {
 #pragma unroll
                 for (int kk = 0; kk < C::DK; ++kk) {
-                    const X8 ka = lds_read_x8<X8>(ks_addr + k_lane + h * SUBB + kk * KKB);
+                    const X8 ka = lds_read_x8<X8>(C::Tile::row_at(ks_addr, k_lane, kk));
                     c = E::mfma(ka, qf[kk], c, 0, 0, 0);
                 }
                 return c;
@@ -453,7 +434,7 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
             // vh[((h * DT + dt) * 2 + ks) * 2 + {0, 1}] = the two halves of the operand of half h,
             // 32-column block dt, k-step ks
             auto issue_v = [&](uint32_t vt_addr, lds_half_operand (&vh)[4 * C::DT * C::NSUB]) {
-                issue_v_all<C, 0, 2 * C::DT * C::NSUB>(vt_addr, vh);
+                quad_tile_issue_blocks<D, 0, C::DT>(vt_addr, v_lane, vh);
             };
             // value MFMAs of a whole tile: w[2 * h + ks] = the weights of half h, k-step ks
             auto value_mfmas = [&](uint32_t vt_addr, const X8* w) {
@@ -532,7 +513,7 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
                         weights(t[h], pb + 2 * h, rs);
                         l += rs;
                     }
-                    value_mfmas(Ks + C::TILE_BYTES + v_lane, pb);
+                    value_mfmas(Ks + C::TILE_BYTES, pb);
                     advance();
                 }
             } else {
@@ -577,7 +558,7 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
                     for (int h = 0; h < C::NSUB; ++h)
                         sh_a[h] = logit_mfmas(stage_addr(buf), h, plain0 ? negm : masked_c((jt_lo + ws0) * TJ + 32 * h));
                 }
-                uint32_t vt_prev = stage_addr(buf) + (uint32_t)C::TILE_BYTES + v_lane;
+                uint32_t vt_prev = stage_addr(buf) + (uint32_t)C::TILE_BYTES;
                 advance();
                 // One step: logits of tile s into `cur`, weights and value MFMAs of tile s-1 from `prev`.
                 // PLAIN: the tile needs no mask.  DMA: the step requests a tile (all but the last
@@ -591,7 +572,7 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
 #pragma unroll
                     for (int h = 0; h < C::NSUB; ++h)
 #pragma unroll
-                        for (int kk = 0; kk < C::DK; ++kk) ka[h][kk] = lds_read_x8<X8>(ks_addr + k_lane + h * SUBB + kk * KKB);
+                        for (int kk = 0; kk < C::DK; ++kk) ka[h][kk] = lds_read_x8<X8>(C::Tile::row_at(ks_addr, k_lane, kk));
                     // the reference point (and, on the window-edge tiles, the mask) is the
                     // C operand of the first logit MFMA
                     if constexpr (PLAIN) cur[0] = E::mfma(ka[0][0], qf[0], negm, 0, 0, 0);
@@ -621,7 +602,7 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
                     asm volatile("" : "+v"(pb[0]));              // (the wait below stays behind the first weights)
                     lds_settle(vh);
                     // The barrier stands in front of the value MFMAs: they only read registers.
-                    vt_prev = ks_addr + (uint32_t)C::TILE_BYTES + v_lane;
+                    vt_prev = ks_addr + (uint32_t)C::TILE_BYTES;
                     if constexpr (DMA) asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)\n\ts_barrier" ::: "memory");
                     else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
                     buf = (buf + 1) & (C::NSTAGE - 1);
