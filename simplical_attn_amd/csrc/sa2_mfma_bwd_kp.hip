@@ -1,4 +1,5 @@
-// MFMA backward for gfx950 (bf16 or fp16 elements), the K'-side kernel: dQ, dK' and dV'.
+// MFMA backward for gfx950 (bf16 or fp16 elements), the K'-side kernel: dQ, dK' and dV'.  Wide K windows go to the kernel of
+// sa2_mfma_bwd_kp_lone.h (KpLoneCfg::wanted), under the same plan.
 //
 // Expanded rows r = (i, k), k = i - delta in the K' window of i.  A workgroup owns 32
 // consecutive K' rows k0..k0+31 and every delta: unit delta is the 32 rows
@@ -28,7 +29,7 @@
 // operands come from the row-major tiles through ds_read_b64_tr_b16.
 #include <type_traits>
 
-#include "sa2_mfma_common.h"
+#include "sa2_mfma_bwd_kp_plan.h"
 
 namespace sa2 {
 namespace {
@@ -846,14 +847,24 @@ int launch_kp(const Problem& p, hipStream_t st, BwdSums* sums) {
                            (int)total_left, part, 0, 1, p.w2 + 1, (float*)nullptr);
         if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
     }
+    const auto lone = [&]() {
+        if constexpr (D == 64 || D == 128) return KpLoneCfg<D>::wanted(p.N, p.w1) && KpLoneCfg<D>::fits(w2s);
+        else return false;
+    };
     auto go = [&](auto kernel) {
         if (!allow_full_lds((const void*)kernel)) return false;
         hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(KT), lds, st, p, nkb, (int)total, part, left, pl.nseg, pl.segw, kpart);
         return hipGetLastError() == hipSuccess;
     };
-    const bool ok = pl.nseg > 1 ? (raw ? go(mfma_bwd_kp_kernel<E, D, true, false, U, true, PAD>) : go(mfma_bwd_kp_kernel<E, D, false, false, U, true, PAD>))
-                                : (raw ? go(mfma_bwd_kp_kernel<E, D, true, false, U, false, PAD>) : go(mfma_bwd_kp_kernel<E, D, false, false, U, false, PAD>));
-    if (!ok) return SA2_ERR_LAUNCH_FAILED;
+    auto two_wavefronts = [&]() {
+        return pl.nseg > 1 ? (raw ? go(mfma_bwd_kp_kernel<E, D, true, false, U, true, PAD>) : go(mfma_bwd_kp_kernel<E, D, false, false, U, true, PAD>))
+                           : (raw ? go(mfma_bwd_kp_kernel<E, D, true, false, U, false, PAD>) : go(mfma_bwd_kp_kernel<E, D, false, false, U, false, PAD>));
+    };
+    if (lone()) {
+        const KpLaunch l{pl, nkb, (int)total, left, part, kpart};
+        const int rc = E::DTYPE == SA2_F16 ? launch_mfma_bwd_kp_lone_fp16(p, l, st) : launch_mfma_bwd_kp_lone_bf16(p, l, st);
+        if (rc != SA2_OK) return rc;
+    } else if (!two_wavefronts()) return SA2_ERR_LAUNCH_FAILED;
     sums->dq = p.dq.p ? part : nullptr;
     sums->nkb = nkb;
     sums->nseg = pl.nseg;

@@ -1,0 +1,56 @@
+// The K'-side backward kernel for wide K windows (sa2_mfma_bwd_kp_lone.h): its layout in LDS, when it is taken, and what a
+// launch of it is made of.
+#pragma once
+
+#include "sa2_mfma_common.h"
+
+namespace sa2 {
+
+// A launch of a main kernel of the K' side
+struct KpLaunch {
+    KpPlan plan;
+    int nkb, total, left;
+    float *dq_part, *kpart;
+};
+int launch_mfma_bwd_kp_lone_bf16(const Problem& p, const KpLaunch& l, hipStream_t st);
+int launch_mfma_bwd_kp_lone_fp16(const Problem& p, const KpLaunch& l, hipStream_t st);
+
+namespace {
+
+template <int D>
+struct KpLoneCfg {
+    static constexpr int W = 4, T = W * 64;    // wavefronts, threads per workgroup
+    static constexpr int U = D == 64 ? 2 : 1;  // units (consecutive deltas) a wavefront holds per round
+    static constexpr int DK = D / 16, DT = D / 32;
+    using Tile = QuadTile<D>;                  // K and V tiles in LDS
+    static constexpr int NREQ = Tile::NGROUP / W;                    // groups of a tile a wavefront requests
+    static constexpr int TILE_BYTES = Tile::BYTES;
+    static constexpr int STAGE_BYTES = 2 * TILE_BYTES;               // K tile, then V tile
+    static constexpr int NSTAGE = 4;
+    static constexpr int AS = D + 4;           // fp32 accumulator row stride
+    static constexpr size_t LDS_LIMIT = 160 * 1024;
+    static constexpr size_t row_bytes(int rows) { return (size_t)((rows + Tile::RPW - 1) / Tile::RPW) * Tile::GROUP; }     // rows laid out as in a tile
+    // raw = true: the q and dO rows the workgroup touches are copied to LDS; otherwise the
+    // wavefronts read them from global memory once per unit
+    static size_t main_bytes(int w2, bool raw) {
+        const int rq = BQ + w2;
+        return (size_t)NSTAGE * STAGE_BYTES + 2 * row_bytes(BQ) + (raw ? 2 * row_bytes(rq) : 0) + 2 * ((rq + 3) / 4 * 4) * 4 + (size_t)rq * AS * 4;
+    }
+    static size_t final_bytes() { return (size_t)W * 2 * BQ * AS * 4; }
+    static size_t lds_bytes(int w2, bool raw) { return main_bytes(w2, raw) > final_bytes() ? main_bytes(w2, raw) : final_bytes(); }
+    static bool raw_fits(int w2) { return lds_bytes(w2, true) <= LDS_LIMIT; }
+    static bool fits(int w2) { return lds_bytes(w2, false) <= LDS_LIMIT; }
+    // Whether the kernel is taken, by the keys a K' row's queries see on average (the window, less where the sequence begins).  A
+    // tile of the sweep takes it 0.76 us per eight deltas (head_dim 64; the two-wavefront kernel 1.04) or 0.71 per four (128; 0.89),
+    // but what lies between two sweeps and around them is not overlapped: 2.4 and 4.0 us more per round.  Measured at B1 H16 N4096,
+    // K' windows 7 .. 31, time of the two-wavefront kernel over this one's: head_dim 64, K window 128 0.94, 256 1.00 - 1.03, 384
+    // 1.09, 512 1.08 - 1.13, 1024 1.18; head_dim 128: 256 0.94, 384 1.00, 512 1.02 - 1.04, 768 1.09, 1024 1.11.  (At head_dim 32
+    // the best was 1.03 at 512.)
+    static bool wanted(int N, int w1) {
+        const int64_t w = w1 < N ? w1 : N;
+        return w - w * w / (2 * (int64_t)N) >= (D == 64 ? 300 : 420);
+    }
+};
+
+}  // namespace
+}  // namespace sa2

@@ -630,7 +630,8 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit, float* __rest
         float* pdst = nsplit > 1 ? part + ((((role ? 0 : 1) * (int64_t)nsplit + sp) * BH + bh) * N + (j < N ? j : N - 1)) * D + 4 * hf : nullptr;
         static_for<4 * DT>([&](auto Y) __attribute__((always_inline)) {
             constexpr int dt = decltype(Y)::value / 4, g4 = decltype(Y)::value % 4, at = (role ? DK0 : DV0) + (sb * DT + dt) * 16 + 4 * g4;
-            const float x0 = L::get_reg<at>() * sc, x1 = L::get_reg<at + 1>() * sc, x2 = L::get_reg<at + 2>() * sc, x3 = L::get_reg<at + 3>() * sc;
+            const float4 x = L::get_regs<at>();
+            const float x0 = x.x * sc, x1 = x.y * sc, x2 = x.z * sc, x3 = x.w * sc;
             if (j >= N) return;
             if (nsplit > 1) {
                 *(float4*)(pdst + dt * 32 + 8 * g4) = make_float4(x0, x1, x2, x3);

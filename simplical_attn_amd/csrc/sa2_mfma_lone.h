@@ -81,6 +81,10 @@ struct Lone {
         LONE_MFMA("%0, %1, a[%3:%4], %2", "=&v"(d), "v"(a), "v"(c), "n"(B), "n"(B + 3))
     }
     template <int B, class X8>
+    static __device__ __forceinline__ void tile_start(floatx16& d, const X8& a) {            // (c = 0)
+        LONE_MFMA("%0, %1, a[%2:%3], 0", "=&v"(d), "v"(a), "n"(B), "n"(B + 3))
+    }
+    template <int B, class X8>
     static __device__ __forceinline__ void tile_more(floatx16& d, const X8& a) {
         LONE_MFMA("%0, %1, a[%2:%3], %0", "+v"(d), "v"(a), "n"(B), "n"(B + 3))
     }
@@ -100,16 +104,21 @@ struct Lone {
         if constexpr (ALL) asm volatile("" ::: LONE_REGS_ALL);
         else asm volatile("" ::: LONE_REGS);
     }
+    // registers R .. R+3, R a multiple of four (one by one the compiler would put a wait between them)
     template <int R>
-    static __device__ __forceinline__ void set_reg(uint32_t x) {
-        if constexpr (ALL) asm volatile("v_accvgpr_write_b32 a[%1:%1], %0" ::"v"(x), "n"(R) : LONE_REGS_ALL);
-        else asm volatile("v_accvgpr_write_b32 a[%1:%1], %0" ::"v"(x), "n"(R) : LONE_REGS);
+    static __device__ __forceinline__ void set_regs(uint32_t x0, uint32_t x1, uint32_t x2, uint32_t x3) {
+#define LONE_SET "v_accvgpr_write_b32 a[%4:%4], %0\n\tv_accvgpr_write_b32 a[%5:%5], %1\n\tv_accvgpr_write_b32 a[%6:%6], %2\n\tv_accvgpr_write_b32 a[%7:%7], %3"
+        if constexpr (ALL) asm volatile(LONE_SET ::"v"(x0), "v"(x1), "v"(x2), "v"(x3), "n"(R), "n"(R + 1), "n"(R + 2), "n"(R + 3) : LONE_REGS_ALL);
+        else asm volatile(LONE_SET ::"v"(x0), "v"(x1), "v"(x2), "v"(x3), "n"(R), "n"(R + 1), "n"(R + 2), "n"(R + 3) : LONE_REGS);
+#undef LONE_SET
     }
     template <int R>
-    static __device__ __forceinline__ float get_reg() {
-        float x;
-        if constexpr (ALL) asm volatile("v_accvgpr_read_b32 %0, a[%1:%1]" : "=v"(x) : "n"(R) : LONE_REGS_ALL);
-        else asm volatile("v_accvgpr_read_b32 %0, a[%1:%1]" : "=v"(x) : "n"(R) : LONE_REGS);
+    static __device__ __forceinline__ float4 get_regs() {
+        float4 x;
+#define LONE_GET "v_accvgpr_read_b32 %0, a[%4:%4]\n\tv_accvgpr_read_b32 %1, a[%5:%5]\n\tv_accvgpr_read_b32 %2, a[%6:%6]\n\tv_accvgpr_read_b32 %3, a[%7:%7]"
+        if constexpr (ALL) asm volatile(LONE_GET : "=v"(x.x), "=v"(x.y), "=v"(x.z), "=v"(x.w) : "n"(R), "n"(R + 1), "n"(R + 2), "n"(R + 3) : LONE_REGS_ALL);
+        else asm volatile(LONE_GET : "=v"(x.x), "=v"(x.y), "=v"(x.z), "=v"(x.w) : "n"(R), "n"(R + 1), "n"(R + 2), "n"(R + 3) : LONE_REGS);
+#undef LONE_GET
         return x;
     }
     // registers R .. R+3 from global memory (a vector-memory operation that the compiler does not count)
@@ -120,10 +129,20 @@ struct Lone {
     }
 };
 
+// what the vector ALU has made of x by here is not put off behind a branch
+template <class T>
+__device__ __forceinline__ void stays(T& x) { asm volatile("" : "+v"(x)); }
+// the MFMAs that write the two tiles have ended
+__device__ __forceinline__ void finished(floatx16& a, floatx16& b) { asm volatile("s_nop 15\n\ts_nop 15" : "+v"(a), "+v"(b)); }
+
 // 16 bytes per lane from global memory straight to LDS, lane L to `to` + 16 * L.  Opaque: the compiler would wait for it
 // before every read of LDS.
 __device__ __forceinline__ void lds_request(const void* src, uint32_t to) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(__builtin_amdgcn_readfirstlane(to)), "v"(src) : "memory");
+}
+// the same from a base that all lanes share and a byte offset of the lane's own
+__device__ __forceinline__ void lds_request(const void* base, uint32_t off, uint32_t to) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(to)), "v"(off), "s"(base) : "memory");
 }
 
 }  // namespace
