@@ -36,7 +36,8 @@ FLAGS = [
 # sources with hand-placed MFMAs -> their kernels and the accumulation registers these own; the compiler's listing of them
 # is checked (see listing_check.py)
 HAND_PLACED = {"sa2_mfma_bwd_kv_bf16.hip": ("mfma_bwd_kv_kernel", 192), "sa2_mfma_bwd_kv_fp16.hip": ("mfma_bwd_kv_kernel", 192),
-               "sa2_mfma_bwd_kp_lone_bf16.hip": ("mfma_bwd_kp_lone_kernel", 256), "sa2_mfma_bwd_kp_lone_fp16.hip": ("mfma_bwd_kp_lone_kernel", 256)}
+               "sa2_mfma_bwd_kp_lone_bf16.hip": ("mfma_bwd_kp_lone_kernel", 256), "sa2_mfma_bwd_kp_lone_fp16.hip": ("mfma_bwd_kp_lone_kernel", 256),
+               "sa2_mfma_fwd_lone_bf16.hip": ("mfma_fwd_lone_kernel", 96), "sa2_mfma_fwd_lone_fp16.hip": ("mfma_fwd_lone_kernel", 96)}
 
 
 def _compile(src, extra):

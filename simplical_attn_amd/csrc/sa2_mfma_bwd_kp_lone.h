@@ -30,7 +30,7 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
     typedef typename E::x8 X8;
     using C = KpLoneCfg<D>;
     constexpr int U = C::U, KW = C::W, KT = C::T;
-    using L = Lone<true>;
+    using L = Lone<256>;
     constexpr int UPR = KW * U;                               // units per round
     constexpr int DK = C::DK, DT = C::DT;
     constexpr bool DVV = D == 128;

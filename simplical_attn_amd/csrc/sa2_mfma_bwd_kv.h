@@ -67,7 +67,7 @@ __global__ __launch_bounds__(VT) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit, float* __restrict__ part, int ws_arg) {
     typedef typename E::x8 X8;
     using C = KvCfg<D, KB>;
-    using L = Lone<false>;
+    using L = Lone<192>;
     constexpr int VJ = C::VJ, DK = C::DK, DT = C::DT, NCH = C::NCH, RPW = C::RPW;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     const int N = p.N, w1 = p.w1, w2 = p.w2;

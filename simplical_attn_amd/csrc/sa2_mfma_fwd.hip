@@ -37,6 +37,7 @@
 #include <type_traits>
 
 #include "sa2_mfma_common.h"
+#include "sa2_mfma_fwd_lone_plan.h"
 
 namespace sa2 {
 namespace {
@@ -1033,15 +1034,29 @@ int launch_fwd_kernels(const Problem& p, int nqb, int total, hipStream_t st) {
                            (FwdArgs{p, ngrp, total_left, 0}));
         if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
     }
-    auto go = [&](auto kernel, int64_t grid) {
+    auto go = [&](auto kernel, int64_t grid, int blocks) {
         if (!allow_full_lds((const void*)kernel)) return false;
-        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(FT), lds, st, (FwdArgs{p, nqb, (int)grid, left}));
+        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(FT), lds, st, (FwdArgs{p, blocks, (int)grid, left}));
         return hipGetLastError() == hipSuccess;
     };
-    if (p.nsplit <= 1) return go(mfma_fwd_kernel<E, D, MODE_FAST, SIDE, PAD, false>, total) ? SA2_OK : SA2_ERR_LAUNCH_FAILED;
+    if constexpr (!PAD && D >= 64) {
+        using L = FwdLoneCfg<D>;
+        if (p.nsplit <= 1 || !L::FIRST_ELSEWHERE) {
+            const int64_t grid = (int64_t)total * (p.nsplit > 1 ? p.nsplit : 1);
+            if (L::wanted(grid, (p.w2 < p.N - 1 ? p.w2 : p.N - 1) + 1 - left, p.N, p.w1)) {
+                if (grid > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
+                // (one block per head: the first one)
+                if (L::FIRST_ELSEWHERE && !go(mfma_fwd_kernel<E, D, MODE_FAST, SIDE, PAD, false>, total / nqb, 1)) return SA2_ERR_LAUNCH_FAILED;
+                const FwdLoneArgs args{p, nqb, (int)grid, left};
+                const int rc = E::DTYPE == SA2_F16 ? launch_mfma_fwd_lone_fp16(args, st) : launch_mfma_fwd_lone_bf16(args, st);
+                return rc != SA2_OK || p.nsplit <= 1 ? rc : launch_fwd_merge(p, D, E::DTYPE, st);
+            }
+        }
+    }
+    if (p.nsplit <= 1) return go(mfma_fwd_kernel<E, D, MODE_FAST, SIDE, PAD, false>, total, nqb) ? SA2_OK : SA2_ERR_LAUNCH_FAILED;
     const int64_t grid = (int64_t)total * p.nsplit;
     if (grid > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
-    if (!go(mfma_fwd_kernel<E, D, MODE_FAST, SIDE, PAD, true>, grid)) return SA2_ERR_LAUNCH_FAILED;
+    if (!go(mfma_fwd_kernel<E, D, MODE_FAST, SIDE, PAD, true>, grid, nqb)) return SA2_ERR_LAUNCH_FAILED;
     return launch_fwd_merge(p, D, E::DTYPE, st);
 }
 

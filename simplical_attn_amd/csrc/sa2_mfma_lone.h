@@ -43,17 +43,18 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 typedef const u4 __attribute__((address_space(3)))* lds_u4;
 
-// Accumulation registers 0 .. 191 (ALL: 0 .. 255) belong to the kernel, not to the compiler: the sums that live through a
+// Accumulation registers 0 .. OWNED-1 (96, 192 or 256) belong to the kernel, not to the compiler: the sums that live through a
 // sweep and the resident operands are named by number in the instructions below, and each of these says that it destroys
 // them all, so that nothing else is ever kept there.  (Left to the compiler, beside 300 other registers of the sweep, sums and
 // operands move between the two files or to scratch memory in every step.)
-#define LONE_REGS \
+#define LONE_REGS_96 \
     "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", "a10", "a11", "a12", "a13", "a14", "a15", \
     "a16", "a17", "a18", "a19", "a20", "a21", "a22", "a23", "a24", "a25", "a26", "a27", "a28", "a29", "a30", "a31", \
     "a32", "a33", "a34", "a35", "a36", "a37", "a38", "a39", "a40", "a41", "a42", "a43", "a44", "a45", "a46", "a47", \
     "a48", "a49", "a50", "a51", "a52", "a53", "a54", "a55", "a56", "a57", "a58", "a59", "a60", "a61", "a62", "a63", \
     "a64", "a65", "a66", "a67", "a68", "a69", "a70", "a71", "a72", "a73", "a74", "a75", "a76", "a77", "a78", "a79", \
-    "a80", "a81", "a82", "a83", "a84", "a85", "a86", "a87", "a88", "a89", "a90", "a91", "a92", "a93", "a94", "a95", \
+    "a80", "a81", "a82", "a83", "a84", "a85", "a86", "a87", "a88", "a89", "a90", "a91", "a92", "a93", "a94", "a95"
+#define LONE_REGS LONE_REGS_96, \
     "a96", "a97", "a98", "a99", "a100", "a101", "a102", "a103", "a104", "a105", "a106", "a107", "a108", "a109", "a110", "a111", \
     "a112", "a113", "a114", "a115", "a116", "a117", "a118", "a119", "a120", "a121", "a122", "a123", "a124", "a125", "a126", "a127", \
     "a128", "a129", "a130", "a131", "a132", "a133", "a134", "a135", "a136", "a137", "a138", "a139", "a140", "a141", "a142", "a143", \
@@ -65,14 +66,16 @@ typedef const u4 __attribute__((address_space(3)))* lds_u4;
     "a208", "a209", "a210", "a211", "a212", "a213", "a214", "a215", "a216", "a217", "a218", "a219", "a220", "a221", "a222", "a223", \
     "a224", "a225", "a226", "a227", "a228", "a229", "a230", "a231", "a232", "a233", "a234", "a235", "a236", "a237", "a238", "a239", \
     "a240", "a241", "a242", "a243", "a244", "a245", "a246", "a247", "a248", "a249", "a250", "a251", "a252", "a253", "a254", "a255"
-template <bool ALL>
+template <int OWNED>
 struct Lone {
 #define LONE_MFMA(text, out, ...) \
     if constexpr (std::is_same<X8, bf16x8>::value) { \
-        if constexpr (ALL) asm volatile("v_mfma_f32_32x32x16_bf16 " text : out : __VA_ARGS__ : LONE_REGS_ALL); \
+        if constexpr (OWNED == 256) asm volatile("v_mfma_f32_32x32x16_bf16 " text : out : __VA_ARGS__ : LONE_REGS_ALL); \
+        else if constexpr (OWNED == 96) asm volatile("v_mfma_f32_32x32x16_bf16 " text : out : __VA_ARGS__ : LONE_REGS_96); \
         else asm volatile("v_mfma_f32_32x32x16_bf16 " text : out : __VA_ARGS__ : LONE_REGS); \
     } else { \
-        if constexpr (ALL) asm volatile("v_mfma_f32_32x32x16_f16 " text : out : __VA_ARGS__ : LONE_REGS_ALL); \
+        if constexpr (OWNED == 256) asm volatile("v_mfma_f32_32x32x16_f16 " text : out : __VA_ARGS__ : LONE_REGS_ALL); \
+        else if constexpr (OWNED == 96) asm volatile("v_mfma_f32_32x32x16_f16 " text : out : __VA_ARGS__ : LONE_REGS_96); \
         else asm volatile("v_mfma_f32_32x32x16_f16 " text : out : __VA_ARGS__ : LONE_REGS); \
     }
     // d = a * operand B + c, d += a * operand B: tiles in vector registers, whose first reader comes at least two MFMAs later
@@ -101,14 +104,16 @@ struct Lone {
 #undef LONE_MFMA
     // (a value that is read between two of these instructions only could still be given one of the registers)
     static __device__ __forceinline__ void keep_out() {
-        if constexpr (ALL) asm volatile("" ::: LONE_REGS_ALL);
+        if constexpr (OWNED == 256) asm volatile("" ::: LONE_REGS_ALL);
+        else if constexpr (OWNED == 96) asm volatile("" ::: LONE_REGS_96);
         else asm volatile("" ::: LONE_REGS);
     }
     // registers R .. R+3, R a multiple of four (one by one the compiler would put a wait between them)
     template <int R>
     static __device__ __forceinline__ void set_regs(uint32_t x0, uint32_t x1, uint32_t x2, uint32_t x3) {
 #define LONE_SET "v_accvgpr_write_b32 a[%4:%4], %0\n\tv_accvgpr_write_b32 a[%5:%5], %1\n\tv_accvgpr_write_b32 a[%6:%6], %2\n\tv_accvgpr_write_b32 a[%7:%7], %3"
-        if constexpr (ALL) asm volatile(LONE_SET ::"v"(x0), "v"(x1), "v"(x2), "v"(x3), "n"(R), "n"(R + 1), "n"(R + 2), "n"(R + 3) : LONE_REGS_ALL);
+        if constexpr (OWNED == 256) asm volatile(LONE_SET ::"v"(x0), "v"(x1), "v"(x2), "v"(x3), "n"(R), "n"(R + 1), "n"(R + 2), "n"(R + 3) : LONE_REGS_ALL);
+        else if constexpr (OWNED == 96) asm volatile(LONE_SET ::"v"(x0), "v"(x1), "v"(x2), "v"(x3), "n"(R), "n"(R + 1), "n"(R + 2), "n"(R + 3) : LONE_REGS_96);
         else asm volatile(LONE_SET ::"v"(x0), "v"(x1), "v"(x2), "v"(x3), "n"(R), "n"(R + 1), "n"(R + 2), "n"(R + 3) : LONE_REGS);
 #undef LONE_SET
     }
@@ -116,7 +121,8 @@ struct Lone {
     static __device__ __forceinline__ float4 get_regs() {
         float4 x;
 #define LONE_GET "v_accvgpr_read_b32 %0, a[%4:%4]\n\tv_accvgpr_read_b32 %1, a[%5:%5]\n\tv_accvgpr_read_b32 %2, a[%6:%6]\n\tv_accvgpr_read_b32 %3, a[%7:%7]"
-        if constexpr (ALL) asm volatile(LONE_GET : "=v"(x.x), "=v"(x.y), "=v"(x.z), "=v"(x.w) : "n"(R), "n"(R + 1), "n"(R + 2), "n"(R + 3) : LONE_REGS_ALL);
+        if constexpr (OWNED == 256) asm volatile(LONE_GET : "=v"(x.x), "=v"(x.y), "=v"(x.z), "=v"(x.w) : "n"(R), "n"(R + 1), "n"(R + 2), "n"(R + 3) : LONE_REGS_ALL);
+        else if constexpr (OWNED == 96) asm volatile(LONE_GET : "=v"(x.x), "=v"(x.y), "=v"(x.z), "=v"(x.w) : "n"(R), "n"(R + 1), "n"(R + 2), "n"(R + 3) : LONE_REGS_96);
         else asm volatile(LONE_GET : "=v"(x.x), "=v"(x.y), "=v"(x.z), "=v"(x.w) : "n"(R), "n"(R + 1), "n"(R + 2), "n"(R + 3) : LONE_REGS);
 #undef LONE_GET
         return x;
@@ -124,7 +130,8 @@ struct Lone {
     // registers R .. R+3 from global memory (a vector-memory operation that the compiler does not count)
     template <int R>
     static __device__ __forceinline__ void load_regs(const void* src) {
-        if constexpr (ALL) asm volatile("global_load_dwordx4 a[%1:%2], %0, off" ::"v"(src), "n"(R), "n"(R + 3) : "memory", LONE_REGS_ALL);
+        if constexpr (OWNED == 256) asm volatile("global_load_dwordx4 a[%1:%2], %0, off" ::"v"(src), "n"(R), "n"(R + 3) : "memory", LONE_REGS_ALL);
+        else if constexpr (OWNED == 96) asm volatile("global_load_dwordx4 a[%1:%2], %0, off" ::"v"(src), "n"(R), "n"(R + 3) : "memory", LONE_REGS_96);
         else asm volatile("global_load_dwordx4 a[%1:%2], %0, off" ::"v"(src), "n"(R), "n"(R + 3) : "memory", LONE_REGS);
     }
 };
