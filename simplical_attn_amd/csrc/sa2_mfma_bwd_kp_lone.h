@@ -298,10 +298,15 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
         s[u][e + 1] = y;
         if constexpr (i > 0) round_p(UN, LONE_C(i - 1));
     };
+    // dS from the rounded weights, as in the two-wavefront kernel: the first queries have few weights, all large, and their gradients
+    // follow the rounding of each closely (from the unrounded ones they came out up to 0.6 of a gradient's root mean square
+    // elsewhere, B1 H8 N32768 D128 w 1024/64; now 0.03).  It costs two instructions a pair, 3 % of a training step.  (A second
+    // copy of the sweep for the first queries alone does not fit the registers: 560 bytes per lane of scratch.)
     auto ds_item = [&](auto UN, auto I) __attribute__((always_inline)) {
         constexpr int u = decltype(UN)::value, i = decltype(I)::value, ks = i / 4, t = i % 4, e = 2 * i;
         if constexpr (i == 0) round_p(UN, LONE_C(7));
-        uint32_t w = pack2<E>(s[u][e] * (dp[u][e] - drow_sum[u]), s[u][e + 1] * (dp[u][e + 1] - drow_sum[u]));
+        const uint32_t pp = pw[u][ks][t];
+        uint32_t w = pack2<E>(E::lo(pp) * (dp[u][e] - drow_sum[u]), E::hi(pp) * (dp[u][e + 1] - drow_sum[u]));
         stays(w);
         dw[u][ks][t] = w;
     };

@@ -349,10 +349,12 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit, float* __rest
         s[x][e + 1] = fast_exp2(s[x][e + 1]);
         if constexpr (i > 0) round_p(XP, std::integral_constant<int, i - 1>{});
     };
+    // (from the rounded weights; see the K'-side kernel, sa2_mfma_bwd_kp_lone.h)
     auto ds_item = [&](auto XP, auto I) __attribute__((always_inline)) {
         constexpr int x = decltype(XP)::value, i = decltype(I)::value, ks = i / 4, t = i % 4, e = 2 * i;
         if constexpr (i == 0) round_p(XP, std::integral_constant<int, 7>{});
-        dw[x][ks][t] = pack2<E>(s[x][e] * dp[x][e], s[x][e + 1] * dp[x][e + 1]);
+        const uint32_t pp = pw[x][ks][t];
+        dw[x][ks][t] = pack2<E>(E::lo(pp) * dp[x][e], E::hi(pp) * dp[x][e + 1]);
     };
     auto unit_barrier = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
     // One K block per unit.  A(t), under the forming of unit t+2; then C(t-1), whose four groups of MFMAs (dV^T and dK^T, each

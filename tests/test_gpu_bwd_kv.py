@@ -2,7 +2,9 @@
 64 .. 256 heads take two at head_dim 32 and 64), shares that begin inside a query block, blocks of one unit (w2 = 0), K'
 windows that just fit LDS and that are walked in segments, first and last blocks cut by the windows.  Against the fp32 FMA
 kernels on the same inputs; the products, weights and dS are rounded to 16 bits in between, which the bar of the other
-16-bit tests (2e-2 of the largest element, fp16 1.5e-2) covers."""
+16-bit tests (2e-2 of the largest element, fp16 1.5e-2) covers.  At 16 columns dP = sum of dout*v2 * v1 averages the roundings of its
+products over a quarter of the terms that it has at 64, so its error may be sqrt(4) as large there (4e-2); 2.4e-2 is the largest
+seen over five seeds, the same with the kernels whose P crosses between wavefronts in 16 bits, and 3e-2 the bar."""
 import pytest
 import torch
 
@@ -33,6 +35,7 @@ def test_k_side_matches_the_fma_kernels(dtype, B, N, H, D, w1, w2, bias):
     got = sa.simplicial_backward(*x[:5], out, lse, x[5], w1, w2, **kw)
     want = sa.simplicial_backward(*x[:5], out, lse, x[5], w1, w2, flags=1, **kw)
     for name, i in (("dk1", 1), ("dv1", 3)):
-        assert_close_rel(got[i], want[i].cpu(), 2e-2 if dtype == BF else 1.5e-2, name, atol=2e-3)
+        bar = 3e-2 if D == 16 else 2e-2 if dtype == BF else 1.5e-2
+        assert_close_rel(got[i], want[i].cpu(), bar, name, atol=2e-3)
     again = sa.simplicial_backward(*x[:5], out, lse, x[5], w1, w2, **kw)
     assert torch.equal(got[1], again[1]) and torch.equal(got[3], again[3])
