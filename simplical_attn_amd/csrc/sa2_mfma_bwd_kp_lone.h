@@ -10,7 +10,7 @@
 // What bounds it: at head_dim 64 the instructions beside the MFMAs (32 MFMAs per tile, 0.44 us of 0.76; 18 tiles take 14 us of
 // a round's 23, masks 1.8, the sums over the units and dQ 3, forming 1); at head_dim 128 also power.  K' side with its
 // pre-pass, against the two-wavefront kernel: B2 H8 N2048 D64 w 512/32 427 -> 392 us, B1 H16 N8192 D128 w 512/32 2835 -> 2737,
-// B1 H8 N8192 w 1024/64 D128 4675 -> 4219, D64 2571 -> 2170 (bf16).
+// B1 H8 N8192 w 1024/64 D128 4675 -> 4219, D64 2571 -> 2170 (bf16; dS from unrounded weights).  With the rounding 388 and 2728.
 #pragma once
 
 #include "sa2_mfma_bwd_kp_plan.h"

@@ -1,4 +1,6 @@
-// MFMA forward for gfx950 (bf16 or fp16 elements), head_dim 32, 64 or 128.
+// MFMA forward for gfx950 (bf16 or fp16 elements), head_dim 32, 64 or 128.  The launches, and the kernel with eight wavefronts of one
+// unit each; most problems of head_dim 64 and 128 take the one with two units per wavefront (sa2_mfma_fwd_lone.h), which
+// sa2_mfma_fwd_lone_plan.h chooses.
 //
 // Formulation: expand every query i by its K' window into rows r = (i, delta),
 // delta = i - k in [0, w2], with Q~[r,:] = q[i,:] * (k2[i-delta,:] + k2_bias) *
@@ -1024,7 +1026,8 @@ int launch_fwd_kernels(const Problem& p, int nqb, int total, hipStream_t st) {
     using C = Cfg<D>;
     const size_t lds = C::lds_bytes(fwd_side_span(p));
     // one unit left over after the rounds of eight: the pre-pass takes it, unless the grid is so
-    // small that a further launch costs more than the lone round
+    // small that a further launch costs more than the lone round (also with two units per wavefront: B1 H16 N8192 D64 w 512/32
+    // 626 us with it, 654 without; B1 H16 N4096 w 256/8 79 and 90; B1 H16 N1600 w 256/16, 800 workgroups, 66 and 60)
     const int left = (p.nsplit <= 1 && p.w2 >= FW && p.w2 % FW == 0 && (p.force_prepass || total >= PREPASS_MIN_WORKGROUPS)) ? 1 : 0;
     if (left) {
         const int ngrp = (nqb + FW - 1) / FW;
