@@ -68,3 +68,21 @@ def test_a_key_that_is_not_a_number_stays_in_its_window(D, heads, w2):
     out, lse = sa.simplicial_forward(*x, 230, w2)
     rows = lse[0].isnan()
     assert rows[:, 350:581].all() and rows.sum().item() == 231 * heads and torch.equal(out[0].isnan().any(-1).T, rows)
+
+
+@pytest.mark.parametrize("D,N,heads,w1,w2", [(64, 1500, 6, 200, 20), (128, 4100, 16, 300, 24)])
+def test_layouts_and_half_open_windows(D, N, heads, w1, w2):
+    """Views of one fused projection [B, N, 5, H, D] and of [B, H, N, D] tensors give what contiguous copies give, bit for bit."""
+    import simplical_attn_amd as sa
+    g = torch.Generator(device="cuda").manual_seed(D)
+    packed = torch.randn(1, N, 5, heads, D, generator=g, device="cuda").to(BF)
+    x = packed.unbind(2)
+    turned = [t.transpose(1, 2).contiguous().transpose(1, 2) for t in x]
+    kw = dict(window_inclusive=False)
+    want = sa.simplicial_forward(*[t.contiguous() for t in x], w1, w2, **kw)
+    for views in (x, turned):
+        got = sa.simplicial_forward(*views, w1, w2, **kw)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    exact, lse = sa.simplicial_forward(*x, w1, w2, flags=1, **kw)
+    assert_close_rel(want[0], exact.float().cpu(), 2e-2, "out")
+    assert_close_rel(want[1], lse.cpu(), 2e-2, "lse")
