@@ -27,9 +27,15 @@ namespace {
 
 // The first pass keeps one reference point per row and wavefront: the largest logit of its first two units in the queries' own
 // tile, which holds a key of every row (fp16: and in the tile before, since a weight must stay below 65504).  A row whose sum
-// is not finite afterwards sends the workgroup through the SAFE pass, where every unit has a reference point of its own, which
-// follows the maxima.  The first 32 queries, whose windows are a single tile, take that pass at once: their few weights are rounded
-// less often so (a unit's largest one is 1).  At head_dim 128 the eight-wavefront kernel takes them (FwdLoneCfg::FIRST_ELSEWHERE).
+// is not finite afterwards sends the workgroup through the SAFE pass.  At head_dim 64 every unit has a reference point of its own there,
+// which follows the maxima; the first 32 queries, whose windows are a single tile, take that pass at once: their few weights are
+// rounded less often so (a unit's largest one is 1).  At head_dim 128, where the eight-wavefront kernel takes the first queries
+// (FwdLoneCfg::FIRST_ELSEWHERE), a sweep of the logit MFMAs alone finds the largest logit of a row in both units, and the sweep of
+// the first pass follows from that point, with explicit masks where a tile needs them.  (Following the maxima there, a wavefront
+// alone on its SIMD ran MFMAs, exponentials and the rescaling of sums one after the other, and the second pass cost more than that of
+// the eight-wavefront kernel.  Forward, us, eight wavefronts / maxima followed / this; fp16 B1 H16 N8192 w 512/32, q, k1 and k2
+// N(0, std^2): std 1.25 2160 / 1750 / 1600, 1.5 3320 / 4370 / 3265, 2 and more 3270 / 4600 / 3430; bf16, std 2 1309 / 1305 / 1238,
+// 3 3165 / 4570 / 3380.  At head_dim 64 following costs less than the pass it replaced: fp16 B2 H8 N2048 w 512/32, std 2 582 / 559.)
 template <class E, int D, bool SAFE, bool SPLIT>
 __device__ __forceinline__ bool fwd_lone_block(const Problem& p, int nqb, int total, int left) {
     typedef typename E::scalar EL;
@@ -241,6 +247,11 @@ __device__ __forceinline__ bool fwd_lone_block(const Problem& p, int nqb, int to
         if constexpr (i == 0) L::template tile_start<at>(s[u], ka[0], nl);
         else L::template tile_more<at>(s[u], ka[i]);
     };
+    auto logit_mfma = [&](auto UN, auto I) __attribute__((always_inline)) {         // (from zero)
+        constexpr int u = decltype(UN)::value, i = decltype(I)::value, at = Q0 + (u * DK + i) * 4;
+        if constexpr (i == 0) L::template tile_start<at>(s[u], ka[0]);
+        else L::template tile_more<at>(s[u], ka[i]);
+    };
     auto c_mfma = [&](auto UN, auto I) __attribute__((always_inline)) {
         constexpr int u = decltype(UN)::value, ks = decltype(I)::value / DT, dt = decltype(I)::value % DT;
         L::template sum_more<R0 + (u * DT + dt) * 16>(vt[dt][ks], __builtin_bit_cast(X8, pw[u][ks]));
@@ -345,12 +356,14 @@ __device__ __forceinline__ bool fwd_lone_block(const Problem& p, int nqb, int to
         return seen;
     };
     bool unmasked = false;
+    float round_max = -INFINITY;                              // (second pass at head_dim 128) reference point of the round's units
     auto enter_tile = [&](int jt) __attribute__((always_inline)) {                  // the start of the S tiles of tile jt
         const bool plain = jt >= p_lo && jt < jt_hi;
         if (plain && unmasked) return;
         unmasked = plain;
         const uint32_t seen = plain ? ~0u : keys_seen(jt);
-        const int v0 = Mw == -INFINITY ? 0 : __float_as_int(-Mw), v1 = __float_as_int(-INFINITY);
+        const float ref = SAFE ? round_max : Mw;
+        const int v0 = ref == -INFINITY ? 0 : __float_as_int(-ref), v1 = __float_as_int(-INFINITY);
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
             int m = (int)(seen << (31 - 8 * (v >> 2) - (v & 3))) >> 31;
@@ -429,7 +442,7 @@ __device__ __forceinline__ bool fwd_lone_block(const Problem& p, int nqb, int to
 
         if (!any) {
             // no unit for this wavefront in this round: keep the requests moving
-            for (int jt = jt_hi; jt >= jt_lo; --jt) {
+            for (int jt = (SAFE && C::MAXIMA_FIRST ? 2 : 1) * (jt_hi - jt_lo + 1); jt > 0; --jt) {
                 step_barrier();
                 next_request();
                 request_tile(sc);
@@ -438,7 +451,91 @@ __device__ __forceinline__ bool fwd_lone_block(const Problem& p, int nqb, int to
             continue;
         }
         float mu[U];                                          // (SAFE) reference points of the units
-        if constexpr (SAFE) {
+        // (SAFE) the tile whose logits `tile_logits` left: weights of a unit from its reference point, sums of both, the next tile's rows
+        auto weigh = [&](auto UN, float m0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) s[decltype(UN)::value][v] -= m0;
+            static_for<ITEMS>([&](auto X) __attribute__((always_inline)) { item(UN, X); });
+        };
+        auto tile_sums = [&]() __attribute__((always_inline)) {
+            static_for<NE>([&](auto X) __attribute__((always_inline)) { read_column(X, sa); });
+            asm volatile("s_nop 7" ::: "memory");
+            static_for<U * NE>([&](auto I) __attribute__((always_inline)) { c_mfma(LONE_C(decltype(I)::value / NE), LONE_C(decltype(I)::value % NE)); });
+            asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+        };
+        auto next_rows = [&]() __attribute__((always_inline)) {
+            step_barrier();
+            next_request();
+            request_tile(sc);
+            static_for<DK>([&](auto KK) __attribute__((always_inline)) { read_row(KK, sb); });
+            rotate();
+        };
+        if constexpr (SAFE && C::MAXIMA_FIRST) {
+            // a sweep for the largest logit of the row in both units, then the sweep of the first pass where no tile needs a mask
+            float top[U], mx[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) top[u] = -INFINITY;
+            for (int jt = jt_hi; jt >= jt_lo; --jt) {
+                if (jt == jt_hi || jt < p_lo) {
+                    tile_logits(jt, d0, mx);
+#pragma unroll
+                    for (int u = 0; u < U; ++u) top[u] = fmaxf(top[u], mx[u]);
+                    next_rows();
+                    continue;
+                }
+                static_for<NE>([&](auto I) __attribute__((always_inline)) {
+                    logit_mfma(LONE_C(0), I);
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+                step_barrier();
+                next_request();
+                request_tile(sc);
+                static_for<NE>([&](auto I) __attribute__((always_inline)) {
+                    constexpr int i = decltype(I)::value;
+                    logit_mfma(LONE_C(1), I);
+                    if constexpr (i >= 2) read_row(LONE_C(i - 2), sb);              // (the MFMA that read its register is past)
+                    deal<16, i - 2, NE - 2>([&](auto X) __attribute__((always_inline)) { top[0] = fmaxf(top[0], s[0][decltype(X)::value]); });
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+                finished(s[0], s[1]);
+                static_for<2>([&](auto X) __attribute__((always_inline)) { read_row(LONE_C(NE - 2 + decltype(X)::value), sb); });
+#pragma unroll
+                for (int v = 0; v < 16; ++v) top[1] = fmaxf(top[1], s[1][v]);
+                rotate();
+            }
+            const int row = i0 + (here() & 31);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const float m = fmaxf(top[u], other_half(top[u]));
+                top[u] = row < N && row >= d0 + u && d0 + u < n_units ? m : -INFINITY;
+            }
+            round_max = fmaxf(top[0], top[1]);
+            const float ref = round_max == -INFINITY ? 0.f : round_max;
+#pragma unroll
+            for (int u = 0; u < U; ++u) mu[u] = round_max;
+            unmasked = false;
+            for (int jt = jt_hi; jt >= jt_lo;) {
+                if (jt == jt_hi || jt < p_lo) {
+                    tile_logits(jt, d0, mx);
+                    static_for<U>([&](auto UN) __attribute__((always_inline)) { weigh(UN, ref); });
+                    tile_sums();
+                    next_rows();
+                    --jt;
+                    continue;
+                }
+                enter_tile(jt);
+                aim_ahead();
+                step(no, no);
+                rotate();
+                for (--jt; jt >= p_lo && jt >= jt_lo; --jt) {
+                    aim_ahead();
+                    step(yes, no);
+                    rotate();
+                }
+                last_step();
+                asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+            }
+        } else if constexpr (SAFE) {
 #pragma unroll
             for (int u = 0; u < U; ++u) mu[u] = -INFINITY;
             for (int jt = jt_hi; jt >= jt_lo; --jt) {
@@ -454,19 +551,10 @@ __device__ __forceinline__ bool fwd_lone_block(const Problem& p, int nqb, int to
                         const float4 x = L::template get_regs<r>();
                         L::template set_regs<r>(__float_as_uint(x.x * alpha), __float_as_uint(x.y * alpha), __float_as_uint(x.z * alpha), __float_as_uint(x.w * alpha));
                     });
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) s[u][v] -= m0;
-                    static_for<ITEMS>([&](auto X) __attribute__((always_inline)) { item(UN, X); });
+                    weigh(UN, m0);
                 });
-                static_for<NE>([&](auto X) __attribute__((always_inline)) { read_column(X, sa); });
-                asm volatile("s_nop 7" ::: "memory");
-                static_for<U * NE>([&](auto I) __attribute__((always_inline)) { c_mfma(LONE_C(decltype(I)::value / NE), LONE_C(decltype(I)::value % NE)); });
-                asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
-                step_barrier();
-                next_request();
-                request_tile(sc);
-                static_for<DK>([&](auto KK) __attribute__((always_inline)) { read_row(KK, sb); });
-                rotate();
+                tile_sums();
+                next_rows();
             }
         } else {
             if (round == round0) {

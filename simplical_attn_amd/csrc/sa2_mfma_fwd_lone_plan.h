@@ -22,6 +22,7 @@ struct FwdLoneCfg {
     static constexpr int OWNED = U * (DT * 16 + DK * 4);             // accumulation registers
     static constexpr int PER_SIMD = D == 64 ? 2 : 1;                 // wavefronts per SIMD (two workgroups per CU at head_dim 64)
     static constexpr bool UNROLL = D == 128;   // tiles of a sweep in fours: 1080 against 1095 us at B1 H16 N8192 w 512/31; at head_dim 64 +3 %
+    static constexpr bool MAXIMA_FIRST = D == 128;                   // in the second pass: a sweep for the reference points (sa2_mfma_fwd_lone.h)
     using Tile = QuadTile<D>;                  // K and V tiles in LDS
     static constexpr int NREQ = Tile::NGROUP / W;                    // groups of a tile a wavefront requests
     static constexpr int TILE_BYTES = Tile::BYTES;

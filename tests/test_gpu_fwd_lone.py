@@ -24,6 +24,8 @@ BF, FP = torch.bfloat16, torch.float16
     (FP, 1, 900, 50, 64, 256, 130, 0.0),
     (BF, 1, 2500, 12, 128, 256, 150, 0.2),
     (BF, 2, 512, 4, 64, 256, 256, 0.0),
+    (FP, 1, 5000, 24, 128, 600, 12, 0.1),   # head_dim 128 where the sweeps are long enough for this kernel (FwdLoneCfg::FIRST_PAYS)
+    (BF, 1, 4001, 26, 128, 300, 32, 0.0),   # and with the pre-pass's unit
 ])
 def test_forward_matches_the_fma_kernels(dtype, B, N, H, D, w1, w2, bias):
     import simplical_attn_amd as sa
@@ -39,7 +41,7 @@ def test_forward_matches_the_fma_kernels(dtype, B, N, H, D, w1, w2, bias):
 
 
 @pytest.mark.parametrize("dtype", [BF, FP])
-@pytest.mark.parametrize("D,w2,heads", [(64, 5, 20), (64, 45, 2), (64, 16, 60), (128, 30, 200), (128, 16, 400)])
+@pytest.mark.parametrize("D,w2,heads", [(64, 5, 20), (64, 45, 2), (64, 16, 60), (128, 30, 200), (128, 16, 400), (128, 30, 300), (128, 24, 400)])
 def test_logits_that_leave_the_reference_point_behind(dtype, D, w2, heads):
     """Logits fall along the sequence, from 300 or 60 to 0 within a window: an early key outweighs the queries' own tile by hundreds of octaves."""
     import simplical_attn_amd as sa
@@ -59,6 +61,26 @@ def test_logits_that_leave_the_reference_point_behind(dtype, D, w2, heads):
     assert_close_rel(lse, want_lse.cpu(), 4e-3, "lse")
 
 
+@pytest.mark.parametrize("B,N,H,D,w1,w2,bias", [
+    (1, 1000, 9, 64, 200, 9, 0.0),
+    (1, 4115, 10, 128, 1000, 31, 0.0),
+    (1, 4001, 26, 128, 300, 32, 0.0),       # the pre-pass's unit is computed again
+    (1, 4100, 128, 128, 40, 31, 0.2),       # no tile that needs no mask
+    (1, 2500, 12, 128, 256, 150, 0.0),
+])
+def test_second_pass_on_widely_spread_logits(B, N, H, D, w1, w2, bias):
+    """fp16 weights overflow in most blocks.  Logits of standard deviation 8 are off by 8 * 2^-12 / sqrt(3) = 1.1e-3 each (products q*k2
+    rounded to 16 bits), 5e-3 at most, and an output averages what its largest weights have of it."""
+    import simplical_attn_amd as sa
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x = [(torch.randn(B, N, H, D, generator=g, device="cuda") * (2 if t < 3 else 1)).to(FP) for t in range(5)]
+    kw = dict(k2_bias=bias, v2_bias=bias)
+    out, lse = sa.simplicial_forward(*x, w1, w2, **kw)
+    want, want_lse = sa.simplicial_forward(*x, w1, w2, flags=1, **kw)
+    assert_close_rel(out, want.float().cpu(), 4e-3, "out")
+    assert_close_rel(lse, want_lse.cpu(), 4e-3, "lse")
+
+
 @pytest.mark.parametrize("D,heads,w2", [(64, 24, 20), (128, 400, 31)])
 def test_a_key_that_is_not_a_number_stays_in_its_window(D, heads, w2):
     import simplical_attn_amd as sa
@@ -70,7 +92,7 @@ def test_a_key_that_is_not_a_number_stays_in_its_window(D, heads, w2):
     assert rows[:, 350:581].all() and rows.sum().item() == 231 * heads and torch.equal(out[0].isnan().any(-1).T, rows)
 
 
-@pytest.mark.parametrize("D,N,heads,w1,w2", [(64, 1500, 6, 200, 20), (128, 4100, 16, 300, 24)])
+@pytest.mark.parametrize("D,N,heads,w1,w2", [(64, 1500, 6, 200, 20), (128, 4100, 16, 300, 24), (128, 4100, 32, 300, 24)])
 def test_layouts_and_half_open_windows(D, N, heads, w1, w2):
     """Views of one fused projection [B, N, 5, H, D] and of [B, H, N, D] tensors give what contiguous copies give, bit for bit."""
     import simplical_attn_amd as sa
