@@ -52,6 +52,7 @@ __device__ __forceinline__ bool fwd_lone_block(const Problem& p, int nqb, int to
     float* xch_m = (float*)(smem_raw + C::X_AT);              // [KW][BQ] reference points
     float* xch_l = xch_m + KW * BQ;                           // [KW][BQ] sums
     float* lam_s = xch_l + KW * BQ;                           // [BQ] reference point of the pre-pass partial
+    int* given_up = (int*)(smem_raw + C::UP_AT);              // [round % 2] a sum of the block is not finite
 
     auto here = [&]() __attribute__((always_inline)) {        // (lane parts of what happens once per round are computed there)
         int t = threadIdx.x;
@@ -202,6 +203,7 @@ __device__ __forceinline__ bool fwd_lone_block(const Problem& p, int nqb, int to
             next_request();
             request_tile(lds0 + x * C::STAGE_BYTES);
         }
+        if (tid < 2) given_up[tid] = 0;
         const float qscale = p.scale * LOG2E;
 #pragma unroll
         for (int x = 0; x < NQ; ++x) {
@@ -405,6 +407,9 @@ __device__ __forceinline__ bool fwd_lone_block(const Problem& p, int nqb, int to
     constexpr std::true_type yes{};
     constexpr std::false_type no{};
     for (int round = round0; round < round1; ++round) {
+        // A block that takes the second pass gives up the first one: what was written at the end of the round before the last
+        // one all wavefronts see alike, since every round has a barrier.
+        if (!SAFE && __builtin_amdgcn_readfirstlane(given_up[round & 1])) break;
         const int d0 = round * UPR + wave * U;                // first delta of this wavefront
         const bool any = d0 < n_units;
         request_octet(-8 * (round + 2));                      // (landed two tiles from now; their slots hold rows of no round from the last one on)
@@ -641,6 +646,10 @@ __device__ __forceinline__ bool fwd_lone_block(const Problem& p, int nqb, int to
                 static_for<U>([&](auto UN) __attribute__((always_inline)) { join(UN, yes, no, 1.f); });
             } else {
                 static_for<U>([&](auto UN) __attribute__((always_inline)) { join(UN, no, no, 1.f); });
+            }
+            if (!SAFE && __builtin_amdgcn_ballot_w64(bad)) {
+                if ((t & 63) == 0) given_up[round & 1] = 1;
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");             // (a sweep's barriers do not wait for it)
             }
         }
         L::keep_out();

@@ -32,7 +32,7 @@ struct FwdLoneCfg {
     static constexpr int QS = D + 4, AS = D + 4;                     // row strides of q and of the merged sums (fp32)
     static constexpr int K2_AT = NSTAGE * STAGE_BYTES, V2_AT = K2_AT + SLOTS / Tile::RPW * Tile::GROUP;
     static constexpr int Q_AT = V2_AT + SLOTS / Tile::RPW * Tile::GROUP, X_AT = Q_AT + BQ * QS * 4;
-    static constexpr int LDS_BYTES = X_AT + (2 * W + 1) * BQ * 4;
+    static constexpr int UP_AT = X_AT + (2 * W + 1) * BQ * 4, LDS_BYTES = UP_AT + 16;
     static_assert(W * BQ * AS * 4 <= Q_AT, "the merged sums lie over the rings");
     static_assert(LDS_BYTES <= 160 * 1024, "");
     // Gradients of the first queries, whose weights are few, follow the rounding of their outputs closely.  At head_dim 128 the

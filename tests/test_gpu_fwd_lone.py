@@ -67,6 +67,7 @@ def test_logits_that_leave_the_reference_point_behind(dtype, D, w2, heads):
     (1, 4001, 26, 128, 300, 32, 0.0),       # the pre-pass's unit is computed again
     (1, 4100, 128, 128, 40, 31, 0.2),       # no tile that needs no mask
     (1, 2500, 12, 128, 256, 150, 0.0),
+    (2, 517, 2, 64, 255, 200, 0.0),         # shares of four rounds, of which the first pass gives up the last two
 ])
 def test_second_pass_on_widely_spread_logits(B, N, H, D, w1, w2, bias):
     """fp16 weights overflow in most blocks.  Logits of standard deviation 8 are off by 8 * 2^-12 / sqrt(3) = 1.1e-3 each (products q*k2
