@@ -228,6 +228,11 @@ struct BwdSums {
 };
 int launch_bwd_sums(const Problem& p, const BwdSums& sums, int width, int dtype, hipStream_t st);
 int launch_mfma_bwd_kp(const Problem& p, int dtype, hipStream_t st, BwdSums* sums);
+// What a 16-bit launch is made of, for tests that are about one kernel: bit 0 the pre-pass runs, bit 1 the main kernel is the
+// one of sa2_mfma_fwd_lone.h or sa2_mfma_bwd_kp_lone.h, from bit 8 on shares or segments (K side: bits 0-7 K blocks per wavefront)
+int mfma_fwd_route(int B, int N, int H, int head_dim, int w1, int w2, bool force_prepass);
+int mfma_kp_route(int B, int N, int H, int head_dim, int w1, int w2, bool force_prepass);
+int mfma_kv_route(int B, int N, int H, int head_dim, int w1, int w2);
 // K-side backward kernel (dK, dV) with paired wavefronts; for small grids it splits a key block's
 // query blocks over several workgroups, whose fp32 partial sums lie in the workspace behind the
 // K'-side part (kp_side_scratch_bytes); K' windows too wide for its LDS rows are walked in segments

@@ -821,6 +821,21 @@ KpPlan kp_plan(int B, int N, int H, int D, int w1, int w2, size_t room) {
     return D == 128 ? kp_plan_of<128>(B, N, H, w1, w2, room) : D == 64 ? kp_plan_of<64>(B, N, H, w1, w2, room) : kp_plan_of<32>(B, N, H, w1, w2, room);
 }
 
+// The kernels of a launch: whether the pre-pass takes the unit delta = w2, and which main kernel runs
+struct KpRoute {
+    int left;
+    bool lone;
+};
+template <int D>
+KpRoute kp_route(int N, int w1, int w2, int64_t total, const KpPlan& pl, bool force_prepass) {
+    // one unit left over after the rounds of four: the pre-pass takes it
+    // (unless the grid is so small that a further launch costs more than the lone round)
+    const int left = pl.nseg == 1 && w2 >= NPAIR && w2 % NPAIR == 0 && (force_prepass || total >= 768) ? 1 : 0;
+    const int all = (w2 < N - 1 ? w2 : N - 1) + 1 - left, units = all < pl.segw ? all : pl.segw;
+    if constexpr (D == 64 || D == 128) return {left, KpLoneCfg<D>::fits(pl.segw - 1) && KpLoneCfg<D>::wanted(N, w1, units, total)};
+    else return {left, false};
+}
+
 template <class E, int D, bool PAD>
 int launch_kp(const Problem& p, hipStream_t st, BwdSums* sums) {
     constexpr int U = kp_units<D>();
@@ -833,11 +848,10 @@ int launch_kp(const Problem& p, hipStream_t st, BwdSums* sums) {
     const int w2s = pl.segw - 1;
     const bool raw = C::raw_fits(w2s);
     const size_t lds = C::lds_bytes(w2s, raw);
+    const KpRoute route = kp_route<D>(p.N, p.w1, p.w2, total, pl, p.force_prepass);
+    const int left = route.left;
     float* part = (float*)p.scratch;
     float* kpart = (float*)((char*)p.scratch + kp_dq_part_bytes(p.B, p.N, p.H, D, pl));
-    // one unit left over after the rounds of four: the pre-pass takes it
-    // (unless the grid is so small that a further launch costs more than the lone round)
-    const int left = (pl.nseg == 1 && p.w2 >= NPAIR && p.w2 % NPAIR == 0 && (p.force_prepass || total >= 768)) ? 1 : 0;
     if (left) {
         const size_t lds_left = (size_t)C::NSTAGE * C::STAGE * 2 + KpCfg<D, 1>::PX_BYTES;
         const int ngrp = (nkb + NPAIR - 1) / NPAIR;
@@ -847,10 +861,6 @@ int launch_kp(const Problem& p, hipStream_t st, BwdSums* sums) {
                            (int)total_left, part, 0, 1, p.w2 + 1, (float*)nullptr);
         if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
     }
-    const auto lone = [&]() {
-        if constexpr (D == 64 || D == 128) return KpLoneCfg<D>::wanted(p.N, p.w1) && KpLoneCfg<D>::fits(w2s);
-        else return false;
-    };
     auto go = [&](auto kernel) {
         if (!allow_full_lds((const void*)kernel)) return false;
         hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(KT), lds, st, p, nkb, (int)total, part, left, pl.nseg, pl.segw, kpart);
@@ -860,7 +870,7 @@ int launch_kp(const Problem& p, hipStream_t st, BwdSums* sums) {
         return pl.nseg > 1 ? (raw ? go(mfma_bwd_kp_kernel<E, D, true, false, U, true, PAD>) : go(mfma_bwd_kp_kernel<E, D, false, false, U, true, PAD>))
                            : (raw ? go(mfma_bwd_kp_kernel<E, D, true, false, U, false, PAD>) : go(mfma_bwd_kp_kernel<E, D, false, false, U, false, PAD>));
     };
-    if (lone()) {
+    if (route.lone) {
         const KpLaunch l{pl, nkb, (int)total, left, part, kpart};
         const int rc = E::DTYPE == SA2_F16 ? launch_mfma_bwd_kp_lone_fp16(p, l, st) : launch_mfma_bwd_kp_lone_bf16(p, l, st);
         if (rc != SA2_OK) return rc;
@@ -881,6 +891,15 @@ size_t kp_scratch_bytes(int B, int N, int H, int head_dim, int w1, int w2, size_
     const int D = mfma_width(head_dim);
     const KpPlan pl = kp_plan(B, N, H, D, w1, w2, room);
     return kp_dq_part_bytes(B, N, H, D, pl) + kp_part_bytes(B, N, H, D, pl);
+}
+
+int mfma_kp_route(int B, int N, int H, int head_dim, int w1, int w2, bool force_prepass) {
+    const int D = mfma_width(head_dim);
+    const KpPlan pl = kp_plan(B, N, H, D, w1, w2, ROOM_ANY);
+    const int64_t total = (int64_t)((N + BQ - 1) / BQ) * B * H * pl.nseg;
+    const KpRoute r = D == 128 ? kp_route<128>(N, w1, w2, total, pl, force_prepass) : D == 64 ? kp_route<64>(N, w1, w2, total, pl, force_prepass)
+                                                                                             : kp_route<32>(N, w1, w2, total, pl, force_prepass);
+    return r.left | (r.lone ? 2 : 0) | pl.nseg << 8;
 }
 
 int launch_mfma_bwd_kp(const Problem& p, int dtype, hipStream_t st, BwdSums* sums) {

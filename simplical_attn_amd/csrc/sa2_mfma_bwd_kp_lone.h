@@ -429,7 +429,7 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
     if (nrounds > 0) read_first_rows(sa);
 
     for (int round = 0; round < nrounds; ++round) {
-        // ---- operands, sums and row values of the round's units (one that does not exist: its neighbour's, with weights of zero) ----
+        // ---- operands, sums and row values of the round's units (one that does not exist: its neighbour's, and left out of all sums) ----
         const int d0 = round * UPR + wave * U;                // first delta of this wavefront
         const bool any = d0 < n_units;
         float lse2[U];
@@ -486,7 +486,6 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
             range(both ? d0 + 1 : d0, t2, t3, q0, q1);
             p0 = q0 > p0 ? q0 : p0;
             p1 = q1 < p1 ? q1 : p1;
-            if (U > 1 && !both) p1 = p0 - 1;                  // (the second unit is masked throughout)
         }
         const int a0 = t0 > t2 ? t0 : t2, a1 = t1 < t3 ? t1 : t3;         // tiles of all units
         bool unmasked = false;

@@ -42,13 +42,15 @@ struct KpLoneCfg {
     static bool fits(int w2) { return lds_bytes(w2, false) <= LDS_LIMIT; }
     // Whether the kernel is taken, by the keys a K' row's queries see on average (the window, less where the sequence begins).  A
     // tile of the sweep takes it 0.76 us per eight deltas (head_dim 64; the two-wavefront kernel 1.04) or 0.71 per four (128; 0.89),
-    // but what lies between two sweeps and around them is not overlapped: 2.4 and 4.0 us more per round.  Measured at B1 H16 N4096,
-    // K' windows 7 .. 31, time of the two-wavefront kernel over this one's: head_dim 64, K window 128 0.94, 256 1.00 - 1.03, 384
-    // 1.09, 512 1.08 - 1.13, 1024 1.18; head_dim 128: 256 0.94, 384 1.00, 512 1.02 - 1.04, 768 1.09, 1024 1.11.  (At head_dim 32
-    // the best was 1.03 at 512.)
-    static bool wanted(int N, int w1) {
+    // but what lies between two sweeps and around them is not overlapped: 2.4 and 4.0 us more per round, and more again once per
+    // launch and where the last wave of workgroups is not full.  Fitted to both kernels' times at 12 sizes by 12 K' windows each
+    // (profiles/plan_cuts.md): what is taken is at most 1 % slower than the other one.  `units`: deltas of a workgroup.
+    static bool wanted(int N, int w1, int units, int64_t workgroups) {
         const int64_t w = w1 < N ? w1 : N;
-        return w - w * w / (2 * (int64_t)N) >= (D == 64 ? 300 : 420);
+        const double keys = w - w * w / (2.0 * N), waves = (double)workgroups / CUS;
+        if (D == 64) return keys >= 300 && keys >= 250 + 1000.0 / units;             // (a wavefront holds two units, of which one may not exist)
+        const int rounds = (units + U * W - 1) / (U * W);
+        return keys >= 420 && keys >= 320 + (160 + 3000.0 / rounds) / waves;
     }
 };
 

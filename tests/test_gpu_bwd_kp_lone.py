@@ -24,6 +24,15 @@ BF, FP = torch.bfloat16, torch.float16
     (BF, 1, 1024, 30, 128, 1000, 64, 0.0),  # rows of q and dO from global memory
     (BF, 1, 900, 1, 128, 899, 200, 0.0),
     (BF, 1, 1500, 20, 128, 512, 1, 0.0),
+    # (the first two, and those of few deltas, take the kernel with two wavefronts per SIMD; the ones below this one, which
+    # test_routes.py watches)
+    (BF, 1, 2051, 20, 64, 512, 17, 0.0),
+    (FP, 1, 1100, 26, 64, 1000, 6, 0.3),    # the last wavefront has one unit of two
+    (FP, 4, 611, 20, 64, 2000, 33, 0.1),
+    (BF, 1, 1003, 26, 128, 900, 40, 0.0),   # the pre-pass took the last delta
+    (FP, 1, 2051, 20, 128, 900, 17, 0.2),
+    (BF, 1, 2300, 40, 128, 1500, 1, 0.0),   # two units of four
+    (BF, 1, 900, 8, 128, 899, 200, 0.0),    # segments
 ])
 def test_kp_side_matches_the_fma_kernels(dtype, B, N, H, D, w1, w2, bias):
     import simplical_attn_amd as sa
@@ -38,3 +47,24 @@ def test_kp_side_matches_the_fma_kernels(dtype, B, N, H, D, w1, w2, bias):
         assert_close_rel(got[i], want[i].cpu(), 2e-2 if dtype == BF else 1.5e-2, name, atol=2e-3)
     again = sa.simplicial_backward(*x[:5], out, lse, x[5], w1, w2, needs=(False, False, True, False, True), **kw)
     assert torch.equal(got[2], again[2]) and torch.equal(got[4], again[4])
+
+
+@pytest.mark.parametrize("D,N,heads,w1,w2", [(64, 2051, 20, 513, 18), (128, 1003, 26, 901, 41)])
+def test_layouts_and_half_open_windows(D, N, heads, w1, w2):
+    """Views of one fused projection [B, N, 5, H, D] and of [B, H, N, D] tensors give what contiguous copies give, bit for bit, in all
+    five gradients (the K-side kernel's too)."""
+    import simplical_attn_amd as sa
+    g = torch.Generator(device="cuda").manual_seed(D)
+    packed = torch.randn(1, N, 6, heads, D, generator=g, device="cuda").to(BF)
+    x = packed.unbind(2)
+    turned = [t.transpose(1, 2).contiguous().transpose(1, 2) for t in x]
+    plain = [t.contiguous() for t in x]
+    kw = dict(window_inclusive=False)
+    out, lse = sa.simplicial_forward(*plain[:5], w1, w2, **kw)
+    want = sa.simplicial_backward(*plain[:5], out, lse, plain[5], w1, w2, **kw)
+    for views in (x, turned):
+        got = sa.simplicial_backward(*views[:5], out, lse, views[5], w1, w2, **kw)
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+    exact = sa.simplicial_backward(*plain[:5], out, lse, plain[5], w1, w2, flags=1, **kw)
+    for name, a, b in zip(("dq", "dk1", "dk2", "dv1", "dv2"), want, exact):
+        assert_close_rel(a, b.cpu(), 2e-2, name, atol=2e-3)

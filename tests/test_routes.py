@@ -1,0 +1,55 @@
+"""Which kernels the 16-bit launches are made of, asked of the library on the host: the cases of the GPU tests that are about one
+kernel reach it, and plans hold where they were measured."""
+import ctypes
+
+import pytest
+
+from simplical_attn_amd import _lib
+from tests import test_gpu_bwd_kp_lone, test_gpu_bwd_kv, test_gpu_fwd_lone
+
+
+def _ask(name, B, N, H, D, w1, w2, force=None):
+    f = getattr(_lib.load(), name)          # (functions of namespace sa2, declared in csrc/sa2_common.h)
+    args = [ctypes.c_int(x) for x in (B, N, H, D, min(w1, N - 1), min(w2, N - 1))]
+    return f(*args) if force is None else f(*args, ctypes.c_bool(force))
+
+
+def forward_route(B, N, H, D, w1, w2, force=False):
+    """(pre-pass, two units per wavefront, shares)"""
+    r = _ask("_ZN3sa214mfma_fwd_routeEiiiiiib", B, N, H, D, w1, w2, force)
+    return bool(r & 1), bool(r & 2), r >> 8
+
+
+def kp_route(B, N, H, D, w1, w2, force=False):
+    """(pre-pass, one wavefront per SIMD, segments)"""
+    r = _ask("_ZN3sa213mfma_kp_routeEiiiiiib", B, N, H, D, w1, w2, force)
+    return bool(r & 1), bool(r & 2), r >> 8
+
+
+def kv_route(B, N, H, D, w1, w2):
+    """(32-row K blocks per wavefront, shares)"""
+    r = _ask("_ZN3sa213mfma_kv_routeEiiiiii", B, N, H, D, w1, w2)
+    return r & 255, r >> 8
+
+
+def _cases(test):
+    return next(m for m in test.pytestmark if m.name == "parametrize").args[1]
+
+
+@pytest.mark.parametrize("B,N,H,D,w1,w2,lone", [
+    (1, 4096, 8, 64, 512, 0, False),        # one delta: half of what a wavefront with two units computes is thrown away
+    (1, 4096, 16, 64, 512, 2, False), (1, 4096, 16, 64, 512, 6, True), (2, 2048, 8, 64, 512, 32, True),
+    (1, 4096, 16, 128, 512, 1, False), (1, 3000, 8, 128, 500, 31, False), (1, 8192, 16, 128, 512, 32, True), (1, 32768, 8, 128, 1024, 64, True),
+])
+def test_kp_side_by_keys_deltas_and_grid(B, N, H, D, w1, w2, lone):
+    assert kp_route(B, N, H, D, w1, w2)[1] == lone
+
+
+def test_kp_cases_reach_the_kernel():
+    cases = _cases(test_gpu_bwd_kp_lone.test_kp_side_matches_the_fma_kernels)
+    at = next(i for i, c in enumerate(cases) if c[1:4] == (1, 2051, 20))
+    routes = {c[1:7]: kp_route(*c[1:7]) for c in cases[at:]}
+    assert all(lone for _, lone, _ in routes.values())
+    assert routes[1, 1003, 26, 128, 900, 40][0] and routes[1, 900, 8, 128, 899, 200][2] > 1
+    for D, N, heads, w1, w2 in _cases(test_gpu_bwd_kp_lone.test_layouts_and_half_open_windows):
+        assert kp_route(1, N, heads, D, w1 - 1, w2 - 1)[1]
