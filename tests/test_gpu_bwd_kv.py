@@ -25,6 +25,8 @@ BF, FP = torch.bfloat16, torch.float16
     (BF, 1, 321, 1, 128, 31, 120, 0.0),     # the widest window that LDS holds ...
     (BF, 1, 321, 1, 128, 1000, 121, 0.0),   # ... and one more
     (BF, 1, 700, 1, 64, 33, 511, 0.1),
+    (FP, 2, 17, 4, 64, 16, 16, 0.0),        # one query block, in shares of two and three units
+    (BF, 1, 31, 2, 32, 20, 30, 0.2),
 ])
 def test_k_side_matches_the_fma_kernels(dtype, B, N, H, D, w1, w2, bias):
     import simplical_attn_amd as sa

@@ -53,3 +53,17 @@ def test_kp_cases_reach_the_kernel():
     assert routes[1, 1003, 26, 128, 900, 40][0] and routes[1, 900, 8, 128, 899, 200][2] > 1
     for D, N, heads, w1, w2 in _cases(test_gpu_bwd_kp_lone.test_layouts_and_half_open_windows):
         assert kp_route(1, N, heads, D, w1 - 1, w2 - 1)[1]
+
+
+def test_kv_cases_have_both_geometries_and_shares():
+    routes = {c[1:7]: kv_route(*c[1:7]) for c in _cases(test_gpu_bwd_kv.test_k_side_matches_the_fma_kernels)}
+    assert routes[4, 520, 64, 64, 300, 3] == (2, 1) and routes[1, 400, 130, 64, 390, 0] == (2, 1) and routes[1, 129, 1, 64, 40, 33][1] > 1
+    assert routes[2, 17, 4, 64, 16, 16] == (1, 8) and routes[1, 31, 2, 32, 20, 30][1] > 1
+
+
+@pytest.mark.parametrize("B,N,H,D,w1,w2,want", [
+    (2, 17, 4, 64, 128, 24, (1, 8)), (2, 17, 4, 16, 128, 24, (1, 8)), (2, 9, 4, 64, 128, 24, (1, 1)),       # one query block
+    (5, 448, 29, 32, 816, 96, (1, 2)), (2, 2048, 8, 64, 512, 32, (2, 2)), (1, 8192, 16, 128, 512, 32, (1, 1)),
+])
+def test_k_side_plan(B, N, H, D, w1, w2, want):
+    assert kv_route(B, N, H, D, w1, w2) == want
