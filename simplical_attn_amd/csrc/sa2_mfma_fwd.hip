@@ -1021,14 +1021,31 @@ inline int fwd_side_span(const Problem& p) {
     return deltas - 1 < p.w2 ? deltas - 1 : p.w2;
 }
 
+// The kernels of a launch: whether the pre-pass takes the unit delta = w2, and which main kernel runs
+struct FwdRoute {
+    int left;
+    bool two_units;
+};
+template <int D>
+FwdRoute fwd_route(int N, int w1, int w2, int64_t total, int nsplit, bool force_prepass) {
+    // one unit left over after the rounds of eight: the pre-pass takes it, unless the grid is so
+    // small that a further launch costs more than the lone round (also with two units per wavefront: B1 H16 N8192 D64 w 512/32
+    // 626 us with it, 654 without; B1 H16 N4096 w 256/8 79 and 90; B1 H16 N1600 w 256/16, 800 workgroups, 66 and 60)
+    const int left = nsplit <= 1 && w2 >= FW && w2 % FW == 0 && (force_prepass || total >= PREPASS_MIN_WORKGROUPS) ? 1 : 0;
+    if constexpr (D >= 64) {
+        using L = FwdLoneCfg<D>;
+        if (nsplit <= 1 || !L::FIRST_ELSEWHERE)
+            return {left, L::wanted(total * (nsplit > 1 ? nsplit : 1), (w2 < N - 1 ? w2 : N - 1) + 1 - left, N, w1)};
+    }
+    return {left, false};
+}
+
 template <class E, int D, bool SIDE, bool PAD>
 int launch_fwd_kernels(const Problem& p, int nqb, int total, hipStream_t st) {
     using C = Cfg<D>;
     const size_t lds = C::lds_bytes(fwd_side_span(p));
-    // one unit left over after the rounds of eight: the pre-pass takes it, unless the grid is so
-    // small that a further launch costs more than the lone round (also with two units per wavefront: B1 H16 N8192 D64 w 512/32
-    // 626 us with it, 654 without; B1 H16 N4096 w 256/8 79 and 90; B1 H16 N1600 w 256/16, 800 workgroups, 66 and 60)
-    const int left = (p.nsplit <= 1 && p.w2 >= FW && p.w2 % FW == 0 && (p.force_prepass || total >= PREPASS_MIN_WORKGROUPS)) ? 1 : 0;
+    const FwdRoute route = fwd_route<D>(p.N, p.w1, p.w2, total, p.nsplit, p.force_prepass);
+    const int left = route.left;
     if (left) {
         const int ngrp = (nqb + FW - 1) / FW;
         const int total_left = ngrp * (total / nqb);
@@ -1043,17 +1060,14 @@ int launch_fwd_kernels(const Problem& p, int nqb, int total, hipStream_t st) {
         return hipGetLastError() == hipSuccess;
     };
     if constexpr (!PAD && D >= 64) {
-        using L = FwdLoneCfg<D>;
-        if (p.nsplit <= 1 || !L::FIRST_ELSEWHERE) {
+        if (route.two_units) {
             const int64_t grid = (int64_t)total * (p.nsplit > 1 ? p.nsplit : 1);
-            if (L::wanted(grid, (p.w2 < p.N - 1 ? p.w2 : p.N - 1) + 1 - left, p.N, p.w1)) {
-                if (grid > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
-                // (one block per head: the first one)
-                if (L::FIRST_ELSEWHERE && !go(mfma_fwd_kernel<E, D, MODE_FAST, SIDE, PAD, false>, total / nqb, 1)) return SA2_ERR_LAUNCH_FAILED;
-                const FwdLoneArgs args{p, nqb, (int)grid, left};
-                const int rc = E::DTYPE == SA2_F16 ? launch_mfma_fwd_lone_fp16(args, st) : launch_mfma_fwd_lone_bf16(args, st);
-                return rc != SA2_OK || p.nsplit <= 1 ? rc : launch_fwd_merge(p, D, E::DTYPE, st);
-            }
+            if (grid > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
+            // (one block per head: the first one)
+            if (FwdLoneCfg<D>::FIRST_ELSEWHERE && !go(mfma_fwd_kernel<E, D, MODE_FAST, SIDE, PAD, false>, total / nqb, 1)) return SA2_ERR_LAUNCH_FAILED;
+            const FwdLoneArgs args{p, nqb, (int)grid, left};
+            const int rc = E::DTYPE == SA2_F16 ? launch_mfma_fwd_lone_fp16(args, st) : launch_mfma_fwd_lone_bf16(args, st);
+            return rc != SA2_OK || p.nsplit <= 1 ? rc : launch_fwd_merge(p, D, E::DTYPE, st);
         }
     }
     if (p.nsplit <= 1) return go(mfma_fwd_kernel<E, D, MODE_FAST, SIDE, PAD, false>, total, nqb) ? SA2_OK : SA2_ERR_LAUNCH_FAILED;
@@ -1104,6 +1118,14 @@ int mfma_fwd_nsplit(int B, int N, int H, int D, int w1, int w2, bool force_prepa
     return force_prepass && w2 >= FW && w2 % FW == 0 ? 1 : plan_forward(B, N, H, mfma_width(D), w1, w2, FW);
 }
 size_t mfma_fwd_part_bytes(int B, int N, int H, int D, int nsplit) { return fwd_part_bytes(B, N, H, mfma_width(D), nsplit); }
+
+int mfma_fwd_route(int B, int N, int H, int D, int w1, int w2, bool force_prepass) {
+    const int nsplit = mfma_fwd_nsplit(B, N, H, D, w1, w2, force_prepass);
+    const int64_t total = (int64_t)((N + BQ - 1) / BQ) * B * H;
+    const FwdRoute r = D == 128 ? fwd_route<128>(N, w1, w2, total, nsplit, force_prepass) : D == 64 ? fwd_route<64>(N, w1, w2, total, nsplit, force_prepass)
+                                                                                                   : fwd_route<32>(N, w1, w2, total, nsplit, force_prepass);
+    return r.left | (r.two_units ? 2 : 0) | nsplit << 8;
+}
 
 int launch_mfma_fwd(const Problem& p, int dtype, hipStream_t st) {
     const int nqb = (p.N + BQ - 1) / BQ;

@@ -41,7 +41,7 @@ def test_forward_matches_the_fma_kernels(dtype, B, N, H, D, w1, w2, bias):
 
 
 @pytest.mark.parametrize("dtype", [BF, FP])
-@pytest.mark.parametrize("D,w2,heads", [(64, 5, 20), (64, 45, 2), (64, 16, 60), (128, 30, 200), (128, 16, 400), (128, 30, 300), (128, 24, 400)])
+@pytest.mark.parametrize("D,w2,heads", [(64, 5, 20), (64, 45, 2), (64, 16, 60), (128, 30, 200), (128, 16, 400), (128, 30, 300), (128, 24, 400), (64, 130, 6)])
 def test_logits_that_leave_the_reference_point_behind(dtype, D, w2, heads):
     """Logits fall along the sequence, from 300 or 60 to 0 within a window: an early key outweighs the queries' own tile by hundreds of octaves."""
     import simplical_attn_amd as sa

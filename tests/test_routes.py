@@ -55,6 +55,23 @@ def test_kp_cases_reach_the_kernel():
         assert kp_route(1, N, heads, D, w1 - 1, w2 - 1)[1]
 
 
+def test_forward_cases_reach_the_kernel():
+    t = test_gpu_fwd_lone
+    routes = [(c[0], c[4], *forward_route(*c[1:7])) for c in _cases(t.test_forward_matches_the_fma_kernels)]
+    reached = {(dtype, D, left) for dtype, D, left, two, shares in routes if two}
+    assert {(t.BF, 64, False), (t.FP, 64, False), (t.BF, 64, True), (t.BF, 128, False), (t.FP, 128, False), (t.BF, 128, True)} <= reached
+    assert any(two and shares > 1 for _, _, _, two, shares in routes)
+    far = next(m.args[1] for m in t.test_logits_that_leave_the_reference_point_behind.pytestmark if "," in m.args[0])
+    routes = {(D, w2, heads): forward_route(1, 470, heads, D, 300, w2) for D, w2, heads in far}
+    assert routes[64, 5, 20][1:] == (True, 1) and routes[64, 16, 60][:2] == (True, True) and routes[128, 30, 300][:2] == (False, True)
+    assert routes[128, 24, 400][:2] == (True, True) and routes[64, 130, 6][1] and routes[64, 130, 6][2] > 1
+    for c in _cases(t.test_second_pass_on_widely_spread_logits):
+        assert forward_route(*c[:6])[1]
+    for D, heads, w2 in _cases(t.test_a_key_that_is_not_a_number_stays_in_its_window):
+        assert forward_route(1, 600, heads, D, 230, w2)[1]
+    assert {c[0] for c in _cases(t.test_layouts_and_half_open_windows) if forward_route(1, c[1], c[2], c[0], c[3] - 1, c[4] - 1)[1]} == {64, 128}
+
+
 def test_kv_cases_have_both_geometries_and_shares():
     routes = {c[1:7]: kv_route(*c[1:7]) for c in _cases(test_gpu_bwd_kv.test_k_side_matches_the_fma_kernels)}
     assert routes[4, 520, 64, 64, 300, 3] == (2, 1) and routes[1, 400, 130, 64, 390, 0] == (2, 1) and routes[1, 129, 1, 64, 40, 33][1] > 1
