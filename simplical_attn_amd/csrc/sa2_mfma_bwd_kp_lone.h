@@ -316,18 +316,16 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
     };
     // One unit: A(t), then C(t-1), whose four groups of MFMAs (R^T and G^T, each from the keys' first and second half) free
     // the halves of P and dS one after the other for B(t).
-    constexpr int BAR = LONG ? 2 * DT : 0;                    // MFMA of phase C that the tile's barrier stands before
+    constexpr int BAR = 2 * DT;                               // MFMA of phase C that the tile's barrier stands before
     auto single = [&](auto DO_C) __attribute__((always_inline)) {
         constexpr bool CC = decltype(DO_C)::value;
+        static_assert(LONG && sizeof(DO_C) > 0, "one unit per wavefront: head_dim 128");
         static_for<NE>([&](auto I) __attribute__((always_inline)) {
             constexpr int i = decltype(I)::value;
             a_mfma(LONE_C(0), I);
-            if constexpr (LONG && i < DK) read_row(LONE_C(1), I, sa);
+            if constexpr (i < DK) read_row(LONE_C(1), I, sa);
             next_piece(LONE_C(i - 1));
-            if constexpr (CC) {
-                if constexpr (LONG) deal<12, i - 4, 12>([&](auto X) __attribute__((always_inline)) { read_column(X, sc); });
-                else deal<4 * DT, i, NE - 2>([&](auto X) __attribute__((always_inline)) { read_column(X, sc); });
-            }
+            if constexpr (CC) deal<12, i - 4, 12>([&](auto X) __attribute__((always_inline)) { read_column(X, sc); });
             __builtin_amdgcn_sched_barrier(0);
         });
         static_for<NE>([&](auto I) __attribute__((always_inline)) {
@@ -335,14 +333,13 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
             if constexpr (i == BAR) step_barrier();
             if constexpr (CC) {
                 c_mfma(LONE_C(0), I);
-                if constexpr (LONG && i < 4) read_column(LONE_C(12 + i), sc);
+                if constexpr (i < 4) read_column(LONE_C(12 + i), sc);
             }
-            if constexpr (LONG && i >= BAR) read_row(LONE_C(0), LONE_C(i - BAR), sb);
-            if constexpr (!LONG) read_row(LONE_C(i / DK), LONE_C(i % DK), sb);
+            if constexpr (i >= BAR) read_row(LONE_C(0), LONE_C(i - BAR), sb);
             if constexpr (group == 1 || group == 2) deal<8, i - DT, 2 * DT>([&](auto X) __attribute__((always_inline)) { p_item(LONE_C(0), X); });
             if constexpr (group == 3) deal<4, i - 3 * DT, DT>([&](auto X) __attribute__((always_inline)) { ds_item(LONE_C(0), X); });
             if constexpr (i == BAR) request_tile(sc, true, false);
-            if constexpr (i == (LONG ? BAR + 4 : NE - 1)) request_tile(sc, false, true);
+            if constexpr (i == BAR + 4) request_tile(sc, false, true);
             __builtin_amdgcn_sched_barrier(0);
         });
         static_for<4>([&](auto X) __attribute__((always_inline)) { ds_item(LONE_C(0), LONE_C(4 + decltype(X)::value)); });

@@ -763,7 +763,8 @@ int launch_fwd_lone_width(const FwdLoneArgs& args, hipStream_t st) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)args.total), dim3(C::T), C::LDS_BYTES, st, args);
         return hipGetLastError() == hipSuccess ? SA2_OK : SA2_ERR_LAUNCH_FAILED;
     };
-    return args.p.nsplit > 1 ? go(mfma_fwd_lone_kernel<E, D, true>) : go(mfma_fwd_lone_kernel<E, D, false>);
+    if constexpr (C::FIRST_ELSEWHERE) return args.p.nsplit > 1 ? SA2_ERR_UNSUPPORTED : go(mfma_fwd_lone_kernel<E, D, false>);
+    else return args.p.nsplit > 1 ? go(mfma_fwd_lone_kernel<E, D, true>) : go(mfma_fwd_lone_kernel<E, D, false>);
 }
 template <class E>
 int launch_fwd_lone(const FwdLoneArgs& args, hipStream_t st) {
