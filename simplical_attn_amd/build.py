@@ -33,11 +33,13 @@ FLAGS = [
     "-Wno-unused-command-line-argument",
     "-I", os.path.join(ROOT, "include"), "-I", CSRC,
 ]
-# sources with hand-placed MFMAs -> their kernels and the accumulation registers these own; the compiler's listing of them
-# is checked (see listing_check.py)
-HAND_PLACED = {"sa2_mfma_bwd_kv_bf16.hip": ("mfma_bwd_kv_kernel", 192), "sa2_mfma_bwd_kv_fp16.hip": ("mfma_bwd_kv_kernel", 192),
-               "sa2_mfma_bwd_kp_lone_bf16.hip": ("mfma_bwd_kp_lone_kernel", 256), "sa2_mfma_bwd_kp_lone_fp16.hip": ("mfma_bwd_kp_lone_kernel", 256),
-               "sa2_mfma_fwd_lone_bf16.hip": ("mfma_fwd_lone_kernel", 96), "sa2_mfma_fwd_lone_fp16.hip": ("mfma_fwd_lone_kernel", 96)}
+# sources with hand-placed MFMAs -> their kernels (patterns of the mangled names, ...Li128E...: head_dim 128) and the
+# accumulation registers these own (OWNED of their Lone<>); the compiler's listing of them is checked (see listing_check.py)
+_KV, _KP = (("mfma_bwd_kv_kernel", 192),), (("mfma_bwd_kp_lone_kernel", 256),)
+_FWD = (("mfma_fwd_lone_kernel.*Li64E", 96), ("mfma_fwd_lone_kernel.*Li128E", 192))
+HAND_PLACED = {"sa2_mfma_bwd_kv_bf16.hip": _KV, "sa2_mfma_bwd_kv_fp16.hip": _KV,
+               "sa2_mfma_bwd_kp_lone_bf16.hip": _KP, "sa2_mfma_bwd_kp_lone_fp16.hip": _KP,
+               "sa2_mfma_fwd_lone_bf16.hip": _FWD, "sa2_mfma_fwd_lone_fp16.hip": _FWD}
 
 
 def _compile(src, extra):
@@ -54,7 +56,8 @@ def _compile(src, extra):
     if res.returncode != 0:
         raise RuntimeError("hipcc failed on %s:\n%s" % (src, err))
     if keep:
-        listing_check.check(glob.glob(os.path.join(tmp, "*gfx950*.s"))[0], *HAND_PLACED[name])
+        for kernels, owned in HAND_PLACED[name]:
+            listing_check.check(glob.glob(os.path.join(tmp, "*gfx950*.s"))[0], kernels, owned)
         os.replace(out, obj)
         shutil.rmtree(tmp)
     return obj, err

@@ -25,12 +25,12 @@ def _regs(text):
 
 
 def violations(lines, kernels, owned):
-    """Rule breaks in a compiler listing (an iterable of lines) of the functions whose name holds `kernels`, and their number."""
+    """Rule breaks in a compiler listing (an iterable of lines) of the functions whose name matches `kernels`, and their number."""
     bad, found, on, hand, name = [], 0, False, False, ""
     for line in lines:
         m = re.match(r"^(_Z\w+|\w+_kernel\w*):", line)
         if m:
-            name, on, hand = m.group(1), kernels in m.group(1), False
+            name, on, hand = m.group(1), bool(re.search(kernels, m.group(1))), False
             found += on
             recent, tiles, at, mfmas = [], {}, 0, 0
             continue

@@ -30,3 +30,17 @@ def test_planted_breaks(old, new, rule):
     bad, found = listing_check.violations(CLEAN.replace(old, new, 1).splitlines(), "k_kernel", 192)
     assert found == 1
     assert {b[0] for b in bad} == (set() if rule is None else {rule})
+
+
+@pytest.mark.parametrize("name,register", [("_Z20mfma_fwd_lone_kernelI8ElemBF16Li128ELb0EEv", 150), ("_Z20mfma_fwd_lone_kernelI7ElemF16Li64ELb1EEv", 95),
+                                           ("_Z18mfma_bwd_kv_kernelI7ElemF16Li64EEv", 191), ("_Z23mfma_bwd_kp_lone_kernelI7ElemF16Li64EEv", 255)])
+def test_every_owned_register_is_watched(name, register):
+    """The table that the build uses finds an instruction of the compiler's in any register that a kernel owns."""
+    from simplical_attn_amd import build
+    code = CLEAN.replace("k_kernel", name).replace("a192, v9", "a%d, v9" % register)
+    found = {}
+    for source, kernels in build.HAND_PLACED.items():
+        for pattern, owned in kernels:
+            found.setdefault(source, []).extend(r[0] for r in listing_check.violations(code.splitlines(), pattern, owned)[0])
+    hits = [source for source, rules in found.items() if rules]
+    assert len(hits) == 2 and all(found[s] == [1] for s in hits)       # the bf16 and the fp16 source of that kernel
