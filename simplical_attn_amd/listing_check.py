@@ -6,6 +6,8 @@ nor guards): build.py runs it on every build and refuses code that breaks one of
 2. Two instructions lie between a vector instruction that writes an operand of an MFMA and that MFMA.
 3. What an MFMA writes to vector registers is read, or overwritten by something else, no sooner than two further MFMAs or
    twenty instructions later.
+4. Only the hand-placed instructions name m0 (they write it, and it is a reserved register that an asm statement cannot declare
+   as destroyed).
 Branches are ignored: instructions are taken in the order they stand in.
 """
 import re
@@ -49,6 +51,8 @@ def violations(lines, kernels, owned):
         src = _regs(",".join(args)) if store else _regs(",".join(args[1:]))
         if not hand and any(r[0] == "a" and r[1] < owned for r in dst | src):
             bad.append((1, name, text))
+        if not hand and re.search(r"\bm0\b", text):
+            bad.append((4, name, text))
         if mfma:
             if any(w & src for o, w in recent[-2:] if o.startswith("v_") and not o.startswith("v_mfma")):
                 bad.append((2, name, text))

@@ -25,6 +25,7 @@ CLEAN = """k_kernel:
     ("v_accvgpr_write_b32 a192", "v_accvgpr_write_b32 a191", 1),
     ("v_mov_b32_e32 v8, 0", "v_mov_b32_e32 v4, 0", 2),
     ("\tv_mfma_f32_32x32x16_bf16 a[16:31], v[4:7], v[0:3], a[16:31]\n", "", 3),
+    ("v_mov_b32_e32 v8, 0", "s_mov_b32 m0, s4", 4),
 ])
 def test_planted_breaks(old, new, rule):
     bad, found = listing_check.violations(CLEAN.replace(old, new, 1).splitlines(), "k_kernel", 192)
