@@ -89,7 +89,9 @@ bool allow_full_lds(const void* kernel);
 // sequence), the plans below cut the work of a workgroup into shares with fp32 partial sums, which cost their write and
 // read (2.5 MB per unit of time, a sweep step of about 1 us) and a summation launch.  The constants are the ones whose
 // choices lost least against the best of up to sixteen measured cuts (2.6 % on average for the K'-side kernel at nineteen
-// sizes; the 16-bit K-side kernel has its own, see kv_plan).  All plans depend on the problem's sizes only.
+// sizes; the 16-bit K-side kernel has its own, see kv_plan).  In 16 bits they were measured with paired wavefronts on the K' side and
+// one unit per wavefront in the forward, and hold for what runs there now as far as its times are alike.  All plans depend on
+// the problem's sizes only.
 constexpr int CUS = 256;
 inline double grid_time(int64_t workgroups, double longest, double mean) {
     const int64_t waves = workgroups / CUS;
@@ -233,8 +235,8 @@ int launch_mfma_bwd_kp(const Problem& p, int dtype, hipStream_t st, BwdSums* sum
 int mfma_fwd_route(int B, int N, int H, int head_dim, int w1, int w2, bool force_prepass);
 int mfma_kp_route(int B, int N, int H, int head_dim, int w1, int w2, bool force_prepass);
 int mfma_kv_route(int B, int N, int H, int head_dim, int w1, int w2);
-// K-side backward kernel (dK, dV) with paired wavefronts; for small grids it splits a key block's
-// query blocks over several workgroups, whose fp32 partial sums lie in the workspace behind the
+// K-side backward kernel (dK, dV), one wavefront per SIMD; for small grids it splits a key block's stream of
+// units over several workgroups, whose fp32 partial sums lie in the workspace behind the
 // K'-side part (kp_side_scratch_bytes); K' windows too wide for its LDS rows are walked in segments
 size_t kv_split_scratch_bytes(int B, int N, int H, int D, int w1, int w2, size_t room);
 size_t kp_side_scratch_bytes(int B, int N, int H, int D, int w1, int w2, size_t room);

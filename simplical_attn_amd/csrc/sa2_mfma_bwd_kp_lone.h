@@ -8,9 +8,9 @@
 // B between the MFMAs of A and C of the other unit (of the next tile at head_dim 128), operand reads eight MFMAs ahead of their
 // use: nothing is handed from one wavefront to another, and every operand read serves all units of the wavefront.
 // What bounds it: at head_dim 64 the instructions beside the MFMAs (32 MFMAs per tile, 0.44 us of 0.76; 18 tiles take 14 us of
-// a round's 23, masks 1.8, the sums over the units and dQ 3, forming 1); at head_dim 128 also power.  K' side with its
-// pre-pass, against the two-wavefront kernel: B2 H8 N2048 D64 w 512/32 427 -> 392 us, B1 H16 N8192 D128 w 512/32 2835 -> 2737,
-// B1 H8 N8192 w 1024/64 D128 4675 -> 4219, D64 2571 -> 2170 (bf16; dS from unrounded weights).  With the rounding 388 and 2728.
+// a round's 23, masks 1.8, the sums over the units and dQ 3, forming 1); at head_dim 128 also power.  K' side with row term,
+// pre-pass and sums against the two-wavefront kernel, in turn on one machine (bf16): B2 H8 N2048 D64 w 512/32 428 -> 400 us,
+// B1 H16 N8192 D128 w 512/32 2831 -> 2747, B1 H8 N8192 w 1024/64 D128 4780 -> 4451, D64 2590 -> 2250.
 #pragma once
 
 #include "sa2_mfma_bwd_kp_plan.h"
@@ -298,10 +298,12 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
         s[u][e + 1] = y;
         if constexpr (i > 0) round_p(UN, LONE_C(i - 1));
     };
-    // dS from the rounded weights, as in the two-wavefront kernel: the first queries have few weights, all large, and their gradients
-    // follow the rounding of each closely (from the unrounded ones they came out up to 0.6 of a gradient's root mean square
-    // elsewhere, B1 H8 N32768 D128 w 1024/64; now 0.03).  It costs two instructions a pair, 3 % of a training step.  (A second
-    // copy of the sweep for the first queries alone does not fit the registers: 560 bytes per lane of scratch.)
+    // dS from the rounded weights, as in the two-wavefront kernel, so that a gradient does not depend on which of them a problem is
+    // given to: the first queries have few weights, all large, and single gradients there follow the rounding of each (up to 0.6 of
+    // a gradient's root mean square elsewhere from the unrounded ones, B1 H8 N32768 D128 w 1024/64; now 0.03).  It is not the more
+    // exact way: against fp32 the unrounded weights give dQ, dK and dK' errors 4 - 9 % smaller in the 2-norm, the first queries
+    // included, and worst elements that move both ways.  It costs two instructions a pair, in both backward kernels together 1 - 3 % of a
+    // training step.  (A second copy of the sweep for the first queries alone does not fit the registers: 560 bytes per lane of scratch.)
     auto ds_item = [&](auto UN, auto I) __attribute__((always_inline)) {
         constexpr int u = decltype(UN)::value, i = decltype(I)::value, ks = i / 4, t = i % 4, e = 2 * i;
         if constexpr (i == 0) round_p(UN, LONE_C(7));

@@ -13,8 +13,8 @@
 // stand between the MFMAs of A(t+1) and C(t), operand reads eight MFMAs ahead of their use.
 // The arrangement before it (two wavefronts per SIMD, one with S, P and dV, one with dP, dS and dK, P handed over in LDS, a
 // barrier per unit) ran matrix pipe, vector ALU and LDS one after the other, 2500 cycles per unit of 1024 MFMA cycles; here
-// it is 1700 to 1800.  With the row-term kernel, us: B2 H8 N2048 D64 w 512/32 458 -> 317, B1 H16 N8192 D128 w 512/32
-// 2714 -> 2315 (309 and 2260 with dS from unrounded weights; at D128 the board's power is the next limit).
+// it is 1700 to 1800.  With the row-term kernel, us: B2 H8 N2048 D64 w 512/32 458 -> 323, B1 H16 N8192 D128 w 512/32
+// 2715 -> 2300 (312 and 2280 with dS from unrounded weights; at D128 the board's power is the next limit).
 //
 // Small grids (fewer workgroups than the chip holds) split a key block's stream of units over up to sixteen workgroups
 // (shares of whole units, at least four each); each writes its fp32 partial dK and dV to the workspace and bwd_sum_kernel

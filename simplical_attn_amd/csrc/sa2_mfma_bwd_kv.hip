@@ -19,7 +19,7 @@ constexpr int KV_MIN_SHARE = 4, KV_MIN_SHARE_ONE = 2;      // units a share hold
 // 3 - 18 % off at 12 (most of one head or up to 64 queries, 1 to 3 us), and 43 % where the bytes bind.  The partial sums
 // stay under what SA2_STATIC_WORKSPACE_BYTES leaves beside the K'-side kernel's, or 128 MiB where those alone exceed it.
 // Measured with the row term and the sums (us, the kernel with two wavefronts per SIMD -> now): B2 H4 N512 D64 w 256/256
-// 256 -> 185, B3 H6 N777 D64 w 100/20 102 -> 68, B2 H8 N2048 D64 w 512/32 458 -> 330, B5 H29 N448 D32 w 816/96 1183 -> 1130 (two
+// 256 -> 185, B3 H6 N777 D64 w 100/20 102 -> 68, B2 H8 N2048 D64 w 512/32 458 -> 323, B5 H29 N448 D32 w 816/96 1183 -> 1130 (two
 // shares, all that the bytes allow; the best eight take 790), B1 H4 N2048 D128 w 512/32 199 -> 160, B2 H4 N17 D64 w 16/16 14.2 -> 13.8.
 // At head_dim 128 and up to 130 queries the present kernel is 1 to 2 us slower than that one (B2 H4 w 128/24, N 33 18.4 -> 20.3, N 130
 // 30.8 -> 31.6): its own time, 12.8 -> 14.7 us for shares of five units.

@@ -10,10 +10,10 @@
 // R * (v2 + bias) stay in registers for all rounds and the four wavefronts are merged once, in fp32.  The K' and V' rows are
 // a ring of 64 rows in LDS, of which a round needs 39 and eight new ones: any K' window.
 //
-// At head_dim 128 a wavefront has a SIMD to itself (508 registers).  At head_dim 64 it needs 256 and two workgroups share a CU: one
+// At head_dim 128 a wavefront has a SIMD to itself (504 registers).  At head_dim 64 it needs 256 and two workgroups share a CU: one
 // computes under the prologue, the forming of Q~ and the merge of the other, and scalar, LDS and vector instructions of one issue
 // beside those of the other (one workgroup per CU: 176 us where two take 146, B2 H8 N2048 w 512/31).
-// What bounds it: the instructions beside the MFMAs.  An MFMA takes 33 cycles, under which four others are free; a tile has 32 (head_dim
+// What bounds it: the instructions beside the MFMAs (sa2_mfma_lone.h: four of them are free under each).  A tile has 32 (head_dim
 // 128) or 16 MFMAs and 145 or 110 others.  Forward, bf16: B1 H16 N8192 D128 w 512/32 1274 -> 1174 us, B2 H8 N2048 D64 w 512/31
 // 180 -> 146, B1 H16 N4096 D64 w 64/31 153 -> 98, B2 H4 N512 D64 w 256/256 128 -> 100.  (A(0) taken in turn
 // with C'(0), A(1) with C'(1), so that no MFMA follows the one it adds to: 2 % slower at head_dim 128.)
@@ -33,9 +33,10 @@ namespace {
 // (FwdLoneCfg::FIRST_ELSEWHERE), a sweep of the logit MFMAs alone finds the largest logit of a row in both units, and the sweep of
 // the first pass follows from that point, with explicit masks where a tile needs them.  (Following the maxima there, a wavefront
 // alone on its SIMD ran MFMAs, exponentials and the rescaling of sums one after the other, and the second pass cost more than that of
-// the eight-wavefront kernel.  Forward, us, eight wavefronts / maxima followed / this; fp16 B1 H16 N8192 w 512/32, q, k1 and k2
-// N(0, std^2): std 1.25 2160 / 1750 / 1600, 1.5 3320 / 4370 / 3265, 2 and more 3270 / 4600 / 3430; bf16, std 2 1309 / 1305 / 1238,
-// 3 3165 / 4570 / 3380.  At head_dim 64 following costs less than the pass it replaced: fp16 B2 H8 N2048 w 512/32, std 2 582 / 559.)
+// the eight-wavefront kernel.)  A block that has found a sum that is not finite gives the first pass up two rounds later.
+// Forward, us, eight wavefronts / maxima followed / this; fp16 B1 H16 N8192 D128 w 512/32, q, k1 and k2 N(0, std^2): std 1 (no second
+// pass) 1324 / 1249 / 1259, 1.25 2206 / 1644 / 1463, 1.5 3287 / 4368 / 2836, 2 and more 3274 / 4608 / 2942; bf16, std 2 1268 / 1196 / 1192,
+// 3 3167 / 4563 / 2886.  fp16 B2 H8 N2048 D64 w 512/32, std 2 582 / 559 / 492 (maxima followed: rescaling costs two wavefronts per SIMD less).
 template <class E, int D, bool SAFE, bool SPLIT>
 __device__ __forceinline__ bool fwd_lone_block(const Problem& p, int nqb, int total, int left) {
     typedef typename E::scalar EL;

@@ -1,9 +1,9 @@
-// Building blocks of the kernels that run one wavefront per SIMD with all 512 registers and place their MFMAs by hand
-// (16-bit backward, head_dim up to 128).
+// Building blocks of the 16-bit kernels that place their MFMAs by hand, head_dim up to 128: one wavefront per SIMD with up to
+// 512 registers (forward at head_dim 128, both backward kernels) or two with 256 each (forward at head_dim 64).
 //
 // A lone wavefront hides its latencies itself, so the order of instructions is fixed in the source (a sched_barrier behind
-// every MFMA).  What costs what was measured on the instructions alone: an MFMA takes 33 cycles, under which five more vector
-// instructions are free; a read of LDS takes 4 to 7 of its own right behind an MFMA and 14 behind vector instructions; an
+// every MFMA).  What costs what was measured on the instructions alone: an MFMA takes 33 cycles, under which four more vector
+// instructions are free (with six it takes 45, with eight 48); a read of LDS takes 4 to 7 of its own right behind an MFMA and 14 behind vector instructions; an
 // s_nop up to 9, which is why no instruction there reads the result of an exponential or the operand of an MFMA just written.
 //
 // The MFMAs are opaque to the compiler, which neither guards nor schedules them: listing_check.py looks over what it makes

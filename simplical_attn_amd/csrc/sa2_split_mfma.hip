@@ -22,7 +22,8 @@
 // transposed (S^T = K1 . Q~^T) a lane's accumulator registers are, once split, the B operand of R^T += V1^T . P^T.
 //
 // K/V (or unit) tiles go through LDS as planes, row-major with a row stride of D + 16 elements: row operands are 16-byte
-// reads of a row, transposed operands ds_read_b64_tr_b16 reads of the same tile, both free of bank conflicts.  A tile
+// reads of a row, transposed operands ds_read_b64_tr_b16 reads of the same tile.  (Neither is free of bank conflicts in every width: at
+// head_dim 64 in fp32 38 to 43 % of the cycles of LDS are lost to them, see profiles/pmc_counters_c2f32.md.)  A tile
 // is read from global memory into registers a step ahead, split on its way into LDS, one barrier per tile.
 //
 //   split_fwd_kernel    32 queries per workgroup; wavefront w takes delta = w, w+W, ... and keeps one
