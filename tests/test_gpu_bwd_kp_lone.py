@@ -68,3 +68,34 @@ def test_layouts_and_half_open_windows(D, N, heads, w1, w2):
     exact = sa.simplicial_backward(*plain[:5], out, lse, plain[5], w1, w2, flags=1, **kw)
     for name, a, b in zip(("dq", "dk1", "dk2", "dv1", "dv2"), want, exact):
         assert_close_rel(a, b.cpu(), 2e-2, name, atol=2e-3)
+
+
+@pytest.mark.parametrize("D,N,heads,w1,w2", [(64, 2051, 20, 512, 17), (128, 1003, 26, 900, 40)])
+def test_widely_spread_logits(D, N, heads, w1, w2):
+    """fp16, logits of standard deviation 8: off by 8 * 2^-12 / sqrt(3) = 1.1e-3 each (products q*k2 rounded to 16 bits), 5e-3 at most, as are the
+    weights, of which few are large: three times that covers a gradient, which has two of them (dS = P * (dP - D))."""
+    import simplical_attn_amd as sa
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x = [(torch.randn(1, N, heads, D, generator=g, device="cuda") * (2 if t < 3 else 1)).to(FP) for t in range(6)]
+    out, lse = sa.simplicial_forward(*x[:5], w1, w2)
+    got = sa.simplicial_backward(*x[:5], out, lse, x[5], w1, w2)
+    want = sa.simplicial_backward(*x[:5], out, lse, x[5], w1, w2, flags=1)
+    for name, a, b in zip(("dq", "dk1", "dk2", "dv1", "dv2"), got, want):
+        assert_close_rel(a, b.cpu(), 1.5e-2, name, atol=2e-3)
+
+
+@pytest.mark.parametrize("D,N,heads,w1,w2", [(64, 2051, 20, 512, 17), (128, 1003, 26, 900, 40)])
+def test_a_gradient_that_is_not_a_number_stays_in_its_windows(D, N, heads, w1, w2):
+    """Query r reaches its own row of dQ, its K' window of dK' and dV' and its K window of dK and dV (there to whole tiles of 32
+    rows); everything else keeps its bits."""
+    import simplical_attn_amd as sa
+    r = N // 2
+    g = torch.Generator(device="cuda").manual_seed(D)
+    x = [torch.randn(1, N, heads, D, generator=g, device="cuda").to(BF) for _ in range(6)]
+    out, lse = sa.simplicial_forward(*x[:5], w1, w2)
+    clean = sa.simplicial_backward(*x[:5], out, lse, x[5], w1, w2)
+    x[5][:, r] = float("nan")
+    got = sa.simplicial_backward(*x[:5], out, lse, x[5], w1, w2)
+    for a, b, lo, hi in zip(got, clean, (r, max(r - w1, 0) // 32 * 32, r - w2, max(r - w1, 0) // 32 * 32, r - w2), (r, r // 32 * 32 + 31, r, r // 32 * 32 + 31, r)):
+        assert a[:, max(r - (w2 if hi == r and lo != r else 0), lo):r + 1].isnan().all()
+        assert torch.equal(a[:, :lo], b[:, :lo]) and torch.equal(a[:, hi + 1:], b[:, hi + 1:])
