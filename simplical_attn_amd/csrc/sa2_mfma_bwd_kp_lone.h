@@ -298,17 +298,13 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
         s[u][e + 1] = y;
         if constexpr (i > 0) round_p(UN, LONE_C(i - 1));
     };
-    // dS from the rounded weights, as in the two-wavefront kernel, so that a gradient does not depend on which of them a problem is
-    // given to: the first queries have few weights, all large, and single gradients there follow the rounding of each (up to 0.6 of
-    // a gradient's root mean square elsewhere from the unrounded ones, B1 H8 N32768 D128 w 1024/64; now 0.03).  It is not the more
-    // exact way: against fp32 the unrounded weights give dQ, dK and dK' errors 4 - 9 % smaller in the 2-norm, the first queries
-    // included, and worst elements that move both ways.  It costs two instructions a pair, in both backward kernels together 1 - 3 % of a
-    // training step.  (A second copy of the sweep for the first queries alone does not fit the registers: 560 bytes per lane of scratch.)
+    // dS from the unrounded weights: nothing but dS itself is rounded to 16 bits.  (From the rounded ones, as the two-wavefront kernel
+    // forms it, whose weights cross LDS in 16 bits: two instructions a pair more, B2 H8 N2048 D64 w 512/32 881 against 858 us a step with both
+    // backward kernels, B1 H16 N8192 D128 w 512/32 6203 against 6125, and errors of dQ, dK and dK' against fp32 4 - 9 % larger in the 2-norm.)
     auto ds_item = [&](auto UN, auto I) __attribute__((always_inline)) {
         constexpr int u = decltype(UN)::value, i = decltype(I)::value, ks = i / 4, t = i % 4, e = 2 * i;
         if constexpr (i == 0) round_p(UN, LONE_C(7));
-        const uint32_t pp = pw[u][ks][t];
-        uint32_t w = pack2<E>(E::lo(pp) * (dp[u][e] - drow_sum[u]), E::hi(pp) * (dp[u][e + 1] - drow_sum[u]));
+        uint32_t w = pack2<E>(s[u][e] * (dp[u][e] - drow_sum[u]), s[u][e + 1] * (dp[u][e + 1] - drow_sum[u]));
         stays(w);
         dw[u][ks][t] = w;
     };
