@@ -7,10 +7,12 @@
 //   A: S^T = K1.Q~^T - LSE and dP^T = V1.dO~^T,  B: P = exp2(S) and dS = P * (dP - D),  C: R^T += V1^T.P^T and G^T += K1^T.dS^T,
 // B between the MFMAs of A and C of the other unit (of the next tile at head_dim 128), operand reads eight MFMAs ahead of their
 // use: nothing is handed from one wavefront to another, and every operand read serves all units of the wavefront.
+// Within a sweep the next tile's address is one addition per tensor; only the last three tiles, which ask for the next round's
+// first ones, work it out (some fifty scalar instructions, which cost a lone wavefront as much as vector ones).
 // What bounds it: at head_dim 64 the instructions beside the MFMAs (32 MFMAs per tile, 0.44 us of 0.76; 18 tiles take 14 us of
 // a round's 23, masks 1.8, the sums over the units and dQ 3, forming 1); at head_dim 128 also power.  K' side with row term,
 // pre-pass and sums against the two-wavefront kernel, in turn on one machine (bf16): B2 H8 N2048 D64 w 512/32 428 -> 400 us,
-// B1 H16 N8192 D128 w 512/32 2831 -> 2747, B1 H8 N8192 w 1024/64 D128 4780 -> 4451, D64 2590 -> 2250.
+// B1 H16 N8192 D128 w 512/32 2831 -> 2600, B1 H8 N8192 w 1024/64 D128 4780 -> 4451, D64 2590 -> 2250.
 #pragma once
 
 #include "sa2_mfma_bwd_kp_plan.h"
@@ -114,19 +116,26 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
             v_off[x] = ((uint32_t)r * (uint32_t)p.v1.sn + col) * 2u;
         }
     };
-    auto request_tile = [&](uint32_t stage, bool k_part = true, bool v_part = true) __attribute__((always_inline)) {
-#pragma unroll
-        for (int x = 0; x < C::NREQ; ++x) {
-            const uint32_t to = stage + (uint32_t)((wave + KW * x) * T::GROUP);
-            if (k_part) lds_request(k_next, k_off[x], to);
-            if (v_part) lds_request(v_next, v_off[x], to + C::TILE_BYTES);
-        }
+    auto request_part = [&](auto X, uint32_t stage) __attribute__((always_inline)) {        // K's groups, then V's
+        constexpr int x = decltype(X)::value % C::NREQ;
+        const uint32_t to = stage + (uint32_t)((wave + KW * x) * T::GROUP);
+        if constexpr (decltype(X)::value < C::NREQ) lds_request(k_next, k_off[x], to);
+        else lds_request(v_next, v_off[x], to + C::TILE_BYTES);
+    };
+    auto request_tile = [&](uint32_t stage) __attribute__((always_inline)) {
+        static_for<2 * C::NREQ>([&](auto X) __attribute__((always_inline)) { request_part(X, stage); });
     };
     // The tile after the one requested last (behind the last round: that one again, which nothing reads).  In pieces without
-    // branches, which ride on MFMAs: scalar instructions cost a lone wavefront as much as vector ones.
+    // branches, which ride on MFMAs: scalar instructions cost a lone wavefront as much as vector ones.  ON: within a sweep
+    // (the caller counts next_tile up).
     int wrap = 0, nr = 0, more = 0, first = 0, last = 0;
-    auto next_piece = [&](auto I) __attribute__((always_inline)) {
+    auto next_piece = [&](auto I, auto ON) __attribute__((always_inline)) {
         constexpr int i = decltype(I)::value;
+        if constexpr (decltype(ON)::value) {
+            if constexpr (i == 0) k_next += k_step;
+            if constexpr (i == 1) v_next += v_step;
+            return;
+        }
         auto here_on = [](int& x) __attribute__((always_inline)) {       // (no piece moves up to another)
             x = __builtin_amdgcn_readfirstlane(x);
             asm volatile("" : "+s"(x));
@@ -160,7 +169,7 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
         }
     };
     auto next_request = [&]() __attribute__((always_inline)) {
-        static_for<6>([&](auto I) __attribute__((always_inline)) { next_piece(I); });
+        static_for<6>([&](auto I) __attribute__((always_inline)) { next_piece(I, std::false_type{}); });
         if (near_end) aim(next_tile);
     };
     constexpr int INFLIGHT = 2 * C::NREQ;                     // requests of one tile (two are under way)
@@ -194,7 +203,7 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
         }
         if (nrounds > 0) {
             aim(next_tile);
-            static_for<2>([&](auto I) __attribute__((always_inline)) { next_piece(LONE_C(4 + decltype(I)::value)); });
+            static_for<2>([&](auto I) __attribute__((always_inline)) { next_piece(LONE_C(4 + decltype(I)::value), std::false_type{}); });
             request_tile(lds0);
 #pragma unroll 1
             for (int x = 1; x < C::NSTAGE - 1; ++x) {
@@ -312,44 +321,79 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
         static_for<8>([&](auto X) __attribute__((always_inline)) { p_item(UN, X); });
         static_for<8>([&](auto X) __attribute__((always_inline)) { ds_item(UN, X); });
     };
-    // One unit: A(t), then C(t-1), whose four groups of MFMAs (R^T and G^T, each from the keys' first and second half) free
-    // the halves of P and dS one after the other for B(t).
+    // One unit: A(t), then C(t-1), whose four groups of MFMAs (R^T and G^T, each from the keys' first and second half) free the
+    // halves of P and dS one after the other for B(t).  B(t) starts beside the second half of A(t), where the logits are done,
+    // forms dS in fp32 in the place of dP, and rounds its second half beside the first MFMAs of A(t+1): nothing is left to do between two tiles.
     constexpr int BAR = 2 * DT;                               // MFMA of phase C that the tile's barrier stands before
-    auto single = [&](auto DO_C) __attribute__((always_inline)) {
+    auto exp_item = [&](auto I) __attribute__((always_inline)) {
+        float x = fast_exp2(s[0][decltype(I)::value]);
+        stays(x);
+        s[0][decltype(I)::value] = x;
+    };
+    auto p_word = [&](auto I) __attribute__((always_inline)) {
+        constexpr int i = decltype(I)::value;
+        uint32_t w = pack2<E>(s[0][2 * i], s[0][2 * i + 1]);
+        stays(w);
+        pw[0][i / 4][i % 4] = w;
+    };
+    auto ds_value = [&](auto I) __attribute__((always_inline)) {
+        constexpr int e = decltype(I)::value;
+        float x = s[0][e] * (dp[0][e] - drow_sum[0]);
+        stays(x);
+        dp[0][e] = x;
+    };
+    auto ds_word = [&](auto I) __attribute__((always_inline)) {
+        constexpr int i = decltype(I)::value;
+        uint32_t w = pack2<E>(dp[0][2 * i], dp[0][2 * i + 1]);
+        stays(w);
+        dw[0][i / 4][i % 4] = w;
+    };
+    // items LO .. HI-1 of a kind
+    auto items = [&](auto LO, auto HI, auto&& f) __attribute__((always_inline)) {
+        static_for<decltype(HI)::value - decltype(LO)::value>([&](auto X) __attribute__((always_inline)) { f(LONE_C(decltype(LO)::value + decltype(X)::value)); });
+    };
+    auto single = [&](auto DO_C, auto ON) __attribute__((always_inline)) {
         constexpr bool CC = decltype(DO_C)::value;
         static_assert(LONG && sizeof(DO_C) > 0, "one unit per wavefront: head_dim 128");
         static_for<NE>([&](auto I) __attribute__((always_inline)) {
             constexpr int i = decltype(I)::value;
             a_mfma(LONE_C(0), I);
             if constexpr (i < DK) read_row(LONE_C(1), I, sa);
-            next_piece(LONE_C(i - 1));
+            next_piece(LONE_C(i - 1), ON);
             if constexpr (CC) deal<12, i - 4, 12>([&](auto X) __attribute__((always_inline)) { read_column(X, sc); });
+            if constexpr (CC && i < 4) ds_word(LONE_C(4 + i));
+            if constexpr (i >= DK + 2) items(LONE_C(2 * (i - DK - 2)), LONE_C(2 * (i - DK - 2) + 2), exp_item);
             __builtin_amdgcn_sched_barrier(0);
         });
+        if constexpr (!CC) finished(s[0], dp[0]);
         static_for<NE>([&](auto I) __attribute__((always_inline)) {
-            constexpr int i = decltype(I)::value, group = i / DT;
+            constexpr int i = decltype(I)::value;
             if constexpr (i == BAR) step_barrier();
             if constexpr (CC) {
                 c_mfma(LONE_C(0), I);
                 if constexpr (i < 4) read_column(LONE_C(12 + i), sc);
             }
             if constexpr (i >= BAR) read_row(LONE_C(0), LONE_C(i - BAR), sb);
-            if constexpr (group == 1 || group == 2) deal<8, i - DT, 2 * DT>([&](auto X) __attribute__((always_inline)) { p_item(LONE_C(0), X); });
-            if constexpr (group == 3) deal<4, i - 3 * DT, DT>([&](auto X) __attribute__((always_inline)) { ds_item(LONE_C(0), X); });
-            if constexpr (i == BAR) request_tile(sc, true, false);
-            if constexpr (i == BAR + 4) request_tile(sc, false, true);
+            constexpr int EXPS[17] = {12, 14, 16, 16, 16, 16, 16, 16, 16, 16, 16, 16, 16, 16, 16, 16, 16};
+            constexpr int PW[17] = {0, 0, 0, 0, 0, 2, 4, 4, 4, 6, 8, 8, 8, 8, 8, 8, 8};
+            constexpr int DSV[17] = {0, 0, 0, 2, 4, 5, 6, 8, 10, 10, 11, 12, 14, 15, 16, 16, 16};
+            constexpr int DSW[17] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 1, 2, 3, 4};
+            items(LONE_C(EXPS[i]), LONE_C(EXPS[i + 1]), exp_item);
+            items(LONE_C(PW[i]), LONE_C(PW[i + 1]), p_word);
+            items(LONE_C(DSV[i]), LONE_C(DSV[i + 1]), ds_value);
+            items(LONE_C(DSW[i]), LONE_C(DSW[i + 1]), ds_word);
+            if constexpr (i >= BAR) deal<2 * C::NREQ, (i - BAR) / 2, NE - BAR - DT>([&](auto X) __attribute__((always_inline)) { if constexpr (i % 2 == 0) request_part(X, sc); });
             __builtin_amdgcn_sched_barrier(0);
         });
-        static_for<4>([&](auto X) __attribute__((always_inline)) { ds_item(LONE_C(0), LONE_C(4 + decltype(X)::value)); });
-        stays(dw[0][1]);
     };
     auto single_last = [&]() __attribute__((always_inline)) {                       // C of tile t-1 alone
+        items(LONE_C(4), LONE_C(8), ds_word);
         static_for<4 * DT>([&](auto X) __attribute__((always_inline)) { read_column(X, sc); });
         static_for<NE>([&](auto I) __attribute__((always_inline)) { c_mfma(LONE_C(0), I); });
     };
     // Two units: A(t, 0), C(t-1, 1), A(t, 1), C(t, 0); the transposed operands of tile t serve C(t, 0) and C(t, 1).
     // The weights and dS of a unit are formed from the end of its phase A to the beginning of its phase C.
-    auto pair = [&](auto DO_C) __attribute__((always_inline)) {
+    auto pair = [&](auto DO_C, auto ON) __attribute__((always_inline)) {
         constexpr bool CC = decltype(DO_C)::value;
         auto later = [&](auto UN, auto I) __attribute__((always_inline)) {
             deal<8, decltype(I)::value, NE>([&](auto X) __attribute__((always_inline)) { ds_item(UN, X); });
@@ -359,14 +403,14 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
         };
         static_for<NE>([&](auto I) __attribute__((always_inline)) {
             a_mfma(LONE_C(0), I);
-            if constexpr (decltype(I)::value % 2 == 0) next_piece(LONE_C(decltype(I)::value / 2 - 1));
+            if constexpr (decltype(I)::value % 2 == 0) next_piece(LONE_C(decltype(I)::value / 2 - 1), ON);
             if constexpr (CC) later(LONE_C(U - 1), I);
             __builtin_amdgcn_sched_barrier(0);
         });
         static_for<NE>([&](auto I) __attribute__((always_inline)) {
             constexpr int i = decltype(I)::value;
             if constexpr (CC) c_mfma(LONE_C(U - 1), I);
-            if constexpr (i % 2 == 0 && i / 2 < 3) next_piece(LONE_C(3 + i / 2));
+            if constexpr (i % 2 == 0 && i / 2 < 3) next_piece(LONE_C(3 + i / 2), ON);
             early(LONE_C(0), I);
             if constexpr (i >= 2) read_column(LONE_C(i - 2), sa);                   // (the MFMA that read its register is past)
             __builtin_amdgcn_sched_barrier(0);
@@ -384,8 +428,8 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
             c_mfma(LONE_C(0), I);
             read_row(LONE_C(i / DK), LONE_C(i % DK), sb);
             early(LONE_C(U - 1), I);
-            if constexpr (i == 1) request_tile(sc, true, false);
-            if constexpr (i == NE - 2) request_tile(sc, false, true);
+            if constexpr (i == 1) static_for<C::NREQ>([&](auto X) __attribute__((always_inline)) { request_part(X, sc); });
+            if constexpr (i == NE - 2) static_for<C::NREQ>([&](auto X) __attribute__((always_inline)) { request_part(LONE_C(C::NREQ + decltype(X)::value), sc); });
             __builtin_amdgcn_sched_barrier(0);
         });
         stays(s[U - 1]);
@@ -519,7 +563,7 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
         auto aim_ahead = [&]() __attribute__((always_inline)) {        // (for the request of the step that follows)
             if (near_end) {
                 const int t = next_tile, n = next_round, z = next_last;
-                static_for<4>([&](auto I) __attribute__((always_inline)) { next_piece(I); });
+                static_for<4>([&](auto I) __attribute__((always_inline)) { next_piece(I, std::false_type{}); });
                 aim(next_tile);
                 next_tile = t;
                 next_round = n;
@@ -530,17 +574,24 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
             if (jt >= a0 && jt <= a1) {
                 enter_tile(jt);
                 aim_ahead();
-                if constexpr (U == 1) single(no);
-                else pair(no);
+                if constexpr (U == 1) single(no, no);
+                else pair(no, no);
                 rotate();
                 ++jt;
                 while (jt <= a1) {
                     enter_tile(jt);
                     aim_ahead();
-                    const int n = until(jt);
-                    for (int k = n; k > 0; --k) {
-                        if constexpr (U == 1) single(yes);
-                        else pair(yes);
+                    // those of them that request within the sweep, then the others
+                    const int n = until(jt), on = near_end ? 0 : n < next_last - next_tile ? n : next_last - next_tile;
+                    for (int k = on; k > 0; --k) {
+                        if constexpr (U == 1) single(yes, yes);
+                        else pair(yes, yes);
+                        rotate();
+                    }
+                    next_tile += on;
+                    for (int k = n - on; k > 0; --k) {
+                        if constexpr (U == 1) single(yes, no);
+                        else pair(yes, no);
                         rotate();
                     }
                     jt += n;
