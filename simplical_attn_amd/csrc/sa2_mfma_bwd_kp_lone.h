@@ -9,10 +9,12 @@
 // use: nothing is handed from one wavefront to another, and every operand read serves all units of the wavefront.
 // Within a sweep the next tile's address is one addition per tensor; only the last three tiles, which ask for the next round's
 // first ones, work it out (some fifty scalar instructions, which cost a lone wavefront as much as vector ones).
-// What bounds it: at head_dim 64 the instructions beside the MFMAs (32 MFMAs per tile, 0.44 us of 0.76; 18 tiles take 14 us of
-// a round's 23, masks 1.8, the sums over the units and dQ 3, forming 1); at head_dim 128 also power.  K' side with row term,
-// pre-pass and sums against the two-wavefront kernel, in turn on one machine (bf16): B2 H8 N2048 D64 w 512/32 428 -> 400 us,
-// B1 H16 N8192 D128 w 512/32 2831 -> 2600, B1 H8 N8192 w 1024/64 D128 4780 -> 4451, D64 2590 -> 2250.
+// Where LDS has the room the K' rows lie there in fp32 as (k2 + bias) * scale * log2(e): a word of Q~ takes five vector instructions
+// instead of eleven, an element of dQ's sums three instead of five (K' side 2433 -> 2400 us and 394 -> 374 at the first two sizes below).
+// What bounds it: the instructions beside the MFMAs, at head_dim 128 also power.  Time stamps of a workgroup's rounds, us: B1 H16 N8192
+// D128 w 512/32 forming 1.8, sweep of 18 tiles 13.3, sums 1.8, dQ 1.5; B2 H8 N2048 D64 w 512/32 1.6, 17.2, 2.1, 1.8.  K' side with row term,
+// pre-pass and sums against the two-wavefront kernel, in turn on one machine (bf16): B2 H8 N2048 D64 w 512/32 428 -> 375 us,
+// B1 H16 N8192 D128 w 512/32 2831 -> 2570.
 #pragma once
 
 #include "sa2_mfma_bwd_kp_plan.h"
@@ -21,11 +23,11 @@
 namespace sa2 {
 namespace {
 
-// RAW: see KpLoneCfg::main_bytes.  The K' window is cut into nseg runs of segw deltas, one workgroup per (K' block, segment).
+// RAW, WIDE: see KpLoneCfg::main_bytes.  The K' window is cut into nseg runs of segw deltas, one workgroup per (K' block, segment).
 // Each writes its own dQ partial (rows k0 + seg*segw ..) and, when nseg > 1, fp32 partial dK' and dV' to `kpart`
 // ([dV' | dK'][nseg][B*H][N][D]) for bwd_sum_kernel.  left = 1: the pre-pass took the unit delta = w2 of every block and left
 // its results in the output tensors and in rows w2 .. of the dQ partials.
-template <class E, int D, bool RAW>
+template <class E, int D, bool RAW, bool WIDE>
 __global__ __launch_bounds__(KpLoneCfg<D>::T) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ dq_part, int left, int nseg, int segw, float* __restrict__ kpart) {
     typedef typename E::scalar EL;
@@ -41,8 +43,9 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
     const int N = p.N, w1 = p.w1, w2 = p.w2;
     const int w2s = segw - 1;                                 // deltas of a segment, minus one (w2 when there is one segment)
     const int RQ = BQ + w2s;                                  // query rows this workgroup touches
-    unsigned char* k2_s = smem_raw + (size_t)C::NSTAGE * C::STAGE_BYTES;               // K' rows k0 .. k0+31, as in a tile
-    unsigned char* v2_s = k2_s + C::row_bytes(BQ);            // V' rows
+    unsigned char* k2_s = smem_raw + (size_t)C::NSTAGE * C::STAGE_BYTES;               // K' rows k0 .. k0+31, as in a tile, or
+    float* kt_s = (float*)k2_s;                               // (WIDE) [BQ][AS] times scale * log2(e)
+    unsigned char* v2_s = k2_s + (WIDE ? (size_t)BQ * C::AS * 4 : C::row_bytes(BQ));   // V' rows
     unsigned char* q_s = v2_s + C::row_bytes(BQ);             // q rows kq .. kq+RQ-1  (when RAW)
     unsigned char* do_s = q_s + C::row_bytes(RQ);             // dO rows               (when RAW)
     const int RQ4 = (RQ + 3) & ~3;
@@ -195,7 +198,17 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
             for (int x = 0; x < D / 32; ++x)
                 from_left[x] = *(const u4*)(dq_part + (((int64_t)bh * nkb + kb) * RQ + w2) * D + (tid + x * KT) * 4);
         }
-        request_rows(k2p, p.k2.sn, k0, BQ, k2_s);
+        constexpr int NK2 = BQ * (D / 8) / KT;                // 16-byte chunks of the K' rows per thread
+        uint4 kraw[NK2];
+        if constexpr (WIDE) {
+#pragma unroll
+            for (int x = 0; x < NK2; ++x) {
+                const int c = tid + x * KT, r = k0 + c / (D / 8);
+                kraw[x] = *(const uint4*)(k2p + (int64_t)(r < N ? r : N - 1) * p.k2.sn + c % (D / 8) * 8);
+            }
+        } else {
+            request_rows(k2p, p.k2.sn, k0, BQ, k2_s);
+        }
         request_rows(v2p, p.v2.sn, k0, BQ, v2_s);
         if constexpr (RAW) {
             request_rows(qp, p.q.sn, kq, RQ, q_s);
@@ -209,6 +222,19 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
             for (int x = 1; x < C::NSTAGE - 1; ++x) {
                 next_request();
                 request_tile(lds0 + x * C::STAGE_BYTES);
+            }
+        }
+        if constexpr (WIDE) {
+            const float qscale = p.scale * LOG2E;
+#pragma unroll
+            for (int x = 0; x < NK2; ++x) {
+                const int c = tid + x * KT;
+                const uint32_t w[4] = {kraw[x].x, kraw[x].y, kraw[x].z, kraw[x].w};
+                float* to = kt_s + c / (D / 8) * C::AS + c % (D / 8) * 8;
+#pragma unroll
+                for (int t = 0; t < 4; t += 2)
+                    *(float4*)(to + 2 * t) = make_float4((E::lo(w[t]) + p.k2_bias) * qscale, (E::hi(w[t]) + p.k2_bias) * qscale,
+                                                         (E::lo(w[t + 1]) + p.k2_bias) * qscale, (E::hi(w[t + 1]) + p.k2_bias) * qscale);
             }
         }
         for (int c = tid; c < RQ * (C::AS / 4); c += KT) ((float4*)dqacc)[c] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -225,7 +251,12 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
 #pragma unroll
             for (int x = 0; x < D / 32; ++x) {
                 const int it = tid + x * KT;
-                *(u4*)(dqacc + (w2 + it / (D / 4)) * C::AS + it % (D / 4) * 4) = from_left[x];
+                float4 y = __builtin_bit_cast(float4, from_left[x]);
+                if constexpr (WIDE) {
+                    const float qscale = p.scale * LOG2E;
+                    y.x *= qscale; y.y *= qscale; y.z *= qscale; y.w *= qscale;
+                }
+                *(float4*)(dqacc + (w2 + it / (D / 4)) * C::AS + it % (D / 4) * 4) = y;
             }
         }
     }
@@ -474,38 +505,66 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
         float lse2[U];
         asm volatile("s_nop 3" : "+v"(zero));
         static_for<2 * U * DT>([&](auto X) __attribute__((always_inline)) { L::sum_zero<16 * decltype(X)::value>(zero); });
-        static_for<U>([&](auto UN) __attribute__((always_inline)) {
-            constexpr int u = decltype(UN)::value;
+        auto form = [&](auto BIASED) __attribute__((always_inline)) {
+            const float kb = decltype(BIASED)::value ? p.k2_bias : 0.f, vb = decltype(BIASED)::value ? p.v2_bias : 0.f;
             const int l = here(), ln_ = l & 31, hf_ = l >> 5 & 1;
-            const int delta = d0 + u < n_units ? d0 + u : n_units - 1;
-            uint4 qx[DK], ox[DK];                             // all reads of the two rows first
+            uint4 qx[U][DK], ox[U][DK];                       // all reads of the rows first
 #pragma unroll
-            for (int kk = 0; kk < DK; ++kk) {
-                if constexpr (RAW) {
-                    qx[kk] = lds_row8(q_s, ln_ + delta, hf_, kk);
-                    ox[kk] = lds_row8(do_s, ln_ + delta, hf_, kk);
-                } else {
-                    qx[kk] = load_cols8<false>(far_row(qp, p.q.sn, ln_ + delta), kk * 16 + hf_ * 8, p.D);
-                    ox[kk] = load_cols8<false>(far_row(dop, p.dout.sn, ln_ + delta), kk * 16 + hf_ * 8, p.D);
+            for (int u = 0; u < U; ++u) {
+                const int delta = d0 + u < n_units ? d0 + u : n_units - 1;
+#pragma unroll
+                for (int kk = 0; kk < DK; ++kk) {
+                    if constexpr (RAW) {
+                        qx[u][kk] = lds_row8(q_s, ln_ + delta, hf_, kk);
+                        ox[u][kk] = lds_row8(do_s, ln_ + delta, hf_, kk);
+                    } else {
+                        qx[u][kk] = load_cols8<false>(far_row(qp, p.q.sn, ln_ + delta), kk * 16 + hf_ * 8, p.D);
+                        ox[u][kk] = load_cols8<false>(far_row(dop, p.dout.sn, ln_ + delta), kk * 16 + hf_ * 8, p.D);
+                    }
                 }
+                lse2[u] = lse_s[ln_ + delta];
+                drow_sum[u] = dsum_s[ln_ + delta];
             }
             static_for<DK>([&](auto KK) __attribute__((always_inline)) {
-                constexpr int kk = decltype(KK)::value, at = (u * DK + kk) * 4;
-                const uint4 kx = lds_row8(k2_s, ln_, hf_, kk), vx = lds_row8(v2_s, ln_, hf_, kk);
-                const uint32_t qw[4] = {qx[kk].x, qx[kk].y, qx[kk].z, qx[kk].w}, kw[4] = {kx.x, kx.y, kx.z, kx.w};
-                const uint32_t ow[4] = {ox[kk].x, ox[kk].y, ox[kk].z, ox[kk].w}, vw[4] = {vx.x, vx.y, vx.z, vx.w};
-                uint32_t qt[4], ot[4];
+                constexpr int kk = decltype(KK)::value;
+                float kt[8], vt_[8];                          // K'~ (scaled) and V'~ of the lane's row: the same for all units
+                if constexpr (WIDE) {
+                    const float* src = kt_s + ln_ * C::AS + kk * 16 + hf_ * 8;
+                    const float4 k0_ = *(const float4*)src, k1_ = *(const float4*)(src + 4);
+                    kt[0] = k0_.x; kt[1] = k0_.y; kt[2] = k0_.z; kt[3] = k0_.w;
+                    kt[4] = k1_.x; kt[5] = k1_.y; kt[6] = k1_.z; kt[7] = k1_.w;
+                } else {
+                    const uint4 kx = lds_row8(k2_s, ln_, hf_, kk);
+                    const uint32_t kw[4] = {kx.x, kx.y, kx.z, kx.w};
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        kt[2 * t] = (E::lo(kw[t]) + kb) * qscale;
+                        kt[2 * t + 1] = (E::hi(kw[t]) + kb) * qscale;
+                    }
+                }
+                const uint4 vx = lds_row8(v2_s, ln_, hf_, kk);
+                const uint32_t vw[4] = {vx.x, vx.y, vx.z, vx.w};
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
-                    qt[t] = pack2<E>(E::lo(qw[t]) * (E::lo(kw[t]) + p.k2_bias) * qscale, E::hi(qw[t]) * (E::hi(kw[t]) + p.k2_bias) * qscale);
-                    ot[t] = pack2<E>(E::lo(ow[t]) * (E::lo(vw[t]) + p.v2_bias), E::hi(ow[t]) * (E::hi(vw[t]) + p.v2_bias));
+                    vt_[2 * t] = E::lo(vw[t]) + vb;
+                    vt_[2 * t + 1] = E::hi(vw[t]) + vb;
                 }
-                L::set_regs<Q0 + at>(qt[0], qt[1], qt[2], qt[3]);
-                L::set_regs<O0 + at>(ot[0], ot[1], ot[2], ot[3]);
+                static_for<U>([&](auto UN) __attribute__((always_inline)) {
+                    constexpr int u = decltype(UN)::value, at = (u * DK + kk) * 4;
+                    const uint32_t qw[4] = {qx[u][kk].x, qx[u][kk].y, qx[u][kk].z, qx[u][kk].w}, ow[4] = {ox[u][kk].x, ox[u][kk].y, ox[u][kk].z, ox[u][kk].w};
+                    uint32_t qt[4], ot[4];
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        qt[t] = pack2<E>(E::lo(qw[t]) * kt[2 * t], E::hi(qw[t]) * kt[2 * t + 1]);
+                        ot[t] = pack2<E>(E::lo(ow[t]) * vt_[2 * t], E::hi(ow[t]) * vt_[2 * t + 1]);
+                    }
+                    L::set_regs<Q0 + at>(qt[0], qt[1], qt[2], qt[3]);
+                    L::set_regs<O0 + at>(ot[0], ot[1], ot[2], ot[3]);
+                });
             });
-            lse2[u] = lse_s[ln_ + delta];
-            drow_sum[u] = dsum_s[ln_ + delta];
-        });
+        };
+        if ((WIDE ? 0.f : p.k2_bias) != 0.f || p.v2_bias != 0.f) form(std::true_type{});
+        else form(std::false_type{});
         L::keep_out();
 
         // ---- the sweep: tiles [t0, t1] hold keys of the first unit, [t2, t3] of the last one; [p0, p1] need no mask ----
@@ -669,27 +728,35 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
             auto add_block = [&](auto B) __attribute__((always_inline)) {
                 constexpr int blk = decltype(B)::value;
                 constexpr int NV = DK / 2;                    // float4 slots of a block
+                const int l = here(), ln_ = l & 31, hf_ = l >> 5 & 1;
+                float4 kt[NV];                                // (WIDE: scaled)
+                // slot e of the block -> 8-column group
+                static_for<NV>([&](auto SL) __attribute__((always_inline)) {
+                    constexpr int e = decltype(SL)::value, g8 = 2 * (blk + 4 * (e >> 1)) + (e & 1);
+                    if constexpr (WIDE) {
+                        kt[e] = *(const float4*)(kt_s + ln_ * C::AS + g8 * 8 + 4 * hf_);
+                    } else {
+                        const uint2 x = lds_row4(k2_s, ln_, hf_, g8);
+                        kt[e] = make_float4(E::lo(x.x) + p.k2_bias, E::hi(x.x) + p.k2_bias, E::lo(x.y) + p.k2_bias, E::hi(x.y) + p.k2_bias);
+                    }
+                });
                 static_for<U>([&](auto UN) __attribute__((always_inline)) {
                     constexpr int u = decltype(UN)::value;
                     if (d0 + u >= n_units) return;
-                    const int l = here(), ln_ = l & 31, hf_ = l >> 5 & 1;
                     float* arow = dqacc + (ln_ + d0 + u) * C::AS + 4 * hf_;
                     float4 a[NV];
-                    uint2 x[NV];
-                    // slot e of the block -> 8-column group
                     static_for<NV>([&](auto SL) __attribute__((always_inline)) {
                         constexpr int e = decltype(SL)::value, g8 = 2 * (blk + 4 * (e >> 1)) + (e & 1);
-                        x[e] = lds_row4(k2_s, ln_, hf_, g8);
                         a[e] = *(float4*)(arow + g8 * 8);
                     });
                     static_for<NV>([&](auto SL) __attribute__((always_inline)) {
                         constexpr int e = decltype(SL)::value, g8 = 2 * (blk + 4 * (e >> 1)) + (e & 1);
                         constexpr int gr = G0 + u * DT * 16 + 4 * g8;
                         const float4 g = L::get_regs<gr>();
-                        a[e].x += g.x * (E::lo(x[e].x) + p.k2_bias);
-                        a[e].y += g.y * (E::hi(x[e].x) + p.k2_bias);
-                        a[e].z += g.z * (E::lo(x[e].y) + p.k2_bias);
-                        a[e].w += g.w * (E::hi(x[e].y) + p.k2_bias);
+                        a[e].x += g.x * kt[e].x;
+                        a[e].y += g.y * kt[e].y;
+                        a[e].z += g.z * kt[e].z;
+                        a[e].w += g.w * kt[e].w;
                         *(float4*)(arow + g8 * 8) = a[e];
                     });
                     // (the second unit's rows overlap the first one's, shifted by one: its reads must see the first
@@ -721,7 +788,8 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
         for (int it = tid_f; it < RQ * CH; it += KT) {
             const int row = it / CH, c0 = (it - row * CH) * 4;
             float4 a = *(const float4*)(dqacc + row * C::AS + c0);
-            a.x *= p.scale; a.y *= p.scale; a.z *= p.scale; a.w *= p.scale;
+            const float sc_ = WIDE ? LN2 : p.scale;           // (WIDE: the sums carry scale * log2(e))
+            a.x *= sc_; a.y *= sc_; a.z *= sc_; a.w *= sc_;
             *(float4*)(dst + (int64_t)row * D + c0) = a;
         }
     }
@@ -798,14 +866,15 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
 template <class E, int D>
 int launch_kp_lone_width(const Problem& p, const KpLaunch& l, hipStream_t st) {
     using C = KpLoneCfg<D>;
-    const bool raw = C::raw_fits(l.plan.segw - 1);
+    const bool raw = C::raw_fits(l.plan.segw - 1), wide = C::wide_fits(l.plan.segw - 1);
     auto go = [&](auto kernel) {
         if (!allow_full_lds((const void*)kernel)) return SA2_ERR_LAUNCH_FAILED;
-        hipLaunchKernelGGL(kernel, dim3((unsigned)l.total), dim3(C::T), C::lds_bytes(l.plan.segw - 1, raw), st, p, l.nkb, l.total, l.dq_part, l.left,
+        hipLaunchKernelGGL(kernel, dim3((unsigned)l.total), dim3(C::T), C::lds_bytes(l.plan.segw - 1, raw, wide), st, p, l.nkb, l.total, l.dq_part, l.left,
                            l.plan.nseg, l.plan.segw, l.kpart);
         return hipGetLastError() == hipSuccess ? SA2_OK : SA2_ERR_LAUNCH_FAILED;
     };
-    return raw ? go(mfma_bwd_kp_lone_kernel<E, D, true>) : go(mfma_bwd_kp_lone_kernel<E, D, false>);
+    if (wide) return raw ? go(mfma_bwd_kp_lone_kernel<E, D, true, true>) : go(mfma_bwd_kp_lone_kernel<E, D, false, true>);
+    return raw ? go(mfma_bwd_kp_lone_kernel<E, D, true, false>) : go(mfma_bwd_kp_lone_kernel<E, D, false, false>);
 }
 template <class E>
 int launch_kp_lone(const Problem& p, const KpLaunch& l, hipStream_t st) {

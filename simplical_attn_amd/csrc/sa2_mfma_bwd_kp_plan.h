@@ -31,14 +31,17 @@ struct KpLoneCfg {
     static constexpr size_t LDS_LIMIT = 160 * 1024;
     static constexpr size_t row_bytes(int rows) { return (size_t)((rows + Tile::RPW - 1) / Tile::RPW) * Tile::GROUP; }     // rows laid out as in a tile
     // raw = true: the q and dO rows the workgroup touches are copied to LDS; otherwise the
-    // wavefronts read them from global memory once per unit
-    static size_t main_bytes(int w2, bool raw) {
+    // wavefronts read them from global memory once per unit.  wide = true: the K' rows lie there as (k2 + bias) * scale * log2(e) in
+    // fp32, rather than as they are
+    static size_t main_bytes(int w2, bool raw, bool wide = false) {
         const int rq = BQ + w2;
-        return (size_t)NSTAGE * STAGE_BYTES + 2 * row_bytes(BQ) + (raw ? 2 * row_bytes(rq) : 0) + 2 * ((rq + 3) / 4 * 4) * 4 + (size_t)rq * AS * 4;
+        return (size_t)NSTAGE * STAGE_BYTES + row_bytes(BQ) + (wide ? (size_t)BQ * AS * 4 : row_bytes(BQ)) + (raw ? 2 * row_bytes(rq) : 0) +
+               2 * ((rq + 3) / 4 * 4) * 4 + (size_t)rq * AS * 4;
     }
     static size_t final_bytes() { return (size_t)W * 2 * BQ * AS * 4; }
-    static size_t lds_bytes(int w2, bool raw) { return main_bytes(w2, raw) > final_bytes() ? main_bytes(w2, raw) : final_bytes(); }
+    static size_t lds_bytes(int w2, bool raw, bool wide = false) { return main_bytes(w2, raw, wide) > final_bytes() ? main_bytes(w2, raw, wide) : final_bytes(); }
     static bool raw_fits(int w2) { return lds_bytes(w2, true) <= LDS_LIMIT; }
+    static bool wide_fits(int w2) { return lds_bytes(w2, raw_fits(w2), true) <= LDS_LIMIT; }
     static bool fits(int w2) { return lds_bytes(w2, false) <= LDS_LIMIT; }
     // Whether the kernel is taken, by the keys a K' row's queries see on average (the window, less where the sequence begins).  A
     // tile of the sweep takes it 0.76 us per eight deltas (head_dim 64; the two-wavefront kernel 1.04) or 0.71 per four (128; 0.89),

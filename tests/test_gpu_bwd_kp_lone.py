@@ -49,6 +49,29 @@ def test_kp_side_matches_the_fma_kernels(dtype, B, N, H, D, w1, w2, bias):
     assert torch.equal(got[2], again[2]) and torch.equal(got[4], again[4])
 
 
+@pytest.mark.parametrize("dtype,B,N,H,D,w1,w2,bias", [
+    (BF, 1, 1100, 26, 128, 900, 24, 0.2),   # K' rows in fp32, with what the pre-pass left; q and dO rows in LDS
+    (FP, 1, 1100, 26, 128, 900, 36, -0.2),  # ... the most deltas (37) that leave room for all three
+    (BF, 1, 1100, 26, 128, 900, 38, 0.3),   # K' rows in 16 bits beside q and dO rows
+    (FP, 1, 1024, 16, 128, 900, 57, 0.3),   # K' rows in fp32, q and dO rows from global memory
+    (BF, 1, 1024, 16, 128, 900, 110, 0.1),  # neither
+    (BF, 1, 1500, 30, 64, 500, 32, 0.2),    # two units
+    (FP, 1, 1500, 30, 64, 500, 61, 0.2),
+])
+def test_k2_rows_in_both_forms(dtype, B, N, H, D, w1, w2, bias):
+    """K' rows in LDS as (k2 + bias) * scale * log2(e) in fp32 or as they are, with a scale of its own: dQ, dK' and dV' as above."""
+    import simplical_attn_amd as sa
+    g = torch.Generator(device="cuda").manual_seed(N + D + w2)
+    x = [torch.randn(B, N, H, D, generator=g, device="cuda").to(dtype) for _ in range(6)]
+    kw = dict(k2_bias=bias, v2_bias=-bias, scale=0.07)
+    out, lse = sa.simplicial_forward(*x[:5], w1, w2, **kw)
+    needs = (True, False, True, False, True)
+    got = sa.simplicial_backward(*x[:5], out, lse, x[5], w1, w2, needs=needs, **kw)
+    want = sa.simplicial_backward(*x[:5], out, lse, x[5], w1, w2, needs=needs, flags=1, **kw)
+    for name, i in (("dq", 0), ("dk2", 2), ("dv2", 4)):
+        assert_close_rel(got[i], want[i].cpu(), 2e-2 if dtype == BF else 1.5e-2, name, atol=2e-3)
+
+
 @pytest.mark.parametrize("D,N,heads,w1,w2", [(64, 2051, 20, 513, 18), (128, 1003, 26, 901, 41)])
 def test_layouts_and_half_open_windows(D, N, heads, w1, w2):
     """Views of one fused projection [B, N, 5, H, D] and of [B, H, N, D] tensors give what contiguous copies give, bit for bit, in all

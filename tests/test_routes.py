@@ -55,6 +55,12 @@ def test_kp_cases_reach_the_kernel():
         assert kp_route(1, N, heads, D, w1 - 1, w2 - 1)[1]
 
 
+def test_k2_row_cases_reach_the_kernel():
+    routes = {c[4:6] + c[6:7]: kp_route(*c[1:7]) for c in _cases(test_gpu_bwd_kp_lone.test_k2_rows_in_both_forms)}
+    assert all(lone for _, lone, _ in routes.values()) and routes[128, 900, 24][0] and routes[64, 500, 32][0]
+    assert all(segments == 1 for _, _, segments in routes.values())
+
+
 def test_forward_cases_reach_the_kernel():
     t = test_gpu_fwd_lone
     routes = [(c[0], c[4], *forward_route(*c[1:7])) for c in _cases(t.test_forward_matches_the_fma_kernels)]
