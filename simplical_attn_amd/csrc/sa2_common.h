@@ -205,7 +205,7 @@ bool f32_mfma_bwd_supported(int D, int w2, int dtype);
 bool f32_mfma_layout_ok(const Problem& p, int dtype, bool backward);
 size_t f32_mfma_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2, int dtype, size_t room);
 int launch_f32_mfma_fwd(const Problem& p, int dtype, hipStream_t st);
-int f32_mfma_fwd_nsplit(int B, int N, int H, int D, int w1, int w2);
+int f32_mfma_fwd_nsplit(int B, int N, int H, int D, int w1, int w2, int dtype);
 size_t f32_mfma_fwd_part_bytes(int B, int N, int H, int D, int nsplit);
 int launch_f32_mfma_bwd(const Problem& p, int dtype, hipStream_t st);
 // 16-bit tensors with head_dim 256 on the 16-bit MFMA (rows 16-byte aligned)

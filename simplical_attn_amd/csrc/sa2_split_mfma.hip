@@ -64,8 +64,9 @@ struct SplitCfg {
     static constexpr int PLANE = 32 * RS;      // elements
     static constexpr int AS = D + 4;           // row stride of fp32 accumulators in LDS
     static constexpr size_t LDS_LIMIT = 160 * 1024;
-    // Forward: eight wavefronts (two per SIMD) where operands and accumulators fit 256 registers, else four.
-    static constexpr int FW = D <= 64 ? 8 : 4;
+    // Forward: eight wavefronts (two per SIMD) where operands and accumulators fit 256 registers, else four: bf16 at 96 columns (254 with
+    // three planes of Q~, 230 with two) 364 -> 239 us at B1 H8 N2048 D96 w 255/31; fp16 takes 350 there.
+    static constexpr int FW = D <= 64 || (D == 96 && T::PLANES == 1) ? 8 : 4;
     static constexpr int KV_TILE = NK * PLANE;             // a K or V tile
     static constexpr int KV_STAGE = 2 * KV_TILE;           // K tile, then V tile
     static constexpr size_t FWD_TILES = (size_t)2 * KV_STAGE * 2;
@@ -348,21 +349,29 @@ struct TileRegs {
         }
     }
 };
-// The product row x * (y + bias) * mul of eight columns from `col` on, split into three planes
-template <class T, bool PAD>
+// The product row x * (y + bias) * mul of eight columns from `col` on, split into three planes; N = 2: x * y, which of two bf16 values
+// has 16 bits and two planes hold exactly
+template <class T, bool PAD, int N = 3>
 __device__ __forceinline__ void product_planes(const typename T::T* xrow, const typename T::T* yrow, int col, int width, float bias, float mul,
-                                               bf16x8 (&o)[3]) {
+                                               bf16x8 (&o)[N]) {
     const float4 x0 = cols4<T, PAD>(xrow, col, width), x1 = cols4<T, PAD>(xrow, col + 4, width);
     const float4 y0 = cols4<T, PAD>(yrow, col, width), y1 = cols4<T, PAD>(yrow, col + 4, width);
+    if constexpr (N == 2) {
+        const float r[8] = {x0.x * y0.x, x0.y * y0.y, x0.z * y0.z, x0.w * y0.w, x1.x * y1.x, x1.y * y1.y, x1.z * y1.z, x1.w * y1.w};
+        split8<2>(r, o);
+        return;
+    }
     const float r[8] = {x0.x * mul * (y0.x + bias), x0.y * mul * (y0.y + bias), x0.z * mul * (y0.z + bias), x0.w * mul * (y0.w + bias),
                         x1.x * mul * (y1.x + bias), x1.y * mul * (y1.y + bias), x1.z * mul * (y1.z + bias), x1.w * mul * (y1.w + bias)};
-    split8<3>(r, o);
+    split8<N>(r, o);
 }
 
 // ================================================================== forward =====
 // SPLIT: one of nsplit shares of the rounds, unnormalised sums to the workspace (see launch_fwd_merge).
-template <class T, int D, int MODE, bool SPLIT>
-__global__ __launch_bounds__((SplitCfg<T, D>::FW * 64)) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 2 : 1, D <= 64 ? 2 : 1)))
+// NQ: planes of Q~; two where q*k2 has 16 bits (bf16 tensors, no bias): the scale is multiplied onto the logits instead, and
+// the logits take two MFMAs per k-step where they took three.
+template <class T, int D, int MODE, bool SPLIT, int NQ>
+__global__ __launch_bounds__((SplitCfg<T, D>::FW * 64)) __attribute__((amdgpu_waves_per_eu(SplitCfg<T, D>::FW / 4, SplitCfg<T, D>::FW / 4)))
 void split_fwd_kernel(Problem p, int nqb, int total) {
     using C = SplitCfg<T, D>;
     constexpr int W = C::FW, NT = W * 64;
@@ -431,11 +440,11 @@ void split_fwd_kernel(Problem p, int nqb, int total) {
         const bool row_ok = ok && i < N && i >= delta;
         const bool rows_full = i0 >= delta && i0 + BQ - 1 < N;
 
-        bf16x8 qf[C::DK][3];
+        bf16x8 qf[C::DK][NQ];
         if (ok) {
 #pragma unroll
             for (int kk = 0; kk < C::DK; ++kk)
-                product_planes<T, PAD>(qp + (int64_t)ic * p.q.sn, k2p + (int64_t)kr * p.k2.sn, kk * 16 + hf * 8, p.D, p.k2_bias, qscale, qf[kk]);
+                product_planes<T, PAD, NQ>(qp + (int64_t)ic * p.q.sn, k2p + (int64_t)kr * p.k2.sn, kk * 16 + hf * 8, p.D, p.k2_bias, qscale, qf[kk]);
         }
         float m = -INFINITY, l = 0.f;
         floatx16 racc[C::DT];
@@ -456,6 +465,7 @@ void split_fwd_kernel(Problem p, int nqb, int total) {
                     logits.add(ka, qf[kk]);
                 }
                 floatx16 sacc = logits.sum();
+                if constexpr (NQ == 2) sacc *= qscale;
                 // register v of this lane: key j0 + 8*(v/4) + 4*hf + v%4
                 const bool interior = rows_full && (j0 + TJ - 1 <= i0) && (j0 >= i0 + BQ - 1 - w1);
                 if (!interior) {
@@ -1258,10 +1268,17 @@ int launch_split_fwd(const Problem& p, hipStream_t st) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(C::FW * 64), C::FWD_LDS, st, p, nqb, (int)grid);
         return hipGetLastError() == hipSuccess;
     };
-    if (p.nsplit <= 1) return go(split_fwd_kernel<T, D, MODE, false>, total) ? SA2_OK : SA2_ERR_LAUNCH_FAILED;
-    const int64_t grid = total * p.nsplit;
-    if (grid > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
-    if (!go(split_fwd_kernel<T, D, MODE, true>, grid)) return SA2_ERR_LAUNCH_FAILED;
+    auto go_split = [&](auto nq) {
+        constexpr int NQ = decltype(nq)::value;
+        if (p.nsplit <= 1) return go(split_fwd_kernel<T, D, MODE, false, NQ>, total);
+        return go(split_fwd_kernel<T, D, MODE, true, NQ>, total * p.nsplit);
+    };
+    if (total * (p.nsplit > 1 ? p.nsplit : 1) > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
+    bool ok;
+    if constexpr (T::PLANES == 1) ok = p.k2_bias == 0.f ? go_split(std::integral_constant<int, 2>{}) : go_split(std::integral_constant<int, 3>{});
+    else ok = go_split(std::integral_constant<int, 3>{});
+    if (!ok) return SA2_ERR_LAUNCH_FAILED;
+    if (p.nsplit <= 1) return SA2_OK;
     return launch_fwd_merge(p, D, T::DTYPE, st);
 }
 
@@ -1402,9 +1419,11 @@ size_t f32_mfma_bwd_scratch_bytes(int B, int N, int H, int head_dim, int w1, int
     return bytes;
 }
 
-int f32_mfma_fwd_nsplit(int B, int N, int H, int head_dim, int w1, int w2) {
-    const int D = split_width(head_dim);
-    return plan_forward(B, N, H, D, w1, w2, D <= 64 ? SplitCfg<MemF32, 64>::FW : SplitCfg<MemF32, 128>::FW);
+int f32_mfma_fwd_nsplit(int B, int N, int H, int head_dim, int w1, int w2, int dtype) {
+    return for_split_width(head_dim, dtype, [&](auto m, auto width, auto) {
+        constexpr int D = decltype(width)::value;
+        return plan_forward(B, N, H, D, w1, w2, SplitCfg<decltype(m), D>::FW);
+    });
 }
 size_t f32_mfma_fwd_part_bytes(int B, int N, int H, int head_dim, int nsplit) { return fwd_part_bytes(B, N, H, split_width(head_dim), nsplit); }
 

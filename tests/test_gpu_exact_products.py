@@ -1,0 +1,28 @@
+"""bf16 tensors of the head dims in between: without biases a product q*k2 or dO*v2 has 16 bits, which two planes hold exactly, and the
+kernels take two where a bias asks for three.  A bias of 1e-30 changes no value (k2 + 1e-30 = k2) but the path: both must be equally
+far from the fp64 oracle.  What differs between them are fp32 roundings, 2^-15 of the rounding of the results, so that the errors differ by
+results on a tie: 1 % is far above that."""
+import pytest
+import torch
+
+from tests.util import make_inputs, oracle_all
+
+pytestmark = pytest.mark.gpu
+NAMES = ("out", "lse", "dq", "dk1", "dk2", "dv1", "dv2")
+
+
+@pytest.mark.parametrize("D", [8, 40, 72, 80, 96, 104, 120])
+@pytest.mark.parametrize("B,N,H,w1,w2,scale", [(1, 33, 1, 5, 1, None), (2, 97, 2, 33, 8, 0.3), (1, 160, 3, 40, 130, None), (1, 300, 1, 310, 0, 0.05), (1, 63, 2, 0, 31, 1.0)])
+def test_two_planes_are_as_exact_as_three(D, B, N, H, w1, w2, scale):
+    import simplical_attn_amd as sa
+    host = make_inputs(B, N, H, D, seed=D + N, dtype=torch.bfloat16)
+    want = oracle_all([x.double() for x in host], w1, w2, scale, 0.0, 0.0)
+    x = [t.to("cuda:0") for t in host]
+    error = {}
+    for bias in (0.0, 1e-30):
+        out, lse = sa.simplicial_forward(*x[:5], w1, w2, scale, bias, bias)
+        got = (out, lse) + sa.simplicial_backward(*x[:5], out, lse, x[5], w1, w2, scale, bias, bias)
+        error[bias] = {n: (g.double().cpu() - want[n].double()).norm().item() for n, g in zip(NAMES, got)}
+        size = {n: want[n].double().norm().item() for n in NAMES}
+    for n in NAMES:
+        assert error[0.0][n] <= 1.01 * error[1e-30][n] + 2e-5 * size[n], (n, error[0.0][n] / size[n], error[1e-30][n] / size[n])
