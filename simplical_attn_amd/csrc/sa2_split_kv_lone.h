@@ -152,9 +152,12 @@ void split_kv_lone_kernel(Problem p, int njb, int total, int nsplit, float* __re
             if (t >= BQ) {
                 lead = lead_planes(row_raw, 0.f);
             } else if (NU == 3) {
-                lead = lse_planes(row_raw);
+                float x = row_raw * LOG2E;
+                stays(x);                                     // (rounded: taken together with the split, lse_rest would count twice)
+                lead = lead_planes(x, lse_rest(row_raw, x));
             } else {
-                const float x = row_raw / p.scale;
+                float x = row_raw / p.scale;
+                stays(x);
                 lead = lead_planes(x, fmaf(-x, p.scale, row_raw) / p.scale);
             }
             *(X8*)(smem_raw + C::LEAD_AT + ((ib & 3) * 2 * BQ + t) * 16) = lead;
