@@ -22,8 +22,7 @@
 // free of bank conflicts.
 #pragma once
 
-#include "sa2_mfma_lone.h"
-#include "sa2_split_common.h"
+#include "sa2_split_lone.h"
 
 namespace sa2 {
 namespace {
@@ -40,21 +39,6 @@ struct SplitKvLoneCfg {
     static constexpr int USED = ONE0 + 4, OWNED = USED <= 192 ? 192 : 256;
     static_assert(USED <= 256 && LDS_BYTES <= 160 * 1024, "");
 };
-// plane products with a sum of planes up to two, the small ones first
-template <int NA, int NB>
-struct Products {
-    int x[NA * NB] = {}, y[NA * NB] = {}, n = 0;
-    constexpr Products() {
-        for (int sum = 2; sum >= 0; --sum)
-            for (int a = 0; a < NA; ++a)
-                if (sum - a >= 0 && sum - a < NB) {
-                    x[n] = a;
-                    y[n] = sum - a;
-                    ++n;
-                }
-    }
-};
-
 template <class T, int D, int NU, int MODE>
 __global__ __launch_bounds__((SplitKvLoneCfg<T, D, NU>::THREADS)) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void split_kv_lone_kernel(Problem p, int njb, int total, int nsplit, float* __restrict__ part) {
@@ -314,42 +298,19 @@ void split_kv_lone_kernel(Problem p, int njb, int total, int nsplit, float* __re
         stays(x);
         dp[i] = x;
     };
-    // (a word of all three planes in four steps of two or three instructions)
     float sh[2];
-    auto split_step = [&](floatx16& of, u4 (&to)[3], auto KS, auto I) __attribute__((always_inline)) {
-        constexpr int t = decltype(I)::value / 4, m = decltype(I)::value % 4, e = 8 * decltype(KS)::value + 2 * t;
-        if constexpr (m == 0 || m == 2) {
-            const uint32_t w = pack2(of[e], of[e + 1]);
-            to[m / 2][t] = w;
-            sh[0] = bf16_lo(w);
-            if constexpr (m == 2) sh[1] = bf16_hi(w);
-            stays(sh[0]);
-        } else if constexpr (m == 1) {
-            float x = of[e] - sh[0], y = of[e + 1] - bf16_hi(to[0][t]);
-            stays(y);
-            of[e] = x;
-            of[e + 1] = y;
-        } else {
-            uint32_t w = pack2(of[e] - sh[0], of[e + 1] - sh[1]);
-            stays(w);
-            to[2][t] = w;
-        }
-    };
-    // items of N that fall to slot SLOT of the slots [FROM, TO)
-    auto within = [&](auto N_, auto SLOT, auto FROM, auto TO, auto&& f) __attribute__((always_inline)) {
-        deal<decltype(N_)::value, decltype(SLOT)::value - decltype(FROM)::value, decltype(TO)::value - decltype(FROM)::value>(f);
-    };
+    auto split_step = [&](floatx16& of, u4 (&to)[3], auto KS, auto I) __attribute__((always_inline)) { split_word_step<decltype(KS)::value, decltype(I)::value>(of, to, sh); };
     // the slots of the forming, where the splits leave room beside the MFMAs; behind them the next unit's rows are requested
     constexpr int FORM = NP >= 5 ? 2 : CH, FORMED = NP >= 5 ? NA + NG : NA + 3 * NG;
     auto beside = [&](auto SLOT, auto DO_C, uint32_t form_at) __attribute__((always_inline)) {
         constexpr int slot = decltype(SLOT)::value;
-        if constexpr (decltype(DO_C)::value) within(LONE_C(16), SLOT, LONE_C(1), LONE_C(CH - 1), [&](auto X) __attribute__((always_inline)) { split_step(dp, dw[1], LONE_C(1), X); });
-        within(LONE_C(16), SLOT, LONE_C(CH + 2), LONE_C(NA + 1), exp_item);
-        within(LONE_C(16), SLOT, LONE_C(NA + 2), LONE_C(NA + NG), ds_item);
-        within(LONE_C(16), SLOT, LONE_C(NA + NG), LONE_C(NA + 2 * NG), [&](auto X) __attribute__((always_inline)) { split_step(s, pw[0], LONE_C(0), X); });
-        within(LONE_C(16), SLOT, LONE_C(NA + 2 * NG), LONE_C(NA + 3 * NG), [&](auto X) __attribute__((always_inline)) { split_step(s, pw[1], LONE_C(1), X); });
-        within(LONE_C(16), SLOT, LONE_C(NA + 3 * NG), LONE_C(NS), [&](auto X) __attribute__((always_inline)) { split_step(dp, dw[0], LONE_C(0), X); });
-        within(LONE_C(NF * STEPS), SLOT, LONE_C(FORM), LONE_C(FORMED), [&](auto X) __attribute__((always_inline)) { form_step(X, form_at); });
+        if constexpr (decltype(DO_C)::value) within<16, slot, 1, CH - 1>([&](auto X) __attribute__((always_inline)) { split_step(dp, dw[1], LONE_C(1), X); });
+        within<16, slot, CH + 2, NA + 1>(exp_item);
+        within<16, slot, NA + 2, NA + NG>(ds_item);
+        within<16, slot, NA + NG, NA + 2 * NG>([&](auto X) __attribute__((always_inline)) { split_step(s, pw[0], LONE_C(0), X); });
+        within<16, slot, NA + 2 * NG, NA + 3 * NG>([&](auto X) __attribute__((always_inline)) { split_step(s, pw[1], LONE_C(1), X); });
+        within<16, slot, NA + 3 * NG, NS>([&](auto X) __attribute__((always_inline)) { split_step(dp, dw[0], LONE_C(0), X); });
+        within<NF * STEPS, slot, FORM, FORMED>([&](auto X) __attribute__((always_inline)) { form_step(X, form_at); });
         if constexpr (slot == FORMED) request_unit();
     };
     auto unit = [&](auto DO_C) __attribute__((always_inline)) {

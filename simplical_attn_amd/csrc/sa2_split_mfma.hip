@@ -44,6 +44,7 @@
 // while the dS wavefront multiplies and splits dS, whose product follows.
 // Every output element has one writer and a fixed summation order: no atomics, bitwise reproducible.
 #include "sa2_fma_rows.h"
+#include "sa2_split_kp_lone_plan.h"
 #include "sa2_split_common.h"
 
 namespace sa2 {
@@ -1131,12 +1132,19 @@ size_t split_dq_part_bytes(int B, int N, int H, int D, const KpPlan& pl) {
 size_t split_kp_bytes(int B, int N, int H, int D, const KpPlan& pl) {
     return split_dq_part_bytes(B, N, H, D, pl) + (pl.nseg > 1 ? (size_t)2 * pl.nseg * B * H * (size_t)N * D * sizeof(float) : 0);
 }
+// Whether the backward runs with one wavefront per SIMD (sa2_split_kv_lone.h, sa2_split_kp_lone.h)
+template <class T, int D, int MODE>
+constexpr bool lone() { return T::DTYPE == SA2_F32 ? MODE != PADDED_FINE && D <= 64 : D == 64 || D == 96; }
 // Deltas per segment: what the dQ accumulator in LDS holds, or fewer where the grid asks for it
-template <class T, int D>
+template <class T, int D, int MODE>
 KpPlan split_kp_plan(int B, int N, int H, int w1, int w2, size_t room) {
     using C = SplitCfg<T, D>;
     int most = NPAIR;
-    while (most < w2 + 1 && C::kp_fits(most + NPAIR - 1)) most += NPAIR;
+    auto fits = [](int segw) {
+        if constexpr (lone<T, D, MODE>()) return SplitKpLoneCfg<D, T::PLANES>::fits(segw);
+        else return C::kp_fits(segw - 1);
+    };
+    while (most < w2 + 1 && fits(most + NPAIR)) most += NPAIR;
     return plan_segments(B, N, H, w1, w2, NPAIR, most, room, [](int) { return false; }, [&](const KpPlan& pl) { return split_kp_bytes(B, N, H, D, pl); });
 }
 
@@ -1166,9 +1174,6 @@ int launch_split_fwd(const Problem& p, hipStream_t st) {
     return launch_fwd_merge(p, D, T::DTYPE, st);
 }
 
-// Whether the K side runs with one wavefront per SIMD (sa2_split_kv_lone.h)
-template <class T, int D, int MODE>
-constexpr bool kv_lone() { return T::DTYPE == SA2_F32 ? MODE != PADDED_FINE && D <= 64 : D == 64 || D == 96; }
 // Whether products of a unit have 16 bits, so that two planes hold them and the scale may wait until they are summed
 template <class T>
 bool exact_products(const Problem& p) {
@@ -1180,7 +1185,7 @@ int launch_split_bwd(const Problem& p, hipStream_t st) {
     using C = SplitCfg<T, D>;
     BwdSums sums = {};
     const size_t room = room_left(p.room, guard_bytes(p.B, p.N, p.H));
-    const KpPlan pl = split_kp_plan<T, D>(p.B, p.N, p.H, p.w1, p.w2, room);
+    const KpPlan pl = split_kp_plan<T, D, MODE>(p.B, p.N, p.H, p.w1, p.w2, room);
     const size_t kp_bytes = (split_kp_bytes(p.B, p.N, p.H, D, pl) + 255) / 256 * 256;
     const int nsplit = split_kv_nsplit(p.B, p.N, p.H, D, p.w1, p.w2, room_left(room, kp_bytes));
     const size_t part_bytes = kp_bytes + split_kv_bytes(p.B, p.N, p.H, D, nsplit);
@@ -1200,10 +1205,17 @@ int launch_split_bwd(const Problem& p, hipStream_t st) {
         if (total > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
         float* part = (float*)p.scratch;
         float* kpart = (float*)((char*)p.scratch + split_dq_part_bytes(p.B, p.N, p.H, D, pl));
-        if (!allow_full_lds((const void*)split_kp_kernel<T, D, MODE>)) return SA2_ERR_LAUNCH_FAILED;
-        hipLaunchKernelGGL((split_kp_kernel<T, D, MODE>), dim3((unsigned)total), dim3(XT), C::kp_lds(pl.segw - 1), st, p, nkb, (int)per_seg, part,
-                           pl.nseg, pl.segw, kpart);
-        if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
+        if constexpr (lone<T, D, MODE>()) {
+            const SplitKpLaunch l = {pl, nkb, (int)per_seg, part, kpart};
+            const int rc = (T::DTYPE == SA2_F32 ? launch_split_kp_lone_fp32 : T::DTYPE == SA2_F16 ? launch_split_kp_lone_fp16 : launch_split_kp_lone_bf16)(
+                p, D, exact_products<T>(p), l, st);
+            if (rc != SA2_OK) return rc;
+        } else {
+            if (!allow_full_lds((const void*)split_kp_kernel<T, D, MODE>)) return SA2_ERR_LAUNCH_FAILED;
+            hipLaunchKernelGGL((split_kp_kernel<T, D, MODE>), dim3((unsigned)total), dim3(XT), C::kp_lds(pl.segw - 1), st, p, nkb, (int)per_seg, part,
+                               pl.nseg, pl.segw, kpart);
+            if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
+        }
         sums.dq = p.dq.p ? part : nullptr;
         sums.nkb = nkb;
         sums.nseg = sums.kp_n = pl.nseg;
@@ -1215,7 +1227,7 @@ int launch_split_bwd(const Problem& p, hipStream_t st) {
         const int64_t total = (int64_t)njb * p.B * p.H * nsplit;
         if (total > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
         float* part = nsplit > 1 ? (float*)((char*)p.scratch + kp_bytes) : nullptr;
-        if constexpr (kv_lone<T, D, MODE>()) {
+        if constexpr (lone<T, D, MODE>()) {
             const int rc = (T::DTYPE == SA2_F32 ? launch_split_kv_lone_fp32 : T::DTYPE == SA2_F16 ? launch_split_kv_lone_fp16 : launch_split_kv_lone_bf16)(
                 p, D, exact_products<T>(p), nsplit, part, st);
             if (rc != SA2_OK) return rc;
@@ -1309,9 +1321,9 @@ size_t f32_mfma_bwd_scratch_bytes(int B, int N, int H, int head_dim, int w1, int
     const size_t guard = guard_bytes(B, N, H);
     size_t bytes = 0;
     room = room_left(room, guard);
-    for_split_width(head_dim, dtype, [&](auto m, auto width, auto) {
+    for_split_width(head_dim, dtype, [&](auto m, auto width, auto mode) {
         constexpr int D = decltype(width)::value;
-        const size_t kp = (split_kp_bytes(B, N, H, D, split_kp_plan<decltype(m), D>(B, N, H, w1, w2, room)) + 255) / 256 * 256;
+        const size_t kp = (split_kp_bytes(B, N, H, D, split_kp_plan<decltype(m), D, decltype(mode)::value>(B, N, H, w1, w2, room)) + 255) / 256 * 256;
         bytes = kp + split_kv_bytes(B, N, H, D, split_kv_nsplit(B, N, H, D, w1, w2, room_left(room, kp))) + guard;
         return 0;
     });
