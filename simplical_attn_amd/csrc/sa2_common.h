@@ -208,7 +208,11 @@ int launch_f32_mfma_fwd(const Problem& p, int dtype, hipStream_t st);
 int f32_mfma_fwd_nsplit(int B, int N, int H, int D, int w1, int w2, int dtype);
 size_t f32_mfma_fwd_part_bytes(int B, int N, int H, int D, int nsplit);
 int launch_f32_mfma_bwd(const Problem& p, int dtype, hipStream_t st);
-// Its K side with one wavefront per SIMD (sa2_split_kv_lone.h).  `width`: of the kernel; `two_planes`: products of a unit have 16 bits
+// Its forward and K side with one wavefront per SIMD (sa2_split_fwd_lone.h, sa2_split_kv_lone.h).  `width`: of the kernel; `two_planes`:
+// products of a unit have 16 bits
+int launch_split_fwd_lone_bf16(const Problem& p, int width, bool two_planes, hipStream_t st);
+int launch_split_fwd_lone_fp16(const Problem& p, int width, bool two_planes, hipStream_t st);
+int launch_split_fwd_lone_fp32(const Problem& p, int width, bool two_planes, hipStream_t st);
 int launch_split_kv_lone_bf16(const Problem& p, int width, bool two_planes, int nsplit, float* part, hipStream_t st);
 int launch_split_kv_lone_fp16(const Problem& p, int width, bool two_planes, int nsplit, float* part, hipStream_t st);
 int launch_split_kv_lone_fp32(const Problem& p, int width, bool two_planes, int nsplit, float* part, hipStream_t st);

@@ -99,7 +99,7 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(Problem p, int D, int64_
         *(float4*)((float*)p.out.p + p.out.off(b, i, h) + col) = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
     else
         *(uint2*)((uint16_t*)p.out.p + p.out.off(b, i, h) + col) = make_uint2(E::pack(acc.x * inv, acc.y * inv), E::pack(acc.z * inv, acc.w * inv));
-    if (col == 0) p.lse[row] = big ? LN2 * Mu + logf(denom) : LN_EPS + logf(denom);
+    if (col == 0) p.lse[row] = exact_lse(Mu, denom, big);
 }
 
 }  // namespace

@@ -115,6 +115,12 @@ int for_mfma_width(int D, int dtype, F&& f) {
     return dtype == SA2_F16 ? of_type(ElemF16{}) : of_type(ElemBF16{});
 }
 
+// LSE of a row whose weights, in units of 2^M, sum to `denom` (`big`), or to denom in units of 1e-8.  In 64 bits, since a reference point
+// that is not the row's maximum leaves a sum whose logarithm is larger and carries a larger rounding (1.1 to 1.2 times the error of an fp32 LSE).
+__device__ __forceinline__ float exact_lse(float M, float denom, bool big) {
+    return (float)((big ? 0.6931471805599453094 * (double)M : -18.420680743952365472) + log((double)denom));
+}
+
 // Exchange between lane l and lane l^32 (one VALU op): returns the partner's value.
 __device__ __forceinline__ float other_half(float x) {
     const unsigned u = __float_as_uint(x);

@@ -12,6 +12,7 @@ __device__ __forceinline__ floatx16 zero16() {
     for (int v = 0; v < 16; ++v) z[v] = 0.f;
     return z;
 }
+constexpr float TINY = 7.888609052210118e-31f;     // 2^-100
 typedef float fx4 __attribute__((ext_vector_type(4)));      // 16 bytes in flight (plain vectors: stay in registers)
 typedef unsigned ux2 __attribute__((ext_vector_type(2)));
 

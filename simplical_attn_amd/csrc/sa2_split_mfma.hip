@@ -29,13 +29,14 @@
 //   split_fwd_kernel    32 queries per workgroup; wavefront w takes delta = w, w+W, ... and keeps one
 //                       online softmax and one output accumulator across its units; the W are
 //                       merged once at the end.
+//                       For fp32 at 64 columns and less (but for the finer sums) and 16 bits at 64 and 96, here and below:
+//                       sa2_split_fwd_lone.h, sa2_split_kp_lone.h and sa2_split_kv_lone.h.
 //   split_kp_kernel     32 K' rows per workgroup and every delta (or a segment of them).  After a unit's
 //                       sweep its three reductions go to fp32 accumulators in LDS in column-rotated
 //                       phases: dK' and dV' rows are aligned with the unit's rows, dQ rows are shifted by
 //                       delta; the dQ accumulator is written once per workgroup as a partial.
 //   split_kv_kernel     128 K/V rows per workgroup (32 per wavefront pair, resident in registers as B
 //                       operands), streaming every unit (query block, delta) that can see them.
-//                       For fp32 at 64 columns and less (but for the finer sums) and 16 bits at 64 and 96: sa2_split_kv_lone.h.
 // The backward kernels pair their eight wavefronts as the 16-bit kernels do (one P and one dS wavefront per SIMD, so that
 // each holds the planes of one operand and one accumulator in 256 registers: four wavefronts that did both needed 350 and
 // moved 136 of them between the two register files per tile; at 128 columns in fp32 they do not fit all the same, and 470
@@ -53,7 +54,6 @@ namespace {
 constexpr int NPAIR = 4;               // wavefront pairs per workgroup of the backward kernels
 constexpr int XT = NPAIR * 2 * 64;     // threads per workgroup
 constexpr int XJ = NPAIR * 32;         // K rows per workgroup of the K-side kernel
-constexpr float TINY = 7.888609052210118e-31f;     // 2^-100
 
 template <class T, int D>
 struct SplitCfg {
@@ -66,9 +66,9 @@ struct SplitCfg {
     static constexpr int PLANE = 32 * RS;      // elements
     static constexpr int AS = D + 4;           // row stride of fp32 accumulators in LDS
     static constexpr size_t LDS_LIMIT = 160 * 1024;
-    // Forward: eight wavefronts (two per SIMD) where operands and accumulators fit 256 registers, else four: bf16 at 96 columns (254 with
-    // three planes of Q~, 230 with two) 364 -> 239 us at B1 H8 N2048 D96 w 255/31; fp16 takes 350 there.
-    static constexpr int FW = D <= 64 || (D == 96 && T::PLANES == 1) ? 8 : 4;
+    // Forward: eight wavefronts (two per SIMD) where operands and accumulators fit 256 registers, else four.  (The kernel with two units
+    // per wavefront has eight units per round as well.)
+    static constexpr int FW = D <= 64 || (D == 96 && T::PLANES < 3) ? 8 : 4;
     static constexpr int KV_TILE = NK * PLANE;             // a K or V tile
     static constexpr int KV_STAGE = 2 * KV_TILE;           // K tile, then V tile
     static constexpr size_t FWD_TILES = (size_t)2 * KV_STAGE * 2;
@@ -253,8 +253,8 @@ __device__ __forceinline__ void product_planes(const typename T::T* xrow, const 
 
 // ================================================================== forward =====
 // SPLIT: one of nsplit shares of the rounds, unnormalised sums to the workspace (see launch_fwd_merge).
-// NQ: planes of Q~; two where q*k2 has 16 bits (bf16 tensors, no bias): the scale is multiplied onto the logits instead, and
-// the logits take two MFMAs per k-step where they took three.
+// NQ: planes of Q~; two where q*k2 has 16 bits (bf16 tensors, no bias): the scale is multiplied onto the logits instead, which take
+// two MFMAs per k-step rather than three.
 template <class T, int D, int MODE, bool SPLIT, int NQ>
 __global__ __launch_bounds__((SplitCfg<T, D>::FW * 64)) __attribute__((amdgpu_waves_per_eu(SplitCfg<T, D>::FW / 4, SplitCfg<T, D>::FW / 4)))
 void split_fwd_kernel(Problem p, int nqb, int total) {
@@ -1132,7 +1132,12 @@ size_t split_dq_part_bytes(int B, int N, int H, int D, const KpPlan& pl) {
 size_t split_kp_bytes(int B, int N, int H, int D, const KpPlan& pl) {
     return split_dq_part_bytes(B, N, H, D, pl) + (pl.nseg > 1 ? (size_t)2 * pl.nseg * B * H * (size_t)N * D * sizeof(float) : 0);
 }
-// Whether the backward runs with one wavefront per SIMD (sa2_split_kv_lone.h, sa2_split_kp_lone.h)
+// Whether products of a unit have 16 bits, so that two planes hold them and the scale may wait until they are summed
+template <class T>
+bool exact_products(const Problem& p, bool backward) {
+    return T::DTYPE == SA2_BF16 && p.k2_bias == 0.f && (!backward || p.v2_bias == 0.f) && p.scale >= 8.6736174e-19f && p.scale <= 1.1529215e18f;     // 2^-60 .. 2^60
+}
+// Whether the kernels with one wavefront per SIMD are taken (sa2_split_fwd_lone.h, sa2_split_kv_lone.h, sa2_split_kp_lone.h)
 template <class T, int D, int MODE>
 constexpr bool lone() { return T::DTYPE == SA2_F32 ? MODE != PADDED_FINE && D <= 64 : D == 64 || D == 96; }
 // Deltas per segment: what the dQ accumulator in LDS holds, or fewer where the grid asks for it
@@ -1151,33 +1156,33 @@ KpPlan split_kp_plan(int B, int N, int H, int w1, int w2, size_t room) {
 // ------------------------------------------------------------------ launchers ----
 template <class T, int D, int MODE>
 int launch_split_fwd(const Problem& p, hipStream_t st) {
-    using C = SplitCfg<T, D>;
-    const int nqb = (p.N + BQ - 1) / BQ;
-    const int64_t total = (int64_t)nqb * p.B * p.H;
-    if (total > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
-    auto go = [&](auto kernel, int64_t grid) {
-        if (!allow_full_lds((const void*)kernel)) return false;
-        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(C::FW * 64), C::FWD_LDS, st, p, nqb, (int)grid);
-        return hipGetLastError() == hipSuccess;
-    };
-    auto go_split = [&](auto nq) {
-        constexpr int NQ = decltype(nq)::value;
-        if (p.nsplit <= 1) return go(split_fwd_kernel<T, D, MODE, false, NQ>, total);
-        return go(split_fwd_kernel<T, D, MODE, true, NQ>, total * p.nsplit);
-    };
-    if (total * (p.nsplit > 1 ? p.nsplit : 1) > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
-    bool ok;
-    if constexpr (T::PLANES == 1) ok = p.k2_bias == 0.f ? go_split(std::integral_constant<int, 2>{}) : go_split(std::integral_constant<int, 3>{});
-    else ok = go_split(std::integral_constant<int, 3>{});
-    if (!ok) return SA2_ERR_LAUNCH_FAILED;
-    if (p.nsplit <= 1) return SA2_OK;
-    return launch_fwd_merge(p, D, T::DTYPE, st);
-}
-
-// Whether products of a unit have 16 bits, so that two planes hold them and the scale may wait until they are summed
-template <class T>
-bool exact_products(const Problem& p) {
-    return T::DTYPE == SA2_BF16 && p.k2_bias == 0.f && p.v2_bias == 0.f && p.scale >= 8.6736174e-19f && p.scale <= 1.1529215e18f;     // 2^-60 .. 2^60
+    if constexpr (lone<T, D, MODE>()) {
+        const int rc = (T::DTYPE == SA2_F32 ? launch_split_fwd_lone_fp32 : T::DTYPE == SA2_F16 ? launch_split_fwd_lone_fp16 : launch_split_fwd_lone_bf16)(
+            p, D, exact_products<T>(p, false), st);
+        return rc != SA2_OK || p.nsplit <= 1 ? rc : launch_fwd_merge(p, D, T::DTYPE, st);
+    } else {
+        using C = SplitCfg<T, D>;
+        const int nqb = (p.N + BQ - 1) / BQ;
+        const int64_t total = (int64_t)nqb * p.B * p.H;
+        if (total > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
+        auto go = [&](auto kernel, int64_t grid) {
+            if (!allow_full_lds((const void*)kernel)) return false;
+            hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(C::FW * 64), C::FWD_LDS, st, p, nqb, (int)grid);
+            return hipGetLastError() == hipSuccess;
+        };
+        auto go_split = [&](auto nq) {
+            constexpr int NQ = decltype(nq)::value;
+            if (p.nsplit <= 1) return go(split_fwd_kernel<T, D, MODE, false, NQ>, total);
+            return go(split_fwd_kernel<T, D, MODE, true, NQ>, total * p.nsplit);
+        };
+        if (total * (p.nsplit > 1 ? p.nsplit : 1) > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
+        bool ok;
+        if constexpr (T::PLANES == 1) ok = p.k2_bias == 0.f ? go_split(std::integral_constant<int, 2>{}) : go_split(std::integral_constant<int, 3>{});
+        else ok = go_split(std::integral_constant<int, 3>{});
+        if (!ok) return SA2_ERR_LAUNCH_FAILED;
+        if (p.nsplit <= 1) return SA2_OK;
+        return launch_fwd_merge(p, D, T::DTYPE, st);
+    }
 }
 
 template <class T, int D, int MODE>
@@ -1208,7 +1213,7 @@ int launch_split_bwd(const Problem& p, hipStream_t st) {
         if constexpr (lone<T, D, MODE>()) {
             const SplitKpLaunch l = {pl, nkb, (int)per_seg, part, kpart};
             const int rc = (T::DTYPE == SA2_F32 ? launch_split_kp_lone_fp32 : T::DTYPE == SA2_F16 ? launch_split_kp_lone_fp16 : launch_split_kp_lone_bf16)(
-                p, D, exact_products<T>(p), l, st);
+                p, D, exact_products<T>(p, true), l, st);
             if (rc != SA2_OK) return rc;
         } else {
             if (!allow_full_lds((const void*)split_kp_kernel<T, D, MODE>)) return SA2_ERR_LAUNCH_FAILED;
@@ -1229,7 +1234,7 @@ int launch_split_bwd(const Problem& p, hipStream_t st) {
         float* part = nsplit > 1 ? (float*)((char*)p.scratch + kp_bytes) : nullptr;
         if constexpr (lone<T, D, MODE>()) {
             const int rc = (T::DTYPE == SA2_F32 ? launch_split_kv_lone_fp32 : T::DTYPE == SA2_F16 ? launch_split_kv_lone_fp16 : launch_split_kv_lone_bf16)(
-                p, D, exact_products<T>(p), nsplit, part, st);
+                p, D, exact_products<T>(p, true), nsplit, part, st);
             if (rc != SA2_OK) return rc;
         } else {
             auto go = [&](auto kernel) {

@@ -1,0 +1,68 @@
+"""out and lse of the plane-split forward with two units per wavefront where its rounds and its stream of tiles can go wrong: rounds of one to
+eight units (four and fewer have one per wavefront), sweeps shorter than the tiles that are requested ahead, windows that end in the
+middle of a tile, a last tile that the sequence does not fill, shares, both plane counts, and logits that leave the reference point of the
+first tile behind (a unit's sums are brought to another one).  Against the fp32 FMA kernels (accurate expf and logf), to the bars of the
+other tests of these kernels; lse to 1e-5 of its largest value (16 bits: of exact products of 16-bit inputs, the same)."""
+import pytest
+import torch
+
+from tests.util import assert_close_rel
+
+pytestmark = pytest.mark.gpu
+BF, FP, F32 = torch.bfloat16, torch.float16, torch.float32
+BAR = {BF: 1e-2, FP: 2e-3, F32: 1e-5}
+TYPES = [(F32, 16), (F32, 32), (F32, 64), (BF, 40), (BF, 56), (BF, 72), (BF, 96), (FP, 48), (FP, 80)]
+
+
+def _inputs(dtype, B, N, H, D, seed, std=1.0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return [(torch.randn(B, N, H, D, generator=g, device="cuda") * (std if t < 3 else 1.0)).to(dtype) for t in range(5)]
+
+
+@pytest.mark.parametrize("dtype,D", TYPES)
+@pytest.mark.parametrize("B,N,H,w1,w2,bias,scale", [
+    (1, 1, 1, 0, 0, 0.0, None), (1, 33, 1, 0, 0, 0.0, None), (1, 300, 2, 40, 0, 0.1, None), (2, 129, 1, 128, 3, 0.0, 0.2), (1, 97, 3, 31, 4, 0.0, None),
+    (1, 200, 1, 500, 8, 0.2, None), (1, 161, 1, 3, 12, 0.0, -0.1), (1, 700, 40, 129, 5, 0.0, None), (1, 520, 2, 95, 33, -0.1, None), (3, 40, 5, 40, 39, 0.0, 0.0),
+    (1, 640, 30, 70, 40, 0.0, None)])
+def test_forward_matches_the_fma_kernels(dtype, D, B, N, H, w1, w2, bias, scale):
+    import simplical_attn_amd as sa
+    x = _inputs(dtype, B, N, H, D, N + D)
+    out, lse = sa.simplicial_forward(*x, w1, w2, scale, bias, -bias)
+    want, want_lse = sa.simplicial_forward(*x, w1, w2, scale, bias, -bias, flags=1)
+    assert_close_rel(out, want.cpu(), BAR[dtype], "out")
+    assert_close_rel(lse, want_lse.cpu(), 1e-5, "lse")
+    assert torch.equal(out, sa.simplicial_forward(*x, w1, w2, scale, bias, -bias)[0])
+
+
+@pytest.mark.parametrize("dtype,D", TYPES)
+@pytest.mark.parametrize("heads,w2,bias", [(2, 12, 0.0), (40, 3, 0.0), (40, 20, 0.3)])
+def test_logits_that_leave_the_reference_point_behind(dtype, D, heads, w2, bias):
+    """Keys away from the queries' own tile have logits more than 64 octaves above it.  A row's largest logits
+    decide it; they are off by 2^-24 of the sum of the products' magnitudes (here up to 2^10) per rounding, which lse shows (absolute)."""
+    import simplical_attn_amd as sa
+    x = _inputs(dtype, 1, 470, heads, D, D)
+    x[0] = x[0].abs() + 0.5
+    x[2] = x[2].abs() + 0.5
+    ramp = torch.where(torch.arange(470, device="cuda") % 170 < 60, 3.0, -3.0)[None, :, None, None]
+    x[1] = (ramp + 0.1 * x[1].float()).to(dtype)
+    out, lse = sa.simplicial_forward(*x, 300, w2, 90.0 / D, bias, bias)
+    want, want_lse = sa.simplicial_forward(*x, 300, w2, 90.0 / D, bias, bias, flags=1)
+    assert torch.isfinite(out).all() and (lse.abs().max() > 100)
+    assert_close_rel(lse, want_lse.cpu(), 2e-5, "lse")
+    assert_close_rel(out, want.cpu(), max(BAR[dtype], 2e-3), "out")
+
+
+@pytest.mark.parametrize("dtype,D", TYPES)
+@pytest.mark.parametrize("std", [3.0, 4.0])
+def test_widely_spread_logits(dtype, D, std):
+    """Logits of standard deviation 27 and 64 on single rows: the reference point moves in some rows and not in others, first rows whose units
+    have no key among them.  They are off by 2^-24 of the sum of the products' magnitudes (some 2^9) per rounding, and so are lse and, near
+    ties, out."""
+    import simplical_attn_amd as sa
+    x = _inputs(dtype, 1, 400, 6, D, D, std)
+    for w2 in (3, 20):
+        out, lse = sa.simplicial_forward(*x, 150, w2)
+        want, want_lse = sa.simplicial_forward(*x, 150, w2, flags=1)
+        assert torch.isfinite(out).all()
+        assert_close_rel(lse, want_lse.cpu(), 1e-5, "lse")
+        assert_close_rel(out, want.cpu(), max(BAR[dtype], 1e-3), "out")
