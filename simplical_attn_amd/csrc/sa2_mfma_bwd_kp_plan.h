@@ -43,17 +43,21 @@ struct KpLoneCfg {
     static bool raw_fits(int w2) { return lds_bytes(w2, true) <= LDS_LIMIT; }
     static bool wide_fits(int w2) { return lds_bytes(w2, raw_fits(w2), true) <= LDS_LIMIT; }
     static bool fits(int w2) { return lds_bytes(w2, false) <= LDS_LIMIT; }
-    // Whether the kernel is taken, by the keys a K' row's queries see on average (the window, less where the sequence begins).  A
-    // tile of the sweep takes it 0.76 us per eight deltas (head_dim 64; the two-wavefront kernel 1.04) or 0.71 per four (128; 0.89),
-    // but what lies between two sweeps and around them is not overlapped: 2.4 and 4.0 us more per round, and more again once per
-    // launch and where the last wave of workgroups is not full.  Fitted to both kernels' times at 12 sizes by 12 K' windows each
-    // (profiles/plan_cuts.md): what is taken is at most 1 % slower than the other one.  `units`: deltas of a workgroup.
+    // Whether the kernel is taken, by the keys a K' row's queries see on average (the window, less where the sequence begins): a tile of
+    // the sweep takes it less than the two-wavefront kernel, but what lies between two sweeps and around them is not overlapped, and a
+    // wavefront without a unit in a round is idle: `busy` is the keys per unit that a round has room for.  `units`: deltas of a
+    // workgroup.  Fitted to both kernels at 150 shapes; time of the other one over this one's, K' side with its pre- and post-pass:
+    // head_dim 64: N3000 BH8 w 150/9 0.98, /20 0.99, /31 1.02, w 250/4 1.01, /9 1.06, /31 1.08; N1500 BH8 w 250/20 1.06; N1000 BH30 w 250/31 1.10;
+    //   BH16 N4096 w 256/64 1.15; N2600 BH4 w 150/40 0.96; one to three deltas 0.80 - 0.99 with up to 240 keys.
+    // head_dim 128: N16384 BH8 w 260/4 1.02, /9 1.05, /31 1.08; N8192 BH3 w 300/4 0.96, /9 1.02, /31 1.04; N1000 BH30 w 300/31 1.06; N1200 BH6 w 260/31 0.90.
+    //   Between one and three workgroups a CU both signs occur (0.96 - 1.10) and the older, later line stays.
     static bool wanted(int N, int w1, int units, int64_t workgroups) {
         const int64_t w = w1 < N ? w1 : N;
         const double keys = w - w * w / (2.0 * N), waves = (double)workgroups / CUS;
-        if (D == 64) return keys >= 300 && keys >= 250 + 1000.0 / units;             // (a wavefront holds two units, of which one may not exist)
         const int rounds = (units + U * W - 1) / (U * W);
-        return keys >= 420 && keys >= 320 + (160 + 3000.0 / rounds) / waves;
+        const double busy = keys * units / (rounds * U * W);
+        if (D == 64) return (units >= 6 && busy >= 136) || (keys >= 300 && keys >= 250 + 1000.0 / units);
+        return (units >= 8 && busy >= 210 && waves >= 3) || (keys >= 420 && keys >= 320 + (160 + 3000.0 / rounds) / waves);
     }
 };
 

@@ -122,3 +122,16 @@ def test_a_gradient_that_is_not_a_number_stays_in_its_windows(D, N, heads, w1, w
     for a, b, lo, hi in zip(got, clean, (r, max(r - w1, 0) // 32 * 32, r - w2, max(r - w1, 0) // 32 * 32, r - w2), (r, r // 32 * 32 + 31, r, r // 32 * 32 + 31, r)):
         assert a[:, max(r - (w2 if hi == r and lo != r else 0), lo):r + 1].isnan().all()
         assert torch.equal(a[:, :lo], b[:, :lo]) and torch.equal(a[:, hi + 1:], b[:, hi + 1:])
+
+
+@pytest.mark.parametrize("dtype,B,N,H,D,w1,w2,bias", [
+    (BF, 1, 353, 8, 64, 2000, 130, 0.1),    # a sequence shorter than its window; segments
+    (FP, 2, 513, 4, 64, 250, 32, 0.0),
+    (BF, 1, 1111, 6, 64, 193, 6, -0.2),     # seven units of eight, the fewest deltas here
+    (FP, 1, 1027, 27, 64, 160, 63, 0.3),
+    (BF, 1, 1601, 17, 128, 233, 15, 0.1),
+    (FP, 1, 1000, 40, 128, 260, 47, -0.3),
+])
+def test_narrower_windows_of_many_deltas(dtype, B, N, H, D, w1, w2, bias):
+    """K windows of a few tiles, whose sweeps mostly begin and end inside one: dQ, dK' and dV' as above."""
+    test_kp_side_matches_the_fma_kernels(dtype, B, N, H, D, w1, w2, bias)

@@ -55,6 +55,16 @@ def test_kp_cases_reach_the_kernel():
         assert kp_route(1, N, heads, D, w1 - 1, w2 - 1)[1]
 
 
+def test_kp_side_of_narrower_windows():
+    """by the keys per unit that a round has room for, and at head_dim 128 by the grid"""
+    cases = _cases(test_gpu_bwd_kp_lone.test_narrower_windows_of_many_deltas)
+    routes = {c[1:7]: kp_route(*c[1:7]) for c in cases}
+    assert all(lone for _, lone, _ in routes.values()) and routes[1, 353, 8, 64, 2000, 130][2] > 1
+    for not_taken in ((1, 3000, 8, 64, 150, 9), (1, 4096, 16, 64, 256, 3), (1, 2048, 4, 64, 128, 32), (1, 1200, 6, 128, 260, 31),
+                      (1, 8192, 16, 128, 256, 4), (1, 8192, 16, 128, 192, 31)):
+        assert not kp_route(*not_taken)[1]
+
+
 def test_k2_row_cases_reach_the_kernel():
     routes = {c[4:6] + c[6:7]: kp_route(*c[1:7]) for c in _cases(test_gpu_bwd_kp_lone.test_k2_rows_in_both_forms)}
     assert all(lone for _, lone, _ in routes.values()) and routes[128, 900, 24][0] and routes[64, 500, 32][0]
