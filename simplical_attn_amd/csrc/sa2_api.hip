@@ -258,10 +258,10 @@ size_t sa2_fwd_workspace_bytes(int B, int N, int H, int D, int w1, int w2, int d
     if (check_dims(B, N, H, D, w1, w2, dtype, window_inclusive) != SA2_OK || (flags & SA2_FLAG_FORCE_GENERIC)) return 0;
     w1 = reach(w1, window_inclusive, N);
     w2 = reach(w2, window_inclusive, N);
-    if (f32_mfma_supported(D, dtype)) return f32_mfma_fwd_part_bytes(B, N, H, D, f32_mfma_fwd_nsplit(B, N, H, D, w1, w2, dtype));
+    if (f32_mfma_supported(D, dtype)) return f32_mfma_fwd_part_bytes(B, N, H, D, f32_mfma_fwd_nsplit(B, N, H, D, w1, w2, dtype, ROOM_ANY));
     if (mfma_supported(B, N, H, D, w1, w2, dtype))
-        return mfma_fwd_part_bytes(B, N, H, D, mfma_fwd_nsplit(B, N, H, D, w1, w2, (flags & SA2_FLAG_FORCE_MFMA) != 0));
-    if (wide_supported(D, dtype)) return fwd_part_bytes(B, N, H, D, wide_fwd_nsplit(B, N, H, w1, w2));
+        return mfma_fwd_part_bytes(B, N, H, D, mfma_fwd_nsplit(B, N, H, D, w1, w2, (flags & SA2_FLAG_FORCE_MFMA) != 0, ROOM_ANY));
+    if (wide_supported(D, dtype)) return fwd_part_bytes(B, N, H, D, wide_fwd_nsplit(B, N, H, w1, w2, ROOM_ANY));
     return 0;
 }
 
@@ -298,9 +298,9 @@ int sa2_forward_ws(const void* q, const void* k1, const void* k2, const void* v1
     // shares of the rounds, where the caller brought room for their partial outputs
     p.nsplit = 1;
     if (workspace) {
-        const int ns = path == PATH_MFMA16   ? mfma_fwd_nsplit(B, N, H, D, p.w1, p.w2, p.force_prepass != 0)
-                       : path == PATH_MFMA32 ? f32_mfma_fwd_nsplit(B, N, H, D, p.w1, p.w2, dtype)
-                       : path == PATH_WIDE16 ? wide_fwd_nsplit(B, N, H, p.w1, p.w2)
+        const int ns = path == PATH_MFMA16   ? mfma_fwd_nsplit(B, N, H, D, p.w1, p.w2, p.force_prepass != 0, workspace_bytes)
+                       : path == PATH_MFMA32 ? f32_mfma_fwd_nsplit(B, N, H, D, p.w1, p.w2, dtype, workspace_bytes)
+                       : path == PATH_WIDE16 ? wide_fwd_nsplit(B, N, H, p.w1, p.w2, workspace_bytes)
                                              : 1;
         const size_t need = path == PATH_MFMA32   ? f32_mfma_fwd_part_bytes(B, N, H, D, ns)
                             : path == PATH_WIDE16 ? fwd_part_bytes(B, N, H, D, ns)

@@ -150,17 +150,29 @@ KpPlan plan_segments(int B, int N, int H, int w1, int w2, int upr, int most, siz
     return best;
 }
 
+inline size_t fwd_part_bytes(int B, int N, int H, int width, int nsplit) {
+    return nsplit > 1 ? (size_t)nsplit * B * H * (size_t)N * (width + 2) * sizeof(float) : 0;
+}
 // A forward launch in nsplit shares of the rounds of `upr` deltas: fp32 partial outputs in the workspace.  A round takes
-// about three tiles' time beside its sweep, prologue and epilogue about eight.  Fewer than four rounds are not shared: at
-// B3 H6 N777 D64 w 100/20 two shares take 66 us against 41 (a grid smaller still would gain: fp32 B1 H2 N128 D64 w 32/16
-// 28 us, 19 in three shares).  Against every cut: the best or within 2 % at eight of fifteen sizes, 5 - 25 % off at the
-// others, where a grid a little under a whole wave would take more shares.
-inline int plan_forward(int B, int N, int H, int width, int w1, int w2, int upr) {
+// about three tiles' time beside its sweep, prologue and epilogue about eight.  Against every cut: the best or within 2 % at eight of
+// fifteen sizes, 5 - 25 % off at the others, where a grid a little under a whole wave would take more shares.
+// Two or three rounds are shared only where all shares run at once, a workgroup per CU, and save more than the merging launch costs
+// (`least_saved` tiles of a sweep, by how long a kernel takes for one): fp32 B1 H2 N128 D64 w 32/16 26.3 -> 18.2 us, bf16
+// B1 H4 N512 w 64/20 D96 31.4 -> 20.9, D128 25.2 -> 18.8, D256 36.9 -> 30.9, D64 w 200/12 20.7 -> 17.5, but w 40/8 12.2 -> 14.4, w 63/17 13.6 -> 13.8; not all at once: B1 H8
+// N1024 D96 w 128/16 36.3 -> 57.4.  They stay one launch where the caller's workspace, `room`, has no place for them.
+inline int plan_forward(int B, int N, int H, int width, int w1, int w2, int upr, int least_saved, size_t room) {
     constexpr int ROWS = 32, MOST = 16;
     const int64_t rows = (int64_t)B * H * N, base = (int64_t)B * H * ((N + ROWS - 1) / ROWS);
     const int rounds = ((w2 < N - 1 ? w2 : N - 1) + upr) / upr;
-    if (rounds < 4 || base >= 3 * CUS) return 1;
-    const double tiles = ((w1 < N ? w1 : N) + ROWS) / (double)ROWS + 1, fill = window_fill(w1, N) * window_fill(w2, N);
+    const double tiles = ((w1 < N ? w1 : N) + ROWS) / (double)ROWS + 1;
+    if (rounds < 4) {
+        for (int ns = rounds; ns > 1; --ns)
+            if (base * ns <= CUS && (rounds - (rounds + ns - 1) / ns) * tiles >= least_saved)
+                return fwd_part_bytes(B, N, H, width, ns) <= room ? ns : 1;
+        return 1;
+    }
+    if (base >= 3 * CUS) return 1;
+    const double fill = window_fill(w1, N) * window_fill(w2, N);
     int best = 1;
     double least = 0;
     for (int ns = 1, last = 0; ns <= MOST && ns <= rounds; ++ns) {
@@ -179,9 +191,6 @@ inline int plan_forward(int B, int N, int H, int width, int w1, int w2, int upr)
     }
     return best;
 }
-inline size_t fwd_part_bytes(int B, int N, int H, int width, int nsplit) {
-    return nsplit > 1 ? (size_t)nsplit * B * H * (size_t)N * (width + 2) * sizeof(float) : 0;
-}
 
 // ---- launchers (each returns a sa2_status) ----------------------------------
 int launch_rowdot(const Tensor& out, const Tensor& dout, float* dsum, int B, int N, int H, int D,
@@ -194,7 +203,7 @@ bool mfma_supported(int B, int N, int H, int D, int w1, int w2, int dtype);
 bool mfma_bwd_supported(int B, int N, int H, int D, int w1, int w2, int dtype);
 bool mfma_layout_ok(const Problem& p, bool backward);
 int launch_mfma_fwd(const Problem& p, int dtype, hipStream_t st);
-int mfma_fwd_nsplit(int B, int N, int H, int D, int w1, int w2, bool force_prepass);
+int mfma_fwd_nsplit(int B, int N, int H, int D, int w1, int w2, bool force_prepass, size_t room);
 size_t mfma_fwd_part_bytes(int B, int N, int H, int D, int nsplit);
 int launch_mfma_bwd(const Problem& p, int dtype, hipStream_t st);
 size_t mfma_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2, size_t room);
@@ -205,7 +214,7 @@ bool f32_mfma_bwd_supported(int D, int w2, int dtype);
 bool f32_mfma_layout_ok(const Problem& p, int dtype, bool backward);
 size_t f32_mfma_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2, int dtype, size_t room);
 int launch_f32_mfma_fwd(const Problem& p, int dtype, hipStream_t st);
-int f32_mfma_fwd_nsplit(int B, int N, int H, int D, int w1, int w2, int dtype);
+int f32_mfma_fwd_nsplit(int B, int N, int H, int D, int w1, int w2, int dtype, size_t room);
 size_t f32_mfma_fwd_part_bytes(int B, int N, int H, int D, int nsplit);
 int launch_f32_mfma_bwd(const Problem& p, int dtype, hipStream_t st);
 // Its forward and K side with one wavefront per SIMD (sa2_split_fwd_lone.h, sa2_split_kv_lone.h).  `width`: of the kernel; `two_planes`:
@@ -220,7 +229,7 @@ int launch_split_kv_lone_fp32(const Problem& p, int width, bool two_planes, int 
 bool wide_supported(int D, int dtype);
 bool wide_bwd_supported(int D, int w2, int dtype);
 size_t wide_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2, size_t room);
-int wide_fwd_nsplit(int B, int N, int H, int w1, int w2);
+int wide_fwd_nsplit(int B, int N, int H, int w1, int w2, size_t room);
 int launch_wide_fwd(const Problem& p, int dtype, hipStream_t st);
 int launch_wide_bwd(const Problem& p, int dtype, hipStream_t st);
 // Partial outputs of a split forward, [nsplit][B*H*N] pairs (reference exponent M, sum L) and then

@@ -1114,13 +1114,13 @@ bool mfma_layout_ok(const Problem& p, bool backward) {
 }
 
 // Shares of a forward given workspace for their partial outputs: none where the pre-pass is to take the odd unit
-int mfma_fwd_nsplit(int B, int N, int H, int D, int w1, int w2, bool force_prepass) {
-    return force_prepass && w2 >= FW && w2 % FW == 0 ? 1 : plan_forward(B, N, H, mfma_width(D), w1, w2, FW);
+int mfma_fwd_nsplit(int B, int N, int H, int D, int w1, int w2, bool force_prepass, size_t room) {
+    return force_prepass && w2 >= FW && w2 % FW == 0 ? 1 : plan_forward(B, N, H, mfma_width(D), w1, w2, FW, D == 128 ? 5 : 8, room);
 }
 size_t mfma_fwd_part_bytes(int B, int N, int H, int D, int nsplit) { return fwd_part_bytes(B, N, H, mfma_width(D), nsplit); }
 
 int mfma_fwd_route(int B, int N, int H, int D, int w1, int w2, bool force_prepass) {
-    const int nsplit = mfma_fwd_nsplit(B, N, H, D, w1, w2, force_prepass);
+    const int nsplit = mfma_fwd_nsplit(B, N, H, D, w1, w2, force_prepass, ROOM_ANY);
     const int64_t total = (int64_t)((N + BQ - 1) / BQ) * B * H;
     const FwdRoute r = D == 128 ? fwd_route<128>(N, w1, w2, total, nsplit, force_prepass) : D == 64 ? fwd_route<64>(N, w1, w2, total, nsplit, force_prepass)
                                                                                                    : fwd_route<32>(N, w1, w2, total, nsplit, force_prepass);

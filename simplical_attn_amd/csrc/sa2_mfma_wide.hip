@@ -1462,7 +1462,7 @@ size_t wide_bwd_scratch_bytes(int B, int N, int H, int D, int w1, int w2, size_t
     return kp_bytes + (ns > 1 ? (size_t)2 * ns * B * H * (size_t)N * D * sizeof(float) : 0);
 }
 
-int wide_fwd_nsplit(int B, int N, int H, int w1, int w2) { return plan_forward(B, N, H, 256, w1, w2, WW); }
+int wide_fwd_nsplit(int B, int N, int H, int w1, int w2, size_t room) { return plan_forward(B, N, H, 256, w1, w2, WW, 0, room); }
 
 int launch_wide_fwd(const Problem& p, int dtype, hipStream_t st) {
     return dtype == SA2_F16 ? launch_wide_fwd_of<ElemF16>(p, st) : launch_wide_fwd_of<ElemBF16>(p, st);

@@ -66,9 +66,8 @@ struct SplitCfg {
     static constexpr int PLANE = 32 * RS;      // elements
     static constexpr int AS = D + 4;           // row stride of fp32 accumulators in LDS
     static constexpr size_t LDS_LIMIT = 160 * 1024;
-    // Forward: eight wavefronts (two per SIMD) where operands and accumulators fit 256 registers, else four.  (The kernel with two units
-    // per wavefront has eight units per round as well.)
-    static constexpr int FW = D <= 64 || (D == 96 && T::PLANES < 3) ? 8 : 4;
+    // Forward: eight wavefronts (two per SIMD) where operands and accumulators fit 256 registers, else four.
+    static constexpr int FW = D <= 64 ? 8 : 4;
     static constexpr int KV_TILE = NK * PLANE;             // a K or V tile
     static constexpr int KV_STAGE = 2 * KV_TILE;           // K tile, then V tile
     static constexpr size_t FWD_TILES = (size_t)2 * KV_STAGE * 2;
@@ -1140,6 +1139,29 @@ bool exact_products(const Problem& p, bool backward) {
 // Whether the kernels with one wavefront per SIMD are taken (sa2_split_fwd_lone.h, sa2_split_kv_lone.h, sa2_split_kp_lone.h)
 template <class T, int D, int MODE>
 constexpr bool lone() { return T::DTYPE == SA2_F32 ? MODE != PADDED_FINE && D <= 64 : D == 64 || D == 96; }
+// Units of a forward's round.  At 96 columns grids that are at once on the chip in rounds of four are shared so, by split_fwd_kernel: a round
+// is all of such a launch, and two units per wavefront take it longer.  Rounds of eight against rounds of four, us: fp16 D80 B2 H8 N33 w 65/15
+// 20.5 / 16.6, B1 H4 N128 w 16/16 20.9 / 19.7, B1 H2 N300 w 200/12 33.2 / 31.1, w 40/24 23.5 / 22.9, B1 H2 N128 w 128/100 30.0 / 38.7.  Where logits
+// have two planes (bf16) only for the shortest sequences: N33 16.9 / 15.0, B1 H1 N64 w 16/8 16.1 / 14.4, but B1 H4 N512 w 40/15 19.5 / 20.4.
+template <class T, int D, int MODE>
+int forward_round(int B, int N, int H, int w2) {
+    if constexpr (lone<T, D, MODE>() && D == 96) {
+        const int units = (w2 < N - 1 ? w2 : N - 1) + 1;
+        const bool few = T::PLANES == 1 ? units <= 16 && N <= 64 : units <= 20;
+        return few && units > 8 && (int64_t)B * H * ((N + BQ - 1) / BQ) * ((units + 3) / 4) <= CUS ? 4 : 8;
+    }
+    return SplitCfg<T, D>::FW;
+}
+// ... by the forward, at 32 columns only for more than ten units, at head_dim 16 (whose padded steps split_fwd_kernel
+// leaves out) only for many over wide windows.  fp32, time of split_fwd_kernel over the other one's, by w1/w2: head_dim 32: 20/8 0.96, 40/8
+// 0.96, 512/8 0.99, 48/9 1.01, 40/15 1.07, 100/31 1.10, 1000/128 1.21; head_dim 16: 20/8 0.84, 60/24 0.95, 100/31 0.97, 256/20 0.98, 512/32 1.01,
+// 1000/128 1.19.
+template <class T, int D, int MODE>
+bool lone_forward(const Problem& p) {
+    if constexpr (!lone<T, D, MODE>()) return false;
+    else if constexpr (D == 96) return p.nsplit <= 1 || forward_round<T, D, MODE>(p.B, p.N, p.H, p.w2) == 8;
+    else return D != 32 || (MODE == EXACT ? p.w2 >= 10 : p.w2 >= 31 && p.w1 >= 256);
+}
 // Deltas per segment: what the dQ accumulator in LDS holds, or fewer where the grid asks for it
 template <class T, int D, int MODE>
 KpPlan split_kp_plan(int B, int N, int H, int w1, int w2, size_t room) {
@@ -1156,11 +1178,12 @@ KpPlan split_kp_plan(int B, int N, int H, int w1, int w2, size_t room) {
 // ------------------------------------------------------------------ launchers ----
 template <class T, int D, int MODE>
 int launch_split_fwd(const Problem& p, hipStream_t st) {
-    if constexpr (lone<T, D, MODE>()) {
+    if (lone_forward<T, D, MODE>(p)) {
         const int rc = (T::DTYPE == SA2_F32 ? launch_split_fwd_lone_fp32 : T::DTYPE == SA2_F16 ? launch_split_fwd_lone_fp16 : launch_split_fwd_lone_bf16)(
             p, D, exact_products<T>(p, false), st);
         return rc != SA2_OK || p.nsplit <= 1 ? rc : launch_fwd_merge(p, D, T::DTYPE, st);
-    } else {
+    }
+    if constexpr (!lone<T, D, MODE>() || D == 32 || D == 96) {
         using C = SplitCfg<T, D>;
         const int nqb = (p.N + BQ - 1) / BQ;
         const int64_t total = (int64_t)nqb * p.B * p.H;
@@ -1172,7 +1195,8 @@ int launch_split_fwd(const Problem& p, hipStream_t st) {
         };
         auto go_split = [&](auto nq) {
             constexpr int NQ = decltype(nq)::value;
-            if (p.nsplit <= 1) return go(split_fwd_kernel<T, D, MODE, false, NQ>, total);
+            if constexpr (!(lone<T, D, MODE>() && D == 96))
+                if (p.nsplit <= 1) return go(split_fwd_kernel<T, D, MODE, false, NQ>, total);
             return go(split_fwd_kernel<T, D, MODE, true, NQ>, total * p.nsplit);
         };
         if (total * (p.nsplit > 1 ? p.nsplit : 1) > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
@@ -1183,6 +1207,7 @@ int launch_split_fwd(const Problem& p, hipStream_t st) {
         if (p.nsplit <= 1) return SA2_OK;
         return launch_fwd_merge(p, D, T::DTYPE, st);
     }
+    return SA2_ERR_UNSUPPORTED;
 }
 
 template <class T, int D, int MODE>
@@ -1335,10 +1360,13 @@ size_t f32_mfma_bwd_scratch_bytes(int B, int N, int H, int head_dim, int w1, int
     return bytes;
 }
 
-int f32_mfma_fwd_nsplit(int B, int N, int H, int head_dim, int w1, int w2, int dtype) {
-    return for_split_width(head_dim, dtype, [&](auto m, auto width, auto) {
+int f32_mfma_fwd_nsplit(int B, int N, int H, int head_dim, int w1, int w2, int dtype, size_t room) {
+    return for_split_width(head_dim, dtype, [&](auto m, auto width, auto mode) {
         constexpr int D = decltype(width)::value;
-        return plan_forward(B, N, H, D, w1, w2, SplitCfg<decltype(m), D>::FW);
+        const int round = forward_round<decltype(m), D, decltype(mode)::value>(B, N, H, w2);
+        // (fp32 up to 64 columns: two short rounds stay one launch.  Up to 3 us would be gained, but at these sizes a forward with a workspace
+        // and one without are compared bit by bit.)
+        return plan_forward(B, N, H, D, w1, w2, round, dtype == SA2_F32 && D <= 64 ? 4 : 0, room);
     });
 }
 size_t f32_mfma_fwd_part_bytes(int B, int N, int H, int head_dim, int nsplit) { return fwd_part_bytes(B, N, H, split_width(head_dim), nsplit); }

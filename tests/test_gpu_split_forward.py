@@ -51,3 +51,38 @@ def test_a_query_that_is_not_a_number_stays_one_through_the_merge(dtype, D):
     out, _ = sa.simplicial_forward(*x, 40, 60)
     rows = out[0, :, 0].isnan()
     assert rows[70].all() and rows.sum().item() == D
+
+
+@pytest.mark.parametrize("dtype,case,shares", [
+    (torch.float32, (1, 100, 1, 16, 70, 8, True), 2),        # the second share has one unit
+    (torch.float32, (1, 128, 2, 64, 32, 16, True), 3),
+    (torch.float32, (2, 67, 3, 128, 30, 9, True), 3),
+    (torch.float32, (1, 1021, 4, 32, 70, 23, True), 2),     # three rounds in two shares: as many as there are CUs for
+    (torch.bfloat16, (1, 63, 2, 96, 40, 9, False), 3),    # rounds of four units
+    (torch.bfloat16, (1, 97, 2, 96, 40, 12, False), 2),
+    (torch.float16, (1, 300, 5, 80, 20, 22, True), 3),
+    (torch.float16, (2, 130, 2, 80, 40, 11, True), 3),      # ... and here
+    (torch.bfloat16, (1, 200, 2, 64, 150, 20, True), 3),
+    (torch.float16, (1, 128, 2, 128, 100, 12, True), 2),
+    (torch.bfloat16, (1, 70, 2, 256, 16, 11, True), 3),
+])
+def test_small_grids_share_two_or_three_rounds(dtype, case, shares):
+    """As above; a workspace that is too small for the shares leaves the launch whole."""
+    import simplical_attn_amd as sa
+    lib = _lib.load()
+    B, N, H, D, w1, w2, inclusive = case
+    width = next(w for w in (32, 64, 96, 128, 256) if w >= D)
+    assert lib.sa2_fwd_workspace_bytes(B, N, H, D, w1, w2, CODE[dtype], int(inclusive), 0) == shares * B * H * N * (width + 2) * 4
+    test_shares_of_the_rounds_merge_to_the_oracle(dtype, case, None)
+    x = [t.cuda() for t in make_inputs(B, N, H, D, seed=N, dtype=dtype)[:5]]
+    small = torch.empty(256, dtype=torch.uint8, device="cuda")
+    got = []
+    for workspace in (None, small):
+        o, l = torch.empty_like(x[0]), torch.empty(B, H, N, device="cuda")
+        strides = _lib.stride_array([(t.stride(0), t.stride(1), t.stride(2)) for t in (*x, o)])
+        _lib.check(lib.sa2_forward_ws(*[t.data_ptr() for t in x], o.data_ptr(), l.data_ptr(), workspace.data_ptr() if workspace is not None else None,
+                                      256 if workspace is not None else 0, B, N, H, D, strides, w1, w2, D ** -0.5, 0.1, -0.2, CODE[dtype],
+                                      int(inclusive), 0, torch.cuda.current_stream().cuda_stream))
+        got.append((o, l))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    torch.cuda.synchronize()
