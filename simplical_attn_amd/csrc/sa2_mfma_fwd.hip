@@ -70,6 +70,7 @@ struct Cfg {
     static constexpr bool NOFOLD = D <= 64;
     using Tile = QuadTile<D>;                                // K and V tiles in LDS
     static constexpr int NGROUP = Tile::NGROUP;
+    static constexpr int LW = 4;                            // wavefronts of a pre-pass workgroup
     static constexpr int SS = D + 8;                        // slab row stride (bf16)
     // (room behind a tile: two slabs lie over a free stage at the end of a round)
     static constexpr int TILE_BYTES = Tile::BYTES > 2 * BQ * SS ? Tile::BYTES : 2 * BQ * SS;
@@ -97,8 +98,11 @@ struct Cfg {
 // its own for the second pass cost every call 4 us at small sizes and 7.6 us at B1 H16 N8192 for
 // workgroups that found nothing to do.)
 // MODE_LEFT: the pre-pass for window sizes that leave one unit over after the rounds of
-// eight (w2 + 1 = 8n + 1).  A workgroup takes eight consecutive query blocks, one per
+// eight (w2 + 1 = 8n + 1).  A workgroup takes four consecutive query blocks, one per
 // wavefront, and computes the unit delta = w2 of each while sharing one sweep of K/V tiles.
+// Four, not eight: the sweep that covers all of their windows is four tiles shorter and the workgroups are twice as many.  Whole
+// forward, bf16, eight / four, us: D64 B2 H8 N2048 w 512/32 172.9 / 163.9 (the pre-pass 28 / 21), B1 H16 N1600 w 256/16 66.9 / 59.4, B6 H8 N5000
+// w 40/8 208 / 187, D128 125.0 / 114.3 and 483 / 461, B1 H16 N8192 w 512/32 1191 / 1187.
 // Nothing is merged across wavefronts: every query's partial result goes to `out` as
 // R * (v2 + bias) / l in bf16 and to `lse` as m + log2(l); the fast kernel, launched next with
 // left = 1, starts its accumulator from that pair and handles delta < w2 in full rounds.
@@ -138,8 +142,8 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
         share = pid % p.nsplit;
         pid /= p.nsplit;
     }
-    // (in the pre-pass nqb counts groups of eight query blocks)
-    const int bh = pid / nqb, qb = LEFT ? (pid - bh * nqb) * FW + wave : pid - bh * nqb;
+    // (in the pre-pass nqb counts groups of LW query blocks)
+    const int bh = pid / nqb, qb = LEFT ? (pid - bh * nqb) * C::LW + wave : pid - bh * nqb;
     const int b = bh / p.H, h = bh - b * p.H;
     const int N = p.N, w1 = p.w1, w2 = p.w2;
     const int i0 = qb * BQ;                      // per wavefront in the pre-pass
@@ -156,7 +160,7 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
 
     constexpr int TJ = C::TK;                    // keys per tile in this kernel
     const int jt_lo = (i0_wg - w1 > 0 ? i0_wg - w1 : 0) / TJ;
-    const int jt_hi = LEFT ? (i0_wg + FW * BQ - 1 < N - 1 ? i0_wg + FW * BQ - 1 : N - 1) / TJ : i_last / TJ;
+    const int jt_hi = LEFT ? (i0_wg + C::LW * BQ - 1 < N - 1 ? i0_wg + C::LW * BQ - 1 : N - 1) / TJ : i_last / TJ;
     const int nt = jt_hi - jt_lo + 1;
     // delta = 0 .. n_units-1; the fast kernel leaves delta = w2 to the pre-pass where that ran
     const bool has_left = left && i_last >= w2;
@@ -183,16 +187,21 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
     // Wavefront w fills group w of the K tile and of the V tile (the first NGROUP wavefronts
     // when D = 64).  Tiles are requested strictly in sweep order into consecutive ring stages.
     const bool t_owner = wave < C::NGROUP;
+    constexpr int NW = LEFT ? C::LW : FW, NREQ = C::NGROUP > NW ? C::NGROUP / NW : 1;       // groups w, w + NW, .. of wavefront w
     const int t_row = wave * C::Tile::RPW + C::Tile::dma_row(lane), t_col = C::Tile::dma_chunk(lane);
     const bool t_inside = t_col * 8 < p.D;                      // (used when PAD)
-    const uint32_t k_off = ((uint32_t)t_row * (uint32_t)p.k1.sn + t_col * 8) * 2u;
-    const uint32_t v_off = ((uint32_t)t_row * (uint32_t)p.v1.sn + t_col * 8) * 2u;
     // the same for the tile that holds the end of the sequence: rows past it are clamped to the
     // last one (they are masked later)
     const int jt_end = (N - 1) / TJ;
-    const int t_row_c = t_row < N - 1 - jt_end * TJ ? t_row : N - 1 - jt_end * TJ;
-    const uint32_t k_off_c = ((uint32_t)t_row_c * (uint32_t)p.k1.sn + t_col * 8) * 2u;
-    const uint32_t v_off_c = ((uint32_t)t_row_c * (uint32_t)p.v1.sn + t_col * 8) * 2u;
+    uint32_t k_off[NREQ], v_off[NREQ], k_off_c[NREQ], v_off_c[NREQ];
+#pragma unroll
+    for (int n = 0; n < NREQ; ++n) {
+        const int row = t_row + n * NW * C::Tile::RPW, row_c = row < N - 1 - jt_end * TJ ? row : N - 1 - jt_end * TJ;
+        k_off[n] = ((uint32_t)row * (uint32_t)p.k1.sn + t_col * 8) * 2u;
+        v_off[n] = ((uint32_t)row * (uint32_t)p.v1.sn + t_col * 8) * 2u;
+        k_off_c[n] = ((uint32_t)row_c * (uint32_t)p.k1.sn + t_col * 8) * 2u;
+        v_off_c[n] = ((uint32_t)row_c * (uint32_t)p.v1.sn + t_col * 8) * 2u;
+    }
     typedef __attribute__((address_space(3))) void* lds_ptr;
     typedef const __attribute__((address_space(1))) void* glb_ptr;
     int dma_tile = 0, dma_stage = 0, dma_count = 0;             // next tile (from jt_lo), its stage, tiles requested
@@ -200,19 +209,22 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
     // into the middle of a step's arithmetic)
     auto dma_next = [&]() {
         const int j0 = (jt_lo + dma_tile) * TJ;
-        if (C::NGROUP >= FW || t_owner) {
+        if (C::NGROUP >= NW || t_owner) {
             const bool at_end = jt_lo + dma_tile == jt_end;
-            const uint32_t ko = at_end ? k_off_c : k_off, vo = at_end ? v_off_c : v_off;
             const char* kb = (const char*)(k1p + (int64_t)j0 * p.k1.sn);
             const char* vb = (const char*)(v1p + (int64_t)j0 * p.v1.sn);
             unsigned char* dst = smem_raw + (size_t)dma_stage * (C::STAGE * 2) + wave * C::Tile::GROUP;
-            const char *ks = kb + ko, *vs = vb + vo;
-            if constexpr (PAD) {
-                ks = t_inside ? ks : (const char*)zero_chunk;
-                vs = t_inside ? vs : (const char*)zero_chunk;
+#pragma unroll
+            for (int n = 0; n < NREQ; ++n) {
+                const uint32_t ko = at_end ? k_off_c[n] : k_off[n], vo = at_end ? v_off_c[n] : v_off[n];
+                const char *ks = kb + ko, *vs = vb + vo;
+                if constexpr (PAD) {
+                    ks = t_inside ? ks : (const char*)zero_chunk;
+                    vs = t_inside ? vs : (const char*)zero_chunk;
+                }
+                __builtin_amdgcn_global_load_lds((glb_ptr)ks, (lds_ptr)(dst + n * NW * C::Tile::GROUP), 16, 0, 0);
+                __builtin_amdgcn_global_load_lds((glb_ptr)vs, (lds_ptr)(dst + n * NW * C::Tile::GROUP + C::TILE_BYTES), 16, 0, 0);
             }
-            __builtin_amdgcn_global_load_lds((glb_ptr)ks, (lds_ptr)dst, 16, 0, 0);
-            __builtin_amdgcn_global_load_lds((glb_ptr)vs, (lds_ptr)(dst + C::TILE_BYTES), 16, 0, 0);
         }
         dma_tile = dma_tile + 1 == nt ? 0 : dma_tile + 1;
         dma_stage = (dma_stage + 1) & (C::NSTAGE - 1);
@@ -326,7 +338,7 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
         if (requested) dma_next();
     };
     auto advance = [&]() {
-        if (requested) asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (requested) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * NREQ) : "memory");
         else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
         buf = (buf + 1) & (C::NSTAGE - 1);
         ++g;
@@ -606,7 +618,7 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
                     lds_settle(vh);
                     // The barrier stands in front of the value MFMAs: they only read registers.
                     vt_prev = ks_addr + (uint32_t)C::TILE_BYTES;
-                    if constexpr (DMA) asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                    if constexpr (DMA) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * NREQ) : "memory");
                     else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
                     buf = (buf + 1) & (C::NSTAGE - 1);
                     ++g;
@@ -1047,10 +1059,10 @@ int launch_fwd_kernels(const Problem& p, int nqb, int total, hipStream_t st) {
     const FwdRoute route = fwd_route<D>(p.N, p.w1, p.w2, total, p.nsplit, p.force_prepass);
     const int left = route.left;
     if (left) {
-        const int ngrp = (nqb + FW - 1) / FW;
+        const int ngrp = (nqb + C::LW - 1) / C::LW;
         const int total_left = ngrp * (total / nqb);
         if (!allow_full_lds((const void*)mfma_fwd_kernel<E, D, MODE_LEFT, false, PAD, false>)) return SA2_ERR_LAUNCH_FAILED;
-        hipLaunchKernelGGL((mfma_fwd_kernel<E, D, MODE_LEFT, false, PAD, false>), dim3((unsigned)total_left), dim3(FT), C::STAGE_BYTES, st,
+        hipLaunchKernelGGL((mfma_fwd_kernel<E, D, MODE_LEFT, false, PAD, false>), dim3((unsigned)total_left), dim3(C::LW * 64), C::STAGE_BYTES, st,
                            (FwdArgs{p, ngrp, total_left, 0}));
         if (hipGetLastError() != hipSuccess) return SA2_ERR_LAUNCH_FAILED;
     }
