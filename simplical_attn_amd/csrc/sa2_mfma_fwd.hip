@@ -102,7 +102,7 @@ struct Cfg {
 // wavefront, and computes the unit delta = w2 of each while sharing one sweep of K/V tiles.
 // Four, not eight: the sweep that covers all of their windows is four tiles shorter and the workgroups are twice as many.  Whole
 // forward, bf16, eight / four, us: D64 B2 H8 N2048 w 512/32 172.9 / 163.9 (the pre-pass 28 / 21), B1 H16 N1600 w 256/16 66.9 / 59.4, B6 H8 N5000
-// w 40/8 208 / 187, D128 125.0 / 114.3 and 483 / 461, B1 H16 N8192 w 512/32 1191 / 1187.
+// w 40/8 208 / 187, D128 125.6 / 115.5 and 484 / 467, B1 H16 N8192 w 512/32 1206 / 1198.
 // Nothing is merged across wavefronts: every query's partial result goes to `out` as
 // R * (v2 + bias) / l in bf16 and to `lse` as m + log2(l); the fast kernel, launched next with
 // left = 1, starts its accumulator from that pair and handles delta < w2 in full rounds.
@@ -187,21 +187,22 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
     // Wavefront w fills group w of the K tile and of the V tile (the first NGROUP wavefronts
     // when D = 64).  Tiles are requested strictly in sweep order into consecutive ring stages.
     const bool t_owner = wave < C::NGROUP;
-    constexpr int NW = LEFT ? C::LW : FW, NREQ = C::NGROUP > NW ? C::NGROUP / NW : 1;       // groups w, w + NW, .. of wavefront w
+    constexpr int NW = LEFT ? C::LW : FW, NREQ = C::NGROUP > NW ? 2 : 1;       // groups of wavefront w: w, w + NW
+    static_assert(C::NGROUP <= NREQ * NW, "");
     const int t_row = wave * C::Tile::RPW + C::Tile::dma_row(lane), t_col = C::Tile::dma_chunk(lane);
     const bool t_inside = t_col * 8 < p.D;                      // (used when PAD)
+    const uint32_t k_off = ((uint32_t)t_row * (uint32_t)p.k1.sn + t_col * 8) * 2u;
+    const uint32_t v_off = ((uint32_t)t_row * (uint32_t)p.v1.sn + t_col * 8) * 2u;
     // the same for the tile that holds the end of the sequence: rows past it are clamped to the
     // last one (they are masked later)
     const int jt_end = (N - 1) / TJ;
-    uint32_t k_off[NREQ], v_off[NREQ], k_off_c[NREQ], v_off_c[NREQ];
-#pragma unroll
-    for (int n = 0; n < NREQ; ++n) {
-        const int row = t_row + n * NW * C::Tile::RPW, row_c = row < N - 1 - jt_end * TJ ? row : N - 1 - jt_end * TJ;
-        k_off[n] = ((uint32_t)row * (uint32_t)p.k1.sn + t_col * 8) * 2u;
-        v_off[n] = ((uint32_t)row * (uint32_t)p.v1.sn + t_col * 8) * 2u;
-        k_off_c[n] = ((uint32_t)row_c * (uint32_t)p.k1.sn + t_col * 8) * 2u;
-        v_off_c[n] = ((uint32_t)row_c * (uint32_t)p.v1.sn + t_col * 8) * 2u;
-    }
+    const int t_row_c = t_row < N - 1 - jt_end * TJ ? t_row : N - 1 - jt_end * TJ;
+    const uint32_t k_off_c = ((uint32_t)t_row_c * (uint32_t)p.k1.sn + t_col * 8) * 2u;
+    const uint32_t v_off_c = ((uint32_t)t_row_c * (uint32_t)p.v1.sn + t_col * 8) * 2u;
+    // the wavefront's second group (NREQ == 2)
+    const int t_row2 = t_row + NW * C::Tile::RPW, t_row2_c = t_row2 < N - 1 - jt_end * TJ ? t_row2 : N - 1 - jt_end * TJ;
+    const uint32_t k_off2 = ((uint32_t)t_row2 * (uint32_t)p.k1.sn + t_col * 8) * 2u, k_off2_c = ((uint32_t)t_row2_c * (uint32_t)p.k1.sn + t_col * 8) * 2u;
+    const uint32_t v_off2 = ((uint32_t)t_row2 * (uint32_t)p.v1.sn + t_col * 8) * 2u, v_off2_c = ((uint32_t)t_row2_c * (uint32_t)p.v1.sn + t_col * 8) * 2u;
     typedef __attribute__((address_space(3))) void* lds_ptr;
     typedef const __attribute__((address_space(1))) void* glb_ptr;
     int dma_tile = 0, dma_stage = 0, dma_count = 0;             // next tile (from jt_lo), its stage, tiles requested
@@ -211,19 +212,21 @@ __device__ __forceinline__ bool fwd_block(const Problem& p, int nqb, int total, 
         const int j0 = (jt_lo + dma_tile) * TJ;
         if (C::NGROUP >= NW || t_owner) {
             const bool at_end = jt_lo + dma_tile == jt_end;
+            const uint32_t ko = at_end ? k_off_c : k_off, vo = at_end ? v_off_c : v_off;
             const char* kb = (const char*)(k1p + (int64_t)j0 * p.k1.sn);
             const char* vb = (const char*)(v1p + (int64_t)j0 * p.v1.sn);
             unsigned char* dst = smem_raw + (size_t)dma_stage * (C::STAGE * 2) + wave * C::Tile::GROUP;
-#pragma unroll
-            for (int n = 0; n < NREQ; ++n) {
-                const uint32_t ko = at_end ? k_off_c[n] : k_off[n], vo = at_end ? v_off_c[n] : v_off[n];
-                const char *ks = kb + ko, *vs = vb + vo;
+            auto request = [&](const char* ks, const char* vs, unsigned char* to) __attribute__((always_inline)) {
                 if constexpr (PAD) {
                     ks = t_inside ? ks : (const char*)zero_chunk;
                     vs = t_inside ? vs : (const char*)zero_chunk;
                 }
-                __builtin_amdgcn_global_load_lds((glb_ptr)ks, (lds_ptr)(dst + n * NW * C::Tile::GROUP), 16, 0, 0);
-                __builtin_amdgcn_global_load_lds((glb_ptr)vs, (lds_ptr)(dst + n * NW * C::Tile::GROUP + C::TILE_BYTES), 16, 0, 0);
+                __builtin_amdgcn_global_load_lds((glb_ptr)ks, (lds_ptr)to, 16, 0, 0);
+                __builtin_amdgcn_global_load_lds((glb_ptr)vs, (lds_ptr)(to + C::TILE_BYTES), 16, 0, 0);
+            };
+            request(kb + ko, vb + vo, dst);
+            if constexpr (NREQ > 1) {
+                request(kb + (at_end ? k_off2_c : k_off2), vb + (at_end ? v_off2_c : v_off2), dst + NW * C::Tile::GROUP);
             }
         }
         dma_tile = dma_tile + 1 == nt ? 0 : dma_tile + 1;
