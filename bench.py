@@ -364,12 +364,12 @@ def main():
     wl = args.workload
     # launches of each group at this workload: pre-passes (a single unit left over after the rounds), main kernels, sums.
     # Beside them a backward launches the row-term kernel and, in fp32, the one that looks at its verdicts.
-    # (The forward of head_dim 128 has one for the first queries of every head.)
-    launches = {"c4": (3, 1, 3), "c2": (2, 2, 3), "c5": (3, 1, 2), "c1": (1, 2, 2), "c2f32": (1, 2, 2)}[wl]
+    # (The forward of head_dim 128 has one for the first queries of every head; small grids one that merges their shares.)
+    launches = {"c4": (3, 1, 3), "c2": (2, 2, 3), "c5": (3, 1, 2), "c1": (2, 2, 2), "c2f32": (1, 2, 2)}[wl]
     if fp32:
-        labels = ("split_fwd_kernel<fp32, %d> (six v_mfma_f32_32x32x16_bf16 per product)" % D, launches[0],
-                  "split_kv_kernel<fp32, %d> + sum (dK, dV)" % D, launches[1],
-                  "split_kp_kernel<fp32, %d> + sum (dQ, dK', dV')" % D, launches[2])
+        labels = ("split_fwd_lone_kernel<fp32, %d>%s (six v_mfma_f32_32x32x16_bf16 per product)" % (D, " + merge" if launches[0] > 1 else ""), launches[0],
+                  "split_kv_lone_kernel<fp32, %d> + sum (dK, dV)" % D, launches[1],
+                  "split_kp_lone_kernel<fp32, %d> + sum (dQ, dK', dV')" % D, launches[2])
     else:
         labels = ("mfma_fwd_lone_kernel<%d> (pre-pass%s + main)" % (D, " + first queries" if launches[0] > 2 else ""), launches[0],
                   "mfma_bwd_kv_kernel<%d>%s (dK, dV)" % (D, " + sum" if launches[1] > 1 else ""), launches[1],

@@ -338,9 +338,20 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
         s[u][e + 1] = y;
         if constexpr (i > 0) round_p(UN, LONE_C(i - 1));
     };
-    // dS from the unrounded weights: nothing but dS itself is rounded to 16 bits.  (From the rounded ones, as the two-wavefront kernel
-    // forms it, whose weights cross LDS in 16 bits: two instructions a pair more, B2 H8 N2048 D64 w 512/32 881 against 858 us a step with both
-    // backward kernels, B1 H16 N8192 D128 w 512/32 6203 against 6125, and errors of dQ, dK and dK' against fp32 4 - 9 % larger in the 2-norm.)
+    // dS from the unrounded weights but for a sweep's first tile: nothing but dS itself is rounded to 16 bits.  (From the rounded ones, as
+    // the two-wavefront kernel forms it, whose weights cross LDS in 16 bits, it is two instructions a pair more and the 2-norm errors of dQ
+    // and dK' against fp32 are 4 - 9 % larger.)  The first tile's weights are rounded before they meet dP: it holds all keys of the first queries,
+    // which have few weights, all large, so that single gradients there follow the rounding of each, and a gradient does not depend on which of
+    // the two kernels a problem is given to (up to 0.5 of its root mean square elsewhere with unrounded ones, B1 H8 N32768 D128 w 1024/64).
+    auto first_tile = [&](auto UN) __attribute__((always_inline)) {
+        constexpr int u = decltype(UN)::value;
+        static_for<8>([&](auto X) __attribute__((always_inline)) {
+            constexpr int e = 2 * decltype(X)::value;
+            const uint32_t w = pack2<E>(s[u][e], s[u][e + 1]);
+            s[u][e] = E::lo(w);
+            s[u][e + 1] = E::hi(w);
+        });
+    };
     auto ds_item = [&](auto UN, auto I) __attribute__((always_inline)) {
         constexpr int u = decltype(UN)::value, i = decltype(I)::value, ks = i / 4, t = i % 4, e = 2 * i;
         if constexpr (i == 0) round_p(UN, LONE_C(7));
@@ -410,6 +421,7 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
             constexpr int DSV[17] = {0, 0, 0, 2, 4, 5, 6, 8, 10, 10, 11, 12, 14, 15, 16, 16, 16};
             constexpr int DSW[17] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 1, 2, 3, 4};
             items(LONE_C(EXPS[i]), LONE_C(EXPS[i + 1]), exp_item);
+            if constexpr (!CC && i == 2) first_tile(LONE_C(0));           // (all weights are formed, none is used yet)
             items(LONE_C(PW[i]), LONE_C(PW[i + 1]), p_word);
             items(LONE_C(DSV[i]), LONE_C(DSV[i + 1]), ds_value);
             items(LONE_C(DSW[i]), LONE_C(DSW[i + 1]), ds_word);
@@ -446,6 +458,7 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
             if constexpr (i >= 2) read_column(LONE_C(i - 2), sa);                   // (the MFMA that read its register is past)
             __builtin_amdgcn_sched_barrier(0);
         });
+        if constexpr (!CC) first_tile(LONE_C(0));
         static_for<NE>([&](auto I) __attribute__((always_inline)) {
             a_mfma(LONE_C(U - 1), I);
             if constexpr (decltype(I)::value < 2) read_column(LONE_C(NE - 2 + decltype(I)::value), sa);
@@ -463,6 +476,7 @@ void mfma_bwd_kp_lone_kernel(Problem p, int nkb, int total, float* __restrict__ 
             if constexpr (i == NE - 2) static_for<C::NREQ>([&](auto X) __attribute__((always_inline)) { request_part(LONE_C(C::NREQ + decltype(X)::value), sc); });
             __builtin_amdgcn_sched_barrier(0);
         });
+        if constexpr (!CC) first_tile(LONE_C(U - 1));
         stays(s[U - 1]);
     };
     auto pair_last = [&]() __attribute__((always_inline)) {                         // C(t-1, 1) alone

@@ -13,8 +13,8 @@
 // stand between the MFMAs of A(t+1) and C(t), operand reads eight MFMAs ahead of their use.
 // The arrangement before it (two wavefronts per SIMD, one with S, P and dV, one with dP, dS and dK, P handed over in LDS, a
 // barrier per unit) ran matrix pipe, vector ALU and LDS one after the other, 2500 cycles per unit of 1024 MFMA cycles; here
-// it is 1700 to 1800.  With the row-term kernel, us: B2 H8 N2048 D64 w 512/32 458 -> 312, B1 H16 N8192 D128 w 512/32
-// 2715 -> 2280; at D128 the board's power is the next limit.
+// it is 1700 to 1800.  With the row-term kernel, us: B2 H8 N2048 D64 w 512/32 458 -> 323, B1 H16 N8192 D128 w 512/32
+// 2715 -> 2300; at D128 the board's power is the next limit.
 //
 // Small grids (fewer workgroups than the chip holds) split a key block's stream of units over up to sixteen workgroups
 // (shares of whole units, at least four each); each writes its fp32 partial dK and dV to the workspace and bwd_sum_kernel
@@ -349,11 +349,13 @@ void mfma_bwd_kv_kernel(Problem p, int njb, int total, int nsplit, float* __rest
         s[x][e + 1] = fast_exp2(s[x][e + 1]);
         if constexpr (i > 0) round_p(XP, std::integral_constant<int, i - 1>{});
     };
-    // (from the unrounded weights; see the K'-side kernel, sa2_mfma_bwd_kp_lone.h)
+    // (from the rounded weights, for the first queries: see the K'-side kernel, sa2_mfma_bwd_kp_lone.h.  Their units, the first of a stream,
+    // go through the same code as all others; the unrounded ones would be two instructions a pair less, 323 -> 312 us at D64, and dK 4 % closer.)
     auto ds_item = [&](auto XP, auto I) __attribute__((always_inline)) {
         constexpr int x = decltype(XP)::value, i = decltype(I)::value, ks = i / 4, t = i % 4, e = 2 * i;
         if constexpr (i == 0) round_p(XP, std::integral_constant<int, 7>{});
-        dw[x][ks][t] = pack2<E>(s[x][e] * dp[x][e], s[x][e + 1] * dp[x][e + 1]);
+        const uint32_t pp = pw[x][ks][t];
+        dw[x][ks][t] = pack2<E>(E::lo(pp) * dp[x][e], E::hi(pp) * dp[x][e + 1]);
     };
     auto unit_barrier = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
     // One K block per unit.  A(t), under the forming of unit t+2; then C(t-1), whose four groups of MFMAs (dV^T and dK^T, each
