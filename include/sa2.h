@@ -97,6 +97,7 @@ int sa2_forward(const void* q, const void* k1, const void* k2, const void* v1, c
  * heads, wide K' windows) the rounds of a block are then shared by several workgroups, whose partial outputs go
  * through the workspace; elsewhere it is not touched.  workspace: sa2_fwd_workspace_bytes(...) bytes, 256-byte
  * aligned, contents on entry ignored; NULL: as sa2_forward.  sa2_fwd_workspace_bytes returns 0 where none is used.
+ * Fewer bytes: SA2_ERR_WORKSPACE_TOO_SMALL, or, where no more than three rounds would be shared, as NULL.
  */
 int sa2_forward_ws(const void* q, const void* k1, const void* k2, const void* v1, const void* v2,
                    void* out, float* lse, void* workspace, size_t workspace_bytes,

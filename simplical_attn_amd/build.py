@@ -43,7 +43,7 @@ HAND_PLACED = {"sa2_mfma_bwd_kv_bf16.hip": _KV, "sa2_mfma_bwd_kv_fp16.hip": _KV,
                "sa2_mfma_bwd_kp_lone_bf16.hip": _KP, "sa2_mfma_bwd_kp_lone_fp16.hip": _KP,
                "sa2_mfma_fwd_lone_bf16.hip": _FWD, "sa2_mfma_fwd_lone_fp16.hip": _FWD,
                "sa2_split_fwd_lone_bf16.hip": _SFWD, "sa2_split_fwd_lone_fp16.hip": (_SFWD[0], _SFWD[2]),
-               "sa2_split_fwd_lone_fp32.hip": (_SFWD[0], ("split_fwd_lone_kernel.*Li32E", 96)),
+               "sa2_split_fwd_lone_fp32.hip": _SFWD[:1],
                "sa2_split_kp_lone_bf16.hip": _SKP, "sa2_split_kp_lone_fp16.hip": _SKP, "sa2_split_kp_lone_fp32.hip": _SKP,
                "sa2_split_kv_lone_bf16.hip": _SKV, "sa2_split_kv_lone_fp32.hip": _SKV,
                "sa2_split_kv_lone_fp16.hip": (("split_kv_lone_kernel.*Li64E", 192), ("split_kv_lone_kernel.*Li96E", 256))}

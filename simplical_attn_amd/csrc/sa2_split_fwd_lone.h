@@ -11,7 +11,7 @@
 //
 // What bounds it: the instructions beside the MFMAs (fp32 head_dim 64: 98 MFMAs, 520 others in a tile's 4500 cycles; bf16 at 96 columns 60 and
 // 380).  Forward, us, eight wavefronts of one unit / this: bf16 B1 H8 N2048 D96 w 255/31 240 / 158 (four wavefronts 364), fp32 B2 H8 N2048 D64
-// w 512/32 812 / 775, B1 H16 N2048 D32 254 / 230, B1 H2 N128 D64 w 32/16 (eight workgroups, not shared) 28.2 / 25.7.
+// w 512/32 812 / 775, B1 H2 N128 D64 w 32/16 (eight workgroups, not shared) 28.2 / 25.7.
 //
 // The reference point m of a row is the largest logit of the wavefront's first two units in the queries' own tile, which holds a key of every
 // row.  The largest of each further tile's logits is looked at before their exponentials: where one lies more than 64 octaves above m

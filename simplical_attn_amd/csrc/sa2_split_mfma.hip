@@ -1152,15 +1152,13 @@ int forward_round(int B, int N, int H, int w2) {
     }
     return SplitCfg<T, D>::FW;
 }
-// ... by the forward, at 32 columns only for more than ten units, at head_dim 16 (whose padded steps split_fwd_kernel
-// leaves out) only for many over wide windows.  fp32, time of split_fwd_kernel over the other one's, by w1/w2: head_dim 32: 20/8 0.96, 40/8
-// 0.96, 512/8 0.99, 48/9 1.01, 40/15 1.07, 100/31 1.10, 1000/128 1.21; head_dim 16: 20/8 0.84, 60/24 0.95, 100/31 0.97, 256/20 0.98, 512/32 1.01,
-// 1000/128 1.19.
+// ... by the forward: at 32 columns not.  (Two units of a wavefront share an accumulator, whose longer chain of sums shows there: 1 - 4 % more error
+// in an fp32 output at head_dim 32 - 0.99 to 1.0 at 64 - for 5 - 10 % less time at most sizes, and 5 - 19 % more with few deltas or at head_dim 16.)
 template <class T, int D, int MODE>
 bool lone_forward(const Problem& p) {
-    if constexpr (!lone<T, D, MODE>()) return false;
+    if constexpr (!lone<T, D, MODE>() || D == 32) return false;
     else if constexpr (D == 96) return p.nsplit <= 1 || forward_round<T, D, MODE>(p.B, p.N, p.H, p.w2) == 8;
-    else return D != 32 || (MODE == EXACT ? p.w2 >= 10 : p.w2 >= 31 && p.w1 >= 256);
+    else return true;
 }
 // Deltas per segment: what the dQ accumulator in LDS holds, or fewer where the grid asks for it
 template <class T, int D, int MODE>
