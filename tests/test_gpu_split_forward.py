@@ -4,6 +4,7 @@ computes the same problem in one workgroup per query block."""
 import pytest
 import torch
 
+from oracle import simplicial_oracle as orc
 from simplical_attn_amd import _lib
 from tests.util import assert_close_rel, make_inputs, oracle_all
 
@@ -86,3 +87,16 @@ def test_small_grids_share_two_or_three_rounds(dtype, case, shares):
         got.append((o, l))
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 64), (torch.bfloat16, 96), (torch.float16, 48), (torch.float32, 128)])
+@pytest.mark.parametrize("w2", [0, 40])
+def test_lse_of_small_logits(dtype, D, w2):
+    """Queries with one key each (the first ones: one K' row too) and logits of 1e-3: LSE is the logit plus the logarithm of the K' rows,
+    to the roundings of both (2^-24 of each; the 1e-8 of the sum is lost beside 1)."""
+    import simplical_attn_amd as sa
+    host = make_inputs(1, 200, 4, D, seed=D, dtype=dtype)
+    x = [t.cuda() for t in host[:5]]
+    lse = sa.simplicial_forward(*x, 0, w2, 1e-4)[1]
+    want = orc.forward_windowed(*[t.double() for t in host[:5]], 0, w2, 1e-4)[1]
+    assert ((lse.double().cpu() - want).abs() <= 1.2e-8 + 2.5e-7 * want.abs()).all()
