@@ -37,12 +37,12 @@ FLAGS = [
 # accumulation registers these own (OWNED of their Lone<>); the compiler's listing of them is checked (see listing_check.py)
 _KV, _KP = (("mfma_bwd_kv_kernel", 192),), (("mfma_bwd_kp_lone_kernel", 256),)
 _SKV, _SKP = (("split_kv_lone_kernel", 192),), (("split_kp_lone_kernel", 256),)
-_SFWD = (("split_fwd_lone_kernel.*Li64E", 192), ("split_fwd_lone_kernel.*Li96ELi2E", 192), ("split_fwd_lone_kernel.*Li96ELi3E", 256))
+_SFWD = (("split_fwd_lone_kernel.*Li64E", 192), ("split_fwd_lone_kernel.*Li96E", 256))
 _FWD = (("mfma_fwd_lone_kernel.*Li64E", 96), ("mfma_fwd_lone_kernel.*Li128E", 192))
 HAND_PLACED = {"sa2_mfma_bwd_kv_bf16.hip": _KV, "sa2_mfma_bwd_kv_fp16.hip": _KV,
                "sa2_mfma_bwd_kp_lone_bf16.hip": _KP, "sa2_mfma_bwd_kp_lone_fp16.hip": _KP,
                "sa2_mfma_fwd_lone_bf16.hip": _FWD, "sa2_mfma_fwd_lone_fp16.hip": _FWD,
-               "sa2_split_fwd_lone_bf16.hip": _SFWD, "sa2_split_fwd_lone_fp16.hip": (_SFWD[0], _SFWD[2]),
+               "sa2_split_fwd_lone_bf16.hip": _SFWD, "sa2_split_fwd_lone_fp16.hip": _SFWD,
                "sa2_split_fwd_lone_fp32.hip": _SFWD[:1],
                "sa2_split_kp_lone_bf16.hip": _SKP, "sa2_split_kp_lone_fp16.hip": _SKP, "sa2_split_kp_lone_fp32.hip": _SKP,
                "sa2_split_kv_lone_bf16.hip": _SKV, "sa2_split_kv_lone_fp32.hip": _SKV,

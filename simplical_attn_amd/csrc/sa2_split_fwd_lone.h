@@ -37,12 +37,9 @@ struct SplitFwdLoneCfg {
     static constexpr size_t larger(size_t a, size_t b) { return a > b ? a : b; }
     static constexpr size_t X_AT = larger(larger(TILES + ROWS, (size_t)W * BQ * AS * 4), smem_bytes(D, W));
     static constexpr size_t LDS_BYTES = X_AT + 2 * W * BQ * 4;
-    // Where the reference point comes off the logits: last, by an MFMA of its planes, or where the chain starts.  Last, it costs one
-    // rounding at the size of the result; a chain that starts from it rounds every step at its size, which fp32 results show (1.2 to 1.5 times
-    // the error) and fp16 ones just so.
-    static constexpr bool LEAD = T::PLANES > 1;
-    // accumulation registers: R tiles, planes of Q~, the reference point's
-    static constexpr int R0 = 0, Q0 = U * DT * 16, M0 = Q0 + U * NQ * DK * 4, USED = M0 + (LEAD ? U * 4 : 0), OWNED = USED <= 96 ? 96 : USED <= 192 ? 192 : 256;
+    // accumulation registers: R tiles, planes of Q~, the reference point's.  (It comes off the logits last, by an MFMA of its planes, which costs
+    // one rounding at the size of the result.  A chain that starts from it rounds every step at its size.)
+    static constexpr int R0 = 0, Q0 = U * DT * 16, M0 = Q0 + U * NQ * DK * 4, USED = M0 + U * 4, OWNED = USED <= 96 ? 96 : USED <= 192 ? 192 : 256;
     static_assert(USED <= 256 && LDS_BYTES <= 160 * 1024, "");
 };
 
@@ -245,13 +242,12 @@ void split_fwd_lone_kernel(Problem p, int nqb, int total) {
     constexpr Products<NK, NQ> PA;                            // plane of the tile, of Q~
     constexpr Products<NK, 3> PC;                             // plane of the tile, of P
     constexpr int NP = PA.n, NC = PC.n;
-    constexpr int NA = NP * DK + C::LEAD, NE = 2 * DT, NV = NE * NC;           // MFMAs of a phase A; V operands; MFMAs of a phase C
+    constexpr int NA = NP * DK + 1, NE = 2 * DT, NV = NE * NC;           // MFMAs of a phase A; V operands; MFMAs of a phase C
     constexpr int P2 = NA, P3 = NA + NV, P4 = 2 * NA + NV, NS = 2 * (NA + NV);         // slots of a tile: A(0), C'(1), A(1), C(0)
     constexpr int AHEAD = NP >= 5 ? 1 : NP == 3 ? 2 : 3;      // k-steps that row operands are read ahead
     static_assert(AHEAD <= DK, "");
     X8 ro[AHEAD + 1][NK], vt[NE][NK];
-    constexpr int NM = C::LEAD ? 1 : 2;
-    floatx16 s[2], nl[NM];                                    // logits; what their chains start from: (LEAD) 0 or -m, -inf where the key is outside the window
+    floatx16 s[2], nl;                                        // logits; what their chains start from: 0, -inf where the key is outside the window
     float m[2];                                               // reference points of the units (of the logits as the chains give them)
     const float limit = NQ == 2 ? 64.f / qscale : 64.f;       // 64 octaves
     const float octaves = NQ == 2 ? qscale : 1.f;
@@ -299,7 +295,7 @@ void split_fwd_lone_kernel(Problem p, int nqb, int total) {
             L::template tile_more<C::M0 + 4 * u>(s[u], ones);
         } else {
             constexpr int kk = i / NP, x = PA.x[i % NP], y = PA.y[i % NP], at = Q0 + ((u * NQ + y) * DK + kk) * 4;
-            if constexpr (i == 0) L::template tile_start<at>(s[u], ro[0][x], nl[u % NM]);
+            if constexpr (i == 0) L::template tile_start<at>(s[u], ro[0][x], nl);
             else L::template tile_more<at>(s[u], ro[kk % (AHEAD + 1)][x]);
         }
     };
@@ -349,7 +345,7 @@ void split_fwd_lone_kernel(Problem p, int nqb, int total) {
             item(UN, X);
         });
     };
-    auto set_reference = [&](auto UN) __attribute__((always_inline)) {              // (LEAD) the planes of m
+    auto set_reference = [&](auto UN) __attribute__((always_inline)) {              // the planes of m
         constexpr int u = decltype(UN)::value;
         const u4 w = __builtin_bit_cast(u4, lead_planes(m[u], 0.f));
         L::template set_regs<C::M0 + 4 * u>(w[0], w[1], w[2], w[3]);
@@ -376,13 +372,7 @@ void split_fwd_lone_kernel(Problem p, int nqb, int total) {
                 l[u] *= alpha;
 #pragma unroll
                 for (int v = 0; v < 16; ++v) s[u][v] -= shift;
-                if constexpr (C::LEAD) {
-                    set_reference(UN);
-                } else {
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) nl[u % NM][v] -= shift;
-                    asm volatile("s_nop 3" : "+v"(nl[u % NM]));
-                }
+                set_reference(UN);
                 static_for<DT * 4>([&](auto X) __attribute__((always_inline)) {
                     constexpr int r = R0 + u * DT * 16 + 4 * decltype(X)::value;
                     const float4 x = L::template get_regs<r>();
@@ -423,7 +413,7 @@ void split_fwd_lone_kernel(Problem p, int nqb, int total) {
             beside(I, DO_C, stage_at);
             __builtin_amdgcn_sched_barrier(0);
         });
-        if constexpr (!CC) finished(s[0], nl[0]);
+        if constexpr (!CC) finished(s[0], nl);
         // V operand e is read again behind its last MFMA
         auto columns_behind = [&](auto J) __attribute__((always_inline)) {
             constexpr int j = decltype(J)::value - 1, e = j / NC - 1, x = j % NC;
@@ -480,7 +470,7 @@ void split_fwd_lone_kernel(Problem p, int nqb, int total) {
             deal<NE * NK, i, NA>([&](auto X) __attribute__((always_inline)) { read_column(LONE_C(decltype(X)::value / NK), LONE_C(decltype(X)::value % NK)); });
             __builtin_amdgcn_sched_barrier(0);
         });
-        finished(s[0], nl[0]);
+        finished(s[0], nl);
         watch(LONE_C(0), LONE_C(0));
         watch(LONE_C(0), LONE_C(1));
         static_for<HALF>([&](auto SLOT) __attribute__((always_inline)) { softmax(LONE_C(0), SLOT); });
@@ -524,28 +514,20 @@ void split_fwd_lone_kernel(Problem p, int nqb, int total) {
         if (plain && unmasked) return;
         unmasked = plain;
         const uint32_t seen = plain ? ~0u : keys_seen(jt);
-        const int v1 = __float_as_int(-INFINITY);
 #pragma unroll
-        for (int u = 0; u < NM; ++u) {
-            const int v0 = C::LEAD ? 0 : __float_as_int(-m[u]);
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                int x = (int)(seen << (31 - 8 * (v >> 2) - (v & 3))) >> 31;
-                asm("" : "+v"(x));
-                nl[u][v] = __int_as_float((v0 & x) | (v1 & ~x));
-            }
-            asm volatile("s_nop 3" : "+v"(nl[u]));
+        for (int v = 0; v < 16; ++v) {
+            int x = (int)(seen << (31 - 8 * (v >> 2) - (v & 3))) >> 31;
+            asm("" : "+v"(x));
+            nl[v] = __int_as_float(__float_as_int(-INFINITY) & ~x);
         }
+        asm volatile("s_nop 3" : "+v"(nl));
     };
     // the units' logits in the tile at sa and their largest ones, where the lane's row has a key; the others become -inf
     auto tile_logits = [&](int jt, int d0, float (&mx)[2]) __attribute__((always_inline)) {
         const int t = here(), i = i0 + (t & 31);
         const uint32_t seen = keys_seen(jt);
-#pragma unroll
-        for (int u = 0; u < NM; ++u) {
-            nl[u] = zero16();
-            asm volatile("s_nop 3" : "+v"(nl[u]));
-        }
+        nl = zero16();
+        asm volatile("s_nop 3" : "+v"(nl));
         at_stage(sa, row_lane, r0, r1);
         static_for<2>([&](auto UN) __attribute__((always_inline)) {
             static_for<DK>([&](auto KK) __attribute__((always_inline)) {
@@ -621,7 +603,7 @@ void split_fwd_lone_kernel(Problem p, int nqb, int total) {
         }
         static_for<2>([&](auto UN) __attribute__((always_inline)) {
             m[decltype(UN)::value] = Mw;
-            if constexpr (C::LEAD) set_reference(UN);
+            set_reference(UN);
         });
         {
             unmasked = false;

@@ -6,6 +6,7 @@ other tests of these kernels; lse to 1e-5 of its largest value (16 bits: of exac
 import pytest
 import torch
 
+from oracle import simplicial_oracle as orc
 from tests.util import assert_close_rel
 
 pytestmark = pytest.mark.gpu
@@ -66,3 +67,26 @@ def test_widely_spread_logits(dtype, D, std):
         assert torch.isfinite(out).all()
         assert_close_rel(lse, want_lse.cpu(), 1e-5, "lse")
         assert_close_rel(out, want.cpu(), max(BAR[dtype], 1e-3), "out")
+
+
+@pytest.mark.parametrize("dtype,D", [(F32, 64), (BF, 40), (BF, 56), (BF, 72), (BF, 96), (FP, 48), (FP, 96)])
+@pytest.mark.parametrize("bias", [0.0, 0.25])
+def test_the_reference_point_comes_off_the_logits_last(dtype, D, bias):
+    """The queries' own tile holds logits of -5, one key before it a small generic one, which decides the row.  Less the reference point it is
+    7.2 octaves, where a rounding has a root mean square of 2^-22 / sqrt(12) octaves (1e-7 in lse): one of the difference, one of the scale
+    where that is multiplied on last, and half of one for the logit's chain at its own size and lse itself.  With the reference point at the start of the chain
+    all 12 to 36 roundings had that size (2.8e-7 to 4.5e-7 in lse)."""
+    import simplical_attn_amd as sa
+    g = torch.Generator().manual_seed(D)
+    x = [torch.randn(2, 64, 16, D, generator=g) for _ in range(5)]
+    x[0], x[2] = 0.5 * x[0], 0.5 * x[2]
+    x[0][..., 0], x[2][..., 0] = 1.0, 1.0 - bias
+    key = x[1][:, 31].clone()
+    x[1][:] = 0.0
+    x[1][..., 0] = -5.0 * D ** 0.5
+    key[..., 0] = 0.0
+    x[1][:, 31] = key
+    x = [t.to(dtype) for t in x]
+    lse = sa.simplicial_forward(*[t.cuda() for t in x], 63, 0, None, bias)[1][:, :, 32:]
+    want = orc.forward_windowed(*[t.double() for t in x], 63, 0, None, bias)[1][:, :, 32:]
+    assert (lse.double().cpu() - want).pow(2).mean().sqrt() < 2.3e-7
