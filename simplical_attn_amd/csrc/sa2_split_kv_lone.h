@@ -23,6 +23,7 @@
 #pragma once
 
 #include "sa2_split_lone.h"
+#include "sa2_units.h"
 
 namespace sa2 {
 namespace {
@@ -148,7 +149,6 @@ void split_kv_lone_kernel(Problem p, int njb, int total, int nsplit, float* __re
         }
     };
     // cursors: the unit that is formed next (two ahead of the one in work), and the one whose K' and V' rows are requested next
-    constexpr int NEVER = 0x7fffffff;
     int f_ib = ib_lo, f_delta = d_first, f_stop = 0, l_ib = ib_lo, l_delta = d_first, l_stop = 0;
     auto stop_of = [&](int ib) __attribute__((always_inline)) { return ib <= ib_hi ? last_unit_of(ib) : NEVER; };
     auto request_unit = [&]() __attribute__((always_inline)) {
@@ -443,9 +443,7 @@ void split_kv_lone_kernel(Problem p, int njb, int total, int nsplit, float* __re
         };
         // units (the present one included) until something changes: the block or its masks, or a cursor's block
         auto until = [&]() __attribute__((always_inline)) {
-            int n = stop - delta + 1;
-            if (f_stop - f_delta + 1 < n) n = f_stop - f_delta + 1;
-            if (l_stop - l_delta + 1 < n) n = l_stop - l_delta + 1;
+            int n = units_left(units_left(stop - delta + 1, f_delta, f_stop), l_delta, l_stop);
             if (stop > ib * BQ) {
                 const int whole = ib * BQ - delta + 1;
                 if (whole < n) n = whole > 1 ? whole : 1;
