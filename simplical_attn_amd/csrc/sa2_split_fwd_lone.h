@@ -14,9 +14,12 @@
 // w 512/32 812 / 775, B1 H2 N128 D64 w 32/16 (eight workgroups, not shared) 28.2 / 25.7.
 //
 // The reference point m of a row is the largest logit of the wavefront's first two units in the queries' own tile, which holds a key of every
-// row.  The largest of each further tile's logits is looked at before their exponentials: where one lies more than 64 octaves above m
-// (weights and their sums stay far from overflow until then) that unit's sums are brought to a reference point there, by a branch that
-// usual logits never take.
+// row.  A logit less m is rounded at the size of the difference.  So the largest logit S of each further tile is looked at before the
+// exponentials, and a unit's sums are brought to a reference point there where S - m is more than 8 octaves and more than twice |S|, at whose size S is
+// rounded in any case, or more than 40 octaves (weights and their sums stay far from overflow until then); the tile's logits are then formed
+// again without m, by a branch that usual logits hardly take.  With keys of the own tile 15, 30, 1e3 and 1e5 octaves below the row's others
+// and only a step at 64 octaves, taken off the rounded difference, fp32 outputs were 1.6, 2.4, 39 and 4800 times as far from fp64 as with a
+// maximum taken per tile; now they are as far (0.97).
 #pragma once
 
 #include "sa2_fma_rows.h"
@@ -249,8 +252,7 @@ void split_fwd_lone_kernel(Problem p, int nqb, int total) {
     X8 ro[AHEAD + 1][NK], vt[NE][NK];
     floatx16 s[2], nl;                                        // logits; what their chains start from: 0, -inf where the key is outside the window
     float m[2];                                               // reference points of the units (of the logits as the chains give them)
-    const float limit = NQ == 2 ? 64.f / qscale : 64.f;       // 64 octaves
-    const float octaves = NQ == 2 ? qscale : 1.f;
+    const float octaves = NQ == 2 ? qscale : 1.f, near = 8.f / octaves, far = 40.f / octaves;
     const X8 ones = lead_ones(hf);
     u4 pw[2][2][3];                                           // planes of the weights: unit, half of the keys
     float l[2], rs[2];                                        // sums of the weights: of the sweep, of the tile
@@ -359,6 +361,30 @@ void split_fwd_lone_kernel(Problem p, int nqb, int total) {
         asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
         return r;
     };
+    // Tile jt_now's logits of a unit, without the reference point, from K rows in global memory: their stage may be written again by now.
+    int jt_now = jt_hi;
+    auto form_logits = [&](auto UN) __attribute__((always_inline)) {
+        constexpr int u = decltype(UN)::value;
+        const int t = here(), j = jt_now * TJ + (t & 31);
+        const EL* row = k1p + (int64_t)(j < N ? j : N - 1) * p.k1.sn;
+        static_for<DK>([&](auto KK) __attribute__((always_inline)) {
+            constexpr int kk = decltype(KK)::value;
+            const int col = kk * 16 + (t >> 5 & 1) * 8;
+            const float4 x0 = cols4<T, PAD>(row, col, p.D), x1 = cols4<T, PAD>(row, col + 4, p.D);
+            const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+            X8 k[NK];
+            split8<NK, T::DTYPE == SA2_F32>(x, k);
+#pragma unroll
+            for (int n = 0; n < NK; ++n) asm volatile("s_nop 3" : "+v"(k[n]));
+            static_for<NP>([&](auto I) __attribute__((always_inline)) {
+                constexpr int i = decltype(I)::value, at = Q0 + ((u * NQ + PA.y[i]) * DK + kk) * 4;
+                if constexpr (kk == 0 && i == 0) L::template tile_start<at>(s[u], k[PA.x[i]], nl);
+                else L::template tile_more<at>(s[u], k[PA.x[i]]);
+            });
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        finished(s[u], nl);
+    };
     auto watch = [&](auto UN, auto PART) __attribute__((always_inline)) {
         constexpr int u = decltype(UN)::value;
         if constexpr (decltype(PART)::value == 0) {
@@ -366,13 +392,20 @@ void split_fwd_lone_kernel(Problem p, int nqb, int total) {
             stays(top);
         } else {
             top = max3(max3(max3(max3(top, s[u][9], s[u][10]), s[u][11], s[u][12]), s[u][13], s[u][14]), s[u][15], s[u][15]);
-            if (__builtin_expect(__builtin_amdgcn_ballot_w64(top > limit) != 0, 0)) {
-                const float row = fmaxf(top, other_half(top)), shift = row > limit ? row : 0.f, alpha = fast_exp2(-shift * octaves);
-                m[u] += shift;
-                l[u] *= alpha;
+            auto too_large = [&](float x) __attribute__((always_inline)) { return x > __builtin_amdgcn_fmed3f(near, far, 2.f * fabsf(m[u] + x)); };
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(too_large(top)) != 0, 0)) {
+                const bool move = too_large(fmaxf(top, other_half(top)));
+                form_logits(UN);
+                float best = s[u][0];
 #pragma unroll
-                for (int v = 0; v < 16; ++v) s[u][v] -= shift;
+                for (int v = 1; v < 16; ++v) best = fmaxf(best, s[u][v]);
+                best = fmaxf(best, other_half(best));
+                const float alpha = move ? fast_exp2((m[u] - best) * octaves) : 1.f;
+                m[u] = move ? best : m[u];
+                l[u] *= alpha;
                 set_reference(UN);
+                L::template tile_more<C::M0 + 4 * u>(s[u], ones);
+                finished(s[u], nl);
                 static_for<DT * 4>([&](auto X) __attribute__((always_inline)) {
                     constexpr int r = R0 + u * DT * 16 + 4 * decltype(X)::value;
                     const float4 x = L::template get_regs<r>();
@@ -599,7 +632,9 @@ void split_fwd_lone_kernel(Problem p, int nqb, int total) {
             float mx[2];
             tile_logits(jt_hi, d0, mx);
             Mw = fmaxf(mx[0], mx[1]);
-            Mw = Mw == -INFINITY ? 0.f : Mw;                  // (a row without a key here: none of its sums are taken)
+            // (No key here: none of the row's sums are taken.  Logits that are all -inf: far below any other.)
+            const int i = i0 + (here() & 31);
+            Mw = Mw != -INFINITY ? Mw : i < N && i >= d0 ? -8.507059173023462e37f : 0.f;
         }
         static_for<2>([&](auto UN) __attribute__((always_inline)) {
             m[decltype(UN)::value] = Mw;
@@ -608,8 +643,8 @@ void split_fwd_lone_kernel(Problem p, int nqb, int total) {
         {
             unmasked = false;
             if (alone) {
-                for (int jt = jt_hi; jt >= jt_lo; --jt) {
-                    enter_tile(jt);
+                for (jt_now = jt_hi; jt_now >= jt_lo; --jt_now) {
+                    enter_tile(jt_now);
                     solo();
                     advance_tile();
                     rotate();
@@ -617,17 +652,17 @@ void split_fwd_lone_kernel(Problem p, int nqb, int total) {
             } else {
                 at_stage(sa, row_lane, r0, r1);
                 read_first_rows();
-                enter_tile(jt_hi);
+                jt_now = jt_hi;
+                enter_tile(jt_now);
                 tile(no);
                 rotate();
-                for (int jt = jt_hi - 1; jt >= jt_lo;) {
-                    enter_tile(jt);
-                    const int n = jt < p_lo ? 1 : jt - p_lo + 1;           // tiles that need nothing done between them
-                    for (int k = n; k > 0; --k) {
+                for (--jt_now; jt_now >= jt_lo;) {
+                    enter_tile(jt_now);
+                    const int stop = jt_now < p_lo ? jt_now : p_lo;        // tiles down to there need nothing done between them
+                    for (; jt_now >= stop; --jt_now) {
                         tile(yes);
                         rotate();
                     }
-                    jt -= n;
                 }
                 last_sums();
             }

@@ -90,3 +90,27 @@ def test_the_reference_point_comes_off_the_logits_last(dtype, D, bias):
     lse = sa.simplicial_forward(*[t.cuda() for t in x], 63, 0, None, bias)[1][:, :, 32:]
     want = orc.forward_windowed(*[t.double() for t in x], 63, 0, None, bias)[1][:, :, 32:]
     assert (lse.double().cpu() - want).pow(2).mean().sqrt() < 2.3e-7
+
+
+@pytest.mark.parametrize("dtype,D", [(F32, 64), (BF, 40), (BF, 56), (BF, 72), (BF, 96), (FP, 48), (FP, 80)])
+@pytest.mark.parametrize("gap", [12.0, 30.0, 60.0, 1e3, 7e3, 1e6, 1e9, None])
+@pytest.mark.parametrize("w2,bias", [(9, 0.0), (2, 0.0), (40, 0.25)])
+def test_an_own_tile_far_below_the_other_keys(dtype, D, gap, w2, bias):
+    """Keys from 64 on are masked by a large finite K row (`gap` octaves; None: their logits overflow to -inf), so that every row from there on
+    has an own tile far below the logits that decide it.  Those logits have a size of up to 8: roundings of 2^-22 / sqrt(12) octaves, some three of them
+    in lse, and to the usual bars in out."""
+    import simplical_attn_amd as sa
+    if dtype == FP and (gap is None or gap > 1e4):
+        pytest.skip("no such K row in fp16")
+    g = torch.Generator().manual_seed(D + w2)
+    x = [torch.randn(2, 150, 8, D, generator=g) for _ in range(5)]
+    size = 1.0 if gap is not None else 8.0
+    x[0][..., 0], x[2][..., 0] = size, size - bias
+    x[1][..., 0] = 0.0
+    x[1][:, 64:] *= 0.1
+    x[1][:, 64:, :, 0] = -3e38 if gap is None else -gap * 0.6931 * D ** 0.5
+    x = [t.to(dtype) for t in x]
+    out, lse = sa.simplicial_forward(*[t.cuda() for t in x], 149, w2, None, bias, -bias)
+    want, want_lse = orc.forward_windowed(*[t.double() for t in x], 149, w2, None, bias, -bias)
+    assert (lse.double().cpu() - want_lse)[:, :, 64:].pow(2).mean().sqrt() < 4.5e-7
+    assert_close_rel(out[:, 64:], want[:, 64:], {F32: 3e-6}.get(dtype, BAR[dtype]), "out")
