@@ -76,30 +76,39 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(Problem p, int D, int64_
     const float2* ml = (const float2*)p.scratch;                       // (M, L) of [share][row]
     const float* part = (const float*)p.scratch + 2 * rows * p.nsplit;
     float M = -INFINITY;
+    int e = -126;
 #pragma unroll 4
-    for (int x = 0; x < p.nsplit; ++x) M = fmaxf(M, ml[x * rows + row].x);
+    for (int x = 0; x < p.nsplit; ++x) {
+        const float2 s = ml[x * rows + row];
+        M = fmaxf(M, s.x);
+        const int es = __builtin_amdgcn_frexp_expf(s.y);
+        e = es > e ? es : e;
+    }
     const float Mu = M == -INFINITY ? 0.f : M;
+    // M need not be the row's maximum: all sums in units of 2^e, so that those of up to sixteen shares add up without overflow
+    e += 4;
+    const float Me = Mu + (float)e;
     float L = 0.f;
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll 4
     for (int x = 0; x < p.nsplit; ++x) {
         const float2 s = ml[x * rows + row];
         if (s.x == -INFINITY && s.y == 0.f) continue;                  // (an empty share left no sums; NaN logits leave L NaN)
-        const float w = fast_exp2(s.x - Mu);
+        const float w = ldexpf(fast_exp2(s.x - Mu), -e);
         const float4 y = *(const float4*)(part + (x * rows + row) * D + col);
         L += w * s.y;
         acc.x += w * y.x; acc.y += w * y.y; acc.z += w * y.z; acc.w += w * y.w;
     }
-    // sum + 1e-8 in units of 2^Mu; for a tiny Mu the epsilon dominates
-    const bool big = Mu > LOG2_EPS;
-    const float denom = big ? L + 1e-8f * fast_exp2(-Mu) : L * fast_exp2(Mu - LOG2_EPS) + 1.f;
-    const float inv = big ? 1.f / denom : fast_exp2(Mu - LOG2_EPS) / denom;
+    // sum + 1e-8 in units of 2^Me; for a tiny Me the epsilon dominates
+    const bool big = Me > LOG2_EPS;
+    const float denom = big ? L + 1e-8f * fast_exp2(-Me) : L * fast_exp2(Me - LOG2_EPS) + 1.f;
+    const float inv = big ? 1.f / denom : fast_exp2(Me - LOG2_EPS) / denom;
     const int i = (int)(row % p.N), bh = (int)(row / p.N), b = bh / p.H, h = bh - b * p.H;
     if constexpr (std::is_same<E, float>::value)
         *(float4*)((float*)p.out.p + p.out.off(b, i, h) + col) = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
     else
         *(uint2*)((uint16_t*)p.out.p + p.out.off(b, i, h) + col) = make_uint2(E::pack(acc.x * inv, acc.y * inv), E::pack(acc.z * inv, acc.w * inv));
-    if (col == 0) p.lse[row] = exact_lse(Mu, denom, big);
+    if (col == 0) p.lse[row] = exact_lse(Mu, denom, big, e);
 }
 
 }  // namespace

@@ -115,16 +115,18 @@ int for_mfma_width(int D, int dtype, F&& f) {
     return dtype == SA2_F16 ? of_type(ElemF16{}) : of_type(ElemBF16{});
 }
 
-// LSE of a row whose weights, in units of 2^M, sum to `denom` (`big`), or to denom in units of 1e-8.  A reference point that is not the
+// LSE of a row whose weights, in units of 2^M * 2^shift, sum to `denom` (`big`), or to denom in units of 1e-8.  A reference point that is not the
 // row's maximum leaves a sum whose logarithm is larger and carries a larger rounding (1.1 to 1.2 times the error of an fp32 LSE): the sum's
 // exponent joins M, exactly, and what is rounded at the size of the result is one product.  (The same in 64 bits: 0.4 us more per launch.)
 // The mantissa is taken from sqrt(1/2) on: below 1 throughout, a sum of one weight would leave ln(1/2), whose rounding stays where M is small.
-__device__ __forceinline__ float exact_lse(float M, float denom, bool big) {
+__device__ __forceinline__ float exact_lse(float M, float denom, bool big, int shift = 0) {
     constexpr float HI = 0.693147182464599609375f, LO = -1.904654323148236e-9f;      // ln 2
     const float x = __builtin_amdgcn_frexp_mantf(denom);
     const bool low = x < 0.70710678f;
-    const float e = (float)(__builtin_amdgcn_frexp_expf(denom) - low), l = logf(low ? 2.f * x : x);
+    float e = (float)(__builtin_amdgcn_frexp_expf(denom) - low);
+    const float l = logf(low ? 2.f * x : x);
     if (!big) return -18.42068099975586f + (fmaf(e, HI, l) + 2.558034936e-7f);         // ln 1e-8
+    e += (float)shift;
     const float s = M + e, b = s - M, rest = (M - (s - b)) + (e - b);
     return fmaf(s, HI, fmaf(s, LO, l) + rest * HI);
 }

@@ -16,7 +16,8 @@
 // The reference point m of a row is the largest logit of the wavefront's first two units in the queries' own tile, which holds a key of every
 // row.  A logit less m is rounded at the size of the difference.  So the largest logit S of each further tile is looked at before the
 // exponentials, and a unit's sums are brought to a reference point there where S - m is more than 8 octaves and more than twice |S|, at whose size S is
-// rounded in any case, or more than 40 octaves (weights and their sums stay far from overflow until then); the tile's logits are then formed
+// rounded in any case, or more than 40 octaves (weights and their sums stay far from overflow until then; a block whose sums of
+// values do not is computed by rows); the tile's logits are then formed
 // again without m, by a branch that usual logits hardly take.  With keys of the own tile 15, 30, 1e3 and 1e5 octaves below the row's others
 // and only a step at 64 octaves, taken off the rounded difference, fp32 outputs were 1.6, 2.4, 39 and 4800 times as far from fp64 as with a
 // maximum taken per tile; now they are as far (0.97).
@@ -739,7 +740,9 @@ void split_fwd_lone_kernel(Problem p, int nqb, int total) {
     __syncthreads();
     constexpr int TPR = KT / BQ;                              // threads per row
     const int row = tid_m / TPR, io = i0 + row;
-    bool nan = false, tiny = false, usual = T::DTYPE != SA2_F32;      // of the results (see split_fwd_kernel)
+    // of the results (see split_fwd_kernel); weights of up to 2^40 may make an infinite sum of values whose mean is finite
+    constexpr float MOST = 3.4028234663852886e38f;
+    bool bad = false, tiny = false, usual = T::DTYPE != SA2_F32;
     if (io < N) {
         float Mx = -INFINITY;
 #pragma unroll
@@ -753,10 +756,13 @@ void split_fwd_lone_kernel(Problem p, int nqb, int total) {
         }
         const int64_t rows = (int64_t)p.B * p.H * N, prow = share * rows + (int64_t)bh * N + io;
         if (SPLIT && tid_m % TPR == 0) ((float2*)p.scratch)[prow] = make_float2(Mx, Ls);
-        // sum_w + 1e-8 in units of 2^Mu (reference.py:74); for a tiny Mu the epsilon dominates
-        const bool big = Mu > LOG2_EPS;
-        const float denom = big ? Ls + 1e-8f * fast_exp2(-Mu) : Ls * fast_exp2(Mu - LOG2_EPS) + 1.f;
-        const float inv = big ? 1.f / denom : fast_exp2(Mu - LOG2_EPS) / denom;
+        // The reference points need not be maxima: results in units of 2^e.  sum_w + 1e-8 in units of 2^Me (reference.py:74); for a tiny Me the
+        // epsilon dominates
+        const int e = __builtin_amdgcn_frexp_expf(Ls);
+        const float Me = Mu + (float)e, Le = ldexpf(Ls, -e);
+        const bool big = Me > LOG2_EPS;
+        const float denom = big ? Le + 1e-8f * fast_exp2(-Me) : Le * fast_exp2(Me - LOG2_EPS) + 1.f;
+        const float inv = big ? 1.f / denom : fast_exp2(Me - LOG2_EPS) / denom;
         EL* orow = (EL*)p.out.p + p.out.off(b, io, h);
 #pragma unroll
         for (int col = 4 * (tid_m % TPR); col < D; col += 4 * TPR) {
@@ -767,10 +773,10 @@ void split_fwd_lone_kernel(Problem p, int nqb, int total) {
                 const float4 y = *(const float4*)(mrg + (w * BQ + row) * C::AS + col);
                 acc.x += wgt[w] * y.x; acc.y += wgt[w] * y.y; acc.z += wgt[w] * y.z; acc.w += wgt[w] * y.w;
             }
-            const float r[4] = {acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv};
+            const float r[4] = {ldexpf(acc.x, -e) * inv, ldexpf(acc.y, -e) * inv, ldexpf(acc.z, -e) * inv, ldexpf(acc.w, -e) * inv};
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                nan |= r[t] != r[t];
+                bad |= !(fabsf(r[t]) <= MOST);
                 if (T::DTYPE == SA2_F32) {
                     usual |= fabsf(r[t]) >= TINY;
                     tiny |= r[t] != 0.f && fabsf(r[t]) < TINY;
@@ -779,14 +785,14 @@ void split_fwd_lone_kernel(Problem p, int nqb, int total) {
             if constexpr (SPLIT) *(float4*)((float*)p.scratch + 2 * rows * p.nsplit + prow * D + col) = acc;
             else T::store(orow + col, r[0], r[1], r[2], r[3]);
         }
-        if (!SPLIT && tid_m % TPR == 0) p.lse[(int64_t)bh * N + io] = exact_lse(Mu, denom, big);
-        nan |= Ls != Ls;
+        if (!SPLIT && tid_m % TPR == 0) p.lse[(int64_t)bh * N + io] = exact_lse(Mu, denom, big, e);
+        bad |= !(Ls <= MOST);
     }
 
     // ---- what the planes do not cover: the block again, by rows (see split_fwd_kernel) ----
-    if (!__syncthreads_or(nan || tiny)) return;
-    const bool any_nan = __syncthreads_or(nan), any_usual = __syncthreads_or(usual);
-    if (!any_nan && any_usual) return;
+    if (!__syncthreads_or(bad || tiny)) return;
+    const bool any_bad = __syncthreads_or(bad), any_usual = __syncthreads_or(usual);
+    if (!any_bad && any_usual) return;
     {
         // (a row whose q holds a NaN is NaN as it stands: a block of such rows is done)
         bool q_nan = false;

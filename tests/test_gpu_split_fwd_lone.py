@@ -114,3 +114,43 @@ def test_an_own_tile_far_below_the_other_keys(dtype, D, gap, w2, bias):
     want, want_lse = orc.forward_windowed(*[t.double() for t in x], 149, w2, None, bias, -bias)
     assert (lse.double().cpu() - want_lse)[:, :, 64:].pow(2).mean().sqrt() < 4.5e-7
     assert_close_rel(out[:, 64:], want[:, 64:], {F32: 3e-6}.get(dtype, BAR[dtype]), "out")
+
+
+def _far_tile(dtype, D, own, far, size, heads=8, N=150):
+    """Rows from 64 on: keys of the own tile at `own` octaves, those before at `far`; values v1 and v2 of a size"""
+    g = torch.Generator().manual_seed(D)
+    x = [torch.randn(2, N, heads, D, generator=g) for _ in range(5)]
+    x[0][..., 0], x[2][..., 0] = 4.0, 4.0
+    x[1] *= 0.1
+    x[1][..., 0] = far * 0.6931 * D ** 0.5 / 16
+    x[1][:, 64:, :, 0] = own * 0.6931 * D ** 0.5 / 16
+    x[3], x[4] = x[3] * size, x[4] * size
+    return [t.to(dtype) for t in x]
+
+
+@pytest.mark.parametrize("dtype,D", [(F32, 64), (BF, 40), (BF, 56), (BF, 72), (BF, 96)])
+@pytest.mark.parametrize("own,far,size", [(10.0, 45.0, 2.0 ** 52), (4.0, 40.0, 2.0 ** 46), (20.0, 50.0, 2.0 ** 56)])
+@pytest.mark.parametrize("w2,heads", [(9, 8), (30, 1)])
+def test_values_that_large_weights_would_make_infinite(dtype, D, own, far, size, w2, heads):
+    """Weights of 2^30 to 2^36, relative to the own tile's, times products v1*v2 of 2^92 to 2^112 are no floats; the outputs are, and so are the
+    sums over shares (one head), with weights up to 1: at most 150 * 31 products of 2^112 * 2^4, 2^128.2 if all had one sign."""
+    import simplical_attn_amd as sa
+    x = _far_tile(dtype, D, own, far, size, heads)
+    out, lse = sa.simplicial_forward(*[t.cuda() for t in x], 149, w2)
+    want, want_lse = orc.forward_windowed(*[t.double() for t in x], 149, w2)
+    assert torch.isfinite(out).all() and want.abs().max() > 2.0 ** 90
+    assert_close_rel(out, want, {F32: 1e-5}.get(dtype, BAR[dtype]), "out")
+    assert_close_rel(lse, want_lse, 1e-5, "lse")
+
+
+@pytest.mark.parametrize("dtype,D", [(F32, 64), (BF, 40), (BF, 56), (BF, 72), (BF, 96)])
+@pytest.mark.parametrize("w2,heads", [(9, 8), (30, 1)])
+def test_weights_far_below_the_epsilon(dtype, D, w2, heads):
+    """Rows whose largest logit is at -125 octaves, 35 above the own tile: out is 2^(26.6 - 125) times the values' sums, which are large.  An octave is
+    rounded at the size of 125 (2^-18: 3e-6 of a weight)."""
+    import simplical_attn_amd as sa
+    x = _far_tile(dtype, D, -160.0, -125.0, 2.0 ** 20, heads)
+    out, lse = sa.simplicial_forward(*[t.cuda() for t in x], 149, w2)
+    want, want_lse = orc.forward_windowed(*[t.double() for t in x], 149, w2)
+    assert_close_rel(out[:, 70:], want[:, 70:], max(BAR[dtype], 3e-5), "out", atol=0.0)
+    assert_close_rel(lse, want_lse, 1e-6, "lse")
