@@ -252,7 +252,7 @@ __device__ __forceinline__ void product_planes(const typename T::T* xrow, const 
 
 // ================================================================== forward =====
 // SPLIT: one of nsplit shares of the rounds, unnormalised sums to the workspace (see launch_fwd_merge).
-// NQ: planes of Q~; two where q*k2 has 16 bits (bf16 tensors, no bias): the scale is multiplied onto the logits instead, which take
+// NQ: planes of Q~; two where q*k2 has 16 bits (exact_products below): the scale is multiplied onto the logits instead, which take
 // two MFMAs per k-step rather than three.
 template <class T, int D, int MODE, bool SPLIT, int NQ>
 __global__ __launch_bounds__((SplitCfg<T, D>::FW * 64)) __attribute__((amdgpu_waves_per_eu(SplitCfg<T, D>::FW / 4, SplitCfg<T, D>::FW / 4)))
@@ -1131,10 +1131,11 @@ size_t split_dq_part_bytes(int B, int N, int H, int D, const KpPlan& pl) {
 size_t split_kp_bytes(int B, int N, int H, int D, const KpPlan& pl) {
     return split_dq_part_bytes(B, N, H, D, pl) + (pl.nseg > 1 ? (size_t)2 * pl.nseg * B * H * (size_t)N * D * sizeof(float) : 0);
 }
-// Whether products of a unit have 16 bits, so that two planes hold them and the scale may wait until they are summed
+// Whether products of a unit have 16 bits, so that two planes hold them and the scale may wait until they are summed (a scale with which such
+// products and sums stay as far from the ends of fp32 as scaled ones)
 template <class T>
 bool exact_products(const Problem& p, bool backward) {
-    return T::DTYPE == SA2_BF16 && p.k2_bias == 0.f && (!backward || p.v2_bias == 0.f) && p.scale >= 8.6736174e-19f && p.scale <= 1.1529215e18f;     // 2^-60 .. 2^60
+    return T::DTYPE == SA2_BF16 && p.k2_bias == 0.f && (!backward || p.v2_bias == 0.f) && p.scale >= 8.6736174e-19f && p.scale <= 1024.f;     // 2^-60 .. 2^10
 }
 // Whether the kernels with one wavefront per SIMD are taken (sa2_split_fwd_lone.h, sa2_split_kv_lone.h, sa2_split_kp_lone.h)
 template <class T, int D, int MODE>
@@ -1199,7 +1200,7 @@ int launch_split_fwd(const Problem& p, hipStream_t st) {
         };
         if (total * (p.nsplit > 1 ? p.nsplit : 1) > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
         bool ok;
-        if constexpr (T::PLANES == 1) ok = p.k2_bias == 0.f ? go_split(std::integral_constant<int, 2>{}) : go_split(std::integral_constant<int, 3>{});
+        if constexpr (T::PLANES == 1) ok = exact_products<T>(p, false) ? go_split(std::integral_constant<int, 2>{}) : go_split(std::integral_constant<int, 3>{});
         else ok = go_split(std::integral_constant<int, 3>{});
         if (!ok) return SA2_ERR_LAUNCH_FAILED;
         if (p.nsplit <= 1) return SA2_OK;

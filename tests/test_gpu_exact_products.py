@@ -26,3 +26,21 @@ def test_two_planes_are_as_exact_as_three(D, B, N, H, w1, w2, scale):
         size = {n: want[n].double().norm().item() for n in NAMES}
     for n in NAMES:
         assert error[0.0][n] <= 1.01 * error[1e-30][n] + 2e-5 * size[n], (n, error[0.0][n] / size[n], error[1e-30][n] / size[n])
+
+
+@pytest.mark.parametrize("D", [8, 24, 72, 96, 104, 120])
+@pytest.mark.parametrize("heads", [1, 40])
+def test_a_scale_that_cannot_wait(D, heads):
+    """q*k2 is no float here (2^-140), scale*q*k2 and the logits are: three planes with the scale in them, in every forward and in the backward."""
+    import simplical_attn_amd as sa
+    host = make_inputs(1, 63, heads, D, seed=D, dtype=torch.bfloat16)
+    host[0], host[2], host[1] = host[0] * 2.0 ** -70, host[2] * 2.0 ** -70, host[1] * 2.0 ** 60
+    scale = 2.0 ** 80 * D ** -0.5
+    want = oracle_all([x.double() for x in host], 40, 9, scale)
+    x = [t.to("cuda:0") for t in host]
+    out, lse = sa.simplicial_forward(*x[:5], 40, 9, scale)
+    got = (out, lse) + sa.simplicial_backward(*x[:5], out, lse, x[5], 40, 9, scale)
+    assert want["lse"].std() > 0.5
+    for n, g in zip(NAMES, got):
+        error = (g.double().cpu() - want[n].double()).norm() / want[n].double().norm()
+        assert error < (1e-6 if n == "lse" else 1e-2), (n, error)
