@@ -518,7 +518,7 @@ void split_fwd_kernel(Problem p, int nqb, int total) {
 
 // ============================================== backward: which arithmetic =====
 // The row term, and whether the planes cover the operands: they do not where one is infinite or NaN, where products of q
-// and K' or of dO and V' may overflow, and (fp32) where all of a tensor's values in a workgroup's rows are so small, and
+// and K' or of dO and V' may overflow, or (bf16) LSE / scale, and (fp32) where all of a tensor's values in a workgroup's rows are so small, and
 // not zero, that products of them come under 2^-110.  Each workgroup takes a run of consecutive rows and leaves its
 // verdict in guard[blockIdx.x]: 0 covered, 1 not, 2 not but every row has a NaN in q or nothing else in dO, which makes
 // everything that such rows reach NaN as it stands.  The two kernels below run whatever it says; where it is 1, or 2 for some
@@ -580,7 +580,7 @@ __global__ __launch_bounds__(256) void split_guard_kernel(Problem p, int lpr_log
             }
             if (sub == 0) {
                 const float lse = p.lse[row];
-                bad |= !(fabsf(lse) < INFINITY);
+                bad |= !(fabsf(lse) < (T::PLANES == 1 ? GUARD_HIGH : INFINITY));
             }
         }
         for (int off = lpr >> 1; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
@@ -1132,7 +1132,7 @@ size_t split_kp_bytes(int B, int N, int H, int D, const KpPlan& pl) {
     return split_dq_part_bytes(B, N, H, D, pl) + (pl.nseg > 1 ? (size_t)2 * pl.nseg * B * H * (size_t)N * D * sizeof(float) : 0);
 }
 // Whether products of a unit have 16 bits, so that two planes hold them and the scale may wait until they are summed (a scale with which such
-// products and sums stay as far from the ends of fp32 as scaled ones)
+// products and sums stay as far from the ends of fp32 as scaled ones; the backward's LSE / scale: see split_guard_kernel)
 template <class T>
 bool exact_products(const Problem& p, bool backward) {
     return T::DTYPE == SA2_BF16 && p.k2_bias == 0.f && (!backward || p.v2_bias == 0.f) && p.scale >= 8.6736174e-19f && p.scale <= 1024.f;     // 2^-60 .. 2^10

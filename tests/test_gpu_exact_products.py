@@ -44,3 +44,20 @@ def test_a_scale_that_cannot_wait(D, heads):
     for n, g in zip(NAMES, got):
         error = (g.double().cpu() - want[n].double()).norm() / want[n].double().norm()
         assert error < (1e-6 if n == "lse" else 1e-2), (n, error)
+
+
+@pytest.mark.parametrize("D", [40, 72, 96])
+def test_logits_that_overflow_without_the_scale(D):
+    """One key with a logit of 2^128 * scale, the largest of every row that sees it: P is 0 or 1 (all of these are powers of two, so that logit and LSE
+    agree to the last bit), and dV and dV' are those of the fp32 FMA kernels."""
+    import simplical_attn_amd as sa
+    x = [t.cuda() for t in make_inputs(1, 150, 2, D, seed=D, dtype=torch.bfloat16)]
+    x[0][..., 0], x[2][..., 0] = 2.0, 1.0
+    x[1][:, 37, :, 0] = 2.0 ** 127
+    out, lse = sa.simplicial_forward(*x[:5], 60, 9, 0.125)
+    assert torch.isfinite(out).all() and lse.max() > 1e37
+    got = sa.simplicial_backward(*x[:5], out, lse, x[5], 60, 9, 0.125)
+    want = sa.simplicial_backward(*x[:5], out, lse, x[5], 60, 9, 0.125, flags=1)
+    for t in (3, 4):
+        assert (got[t] - want[t]).abs().max() <= 1e-2 * want[t].abs().max()
+    assert all(torch.equal(a.isnan(), b.isnan()) for a, b in zip(got, want))
