@@ -368,21 +368,32 @@ void split_fwd_lone_kernel(Problem p, int nqb, int total) {
         constexpr int u = decltype(UN)::value;
         const int t = here(), j = jt_now * TJ + (t & 31);
         const EL* row = k1p + (int64_t)(j < N ? j : N - 1) * p.k1.sn;
-        static_for<DK>([&](auto KK) __attribute__((always_inline)) {
-            constexpr int kk = decltype(KK)::value;
-            const int col = kk * 16 + (t >> 5 & 1) * 8;
-            const float4 x0 = cols4<T, PAD>(row, col, p.D), x1 = cols4<T, PAD>(row, col + 4, p.D);
-            const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-            X8 k[NK];
-            split8<NK, T::DTYPE == SA2_F32>(x, k);
+        constexpr int GROUP = NK == 1 ? DK : NK == 2 && D == 64 ? 2 : 1;      // k-steps whose loads are under way together: what registers there are
+        static_assert(DK % GROUP == 0, "");
+        static_for<DK / GROUP>([&](auto GR) __attribute__((always_inline)) {
+            Raw x[GROUP][2];
 #pragma unroll
-            for (int n = 0; n < NK; ++n) asm volatile("s_nop 3" : "+v"(k[n]));
-            static_for<NP>([&](auto I) __attribute__((always_inline)) {
-                constexpr int i = decltype(I)::value, at = Q0 + ((u * NQ + PA.y[i]) * DK + kk) * 4;
-                if constexpr (kk == 0 && i == 0) L::template tile_start<at>(s[u], k[PA.x[i]], nl);
-                else L::template tile_more<at>(s[u], k[PA.x[i]]);
-            });
+            for (int g = 0; g < GROUP; ++g) {
+                const int col = (decltype(GR)::value * GROUP + g) * 16 + (t >> 5 & 1) * 8;
+                x[g][0] = raw4<T, PAD>(row, col, p.D);
+                x[g][1] = raw4<T, PAD>(row, col + 4, p.D);
+            }
             __builtin_amdgcn_sched_barrier(0);
+            static_for<GROUP>([&](auto KK) __attribute__((always_inline)) {
+                constexpr int kk = decltype(GR)::value * GROUP + decltype(KK)::value;
+                const fx4 a = T::widen(x[decltype(KK)::value][0]), c = T::widen(x[decltype(KK)::value][1]);
+                const float y[8] = {a[0], a[1], a[2], a[3], c[0], c[1], c[2], c[3]};
+                X8 k[NK];
+                split8<NK, T::DTYPE == SA2_F32>(y, k);
+#pragma unroll
+                for (int n = 0; n < NK; ++n) asm volatile("s_nop 3" : "+v"(k[n]));
+                static_for<NP>([&](auto I) __attribute__((always_inline)) {
+                    constexpr int i = decltype(I)::value, at = Q0 + ((u * NQ + PA.y[i]) * DK + kk) * 4;
+                    if constexpr (kk == 0 && i == 0) L::template tile_start<at>(s[u], k[PA.x[i]], nl);
+                    else L::template tile_more<at>(s[u], k[PA.x[i]]);
+                });
+                __builtin_amdgcn_sched_barrier(0);
+            });
         });
         finished(s[u], nl);
     };
