@@ -1142,24 +1142,42 @@ template <class T, int D, int MODE>
 constexpr bool lone() { return T::DTYPE == SA2_F32 ? MODE != PADDED_FINE && D <= 64 : D == 64 || D == 96; }
 // Units of a forward's round.  At 96 columns grids that are at once on the chip in rounds of four are shared so, by split_fwd_kernel: a round
 // is all of such a launch, and two units per wavefront take it longer.  Rounds of eight against rounds of four, us: fp16 D80 B2 H8 N33 w 65/15
-// 20.5 / 16.6, B1 H4 N128 w 16/16 20.9 / 19.7, B1 H2 N300 w 200/12 33.2 / 31.1, w 40/24 23.5 / 22.9, B1 H2 N128 w 128/100 30.0 / 38.7.  Where logits
-// have two planes (bf16) only for the shortest sequences: N33 16.9 / 15.0, B1 H1 N64 w 16/8 16.1 / 14.4, but B1 H4 N512 w 40/15 19.5 / 20.4.
+// 20.5 / 16.6, B1 H4 N128 w 16/16 20.9 / 19.7, B1 H2 N300 w 200/12 33.2 / 31.1, w 40/24 23.5 / 22.9, B1 H4 N46 w 45/46 22.7 / 20.2, H1 N95 w 29/30 22.1 /
+// 20.6, B1 H2 N128 w 128/100 30.0 / 38.7.  Where logits have two planes (bf16) only for the shortest sequences: N33 16.9 / 15.0, B1 H1 N64 w 16/8
+// 16.1 / 14.4, B1 H1 N35 w 34/19 17.5 / 16.1, but B1 H4 N512 w 40/15 19.5 / 20.4.
 template <class T, int D, int MODE>
 int forward_round(int B, int N, int H, int w2) {
     if constexpr (lone<T, D, MODE>() && D == 96) {
         const int units = (w2 < N - 1 ? w2 : N - 1) + 1;
-        const bool few = T::PLANES == 1 ? units <= 16 && N <= 64 : units <= 20;
+        const bool few = T::PLANES == 1 ? units <= 24 && N <= 64 : units <= 20 || N <= 96;
         return few && units > 8 && (int64_t)B * H * ((N + BQ - 1) / BQ) * ((units + 3) / 4) <= CUS ? 4 : 8;
     }
     return SplitCfg<T, D>::FW;
 }
 // ... by the forward: at 32 columns not.  (Two units of a wavefront share an accumulator, whose longer chain of sums shows there: 1 - 4 % more error
 // in an fp32 output at head_dim 32 - 0.99 to 1.0 at 64 - for 5 - 10 % less time at most sizes, and 5 - 19 % more with few deltas or at head_dim 16.)
+// Nor where two units of a wavefront have little to lie beside: few deltas in short sweeps, and sequences of up to three tiles whose rounds are all at
+// once on the chip.  Two units per wavefront against one, us:
+//   fp32 D64: B1 H2 N119 w 23/1 12.9 / 10.0, H1 N826 w 31/2 13.0 / 10.7, B1 H64 N1173 w 17/2 90 / 75, B1 H8 N2054 w 761/2 119 / 109, H2 N756 w 86/4 18.4 /
+//     17.7, H46 N131 w 90/4 19.7 / 18.7, but H7 N388 w 405/4 33.9 / 37.7 and six deltas N1052 w 49 44.4 / 46.2, N388 w 387 34.3 / 38.1
+//   fp16 D48: N119 w 23/1 12.8 / 9.9, N1173 w 17/2 88.6 / 72.9, N274 w 27/5 13.8 / 11.5, N378 w 64/6 33.6 / 28.3, N1698 w 28/7 87 / 78, but w 387/5 31.6 / 35.6,
+//     N4221 w 766/2 126 / 129      D80: N119 w 23/1 15.5 / 12.8, N709 w 12/3 18.5 / 14.5, but N467 w 192/1 24.2 / 25.2, N5041 w 256/3 80 / 87
+//   bf16 D40: N119 w 23/1 10.8 / 9.2, N1173 w 17/2 72 / 66, w 86/4 16.7 / 14.6, N274 w 27/5 11.8 / 10.6, but N467 w 192/1 15.7 / 16.6, N1052 w 49/5 35.1 / 35.4
+//     D96: N45 w 16/1 12.8 / 11.7, w 78/1 14.1 / 13.6, but N826 w 31/2 12.8 / 13.6
+//   N33 - 96, D64 fp32: B1 H25 N33 w 32/13 20.8 / 17.6, H8 N67 w 52/9 23.5 / 20.0, H2 N76 w 76/37 20.9 / 19.3, H1 N46 w 45/46 19.4 / 17.8, but (not at once) H53 N67
+//     w 23/23 29.0 / 35.9
 template <class T, int D, int MODE>
-bool lone_forward(const Problem& p) {
+bool lone_forward(int B, int N, int H, int w1, int w2, int nsplit) {
     if constexpr (!lone<T, D, MODE>() || D == 32) return false;
-    else if constexpr (D == 96) return p.nsplit <= 1 || forward_round<T, D, MODE>(p.B, p.N, p.H, p.w2) == 8;
-    else return true;
+    const int units = (w2 < N - 1 ? w2 : N - 1) + 1, keys = w1 < N ? w1 : N;
+    if constexpr (D == 96) {
+        if (nsplit > 1) return forward_round<T, D, MODE>(B, N, H, w2) == 8;
+        return T::PLANES == 1 ? units > 2 || keys > 96 : units > 4 || keys > 192;
+    }
+    if (N <= 96 && (int64_t)B * H * ((N + BQ - 1) / BQ) * ((units + 7) / 8) <= CUS) return false;
+    if (T::DTYPE == SA2_F32) return units > (keys <= 128 ? 5 : 4);
+    if (T::DTYPE == SA2_F16) return units > 8 || keys > (units <= 4 ? 320 : 192);
+    return units > 8 || keys > (units <= 2 ? 128 : units <= 5 ? 96 : 32);
 }
 // Deltas per segment: what the dQ accumulator in LDS holds, or fewer where the grid asks for it
 template <class T, int D, int MODE>
@@ -1177,36 +1195,29 @@ KpPlan split_kp_plan(int B, int N, int H, int w1, int w2, size_t room) {
 // ------------------------------------------------------------------ launchers ----
 template <class T, int D, int MODE>
 int launch_split_fwd(const Problem& p, hipStream_t st) {
-    if (lone_forward<T, D, MODE>(p)) {
+    if (lone_forward<T, D, MODE>(p.B, p.N, p.H, p.w1, p.w2, p.nsplit)) {
         const int rc = (T::DTYPE == SA2_F32 ? launch_split_fwd_lone_fp32 : T::DTYPE == SA2_F16 ? launch_split_fwd_lone_fp16 : launch_split_fwd_lone_bf16)(
             p, D, exact_products<T>(p, false), st);
         return rc != SA2_OK || p.nsplit <= 1 ? rc : launch_fwd_merge(p, D, T::DTYPE, st);
     }
-    if constexpr (!lone<T, D, MODE>() || D == 32 || D == 96) {
-        using C = SplitCfg<T, D>;
-        const int nqb = (p.N + BQ - 1) / BQ;
-        const int64_t total = (int64_t)nqb * p.B * p.H;
-        if (total > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
-        auto go = [&](auto kernel, int64_t grid) {
-            if (!allow_full_lds((const void*)kernel)) return false;
-            hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(C::FW * 64), C::FWD_LDS, st, p, nqb, (int)grid);
-            return hipGetLastError() == hipSuccess;
-        };
-        auto go_split = [&](auto nq) {
-            constexpr int NQ = decltype(nq)::value;
-            if constexpr (!(lone<T, D, MODE>() && D == 96))
-                if (p.nsplit <= 1) return go(split_fwd_kernel<T, D, MODE, false, NQ>, total);
-            return go(split_fwd_kernel<T, D, MODE, true, NQ>, total * p.nsplit);
-        };
-        if (total * (p.nsplit > 1 ? p.nsplit : 1) > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
-        bool ok;
-        if constexpr (T::PLANES == 1) ok = exact_products<T>(p, false) ? go_split(std::integral_constant<int, 2>{}) : go_split(std::integral_constant<int, 3>{});
-        else ok = go_split(std::integral_constant<int, 3>{});
-        if (!ok) return SA2_ERR_LAUNCH_FAILED;
-        if (p.nsplit <= 1) return SA2_OK;
-        return launch_fwd_merge(p, D, T::DTYPE, st);
-    }
-    return SA2_ERR_UNSUPPORTED;
+    using C = SplitCfg<T, D>;
+    const int nqb = (p.N + BQ - 1) / BQ;
+    const int64_t total = (int64_t)nqb * p.B * p.H, grid = total * (p.nsplit > 1 ? p.nsplit : 1);
+    if (grid > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
+    auto go = [&](auto kernel) {
+        if (!allow_full_lds((const void*)kernel)) return false;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(C::FW * 64), C::FWD_LDS, st, p, nqb, (int)grid);
+        return hipGetLastError() == hipSuccess;
+    };
+    auto go_split = [&](auto nq) {
+        constexpr int NQ = decltype(nq)::value;
+        return p.nsplit > 1 ? go(split_fwd_kernel<T, D, MODE, true, NQ>) : go(split_fwd_kernel<T, D, MODE, false, NQ>);
+    };
+    bool ok;
+    if constexpr (T::PLANES == 1) ok = exact_products<T>(p, false) ? go_split(std::integral_constant<int, 2>{}) : go_split(std::integral_constant<int, 3>{});
+    else ok = go_split(std::integral_constant<int, 3>{});
+    if (!ok) return SA2_ERR_LAUNCH_FAILED;
+    return p.nsplit > 1 ? launch_fwd_merge(p, D, T::DTYPE, st) : SA2_OK;
 }
 
 template <class T, int D, int MODE>
@@ -1363,9 +1374,16 @@ int f32_mfma_fwd_nsplit(int B, int N, int H, int head_dim, int w1, int w2, int d
     return for_split_width(head_dim, dtype, [&](auto m, auto width, auto mode) {
         constexpr int D = decltype(width)::value;
         const int round = forward_round<decltype(m), D, decltype(mode)::value>(B, N, H, w2);
-        // (fp32 up to 64 columns: two short rounds stay one launch.  Up to 3 us would be gained, but at these sizes a forward with a workspace
-        // and one without are compared bit by bit.)
+        // (fp32 up to 64 columns: two short rounds stay one launch, though two shares take B1 H1 N1314 D64 w 17/10 17.8 us for 19.8, H3 N253 w 20/11
+        // 17.6 for 19.8: there a forward without a workspace, which captured callers of the static workspace make, gives the bits of one with it.)
         return plan_forward(B, N, H, D, w1, w2, round, dtype == SA2_F32 && D <= 64 ? 4 : 0, room);
+    });
+}
+// (of tests) whether it has two units per wavefront, and 256 * shares
+int split_fwd_route(int B, int N, int H, int head_dim, int w1, int w2, int dtype) {
+    const int ns = f32_mfma_fwd_nsplit(B, N, H, head_dim, w1, w2, dtype, ROOM_ANY);
+    return ns << 8 | for_split_width(head_dim, dtype, [&](auto m, auto width, auto mode) {
+        return (int)lone_forward<decltype(m), decltype(width)::value, decltype(mode)::value>(B, N, H, w1, w2, ns);
     });
 }
 size_t f32_mfma_fwd_part_bytes(int B, int N, int H, int head_dim, int nsplit) { return fwd_part_bytes(B, N, H, split_width(head_dim), nsplit); }

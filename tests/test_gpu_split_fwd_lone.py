@@ -1,7 +1,8 @@
 """out and lse of the plane-split forward with two units per wavefront where its rounds and its stream of tiles can go wrong: rounds of one to
 eight units (four and fewer have one per wavefront), sweeps shorter than the tiles that are requested ahead, windows that end in the
 middle of a tile, a last tile that the sequence does not fill, shares, both plane counts, and logits that leave the reference point of the
-first tile behind (a unit's sums are brought to another one).  Against the fp32 FMA kernels (accurate expf and logf), to the bars of the
+first tile behind (a unit's sums are brought to another one).  (Up to 32 columns, few deltas and short sequences: the same cases on the kernel
+with one unit per wavefront; tests/test_routes.py says which.)  Against the fp32 FMA kernels (accurate expf and logf), to the bars of the
 other tests of these kernels; lse to 1e-5 of its largest value (16 bits: of exact products of 16-bit inputs, the same)."""
 import pytest
 import torch
@@ -33,6 +34,13 @@ def test_forward_matches_the_fma_kernels(dtype, D, B, N, H, w1, w2, bias, scale)
     assert_close_rel(out, want.cpu(), BAR[dtype], "out")
     assert_close_rel(lse, want_lse.cpu(), 1e-5, "lse")
     assert torch.equal(out, sa.simplicial_forward(*x, w1, w2, scale, bias, -bias)[0])
+
+
+@pytest.mark.parametrize("dtype,D", TYPES[2:])
+@pytest.mark.parametrize("B,N,H,w1,w2,bias", [(1, 33, 150, 20, 20, 0.1), (2, 40, 80, 40, 39, 0.0), (1, 65, 90, 64, 11, -0.2), (3, 96, 33, 5, 9, 0.0), (1, 130, 70, 200, 15, 0.0)])
+def test_short_sequences_of_many_heads(dtype, D, B, N, H, w1, w2, bias):
+    """Sequences of two to five tiles, too many for the kernel with one unit per wavefront."""
+    test_forward_matches_the_fma_kernels(dtype, D, B, N, H, w1, w2, bias, None)
 
 
 @pytest.mark.parametrize("dtype,D", TYPES)
@@ -72,14 +80,15 @@ def test_widely_spread_logits(dtype, D, std):
 @pytest.mark.parametrize("dtype,D", [(F32, 64), (BF, 40), (BF, 56), (BF, 72), (BF, 96), (FP, 48), (FP, 96)])
 @pytest.mark.parametrize("bias", [0.0, 0.25])
 def test_the_reference_point_comes_off_the_logits_last(dtype, D, bias):
-    """The queries' own tile holds logits of -5, one key before it a small generic one, which decides the row.  Less the reference point it is
+    """The queries' own tile holds logits of -5, one key before it a small generic one, which decides the row (all K' rows are the same, so that the
+    nine deltas agree in every rounding).  Less the reference point it is
     7.2 octaves, where a rounding has a root mean square of 2^-22 / sqrt(12) octaves (1e-7 in lse): one of the difference, one of the scale
     where that is multiplied on last, and half of one for the logit's chain at its own size and lse itself.  With the reference point at the start of the chain
     all 12 to 36 roundings had that size (2.8e-7 to 4.5e-7 in lse)."""
     import simplical_attn_amd as sa
     g = torch.Generator().manual_seed(D)
-    x = [torch.randn(2, 64, 16, D, generator=g) for _ in range(5)]
-    x[0], x[2] = 0.5 * x[0], 0.5 * x[2]
+    x = [torch.randn(2, 64, 70, D, generator=g) for _ in range(5)]
+    x[0], x[2] = 0.5 * x[0], (0.5 * x[2][:, :1]).expand_as(x[2]).contiguous()
     x[0][..., 0], x[2][..., 0] = 1.0, 1.0 - bias
     key = x[1][:, 31].clone()
     x[1][:] = 0.0
@@ -87,9 +96,10 @@ def test_the_reference_point_comes_off_the_logits_last(dtype, D, bias):
     key[..., 0] = 0.0
     x[1][:, 31] = key
     x = [t.to(dtype) for t in x]
-    lse = sa.simplicial_forward(*[t.cuda() for t in x], 63, 0, None, bias)[1][:, :, 32:]
-    want = orc.forward_windowed(*[t.double() for t in x], 63, 0, None, bias)[1][:, :, 32:]
-    assert (lse.double().cpu() - want).pow(2).mean().sqrt() < 2.3e-7
+    lse = sa.simplicial_forward(*[t.cuda() for t in x], 63, 8, None, bias)[1][:, :, 32:]
+    want = orc.forward_windowed(*[t.double() for t in x], 63, 8, None, bias)[1][:, :, 32:]
+    error = (lse.double().cpu() - want).pow(2).mean().sqrt().item()
+    assert error < 2.3e-7, error
 
 
 @pytest.mark.parametrize("dtype,D", [(F32, 64), (BF, 40), (BF, 56), (BF, 72), (BF, 96), (FP, 48), (FP, 80)])

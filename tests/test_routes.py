@@ -3,9 +3,10 @@ kernel reach it, and plans hold where they were measured."""
 import ctypes
 
 import pytest
+import torch
 
 from simplical_attn_amd import _lib
-from tests import test_gpu_bwd_kp_lone, test_gpu_bwd_kv, test_gpu_fwd_lone
+from tests import test_gpu_bwd_kp_lone, test_gpu_bwd_kv, test_gpu_fwd_lone, test_gpu_split_fwd_lone
 
 
 def _ask(name, B, N, H, D, w1, w2, force=None):
@@ -30,6 +31,14 @@ def kv_route(B, N, H, D, w1, w2):
     """(32-row K blocks per wavefront, shares)"""
     r = _ask("_ZN3sa213mfma_kv_routeEiiiiii", B, N, H, D, w1, w2)
     return r & 255, r >> 8
+
+
+def split_route(what, dtype, B, N, H, D, w1, w2):
+    """Plane-split kernels: (one wavefront per SIMD, shares or segments)"""
+    f = getattr(_lib.load(), "_ZN3sa215split_%s_routeEiiiiiii" % what if what == "fwd" else "_ZN3sa214split_%s_routeEiiiiiii" % what)
+    code = {torch.float32: _lib.SA2_F32, torch.bfloat16: _lib.SA2_BF16, torch.float16: _lib.SA2_F16}[dtype]
+    r = f(*[ctypes.c_int(x) for x in (B, N, H, D, min(w1, N - 1), min(w2, N - 1), code)])
+    return bool(r & 1), r >> 8
 
 
 def _cases(test):
@@ -101,3 +110,34 @@ def test_kv_cases_have_both_geometries_and_shares():
 ])
 def test_k_side_plan(B, N, H, D, w1, w2, want):
     assert kv_route(B, N, H, D, w1, w2) == want
+
+
+def test_plane_split_forward_cases_reach_both_kernels():
+    """Two units per wavefront where their test is about them: rounds of one to eight units, short sweeps, shares, moved reference points."""
+    t = test_gpu_split_fwd_lone
+    for dtype, D in t.TYPES:
+        route = lambda B, N, H, w1, w2: split_route("fwd", dtype, B, N, H, D, w1, w2)
+        matches = {c[:5]: route(*c[:5]) for c in _cases(t.test_forward_matches_the_fma_kernels)}
+        many = [route(*c[:5]) for c in _cases(t.test_short_sequences_of_many_heads)]
+        if D <= 32:
+            assert not any(lone for lone, _ in list(matches.values()) + many)
+            continue
+        assert all(lone for lone, _ in many)
+        two = (dtype, D) != (t.FP, 80)                      # (there shares of up to twenty deltas have one unit per wavefront)
+        for case in ((1, 520, 2, 95, 33), (1, 640, 30, 70, 40), *(((1, 200, 1, 500, 8), (1, 161, 1, 3, 12)) if D <= 64 else ())):
+            assert matches[case][0]
+        assert matches[1, 520, 2, 95, 33][1] > 1 and not matches[1, 33, 1, 0, 0][0]
+        assert route(1, 470, 2, 300, 12)[0] == two and route(1, 470, 40, 300, 20)[0] and route(1, 400, 6, 150, 20)[0]
+        assert route(2, 150, 8, 149, 9)[0] == two and route(2, 150, 8, 149, 40)[0] and route(2, 150, 1, 149, 30)[0] and route(2, 64, 70, 63, 8)[0]
+
+
+@pytest.mark.parametrize("dtype,D,shape,lone", [
+    (torch.float32, 64, (1, 826, 1, 31, 2), False), (torch.float32, 64, (1, 131, 46, 90, 4), False), (torch.float32, 64, (1, 388, 7, 405, 4), True),
+    (torch.float32, 64, (1, 1052, 19, 49, 5), True), (torch.float32, 64, (1, 67, 8, 52, 9), False), (torch.float32, 64, (1, 67, 53, 23, 23), True),
+    (torch.float32, 64, (2, 2048, 8, 512, 32), True), (torch.float16, 48, (1, 378, 31, 64, 6), False), (torch.float16, 48, (1, 388, 7, 387, 5), True),
+    (torch.float16, 48, (1, 4221, 4, 766, 2), True), (torch.float16, 80, (1, 709, 11, 12, 3), False), (torch.float16, 80, (1, 5041, 4, 256, 3), True),
+    (torch.bfloat16, 40, (1, 274, 1, 27, 5), False), (torch.bfloat16, 40, (1, 1052, 19, 49, 5), True), (torch.bfloat16, 96, (1, 45, 16, 16, 1), False),
+    (torch.bfloat16, 96, (1, 826, 1, 31, 2), True), (torch.bfloat16, 96, (1, 2048, 8, 255, 31), True)])
+def test_plane_split_forward_by_deltas_and_sweep(dtype, D, shape, lone):
+    B, N, H, w1, w2 = shape
+    assert split_route("fwd", dtype, B, N, H, D, w1, w2)[0] == lone
