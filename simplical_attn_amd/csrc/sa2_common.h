@@ -217,6 +217,8 @@ int launch_f32_mfma_fwd(const Problem& p, int dtype, hipStream_t st);
 int f32_mfma_fwd_nsplit(int B, int N, int H, int D, int w1, int w2, int dtype, size_t room);
 size_t f32_mfma_fwd_part_bytes(int B, int N, int H, int D, int nsplit);
 int split_fwd_route(int B, int N, int H, int D, int w1, int w2, int dtype);
+int split_kp_route(int B, int N, int H, int D, int w1, int w2, int dtype);
+int split_kv_route(int B, int N, int H, int D, int w1, int w2, int dtype);
 int launch_f32_mfma_bwd(const Problem& p, int dtype, hipStream_t st);
 // Its forward and K side with one wavefront per SIMD (sa2_split_fwd_lone.h, sa2_split_kv_lone.h).  `width`: of the kernel; `two_planes`:
 // products of a unit have 16 bits

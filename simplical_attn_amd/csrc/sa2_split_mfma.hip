@@ -1192,6 +1192,22 @@ KpPlan split_kp_plan(int B, int N, int H, int w1, int w2, size_t room) {
     return plan_segments(B, N, H, w1, w2, NPAIR, most, room, [](int) { return false; }, [&](const KpPlan& pl) { return split_kp_bytes(B, N, H, D, pl); });
 }
 
+// Whether the K' side takes its kernel with one wavefront per SIMD: not where all rounds of four deltas are at once on the chip, so that each is
+// all of a workgroup, and the sweeps are short.  One wavefront per SIMD against pairs there, K' side with guard and sums, us: fp32 D16 B1 H1 N58 w 35/12 23.7 /
+// 21.6, H2 N225 w 89/10 28.0 / 27.2, H1 N1314 w 17/10 26.0 / 24.3, D32 H2 N119 w 23/1 24.4 / 23.2, fp16 D48 H2 N119 w 23/1 26.4 / 24.7, N1314 w 17/10 29.8 /
+// 27.8, D80 34.9 / 31.9 (N58), 42.0 / 39.9 (N225), bf16 D40 24.8 / 22.9 and 28.7 / 28.0; wide windows: fp32 D16 H1 N599 w 465/1 1.05, D32 1.07, bf16 D40 1.06 the
+// other way, fp16 0.98.  fp32 D64 and bf16 at 96 columns are faster with one everywhere (1.04 and 1.13 at the median of such grids).
+template <class T, int D, int MODE>
+bool lone_kp(int B, int N, int H, int w1, int w2, const KpPlan& pl) {
+    if constexpr (!lone<T, D, MODE>()) return false;
+    if constexpr (T::DTYPE == SA2_F32 ? D == 64 : T::PLANES == 1 && D == 96) return true;
+    const int units = (w2 < N - 1 ? w2 : N - 1) + 1, keys = w1 < N ? w1 : N;
+    const int64_t rounds = (int64_t)B * H * ((N + BQ - 1) / BQ) * ((units + NPAIR - 1) / NPAIR);
+    return rounds > CUS || keys > (T::DTYPE == SA2_F16 ? 256 : 128) || !SplitCfg<T, D>::kp_fits(pl.segw - 1);
+}
+template <class T, int D, int MODE>
+bool lone_kv(int N, int w2) { return lone<T, D, MODE>(); }
+
 // ------------------------------------------------------------------ launchers ----
 template <class T, int D, int MODE>
 int launch_split_fwd(const Problem& p, hipStream_t st) {
@@ -1245,12 +1261,12 @@ int launch_split_bwd(const Problem& p, hipStream_t st) {
         if (total > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
         float* part = (float*)p.scratch;
         float* kpart = (float*)((char*)p.scratch + split_dq_part_bytes(p.B, p.N, p.H, D, pl));
-        if constexpr (lone<T, D, MODE>()) {
+        if (lone_kp<T, D, MODE>(p.B, p.N, p.H, p.w1, p.w2, pl)) {
             const SplitKpLaunch l = {pl, nkb, (int)per_seg, part, kpart};
             const int rc = (T::DTYPE == SA2_F32 ? launch_split_kp_lone_fp32 : T::DTYPE == SA2_F16 ? launch_split_kp_lone_fp16 : launch_split_kp_lone_bf16)(
                 p, D, exact_products<T>(p, true), l, st);
             if (rc != SA2_OK) return rc;
-        } else {
+        } else if constexpr (!(lone<T, D, MODE>() && (T::DTYPE == SA2_F32 ? D == 64 : T::PLANES == 1 && D == 96))) {
             if (!allow_full_lds((const void*)split_kp_kernel<T, D, MODE>)) return SA2_ERR_LAUNCH_FAILED;
             hipLaunchKernelGGL((split_kp_kernel<T, D, MODE>), dim3((unsigned)total), dim3(XT), C::kp_lds(pl.segw - 1), st, p, nkb, (int)per_seg, part,
                                pl.nseg, pl.segw, kpart);
@@ -1267,11 +1283,11 @@ int launch_split_bwd(const Problem& p, hipStream_t st) {
         const int64_t total = (int64_t)njb * p.B * p.H * nsplit;
         if (total > 0x7fffffffLL) return SA2_ERR_TOO_LARGE;
         float* part = nsplit > 1 ? (float*)((char*)p.scratch + kp_bytes) : nullptr;
-        if constexpr (lone<T, D, MODE>()) {
+        if (lone_kv<T, D, MODE>(p.N, p.w2)) {
             const int rc = (T::DTYPE == SA2_F32 ? launch_split_kv_lone_fp32 : T::DTYPE == SA2_F16 ? launch_split_kv_lone_fp16 : launch_split_kv_lone_bf16)(
                 p, D, exact_products<T>(p, true), nsplit, part, st);
             if (rc != SA2_OK) return rc;
-        } else {
+        } else if constexpr (!lone<T, D, MODE>()) {
             auto go = [&](auto kernel) {
                 if (!allow_full_lds((const void*)kernel)) return false;
                 hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(XT), C::KV_LDS, st, p, njb, (int)total, nsplit, part);
@@ -1379,7 +1395,19 @@ int f32_mfma_fwd_nsplit(int B, int N, int H, int head_dim, int w1, int w2, int d
         return plan_forward(B, N, H, D, w1, w2, round, dtype == SA2_F32 && D <= 64 ? 4 : 0, room);
     });
 }
-// (of tests) whether it has two units per wavefront, and 256 * shares
+// (of tests) whether its forward has two units per wavefront, and 256 * shares; whether its K' and K side have one wavefront per SIMD, and 256 *
+// segments or shares
+int split_kp_route(int B, int N, int H, int head_dim, int w1, int w2, int dtype) {
+    return for_split_width(head_dim, dtype, [&](auto m, auto width, auto mode) {
+        const KpPlan pl = split_kp_plan<decltype(m), decltype(width)::value, decltype(mode)::value>(B, N, H, w1, w2, ROOM_ANY);
+        return pl.nseg << 8 | (int)lone_kp<decltype(m), decltype(width)::value, decltype(mode)::value>(B, N, H, w1, w2, pl);
+    });
+}
+int split_kv_route(int B, int N, int H, int head_dim, int w1, int w2, int dtype) {
+    return for_split_width(head_dim, dtype, [&](auto m, auto width, auto mode) {
+        return split_kv_nsplit(B, N, H, decltype(width)::value, w1, w2, ROOM_ANY) << 8 | (int)lone_kv<decltype(m), decltype(width)::value, decltype(mode)::value>(N, w2);
+    });
+}
 int split_fwd_route(int B, int N, int H, int head_dim, int w1, int w2, int dtype) {
     const int ns = f32_mfma_fwd_nsplit(B, N, H, head_dim, w1, w2, dtype, ROOM_ANY);
     return ns << 8 | for_split_width(head_dim, dtype, [&](auto m, auto width, auto mode) {

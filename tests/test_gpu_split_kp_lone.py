@@ -1,6 +1,7 @@
 """dQ, dK' and dV' of the plane-split K' side with one wavefront per SIMD where its rounds and its stream of tiles can go wrong: wavefronts
 without a unit in the last round, sweeps shorter than the tiles that are requested ahead, windows that begin and end in the middle of a
-tile, a last tile that the sequence does not fill, segments, q and dO rows that do not fit LDS, both plane counts.  Against the fp32 FMA
+tile, a last tile that the sequence does not fill, segments, q and dO rows that do not fit LDS, both plane counts.  (Small grids with short
+sweeps: some types' kernel with two wavefronts per SIMD; tests/test_routes.py says which.)  Against the fp32 FMA
 kernels, to the bars of the other tests of these kernels (fp32 1e-5, bf16 2e-2, fp16 1e-2)."""
 import pytest
 import torch
@@ -32,3 +33,11 @@ def test_kp_side_matches_the_fma_kernels(dtype, D, B, N, H, w1, w2, bias):
         assert_close_rel(got[i], want[i].cpu(), BAR[dtype], name, atol=atol)
     again = sa.simplicial_backward(*x[:5], out, lse, x[5], w1, w2, needs=(False, False, True, False, True), **kw)
     assert torch.equal(got[2], again[2]) and torch.equal(got[4], again[4])
+
+
+@pytest.mark.parametrize("dtype,D", [(F32, 16), (F32, 32), (F32, 64), (BF, 40), (BF, 56), (BF, 72), (BF, 96), (FP, 48), (FP, 80)])
+@pytest.mark.parametrize("B,N,H,w1,w2,bias", [
+    (1, 1, 300, 0, 0, 0.0), (1, 33, 130, 0, 0, 0.0), (1, 65, 90, 64, 11, 0.1), (2, 40, 80, 40, 39, 0.0), (1, 97, 70, 31, 2, -0.2), (1, 130, 60, 5, 1, 0.0)])
+def test_short_sequences_of_many_heads(dtype, D, B, N, H, w1, w2, bias):
+    """One to five tiles, more rounds than are at once on the chip."""
+    test_kp_side_matches_the_fma_kernels(dtype, D, B, N, H, w1, w2, bias)

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from simplical_attn_amd import _lib
-from tests import test_gpu_bwd_kp_lone, test_gpu_bwd_kv, test_gpu_fwd_lone, test_gpu_split_fwd_lone
+from tests import test_gpu_bwd_kp_lone, test_gpu_bwd_kv, test_gpu_fwd_lone, test_gpu_split_fwd_lone, test_gpu_split_kp_lone, test_gpu_split_kv_lone
 
 
 def _ask(name, B, N, H, D, w1, w2, force=None):
@@ -35,7 +35,7 @@ def kv_route(B, N, H, D, w1, w2):
 
 def split_route(what, dtype, B, N, H, D, w1, w2):
     """Plane-split kernels: (one wavefront per SIMD, shares or segments)"""
-    f = getattr(_lib.load(), "_ZN3sa215split_%s_routeEiiiiiii" % what if what == "fwd" else "_ZN3sa214split_%s_routeEiiiiiii" % what)
+    f = getattr(_lib.load(), "_ZN3sa2%dsplit_%s_routeEiiiiiii" % (len("split__route" + what), what))
     code = {torch.float32: _lib.SA2_F32, torch.bfloat16: _lib.SA2_BF16, torch.float16: _lib.SA2_F16}[dtype]
     r = f(*[ctypes.c_int(x) for x in (B, N, H, D, min(w1, N - 1), min(w2, N - 1), code)])
     return bool(r & 1), r >> 8
@@ -43,6 +43,10 @@ def split_route(what, dtype, B, N, H, D, w1, w2):
 
 def _cases(test):
     return next(m for m in test.pytestmark if m.name == "parametrize").args[1]
+
+
+def _types(test):
+    return next(m for m in test.pytestmark if m.name == "parametrize" and m.args[0] == "dtype,D").args[1]
 
 
 @pytest.mark.parametrize("B,N,H,D,w1,w2,lone", [
@@ -141,3 +145,31 @@ def test_plane_split_forward_cases_reach_both_kernels():
 def test_plane_split_forward_by_deltas_and_sweep(dtype, D, shape, lone):
     B, N, H, w1, w2 = shape
     assert split_route("fwd", dtype, B, N, H, D, w1, w2)[0] == lone
+
+
+def test_plane_split_kp_cases_reach_both_kernels():
+    t = test_gpu_split_kp_lone
+    for dtype, D in _types(t.test_kp_side_matches_the_fma_kernels):
+        route = lambda c: split_route("kp", dtype, c[0], c[1], c[2], D, c[3], c[4])
+        assert all(route(c)[0] for c in _cases(t.test_short_sequences_of_many_heads))
+        matches = {c[:5]: route(c) for c in _cases(t.test_kp_side_matches_the_fma_kernels)}
+        assert matches[1, 640, 16, 70, 400][0] and matches[1, 640, 16, 70, 400][1] > 1 and matches[1, 700, 40, 129, 3][0]
+        assert matches[1, 33, 1, 0, 0][0] == ((dtype, D) in ((t.F32, 64), (t.BF, 72), (t.BF, 96)))
+
+
+@pytest.mark.parametrize("dtype,D,shape,lone", [
+    (torch.float32, 16, (1, 1314, 1, 17, 10), False), (torch.float32, 16, (1, 599, 1, 465, 1), True), (torch.float32, 32, (1, 119, 2, 23, 1), False),
+    (torch.float32, 64, (1, 119, 2, 23, 1), True), (torch.float16, 48, (1, 225, 2, 89, 10), False), (torch.float16, 80, (1, 773, 1, 236, 1), False),
+    (torch.float16, 80, (1, 2048, 8, 255, 31), True), (torch.bfloat16, 40, (1, 58, 1, 35, 12), False), (torch.bfloat16, 40, (1, 381, 2, 380, 9), True),
+    (torch.bfloat16, 96, (1, 58, 1, 35, 12), True)])
+def test_plane_split_kp_side_by_grid_and_sweep(dtype, D, shape, lone):
+    B, N, H, w1, w2 = shape
+    assert split_route("kp", dtype, B, N, H, D, w1, w2)[0] == lone
+
+
+def test_plane_split_kv_cases_reach_both_kernels():
+    t = test_gpu_split_kv_lone
+    for dtype, D in _types(t.test_k_side_matches_the_fma_kernels):
+        routes = {c[:5]: split_route("kv", dtype, c[0], c[1], c[2], D, c[3], c[4]) for c in _cases(t.test_k_side_matches_the_fma_kernels)}
+        assert all(lone for (B, N, H, w1, w2), (lone, _) in routes.items())
+        assert routes[1, 520, 2, 95, 33][1] > 1 and routes[3, 40, 5, 40, 39][0]
