@@ -1205,8 +1205,10 @@ bool lone_kp(int B, int N, int H, int w1, int w2, const KpPlan& pl) {
     const int64_t rounds = (int64_t)B * H * ((N + BQ - 1) / BQ) * ((units + NPAIR - 1) / NPAIR);
     return rounds > CUS || keys > (T::DTYPE == SA2_F16 ? 256 : 128) || !SplitCfg<T, D>::kp_fits(pl.segw - 1);
 }
+// ... and the K side: in fp16 not for few deltas of sequences that leave its blocks of 128 keys half empty.  us, one wavefront per SIMD against pairs: D48
+// B1 H1 N58 w 35/12 27.3 / 26.5, H17 N79 w 125/1 26.8 / 24.5, D80 35.8 / 33.9 and 35.2 / 31.9, but H2 N76 w 76/37 36.2 / 39.2, H50 N74 w 73/55 117 / 145.
 template <class T, int D, int MODE>
-bool lone_kv(int N, int w2) { return lone<T, D, MODE>(); }
+bool lone_kv(int N, int w2) { return lone<T, D, MODE>() && (T::DTYPE != SA2_F16 || N > 80 || w2 >= 20); }
 
 // ------------------------------------------------------------------ launchers ----
 template <class T, int D, int MODE>
@@ -1287,7 +1289,7 @@ int launch_split_bwd(const Problem& p, hipStream_t st) {
             const int rc = (T::DTYPE == SA2_F32 ? launch_split_kv_lone_fp32 : T::DTYPE == SA2_F16 ? launch_split_kv_lone_fp16 : launch_split_kv_lone_bf16)(
                 p, D, exact_products<T>(p, true), nsplit, part, st);
             if (rc != SA2_OK) return rc;
-        } else if constexpr (!lone<T, D, MODE>()) {
+        } else if constexpr (!lone<T, D, MODE>() || T::DTYPE == SA2_F16) {
             auto go = [&](auto kernel) {
                 if (!allow_full_lds((const void*)kernel)) return false;
                 hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(XT), C::KV_LDS, st, p, njb, (int)total, nsplit, part);

@@ -1,6 +1,6 @@
 """dK and dV of the plane-split K side with one wavefront per SIMD where its stream of units can go wrong: one delta per query block, key blocks
 that some or all wavefronts have no keys of, windows that begin and end in the middle of a block, more and fewer units than are formed
-ahead, shares, both plane counts.  Against the fp32 FMA kernels, to the bars of the other tests of these kernels (fp32 1e-5, 16 bits
+ahead, shares, both plane counts.  (fp16, few deltas of up to 80 queries: the kernel with two wavefronts per SIMD.)  Against the fp32 FMA kernels, to the bars of the other tests of these kernels (fp32 1e-5, 16 bits
 half an ulp of the results and what D = sum dO * out loses with a rounded out: 2e-2, fp16 1e-2)."""
 import pytest
 import torch
