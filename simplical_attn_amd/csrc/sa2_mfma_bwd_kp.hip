@@ -832,7 +832,7 @@ KpRoute kp_route(int N, int w1, int w2, int64_t total, const KpPlan& pl, bool fo
     // (unless the grid is so small that a further launch costs more than the lone round)
     const int left = pl.nseg == 1 && w2 >= NPAIR && w2 % NPAIR == 0 && (force_prepass || total >= 768) ? 1 : 0;
     const int all = (w2 < N - 1 ? w2 : N - 1) + 1 - left, units = all < pl.segw ? all : pl.segw;
-    if constexpr (D == 64 || D == 128) return {left, KpLoneCfg<D>::fits(pl.segw - 1) && KpLoneCfg<D>::wanted(N, w1, units, total)};
+    if constexpr (D == 64 || D == 128) return {left, KpLoneCfg<D>::fits(pl.segw - 1) && KpLoneCfg<D>::wanted(N, w1, units, (double)all / pl.nseg, total)};
     else return {left, false};
 }
 

@@ -52,6 +52,7 @@ def _types(test):
 @pytest.mark.parametrize("B,N,H,D,w1,w2,lone", [
     (1, 4096, 8, 64, 512, 0, False),        # one delta: half of what a wavefront with two units computes is thrown away
     (1, 4096, 16, 64, 512, 2, False), (1, 4096, 16, 64, 512, 6, True), (2, 2048, 8, 64, 512, 32, True),
+    (1, 2600, 4, 64, 150, 40, False), (1, 6950, 1, 64, 226, 40, False), (1, 969, 7, 64, 272, 20, True),
     (1, 4096, 16, 128, 512, 1, False), (1, 3000, 8, 128, 500, 31, False), (1, 8192, 16, 128, 512, 32, True), (1, 32768, 8, 128, 1024, 64, True),
 ])
 def test_kp_side_by_keys_deltas_and_grid(B, N, H, D, w1, w2, lone):
