@@ -9,16 +9,16 @@
 // ring of three; others are split by all threads between the MFMAs, one tile ahead, into a ring of two.  K' and V' rows lie in a ring of 64,
 // eight new ones a round.  Running sums of R * (v2 + bias) stay in registers for all rounds and the wavefronts are merged once.
 //
-// What bounds it: the instructions beside the MFMAs (fp32 head_dim 64: 98 MFMAs, 520 others in a tile's 4500 cycles; bf16 at 96 columns 60 and
-// 380).  Forward, us, eight wavefronts of one unit / this: bf16 B1 H8 N2048 D96 w 255/31 240 / 158 (four wavefronts 364), fp32 B2 H8 N2048 D64
-// w 512/32 812 / 775, B1 H2 N128 D64 w 32/16 (eight workgroups, not shared) 28.2 / 25.7.
+// What bounds it: the instructions beside the MFMAs (fp32 head_dim 64: 98 MFMAs, 520 others in a tile's 4500 cycles; bf16 at 96 columns 62 and
+// 380).  Forward, us, one unit per wavefront (eight of them at 64 columns, four at 96) / this: bf16 B1 H8 N2048 D96 w 255/31 330 / 141, fp16 D80 393 / 219,
+// fp32 B2 H8 N2048 D64 w 512/32 795 / 737, bf16 B2 H4 N2048 D40 w 255/31 143 / 113.
 //
 // The reference point m of a row is the largest logit of the wavefront's first two units in the queries' own tile, which holds a key of every
 // row.  A logit less m is rounded at the size of the difference.  So the largest logit S of each further tile is looked at before the
 // exponentials, and a unit's sums are brought to a reference point there where S - m is more than 8 octaves and more than twice |S|, at whose size S is
-// rounded in any case, or more than 40 octaves (weights and their sums stay far from overflow until then; a block whose sums of
-// values do not is computed by rows); the tile's logits are then formed
-// again without m, by a branch that usual logits hardly take.  With keys of the own tile 15, 30, 1e3 and 1e5 octaves below the row's others
+// rounded in any case, or more than 40 octaves (weights and their sums stay far from overflow until then; a block whose sums of values do not
+// is computed by rows).  The tile's logits are then formed again without m, by a branch that usual logits hardly take (with eight times their
+// spread the first two sizes above take 165 and 245).  With keys of the own tile 15, 30, 1e3 and 1e5 octaves below the row's others
 // and only a step at 64 octaves, taken off the rounded difference, fp32 outputs were 1.6, 2.4, 39 and 4800 times as far from fp64 as with a
 // maximum taken per tile; now they are as far (0.97).
 #pragma once

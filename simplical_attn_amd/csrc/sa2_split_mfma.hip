@@ -29,8 +29,9 @@
 //   split_fwd_kernel    32 queries per workgroup; wavefront w takes delta = w, w+W, ... and keeps one
 //                       online softmax and one output accumulator across its units; the W are
 //                       merged once at the end.
-//                       For fp32 at 64 columns and less (but for the finer sums) and 16 bits at 64 and 96, here and below:
-//                       sa2_split_fwd_lone.h, sa2_split_kp_lone.h and sa2_split_kv_lone.h.
+//                       At 64 columns (fp32 but for the finer sums) and in 16 bits at 96 mostly sa2_split_fwd_lone.h (lone_forward
+//                       below).  Backward: fp32 at 64 columns and less (but for the finer sums) and 16 bits at 64 and 96 mostly
+//                       sa2_split_kp_lone.h (lone_kp) and sa2_split_kv_lone.h (lone_kv).
 //   split_kp_kernel     32 K' rows per workgroup and every delta (or a segment of them).  After a unit's
 //                       sweep its three reductions go to fp32 accumulators in LDS in column-rotated
 //                       phases: dK' and dV' rows are aligned with the unit's rows, dQ rows are shifted by
